@@ -89,7 +89,23 @@ struct GemmGroups {
   const int32_t* row_pair;
   int top;
 };
-template <int BN, int BM, int WN, int WM, int BK, int S, int EPI, typename TO, bool WF, int GR = 0>
+//
+// F32: float32 operands on the float32 MFMA (float32 products and sums).  Bytes are what the loads, the stages and the fragments are
+// made of, so a float32 matrix goes through as rows of twice as many 16-bit places (k counts those): 16 bytes of a row are 4
+// floats instead of 8 bfloat16 values, and a fragment-major float32 W (blocks of 16 rows x 16 floats, 1 KB) has its chunks where
+// the bfloat16 one has them.
+template <bool F32>
+__device__ __forceinline__ f32x16_t dma_mfma(const Frag8& a, const Frag8& b, f32x16_t c) {
+  if constexpr (F32) {
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.u.x), __uint_as_float(b.u.x), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.u.y), __uint_as_float(b.u.y), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.u.z), __uint_as_float(b.u.z), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.u.w), __uint_as_float(b.u.w), c, 0, 0, 0);
+  } else {
+    return mfma32(a, b, c);
+  }
+}
+template <int BN, int BM, int WN, int WM, int BK, int S, int EPI, typename TO, bool WF, int GR = 0, bool F32 = false>
 __global__ __launch_bounds__(64 * (BN / WN) * (BM / WM)) void gemm_dma_kernel(const bf16_t* __restrict__ x,
                                                        const bf16_t* __restrict__ w, TO* __restrict__ c,
                                                        float* __restrict__ slabs, int m, int n, int k, int m_tiles,
@@ -228,7 +244,7 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BM / WM)) void gemm_dma_kernel(co
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = mfma32(b[buf2][j], a[buf2][i], acc[i][j]);
+      for (int j = 0; j < TM; ++j) acc[i][j] = dma_mfma<F32>(b[buf2][j], a[buf2][i], acc[i][j]);
   };
 
   // ---- main loop.  The barrier that hands over tile kt + 1 stands before the last depth step
@@ -271,7 +287,7 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BM / WM)) void gemm_dma_kernel(co
     for (int ks = 0; ks + 1 < KSTEPS; ++ks) {
 #pragma unroll
       for (int q = 0; q < NM; ++q) {
-        acc[q / TM][q % TM] = mfma32(b[ks & 1][q % TM], a[ks & 1][q / TM], acc[q / TM][q % TM]);
+        acc[q / TM][q % TM] = dma_mfma<F32>(b[ks & 1][q % TM], a[ks & 1][q / TM], acc[q / TM][q % TM]);
 #pragma unroll
         for (int f = q; f < TN + TM; f += NM) frag_one((ks + 1) & 1, kt, ks + 1, f);
         __builtin_amdgcn_sched_barrier(0);
@@ -285,7 +301,7 @@ __global__ __launch_bounds__(64 * (BN / WN) * (BM / WM)) void gemm_dma_kernel(co
   auto last_step = [&](auto once, int kt, bool fetch) {
 #pragma unroll
     for (int q = 0; q < NM; ++q) {
-      acc[q / TM][q % TM] = mfma32(b[LASTBUF][q % TM], a[LASTBUF][q / TM], acc[q / TM][q % TM]);
+      acc[q / TM][q % TM] = dma_mfma<F32>(b[LASTBUF][q % TM], a[LASTBUF][q / TM], acc[q / TM][q % TM]);
       if (fetch) {
 #pragma unroll
         for (int l = q; l < LOADS; l += NM) issue_one(once, kt + S, l);

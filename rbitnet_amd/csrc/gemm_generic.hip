@@ -7,6 +7,7 @@
 // Reference: y[o] = sum_i W[i + o * n_in] * x[i] (llama/model.rs:67-91).
 #include "api.h"
 #include "common.h"
+#include "gemm_internal.h"
 
 #define GT 64      // tile of C: GT x GT
 #define GK 16      // depth of one stage
@@ -276,8 +277,8 @@ static void launch_f32_few(const float* x, const float* w, bool w_frag, float* c
   else gemm_f32_few_kernel<MB, 1, false><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
 }
 
-// Float32 operands and more than 16 tokens with K a multiple of 16 (the float32 path's
-// prefill): the float32 MFMA (v_mfma_f32_32x32x2_f32: float32 inputs, float32 products and
+// Float32 operands and more than 16 tokens with K a multiple of 16 that is not one of 32, or operands
+// that are not 16-byte aligned (everything else: gemm_f32.hip): the float32 MFMA (v_mfma_f32_32x32x2_f32: float32 inputs, float32 products and
 // sums; no reduced-precision mode).  128 x 128 tiles, 16 deep, one wave per 64 x 64 piece.  W
 // and the tokens are read with 16-byte loads along K and stored in LDS depth-major
 // ([k][row], rows padded by 4 floats), so that the 32 lanes that read one depth value of 32
@@ -423,6 +424,14 @@ extern "C" int rb_gemm_generic(const void* a, const void* w, int w_layout, void*
     else gemm_f32_skinny_kernel<16><<<blocks, 256, 0, s>>>(af, wf, (float*)c, m, n, k);
     RB_LAUNCH_CHECK();
     return 0;
+  }
+  if (dtype_in == RB_F32 && dtype_out == RB_F32 && m > 16) {
+    int rc = 0;
+    if (gemm_f32_dma_try((const float*)a, (const float*)w, w_frag, (float*)c, m, n, k, s, &rc)) {
+      if (rc) return rc;
+      RB_LAUNCH_CHECK();
+      return 0;
+    }
   }
   if (dtype_in == RB_F32 && dtype_out == RB_F32 && m > 16 && k % GM_K == 0) {
     dim3 tiles((n + GM_T - 1) / GM_T, (m + GM_T - 1) / GM_T);

@@ -49,3 +49,6 @@ bool gemm_resident_try(const GemmTokens& x, const bf16_t* w, void* c, int dtype_
 int gemm_tiled_parts(int m, int n, int k, int epilogue);
 int gemm_tiled_launch(const bf16_t* x, const bf16_t* w, bool w_frag, void* c, float* workspace, int dtype_out,
                       int epilogue, int m, int n, int k, hipStream_t s, const float* act = nullptr);
+// float32, more than 16 tokens, K % 32 == 0: tiles through LDS on the float32 MFMA (gemm_f32.hip); false: these operands are not
+// for it and nothing was launched
+bool gemm_f32_dma_try(const float* x, const float* w, bool w_frag, float* c, int m, int n, int k, hipStream_t s, int* rc);
