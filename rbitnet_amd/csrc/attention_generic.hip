@@ -14,6 +14,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "mfma.h"
 
 #define AG_MAX_D 512
 #define AG_MAX_D_VEC 256      // the 16-byte kernel deals a row's quads to the lanes of one wave
@@ -280,8 +281,237 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_generic_vec_
   }
 }
 
+// Float32 attention on the float32 MFMA (16x16x4: float32 inputs, products and sums), for head sizes that are multiples of 4 up to
+// 128.  The 16 columns of the MFMAs are queries: the heads that share a key/value head, of one token or of as many consecutive
+// tokens as fit, so that a key is read once for all of them.  Scores are K Q^T (a lane takes one key's row, 16 bytes at a time, and
+// four MFMAs use the four floats of it), so that a lane ends up with 4 keys' weights of one query, which is what the second
+// product, V^T P^T, takes as its operand as they are; V's rows are dealt to the lanes NB numbers at a time (MFMA dt works on the
+// numbers NB r + dt of a head for its row r), so that they come with wide loads and leave as pieces of rows.  The waves of a workgroup
+// share the keys, 32 at a time, and merge through LDS at the end.  Softmax, its running maximum, caps, sinks, windows, kept first
+// keys, chunks and sigmoid weights as in the kernels above.
+// Bound by the MFMAs for prompts (2 x 32 cycles for 16 keys, 16 queries and 4 numbers) and by a chain of loads in single-token
+// steps.  Measured beside the kernel above (a lane per key on the vector units), 24 heads of 128 on 8: four prompts of 131 to 512 tokens
+// 600 -> 125 us a layer, one token for each of four sequences at 131 to 520 keys 29 -> 24 us (32 workgroups,
+// whose matrix cores three of sixteen columns keep busy: what bounds it now).
+template <int NB>
+__global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_kernel(
+    const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages, float* __restrict__ out,
+    const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ block_table, int bt_stride,
+    int n_tokens, int n_heads, int n_kv, int head_dim, float scale, int window, const float* __restrict__ sinks, int keep_first,
+    float softcap, int chunk, const float* __restrict__ sig_bias, int tokens_per_block, int head_chunks) {
+  constexpr int VW = NB < 4 ? NB : 4;                  // floats of a load of V
+  constexpr int LD = 16 * NB + 4;                      // a query's row in LDS: outputs, then maximum and sum
+  extern __shared__ __attribute__((aligned(16))) float merged[];      // [waves][16][LD]
+  const int lane = threadIdx.x & (RB_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / RB_WAVE), n_waves = blockDim.x / RB_WAVE;
+  const int col = lane & 15, g = lane >> 4;
+  const int group = n_heads / n_kv;
+  const int kvh = blockIdx.y / head_chunks, first = (blockIdx.y % head_chunks) * 16;
+  const int h_count = group - first < 16 ? group - first : 16;
+  const int h0 = kvh * group + first;
+  // late tokens first: they have the most keys
+  const int t0 = (gridDim.x - 1 - blockIdx.x) * tokens_per_block;
+  const int t1 = t0 + tokens_per_block < n_tokens ? t0 + tokens_per_block : n_tokens;
+  const int t = t0 + col / h_count, h = h0 + col % h_count;
+  const bool on = t < t1;
+  const int my_pos = on ? tok_pos[t] : -1;
+  const int my_lo = on ? first_visible(my_pos, window, chunk) : 0;
+
+  f32x4_t qv[NB], acc[NB];
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    qv[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    if (on && 16 * c + 4 * g < head_dim)
+      qv[c] = *reinterpret_cast<const f32x4_t*>(q + ((size_t)t * n_heads + h) * head_dim + 16 * c + 4 * g);
+    acc[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  }
+  const float sb = sig_bias && on ? sig_bias[h] : 0.f;
+  float m_run = sig_bias ? 0.f : -INFINITY, l_run = 0.f;
+
+  // the tokens of a block belong to one sequence, but for a block over a boundary: sequence after sequence then, the other's
+  // queries seeing nothing
+  for (int seg = t0; seg < t1;) {
+    const int seq = tok_seq[seg];
+    int end = seg + 1;
+    while (end < t1 && tok_seq[end] == seq) ++end;
+    const int32_t* pages = block_table + (size_t)seq * bt_stride;
+    const int hi = tok_pos[end - 1], lo = first_visible(tok_pos[seg], window, chunk);
+    const bool mine = t >= seg && t < end;
+    const int lo_unit = lo / 32;
+    const int kept = keep_first > 0 ? (keep_first + 31) / 32 : 0;
+    const int n_first = kept < lo_unit ? kept : lo_unit;
+    const int n_walk = n_first + hi / 32 - lo_unit + 1;
+    for (int walk = wave; walk < n_walk; walk += n_waves) {
+      const int key0 = 32 * (walk < n_first ? walk : lo_unit + walk - n_first);
+      const size_t base = ((size_t)pages[key0 / RB_PAGE] * n_kv + kvh) * RB_PAGE * head_dim + (size_t)(key0 % RB_PAGE) * head_dim;
+      // keys behind the last one are not written yet: the last one's numbers stand in for them, with weight 0
+      f32x4_t kf[2][NB];
+      float vf[2][4][NB];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int kr = (key0 + 16 * b + col < hi ? key0 + 16 * b + col : hi) - key0;
+        const float* krow = k_pages + base + (size_t)kr * head_dim + 4 * g;
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+          kf[b][c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+          if (16 * c + 4 * g < head_dim) kf[b][c] = *reinterpret_cast<const f32x4_t*>(krow + 16 * c);
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = key0 + 16 * b + 4 * g + i;
+          const float* vrow = v_pages + base + (size_t)((key < hi ? key : hi) - key0) * head_dim + NB * col;
+#pragma unroll
+          for (int d = 0; d < NB; d += VW) {
+            if (NB * col + d < head_dim) {
+              if (VW == 4) *reinterpret_cast<f32x4_t*>(&vf[b][i][d]) = *reinterpret_cast<const f32x4_t*>(vrow + d);
+              else *reinterpret_cast<float2*>(&vf[b][i][d]) = *reinterpret_cast<const float2*>(vrow + d);
+            } else {
+#pragma unroll
+              for (int e = 0; e < VW; ++e) vf[b][i][d + e] = 0.f;
+            }
+          }
+        }
+      f32x4_t sc[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        sc[b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][c][i], qv[c][i], sc[b], 0, 0, 0);
+      }
+      float top = -INFINITY;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = key0 + 16 * b + 4 * g + i;
+          float s = sc[b][i] * scale;
+          if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+          s = mine && key <= my_pos && (key >= my_lo || key < keep_first) ? s : -INFINITY;
+          sc[b][i] = s;
+          top = fmaxf(top, s);
+        }
+      top = fmaxf(top, __shfl_xor(top, 16, RB_WAVE));
+      top = fmaxf(top, __shfl_xor(top, 32, RB_WAVE));
+      const float m_new = sig_bias ? 0.f : fmaxf(m_run, top);
+      const float corr = m_run == -INFINITY ? 0.f : expf(m_run - m_new);      // nothing seen yet: nothing to rescale
+      m_run = m_new;
+      l_run *= corr;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float s = sc[b][i];
+          const float p = s == -INFINITY ? 0.f : (sig_bias ? 1.0f / (1.0f + expf(-(s + sb))) : expf(s - m_new));
+          l_run += p;
+          sc[b][i] = p;
+        }
+#pragma unroll
+      for (int d = 0; d < NB; ++d) acc[d] *= corr;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int d = 0; d < NB; ++d) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][i][d], sc[b][i], acc[d], 0, 0, 0);
+    }
+    seg = end;
+  }
+  l_run += __shfl_xor(l_run, 16, RB_WAVE);
+  l_run += __shfl_xor(l_run, 32, RB_WAVE);
+
+  // lane holds, for query col, the numbers NB (4 g + j) + d of the head
+  if (n_waves == 1) {
+    if (!on) return;
+    if (sinks) l_run += expf(sinks[h] - m_run);
+    const float inv = sig_bias ? 1.0f : (l_run > 0.f ? 1.0f / l_run : 0.f);
+    float* orow = out + ((size_t)t * n_heads + h) * head_dim;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int d = 0; d < NB; ++d) {
+        const int at = NB * (4 * g + j) + d;
+        if (at < head_dim) orow[at] = acc[d][j] * inv;
+      }
+    return;
+  }
+  float* row = merged + ((size_t)wave * 16 + col) * LD;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int d = 0; d < NB; ++d) row[NB * (4 * g + j) + d] = acc[d][j];
+  if (g == 0) {
+    row[16 * NB] = m_run;
+    row[16 * NB + 1] = l_run;
+  }
+  __syncthreads();
+  // every thread finishes a few numbers of a query: the waves' sums under their common maximum, in the order of the waves
+  const int queries = (t1 - t0) * h_count;
+  for (int idx = threadIdx.x; idx < queries * head_dim; idx += blockDim.x) {
+    const int cc = idx / head_dim, d = idx - cc * head_dim;
+    const int hh = h0 + cc % h_count;
+    const float* src = merged + (size_t)cc * LD;
+    float mx = -INFINITY;
+    for (int w = 0; w < n_waves; ++w) mx = fmaxf(mx, src[(size_t)w * 16 * LD + 16 * NB]);
+    float l = 0.f, o = 0.f;
+    for (int w = 0; w < n_waves; ++w) {
+      const float mw = src[(size_t)w * 16 * LD + 16 * NB];
+      const float f = mw == -INFINITY ? 0.f : expf(mw - mx);
+      l += src[(size_t)w * 16 * LD + 16 * NB + 1] * f;
+      o += src[(size_t)w * 16 * LD + d] * f;
+    }
+    if (sinks) l += expf(sinks[hh] - mx);
+    const float inv = sig_bias ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
+    out[((size_t)(t0 + cc / h_count) * n_heads + hh) * head_dim + d] = o * inv;
+  }
+}
+
+struct AttentionF32 {
+  const float *q, *k_pages, *v_pages;
+  float* out;
+  const int32_t *tok_pos, *tok_seq, *block_table;
+  int bt_stride, n_tokens, n_heads, n_kv, head_dim;
+  float scale;
+  int window;
+  const float* sinks;
+  int keep_first;
+  float softcap;
+  int chunk;
+  const float* sig_bias;
+};
+
+template <int NB>
+static int launch_attention_f32(const AttentionF32& a, hipStream_t s) {
+  const int group = a.n_heads / a.n_kv, chunks = (group + 15) / 16;
+  // One token a block while that leaves the GPU room (single-token steps above all: a block of tokens of several sequences takes
+  // them one after another), as many as the 16 columns hold beyond.
+  const long long cus = rb_compute_units();
+  const int per_block = (long long)a.n_tokens * a.n_kv * chunks >= 4 * cus && group < 16 ? 16 / group : 1;
+  const long long blocks = ((long long)a.n_tokens + per_block - 1) / per_block;
+  int n_waves = 1;
+  while (n_waves < AG_MAX_WAVES && blocks * a.n_kv * chunks * n_waves < 8 * cus) n_waves *= 2;
+  RB_REQUIRE((long long)a.n_kv * chunks <= 65535, "rb_attention_generic: too many heads %d", a.n_heads);
+  const size_t lds = n_waves > 1 ? (size_t)n_waves * 16 * (16 * NB + 4) * sizeof(float) : 0;
+  auto kern = attention_f32_mfma_kernel<NB>;
+  static bool configured = false;
+  if (!configured) {
+    const size_t most = (size_t)AG_MAX_WAVES * 16 * (16 * NB + 4) * sizeof(float);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
+    RB_REQUIRE(e == hipSuccess, "rb_attention_generic: cannot reserve %zu bytes of LDS: %s", most, hipGetErrorString(e));
+    configured = true;
+  }
+  kern<<<dim3((unsigned)blocks, (unsigned)(a.n_kv * chunks)), RB_WAVE * n_waves, lds, s>>>(
+      a.q, a.k_pages, a.v_pages, a.out, a.tok_pos, a.tok_seq, a.block_table, a.bt_stride, a.n_tokens, a.n_heads, a.n_kv, a.head_dim,
+      a.scale, a.window, a.sinks, a.keep_first, a.softcap, a.chunk, a.sig_bias, per_block, chunks);
+  return 0;
+}
+
 static int g_attention_vec = 1;
-extern "C" void rb_tune_attention_vec(int on) { g_attention_vec = on; }      // experiments and tests: 0 = the scalar kernel for every head size
+extern "C" void rb_tune_attention_vec(int on) { g_attention_vec = on; }      // experiments and tests: 0 = the scalar kernel for every head size, 2 = not the float32 matrix cores
 
 extern "C" int rb_attention_generic(const void* q, const void* k_pages, const void* v_pages, void* out, int dtype,
                                     const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* block_table,
@@ -338,6 +568,15 @@ extern "C" int rb_attention_generic_chunked(const void* q, const void* k_pages, 
   RB_REQUIRE(window >= 0, "rb_attention_generic: negative window");
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
+  const bool wide = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) & 15) == 0;
+  if (dtype == RB_F32 && head_dim % 4 == 0 && head_dim <= 128 && wide && g_attention_vec == 1) {
+    const AttentionF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, (float*)out, tok_pos, tok_seq, block_table,
+                            bt_stride, n_tokens, n_heads, n_kv_heads, head_dim, scale, window, sinks, keep_first, softcap, chunk, sig_bias};
+    const int rc = head_dim <= 32 ? launch_attention_f32<2>(a, s) : head_dim <= 64 ? launch_attention_f32<4>(a, s) : launch_attention_f32<8>(a, s);
+    if (rc) return rc;
+    RB_LAUNCH_CHECK();
+    return 0;
+  }
   dim3 grid(n_tokens, n_heads);
   // waves per (token, head): enough to give every SIMD of the GPU two waves, at most 8
   int n_waves = 1;

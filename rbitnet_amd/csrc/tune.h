@@ -17,7 +17,7 @@ void rb_tune_f32_tile(int tile);                                // float32 produ
 void rb_tune_use_stream(int on);                                // 0: the skinny product up to 64 tokens
 void rb_tune_tiles(int cfg, int parts);                         // tiled product: tile configuration and K slices
 int rb_tune_plan(int m, int n, int k, int epilogue);            // tiled product: the built-in choice, 100 * cfg + parts
-void rb_tune_attention_vec(int on);                             // generic attention: 0 = the scalar kernel also for head sizes that are multiples of 4
+void rb_tune_attention_vec(int on);                             // generic attention: 0 = the scalar kernel also for head sizes that are multiples of 4, 2 = the vector units for float32 too
 void rb_tune_prefill_waves(int waves);                          // prefill attention: 4 or 8
 void rb_tune_prefill_paired(int on);                           // prefill attention: 0 = late blocks first only, no pairing of heavy and light workgroups
 void rb_tune_decode_mfma(int mode);                             // decode attention: 1 matrix cores, 2 vector units

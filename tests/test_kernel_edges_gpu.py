@@ -49,3 +49,81 @@ def test_float32_tiles_of_operands_at_odd_addresses(lib, m, n, k):
     c = torch.full((m, n), float("nan"), device=DEV)
     lib.gemm_generic(a, w, c)
     _within(c, a.double() @ w.double().T, k * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T))
+
+
+# ---------------------------------------------------------------- float32 attention on the matrix cores
+def _paged(lengths, heads, dim, generator, spare=7):
+    """Keys (or values) of sequences of these lengths in pages that are handed out in a mixed order, NaN where nothing was written."""
+    need = [(n + 63) // 64 for n in lengths]
+    order = torch.randperm(sum(need) + spare, generator=generator).tolist()
+    pages = torch.full((sum(need) + spare, heads, 64, dim), float("nan"))
+    rows, at = [], 0
+    table = torch.zeros(len(lengths), max(need), dtype=torch.int32)
+    for b, n in enumerate(lengths):
+        mine = order[at:at + need[b]]
+        at += need[b]
+        table[b, :need[b]] = torch.tensor(mine, dtype=torch.int32)
+        x = torch.randn(n, heads, dim, generator=generator)
+        for j in range(n):
+            pages[mine[j // 64], :, j % 64] = x[j]
+        rows.append(x)
+    return pages, table, rows
+
+
+def _attention64(q, k, v, pos, scale, window=0, keep=0, cap=0.0, sinks=None, chunk=0, sig=None):
+    """q [T, H, D] at positions pos [T] over k, v [N, G, D] in float64."""
+    t, h, _ = q.shape
+    rep = h // k.shape[1]
+    s = torch.einsum("thd,nhd->htn", q.double(), k.double().repeat_interleave(rep, 1)) * scale
+    if cap > 0:
+        s = cap * torch.tanh(s / cap)
+    i, j = pos[:, None], torch.arange(k.shape[0])[None, :]
+    seen = j <= i
+    if window:
+        seen = seen & ((i - j < window) | (j < keep))
+    if chunk:
+        seen = seen & (i // chunk == j // chunk)
+    if sig is not None:
+        w = torch.sigmoid(s + sig.double()[:, None, None]) * seen
+    else:
+        s = s.masked_fill(~seen, float("-inf"))
+        top = s.amax(-1, keepdim=True)
+        if sinks is not None:
+            top = torch.maximum(top, sinks.double()[:, None, None])
+        w = torch.exp(s - top)
+        w = w / (w.sum(-1, keepdim=True) + (0 if sinks is None else torch.exp(sinks.double()[:, None, None] - top)))
+    return torch.einsum("htn,nhd->thd", w, v.double().repeat_interleave(rep, 1))
+
+
+@pytest.mark.parametrize("heads,kv,dim", [(4, 1, 24), (3, 3, 4), (24, 8, 128), (16, 1, 64), (40, 2, 100), (6, 2, 32)])
+@pytest.mark.parametrize("past,new", [([0], [1]), ([62, 0, 130, 31], [1, 1, 1, 1]), ([0, 0, 0], [5, 17, 77]), ([40, 129], [70, 3]),
+                                      ([0, 500], [600, 1])])
+@pytest.mark.parametrize("more", [{}, {"window": 50, "keep": 9, "cap": 3.0}, {"sinks": True, "chunk": 48}, {"sig": True, "chunk": 64}])
+def test_float32_attention(lib, heads, kv, dim, past, new, more):
+    g = torch.Generator().manual_seed(heads * 7 + dim + len(past) + sum(new))
+    more = dict(more)
+    lengths = [p + n for p, n in zip(past, new)]
+    kp, table, ks = _paged(lengths, kv, dim, g)
+    vp, vs = torch.full_like(kp, float("nan")), []
+    for b, n in enumerate(lengths):
+        x = torch.randn(n, kv, dim, generator=g)
+        for j in range(n):
+            vp[table[b, j // 64], :, j % 64] = x[j]
+        vs.append(x)
+    q = torch.randn(sum(new), heads, dim, generator=g)
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip(past, new)])
+    seq = torch.repeat_interleave(torch.arange(len(new)), torch.tensor(new))
+    for name in ("sinks", "sig"):
+        if more.get(name):
+            more[name] = torch.randn(heads, generator=g)
+    scale = dim ** -0.5
+    want = torch.cat([_attention64(q[seq == b], ks[b], vs[b], pos[seq == b], scale, **more) for b in range(len(new))])
+    out = torch.full((sum(new), heads * dim), float("nan"), device=DEV)
+    i32 = lambda x: x.to(torch.int32).to(DEV)
+    dev = lambda x: None if x is None else x.to(DEV)
+    lib.attention_opts(q.to(DEV), kp.to(DEV), vp.to(DEV), out, i32(pos), i32(seq), table.to(DEV), heads, kv, dim, scale,
+                       more.get("window", 0), more.get("keep", 0), more.get("cap", 0.0), dev(more.get("sinks")), more.get("chunk", 0),
+                       dev(more.get("sig")))
+    # scores are sums of `dim` products of a few units: their error, at most dim 2^-24 of the sum of absolute products, moves a
+    # weight by as much relatively, and the outputs are sums of weights times values of a few units
+    _within(out.view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
