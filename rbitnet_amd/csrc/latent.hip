@@ -8,6 +8,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "mfma.h"
 
 // proj [T, stride] float32 holds, per token, q_rank numbers at column 0 and kv_rank numbers at column kv_col.
 // cq[t] = rmsnorm(proj[t, 0:q_rank]) * q_gain; c = rmsnorm(proj[t, kv_col:kv_col + kv_rank]) * kv_gain goes into the
@@ -21,15 +22,17 @@ __global__ void latent_norm_store_kernel(const float* __restrict__ proj, size_t 
                                          int rot = 0, const float* __restrict__ cos_t = nullptr,
                                          const float* __restrict__ sin_t = nullptr, int style = 0) {
   __shared__ float scratch[16];
+  // the two norms are two workgroups of a token: one behind the other they were a chain of four trips to memory (four tokens,
+  // ranks of 768 and 96: 6.0 -> 4.2 us)
   const int t = blockIdx.x;
   const float* row = proj + (size_t)t * stride;
-  if (q_rank > 0) {
+  if (q_rank > 0 && blockIdx.y == 0) {
     float ss = 0.f;
     for (int j = threadIdx.x; j < q_rank; j += blockDim.x) ss = fmaf(row[j], row[j], ss);
     const float f = 1.0f / sqrtf(block_sum(ss, scratch) / (float)q_rank + eps);
     for (int j = threadIdx.x; j < q_rank; j += blockDim.x) Num<TC>::store(cq + (size_t)t * q_rank + j, row[j] * f * q_gain[j]);
   }
-  if (kv_rank > 0) {
+  if (kv_rank > 0 && blockIdx.y == gridDim.y - 1) {
     const int pos = tok_pos[t];
     const int page = block_table[(size_t)tok_seq[t] * bt_stride + pos / RB_PAGE];
     TC* dst = pages + ((size_t)page * RB_PAGE + (size_t)(pos % RB_PAGE)) * page_width;
@@ -69,15 +72,40 @@ extern "C" int rb_latent_norm_store(const float* proj, long long stride, int q_r
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == RB_F32)
-    latent_norm_store_kernel<float><<<n_tokens, 256, 0, s>>>(proj, (size_t)stride, q_rank, q_gain, (float*)cq, kv_col, kv_rank,
+    latent_norm_store_kernel<float><<<dim3(n_tokens, q_rank > 0 && kv_rank > 0 ? 2 : 1), 256, 0, s>>>(proj, (size_t)stride, q_rank, q_gain, (float*)cq, kv_col, kv_rank,
                                                              kv_gain, (float*)pages, kv_rank, tok_pos, tok_seq, block_table, bt_stride, eps);
   else if (dtype == RB_BF16)
-    latent_norm_store_kernel<bf16_t><<<n_tokens, 256, 0, s>>>(proj, (size_t)stride, q_rank, q_gain, (bf16_t*)cq, kv_col, kv_rank,
+    latent_norm_store_kernel<bf16_t><<<dim3(n_tokens, q_rank > 0 && kv_rank > 0 ? 2 : 1), 256, 0, s>>>(proj, (size_t)stride, q_rank, q_gain, (bf16_t*)cq, kv_col, kv_rank,
                                                               kv_gain, (bf16_t*)pages, kv_rank, tok_pos, tok_seq, block_table, bt_stride, eps);
   else
     RB_REQUIRE(false, "rb_latent_norm_store: unknown dtype %d", dtype);
   RB_LAUNCH_CHECK();
   return 0;
+}
+
+// The `rot` numbers at x_rot_col of head h of the tokens t0.., rotated by the tokens' positions, go to y at y_rot_col, and what lies
+// behind them in the head of y becomes zero.
+template <typename TX, typename TY>
+__device__ __forceinline__ void heads_rotated_part(const TX* __restrict__ x, TY* __restrict__ y, int t0, int nt, int h, int n_heads,
+                                                   size_t x_hs, size_t y_hs, int rot, int x_rot_col, int y_rot_col,
+                                                   const float* __restrict__ cos_t, const float* __restrict__ sin_t, int style,
+                                                   const int32_t* __restrict__ tok_pos) {
+  const int half = rot / 2, tail = (int)y_hs - y_rot_col - rot, per = half + tail;
+  for (int idx = threadIdx.x; idx < nt * per; idx += blockDim.x) {
+    const int tt = idx / per, i = idx - tt * per;
+    const TX* src = x + ((size_t)(t0 + tt) * n_heads + h) * x_hs + x_rot_col;
+    TY* dst = y + ((size_t)(t0 + tt) * n_heads + h) * y_hs + y_rot_col;
+    if (i < half) {
+      const size_t at = (size_t)tok_pos[t0 + tt] * half + i;
+      const int a = style == 0 ? 2 * i : i, b = style == 0 ? 2 * i + 1 : i + half;
+      float y0, y1;
+      rotate_pair(Num<TX>::load(src + a), Num<TX>::load(src + b), cos_t[at], sin_t[at], y0, y1);
+      Num<TY>::store(dst + a, y0);
+      Num<TY>::store(dst + b, y1);
+    } else {
+      Num<TY>::store(dst + rot + (i - half), 0.f);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- a product per head
@@ -102,24 +130,8 @@ __global__ __launch_bounds__(RB_WAVE * HL_WAVES) void heads_linear_kernel(const 
   const int lane = threadIdx.x & (RB_WAVE - 1), wave = threadIdx.x / RB_WAVE;
   const int nt = n_tokens - t0 < HL_TOKENS ? n_tokens - t0 : HL_TOKENS;
   if ((int)blockIdx.z == n_col_tiles) {
-    // one more workgroup per (tokens, head): the `rot` numbers at x_rot_col of the head, rotated by the token's position, go to
-    // y at y_rot_col, and what lies behind them in the head of y becomes zero
-    const int half = rot / 2, tail = (int)y_hs - y_rot_col - rot, per = half + tail;
-    for (int idx = threadIdx.x; idx < nt * per; idx += blockDim.x) {
-      const int tt = idx / per, i = idx - tt * per;
-      const TX* src = x + ((size_t)(t0 + tt) * n_heads + h) * x_hs + x_rot_col;
-      TY* dst = y + ((size_t)(t0 + tt) * n_heads + h) * y_hs + y_rot_col;
-      if (i < half) {
-        const size_t at = (size_t)tok_pos[t0 + tt] * half + i;
-        const int a = style == 0 ? 2 * i : i, b = style == 0 ? 2 * i + 1 : i + half;
-        float y0, y1;
-        rotate_pair(Num<TX>::load(src + a), Num<TX>::load(src + b), cos_t[at], sin_t[at], y0, y1);
-        Num<TY>::store(dst + a, y0);
-        Num<TY>::store(dst + b, y1);
-      } else {
-        Num<TY>::store(dst + rot + (i - half), 0.f);
-      }
-    }
+    // one more workgroup per (tokens, head)
+    heads_rotated_part(x, y, t0, nt, h, n_heads, x_hs, y_hs, rot, x_rot_col, y_rot_col, cos_t, sin_t, style, tok_pos);
     return;
   }
   // the tokens' inputs, eight loads in flight per lane (a step of few tokens is a chain of trips to memory otherwise)
@@ -199,6 +211,119 @@ static void launch_heads_linear(const void* x, const void* w, void* y, int n_tok
                                                                         m.cos_t, m.sin_t, m.style, m.tok_pos, n_col_tiles);
 }
 
+// The same products on the matrix cores: bfloat16 weights, fragment-major per head ([H][N / 16][K / 32] blocks of 1 KB, see
+// gemm_internal.h), K a multiple of 32 up to 128, N of 16.  A wave takes 16 tokens of one head, holds their inputs as operands, and
+// walks `tiles` of the head's blocks of 16 outputs, so that all of a wave's loads are on their way at once: the vector kernel above
+// was a chain of three trips to memory in single-token steps, and a lane a column could not keep up with prompts.  Float32 inputs
+// go in as three bfloat16 numbers each (the 24 bits of the significand cut in three, x = hi + mid + lo without a remainder), so that
+// every product is exact and is summed in float32, as in the vector kernel.  Measured, 16 heads of 128 by 128:
+// four tokens 9.7 -> 3.7 us from float32 and 4.5 from bfloat16, 3,782 tokens 82 -> 18 and 16; 32 heads of 64 by 96 with a rotated part,
+// 3,782 tokens 93 -> 31.
+template <typename TX>
+struct HeadInput;
+template <>
+struct HeadInput<bf16_t> {
+  static constexpr int PARTS = 1;
+  static __device__ __forceinline__ void load(const bf16_t* p, Frag8 (&out)[1]) { out[0].u = load16(p); }
+};
+template <>
+struct HeadInput<float> {
+  static constexpr int PARTS = 3;
+  static __device__ __forceinline__ void cut(float v, uint32_t (&part)[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      part[i] = __float_as_uint(v) >> 16;
+      // an infinity or a NaN has no remainder
+      v = (part[i] & 0x7f80u) == 0x7f80u ? 0.f : v - __uint_as_float(part[i] << 16);
+    }
+  }
+  static __device__ __forceinline__ void load(const float* p, Frag8 (&out)[3]) {
+    const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    uint32_t w[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t lo[3], hi[3];
+      cut(v[2 * i], lo);
+      cut(v[2 * i + 1], hi);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[q][i] = lo[q] | (hi[q] << 16);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) out[q].u = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
+  }
+};
+
+template <typename TX, typename TY, int KS>
+__global__ __launch_bounds__(256) void heads_mfma_kernel(const TX* __restrict__ x, const bf16_t* __restrict__ w, TY* __restrict__ y,
+                                                         int n_tokens, int n_heads, int n, size_t x_hs, size_t y_hs,
+                                                         const float* __restrict__ gate, size_t gate_stride, int rot, int x_rot_col,
+                                                         int y_rot_col, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+                                                         int style, const int32_t* __restrict__ tok_pos, int tiles) {
+  const int h = blockIdx.y;
+  if (blockIdx.z == 1) {
+    for (int t0 = blockIdx.x * 16; t0 < n_tokens; t0 += gridDim.x * 16)
+      heads_rotated_part(x, y, t0, n_tokens - t0 < 16 ? n_tokens - t0 : 16, h, n_heads, x_hs, y_hs, rot, x_rot_col, y_rot_col, cos_t, sin_t,
+                         style, tok_pos);
+    return;
+  }
+  const int lane = threadIdx.x & (RB_WAVE - 1), r = lane & 15, kq = lane >> 4;
+  const int id = blockIdx.x * (blockDim.x / RB_WAVE) + threadIdx.x / RB_WAVE;
+  const int n_tiles = n / 16, groups = (n_tiles + tiles - 1) / tiles;
+  const int t0 = id / groups * 16, first = id % groups * tiles;
+  if (t0 >= n_tokens) return;
+  const int last = first + tiles < n_tiles ? first + tiles : n_tiles;
+  const bf16_t* wt = w + ((size_t)h * n_tiles + first) * (KS * 512) + 8 * lane;
+  const int t = t0 + r < n_tokens ? t0 + r : n_tokens - 1;      // a token behind the last: the last one's numbers, never stored
+  Frag8 a[KS], b[KS][HeadInput<TX>::PARTS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) a[ks].u = load16(wt + 512 * ks);
+  const TX* xr = x + ((size_t)t * n_heads + h) * x_hs + 8 * kq;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) HeadInput<TX>::load(xr + 32 * ks, b[ks]);
+  const float g = gate ? 1.0f / (1.0f + expf(-gate[(size_t)t * gate_stride + h])) : 1.0f;      // a gate per head on the way out
+  TY* yr = y + ((size_t)t * n_heads + h) * y_hs + 4 * kq;
+  for (int tile = first; tile < last; ++tile) {
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = HeadInput<TX>::PARTS - 1; q >= 0; --q)         // the smallest parts first
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) acc = mfma16(a[ks], b[ks][q], acc);
+    if (tile + 1 < last) {
+      wt += KS * 512;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) a[ks].u = load16(wt + 512 * ks);
+    }
+    acc *= g;
+    if (t0 + r < n_tokens) {
+      if constexpr (sizeof(TY) == 2)
+        *reinterpret_cast<uint2*>(yr + 16 * tile) = make_uint2(pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]));
+      else
+        *reinterpret_cast<f32x4_t*>(yr + 16 * tile) = acc;
+    }
+  }
+}
+
+template <typename TX, typename TY>
+static void launch_heads_mfma(const void* x, const void* w, void* y, int n_tokens, int n_heads, int n, int k, size_t x_hs, size_t y_hs,
+                              hipStream_t s, const HeadsLinearMore& m) {
+  // single-token steps: a wave per 16 outputs; prompts: a wave per 16 tokens, while that gives every SIMD of the GPU a few
+  const long long token_tiles = ((long long)n_tokens + 15) / 16, n_tiles = n / 16;
+  int tiles = 1;
+  while (tiles < n_tiles && token_tiles * n_heads * ((n_tiles + tiles - 1) / tiles) > 16LL * rb_compute_units()) tiles *= 2;
+  const long long waves = token_tiles * ((n_tiles + tiles - 1) / tiles);
+  const dim3 grid((unsigned)((waves + 3) / 4), n_heads, m.has_rot ? 2 : 1);
+#define HM_GO(KS)                                                                                                                  \
+  heads_mfma_kernel<TX, TY, KS><<<grid, 256, 0, s>>>((const TX*)x, (const bf16_t*)w, (TY*)y, n_tokens, n_heads, n, x_hs, y_hs, m.gate, \
+                                                     m.gate_stride, m.rot, m.x_rot_col, m.y_rot_col, m.cos_t, m.sin_t, m.style,    \
+                                                     m.tok_pos, tiles)
+  if (k == 32) HM_GO(1);
+  else if (k == 64) HM_GO(2);
+  else if (k == 96) HM_GO(3);
+  else HM_GO(4);
+#undef HM_GO
+}
+
 extern "C" int rb_heads_linear(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype, int n_tokens,
                                int n_heads, int n, int k, void* stream) {
   RB_RECORDED(rb_heads_linear(x, x_dtype, w, w_dtype, y, y_dtype, n_tokens, n_heads, n, k, stream));
@@ -211,19 +336,20 @@ extern "C" int rb_heads_linear_strided(const void* x, int x_dtype, long long x_h
                                        int y_dtype, long long y_head_stride, int n_tokens, int n_heads, int n, int k, void* stream) {
   RB_RECORDED(rb_heads_linear_strided(x, x_dtype, x_head_stride, w, w_dtype, y, y_dtype, y_head_stride, n_tokens, n_heads, n, k,
                                       stream));
-  return rb_heads_linear_more(x, x_dtype, x_head_stride, w, w_dtype, y, y_dtype, y_head_stride, n_tokens, n_heads, n, k, nullptr, 0,
+  return rb_heads_linear_more(x, x_dtype, x_head_stride, w, w_dtype, 0, y, y_dtype, y_head_stride, n_tokens, n_heads, n, k, nullptr, 0,
                               -1, 0, 0, nullptr, nullptr, 0, nullptr, stream);
 }
 
 // The same with two things in the same launch.  gate (float32, rows gate_stride apart; null: none): head h's outputs of token t
 // are multiplied by sigmoid(gate[t * gate_stride + h]).  rot >= 0 (rot < 0: none): the `rot` numbers at x_rot_col of every head
 // of x, rotated by the token's position (cos, sin [positions, rot / 2]; style 0: 2i with 2i + 1, 1: i with i + rot / 2), go to
-// y at y_rot_col, and what lies behind them in a head of y becomes zero.
-extern "C" int rb_heads_linear_more(const void* x, int x_dtype, long long x_head_stride, const void* w, int w_dtype, void* y,
+// y at y_rot_col, and what lies behind them in a head of y becomes zero.  w_layout 1: every head's [N, K] fragment-major (bfloat16, K 32,
+// 64, 96 or 128, N a multiple of 16, x and y and their heads on 16-byte boundaries): the matrix cores' kernel.
+extern "C" int rb_heads_linear_more(const void* x, int x_dtype, long long x_head_stride, const void* w, int w_dtype, int w_layout, void* y,
                                     int y_dtype, long long y_head_stride, int n_tokens, int n_heads, int n, int k, const float* gate,
                                     long long gate_stride, int rot, int x_rot_col, int y_rot_col, const float* cos, const float* sin,
                                     int style, const int32_t* tok_pos, void* stream) {
-  RB_RECORDED(rb_heads_linear_more(x, x_dtype, x_head_stride, w, w_dtype, y, y_dtype, y_head_stride, n_tokens, n_heads, n, k, gate,
+  RB_RECORDED(rb_heads_linear_more(x, x_dtype, x_head_stride, w, w_dtype, w_layout, y, y_dtype, y_head_stride, n_tokens, n_heads, n, k, gate,
                                    gate_stride, rot, x_rot_col, y_rot_col, cos, sin, style, tok_pos, stream));
   HeadsLinearMore more;
   more.gate = gate;
@@ -249,6 +375,19 @@ extern "C" int rb_heads_linear_more(const void* x, int x_dtype, long long x_head
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const size_t xs = (size_t)x_head_stride, ys = (size_t)y_head_stride;
+  if (w_layout == 1) {
+    const long long x_size = x_dtype == RB_F32 ? 4 : 2, y_size = y_dtype == RB_F32 ? 4 : 2;
+    RB_REQUIRE(w_dtype == RB_BF16 && k % 32 == 0 && k <= 128 && n % 16 == 0, "rb_heads_linear: fragment-major weights of %d x %d", n, k);
+    RB_REQUIRE(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y)) & 15) == 0 &&
+                   x_head_stride * x_size % 16 == 0 && y_head_stride * y_size % 16 == 0,
+               "rb_heads_linear: the matrix cores' kernel needs heads on 16-byte boundaries");
+    if (x_dtype == RB_F32 && y_dtype == RB_BF16) launch_heads_mfma<float, bf16_t>(x, w, y, n_tokens, n_heads, n, k, xs, ys, s, more);
+    else if (x_dtype == RB_BF16 && y_dtype == RB_BF16) launch_heads_mfma<bf16_t, bf16_t>(x, w, y, n_tokens, n_heads, n, k, xs, ys, s, more);
+    else RB_REQUIRE(false, "rb_heads_linear: this combination of types is not built fragment-major (x %d, y %d)", x_dtype, y_dtype);
+    RB_LAUNCH_CHECK();
+    return 0;
+  }
+  RB_REQUIRE(w_layout == 0, "rb_heads_linear: unknown layout %d", w_layout);
   const int key = x_dtype * 4 + w_dtype * 2 + y_dtype;
   switch (key) {
     case 0: launch_heads_linear<float, float, float>(x, w, y, n_tokens, n_heads, n, k, xs, ys, s, more); break;
@@ -287,11 +426,11 @@ extern "C" int rb_latent_norm_rope_store(const float* proj, long long stride, in
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == RB_F32)
-    latent_norm_store_kernel<float><<<n_tokens, 256, 0, s>>>(proj, (size_t)stride, q_rank, q_gain, (float*)cq, kv_col, kv_rank,
+    latent_norm_store_kernel<float><<<dim3(n_tokens, q_rank > 0 && kv_rank > 0 ? 2 : 1), 256, 0, s>>>(proj, (size_t)stride, q_rank, q_gain, (float*)cq, kv_col, kv_rank,
                                                              kv_gain, (float*)pages, page_width, tok_pos, tok_seq, block_table,
                                                              bt_stride, eps, rot_col, rot, cos, sin, style);
   else
-    latent_norm_store_kernel<bf16_t><<<n_tokens, 256, 0, s>>>(proj, (size_t)stride, q_rank, q_gain, (bf16_t*)cq, kv_col, kv_rank,
+    latent_norm_store_kernel<bf16_t><<<dim3(n_tokens, q_rank > 0 && kv_rank > 0 ? 2 : 1), 256, 0, s>>>(proj, (size_t)stride, q_rank, q_gain, (bf16_t*)cq, kv_col, kv_rank,
                                                               kv_gain, (bf16_t*)pages, page_width, tok_pos, tok_seq, block_table,
                                                               bt_stride, eps, rot_col, rot, cos, sin, style);
   RB_LAUNCH_CHECK();

@@ -204,7 +204,7 @@ class Kernels:
             "rb_short_conv_bias": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
             "rb_linear_recurrence_bonus": [_P, _P, _L, _P, _L, _P, _L, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
             "rb_gated_rmsnorm_heads": [_P, _P, _L, _P, _L, _I, _F, _P, _I, _I, _I, _I, _P],
-            "rb_heads_linear_more": [_P, _I, _L, _P, _I, _P, _I, _L, _I, _I, _I, _I, _P, _L, _I, _I, _I, _P, _P, _I, _P, _P],
+            "rb_heads_linear_more": [_P, _I, _L, _P, _I, _I, _P, _I, _L, _I, _I, _I, _I, _P, _L, _I, _I, _I, _P, _P, _I, _P, _P],
             "rb_heads_linear_strided": [_P, _I, _L, _P, _I, _P, _I, _L, _I, _I, _I, _I, _P],
             "rb_latent_norm_rope_store": [_P, _L, _I, _P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _P, _I, _I, _P, _P, _P, _I, _F, _I, _P],
             "rb_attention_generic_chunked": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _F, _P, _I, _P, _P],
@@ -1344,12 +1344,20 @@ class Kernels:
         self._ok(self._lib.rb_gated_rmsnorm_heads(_ptr(o), _ptr(weight), vdim, _ptr(gate), n_heads * vdim, int(act), float(eps),
                                                   _ptr(out), dtype_code(out.dtype), n, n_heads, vdim, self._stream()))
 
+    @staticmethod
+    def heads_frag_ok(dtype: torch.dtype, n_out: int, k: int, x_head: int, y_head: int) -> bool:
+        """Whether a product per head of these sizes runs on the matrix cores, its weights stored fragment-major."""
+        return dtype == torch.bfloat16 and k % 32 == 0 and k <= 128 and n_out % 16 == 0 and x_head % 8 == 0 and y_head % 8 == 0
+
     def heads_linear_part(self, x: torch.Tensor, x_head: int, w: torch.Tensor, y: torch.Tensor, y_head: int,
-                          gate: Optional[torch.Tensor] = None, gate_col: int = 0, rope=None) -> None:
-        """y[t, h, :N] = w[h]^T x[t, h, :K] with w [H, K, N]; a head of x takes x_head numbers, a head of y y_head.
+                          gate: Optional[torch.Tensor] = None, gate_col: int = 0, rope=None, w_frag: bool = False) -> None:
+        """y[t, h, :N] = w[h]^T x[t, h, :K] with w [H, K, N]; a head of x takes x_head numbers, a head of y y_head.  w_frag: w
+        [H, N, K], every head's matrix fragment-major (`place_rows(..., frag=True)`; see `heads_frag_ok`).
         gate [T, >= gate_col + H] float32: head h's outputs times sigmoid(gate[:, gate_col + h]).  rope = (x_col, rot, cos, sin,
         style, y_col, tok_pos): the rot numbers at x_col of every head of x, rotated, go to y at y_col, zeros behind them."""
         h, k, n_out = w.shape
+        if w_frag:
+            k, n_out = n_out, k
         n = x.shape[0]
         _check(x, "x", None, (n, h * x_head))
         _check(w, "w")
@@ -1373,7 +1381,7 @@ class Kernels:
                 _check(sin, "sin", torch.float32, cos.shape)
                 if cos.shape[1] != rot // 2:
                     raise KernelError("angle table width mismatch")
-        self._ok(self._lib.rb_heads_linear_more(_ptr(x), dtype_code(x.dtype), x_head, _ptr(w), dtype_code(w.dtype), _ptr(y),
+        self._ok(self._lib.rb_heads_linear_more(_ptr(x), dtype_code(x.dtype), x_head, _ptr(w), dtype_code(w.dtype), int(bool(w_frag)), _ptr(y),
                                                 dtype_code(y.dtype), y_head, n, h, n_out, k, g_ptr, g_stride, int(rot), int(x_col),
                                                 int(y_col), _ptr(cos) if rot > 0 else None, _ptr(sin) if rot > 0 else None, int(style),
                                                 _ptr(tok_pos), self._stream()))

@@ -123,9 +123,24 @@ class LatentAttention(Part):
         uq, o = tensors[n["uq"]], tensors[n["o"]]
         self.w_uq = pack_rows(lib, [(uq, 0, None, None)], uq.shape[0], uq.shape[1], uq.dtype, uq.device, allowed)
         self.w_o = pack_rows(lib, [(o, 0, None, None)], o.shape[0], o.shape[1], o.dtype, o.device, allowed)
-        # per head, stored [inner, outer]: Wuk_i [dim, rank] as it is (q_i -> Wuk_i^T q_i), Wuv_i transposed
+        # per head, stored [inner, outer]: Wuk_i [dim, rank] as it is (q_i -> Wuk_i^T q_i), Wuv_i transposed; for the matrix
+        # cores [outer, inner], fragment-major
         self.w_uk = tensors[n["uk"]].view(self.heads, self.dim, self.kv_rank).contiguous()
         self.w_uv = tensors[n["uv"]].view(self.heads, self.vdim, self.kv_rank).transpose(1, 2).contiguous()
+        self.uk_frag = allowed and lib.heads_frag_ok(first.dtype, self.kv_rank, self.dim, self.dim + self.rot, self.page_width)
+        self.uv_frag = allowed and lib.heads_frag_ok(first.dtype, self.vdim, self.kv_rank, self.page_width, self.vdim)
+
+        def fragments(w: torch.Tensor) -> torch.Tensor:
+            rows = w.transpose(1, 2).contiguous()
+            out = torch.empty_like(rows)
+            for i in range(self.heads):
+                lib.place_rows(rows[i], out[i], frag=True)
+            return out
+
+        if self.uk_frag:
+            self.w_uk = fragments(self.w_uk)
+        if self.uv_frag:
+            self.w_uv = fragments(self.w_uv)
         self.sink = tensors[n["sink"]] if self.has_sink else None
 
     def cache_request(self) -> Optional[CacheRequest]:
@@ -151,9 +166,9 @@ class LatentAttention(Part):
         if self.rot:
             # the queries in the cache's layout: the unrotated part in the latent's space, then the rotated part, then zeros
             lib.heads_linear_part(q, self.dim + self.rot, self.w_uk, ql, r,
-                                  rope=(self.dim, self.rot, cos, sin, style, self.kv_rank, ctx.tok_pos))
+                                  rope=(self.dim, self.rot, cos, sin, style, self.kv_rank, ctx.tok_pos), w_frag=self.uk_frag)
         else:
-            lib.heads_linear(q, self.w_uk, ql)                                # the queries in the latent's space
+            lib.heads_linear_part(q, self.dim, self.w_uk, ql, r, w_frag=self.uk_frag)      # the queries in the latent's space
         ol = torch.empty((t, self.heads * r), dtype=dt, device=h.device)
         q3, pages = ql.view(t, self.heads, r), view.k_pages
         fast = dt == torch.bfloat16 and r in _MATRIX_CORE_RANKS and not getattr(self.env, "generic_only", False)
@@ -169,7 +184,8 @@ class LatentAttention(Part):
                                 self.scale, None, self.sink)
         o = torch.empty((t, self.heads * self.vdim), dtype=dt, device=h.device)
         # the latent's part of every head's sum through the head's value matrix, the head's gate on the way out
-        lib.heads_linear_part(ol, r, self.w_uv, o, self.vdim, gate=down if self.has_gate else None, gate_col=self.gate_col)
+        lib.heads_linear_part(ol, r, self.w_uv, o, self.vdim, gate=down if self.has_gate else None, gate_col=self.gate_col,
+                              w_frag=self.uv_frag)
         return linear_to_stream(lib, o, self.w_o, None, next_norm)
 
 

@@ -127,3 +127,60 @@ def test_float32_attention(lib, heads, kv, dim, past, new, more):
     # scores are sums of `dim` products of a few units: their error, at most dim 2^-24 of the sum of absolute products, moves a
     # weight by as much relatively, and the outputs are sums of weights times values of a few units
     _within(out.view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
+
+
+# ---------------------------------------------------------------- products per head on the matrix cores
+@pytest.mark.parametrize("tokens", [1, 4, 16, 17, 200])
+@pytest.mark.parametrize("heads,k,n,more", [(1, 32, 16, {}), (3, 64, 96, {"rot": 32, "pad": 128}), (16, 128, 128, {}),
+                                            (5, 96, 64, {"gate": True, "wide": 128}), (2, 128, 48, {"gate": True})])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_products_per_head(lib, tokens, heads, k, n, more, dtype):
+    if dtype == torch.bfloat16 and "rot" in more:
+        pytest.skip("a rotated part rides with float32 inputs")
+    g = torch.Generator().manual_seed(tokens + heads + k)
+    rot, x_head, y_head = more.get("rot", 0), more.get("wide", k) + more.get("rot", 0), more.get("pad", n)
+    x = torch.randn(tokens, heads, x_head, generator=g).to(dtype)
+    w = torch.randn(heads, n, k, generator=g).bfloat16()
+    if dtype == torch.float32:                                    # a number whose rounding to bfloat16 would be an infinity
+        x[0, 0, 0], w[0, :, 0] = 3.4e38, w[0, :, 0] * 0.125
+    want = torch.einsum("thk,hnk->thn", x[..., :k].double(), w.double())
+    size = torch.einsum("thk,hnk->thn", x[..., :k].double().abs(), w.double().abs())
+    wf = torch.empty_like(w, device=DEV)
+    for i in range(heads):
+        lib.place_rows(w[i].to(DEV).contiguous(), wf[i], frag=True)
+    y = torch.full((tokens, heads * y_head), float("nan"), dtype=torch.bfloat16, device=DEV)
+    gate = torch.randn(tokens, heads + 3, generator=g)
+    pos = torch.randint(0, 50, (tokens,), generator=g, dtype=torch.int32)
+    angles = torch.rand(50, max(1, rot // 2), generator=g) * 6.0
+    cos, sin = torch.cos(angles), torch.sin(angles)
+    rope = (k, rot, cos.to(DEV), sin.to(DEV), 0, n, pos.to(DEV)) if rot else None
+    lib.heads_linear_part(x.reshape(tokens, -1).to(DEV), x_head, wf, y, y_head, gate=gate.to(DEV) if "gate" in more else None,
+                          gate_col=2, rope=rope, w_frag=True)
+    got = y.view(tokens, heads, y_head).double().cpu()
+    if "gate" in more:
+        factor = torch.sigmoid(gate[:, 2:2 + heads].double())[..., None]
+        want, size = want * factor, size * factor
+    # the output's rounding to 8 bits, and float32 sums of exact products (three parts each)
+    _within(got[..., :n], want, want.abs() * 2.0 ** -8 + size * 3 * k * 2.0 ** -24 + 1e-30)
+    if rot:
+        c, s = cos[pos.long()].double()[:, None], sin[pos.long()].double()[:, None]
+        a, b = x[..., k:k + rot:2].double(), x[..., k + 1:k + rot:2].double()
+        turned = torch.stack([a * c - b * s, b * c + a * s], -1).flatten(-2)
+        _within(got[..., n:n + rot], turned, 2.0 ** -7 * (a.abs().max() + b.abs().max()))
+        assert (got[..., n + rot:] == 0).all()
+
+
+def test_infinite_inputs_of_products_per_head(lib):
+    """An infinite or undefined input makes its own sums so and no other token's or head's."""
+    x = torch.ones(20, 2, 32)
+    x[3, 1, 5], x[7, 0, 1] = float("inf"), float("nan")
+    w = torch.ones(2, 16, 32).bfloat16()
+    wf = torch.empty_like(w, device=DEV)
+    for i in range(2):
+        lib.place_rows(w[i].to(DEV), wf[i], frag=True)
+    y = torch.empty(20, 32, dtype=torch.bfloat16, device=DEV)
+    lib.heads_linear_part(x.reshape(20, -1).to(DEV), 32, wf, y, 16, w_frag=True)
+    got = y.float().cpu().view(20, 2, 16)
+    assert torch.isinf(got[3, 1]).all() and torch.isnan(got[7, 0]).all()
+    got[3, 1] = got[7, 0] = 32.0
+    assert (got == 32.0).all()
