@@ -290,6 +290,7 @@ int rb_routed_experts(const void* h, int dtype, const float* weight, int top, co
                       int n_experts, int width, int ff, float limit, float alpha, void* stream);
 // The same for a step of at most 64 tokens with fragment-major experts: the same sums, bit for bit, in two launches.
 int rb_routed_experts_few(const void* h, const float* weight, int top, const int32_t* row_pair, const int32_t* tile_expert, int max_rows,
+                          int w_layout,
                           const void* w_gate, const void* w_up, const void* w_down, void* y, float* out, int n_tokens, int n_experts,
                           int width, int ff, float limit, float alpha, void* stream);
 // rb_route_top with its choices spelled out.  The router has n_outputs outputs, of which the first n_experts are experts
@@ -428,9 +429,9 @@ int rb_route_choose_units(const float* z, long long z_stride, const float* bias,
 // Experts without gates for steps of many tokens, on the dense product's tiles (gemm_grouped.hip): out[p] = Wd act(Wu h[p / top]) for
 // pairs sorted in runs padded to `unit` rows (64, 128 or 256); experts' matrices fragment-major bfloat16 with sizes that are multiples
 // of 64; act float32 [2] as rb_xielu takes it; y [max_rows, ff] bfloat16 is scratch.
-int rb_routed_experts_tiled(const void* h, int n_tokens, int top, const int32_t* row_pair, const int32_t* tile_expert, int unit, int max_rows,
-                            const void* w_up, const void* w_down, const float* act, void* y, float* out, int n_experts, int width, int ff,
-                            void* stream);
+int rb_routed_experts_tiled(const void* h, int n_tokens, const float* weight, int top, const int32_t* row_pair, const int32_t* tile_expert,
+                            int unit, int max_rows, int gated, const void* w_up, const void* w_down, const float* act, void* xs, void* y,
+                            float* out, int n_experts, int width, int ff, void* stream);
 // rb_rope_store with every query and key head RMS-normed first over its dim numbers, x / sqrt(mean(x^2) + eps) * w, with a
 // weight of dim numbers that the heads share (q_norm, k_norm float32 [dim]).
 int rb_norm_rope_store(const float* qkv, long long row_width, const float* cos, const float* sin, int rot, const float* q_norm,

@@ -185,7 +185,7 @@ class Kernels:
             "rb_pair_norm_mean": [_P, _P, _P, _P, _F, _P, _I, _I, _P],
             "rb_route_top": [_P, _L, _I, _I, _P, _P, _P, _P, _I, _I, _P],
             "rb_routed_experts": [_P, _I, _P, _I, _P, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _F, _F, _P],
-            "rb_routed_experts_few": [_P, _P, _I, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _F, _P],
+            "rb_routed_experts_few": [_P, _P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _F, _P],
             "rb_pairs_sum": [_P, _I, _P, _I, _I, _P],
             "rb_route_choose": [_P, _L, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P],
             "rb_experts_combine": [_P, _P, _P, _I, _I, _P, _I, _P, _P, _L, _P, _I, _I, _P],
@@ -217,7 +217,7 @@ class Kernels:
             "rb_lightning_chunks": [_P, _P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
             "rb_gated_rmsnorm_rows": [_P, _P, _P, _L, _I, _F, _P, _I, _I, _I, _P],
             "rb_route_choose_units": [_P, _L, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
-            "rb_routed_experts_tiled": [_P, _I, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+            "rb_routed_experts_tiled": [_P, _I, _P, _I, _P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
             "rb_route_choose_bias": [_P, _L, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P],
             "rb_attention_mixed": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _I, _I, _P],
             "rb_attention_mixed_bf16": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _I, _I, _I, _P, _P],
@@ -907,12 +907,14 @@ class Kernels:
                                         _ptr(tile_expert), max_rows, n, self._stream()))
 
     def routed_experts(self, h: torch.Tensor, weight: torch.Tensor, top: int, row_pair: torch.Tensor, tile_expert: torch.Tensor,
-                       w_gate: Optional[torch.Tensor], w_up: torch.Tensor, w_down: torch.Tensor, y: torch.Tensor, out: torch.Tensor,
+                       w_gate: Optional[torch.Tensor], w_up: Optional[torch.Tensor], w_down: torch.Tensor, y: torch.Tensor, out: torch.Tensor,
                        limit: float, alpha: float, w_frag: bool = False) -> None:
         """w_frag: every expert's matrices are stored fragment-major (`place_rows(..., frag=True)` on each).  w_gate None: experts
-        without a gate, Wd max(Wu x, 0)^2."""
+        without a gate, Wd max(Wu x, 0)^2.  w_up None (w_frag): w_gate [experts, 2 ff, width] holds gate and up rows interleaved in
+        blocks of 16."""
         n, width = h.shape
-        n_experts, ff, _ = w_up.shape
+        n_experts, _, ff = w_down.shape
+        layout = 0 if not w_frag else 1 if w_up is not None else 2
         max_rows = row_pair.shape[0]
         _check(h, "h")
         if weight is not None:                   # None: the experts' inputs are not scaled
@@ -920,18 +922,19 @@ class Kernels:
         _check(row_pair, "row_pair", torch.int32)
         _check(tile_expert, "tile_expert", torch.int32, (2 * (max_rows // 16),))
         if w_gate is not None:
-            _check(w_gate, "w_gate", h.dtype, (n_experts, ff, width))
-        _check(w_up, "w_up", h.dtype, (n_experts, ff, width))
+            _check(w_gate, "w_gate", h.dtype, (n_experts, 2 * ff if layout == 2 else ff, width))
+        if w_up is not None or layout != 2:
+            _check(w_up, "w_up", h.dtype, (n_experts, ff, width))
         _check(w_down, "w_down", h.dtype, (n_experts, width, ff))
         _check(y, "y", h.dtype, (max_rows, ff + width))
         _check(out, "out", torch.float32, (n * top, width))
         if w_frag and n <= ROUTED_FEW_TOKENS:
-            self._ok(self._lib.rb_routed_experts_few(_ptr(h), _ptr(weight), top, _ptr(row_pair), _ptr(tile_expert), max_rows, _ptr(w_gate),
+            self._ok(self._lib.rb_routed_experts_few(_ptr(h), _ptr(weight), top, _ptr(row_pair), _ptr(tile_expert), max_rows, layout, _ptr(w_gate),
                                                      _ptr(w_up), _ptr(w_down), _ptr(y), _ptr(out), n, n_experts, width, ff, float(limit),
                                                      float(alpha), self._stream()))
             return
         self._ok(self._lib.rb_routed_experts(_ptr(h), dtype_code(h.dtype), _ptr(weight), top, _ptr(row_pair), _ptr(tile_expert),
-                                             max_rows, _ptr(w_gate), _ptr(w_up), _ptr(w_down), int(bool(w_frag)), _ptr(y), _ptr(out),
+                                             max_rows, _ptr(w_gate), _ptr(w_up), _ptr(w_down), layout, _ptr(y), _ptr(out),
                                              n_experts, width, ff, float(limit), float(alpha), self._stream()))
 
     def route_choose(self, z: torch.Tensor, n_outputs: int, n_experts: int, top: int, score: int,
@@ -959,25 +962,33 @@ class Kernels:
                                                  _ptr(correction), _ptr(sel), _ptr(weight), _ptr(row_pair), _ptr(tile_expert), max_rows,
                                                  int(unit), n, self._stream()))
 
-    def routed_experts_tiled(self, h: torch.Tensor, top: int, row_pair: torch.Tensor, tile_expert: torch.Tensor, unit: int,
-                             w_up: torch.Tensor, w_down: torch.Tensor, act: torch.Tensor, y: torch.Tensor, out: torch.Tensor) -> None:
-        """Experts without gates on the dense product's tiles: out[p] = Wd act(Wu h[p // top]) for pairs sorted in runs padded to
-        `unit` rows (64, 128, 256); bfloat16, fragment-major experts; act float32 [2] as `xielu` takes it; y [rows, ff] is scratch."""
+    def routed_experts_tiled(self, h: torch.Tensor, weight: Optional[torch.Tensor], top: int, row_pair: torch.Tensor, tile_expert: torch.Tensor,
+                             unit: int, w_up: torch.Tensor, w_down: torch.Tensor, gated: bool, act: Optional[torch.Tensor],
+                             xs: Optional[torch.Tensor], y: torch.Tensor, out: torch.Tensor) -> None:
+        """Experts on the dense product's tiles for pairs sorted in runs padded to `unit` rows (64, 128, 256); bfloat16, fragment-major.
+        Not gated: out[p] = Wd act(Wu h[p // top]), act float32 [2] as `xielu` takes it.  Gated: w_up [experts, 2 ff, width] holds gate
+        and up rows interleaved in blocks of 16, act None or float32 [2] = (limit, alpha); `weight` [pairs] then may scale the inputs,
+        with xs [rows, width] as scratch.  y [rows, ff] is scratch."""
         n, width = h.shape
-        n_experts, ff, _ = w_up.shape
+        n_experts, _, ff = w_down.shape
         max_rows = row_pair.shape[0]
         _check(h, "h", torch.bfloat16)
         _check(row_pair, "row_pair", torch.int32)
         if unit not in (64, 128, 256) or max_rows % unit or max_rows < self.routed_rows(n, top, n_experts, unit):
             raise KernelError(f"routed_experts_tiled: {max_rows} rows in runs padded to {unit}")
         _check(tile_expert, "tile_expert", torch.int32, (2 * (max_rows // unit),))
-        _check(w_up, "w_up", torch.bfloat16, (n_experts, ff, width))
+        _check(w_up, "w_up", torch.bfloat16, (n_experts, 2 * ff if gated else ff, width))
         _check(w_down, "w_down", torch.bfloat16, (n_experts, width, ff))
-        _check(act, "act", torch.float32, (2,))
+        if act is not None or not gated:
+            _check(act, "act", torch.float32, (2,))
+        if weight is not None:
+            _check(weight, "weight", torch.float32, (n * top,))
+            _check(xs, "xs", torch.bfloat16, (max_rows, width))
         _check(y, "y", torch.bfloat16, (max_rows, ff))
         _check(out, "out", torch.float32, (n * top, width))
-        self._ok(self._lib.rb_routed_experts_tiled(_ptr(h), n, top, _ptr(row_pair), _ptr(tile_expert), int(unit), max_rows, _ptr(w_up),
-                                                   _ptr(w_down), _ptr(act), _ptr(y), _ptr(out), n_experts, width, ff, self._stream()))
+        self._ok(self._lib.rb_routed_experts_tiled(_ptr(h), n, _ptr(weight), top, _ptr(row_pair), _ptr(tile_expert), int(unit), max_rows,
+                                                   int(bool(gated)), _ptr(w_up), _ptr(w_down), _ptr(act), _ptr(xs), _ptr(y), _ptr(out),
+                                                   n_experts, width, ff, self._stream()))
 
     def experts_combine(self, pairs: torch.Tensor, sel: torch.Tensor, weight: torch.Tensor, top: int, n_experts: int,
                         h: torch.Tensor, shared: Optional[torch.Tensor], gate: Optional[torch.Tensor], gate_col: int,

@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256) void routed_up_few_kernel(const bf16_t* __rest
                                                             const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
                                                             const int32_t* __restrict__ tile_pos, const bf16_t* __restrict__ w_gate,
                                                             const bf16_t* __restrict__ w_up, bf16_t* __restrict__ y, int width, int ff,
-                                                            float limit, float alpha, int n_tiles) {
+                                                            float limit, float alpha, int n_tiles, int rows) {
   const int t0 = blockIdx.y, e = tile_expert[t0];
   if (e < 0 || tile_pos[t0] % NT != 0) return;
   const int lane = threadIdx.x & (RB_WAVE - 1), wave = threadIdx.x / RB_WAVE;
@@ -354,8 +354,8 @@ __global__ __launch_bounds__(256) void routed_up_few_kernel(const bf16_t* __rest
     wt[j] = (WEIGHTED && p >= 0) ? weight[p] : 1.0f;
     xr[j] = h + (size_t)(p >= 0 ? p / top : 0) * width + 8 * grp;
   }
-  const bf16_t* gr = GATED ? w_gate + ((size_t)e * ff + c0) * width + 8 * lane : nullptr;
-  const bf16_t* ur = w_up + ((size_t)e * ff + c0) * width + 8 * lane;
+  const bf16_t* gr = GATED ? w_gate + ((size_t)e * ff + c0) * rows * width + 8 * lane : nullptr;
+  const bf16_t* ur = w_up + ((size_t)e * ff + c0) * rows * width + 8 * lane;
   f32x4_t ag[NT], au[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) ag[j] = au[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(RT_THREADS) void routed_up_mfma_kernel(const bf16_t
                                                              const int32_t* __restrict__ tile_pos,
                                                              const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_up,
                                                              bf16_t* __restrict__ y, int width, int ff, float limit, float alpha,
-                                                             int n_tiles) {
+                                                             int n_tiles, int rows) {
   constexpr int CB = GATED ? 2 : 4;                     // blocks of 16 channels a wave: its loads and products keep their proportion
   // blockIdx.x counts the channels, so that workgroups that follow one another share their rows of the step (which
   // then come from memory once) and walk through an expert's matrices together
@@ -476,9 +476,10 @@ __global__ __launch_bounds__(RT_THREADS) void routed_up_mfma_kernel(const bf16_t
   const int n_cb = (ff - c0) / 16 < CB ? (ff - c0) / 16 : CB;        // ff is a multiple of 32, not always of 64
   const int r = lane & 15, grp = lane >> 4;
   const bf16_t* xr = xs + (size_t)t0 * RT_TILE * width + 8 * lane;
-  const bf16_t* gr = GATED ? w_gate + ((size_t)e * ff + c0) * width + 8 * lane : nullptr;
-  const bf16_t* ur = w_up + ((size_t)e * ff + c0) * width + 8 * lane;
-  const size_t blk = (size_t)16 * width;               // 16 rows further: the next block of channels, the next tile
+  const bf16_t* gr = GATED ? w_gate + ((size_t)e * ff + c0) * rows * width + 8 * lane : nullptr;
+  const bf16_t* ur = w_up + ((size_t)e * ff + c0) * rows * width + 8 * lane;
+  const size_t blk = (size_t)16 * width;               // 16 rows further: the next tile
+  const size_t wblk = blk * rows;                      // the next block of channels
   f32x4_t ag[RT_GROUP][CB], au[RT_GROUP][CB];
 #pragma unroll
   for (int j = 0; j < RT_GROUP; ++j)
@@ -488,8 +489,8 @@ __global__ __launch_bounds__(RT_THREADS) void routed_up_mfma_kernel(const bf16_t
     Frag8 fg[CB], fu[CB], fx[RT_GROUP];
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
-      if (GATED) fg[cb].u = load16(gr + cb * blk + k);
-      fu[cb].u = cb < n_cb ? load16(ur + cb * blk + k) : zero16();
+      if (GATED) fg[cb].u = load16(gr + cb * wblk + k);
+      fu[cb].u = cb < n_cb ? load16(ur + cb * wblk + k) : zero16();
     }
 #pragma unroll
     for (int j = 0; j < RT_GROUP; ++j) fx[j].u = j < nt ? load16(xr + j * blk + k) : zero16();
@@ -577,7 +578,8 @@ __global__ __launch_bounds__(RT_THREADS) void routed_down_mfma_kernel(const bf16
   }
 }
 
-// h [T, width], weight [T * top], w_gate and w_up [experts, ff, width], w_down [experts, width, ff], all of dtype;
+// h [T, width], weight [T * top], w_gate and w_up [experts, ff, width], w_down [experts, width, ff], all of dtype; w_layout 2: as 1
+// (fragment-major), and w_gate holds both, [experts, 2 ff, width] with gate and up rows interleaved in blocks of 16 (w_up: null);
 // y [max_rows, ff + width] of dtype is scratch; out [T * top, width] float32: the pairs' results.  tile_expert holds
 // max_rows / 16 experts and then as many positions of the tiles in their experts' runs, as rb_route_top leaves them.
 extern "C" int rb_routed_experts(const void* h, int dtype, const float* weight, int top, const int32_t* row_pair,
@@ -586,6 +588,12 @@ extern "C" int rb_routed_experts(const void* h, int dtype, const float* weight, 
                                  void* stream) {
   RB_RECORDED(rb_routed_experts(h, dtype, weight, top, row_pair, tile_expert, max_rows, w_gate, w_up, w_down, w_layout, y, out,
                                 n_experts, width, ff, limit, alpha, stream));
+  const int rows = w_layout == 2 ? 2 : 1;
+  if (w_layout == 2) {
+    RB_REQUIRE(w_gate && !w_up, "rb_routed_experts: interleaved experts have gates");
+    w_layout = 1;
+    w_up = (const bf16_t*)w_gate + (size_t)16 * width;
+  }
   RB_REQUIRE(w_layout == 0 || (w_layout == 1 && dtype == RB_BF16 && width % 32 == 0 && ff % 32 == 0),
              "rb_routed_experts: fragment-major experts are bfloat16 with sizes that are multiples of 32");
   RB_REQUIRE(max_rows >= 0 && max_rows % RT_TILE == 0 && n_experts > 0 && width > 0 && ff > 0 && top > 0,
@@ -603,7 +611,7 @@ extern "C" int rb_routed_experts(const void* h, int dtype, const float* weight, 
     routed_gather_kernel<<<tiles, 256, 0, s>>>((const bf16_t*)h, weight, top, row_pair, tile_expert, xs, width);
     auto up = w_gate ? routed_up_mfma_kernel<true> : routed_up_mfma_kernel<false>;
     up<<<dim3(w_gate ? (ff + 63) / 64 : (ff + 127) / 128, tiles), RT_THREADS, 0, s>>>(xs, row_pair, tile_expert, tile_expert + tiles, (const bf16_t*)w_gate,
-                                                          (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha, tiles);
+                                                          (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha, tiles, rows);
     routed_down_mfma_kernel<<<dim3((width + 127) / 128, tiles), RT_THREADS, 0, s>>>((const bf16_t*)y, row_pair, tile_expert,
                                                                              tile_expert + tiles, (const bf16_t*)w_down, out, width,
                                                                              ff, tiles);
@@ -626,10 +634,13 @@ extern "C" int rb_routed_experts(const void* h, int dtype, const float* weight, 
 // rb_routed_experts for a step of at most 64 tokens with fragment-major experts (bfloat16, sizes that are multiples of 32): the
 // same sums in the same order, two launches whose waves keep more of the experts' matrices on their way.  n_tokens: rows of h.
 extern "C" int rb_routed_experts_few(const void* h, const float* weight, int top, const int32_t* row_pair, const int32_t* tile_expert,
-                                     int max_rows, const void* w_gate, const void* w_up, const void* w_down, void* y, float* out,
+                                     int max_rows, int w_layout, const void* w_gate, const void* w_up, const void* w_down, void* y, float* out,
                                      int n_tokens, int n_experts, int width, int ff, float limit, float alpha, void* stream) {
-  RB_RECORDED(rb_routed_experts_few(h, weight, top, row_pair, tile_expert, max_rows, w_gate, w_up, w_down, y, out, n_tokens, n_experts, width,
+  RB_RECORDED(rb_routed_experts_few(h, weight, top, row_pair, tile_expert, max_rows, w_layout, w_gate, w_up, w_down, y, out, n_tokens, n_experts, width,
                                     ff, limit, alpha, stream));
+  const int rows = w_layout == 2 ? 2 : 1;
+  RB_REQUIRE(w_layout == 1 || (w_layout == 2 && w_gate && !w_up), "rb_routed_experts_few: layout %d of the experts", w_layout);
+  if (w_layout == 2) w_up = (const bf16_t*)w_gate + (size_t)16 * width;
   RB_REQUIRE(n_tokens >= 0 && n_tokens <= RT_FEW_MOST, "rb_routed_experts_few: %d tokens (at most %d)", n_tokens, RT_FEW_MOST);
   RB_REQUIRE(max_rows >= 0 && max_rows % RT_TILE == 0 && max_rows / RT_TILE <= 65535 && n_experts > 0 && width > 0 && ff > 0 && top > 0 &&
                  width % 32 == 0 && ff % 32 == 0,
@@ -643,7 +654,7 @@ extern "C" int rb_routed_experts_few(const void* h, const float* weight, int top
   const dim3 gu((ff + 63) / 64, tiles), gd((width + 63) / 64, tiles);
 #define RT_UP(NT, WEIGHTED)                                                                                                           \
   (w_gate ? routed_up_few_kernel<NT, WEIGHTED, true> : routed_up_few_kernel<NT, WEIGHTED, false>)<<<gu, 256, 0, s>>>((const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles,    \
-                                                        (const bf16_t*)w_gate, (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha, tiles)
+                                                        (const bf16_t*)w_gate, (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha, tiles, rows)
 #define RT_DOWN(NT)                                                                                                       \
   routed_down_few_kernel<NT><<<gd, 256, 0, s>>>((const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles,             \
                                                 (const bf16_t*)w_down, out, width, ff, tiles)

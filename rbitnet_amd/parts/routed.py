@@ -36,7 +36,7 @@ import torch
 from ..errors import ConfigError
 from .base import BuildEnv, Part, TensorSpec, register_feed_forward
 from .feed_forward import DenseAct, SwiGLU
-from .linear import linear, pack_rows
+from .linear import GATE_BLOCK, linear, pack_rows
 from .stream import ExpertPairs
 
 DEFAULT_NAMES = {"router": "router", "expert": "e{i}", "gate": "gate", "up": "up", "down": "down", "correction": "correction",
@@ -44,6 +44,7 @@ DEFAULT_NAMES = {"router": "router", "expert": "e{i}", "gate": "gate", "up": "up
 MAX_EXPERTS = 1024
 MAX_CHOSEN = 64            # of the softmax over the chosen logits
 TILED_FROM = 65            # tokens of a step from which experts without gates run on the dense product's tiles
+GATED_TILED_FROM = 112     # rows of an expert's run, in the mean, from which gated ones do
 
 
 def tile_rows(n_pairs: int, n_experts: int) -> int:
@@ -152,33 +153,55 @@ class RoutedExperts(Part):
                 lib.place_rows(tensors[self._name(i, what)].contiguous(), out[i], frag=self.frag)
             return out
 
-        # without gates a step of many tokens runs on the dense product's tiles
-        self.tiled = bool(self.frag and self.unit == "squared_relu" and self.weight_on == "output" and self.hidden % 64 == 0 and self.ff % 64 == 0)
-        self.act = torch.tensor([float("nan"), 1.0], dtype=torch.float32, device=r.device) if self.tiled else None     # (see DenseAct)
-        self.w_gate = stack("gate") if self.unit == "gated" else None
-        self.w_up, self.w_down = stack("up"), stack("down")
+        def stack_gated() -> torch.Tensor:    # gate and up rows interleaved in blocks of 16, as the dense gated product has them
+            first = tensors[self._name(0, "gate")]
+            out = torch.empty((self.n_experts, 2 * self.ff, self.hidden), dtype=first.dtype, device=first.device)
+            for i in range(self.n_experts):
+                for row0, what in ((0, "gate"), (GATE_BLOCK, "up")):
+                    lib.place_rows(tensors[self._name(i, what)].contiguous(), out[i], row0, GATE_BLOCK, 2 * GATE_BLOCK, frag=True)
+            return out
+
+        # a step of many tokens runs on the dense product's tiles
+        gated = self.unit == "gated"
+        self.tiled = bool(self.frag and (gated or self.weight_on == "output") and self.hidden % 64 == 0 and self.ff % 64 == 0)
+        self.act = None
+        if self.tiled and not gated:
+            self.act = torch.tensor([float("nan"), 1.0], dtype=torch.float32, device=r.device)     # (see DenseAct)
+        elif self.tiled and self.limit is not None:
+            self.act = torch.tensor([self.limit, self.alpha], dtype=torch.float32, device=r.device)
+        self.w_down = stack("down")
+        if gated and self.frag:
+            self.w_gate, self.w_up = stack_gated(), None
+        else:
+            self.w_gate, self.w_up = stack("gate") if gated else None, stack("up")
 
     def forward(self, h: torch.Tensor, ctx=None, stream: Optional[torch.Tensor] = None, next_norm=None, pairs: bool = False):
         """-> float32 [T, E], or, with pairs=True (where `leaves_pairs` or `leaves_shared_pairs`), the `ExpertPairs` of the step."""
         lib, t, dev = self.env.lib, h.shape[0], h.device
         z = linear(lib, h, self.w_router, torch.float32)
         n_pairs = t * self.top
-        tiled = self.tiled and t >= TILED_FROM
+        # (gated experts have a kernel for runs of a few dozen rows that is as fast; a row's place is a 32-bit byte offset in the tiles)
+        tiled = self.tiled and t >= (TILED_FROM if self.w_gate is None else GATED_TILED_FROM * self.n_experts / self.top) \
+            and t * self.hidden * 2 < 1 << 32
         unit = tile_rows(n_pairs, self.n_experts) if tiled else 16
         max_rows = lib.routed_rows(t, self.top, self.n_experts, unit)
         sel = torch.empty(n_pairs, dtype=torch.int32, device=dev)
         weight = torch.empty(n_pairs, dtype=torch.float32, device=dev)
         row_pair = torch.empty(max_rows, dtype=torch.int32, device=dev)
         tile_expert = torch.empty(2 * (max_rows // unit), dtype=torch.int32, device=dev)      # experts, then positions in their runs
-        if self.plain:
+        if self.plain and unit == 16:
             lib.route_top(z, self.n_experts, self.top, sel, weight, row_pair, tile_expert)
         else:
             lib.route_choose(z, self.n_outputs, self.n_experts, self.top, self.score, self.correction, sel, weight, row_pair,
                              tile_expert, bias=self.bias, unit=unit)
         out = torch.empty((n_pairs, self.hidden), dtype=torch.float32, device=dev)
         if tiled:
+            gated = self.w_gate is not None
+            scaled = weight if self.weight_on == "input" else None
             y = torch.empty((max_rows, self.ff), dtype=h.dtype, device=dev)
-            lib.routed_experts_tiled(h, self.top, row_pair, tile_expert, unit, self.w_up, self.w_down, self.act, y, out)
+            xs = torch.empty((max_rows, self.hidden), dtype=h.dtype, device=dev) if scaled is not None else None
+            lib.routed_experts_tiled(h, scaled, self.top, row_pair, tile_expert, unit, self.w_gate if gated else self.w_up, self.w_down,
+                                     gated, self.act, xs, y, out)
         else:
             y = torch.empty((max_rows, self.ff + self.hidden), dtype=h.dtype, device=dev)     # scratch: gated units, scaled inputs
             lib.routed_experts(h, weight if self.weight_on == "input" else None, self.top, row_pair, tile_expert, self.w_gate,

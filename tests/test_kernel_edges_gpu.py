@@ -184,3 +184,58 @@ def test_infinite_inputs_of_products_per_head(lib):
     assert torch.isinf(got[3, 1]).all() and torch.isnan(got[7, 0]).all()
     got[3, 1] = got[7, 0] = 32.0
     assert (got == 32.0).all()
+
+
+# ---------------------------------------------------------------- gated experts on the dense product's tiles
+@pytest.mark.parametrize("tokens,top,experts,width,ff", [(112, 1, 1, 64, 64), (150, 2, 2, 128, 192), (131, 3, 3, 64, 320), (1600, 2, 2, 64, 64),
+                                                         (700, 4, 16, 256, 128)])
+@pytest.mark.parametrize("weight_on,limit", [("input", 1.5), ("output", None), ("output", 2.0)])
+def test_gated_experts_on_tiles(lib, tokens, top, experts, width, ff, weight_on, limit):
+    from rbitnet_amd.parts.routed import tile_rows
+    g = torch.Generator().manual_seed(tokens + ff)
+    r = lambda *s, f=1.0: (torch.randn(*s, generator=g) * f).bfloat16()
+    h, gate, up, down = r(tokens, width), r(experts, ff, width, f=width ** -0.5 * 2), r(experts, ff, width, f=width ** -0.5 * 2), r(experts, width, ff, f=ff ** -0.5)
+    z = torch.randn(tokens, experts, generator=g)
+    unit = tile_rows(tokens * top, experts)
+    rows = lib.routed_rows(tokens, top, experts, unit)
+    i32 = lambda n: torch.empty(n, dtype=torch.int32, device=DEV)
+    sel, row_pair, tile_expert = i32(tokens * top), i32(rows), i32(2 * (rows // unit))
+    weight = torch.empty(tokens * top, device=DEV)
+    lib.route_choose(z.to(DEV), experts, experts, top, 0, None, sel, weight, row_pair, tile_expert, unit=unit)
+    both, wd = torch.empty(experts, 2 * ff, width, dtype=torch.bfloat16, device=DEV), torch.empty(experts, width, ff, dtype=torch.bfloat16, device=DEV)
+    for e in range(experts):
+        lib.place_rows(gate[e].to(DEV), both[e], 0, 16, 32, frag=True)
+        lib.place_rows(up[e].to(DEV), both[e], 16, 16, 32, frag=True)
+        lib.place_rows(down[e].to(DEV), wd[e], frag=True)
+    act = None if limit is None else torch.tensor([limit, 1.702], device=DEV)
+    scaled = weight if weight_on == "input" else None
+    xs = torch.full((rows, width), float("nan"), dtype=torch.bfloat16, device=DEV)
+    y = torch.full((rows, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
+    out = torch.full((tokens * top, width), float("nan"), device=DEV)
+    lib.routed_experts_tiled(h.to(DEV), scaled, top, row_pair, tile_expert, unit, both, wd, True, act, xs, y, out)
+    s, wt = sel.cpu().long(), weight.cpu()
+    x = h.double().repeat_interleave(top, 0)
+    if scaled is not None:
+        x = (h.float().repeat_interleave(top, 0) * wt[:, None]).bfloat16().double()
+    for e in range(experts):
+        at = torch.nonzero(s == e)[:, 0]
+        a, b = x[at] @ gate[e].double().T, x[at] @ up[e].double().T
+        if limit is not None:
+            a, b = a.clamp(max=limit), b.clamp(-limit, limit)
+            u = a * torch.sigmoid(float(torch.tensor(1.702)) * a) * (b + 1)
+        else:
+            u = a * torch.sigmoid(a) * b
+        want = u @ down[e].double().T
+        # the units are rounded to 8 bits, everything else is float32
+        _within(out[at], want, (u.abs() * 2.0 ** -8 + 1e-4) @ down[e].double().abs().T)
+    # the kernels for few tokens and for runs of a few rows read the same interleaved matrices
+    for n in (1, 9, 40, 100):
+        n = min(n, tokens)
+        few_rows = lib.routed_rows(n, top, experts)
+        sel2, row2, tile2, weight2 = i32(n * top), i32(few_rows), i32(2 * (few_rows // 16)), torch.empty(n * top, device=DEV)
+        lib.route_choose(z[:n].to(DEV), experts, experts, top, 0, None, sel2, weight2, row2, tile2)
+        y2 = torch.empty((few_rows, ff + width), dtype=torch.bfloat16, device=DEV)
+        out2 = torch.full((n * top, width), float("nan"), device=DEV)
+        lib.routed_experts(h[:n].to(DEV), weight2 if scaled is not None else None, top, row2, tile2, both, None, wd, y2, out2, limit or 0.0, 1.702,
+                           w_frag=True)
+        _within(out2, out[:n * top].double(), 0.05)
