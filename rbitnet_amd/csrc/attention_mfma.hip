@@ -988,9 +988,10 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_mfma_kernel(
       pf[s2].u.w = pack_bf16x2(sc[2 * s2 + 1][2], sc[2 * s2 + 1][3]);
     }
     // ---- the page of V has arrived (loads complete in issue order; the next page's keys,
-    // asked for after it, may still be on their way)
-    if (more2) wait_vm<4 * KS + 1>();
-    else if (more) wait_vm<4 * KS>();
+    // asked for after it, may still be on their way).  The number of the page after that is no part of the count: it is the
+    // same for the whole wave, and the compiler fetches it through the scalar cache, which counts elsewhere.  (Counted as one more
+    // load, it let a wave with three pages and more read the last four rows of a page of V before they had arrived.)
+    if (more) wait_vm<4 * KS>();
     else wait_vm<0>();
     if (pg == last_page) {
       const int r_pos = pos % RB_PAGE;

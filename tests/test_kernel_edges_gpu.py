@@ -239,3 +239,32 @@ def test_gated_experts_on_tiles(lib, tokens, top, experts, width, ff, weight_on,
         lib.routed_experts(h[:n].to(DEV), weight2 if scaled is not None else None, top, row2, tile2, both, None, wd, y2, out2, limit or 0.0, 1.702,
                            w_frag=True)
         _within(out2, out[:n * top].double(), 0.05)
+
+
+# ---------------------------------------------------------------- single-token attention over several pages a wave
+@pytest.mark.parametrize("dim,heads,kv,length,splits", [(128, 32, 8, 8001, 8), (128, 16, 1, 1500, 1), (64, 8, 2, 4000, 2), (128, 4, 4, 2100, 1)])
+def test_single_token_attention_over_many_pages(lib, dim, heads, kv, length, splits):
+    """Every wave walks three pages and more: the same bits every time, and the weighted sum of every row of every page."""
+    g = torch.Generator().manual_seed(length)
+    n = (length + 63) // 64
+    order = torch.randperm(n, generator=g)
+    k = torch.randn(n * 64, kv, dim, generator=g).bfloat16()
+    v = torch.randn(n * 64, kv, dim, generator=g).bfloat16()
+    # pages that differ much from one another: a row of another page in the place of one's own shows
+    v = (v.float() + 40.0 * torch.randn(n, 1, 1, generator=g).repeat_interleave(64, 0)).bfloat16()
+    paged = lambda x: x.view(n, 64, kv, dim).transpose(1, 2).contiguous()[torch.argsort(order)]
+    kp, vp = paged(k).to(DEV), paged(v).to(DEV)
+    q = torch.randn(1, heads, dim, generator=g).bfloat16()
+    table = order.to(torch.int32)[None].to(DEV)
+    pos = torch.tensor([length - 1], dtype=torch.int32)
+    ws = torch.empty(heads * splits * (dim + 2), device=DEV)
+    outs = []
+    for _ in range(20):
+        out = torch.full((1, heads * dim), float("nan"), dtype=torch.bfloat16, device=DEV)
+        lib.attention_decode_bf16(q.to(DEV), kp, vp, out, pos.to(DEV), table, heads, kv, dim, 0.05, None, splits, ws)
+        outs.append(out)
+    want = _attention64(q.float(), k[:length].float(), v[:length].float(), pos, 0.05)
+    # weights and outputs are rounded to 8 bits each
+    _within(outs[0].view(want.shape), want, 2.0 ** -7 * float(v.abs().max()))
+    for out in outs[1:]:
+        assert torch.equal(out, outs[0])
