@@ -1074,28 +1074,51 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_mfma_kernel(
   }
 }
 
+// The splits of a (sequence, head) into one: a thread a number of the head, the splits' maxima and sums a lane each, so that all
+// of them are one trip to memory (a loop over the splits, once for the maximum and once for the sums, took 6.2 us for 8 splits
+// of 32 heads, 4.7 this way with 16 splits of 32 heads).
 // sum_only: the splits' outputs are added as they are (sigmoid weights), without maxima and denominators
 template <int D>
 __global__ void attn_decode_combine_kernel(const float* __restrict__ ws, bf16_t* __restrict__ out, int n_splits,
                                            const float* __restrict__ sinks, int n_heads, int sum_only) {
+  constexpr int AHEAD = 8;
+  __shared__ float factors[D / RB_WAVE][RB_WAVE];
   const size_t row = blockIdx.x;            // sequence * heads + head
-  const int d = threadIdx.x;
+  const int d = threadIdx.x, lane = threadIdx.x & (RB_WAVE - 1);
   const float* src = ws + row * n_splits * (D + 2);
-  if (sum_only) {
-    float v = 0.f;
-    for (int s = 0; s < n_splits; ++s) v += src[(size_t)s * (D + 2) + d];
-    out[row * D + d] = f32_to_bf16(v);
-    return;
-  }
+  float* mine = factors[threadIdx.x / RB_WAVE];      // every wave keeps its own, so that none waits for another
   float mx = -INFINITY;
-  for (int s = 0; s < n_splits; ++s) mx = fmaxf(mx, src[(size_t)s * (D + 2) + D]);
+  if (!sum_only) {
+    for (int s = lane; s < n_splits; s += RB_WAVE) mx = fmaxf(mx, src[(size_t)s * (D + 2) + D]);
+    mx = wave_max(mx);
+  }
   const float m_safe = (mx == -INFINITY) ? 0.f : mx;
   float a = 0.f, l = 0.f;
-  for (int s = 0; s < n_splits; ++s) {
-    const float f = exp2f(src[(size_t)s * (D + 2) + D] - m_safe);
-    a += src[(size_t)s * (D + 2) + d] * f;
-    l += src[(size_t)s * (D + 2) + D + 1] * f;
+  for (int s0 = 0; s0 < n_splits; s0 += RB_WAVE) {
+    const int here = n_splits - s0 < RB_WAVE ? n_splits - s0 : RB_WAVE;
+    float f = 1.f;
+    if (!sum_only && lane < here) {
+      const float* of = src + (size_t)(s0 + lane) * (D + 2);
+      f = exp2f(of[D] - m_safe);
+      l += of[D + 1] * f;
+    }
+    mine[lane] = f;                                   // this wave's alone; a wave's LDS accesses complete in order
+    __builtin_amdgcn_wave_barrier();
+    for (int s1 = 0; s1 < here; s1 += AHEAD) {
+      float v[AHEAD];
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) v[u] = src[(size_t)(s0 + (s1 + u < here ? s1 + u : s1)) * (D + 2) + d];
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u)
+        if (s1 + u < here) a = sum_only ? a + v[u] : fmaf(v[u], mine[s1 + u], a);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
+  if (sum_only) {
+    out[row * D + d] = f32_to_bf16(a);
+    return;
+  }
+  l = wave_sum(l);
   if (sinks) l += exp2f(fmaf(sinks[row % n_heads], LOG2E, -m_safe));          // the sink: in the denominator only
   out[row * D + d] = f32_to_bf16(l > 0.f ? a / l : 0.f);
 }

@@ -50,6 +50,18 @@ def decode_splits(n_seqs: int, n_kv_heads: int, bucket: int, n_compute_units: in
     return max(1, min(int(bucket), 16, n_compute_units // max(1, n_seqs * max(1, n_kv_heads))))
 
 
+def decode_workgroups(n_seqs: int, n_kv_heads: int, bucket: int, n_compute_units: int) -> int:
+    """`decode_splits`, and more where few (sequence, kv head) pairs leave the GPU empty: a wave then takes a page or two at
+    contexts of 16 pages and more, up to 16 workgroups a pair and one a compute unit.  Measured with the combination of the splits,
+    heads of 128: 4 sequences of 390 to 1,500 keys on one kv head 18.8 us with 2 workgroups a pair, 14.1 with 8, 14.9 with 16; one
+    sequence of 8,010 keys on 8 kv heads 21.2 with 8, 16.8 with 16, 17.9 with 32; 8 of 1,200 to 2,000 keys on 8 kv heads 21.0
+    with 2, 17.5 with 4 (256 workgroups), 18.9 with 8; below 16 pages the second launch costs what the shorter walk gives."""
+    splits = decode_splits(n_seqs, n_kv_heads, bucket, n_compute_units)
+    if FORCED_DECODE_SPLITS or bucket < 2:
+        return splits
+    return max(splits, min(16, 4 * int(bucket), n_compute_units // max(1, n_seqs * max(1, n_kv_heads))))
+
+
 @dataclass
 class StepBatch:
     """One step as the host knows it."""
@@ -208,7 +220,7 @@ class StepContext:
     def decode_workspace(self, n_heads: int, head_dim: int, n_kv_heads: int = 1) -> Tuple:
         """Split count and scratch for decode attention: enough workgroups to fill the
         GPU, whatever the context length (each split strides over the pages)."""
-        n_splits = decode_splits(self.n_seqs, n_kv_heads, self.bucket, self.n_compute_units)
+        n_splits = decode_workgroups(self.n_seqs, n_kv_heads, self.bucket, self.n_compute_units)
         key = (n_heads, head_dim, n_kv_heads, n_splits)
         if key not in self._workspaces:
             ws = torch.empty(self.n_seqs * n_heads * n_splits * (head_dim + 2), dtype=torch.float32,

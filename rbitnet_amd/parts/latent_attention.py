@@ -130,11 +130,10 @@ class LatentAttention(Part):
         self.uk_frag = allowed and lib.heads_frag_ok(first.dtype, self.kv_rank, self.dim, self.dim + self.rot, self.page_width)
         self.uv_frag = allowed and lib.heads_frag_ok(first.dtype, self.vdim, self.kv_rank, self.page_width, self.vdim)
 
-        def fragments(w: torch.Tensor) -> torch.Tensor:
+        def fragments(w: torch.Tensor) -> torch.Tensor:      # (the heads' blocks of 16 rows follow one another)
             rows = w.transpose(1, 2).contiguous()
             out = torch.empty_like(rows)
-            for i in range(self.heads):
-                lib.place_rows(rows[i], out[i], frag=True)
+            lib.place_rows(rows.view(-1, rows.shape[2]), out.view(-1, rows.shape[2]), frag=True)
             return out
 
         if self.uk_frag:
