@@ -30,28 +30,51 @@ struct FoldArgs {
   const float* gain;            // epilogue 3: [N]
   bf16_t* gained;               // epilogue 3: [M, N]
   float* squares_out;           // epilogue 3: [M, ceil(N / 16)]
+  int wide;                     // C, the gain and the prepared rows can be read and written four columns at a time
   int w_frag;                   // W is stored fragment-major (see gemm_internal.h)
   const float* act;             // epilogue 0: xIELU's two numbers, applied to the sums before they are stored; null: none
 };
 
+// Epilogue 0 with xIELU, a kernel of its own: as a run-time choice its code lay in the way of every product (2,048 rows at K = 2048,
+// 4 tokens: 4.8 us with it, 4.5 without).
+constexpr int EPI_ACT = 4;
+
 // What a lane does with its 4 consecutive sums of token mm, columns nn.. (epilogues 0, 2, 3).
 // All 64 lanes come here together: the sums of squares go round the four lanes that share
 // a token's 16 columns.
-template <int EPI, typename TO>
+// MAY: four columns at a time where FoldArgs::wide says so.
+template <int EPI, bool MAY, typename TO>
 __device__ __forceinline__ void store_sums(TO* __restrict__ c, const f32x4_t& sums, const f32x4_t& before,
                                            const f32x4_t& gain, int mm, int nn, int m, int n, int tile, int kq,
                                            const FoldArgs& fa) {
   const bool row_ok = mm < m;
   float sq = 0.f;
   XieluPair xa = {0.f, 0.f};
-  if (EPI == 0 && fa.act) xa = xielu_pair(fa.act);
-  if (row_ok) {
+  if (EPI == EPI_ACT) xa = xielu_pair(fa.act);
+  if (MAY && row_ok && fa.wide) {
+    if (nn < n) {
+      f32x4_t v = EPI == 2 || EPI == 3 ? before + sums : sums;
+      if (EPI == EPI_ACT) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = xielu_value(v[i], xa.ap, xa.an);
+      }
+      TO* dst = c + (size_t)mm * n + nn;
+      if constexpr (sizeof(TO) == 2) *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+      else *reinterpret_cast<f32x4_t*>(dst) = v;
+      if (EPI == 3) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sq += v[i] * v[i];
+        const f32x4_t p = v * gain;
+        *reinterpret_cast<uint2*>(fa.gained + (size_t)mm * n + nn) = make_uint2(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]));
+      }
+    }
+  } else if (row_ok) {
     TO* dst = c + (size_t)mm * n + nn;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (nn + i >= n) continue;
-      float v = EPI >= 2 ? before[i] + sums[i] : sums[i];
-      if (EPI == 0 && fa.act) v = xielu_value(v, xa.ap, xa.an);
+      float v = EPI == 2 || EPI == 3 ? before[i] + sums[i] : sums[i];
+      if (EPI == EPI_ACT) v = xielu_value(v, xa.ap, xa.an);
       Num<TO>::store(dst + i, v);
       if (EPI == 3) {
         sq += v * v;
@@ -100,13 +123,17 @@ __device__ __forceinline__ float squares_sum(const SquaresShare& s) {
   return t;
 }
 
-template <int MB, int R, int U, bool FAST, int EPI, typename TO, bool SCALED>
+// FAST: K % 128 == 0, the K / 128 stages of 128 depth values dealt to the waves as evenly as they go, one stage in flight while the one
+// before is multiplied; else any K % 8 == 0, with bounds checks.  WF (up to 16 tokens): W is stored fragment-major.
+// (All of a wave's stages asked for at once instead, W's first, for up to four stages a wave: no faster at K = 128 to 4096 with any
+// number of waves, 2,048 rows at K = 2048 4.5 us either way, 8,192 rows 7.6 -> 8.3.)
+template <int MB, int R, bool FAST, bool WF, int EPI, typename TO, bool SCALED>
 __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restrict__ x,
                                                           const bf16_t* __restrict__ w, TO* __restrict__ c,
                                                           int m, int n, int k, int k_per_wave, FoldArgs fa) {
-  extern __shared__ float red[];      // [waves - 1][ACCX][64]
-  constexpr int ACC = R * MB * 4;
-  constexpr int ACCX = ACC + (SCALED ? MB : 0);      // the sums of squares travel with the partial sums
+  // [waves - 1][R * MB][64] pieces of four sums, then, with SCALED, [waves - 1][MB][64] sums of squares
+  extern __shared__ __attribute__((aligned(16))) float red[];
+  constexpr int ACC = R * MB;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int n_waves = blockDim.x >> 6;
@@ -123,17 +150,28 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
   // Where a lane finds its 8 values at depth kstart (a multiple of 32) + 8 kq of row tile rt:
   // wrow[rt] + kstart * wk.  Rows [N, K]: the row's start + 8 kq, wk = 1.  Fragment-major: the
   // tile's start + 8 lane, wk = 16 (a block of 16 rows x 32 depth values is 512 values).
-  const bool wf = fa.w_frag != 0;
-  const int wk = wf ? 16 : 1;
+  const bool frag = MB == 1 ? WF : fa.w_frag != 0;      // (compiled in for up to 16 tokens)
+  const int wk = frag ? 16 : 1;
   const bf16_t* wrow[R];
   bool wok[R];
 #pragma unroll
   for (int rt = 0; rt < R; ++rt) {
     const int row = n0 + 16 * rt + r;
     wok[rt] = row < n;
-    if (wf) wrow[rt] = w + (size_t)(n0 + 16 * rt < n ? n0 + 16 * rt : 0) * k + 8 * lane;
+    if (frag) wrow[rt] = w + (size_t)(n0 + 16 * rt < n ? n0 + 16 * rt : 0) * k + 8 * lane;
     else wrow[rt] = w + (size_t)(wok[rt] ? row : 0) * k + 8 * kq;
   }
+  Frag8 a[R][4], b[MB][4];
+  auto load_w = [&](int ks) {                         // depth values ks..ks + 127 of the wave's rows
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int rt = 0; rt < R; ++rt) {
+        const bf16_t* src = wrow[rt] + (size_t)(ks + 32 * j) * wk;
+        if (frag) a[rt][j].u = load16_stream(src);      // read once, whole lines at a time: past the caches
+        else a[rt][j].u = load16(src);
+      }
+  };
   const bf16_t* xrow[MB];
   bool xok[MB];
   float ss[MB];
@@ -160,91 +198,74 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
     const int nn = n0 + 16 * rt + 4 * kq;
     gain[rt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     if (EPI == 3 && wave == 0) {
+      if (fa.wide) {
+        if (nn < n) gain[rt] = *reinterpret_cast<const f32x4_t*>(fa.gain + nn);
+      } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (nn + i < n) gain[rt][i] = fa.gain[nn + i];
+        for (int i = 0; i < 4; ++i)
+          if (nn + i < n) gain[rt][i] = fa.gain[nn + i];
+      }
     }
 #pragma unroll
     for (int cb = 0; cb < MB; ++cb) {
       before[rt][cb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-      if (EPI >= 2 && wave == 0) {
+      if ((EPI == 2 || EPI == 3) && wave == 0) {
         const int mm = 16 * cb + r;
+        if (sizeof(TO) == 4 && fa.wide) {
+          if (mm < m && nn < n) before[rt][cb] = *reinterpret_cast<const f32x4_t*>(c + (size_t)mm * n + nn);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (mm < m && nn + i < n) before[rt][cb][i] = Num<TO>::load(c + (size_t)mm * n + nn + i);
+          for (int i = 0; i < 4; ++i)
+            if (mm < m && nn + i < n) before[rt][cb][i] = Num<TO>::load(c + (size_t)mm * n + nn + i);
+        }
       }
     }
   }
 
-  int k_begin = wave * k_per_wave;
-  const int k_end = (k_begin + k_per_wave < k) ? k_begin + k_per_wave : k;
-  if (FAST) {
+  auto multiply_stage = [&]() {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int rt = 0; rt < R; ++rt)
+#pragma unroll
+        for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = mfma16(a[rt][j], b[cb][j], acc[rt][cb]);
+  };
+  if constexpr (FAST) {
     // K and every wave's range are multiples of 128: no bounds checks.  Rows beyond N or M
-    // are read from row 0 instead and their results never stored.  U stages of 128 depth
-    // values stay in flight: as soon as a stage has been multiplied, its registers are
-    // loaded again with the stage U further on.
-    // Every wave has at least one stage (the host launches no more waves than stages), and a
-    // wave's stage count is a multiple of U: the loads below are unconditional, which lets the
-    // compiler count outstanding loads exactly and start multiplying when the oldest stage
-    // arrives.  The K / 128 stages are dealt to the waves as evenly as they go: the first
-    // K / 128 % waves waves take one more (K = 11008 = 86 stages over 8 waves: six times 11,
-    // twice 10).
-    static_assert(U == 1, "uneven stage counts per wave need one stage in flight");
+    // are read from row 0 instead and their results never stored.
+    // Every wave has at least one stage (the host launches no more waves than stages): the loads below are unconditional, which
+    // lets the compiler count outstanding loads exactly.  The first K / 128 % waves waves take one stage more (K = 11008 = 86
+    // stages over 8 waves: six times 11, twice 10).
     const int total = k / 128, base = total / n_waves, extra = total % n_waves;
     const int stages = base + (wave < extra ? 1 : 0);
-    k_begin = 128 * (wave * base + (wave < extra ? wave : extra));
-    Frag8 a[U][R][4], b[U][MB][4];
-    auto load_stage = [&](int u, int st) {
+    const int k_begin = 128 * (wave * base + (wave < extra ? wave : extra));
+    auto load_stage = [&](int st) {
       const int ks = k_begin + 128 * st;
-      const int kk = ks + 8 * kq;
-      if (wf) {           // read once, whole lines at a time: past the caches
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int rt = 0; rt < R; ++rt) a[u][rt][j].u = load16_stream(wrow[rt] + (size_t)(ks + 32 * j) * 16);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int rt = 0; rt < R; ++rt) a[u][rt][j].u = load16(wrow[rt] + ks + 32 * j);
-      }
+      load_w(ks);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int cb = 0; cb < MB; ++cb) b[u][cb][j].u = load16(xrow[cb] + kk + 32 * j);
+        for (int cb = 0; cb < MB; ++cb) b[cb][j].u = load16(xrow[cb] + ks + 8 * kq + 32 * j);
     };
-    auto multiply_stage = [&](int u) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int rt = 0; rt < R; ++rt)
-#pragma unroll
-          for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = mfma16(a[u][rt][j], b[u][cb][j], acc[rt][cb]);
-    };
-#pragma unroll
-    for (int u = 0; u < U; ++u) load_stage(u, u);
+    load_stage(0);
     // the sums of squares were asked for before the first stage and arrive before it: added up
     // here, they do not occupy registers during the loop
     if (SCALED) {
 #pragma unroll
       for (int cb = 0; cb < MB; ++cb) ss[cb] = squares_sum(asked[cb]);
     }
-    for (int s0 = 0; s0 + U < stages; s0 += U) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        multiply_stage(u);
-        load_stage(u, s0 + u + U);
-      }
+    for (int st = 1; st < stages; ++st) {
+      multiply_stage();
+      load_stage(st);
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u) multiply_stage(u);
+    multiply_stage();
   } else {
     if (SCALED) {
 #pragma unroll
       for (int cb = 0; cb < MB; ++cb) ss[cb] = squares_sum(asked[cb]);
     }
+    const int k_begin = wave * k_per_wave, k_end = (k_begin + k_per_wave < k) ? k_begin + k_per_wave : k;
     for (int k0 = k_begin; k0 < k_end; k0 += 128) {
-      Frag8 a[R][4], b[MB][4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int kk = k0 + 32 * j + 8 * kq;
@@ -255,12 +276,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
 #pragma unroll
         for (int cb = 0; cb < MB; ++cb) b[cb][j].u = (in && xok[cb]) ? load16(xrow[cb] + kk) : zero16();
       }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int rt = 0; rt < R; ++rt)
-#pragma unroll
-          for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = mfma16(a[rt][j], b[cb][j], acc[rt][cb]);
+      multiply_stage();
     }
   }
 
@@ -275,32 +291,29 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
 
   // ---- partial sums of waves 1.. go through LDS to wave 0
   if (n_waves > 1) {
+    float* sq = red + (size_t)(n_waves - 1) * ACC * 256;
     if (wave > 0) {
-      float* dst = red + (size_t)(wave - 1) * ACCX * 64 + lane;
+      float* dst = red + (size_t)(wave - 1) * ACC * 256 + 4 * lane;
 #pragma unroll
       for (int rt = 0; rt < R; ++rt)
 #pragma unroll
-        for (int cb = 0; cb < MB; ++cb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) dst[((rt * MB + cb) * 4 + i) * 64] = acc[rt][cb][i];
+        for (int cb = 0; cb < MB; ++cb) *reinterpret_cast<f32x4_t*>(dst + (rt * MB + cb) * 256) = acc[rt][cb];
       if (SCALED) {
 #pragma unroll
-        for (int cb = 0; cb < MB; ++cb) dst[(ACC + cb) * 64] = ss[cb];
+        for (int cb = 0; cb < MB; ++cb) sq[((wave - 1) * MB + cb) * 64 + lane] = ss[cb];
       }
     }
     __syncthreads();
     if (wave == 0) {
       for (int ww = 0; ww < n_waves - 1; ++ww) {
-        const float* src = red + (size_t)ww * ACCX * 64 + lane;
+        const float* src = red + (size_t)ww * ACC * 256 + 4 * lane;
 #pragma unroll
         for (int rt = 0; rt < R; ++rt)
 #pragma unroll
-          for (int cb = 0; cb < MB; ++cb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[rt][cb][i] += src[((rt * MB + cb) * 4 + i) * 64];
+          for (int cb = 0; cb < MB; ++cb) acc[rt][cb] += *reinterpret_cast<const f32x4_t*>(src + (rt * MB + cb) * 256);
         if (SCALED) {
 #pragma unroll
-          for (int cb = 0; cb < MB; ++cb) ss[cb] += src[(ACC + cb) * 64];
+          for (int cb = 0; cb < MB; ++cb) ss[cb] += sq[(ww * MB + cb) * 64 + lane];
         }
       }
     }
@@ -324,7 +337,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
     for (int rt = 0; rt < R; ++rt)
 #pragma unroll
       for (int cb = 0; cb < MB; ++cb)
-        store_sums<EPI, TO>(c, acc[rt][cb], before[rt][cb], gain[rt], 16 * cb + r, n0 + 16 * rt + 4 * kq, m, n,
+        store_sums<EPI, true, TO>(c, acc[rt][cb], before[rt][cb], gain[rt], 16 * cb + r, n0 + 16 * rt + 4 * kq, m, n,
                             n0 / 16 + rt, kq, fa);
   } else {
     const int half_n = n / 2;
@@ -337,9 +350,16 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
         const int nn = n0 / 2 + 16 * (rt / 2) + 4 * kq;
         if (mm >= m) continue;
         TO* dst = c + (size_t)mm * half_n + nn;
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = gated_value(acc[rt][cb][i], acc[rt + 1][cb][i], gp);
+        if (sizeof(TO) == 2 && fa.wide) {                  // (n is a multiple of 32)
+          if (nn < half_n) *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+          continue;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (nn + i < half_n) Num<TO>::store(dst + i, gated_value(acc[rt][cb][i], acc[rt + 1][cb][i], gp));
+          if (nn + i < half_n) Num<TO>::store(dst + i, v[i]);
       }
   }
 }
@@ -350,19 +370,24 @@ extern "C" void rb_tune(int r, int waves) {       // experiments only; 0 = the b
   g_tune_waves = waves;
 }
 
-static FoldArgs fold_args(const GemmTokens& x, const GemmAfter& after) {
-  return FoldArgs{x.squares, x.rows, x.eps, after.gain, after.gained, after.squares, after.w_frag ? 1 : 0,
+static FoldArgs fold_args(const GemmTokens& x, const GemmAfter& after, const void* c, int n) {
+  const uintptr_t all = reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(after.gain) | reinterpret_cast<uintptr_t>(after.gained);
+  return FoldArgs{x.squares, x.rows, x.eps, after.gain, after.gained, after.squares, n % 4 == 0 && (all & 15) == 0 ? 1 : 0, after.w_frag ? 1 : 0,
                   after.epilogue <= 1 ? after.act : nullptr};
 }
 
-template <int MB, int R, int U, bool FAST, int EPI, typename TO, bool SCALED>
+template <int MB, int R, bool FAST, int EPI, typename TO, bool SCALED>
 static int launch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
                          int n_waves, int k_per_wave, hipStream_t s) {
   const size_t lds = (size_t)(n_waves - 1) * (R * MB * 4 + (SCALED ? MB : 0)) * 64 * sizeof(float);
   RB_REQUIRE(lds <= 64 * 1024, "rb_gemm_bf16: internal: reduction buffer of %zu bytes", lds);
   const int grid = (n + 16 * R - 1) / (16 * R);
-  gemm_skinny_kernel<MB, R, U, FAST, EPI, TO, SCALED>
-      <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, k_per_wave, fold_args(x, after));
+  if (MB == 1 && after.w_frag)
+    gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED>
+        <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, k_per_wave, fold_args(x, after, c, n));
+  else
+    gemm_skinny_kernel<MB, R, FAST, false, EPI, TO, SCALED>
+        <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, k_per_wave, fold_args(x, after, c, n));
   return 0;
 }
 
@@ -385,20 +410,20 @@ static int launch_skinny_u(const GemmTokens& x, const bf16_t* w, void* c, const 
     int nw = g_tune_waves ? g_tune_waves : ((k >= 8192 || wgs <= rb_compute_units() || max_waves < 4) ? max_waves : 4);
     if (nw > max_waves) nw = max_waves;
     if (nw > t) nw = t;
-    return launch_skinny<MB, R, 1, true, EPI, TO, SCALED>(x, w, c, after, m, n, k, nw, 0, s);
+    return launch_skinny<MB, R, true, EPI, TO, SCALED>(x, w, c, after, m, n, k, nw, 0, s);
   }
   int n_waves = k / 256;
   if (n_waves < 1) n_waves = 1;
   if (n_waves > max_waves) n_waves = max_waves;
   int k_per_wave = (k + n_waves - 1) / n_waves;
   k_per_wave = (k_per_wave + 127) / 128 * 128;
-  return launch_skinny<MB, R, 1, false, EPI, TO, SCALED>(x, w, c, after, m, n, k, n_waves, k_per_wave, s);
+  return launch_skinny<MB, R, false, EPI, TO, SCALED>(x, w, c, after, m, n, k, n_waves, k_per_wave, s);
 }
 
 template <int EPI, typename TO, bool SCALED>
 static int dispatch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
                            hipStream_t s) {
-  constexpr bool FOLDS = SCALED || EPI >= 2;      // compiled for up to 16 tokens only
+  constexpr bool FOLDS = SCALED || EPI == 2 || EPI == 3;      // compiled for up to 16 tokens only
   const int mb = (m + 15) / 16;
   RB_REQUIRE(!FOLDS || mb == 1, "rb_gemm_bf16: a product that folds its neighbours in takes at most 16 tokens, not %d",
              m);
@@ -589,14 +614,14 @@ __global__ __launch_bounds__(512) void gemm_resident_kernel(const bf16_t* __rest
         const int mm = 16 * cb + r;
         const int nn = tile * 16 + 4 * kq;
         f32x4_t before = (f32x4_t){0.f, 0.f, 0.f, 0.f}, gain = before;
-        if (EPI >= 2) {
+        if (EPI == 2 || EPI == 3) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             if (mm < m && nn + i < n) before[i] = Num<TO>::load(cpart + (size_t)mm * n + nn + i);
             if (EPI == 3 && nn + i < n) gain[i] = fa.gain[nn + i];
           }
         }
-        store_sums<EPI, TO>(cpart, acc[cb], before, gain, mm, nn, m, n, tile, kq, fa);
+        store_sums<EPI, EPI == 2 || EPI == 3, TO>(cpart, acc[cb], before, gain, mm, nn, m, n, tile, kq, fa);
       }
     } else if ((t & 1) == 0) {
 #pragma unroll
@@ -654,7 +679,7 @@ static int launch_resident(const GemmTokens& x, const bf16_t* w, void* c, const 
   const size_t lds = ((size_t)2 * (n_waves - 1) * MB * 4 * 64 + (SCALED ? n_waves * MB * 16 : 0)) * sizeof(float);
   dim3 grid((n_tiles + tiles - 1) / tiles, parts);
   gemm_resident_kernel<MB, XQ, EPI, TO, SCALED>
-      <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, tiles, fold_args(x, after));
+      <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, tiles, fold_args(x, after, c, n));
   return 0;
 }
 
@@ -662,7 +687,7 @@ static int launch_resident(const GemmTokens& x, const bf16_t* w, void* c, const 
 template <int EPI, typename TO, bool SCALED>
 static bool try_resident(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
                          int parts, hipStream_t s, int* rc) {
-  constexpr bool FOLDS = SCALED || EPI >= 2;      // compiled for up to 16 tokens and all of K in one workgroup
+  constexpr bool FOLDS = SCALED || EPI == 2 || EPI == 3;      // compiled for up to 16 tokens and all of K in one workgroup
   const int mb = (m + 15) / 16;
   const int xq = mb == 1 ? 16 : (mb == 2 ? 8 : 4);
   if (k % (32 * xq) != 0) return false;
@@ -694,7 +719,8 @@ static bool try_resident(const GemmTokens& x, const bf16_t* w, void* c, const Ge
 // One instance per (epilogue, output type, kind of tokens).  Epilogues 2 and 3 are float32 and
 // take plain tokens; prepared tokens go with epilogues 0 and 1.
 #define RB_PLAIN(FN, ...)                                                                                  \
-  (after.epilogue == 3 ? FN<3, float, false>(__VA_ARGS__)                                                  \
+  (after.epilogue == 0 && after.act ? (dtype_out == RB_F32 ? FN<EPI_ACT, float, false>(__VA_ARGS__) : FN<EPI_ACT, bf16_t, false>(__VA_ARGS__)) : \
+   after.epilogue == 3 ? FN<3, float, false>(__VA_ARGS__)                                                  \
    : after.epilogue == 2 ? FN<2, float, false>(__VA_ARGS__)                                                \
    : after.epilogue == 0 ? (dtype_out == RB_F32 ? FN<0, float, false>(__VA_ARGS__) : FN<0, bf16_t, false>(__VA_ARGS__)) \
                          : (dtype_out == RB_F32 ? FN<1, float, false>(__VA_ARGS__) : FN<1, bf16_t, false>(__VA_ARGS__)))
