@@ -1082,11 +1082,11 @@ template <int D>
 __global__ void attn_decode_combine_kernel(const float* __restrict__ ws, bf16_t* __restrict__ out, int n_splits,
                                            const float* __restrict__ sinks, int n_heads, int sum_only) {
   constexpr int AHEAD = 8;
-  __shared__ float factors[D / RB_WAVE][RB_WAVE];
+  __shared__ float2 factors[D / RB_WAVE][RB_WAVE];
   const size_t row = blockIdx.x;            // sequence * heads + head
   const int d = threadIdx.x, lane = threadIdx.x & (RB_WAVE - 1);
   const float* src = ws + row * n_splits * (D + 2);
-  float* mine = factors[threadIdx.x / RB_WAVE];      // every wave keeps its own, so that none waits for another
+  float2* mine = factors[threadIdx.x / RB_WAVE];     // every wave keeps its own, so that none waits for another
   float mx = -INFINITY;
   if (!sum_only) {
     for (int s = lane; s < n_splits; s += RB_WAVE) mx = fmaxf(mx, src[(size_t)s * (D + 2) + D]);
@@ -1096,13 +1096,10 @@ __global__ void attn_decode_combine_kernel(const float* __restrict__ ws, bf16_t*
   float a = 0.f, l = 0.f;
   for (int s0 = 0; s0 < n_splits; s0 += RB_WAVE) {
     const int here = n_splits - s0 < RB_WAVE ? n_splits - s0 : RB_WAVE;
-    float f = 1.f;
     if (!sum_only && lane < here) {
       const float* of = src + (size_t)(s0 + lane) * (D + 2);
-      f = exp2f(of[D] - m_safe);
-      l += of[D + 1] * f;
+      mine[lane] = make_float2(exp2f(of[D] - m_safe), of[D + 1]);      // this wave's alone; a wave's LDS accesses complete in order
     }
-    mine[lane] = f;                                   // this wave's alone; a wave's LDS accesses complete in order
     __builtin_amdgcn_wave_barrier();
     for (int s1 = 0; s1 < here; s1 += AHEAD) {
       float v[AHEAD];
@@ -1110,7 +1107,15 @@ __global__ void attn_decode_combine_kernel(const float* __restrict__ ws, bf16_t*
       for (int u = 0; u < AHEAD; ++u) v[u] = src[(size_t)(s0 + (s1 + u < here ? s1 + u : s1)) * (D + 2) + d];
 #pragma unroll
       for (int u = 0; u < AHEAD; ++u)
-        if (s1 + u < here) a = sum_only ? a + v[u] : fmaf(v[u], mine[s1 + u], a);
+        if (s1 + u < here) {                            // in the order of the splits
+          if (sum_only) {
+            a += v[u];
+          } else {
+            const float2 f = mine[s1 + u];
+            a = fmaf(v[u], f.x, a);
+            l = fmaf(f.y, f.x, l);
+          }
+        }
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -1118,7 +1123,6 @@ __global__ void attn_decode_combine_kernel(const float* __restrict__ ws, bf16_t*
     out[row * D + d] = f32_to_bf16(a);
     return;
   }
-  l = wave_sum(l);
   if (sinks) l += exp2f(fmaf(sinks[row % n_heads], LOG2E, -m_safe));          // the sink: in the denominator only
   out[row * D + d] = f32_to_bf16(l > 0.f ? a / l : 0.f);
 }

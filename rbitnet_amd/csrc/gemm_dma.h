@@ -83,8 +83,7 @@ __device__ __forceinline__ void store_piece(const f32x16_t& acc, TO* __restrict_
 //
 // GR: a product in groups (W [groups][N, K], one after another): the tokens' rows are sorted by group in runs padded to BM, so
 // that a tile of rows belongs to one group, tile_group[row tile] (-1: none).  GR 1: row r of the tiles is row row_pair[r] / top of x
-// (-1: any); c gets the rows in the tiles' order.  GR 2: x holds the rows in the tiles' order; c gets row r at row_pair[r].  GR 3: both
-// are in the tiles' order.
+// (-1: any); c gets the rows in the tiles' order.  GR 2: x holds the rows in the tiles' order; c gets row r at row_pair[r].
 struct GemmGroups {
   const int32_t* tile_group;
   const int32_t* row_pair;

@@ -2,8 +2,9 @@
 // are sorted by expert in runs padded to the tiles' rows (rb_route_choose_units), so that a tile of rows belongs to one expert, and
 // the tiles are those of the dense product with direct loads into LDS: the way up reads its rows where the tokens lie (a row of a
 // tile is any row of h) and leaves the units of the sorted rows; the way down writes every row to its pair's place.  Gated experts
-// keep their gate and up rows interleaved in blocks of 16, as the dense gated product does, and run its epilogue.  Where the
-// router's weights multiply the experts' inputs, the scaled rows are gathered first, in the tiles' order.
+// keep their gate and up rows interleaved in blocks of 16, as the dense gated product does, and run its epilogue.  (Where the
+// router's weights multiply the experts' inputs the rows would have to be gathered first, which costs what the tiles give: the whole
+// feed-forward below 792 us in routed.hip, 700 gathered, a step of four prompts no faster.)
 // Bound by the matrix cores; measured beside the kernels of routed.hip (a wave's operands straight from memory, 64 rows by 64
 // channels), 3,782 tokens by 4 of 16 experts, width 2,048, 2,048 units an expert: up
 // 410 -> 371 us, down 318 -> 225; 2,048 tokens at width 4,096 with 3,584 units 1,532 -> 1,069 us for the whole feed-forward.
@@ -30,29 +31,11 @@ static int launch_grouped(const bf16_t* x, const bf16_t* w, TO* c, int m_tiles, 
   return 0;
 }
 
-// The rows of the tiles: bf16(weight h[token]) of every pair, in the order of the runs; a row of padding keeps what it holds
-// (nobody stores what comes of it).  A workgroup four rows; bound by memory.
-__global__ __launch_bounds__(256) void gather_scaled_rows_kernel(const bf16_t* __restrict__ h, const float* __restrict__ weight, int top,
-                                                                 const int32_t* __restrict__ row_pair, bf16_t* __restrict__ xs, int width) {
-  const int row = blockIdx.x * 4 + threadIdx.x / RB_WAVE, lane = threadIdx.x & (RB_WAVE - 1);
-  const int p = row_pair[row];
-  if (p < 0) return;
-  const float wt = weight[p];
-  const bf16_t* src = h + (size_t)(p / top) * width;
-  bf16_t* dst = xs + (size_t)row * width;
-  for (int c = 8 * lane; c < width; c += 8 * RB_WAVE) {
-    const uint4 v = load16(src + c);
-    auto both = [&](uint32_t u) { return pack_bf16x2(bf16_bits_to_f32(u & 0xffffu) * wt, bf16_bits_to_f32(u >> 16) * wt); };
-    *reinterpret_cast<uint4*>(dst + c) = make_uint4(both(v.x), both(v.y), both(v.z), both(v.w));
-  }
-}
-
-extern "C" int rb_routed_experts_tiled(const void* h, int n_tokens, const float* weight, int top, const int32_t* row_pair,
-                                       const int32_t* tile_expert, int unit, int max_rows, int gated, const void* w_up,
-                                       const void* w_down, const float* act, void* xs, void* y, float* out, int n_experts, int width,
-                                       int ff, void* stream) {
-  RB_RECORDED(rb_routed_experts_tiled(h, n_tokens, weight, top, row_pair, tile_expert, unit, max_rows, gated, w_up, w_down, act, xs, y, out,
-                                      n_experts, width, ff, stream));
+extern "C" int rb_routed_experts_tiled(const void* h, int n_tokens, int top, const int32_t* row_pair, const int32_t* tile_expert, int unit,
+                                       int max_rows, int gated, const void* w_up, const void* w_down, const float* act, void* y, float* out,
+                                       int n_experts, int width, int ff, void* stream) {
+  RB_RECORDED(rb_routed_experts_tiled(h, n_tokens, top, row_pair, tile_expert, unit, max_rows, gated, w_up, w_down, act, y, out, n_experts,
+                                      width, ff, stream));
   RB_REQUIRE(n_tokens >= 0 && top > 0 && n_experts > 0 && width > 0 && ff > 0 && width % 64 == 0 && ff % 64 == 0,
              "rb_routed_experts_tiled: bad sizes T=%d top=%d experts=%d width=%d ff=%d (sizes are multiples of 64)", n_tokens, top, n_experts,
              width, ff);
@@ -62,9 +45,8 @@ extern "C" int rb_routed_experts_tiled(const void* h, int n_tokens, const float*
   RB_REQUIRE((long long)n_tokens * width * 2 < (1LL << 32) && 256LL * width * 2 < (1LL << 32) && 256LL * ff * 2 < (1LL << 32),
              "rb_routed_experts_tiled: %d tokens of %d numbers are too many", n_tokens, width);
   RB_REQUIRE(act != nullptr || gated, "rb_routed_experts_tiled: the units need their activation's numbers");
-  RB_REQUIRE(weight == nullptr || (gated && xs), "rb_routed_experts_tiled: scaled inputs go with gated experts and need room for the rows");
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  RB_REQUIRE(aligned(xs) && aligned(h) && aligned(w_up) && aligned(w_down) && aligned(y) && aligned(out), "rb_routed_experts_tiled: operands must be 16-byte aligned");
+  RB_REQUIRE(aligned(h) && aligned(w_up) && aligned(w_down) && aligned(y) && aligned(out), "rb_routed_experts_tiled: operands must be 16-byte aligned");
   if (n_tokens == 0 || max_rows == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const GemmGroups groups = {tile_expert, row_pair, top};
@@ -72,16 +54,11 @@ extern "C" int rb_routed_experts_tiled(const void* h, int n_tokens, const float*
   const bf16_t *x = (const bf16_t*)h, *wu = (const bf16_t*)w_up, *wd = (const bf16_t*)w_down;
   bf16_t* yb = (bf16_t*)y;
   int rc;
-  if (weight) {
-    gather_scaled_rows_kernel<<<max_rows / 4, 256, 0, s>>>(x, weight, top, row_pair, (bf16_t*)xs, width);
-    x = (const bf16_t*)xs;
-  }
-#define GR_GO(BN, BM, WN, WM, S)                                                                                               \
-  do {                                                                                                                         \
-    if (!gated) rc = launch_grouped<BN, BM, WN, WM, S, 1, bf16_t>(x, wu, yb, m_tiles, ff, width, act, groups, s);              \
-    else if (weight) rc = launch_grouped<BN, BM, WN, WM, S, 3, bf16_t, 1>(x, wu, yb, m_tiles, 2 * ff, width, act, groups, s);  \
-    else rc = launch_grouped<BN, BM, WN, WM, S, 1, bf16_t, 1>(x, wu, yb, m_tiles, 2 * ff, width, act, groups, s);              \
-    if (!rc) rc = launch_grouped<BN, BM, WN, WM, S, 2, float>(yb, wd, out, m_tiles, width, ff, nullptr, groups, s);            \
+#define GR_GO(BN, BM, WN, WM, S)                                                                                              \
+  do {                                                                                                                        \
+    if (gated) rc = launch_grouped<BN, BM, WN, WM, S, 1, bf16_t, 1>(x, wu, yb, m_tiles, 2 * ff, width, act, groups, s);       \
+    else rc = launch_grouped<BN, BM, WN, WM, S, 1, bf16_t>(x, wu, yb, m_tiles, ff, width, act, groups, s);                    \
+    if (!rc) rc = launch_grouped<BN, BM, WN, WM, S, 2, float>(yb, wd, out, m_tiles, width, ff, nullptr, groups, s);           \
   } while (0)
   if (unit == 256) GR_GO(256, 256, 128, 64, 2);
   else if (unit == 128) GR_GO(256, 128, 64, 64, 3);

@@ -217,7 +217,7 @@ class Kernels:
             "rb_lightning_chunks": [_P, _P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
             "rb_gated_rmsnorm_rows": [_P, _P, _P, _L, _I, _F, _P, _I, _I, _I, _P],
             "rb_route_choose_units": [_P, _L, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
-            "rb_routed_experts_tiled": [_P, _I, _P, _I, _P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+            "rb_routed_experts_tiled": [_P, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
             "rb_route_choose_bias": [_P, _L, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P],
             "rb_attention_mixed": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _I, _I, _P],
             "rb_attention_mixed_bf16": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _I, _I, _I, _P, _P],
@@ -962,13 +962,12 @@ class Kernels:
                                                  _ptr(correction), _ptr(sel), _ptr(weight), _ptr(row_pair), _ptr(tile_expert), max_rows,
                                                  int(unit), n, self._stream()))
 
-    def routed_experts_tiled(self, h: torch.Tensor, weight: Optional[torch.Tensor], top: int, row_pair: torch.Tensor, tile_expert: torch.Tensor,
-                             unit: int, w_up: torch.Tensor, w_down: torch.Tensor, gated: bool, act: Optional[torch.Tensor],
-                             xs: Optional[torch.Tensor], y: torch.Tensor, out: torch.Tensor) -> None:
+    def routed_experts_tiled(self, h: torch.Tensor, top: int, row_pair: torch.Tensor, tile_expert: torch.Tensor, unit: int,
+                             w_up: torch.Tensor, w_down: torch.Tensor, gated: bool, act: Optional[torch.Tensor], y: torch.Tensor,
+                             out: torch.Tensor) -> None:
         """Experts on the dense product's tiles for pairs sorted in runs padded to `unit` rows (64, 128, 256); bfloat16, fragment-major.
         Not gated: out[p] = Wd act(Wu h[p // top]), act float32 [2] as `xielu` takes it.  Gated: w_up [experts, 2 ff, width] holds gate
-        and up rows interleaved in blocks of 16, act None or float32 [2] = (limit, alpha); `weight` [pairs] then may scale the inputs,
-        with xs [rows, width] as scratch.  y [rows, ff] is scratch."""
+        and up rows interleaved in blocks of 16, act None or float32 [2] = (limit, alpha).  y [rows, ff] is scratch."""
         n, width = h.shape
         n_experts, _, ff = w_down.shape
         max_rows = row_pair.shape[0]
@@ -981,13 +980,10 @@ class Kernels:
         _check(w_down, "w_down", torch.bfloat16, (n_experts, width, ff))
         if act is not None or not gated:
             _check(act, "act", torch.float32, (2,))
-        if weight is not None:
-            _check(weight, "weight", torch.float32, (n * top,))
-            _check(xs, "xs", torch.bfloat16, (max_rows, width))
         _check(y, "y", torch.bfloat16, (max_rows, ff))
         _check(out, "out", torch.float32, (n * top, width))
-        self._ok(self._lib.rb_routed_experts_tiled(_ptr(h), n, _ptr(weight), top, _ptr(row_pair), _ptr(tile_expert), int(unit), max_rows,
-                                                   int(bool(gated)), _ptr(w_up), _ptr(w_down), _ptr(act), _ptr(xs), _ptr(y), _ptr(out),
+        self._ok(self._lib.rb_routed_experts_tiled(_ptr(h), n, top, _ptr(row_pair), _ptr(tile_expert), int(unit), max_rows,
+                                                   int(bool(gated)), _ptr(w_up), _ptr(w_down), _ptr(act), _ptr(y), _ptr(out),
                                                    n_experts, width, ff, self._stream()))
 
     def experts_combine(self, pairs: torch.Tensor, sel: torch.Tensor, weight: torch.Tensor, top: int, n_experts: int,

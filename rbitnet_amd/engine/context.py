@@ -217,10 +217,12 @@ class StepContext:
             self._workspaces[key] = (n_splits, ws)
         return self._workspaces[key]
 
-    def decode_workspace(self, n_heads: int, head_dim: int, n_kv_heads: int = 1) -> Tuple:
+    def decode_workspace(self, n_heads: int, head_dim: int, n_kv_heads: int = 1, spread: bool = False) -> Tuple:
         """Split count and scratch for decode attention: enough workgroups to fill the
-        GPU, whatever the context length (each split strides over the pages)."""
-        n_splits = decode_workgroups(self.n_seqs, n_kv_heads, self.bucket, self.n_compute_units)
+        GPU, whatever the context length (each split strides over the pages); `spread`: as many as `decode_workgroups` says, for
+        a walk over the whole context."""
+        count = decode_workgroups if spread else decode_splits
+        n_splits = count(self.n_seqs, n_kv_heads, self.bucket, self.n_compute_units)
         key = (n_heads, head_dim, n_kv_heads, n_splits)
         if key not in self._workspaces:
             ws = torch.empty(self.n_seqs * n_heads * n_splits * (head_dim + 2), dtype=torch.float32,

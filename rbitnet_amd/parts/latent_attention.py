@@ -172,7 +172,7 @@ class LatentAttention(Part):
         q3, pages = ql.view(t, self.heads, r), view.k_pages
         fast = dt == torch.bfloat16 and r in _MATRIX_CORE_RANKS and not getattr(self.env, "generic_only", False)
         if fast and ctx.max_q_len == 1:      # more than 16 heads on the latent run as several groups of at most 16
-            n_splits, workspace = ctx.decode_workspace(self.heads, r, 1)
+            n_splits, workspace = ctx.decode_workspace(self.heads, r, 1, spread=True)
             lib.attention_decode_bf16(q3, pages, pages, ol, ctx.tok_pos, view.block_table, self.heads, 1, r, self.scale, None,
                                       n_splits, workspace, sinks=self.sink)
         elif fast:

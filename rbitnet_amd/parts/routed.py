@@ -161,9 +161,9 @@ class RoutedExperts(Part):
                     lib.place_rows(tensors[self._name(i, what)].contiguous(), out[i], row0, GATE_BLOCK, 2 * GATE_BLOCK, frag=True)
             return out
 
-        # a step of many tokens runs on the dense product's tiles
+        # a step of many tokens runs on the dense product's tiles, where the tiles can read the tokens' rows as they are
         gated = self.unit == "gated"
-        self.tiled = bool(self.frag and (gated or self.weight_on == "output") and self.hidden % 64 == 0 and self.ff % 64 == 0)
+        self.tiled = bool(self.frag and self.weight_on == "output" and self.hidden % 64 == 0 and self.ff % 64 == 0)
         self.act = None
         if self.tiled and not gated:
             self.act = torch.tensor([float("nan"), 1.0], dtype=torch.float32, device=r.device)     # (see DenseAct)
@@ -189,7 +189,7 @@ class RoutedExperts(Part):
         weight = torch.empty(n_pairs, dtype=torch.float32, device=dev)
         row_pair = torch.empty(max_rows, dtype=torch.int32, device=dev)
         tile_expert = torch.empty(2 * (max_rows // unit), dtype=torch.int32, device=dev)      # experts, then positions in their runs
-        if self.plain and unit == 16:
+        if self.plain:
             lib.route_top(z, self.n_experts, self.top, sel, weight, row_pair, tile_expert)
         else:
             lib.route_choose(z, self.n_outputs, self.n_experts, self.top, self.score, self.correction, sel, weight, row_pair,
@@ -197,11 +197,9 @@ class RoutedExperts(Part):
         out = torch.empty((n_pairs, self.hidden), dtype=torch.float32, device=dev)
         if tiled:
             gated = self.w_gate is not None
-            scaled = weight if self.weight_on == "input" else None
             y = torch.empty((max_rows, self.ff), dtype=h.dtype, device=dev)
-            xs = torch.empty((max_rows, self.hidden), dtype=h.dtype, device=dev) if scaled is not None else None
-            lib.routed_experts_tiled(h, scaled, self.top, row_pair, tile_expert, unit, self.w_gate if gated else self.w_up, self.w_down,
-                                     gated, self.act, xs, y, out)
+            lib.routed_experts_tiled(h, self.top, row_pair, tile_expert, unit, self.w_gate if gated else self.w_up, self.w_down, gated,
+                                     self.act, y, out)
         else:
             y = torch.empty((max_rows, self.ff + self.hidden), dtype=h.dtype, device=dev)     # scratch: gated units, scaled inputs
             lib.routed_experts(h, weight if self.weight_on == "input" else None, self.top, row_pair, tile_expert, self.w_gate,

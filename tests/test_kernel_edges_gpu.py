@@ -189,8 +189,8 @@ def test_infinite_inputs_of_products_per_head(lib):
 # ---------------------------------------------------------------- gated experts on the dense product's tiles
 @pytest.mark.parametrize("tokens,top,experts,width,ff", [(112, 1, 1, 64, 64), (150, 2, 2, 128, 192), (131, 3, 3, 64, 320), (1600, 2, 2, 64, 64),
                                                          (700, 4, 16, 256, 128)])
-@pytest.mark.parametrize("weight_on,limit", [("input", 1.5), ("output", None), ("output", 2.0)])
-def test_gated_experts_on_tiles(lib, tokens, top, experts, width, ff, weight_on, limit):
+@pytest.mark.parametrize("limit", [None, 1.5])
+def test_gated_experts_on_tiles(lib, tokens, top, experts, width, ff, limit):
     from rbitnet_amd.parts.routed import tile_rows
     g = torch.Generator().manual_seed(tokens + ff)
     r = lambda *s, f=1.0: (torch.randn(*s, generator=g) * f).bfloat16()
@@ -208,15 +208,11 @@ def test_gated_experts_on_tiles(lib, tokens, top, experts, width, ff, weight_on,
         lib.place_rows(up[e].to(DEV), both[e], 16, 16, 32, frag=True)
         lib.place_rows(down[e].to(DEV), wd[e], frag=True)
     act = None if limit is None else torch.tensor([limit, 1.702], device=DEV)
-    scaled = weight if weight_on == "input" else None
-    xs = torch.full((rows, width), float("nan"), dtype=torch.bfloat16, device=DEV)
     y = torch.full((rows, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
     out = torch.full((tokens * top, width), float("nan"), device=DEV)
-    lib.routed_experts_tiled(h.to(DEV), scaled, top, row_pair, tile_expert, unit, both, wd, True, act, xs, y, out)
-    s, wt = sel.cpu().long(), weight.cpu()
+    lib.routed_experts_tiled(h.to(DEV), top, row_pair, tile_expert, unit, both, wd, True, act, y, out)
+    s = sel.cpu().long()
     x = h.double().repeat_interleave(top, 0)
-    if scaled is not None:
-        x = (h.float().repeat_interleave(top, 0) * wt[:, None]).bfloat16().double()
     for e in range(experts):
         at = torch.nonzero(s == e)[:, 0]
         a, b = x[at] @ gate[e].double().T, x[at] @ up[e].double().T
@@ -236,7 +232,7 @@ def test_gated_experts_on_tiles(lib, tokens, top, experts, width, ff, weight_on,
         lib.route_choose(z[:n].to(DEV), experts, experts, top, 0, None, sel2, weight2, row2, tile2)
         y2 = torch.empty((few_rows, ff + width), dtype=torch.bfloat16, device=DEV)
         out2 = torch.full((n * top, width), float("nan"), device=DEV)
-        lib.routed_experts(h[:n].to(DEV), weight2 if scaled is not None else None, top, row2, tile2, both, None, wd, y2, out2, limit or 0.0, 1.702,
+        lib.routed_experts(h[:n].to(DEV), None, top, row2, tile2, both, None, wd, y2, out2, limit or 0.0, 1.702,
                            w_frag=True)
         _within(out2, out[:n * top].double(), 0.05)
 
