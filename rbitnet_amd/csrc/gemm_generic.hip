@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const TI* __restrict_
   }
 }
 
-// Float32 operands and at most 16 tokens (the float32 path's decode step): bound by reading W
+// Float32 operands and at most 16 tokens, depths that the two kernels below do not take: bound by reading W
 // once.  A wave owns 4 rows of W and walks all of K with 16-byte loads (a row is read as
 // 1 KB contiguous per instruction); the tokens' 1024-deep chunk goes through LDS once for
 // the 4 waves; every lane keeps a partial sum per (row, token) and the wave adds them up at
@@ -141,6 +141,62 @@ __global__ __launch_bounds__(256) void gemm_f32_skinny_kernel(const float* __res
 // before is multiplied.  K is dealt to the waves of a workgroup in stages and their partial sums
 // meet in LDS in a fixed order.
 typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
+
+// At most 16 tokens and a depth of at most 1,024 that is no multiple of 128 (K a multiple of 4, W as rows): a launch that is
+// little more than its trips to memory.  Fragments as in the kernel below, a stage of 128 depth values per wave and trip, what lies
+// behind K counts as zeros.  Every one of a stage's 32 products has an accumulator of its own, and they meet as a tree: no chain
+// of dependent MFMAs, and an error like that of 64 lanes with a partial sum each (relative error at K = 96 / 500 / 1,000:
+// 7.1e-8 / 8.4e-8 / 9.1e-8; the kernel above 7.1e-8 / 8.5e-8 / 9.9e-8; one accumulator for all of them 1.7e-7 / 2.0e-7 / 2.9e-7).
+// 144 rows at K = 96, 4 / 16 tokens: 6.0 / 18.3 us in the kernel above, 3.0 / 3.1 here; 32,000 rows at K = 100 17.0 / 74.8 and 7.7 / 8.7.
+// Its loads take 64 bytes of a row, the kernel above 1 KB: with many rows and K > 128 that one is the better for few tokens (32,000 rows
+// at K = 500: 22.6 against 29.3 us with 4 tokens, 80 against 36 with 16; 4,096 rows at K = 1,000: 9.3 against 7.5).
+__global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ c,
+                                                            int m, int n, int k) {
+  extern __shared__ float red[];      // [waves - 1][4][64]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+  const int r = lane & 15, kq = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  // rows beyond N and tokens beyond M: row 0 and token 0, never stored
+  const float* wrow = w + (size_t)(n0 + r < n ? n0 + r : 0) * k + 4 * kq;
+  const float* xrow = x + (size_t)(r < m ? r : 0) * k + 4 * kq;
+  const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  gf_f32x4_t acc[8][4];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[j][i] = zero;
+  for (int ks = 128 * wave; ks < k; ks += 128 * n_waves) {
+    gf_f32x4_t a[8], b[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const bool in = ks + 16 * j + 4 * kq < k;
+      a[j] = in ? *reinterpret_cast<const gf_f32x4_t*>(wrow + ks + 16 * j) : zero;
+      b[j] = in ? *reinterpret_cast<const gf_f32x4_t*>(xrow + ks + 16 * j) : zero;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][i], b[j][i], acc[j][i], 0, 0, 0);
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j][0] = (acc[j][0] + acc[j][1]) + (acc[j][2] + acc[j][3]);
+  gf_f32x4_t sum = ((acc[0][0] + acc[1][0]) + (acc[2][0] + acc[3][0])) + ((acc[4][0] + acc[5][0]) + (acc[6][0] + acc[7][0]));
+  if (n_waves > 1) {
+    if (wave > 0)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[((wave - 1) * 4 + i) * 64 + lane] = sum[i];
+    __syncthreads();
+    if (wave > 0) return;
+    for (int o = 1; o < n_waves; ++o)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[i] += red[((o - 1) * 4 + i) * 64 + lane];
+  }
+  // lane l holds rows 4 (l / 16) + i of token l % 16
+  if (r < m)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (n0 + 4 * kq + i < n) c[(size_t)r * n + n0 + 4 * kq + i] = sum[i];
+}
 
 template <int MB, int R, bool WF>
 __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -412,6 +468,13 @@ extern "C" int rb_gemm_generic(const void* a, const void* w, int w_layout, void*
     if (mb == 1) launch_f32_few<1>(af, wf, w_frag, (float*)c, m, n, k, s);
     else if (mb == 2) launch_f32_few<2>(af, wf, w_frag, (float*)c, m, n, k, s);
     else launch_f32_few<4>(af, wf, w_frag, (float*)c, m, n, k, s);
+    RB_LAUNCH_CHECK();
+    return 0;
+  }
+  if (dtype_in == RB_F32 && dtype_out == RB_F32 && m <= 16 && k % 4 == 0 && k <= 1024 && (k <= 128 || m > 8 || (long long)n * k <= 1 << 22) && g_f32_few) {
+    const int n_waves = k <= 128 ? 1 : k <= 256 ? 2 : k <= 384 ? 3 : 4;
+    gemm_f32_short_kernel<<<(n + 15) / 16, 64 * n_waves, (size_t)(n_waves - 1) * 4 * 64 * sizeof(float), s>>>((const float*)a, (const float*)w,
+                                                                                                     (float*)c, m, n, k);
     RB_LAUNCH_CHECK();
     return 0;
   }

@@ -264,3 +264,24 @@ def test_single_token_attention_over_many_pages(lib, dim, heads, kv, length, spl
     _within(outs[0].view(want.shape), want, 2.0 ** -7 * float(v.abs().max()))
     for out in outs[1:]:
         assert torch.equal(out, outs[0])
+
+
+# ---------------------------------------------------------------- float32 products of few tokens, any depth
+@pytest.mark.parametrize("m", [1, 4, 16])
+@pytest.mark.parametrize("n,k", [(1, 4), (15, 12), (16, 20), (17, 96), (33, 124), (48, 132), (96, 252), (40, 260), (144, 500), (10, 516), (5, 1348)])
+@pytest.mark.parametrize("odd", [0, 1])
+def test_float32_products_of_few_tokens_and_any_depth(lib, m, n, k, odd):
+    """Depths around the stages of 128 and the four waves; operands also at addresses that are multiples of 4 bytes only; what lies behind
+    the operands is NaN."""
+    g = torch.Generator().manual_seed(m * 31 + n + k)
+    a, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
+
+    def placed(x):
+        room = torch.full((x.numel() + 260,), float("nan"), device=DEV)
+        room[odd:odd + x.numel()] = x.flatten().to(DEV)
+        return room[odd:odd + x.numel()].view(x.shape)
+
+    c = torch.full((m, n), float("nan"), device=DEV)
+    lib.gemm_generic(placed(a), placed(w), c)
+    # K products of 24 bits each, summed one after another: K 2^-24 of the sum of the absolute products at the most
+    _within(c, a.double() @ w.double().T, k * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 1e-30)
