@@ -23,17 +23,18 @@
 
 #define RT_TILE 16
 #define RT_MAX_EXPERTS 1024
+#define RT_FEW_TOKENS 32       // up to so many tokens the choice and the sort are one launch
 #define RT_FEW_MOST 64         // tokens of a step whose experts run in the kernels for few tokens
 
 // ---------------------------------------------------------------- route
 // score 0: sigmoid(z) of the chosen logit.  score 1: the softmax of z over all outputs; the choice then goes by the
 // softmax plus `correction` (null: nothing added), the weight is the softmax itself.  score 2: the choice goes by the logits,
 // the weights are the softmax over the chosen logits alone.  bias (null: none) is added to the logits before anything else.
+template <int PER>             // outputs a lane: 64 PER at the most
 __device__ void route_token(const float* __restrict__ z, size_t z_stride, int n_experts, int top, int score,
                             const float* __restrict__ bias, const float* __restrict__ correction, int32_t* __restrict__ sel,
                             float* __restrict__ weight, int t) {
   const int lane = threadIdx.x & (RB_WAVE - 1);
-  constexpr int PER = RT_MAX_EXPERTS / RB_WAVE;
   float v[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
@@ -113,11 +114,12 @@ __device__ void route_token(const float* __restrict__ z, size_t z_stride, int n_
   }
 }
 
+template <int PER>
 __global__ void route_kernel(const float* __restrict__ z, size_t z_stride, int n_experts, int top, int score,
                              const float* __restrict__ bias, const float* __restrict__ correction, int32_t* __restrict__ sel,
                              float* __restrict__ weight, int n_tokens) {
   const int t = blockIdx.x * (blockDim.x / RB_WAVE) + threadIdx.x / RB_WAVE;
-  if (t < n_tokens) route_token(z, z_stride, n_experts, top, score, bias, correction, sel, weight, t);
+  if (t < n_tokens) route_token<PER>(z, z_stride, n_experts, top, score, bias, correction, sel, weight, t);
 }
 
 // ---------------------------------------------------------------- sort (one workgroup)
@@ -164,10 +166,99 @@ __global__ __launch_bounds__(1024) void route_few_kernel(const float* __restrict
                                                          int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_pos, int max_rows,
                                                          int unit) {
   for (int t = threadIdx.x / RB_WAVE; t < n_tokens; t += blockDim.x / RB_WAVE)
-    route_token(z, z_stride, n_outputs, top, score, bias, correction, sel, weight, t);
+    route_token<RT_MAX_EXPERTS / RB_WAVE>(z, z_stride, n_outputs, top, score, bias, correction, sel, weight, t);
   __threadfence_block();
   __syncthreads();
   route_sort(sel, n_tokens * top, n_experts, row_pair, tile_expert, tile_pos, max_rows, unit);
+}
+
+// The same for at most 64 outputs, which are a lane's each.  A launch of one workgroup is nothing but its chain of trips: the choice is
+// every lane's rank among the lanes, from scalar reads of the lanes' values, instead of `top` reductions one after the other; the place of a
+// pair in its expert's run comes with the count; the runs' starts are a scan over the lanes instead of one thread's walk through
+// the experts.  The choices, the order of the sums and so the weights are those of route_token.  (4 tokens, 16 experts, 4 chosen, in a
+// graph: 7.6 us with route_few_kernel, 3.4 here; after a softmax 10.3 and 3.7.)
+__global__ __launch_bounds__(1024) void route_few_small_kernel(const float* __restrict__ z, size_t z_stride, int n_outputs, int n_experts,
+                                                               int top, int score, const float* __restrict__ bias,
+                                                               const float* __restrict__ correction, int32_t* __restrict__ sel,
+                                                               float* __restrict__ weight, int n_tokens, int32_t* __restrict__ row_pair,
+                                                               int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_pos,
+                                                               int max_rows, int unit) {
+  __shared__ int counts[RB_WAVE], start[RB_WAVE];
+  __shared__ int pair_at[RT_FEW_TOKENS * RB_WAVE];       // a pair's expert and its place in the expert's run: place * 64 + expert
+  const int lane = threadIdx.x & (RB_WAVE - 1);
+  if (threadIdx.x < RB_WAVE) counts[threadIdx.x] = 0;
+  __syncthreads();
+  for (int t = threadIdx.x / RB_WAVE; t < n_tokens; t += blockDim.x / RB_WAVE) {
+    float v = lane < n_outputs ? z[(size_t)t * z_stride + lane] + (bias ? bias[lane] : 0.f) : -INFINITY;
+    const float corr = score == 1 && correction && lane < n_outputs ? correction[lane] : 0.f;
+    if (v != v) v = -INFINITY;
+    float own = 0.f;
+    if (score == 1) {
+      const float m = wave_max(v);
+      own = v == -INFINITY ? 0.f : expf(v - m);
+      own = own / wave_sum(own);
+      if (lane < n_outputs) v = own + corr;
+      if (v != v) v = -INFINITY;
+    }
+    int rank;
+    if (__popcll(__ballot(v > -INFINITY)) >= top) {
+      rank = 0;
+      for (int o = 0; o < n_outputs; ++o) {
+        const float ov = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), o));
+        rank += (ov > v || (ov == v && o < lane)) ? 1 : 0;
+      }
+      if (lane >= n_outputs) rank = RB_WAVE;
+    } else {                  // fewer outputs than are to be chosen have a score: route_token says what is chosen then, some of them twice
+      route_token<1>(z, z_stride, n_outputs, top, score, bias, correction, sel, weight, t);
+      __threadfence_block();
+      for (int k = lane; k < top; k += RB_WAVE) {
+        const int e = sel[(size_t)t * top + k];
+        pair_at[t * top + k] = e < n_experts ? atomicAdd(&counts[e], 1) * RB_WAVE + e : -1;
+      }
+      continue;
+    }
+    float w = 0.f;
+    if (score == 2) {
+      const float first =
+          __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), __ffsll((long long)__ballot(rank == 0)) - 1));
+      const float mine = expf(v - first);
+      float chosen_sum = 0.f;
+      for (int k = 0; k < top; ++k)
+        chosen_sum +=
+            __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), __ffsll((long long)__ballot(rank == k)) - 1));
+      const float inv = chosen_sum > 0.f ? 1.0f / chosen_sum : 0.f;
+      w = inv > 0.f ? mine * inv : 1.0f / (float)top;
+    } else {
+      w = score == 1 ? own : 1.0f / (1.0f + expf(-v));
+    }
+    if (rank < top) {
+      sel[(size_t)t * top + rank] = lane;
+      weight[(size_t)t * top + rank] = w;
+      pair_at[t * top + rank] = lane < n_experts ? atomicAdd(&counts[lane], 1) * RB_WAVE + lane : -1;   // an output behind the experts has no run
+    }
+  }
+  for (int r = threadIdx.x; r < max_rows; r += blockDim.x) row_pair[r] = -1;
+  for (int i = threadIdx.x; i < max_rows / unit; i += blockDim.x) tile_expert[i] = -1;
+  __syncthreads();
+  if (threadIdx.x < RB_WAVE) {
+    const int tiles = lane < n_experts ? (counts[lane] + unit - 1) / unit : 0;
+    int upto = tiles;
+#pragma unroll
+    for (int o = 1; o < RB_WAVE; o <<= 1) {
+      const int below = __shfl_up(upto, o, RB_WAVE);
+      if (lane >= o) upto += below;
+    }
+    start[lane] = (upto - tiles) * unit;
+    for (int i = 0; i < tiles; ++i) {
+      tile_expert[upto - tiles + i] = lane;
+      tile_pos[upto - tiles + i] = i;                 // which tile of its expert's run
+    }
+  }
+  __syncthreads();
+  for (int p = threadIdx.x; p < n_tokens * top; p += blockDim.x) {
+    const int at = pair_at[p];
+    if (at >= 0) row_pair[start[at & (RB_WAVE - 1)] + at / RB_WAVE] = p;
+  }
 }
 
 extern "C" int rb_route_choose(const float* z, long long z_stride, int n_outputs, int n_experts, int top, int score,
@@ -177,7 +268,6 @@ extern "C" int rb_route_choose(const float* z, long long z_stride, int n_outputs
                               max_rows, n_tokens, stream);
 }
 
-#define RT_FEW_TOKENS 32       // up to so many tokens the choice and the sort are one launch
 extern "C" int rb_route_choose_bias(const float* z, long long z_stride, const float* bias, int n_outputs, int n_experts, int top,
                                     int score, const float* correction, int32_t* sel, float* weight, int32_t* row_pair,
                                     int32_t* tile_expert, int max_rows, int n_tokens, void* stream) {
@@ -203,13 +293,21 @@ extern "C" int rb_route_choose_units(const float* z, long long z_stride, const f
              "rb_route_choose: room for %d rows, %lld pairs of %d experts may need more", max_rows, pairs, n_experts);
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
+  if (n_tokens <= RT_FEW_TOKENS && n_outputs <= RB_WAVE) {
+    const int waves = n_tokens < 4 ? 4 : n_tokens < 16 ? n_tokens : 16;
+    route_few_small_kernel<<<1, RB_WAVE * waves, 0, s>>>(z, (size_t)z_stride, n_outputs, n_experts, top, score, bias, correction, sel, weight,
+                                                         n_tokens, row_pair, tile_expert, tile_expert + max_rows / unit, max_rows, unit);
+    RB_LAUNCH_CHECK();
+    return 0;
+  }
   if (n_tokens <= RT_FEW_TOKENS) {
     route_few_kernel<<<1, 1024, 0, s>>>(z, (size_t)z_stride, n_outputs, n_experts, top, score, bias, correction, sel, weight, n_tokens,
                                         row_pair, tile_expert, tile_expert + max_rows / unit, max_rows, unit);
     RB_LAUNCH_CHECK();
     return 0;
   }
-  route_kernel<<<(n_tokens + 3) / 4, 256, 0, s>>>(z, (size_t)z_stride, n_outputs, top, score, bias, correction, sel, weight, n_tokens);
+  (n_outputs <= RB_WAVE ? route_kernel<1> : route_kernel<RT_MAX_EXPERTS / RB_WAVE>)<<<(n_tokens + 3) / 4, 256, 0, s>>>(
+      z, (size_t)z_stride, n_outputs, top, score, bias, correction, sel, weight, n_tokens);
   route_sort_kernel<<<1, 1024, 0, s>>>(sel, (int)pairs, n_experts, row_pair, tile_expert, tile_expert + max_rows / unit, max_rows, unit);
   RB_LAUNCH_CHECK();
   return 0;
@@ -329,18 +427,48 @@ __global__ __launch_bounds__(256) void routed_gather_kernel(const bf16_t* __rest
 // many loads are on their way: a wave takes 16 channels (gate and up) or 16 of the model's channels (down) for all of the
 // run's tiles, walks the depth alone, in the order of the kernels below (so that a row's sums are the same bits), and asks for
 // RT_AHEAD steps at once, the experts' matrices past the caches.  The rows are read where they lie (no gathered copy).
+// A workgroup is one wave: with four waves to a workgroup the 350 of a step of 4 tokens by 4 of 16 experts fell on 256 compute units as
+// one or two each, and the busiest had half as much again as the mean.  In steps of at most 16 tokens the next RT_AHEAD steps are
+// asked for before the last are multiplied, so that a wave's queue is never empty.  4 tokens by 4 of 16 experts, width and units
+// 2,048: up 19.5 us before, 16.2 now, with gates 33.5 and 31.3, down 20 and 16.7, which is 5.5 TB/s of the experts that were chosen.
 #define RT_AHEAD 8
+// The steps of depth, RT_AHEAD at a time; TWICE: the next ones are asked for before those that have come are multiplied.
+template <bool TWICE, typename Ahead, typename Load, typename Multiply>
+__device__ __forceinline__ void walk_ahead(int n_steps, const Load& load, const Multiply& multiply) {
+  Ahead a;
+  const int whole = n_steps / RT_AHEAD * RT_AHEAD;
+  if (TWICE) {
+    Ahead b;
+    if (whole) load(a, 0, RT_AHEAD);
+    for (int s0 = 0; s0 < whole; s0 += 2 * RT_AHEAD) {
+      const bool second = s0 + RT_AHEAD < whole;
+      if (second) load(b, s0 + RT_AHEAD, RT_AHEAD);
+      multiply(a, RT_AHEAD);
+      if (s0 + 2 * RT_AHEAD < whole) load(a, s0 + 2 * RT_AHEAD, RT_AHEAD);
+      if (second) multiply(b, RT_AHEAD);
+    }
+  } else {
+    for (int s0 = 0; s0 < whole; s0 += RT_AHEAD) {
+      load(a, s0, RT_AHEAD);
+      multiply(a, RT_AHEAD);
+    }
+  }
+  if (whole < n_steps) {
+    load(a, whole, n_steps - whole);
+    multiply(a, n_steps - whole);
+  }
+}
+
 template <int NT, bool WEIGHTED, bool GATED>
-__global__ __launch_bounds__(256) void routed_up_few_kernel(const bf16_t* __restrict__ h, const float* __restrict__ weight, int top,
+__global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __restrict__ h, const float* __restrict__ weight, int top,
                                                             const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
                                                             const int32_t* __restrict__ tile_pos, const bf16_t* __restrict__ w_gate,
                                                             const bf16_t* __restrict__ w_up, bf16_t* __restrict__ y, int width, int ff,
                                                             float limit, float alpha, int n_tiles, int rows) {
   const int t0 = blockIdx.y, e = tile_expert[t0];
   if (e < 0 || tile_pos[t0] % NT != 0) return;
-  const int lane = threadIdx.x & (RB_WAVE - 1), wave = threadIdx.x / RB_WAVE;
-  const int c0 = (blockIdx.x * 4 + wave) * 16;
-  if (c0 >= ff) return;
+  const int lane = threadIdx.x;
+  const int c0 = blockIdx.x * 16;
   int nt = 1;
   while (nt < NT && t0 + nt < n_tiles && tile_expert[t0 + nt] == e) ++nt;
   const int r = lane & 15, grp = lane >> 4;
@@ -360,31 +488,34 @@ __global__ __launch_bounds__(256) void routed_up_few_kernel(const bf16_t* __rest
 #pragma unroll
   for (int j = 0; j < NT; ++j) ag[j] = au[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int n_steps = width / 32;
-  auto steps = [&](int s0, int cnt) {
-    Frag8 fg[RT_AHEAD], fu[RT_AHEAD], fx[RT_AHEAD][NT];
+  struct Ahead {
+    Frag8 g[GATED ? RT_AHEAD : 1], u[RT_AHEAD], x[RT_AHEAD][NT];
+  };
+  auto load = [&](Ahead& f, int s0, int cnt) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < RT_AHEAD; ++u) {
       const size_t s = (size_t)(s0 + (u < cnt ? u : 0));
-      if (GATED) fg[u].u = load16_stream(gr + 512 * s);
-      fu[u].u = load16_stream(ur + 512 * s);
+      if (GATED) f.g[u].u = load16_stream(gr + 512 * s);
+      f.u[u].u = load16_stream(ur + 512 * s);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) fx[u][j].u = load16(xr[j] + 32 * s);
+      for (int j = 0; j < NT; ++j) f.x[u][j].u = load16(xr[j] + 32 * s);
     }
-    __builtin_amdgcn_sched_barrier(0);            // all of them are on their way before the first is waited for
+    __builtin_amdgcn_sched_barrier(0);            // all of them are on their way before anything is waited for
+  };
+  auto multiply = [&](Ahead& f, int cnt) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < RT_AHEAD; ++u) {
       if (u >= cnt) break;
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        if (WEIGHTED) fx[u][j].u = scaled16(fx[u][j].u, wt[j]);
-        if (GATED) ag[j] = mfma16(fg[u], fx[u][j], ag[j]);
-        au[j] = mfma16(fu[u], fx[u][j], au[j]);
+        if (WEIGHTED) f.x[u][j].u = scaled16(f.x[u][j].u, wt[j]);
+        if (GATED) ag[j] = mfma16(f.g[u], f.x[u][j], ag[j]);
+        au[j] = mfma16(f.u[u], f.x[u][j], au[j]);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  int s0 = 0;
-  for (; s0 + RT_AHEAD <= n_steps; s0 += RT_AHEAD) steps(s0, RT_AHEAD);
-  if (s0 < n_steps) steps(s0, n_steps - s0);
+  walk_ahead<NT == 1, Ahead>(n_steps, load, multiply);
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     if (!on[j]) continue;
@@ -398,15 +529,14 @@ __global__ __launch_bounds__(256) void routed_up_few_kernel(const bf16_t* __rest
 }
 
 template <int NT>
-__global__ __launch_bounds__(256) void routed_down_few_kernel(const bf16_t* __restrict__ y, const int32_t* __restrict__ row_pair,
+__global__ __launch_bounds__(RB_WAVE) void routed_down_few_kernel(const bf16_t* __restrict__ y, const int32_t* __restrict__ row_pair,
                                                               const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_pos,
                                                               const bf16_t* __restrict__ w_down, float* __restrict__ out, int width, int ff,
                                                               int n_tiles) {
   const int t0 = blockIdx.y, e = tile_expert[t0];
   if (e < 0 || tile_pos[t0] % NT != 0) return;
-  const int lane = threadIdx.x & (RB_WAVE - 1), wave = threadIdx.x / RB_WAVE;
-  const int c0 = (blockIdx.x * 4 + wave) * 16;
-  if (c0 >= width) return;
+  const int lane = threadIdx.x;
+  const int c0 = blockIdx.x * 16;
   int nt = 1;
   while (nt < NT && t0 + nt < n_tiles && tile_expert[t0 + nt] == e) ++nt;
   const int r = lane & 15, grp = lane >> 4;
@@ -419,26 +549,29 @@ __global__ __launch_bounds__(256) void routed_down_few_kernel(const bf16_t* __re
 #pragma unroll
   for (int j = 0; j < NT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int n_steps = ff / 32;
-  auto steps = [&](int s0, int cnt) {
-    Frag8 fd[RT_AHEAD], fy[RT_AHEAD][NT];
+  struct Ahead {
+    Frag8 d[RT_AHEAD], y[RT_AHEAD][NT];
+  };
+  auto load = [&](Ahead& f, int s0, int cnt) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < RT_AHEAD; ++u) {
       const size_t s = (size_t)(s0 + (u < cnt ? u : 0));
-      fd[u].u = load16_stream(dr + 512 * s);
+      f.d[u].u = load16_stream(dr + 512 * s);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) fy[u][j].u = load16(yr + (size_t)(j < nt ? j : 0) * RT_TILE * ff + 512 * s);
+      for (int j = 0; j < NT; ++j) f.y[u][j].u = load16(yr + (size_t)(j < nt ? j : 0) * RT_TILE * ff + 512 * s);
     }
     __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](Ahead& f, int cnt) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < RT_AHEAD; ++u) {
       if (u >= cnt) break;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j] = mfma16(fd[u], fy[u][j], acc[j]);
+      for (int j = 0; j < NT; ++j) acc[j] = mfma16(f.d[u], f.y[u][j], acc[j]);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  int s0 = 0;
-  for (; s0 + RT_AHEAD <= n_steps; s0 += RT_AHEAD) steps(s0, RT_AHEAD);
-  if (s0 < n_steps) steps(s0, n_steps - s0);
+  walk_ahead<NT == 1, Ahead>(n_steps, load, multiply);
 #pragma unroll
   for (int j = 0; j < NT; ++j)
     if (pair[j] >= 0)
@@ -651,12 +784,12 @@ extern "C" int rb_routed_experts_few(const void* h, const float* weight, int top
   if (max_rows == 0 || n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const int tiles = max_rows / RT_TILE;
-  const dim3 gu((ff + 63) / 64, tiles), gd((width + 63) / 64, tiles);
+  const dim3 gu(ff / 16, tiles), gd(width / 16, tiles);      // (both are multiples of 32)
 #define RT_UP(NT, WEIGHTED)                                                                                                           \
-  (w_gate ? routed_up_few_kernel<NT, WEIGHTED, true> : routed_up_few_kernel<NT, WEIGHTED, false>)<<<gu, 256, 0, s>>>((const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles,    \
+  (w_gate ? routed_up_few_kernel<NT, WEIGHTED, true> : routed_up_few_kernel<NT, WEIGHTED, false>)<<<gu, RB_WAVE, 0, s>>>((const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles,    \
                                                         (const bf16_t*)w_gate, (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha, tiles, rows)
 #define RT_DOWN(NT)                                                                                                       \
-  routed_down_few_kernel<NT><<<gd, 256, 0, s>>>((const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles,             \
+  routed_down_few_kernel<NT><<<gd, RB_WAVE, 0, s>>>((const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles,             \
                                                 (const bf16_t*)w_down, out, width, ff, tiles)
   if (n_tokens <= RT_TILE) {                  // a token chooses an expert once: no run is longer than the step's tokens
     if (weight) RT_UP(1, true);

@@ -285,3 +285,47 @@ def test_float32_products_of_few_tokens_and_any_depth(lib, m, n, k, odd):
     lib.gemm_generic(placed(a), placed(w), c)
     # K products of 24 bits each, summed one after another: K 2^-24 of the sum of the absolute products at the most
     _within(c, a.double() @ w.double().T, k * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T) + 1e-30)
+
+
+# ---------------------------------------------------------------- the choice and the sort of a step of few tokens
+@pytest.mark.parametrize("tokens", [1, 5, 17, 32])
+@pytest.mark.parametrize("outputs,experts,top", [(1, 1, 1), (16, 16, 4), (20, 16, 3), (64, 64, 8), (64, 60, 64), (63, 63, 1), (8, 0, 2)])
+@pytest.mark.parametrize("score", [0, 1, 2])
+@pytest.mark.parametrize("extra", [False, True])
+def test_choice_of_a_step_of_few_tokens(lib, tokens, outputs, experts, top, score, extra):
+    """One launch of a rank per lane chooses and weighs, bit for bit, as the launch for many tokens does, which 40 tokens take: with ties,
+    both zeros, infinities, NaN, and rows in which fewer outputs than are chosen have a score; and every pair has its row."""
+    g = torch.Generator().manual_seed(tokens * 100 + outputs + score)
+    z = torch.randn(40, outputs + 3, generator=g)
+    z[1::4] = z[1::4].round()                                   # ties
+    z[2::8] = torch.where(torch.rand(z[2::8].shape, generator=g) < 0.7, torch.tensor(-float("inf")), z[2::8])
+    z[3::8, ::3] = float("nan")
+    z[5] = -0.0
+    z[6, outputs // 2] = float("inf")
+    z[7] = -float("inf")
+    z[0, :] = torch.where(torch.rand(z[0].shape, generator=g) < 0.3, torch.tensor(torch.finfo(torch.float32).min), z[0])
+    z = z.to(DEV)
+    bias = torch.randn(outputs, generator=g).to(DEV) if extra else None
+    correction = torch.randn(outputs, generator=g).to(DEV) if extra and score == 1 else None
+    res = []
+    for n in (tokens, 40):
+        rows = lib.routed_rows(n, top, experts, 16)
+        sel, weight = torch.full((n * top,), -7, dtype=torch.int32, device=DEV), torch.full((n * top,), -7.0, device=DEV)
+        pair, tile = torch.full((rows,), -7, dtype=torch.int32, device=DEV), torch.full((2 * (rows // 16),), -7, dtype=torch.int32, device=DEV)
+        lib.route_choose(z[:n], outputs, experts, top, score, correction, sel, weight, pair, tile, bias=bias)
+        res.append((sel.cpu(), weight.cpu(), pair.cpu(), tile.cpu()))
+    few, many = res
+    assert torch.equal(few[0], many[0][:tokens * top])
+    assert torch.equal(few[1].view(torch.int32), many[1][:tokens * top].view(torch.int32))
+    sel, _, pair, tile = few
+    runs = pair.view(-1, 16)
+    expert, position = tile.view(2, -1)
+    at = 0
+    for e in range(experts):
+        wanted = (sel == e).nonzero().flatten().tolist()
+        n_tiles = (len(wanted) + 15) // 16
+        got = runs[at:at + n_tiles].flatten().tolist()
+        assert sorted(p for p in got if p >= 0) == wanted and expert[at:at + n_tiles].tolist() == [e] * n_tiles
+        assert got[len(wanted):] == [-1] * (16 * n_tiles - len(wanted)) and position[at:at + n_tiles].tolist() == list(range(n_tiles))
+        at += n_tiles
+    assert (runs[at:] == -1).all() and (expert[at:] == -1).all()
