@@ -89,53 +89,51 @@ __device__ __forceinline__ void st4(bf16_t* p, float a, float b, float c, float 
   *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
 }
 
-template <typename TO>
+// NS: the number of copies where it is known (0: up to ST_MAX_STREAMS, with a test at each); ONE: a thread has four values of its row and no
+// more, which stay in registers.  A step of few tokens pays for every barrier and for code that comes from memory: the copies'
+// coefficients are scalar loads, and the two reductions have scratch of their own.  (4 rows of 2,048, four copies updated: 7.2 us for any
+// number of copies by way of LDS, 3.8 here, one copy 5.5 and 3.3; 3,781 rows: four copies 70 and 44, one 46 and 21.)
+template <typename TO, int NS, bool ONE>
 __global__ __launch_bounds__(1024) void streams_layernorm_vec_kernel(
-    float* __restrict__ x, int n_streams, size_t stream_stride, const float* __restrict__ coef, const float* __restrict__ delta,
+    float* __restrict__ x, int n_copies, size_t stream_stride, const float* __restrict__ coef, const float* __restrict__ delta,
     const float* __restrict__ weight, const float* __restrict__ bias, float eps, const int32_t* __restrict__ rows, int width,
     TO* __restrict__ out, const float* __restrict__ mix, const float* __restrict__ out_coef, const float* __restrict__ y,
     const float* __restrict__ scale, const float* __restrict__ delta2, float dscale) {
   extern __shared__ float u[];
-  __shared__ float scratch[16];
-  __shared__ float c_mix[ST_MAX_STREAMS * ST_MAX_STREAMS], c_out[ST_MAX_STREAMS], c_in[ST_MAX_STREAMS];
+  __shared__ float sums[2][16];
+  constexpr int MOST = NS > 0 ? NS : ST_MAX_STREAMS;
+  const int n_streams = NS > 0 ? NS : n_copies;
   const int r = blockIdx.x;
   const size_t src = rows ? (size_t)rows[r] : (size_t)r;
   const bool write_back = delta != nullptr && rows == nullptr && n_streams == 1;
-  if ((int)threadIdx.x < n_streams) {
-    c_in[threadIdx.x] = coef ? coef[threadIdx.x] : 1.0f;
-    if (mix) c_out[threadIdx.x] = out_coef[threadIdx.x];
-  }
-  if (mix && (int)threadIdx.x < n_streams * n_streams) c_mix[threadIdx.x] = mix[threadIdx.x];
-  __syncthreads();
-  float sum = 0.f;
-  for (int j = 4 * threadIdx.x; j < width; j += 4 * blockDim.x) {
+  auto value = [&](int j) {
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (mix) {
-      float4 old[ST_MAX_STREAMS];
+    float4 old[MOST];
 #pragma unroll
-      for (int s = 0; s < ST_MAX_STREAMS; ++s)
-        if (s < n_streams) old[s] = ld4(x + (size_t)s * stream_stride + src * width + j);
+    for (int s = 0; s < MOST; ++s)
+      if (s < n_streams) old[s] = ld4(x + (size_t)s * stream_stride + src * width + j);
+    if (mix) {
       float4 yv = ld4(y + src * width + j);
       if (scale) {
         const float4 sc = ld4(scale + j);
         yv = make_float4(yv.x * sc.x, yv.y * sc.y, yv.z * sc.z, yv.w * sc.w);
       }
 #pragma unroll
-      for (int k = 0; k < ST_MAX_STREAMS; ++k) {
+      for (int k = 0; k < MOST; ++k) {
         if (k < n_streams) {
-          const float oc = c_out[k];
+          const float oc = out_coef[k], ic = coef ? coef[k] : 1.0f;
           float4 nv = make_float4(oc * yv.x, oc * yv.y, oc * yv.z, oc * yv.w);
 #pragma unroll
-          for (int s = 0; s < ST_MAX_STREAMS; ++s)
-            if (s < n_streams) nv = fma4(c_mix[s * n_streams + k], old[s], nv);
+          for (int s = 0; s < MOST; ++s)
+            if (s < n_streams) nv = fma4(mix[s * n_streams + k], old[s], nv);
           *reinterpret_cast<float4*>(x + (size_t)k * stream_stride + src * width + j) = nv;
-          v = fma4(c_in[k], nv, v);
+          v = fma4(ic, nv, v);
         }
       }
     } else {
 #pragma unroll
-      for (int s = 0; s < ST_MAX_STREAMS; ++s)
-        if (s < n_streams) v = fma4(c_in[s], ld4(x + (size_t)s * stream_stride + src * width + j), v);
+      for (int s = 0; s < MOST; ++s)
+        if (s < n_streams) v = fma4(coef ? coef[s] : 1.0f, old[s], v);
     }
     if (delta) {
       float4 d = ld4(delta + src * width + j);
@@ -146,28 +144,51 @@ __global__ __launch_bounds__(1024) void streams_layernorm_vec_kernel(
       v = fma4(dscale, d, v);
     }
     if (write_back) *reinterpret_cast<float4*>(x + src * width + j) = v;
-    *reinterpret_cast<float4*>(u + j) = v;
-    sum += (v.x + v.y) + (v.z + v.w);
+    return v;
+  };
+  // the sum over the workgroup, in block_sum's order
+  auto total = [&](float part, float* scratch) {
+    part = wave_sum(part);
+    if ((threadIdx.x & (RB_WAVE - 1)) == 0) scratch[threadIdx.x / RB_WAVE] = part;
+    __syncthreads();
+    float t = 0.f;
+    for (int i = 0; i < (int)(blockDim.x / RB_WAVE); ++i) t += scratch[i];
+    return t;
+  };
+  const int j0 = 4 * threadIdx.x;
+  float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f);
+  float sum = 0.f;
+  if (ONE) {
+    if (j0 < width) {
+      v0 = value(j0);
+      sum += (v0.x + v0.y) + (v0.z + v0.w);
+    }
+  } else {
+    for (int j = j0; j < width; j += 4 * blockDim.x) {
+      const float4 v = value(j);
+      *reinterpret_cast<float4*>(u + j) = v;
+      sum += (v.x + v.y) + (v.z + v.w);
+    }
   }
   // weight and bias of this thread's first values are asked for now, so that they arrive under the two reductions
-  const int j0 = 4 * threadIdx.x;
   float4 w0 = make_float4(0.f, 0.f, 0.f, 0.f), b0 = w0;
   if (j0 < width) {
     w0 = ld4(weight + j0);
     if (bias) b0 = ld4(bias + j0);
   }
   __builtin_amdgcn_sched_barrier(0);
-  const float mean = block_sum(sum, scratch) / (float)width;
+  const float mean = total(sum, sums[0]) / (float)width;
   float ss = 0.f;
-  for (int j = 4 * threadIdx.x; j < width; j += 4 * blockDim.x) {
-    const float4 v = *reinterpret_cast<const float4*>(u + j);
+  for (int j = j0; j < width; j += 4 * blockDim.x) {
+    const float4 v = ONE ? v0 : *reinterpret_cast<const float4*>(u + j);
     const float a = v.x - mean, b = v.y - mean, c = v.z - mean, d = v.w - mean;
     ss += (a * a + b * b) + (c * c + d * d);
+    if (ONE) break;
   }
-  const float f = 1.0f / sqrtf(block_sum(ss, scratch) / (float)width + eps);
+  const float f = 1.0f / sqrtf(total(ss, sums[1]) / (float)width + eps);
   TO* orow = out + (size_t)r * width;
-  for (int j = 4 * threadIdx.x; j < width; j += 4 * blockDim.x) {
-    const float4 v = *reinterpret_cast<const float4*>(u + j);
+  for (int j = j0; j < width; j += 4 * blockDim.x) {
+    const float4 v = ONE ? v0 : *reinterpret_cast<const float4*>(u + j);
     const float4 wv = j == j0 ? w0 : ld4(weight + j);
     float4 o = make_float4((v.x - mean) * f * wv.x, (v.y - mean) * f * wv.y, (v.z - mean) * f * wv.z, (v.w - mean) * f * wv.w);
     if (bias) {
@@ -175,6 +196,7 @@ __global__ __launch_bounds__(1024) void streams_layernorm_vec_kernel(
       o = make_float4(o.x + bv.x, o.y + bv.y, o.z + bv.z, o.w + bv.w);
     }
     st4(orow + j, o.x, o.y, o.z, o.w);
+    if (ONE) break;
   }
 }
 
@@ -233,12 +255,21 @@ static int layernorm_launch(float* x, int n_streams, long long stream_stride, co
       aligned(y) && aligned(scale) && (out_dtype == RB_F32 || out_dtype == RB_BF16)) {
     int threads = ((width / 4 + RB_WAVE - 1) / RB_WAVE) * RB_WAVE;
     if (threads > 1024) threads = 1024;
-    if (out_dtype == RB_F32)
-      streams_layernorm_vec_kernel<float><<<n_rows, threads, lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight, bias,
-                                                                       eps, rows, width, (float*)out, mix, out_coef, y, scale, delta2, dscale);
-    else
-      streams_layernorm_vec_kernel<bf16_t><<<n_rows, threads, lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight,
-                                                                        bias, eps, rows, width, (bf16_t*)out, mix, out_coef, y, scale, delta2, dscale);
+#define ST_GO(TO, NS, ONE)                                                                                                              \
+  streams_layernorm_vec_kernel<TO, NS, ONE><<<n_rows, threads, (ONE) ? 0 : lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight, bias, \
+                                                                                    eps, rows, width, (TO*)out, mix, out_coef, y, scale, delta2, dscale)
+#define ST_BY_COPIES(TO)                                \
+  do {                                                  \
+    if (width > 4 * threads) ST_GO(TO, 0, false);       \
+    else if (n_streams == 1) ST_GO(TO, 1, true);        \
+    else if (n_streams == 2) ST_GO(TO, 2, true);        \
+    else if (n_streams == 4) ST_GO(TO, 4, true);        \
+    else ST_GO(TO, 0, true);                            \
+  } while (0)
+    if (out_dtype == RB_F32) ST_BY_COPIES(float);
+    else ST_BY_COPIES(bf16_t);
+#undef ST_BY_COPIES
+#undef ST_GO
     RB_LAUNCH_CHECK();
     return 0;
   }

@@ -329,3 +329,42 @@ def test_choice_of_a_step_of_few_tokens(lib, tokens, outputs, experts, top, scor
         assert got[len(wanted):] == [-1] * (16 * n_tiles - len(wanted)) and position[at:at + n_tiles].tolist() == list(range(n_tiles))
         at += n_tiles
     assert (runs[at:] == -1).all() and (expert[at:] == -1).all()
+
+
+# ---------------------------------------------------------------- layer norm over copies of the stream
+@pytest.mark.parametrize("copies", [1, 2, 3, 4, 7])
+@pytest.mark.parametrize("width", [4, 252, 2048, 4096, 4100, 9000])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["plain", "rows", "update"])
+def test_layernorm_over_copies(lib, copies, width, dtype, kind):
+    """One row of values a thread and several; every number of copies that has a kernel of its own and some that have none."""
+    g = torch.Generator().manual_seed(copies * width)
+    n, eps = 5, 1e-5
+    x, weight, bias = torch.randn(copies, n, width, generator=g), torch.randn(width, generator=g), torch.randn(width, generator=g)
+    coef, mix = torch.randn(copies, generator=g), torch.randn(copies, copies, generator=g)
+    out_coef, y, scale, delta = torch.randn(copies, generator=g), torch.randn(n, width, generator=g), torch.randn(width, generator=g), torch.randn(n, width, generator=g)
+    d = [t.to(DEV) for t in (x, coef, weight, bias, mix, out_coef, y, scale, delta)]
+    rows = torch.tensor([3, 0, 3], dtype=torch.int32) if kind == "rows" else None
+    want_x, v = x.double(), None
+    if kind == "update":
+        want_x = torch.einsum("sk,stw->ktw", mix.double(), x.double()) + out_coef.double()[:, None, None] * (scale.double() * y.double())
+    v = (coef.double()[:, None, None] * want_x).sum(0)
+    if kind != "update":
+        v = v + delta.double()
+        if copies == 1 and rows is None:
+            want_x = v[None]
+    v = v if rows is None else v[rows.long()]
+    norm = (v - v.mean(-1, keepdim=True)) / (v.var(-1, unbiased=False, keepdim=True) + eps).sqrt()
+    want = norm * weight.double() + bias.double()
+    out = torch.full((v.shape[0], width), float("nan"), dtype=dtype, device=DEV)
+    lib.streams_layernorm(d[0], d[1], d[2], d[3], eps, None if rows is None else rows.to(DEV), out, delta=None if kind == "update" else d[8],
+                          update=(d[4], d[5], d[6], d[7]) if kind == "update" else None)
+    # a value is a sum of (copies + 1)^2 products at the most, a mean and a variance are sums of `width` terms: each is off by that many
+    # roundings of the largest thing it is made of; then the rounding of the result's type
+    big = (coef.abs().double()[:, None, None] * (want_x.abs() + (x.abs().sum(0) * mix.abs().max() + (scale * y).abs() * out_coef.abs().max()).double())).sum(0).max()
+    sd = (v.var(-1, unbiased=False, keepdim=True) + eps).sqrt()
+    bound = weight.abs().double() * (((copies + 1) ** 2 + 30) * 2.0 ** -23 * big / sd * (1 + norm.abs() * norm.abs().amax(-1, keepdim=True)))
+    bound = bound + want.abs() * (2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -22) + 1e-6
+    _within(out, want, bound)
+    _within(d[0], want_x, ((copies + 3) * 2.0 ** -23) * (x.abs().double().sum(0) * mix.abs().max() + (scale * y).abs().double() * out_coef.abs().max()
+                                                      + x.abs().double().sum(0) * (1 + coef.abs().max()) + delta.abs().double()).max())
