@@ -394,7 +394,7 @@ struct SelectiveArgs {
   size_t dt_stride;
   const float *dt_bias, *a_log, *d;
 };
-template <int DKL, int RG, int CH, int MODE>
+template <int DKL, int RG, int CH, int MODE, bool WIDE>
 __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
     const float* __restrict__ q, const float* __restrict__ k, size_t qk_stride, const float* __restrict__ v,
     size_t v_stride, const float* __restrict__ g, size_t g_stride, const float* __restrict__ beta, float* __restrict__ state,
@@ -405,7 +405,13 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
   constexpr int DK = DKL * RG;               // rows held, >= dim; rows beyond dim stay zero
   constexpr int NQ = DK * CH / RB_WAVE;      // q (or k, or g) values of a chunk per lane
   constexpr int NV = (COLS * CH + RB_WAVE - 1) / RB_WAVE;
-  __shared__ float sq[CH][DK], sk[CH][DK], sg[SELECTIVE ? 1 : CH][SELECTIVE ? CH : DK], sv[CH][COLS], so[CH][COLS], sb[CH];
+  // In LDS a lane's DKL rows start DKL + 4 numbers behind those of the lane before where 16 lanes hold 16 and 32 rows: the reads of lanes
+  // 0, 4, 8 and 12 met in one bank.  (16 heads, 4 sequences of 1,000 tokens: dim 256 1,624 us before, 1,311 with the gap; 8 heads, dim
+  // 512, 2,662 and 1,415.  Up to dim 128 the gap gives nothing: 464 and 467 us.)
+  constexpr int STEP = DK > 128 ? DKL + 4 : DKL, LD = STEP * RG;
+  auto pos = [](int i) { return i + (STEP - DKL) * (i / DKL); };
+  __shared__ __attribute__((aligned(16))) float sq[CH][LD], sk[CH][LD], sg[SELECTIVE ? 1 : CH][SELECTIVE ? CH : LD];
+  __shared__ float sv[CH][COLS], so[CH][COLS], sb[CH];
   const int b = blockIdx.x, h = blockIdx.y;
   const int lane = threadIdx.x;
   const int col0 = blockIdx.z * COLS;
@@ -444,12 +450,32 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
     const int r = rg * DKL + i;
     ub[i] = (BONUS && r < dim) ? bonus[(size_t)h * dim + r] : 0.f;
   }
-  float rq[NQ], rk[NQ], rgt[SELECTIVE ? 1 : NQ], rv[NV], rb = 0.f;
+  float rq[WIDE ? 1 : NQ], rk[WIDE ? 1 : NQ], rgt[SELECTIVE || WIDE ? 1 : NQ], rv[NV], rb = 0.f;
+  float4 wq[WIDE ? NQ / 4 : 1], wk[WIDE ? NQ / 4 : 1], wg[WIDE && !SELECTIVE ? NQ / 4 : 1];
   const float rate = SELECTIVE ? expf(sel.a_log[h]) : 0.f, dt_bias = SELECTIVE ? sel.dt_bias[h] : 0.f, pass = SELECTIVE ? sel.d[h] : 0.f;
+  // WIDE (rows and strides of 16 bytes): a chunk's values reach a lane four in a row, and what lies beyond the tokens or the key's rows is
+  // taken out on the way to LDS and not before the next chunk's loads have come.  Values one by one were as many instructions, masks and addresses, as
+  // the tokens themselves (16 heads, 4 sequences of 1,000 tokens, with that and with tokens read one ahead: dim 64 217 us before, 160
+  // now; dim 128 464 and 343; dim 256 1,624 and 860; 8 heads of dim 512 2,664 and 792).  Fetch j: token wide_t(j) of the chunk, rows wide_i(j) .. + 3.
+  auto wide_t = [&](int j) { return DK <= 256 ? lane / (DK / 4) + j * (DK <= 256 ? 256 / DK : 1) : j / (DK > 256 ? DK / 256 : 1); };
+  auto wide_i = [&](int j) { return DK <= 256 ? 4 * (lane % (DK / 4)) : 4 * lane + 256 * (j % (DK > 256 ? DK / 256 : 1)); };
   auto fetch = [&](int t0) {
     const int nt = n - t0 < CH ? n - t0 : CH;
+    if (WIDE) {
 #pragma unroll
-    for (int j = 0; j < NQ; ++j) {
+      for (int j = 0; j < NQ / 4; ++j) {
+        // beyond the chunk's tokens or the key's rows: the first of them, which is not used
+        const int tt = wide_t(j) < nt ? wide_t(j) : 0, i = wide_i(j) < dim ? wide_i(j) : 0;
+        const size_t t = (size_t)(row0 + t0 + tt);
+        wq[j] = *reinterpret_cast<const float4*>(q + t * qk_stride + (size_t)kvh * dim + i);
+        wk[j] = *reinterpret_cast<const float4*>(k + t * qk_stride + (size_t)kvh * dim + i);
+        if (SELECTIVE) continue;
+        if (g_per_head) wg[j].x = g[t * g_stride + h];
+        else wg[j] = *reinterpret_cast<const float4*>(g + t * g_stride + (size_t)h * dim + i);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < (WIDE ? 0 : NQ); ++j) {
       const int e = lane + RB_WAVE * j, tt = e / DK, i = e - tt * DK;
       const bool in = tt < nt && i < dim;
       const size_t t = (size_t)(row0 + t0 + tt);
@@ -476,12 +502,28 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
   for (int t0 = 0; t0 < n; t0 += CH) {
     const int nt = n - t0 < CH ? n - t0 : CH;
     __syncthreads();                                   // the chunk before has been read and its outputs are out
+    if (WIDE) {
 #pragma unroll
-    for (int j = 0; j < NQ; ++j) {
+      for (int j = 0; j < NQ / 4; ++j) {
+        const int tt = wide_t(j), i = wide_i(j), at = pos(i);
+        float4 fq = wq[j], fk = wk[j], fg = wg[SELECTIVE ? 0 : j];
+        if (!SELECTIVE && g_per_head) fg.y = fg.z = fg.w = fg.x;
+        if (MODE == 2) {
+          fq = make_float4(fq.x * rb_sigmoid(fq.x), fq.y * rb_sigmoid(fq.y), fq.z * rb_sigmoid(fq.z), fq.w * rb_sigmoid(fq.w));
+          fk = make_float4(fk.x * rb_sigmoid(fk.x), fk.y * rb_sigmoid(fk.y), fk.z * rb_sigmoid(fk.z), fk.w * rb_sigmoid(fk.w));
+        }
+        if (tt >= nt || i >= dim) fq = fk = fg = make_float4(0.f, 0.f, 0.f, 0.f);
+        *reinterpret_cast<float4*>(&sq[tt][at]) = fq;
+        *reinterpret_cast<float4*>(&sk[tt][at]) = fk;
+        if (!SELECTIVE) *reinterpret_cast<float4*>(&sg[SELECTIVE ? 0 : tt][SELECTIVE ? 0 : at]) = fg;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < (WIDE ? 0 : NQ); ++j) {
       const int e = lane + RB_WAVE * j, tt = e / DK, i = e - tt * DK;
-      sq[tt][i] = rq[j];
-      sk[tt][i] = rk[j];
-      if (!SELECTIVE) sg[tt][i] = rgt[j];
+      sq[tt][pos(i)] = rq[j];
+      sk[tt][pos(i)] = rk[j];
+      if (!SELECTIVE) sg[tt][pos(i)] = rgt[j];
     }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
@@ -503,41 +545,42 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
     // One token: with D = diag(g) S and u = beta (v - D^T k), the read-out of the updated state is
     // (D + k u^T)^T q = D^T q + u (k . q): one pass over the decayed column gives both dot products, and a token has
     // one reduction among the RG lanes on its way instead of two.  Two partial sums each: shorter chains of additions.
-    auto token = [&](int tt) {
-      const float vv = sv[tt][lane / RG];
-      const float bt = sb[tt];
-      const float gt = SELECTIVE ? sg[0][tt] : 0.f;
+    struct Token {
+      float k[DKL], q[DKL], g[SELECTIVE ? 1 : DKL], v, b;
+    };
+    auto read = [&](Token& r, int tt) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < DKL; ++i) {
+        r.k[i] = sk[tt][rg * STEP + i];
+        r.q[i] = sq[tt][rg * STEP + i];
+        if (!SELECTIVE) r.g[i] = sg[tt][rg * STEP + i];
+      }
+      if (SELECTIVE) r.g[0] = sg[0][tt];
+      r.v = sv[tt][lane / RG];
+      r.b = sb[tt];
+    };
+    auto token = [&](const Token& r, int tt) __attribute__((always_inline)) {
+      const float vv = r.v, bt = r.b, gt = r.g[0];
       float kv0 = 0.f, kv1 = 0.f, dq0 = 0.f, dq1 = 0.f, kq0 = 0.f, kq1 = 0.f;
 #pragma unroll
       for (int i = 0; i < DKL; i += 2) {
-        const float k0 = sk[tt][rg * DKL + i], q0 = sq[tt][rg * DKL + i];
-        const float k1 = sk[tt][rg * DKL + i + 1], q1 = sq[tt][rg * DKL + i + 1];
+        const float k0 = r.k[i], q0 = r.q[i];
+        const float k1 = r.k[i + 1], q1 = r.q[i + 1];
+        kq0 = fmaf(BONUS ? ub[i] * k0 : k0, q0, kq0);
+        kq1 = fmaf(BONUS ? ub[i + 1] * k1 : k1, q1, kq1);
         if (BONUS) {
           dq0 = fmaf(s[i], q0, dq0);
           dq1 = fmaf(s[i + 1], q1, dq1);
-          kq0 = fmaf(ub[i] * k0, q0, kq0);
-          kq1 = fmaf(ub[i + 1] * k1, q1, kq1);
-          s[i] *= sg[tt][rg * DKL + i];
-          s[i + 1] *= sg[tt][rg * DKL + i + 1];
-          continue;
         }
-        if (SELECTIVE) {
-          s[i] *= gt;
-          s[i + 1] *= gt;
-          dq0 = fmaf(s[i], q0, dq0);
-          dq1 = fmaf(s[i + 1], q1, dq1);
-          kq0 = fmaf(k0, q0, kq0);
-          kq1 = fmaf(k1, q1, kq1);
-          continue;
+        s[i] *= SELECTIVE ? gt : r.g[SELECTIVE ? 0 : i];
+        s[i + 1] *= SELECTIVE ? gt : r.g[SELECTIVE ? 0 : i + 1];
+        if (BONUS) continue;
+        if (!SELECTIVE) {
+          kv0 = fmaf(s[i], k0, kv0);
+          kv1 = fmaf(s[i + 1], k1, kv1);
         }
-        s[i] *= sg[tt][rg * DKL + i];
-        s[i + 1] *= sg[tt][rg * DKL + i + 1];
-        kv0 = fmaf(s[i], k0, kv0);
-        kv1 = fmaf(s[i + 1], k1, kv1);
         dq0 = fmaf(s[i], q0, dq0);
         dq1 = fmaf(s[i + 1], q1, dq1);
-        kq0 = fmaf(k0, q0, kq0);
-        kq1 = fmaf(k1, q1, kq1);
       }
       const float kv = (BONUS || SELECTIVE) ? 0.f : lanes_sum<RG>(kv0 + kv1);
       const float dq = lanes_sum<RG>(dq0 + dq1);
@@ -545,15 +588,35 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
       // without beta: the plain rule, S <- diag(g) S + k v^T
       const float u = SELECTIVE ? bt * vv : (!BONUS && beta) ? bt * (vv - kv) : vv;
 #pragma unroll
-      for (int i = 0; i < DKL; ++i) s[i] = fmaf(sk[tt][rg * DKL + i], u, s[i]);
+      for (int i = 0; i < DKL; ++i) s[i] = fmaf(r.k[i], u, s[i]);
       if (rg == 0) so[tt][lane / RG] = SELECTIVE ? fmaf(pass, vv, fmaf(u, kq, dq)) : fmaf(u, kq, dq);
     };
-    if (nt == CH) {
-      // a whole chunk as straight code, so that a token's reads from LDS are issued while the one before is computed
+    if (nt == CH && CH > 1 && DKL <= 16) {
+      // a whole chunk as straight code, each token read from LDS while the one before is computed
+      Token even, odd;
+      read(even, 0);
 #pragma unroll
-      for (int tt = 0; tt < CH; ++tt) token(tt);
+      for (int tt = 0; tt < CH; tt += 2) {
+        read(odd, tt + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        token(even, tt);
+        if (tt + 2 < CH) read(even, tt + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        token(odd, tt + 1);
+      }
+    } else if (nt == CH) {                 // (longer shares of a column: two tokens of them do not fit into registers)
+#pragma unroll
+      for (int tt = 0; tt < CH; ++tt) {
+        Token r;
+        read(r, tt);
+        token(r, tt);
+      }
     } else {
-      for (int tt = 0; tt < nt; ++tt) token(tt);
+      for (int tt = 0; tt < nt; ++tt) {
+        Token r;
+        read(r, tt);
+        token(r, tt);
+      }
     }
     __syncthreads();
     for (int e = lane; e < nt * COLS; e += RB_WAVE) {
@@ -584,8 +647,12 @@ static void launch_delta_rule(const float* q, const float* k, size_t qk_stride, 
   constexpr int COLS = RB_WAVE / RG;
   static_assert((DKL * RG * CH) % RB_WAVE == 0 && CH <= RB_WAVE && DKL % 4 == 0, "a chunk's values are dealt evenly to the lanes");
   dim3 grid(n_seqs, n_heads, (vdim + COLS - 1) / COLS);
-  delta_rule_kernel<DKL, RG, CH, MODE><<<grid, RB_WAVE, 0, s>>>(q, k, qk_stride, v, v_stride, g, g_stride, beta, state, cu_seqlens,
-                                                                 slots, out, n_heads, n_kv, dim, vdim, g_per_head, bonus, sel);
+  auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  constexpr bool MAY = CH > 1 && DKL * RG * CH / RB_WAVE % 4 == 0;
+  const bool wide = MAY && dim % 4 == 0 && qk_stride % 4 == 0 && aligned(q) && aligned(k) &&
+                    (MODE == 3 || g_per_head || (g_stride % 4 == 0 && aligned(g)));
+  (wide ? delta_rule_kernel<DKL, RG, CH, MODE, MAY> : delta_rule_kernel<DKL, RG, CH, MODE, false>)<<<grid, RB_WAVE, 0, s>>>(
+      q, k, qk_stride, v, v_stride, g, g_stride, beta, state, cu_seqlens, slots, out, n_heads, n_kv, dim, vdim, g_per_head, bonus, sel);
 }
 
 extern "C" int rb_delta_rule(const float* q, const float* k, long long qk_stride, const float* v, long long v_stride,

@@ -368,3 +368,45 @@ def test_layernorm_over_copies(lib, copies, width, dtype, kind):
     _within(out, want, bound)
     _within(d[0], want_x, ((copies + 3) * 2.0 ** -23) * (x.abs().double().sum(0) * mix.abs().max() + (scale * y).abs().double() * out_coef.abs().max()
                                                       + x.abs().double().sum(0) * (1 + coef.abs().max()) + delta.abs().double()).max())
+
+
+# ---------------------------------------------------------------- the gated delta rule, token after token
+@pytest.mark.parametrize("dim", [8, 32, 64, 68, 100, 128, 200, 384])
+@pytest.mark.parametrize("lengths", [[1], [1, 1, 1], [15, 16, 17], [70]])
+@pytest.mark.parametrize("heads,per_head", [(2, True), (64, False)])
+@pytest.mark.parametrize("rule", ["delta", "plain"])
+def test_recurrences_of_every_key_size(lib, dim, lengths, heads, per_head, rule):
+    """Every split of a column over lanes, both layouts of a column in LDS, chunks that are whole, in part and of one token; 64 heads fill
+    the GPU and take the longer shares of a column."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(dim + heads + sum(lengths))
+    n, vdim = sum(lengths), 20 if heads == 2 else 128
+    qkv = torch.randn(n, 2 * heads * dim + heads * vdim, generator=g)
+    unit = torch.nn.functional.normalize(qkv[:, :2 * heads * dim].view(n, 2 * heads, dim), dim=-1)
+    qkv[:, :2 * heads * dim] = unit.view(n, -1)
+    decay = 0.8 + 0.2 * torch.rand(n, heads * (1 if per_head else dim), generator=g)
+    beta = torch.rand(n, heads, generator=g)
+    state = torch.randn(len(lengths) + 1, heads, vdim, dim, generator=g)
+    slots = list(range(len(lengths), 0, -1))
+    want, want_state, most, at = torch.empty(n, heads, vdim, dtype=torch.float64), state.double(), 1.0, 0
+    for b, length in enumerate(lengths):
+        S = want_state[slots[b]].transpose(1, 2).clone()              # [H, dim, vdim]
+        for t in range(at, at + length):
+            q, k = unit[t, :heads].double(), unit[t, heads:].double()
+            v = qkv[t, 2 * heads * dim:].view(heads, vdim).double()
+            S = S * decay[t].double().view(heads, -1, 1)
+            u = beta[t].double()[:, None] * (v - torch.einsum("hiv,hi->hv", S, k)) if rule == "delta" else v
+            S = S + k[:, :, None] * u[:, None, :]
+            want[t] = torch.einsum("hiv,hi->hv", S, q)
+            most = max(most, float(S.norm(dim=1).max()))
+        want_state[slots[b]] = S.transpose(1, 2)
+        at += length
+    cu = torch.tensor([0] + torch.tensor(lengths).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    ctx = SimpleNamespace(n_tokens=n, n_seqs=len(lengths), cu_seqlens=cu, slots=torch.tensor(slots, dtype=torch.int32, device=DEV))
+    dev_state, out = state.to(DEV), torch.full((n, heads * vdim), float("nan"), device=DEV)
+    lib.linear_recurrence(qkv.to(DEV), heads, dim, heads, vdim, decay.to(DEV), 0, per_head, beta.to(DEV) if rule == "delta" else None,
+                          dev_state, ctx, out)
+    # unit keys and decays below 1 do not enlarge an error: each token adds the roundings of two sums over `dim` of a column
+    bound = max(lengths) * (2 * dim + 8) * 2.0 ** -24 * most
+    _within(out, want.view(n, -1), bound)
+    _within(dev_state, want_state, bound)
