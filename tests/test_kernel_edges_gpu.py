@@ -410,3 +410,29 @@ def test_recurrences_of_every_key_size(lib, dim, lengths, heads, per_head, rule)
     bound = max(lengths) * (2 * dim + 8) * 2.0 ** -24 * most
     _within(out, want.view(n, -1), bound)
     _within(dev_state, want_state, bound)
+
+
+# ---------------------------------------------------------------- what enters a recurrence
+@pytest.mark.parametrize("tokens", [1, 5, 128, 129])
+@pytest.mark.parametrize("heads,dim,per_head", [(1, 4, True), (2, 100, False), (16, 128, False), (40, 256, True), (3, 300, False), (24, 512, False)])
+@pytest.mark.parametrize("unit", [0, 1])
+def test_what_enters_a_recurrence(lib, tokens, heads, dim, per_head, unit):
+    """Heads that fit registers and longer ones, one workgroup a token and several, down to fewer threads than there is work."""
+    g = torch.Generator().manual_seed(tokens + dim)
+    cols = heads if per_head else heads * dim
+    qk, a, b = torch.randn(tokens, 2 * heads * dim + 3, generator=g), torch.randn(tokens, cols + 1, generator=g), torch.randn(tokens, heads, generator=g)
+    bias, a_log = torch.randn(cols, generator=g), 0.3 * torch.randn(heads, generator=g)
+    d = [t.to(DEV) for t in (qk, a, b, bias, a_log)]
+    beta = torch.full((tokens, heads), float("nan"), device=DEV)
+    lib._ok(lib._lib.rb_recurrence_prep(d[0].data_ptr(), qk.shape[1], heads, dim, unit, 0.25, 1e-6, d[1].data_ptr(), a.shape[1], cols, 0,
+                                        d[3].data_ptr(), d[4].data_ptr(), 1.0, heads, d[2].data_ptr(), heads, beta.data_ptr(), tokens, lib._stream()))
+    v = qk[:, :2 * heads * dim].double().view(tokens, 2, heads, dim)
+    scale = torch.tensor([0.25, 1.0], dtype=torch.float64).view(1, 2, 1, 1)
+    want = v * scale / ((v * v).sum(-1, keepdim=True) + 1e-6).sqrt() if unit else v * scale
+    # a sum of `dim` squares over 64 lanes, a root and a quotient: dim / 64 + 12 roundings
+    _within(d[0][:, :2 * heads * dim], want.view(tokens, -1), (dim / 64 + 12) * 2.0 ** -24 * want.view(tokens, -1).abs() + 1e-30)
+    assert torch.equal(d[0][:, 2 * heads * dim:].cpu(), qk[:, 2 * heads * dim:]) and torch.equal(d[1][:, cols:].cpu(), a[:, cols:])
+    rate = a_log.double().exp().repeat_interleave(cols // heads) * torch.nn.functional.softplus(a[:, :cols].double() + bias.double())
+    # the exponent has the roundings of a sum, an exponential, a softplus and a product, the result those of its exponential
+    _within(d[1][:, :cols], (-rate).exp(), 32 * 2.0 ** -24 * (1 + rate) * (-rate).exp() + 2.0 ** -22 * (-rate).exp() + 1e-37)
+    _within(beta, b.double().sigmoid(), 2.0 ** -20)
