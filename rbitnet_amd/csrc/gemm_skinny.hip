@@ -42,7 +42,8 @@ constexpr int EPI_ACT = 4;
 // What a lane does with its 4 consecutive sums of token mm, columns nn.. (epilogues 0, 2, 3).
 // All 64 lanes come here together: the sums of squares go round the four lanes that share
 // a token's 16 columns.
-// MAY: four columns at a time where FoldArgs::wide says so.
+// MAY: four columns at a time where FoldArgs::wide says so.  The squares are added up with fused operations that are spelled out: left to
+// the compiler, the wide and the narrow store contracted them differently, and what is stored must not depend on addresses.
 template <int EPI, bool MAY, typename TO>
 __device__ __forceinline__ void store_sums(TO* __restrict__ c, const f32x4_t& sums, const f32x4_t& before,
                                            const f32x4_t& gain, int mm, int nn, int m, int n, int tile, int kq,
@@ -63,7 +64,7 @@ __device__ __forceinline__ void store_sums(TO* __restrict__ c, const f32x4_t& su
       else *reinterpret_cast<f32x4_t*>(dst) = v;
       if (EPI == 3) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sq += v[i] * v[i];
+        for (int i = 0; i < 4; ++i) sq = fmaf(v[i], v[i], sq);
         const f32x4_t p = v * gain;
         *reinterpret_cast<uint2*>(fa.gained + (size_t)mm * n + nn) = make_uint2(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]));
       }
@@ -77,7 +78,7 @@ __device__ __forceinline__ void store_sums(TO* __restrict__ c, const f32x4_t& su
       if (EPI == EPI_ACT) v = xielu_value(v, xa.ap, xa.an);
       Num<TO>::store(dst + i, v);
       if (EPI == 3) {
-        sq += v * v;
+        sq = fmaf(v, v, sq);
         fa.gained[(size_t)mm * n + nn + i] = f32_to_bf16(v * gain[i]);
       }
     }

@@ -51,6 +51,34 @@ def test_float32_tiles_of_operands_at_odd_addresses(lib, m, n, k):
     _within(c, a.double() @ w.double().T, k * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T))
 
 
+# ---------------------------------------------------------------- products of few tokens that add to the stream
+@pytest.mark.parametrize("m", [1, 5, 16])
+@pytest.mark.parametrize("n,k", [(48, 96), (64, 128), (272, 768), (8192, 2048)])
+def test_stream_products_do_not_depend_on_addresses(lib, m, n, k):
+    """The stream's new rows, what the next norm takes of them and their sums of squares are the same bits where columns leave four at a
+    time and one by one; a sum of squares is one of products that are not rounded, in the order of the columns."""
+    g = torch.Generator().manual_seed(m + n)
+    a, w = torch.randn(m, k, generator=g).bfloat16().to(DEV), (torch.randn(n, k, generator=g) * 0.02).bfloat16().to(DEV)
+    c0, gain0 = torch.randn(m, n, generator=g).to(DEV), torch.randn(n, generator=g).to(DEV)
+    got = []
+    for off in (0, 1):
+        c, gain = torch.empty(m * n + off, device=DEV)[off:].view(m, n), torch.empty(n + off, device=DEV)[off:]
+        gained = torch.empty(m * n + off, dtype=torch.bfloat16, device=DEV)[off:].view(m, n)
+        squares = torch.full((m, n // 16), float("nan"), device=DEV)
+        c.copy_(c0)
+        gain.copy_(gain0)
+        lib.gemm_bf16_few(a, w, c, 3, gain=gain, gained=gained, squares_out=squares)
+        got.append((c, gained, squares))
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
+    v = got[0][0].double().cpu().view(m, n // 16, 4, 4)
+    four = torch.zeros(m, n // 16, 4)
+    for i in range(4):                       # float64 holds the product and the sum of one fused operation but for ties of ties
+        four = (four.double() + v[..., i] * v[..., i]).float()
+    want = (four[..., 0] + four[..., 1]) + (four[..., 2] + four[..., 3])
+    assert torch.equal(got[0][2].cpu(), want)
+
+
 # ---------------------------------------------------------------- float32 attention on the matrix cores
 def _paged(lengths, heads, dim, generator, spare=7):
     """Keys (or values) of sequences of these lengths in pages that are handed out in a mixed order, NaN where nothing was written."""
