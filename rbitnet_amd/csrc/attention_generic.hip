@@ -281,6 +281,12 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_generic_vec_
   }
 }
 
+// x, for comparisons that are made where they stand: made ahead of a loop, they hold more scalar registers than there are.
+__device__ __forceinline__ int here(int x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+
 // Float32 attention on the float32 MFMA (16x16x4: float32 inputs, products and sums), for head sizes that are multiples of 4 up to
 // 128.  The 16 columns of the MFMAs are queries: the heads that share a key/value head, of one token or of as many consecutive
 // tokens as fit, so that a key is read once for all of them.  Scores are K Q^T (a lane takes one key's row, 16 bytes at a time, and
@@ -291,9 +297,10 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_generic_vec_
 // keys, chunks and sigmoid weights as in the kernels above.
 // Bound by the MFMAs for prompts (2 x 32 cycles for 16 keys, 16 queries and 4 numbers) and by a chain of loads in single-token
 // steps.  Measured beside the kernel above (a lane per key on the vector units), 24 heads of 128 on 8: four prompts of 131 to 512 tokens
-// 600 -> 125 us a layer, one token for each of four sequences at 131 to 520 keys 29 -> 24 us (32 workgroups,
+// 600 -> 130 us a layer, one token for each of four sequences at 131 to 520 keys 29 -> 24 us (32 workgroups,
 // whose matrix cores three of sixteen columns keep busy: what bounds it now).
-template <int NB>
+// ONE: a block is one token's.
+template <int NB, bool ONE>
 __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_kernel(
     const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages, float* __restrict__ out,
     const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ block_table, int bt_stride,
@@ -310,33 +317,39 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
   const int h_count = group - first < 16 ? group - first : 16;
   const int h0 = kvh * group + first;
   // late tokens first: they have the most keys
-  const int t0 = (gridDim.x - 1 - blockIdx.x) * tokens_per_block;
-  const int t1 = t0 + tokens_per_block < n_tokens ? t0 + tokens_per_block : n_tokens;
-  const int t = t0 + col / h_count, h = h0 + col % h_count;
-  const bool on = t < t1;
+  const int t0 = (gridDim.x - 1 - blockIdx.x) * (ONE ? 1 : tokens_per_block);
+  const int t1 = ONE ? t0 + 1 : t0 + tokens_per_block < n_tokens ? t0 + tokens_per_block : n_tokens;
+  const int t = ONE ? t0 : t0 + col / h_count, h = ONE ? h0 + col : h0 + col % h_count;
+  const bool on = ONE ? col < h_count : t < t1;
   const int my_pos = on ? tok_pos[t] : -1;
   const int my_lo = on ? first_visible(my_pos, window, chunk) : 0;
 
-  f32x4_t qv[NB], acc[NB];
+  f32x4_t qv[NB];
 #pragma unroll
   for (int c = 0; c < NB; ++c) {
     qv[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     if (on && 16 * c + 4 * g < head_dim)
       qv[c] = *reinterpret_cast<const f32x4_t*>(q + ((size_t)t * n_heads + h) * head_dim + 16 * c + 4 * g);
-    acc[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   }
   const float sb = sig_bias && on ? sig_bias[h] : 0.f;
-  float m_run = sig_bias ? 0.f : -INFINITY, l_run = 0.f;
 
-  // the tokens of a block belong to one sequence, but for a block over a boundary: sequence after sequence then, the other's
-  // queries seeing nothing
-  for (int seg = t0; seg < t1;) {
+  // Sequence after sequence: almost always the whole block is one's.  Each starts anew and leaves with its own columns only, so that
+  // nothing of another sequence comes into a query's sums.
+  for (int seg = t0, end; seg < t1; seg = end) {
     const int seq = tok_seq[seg];
-    int end = seg + 1;
-    while (end < t1 && tok_seq[end] == seq) ++end;
+    end = seg + 1;
+    while (!ONE && end < t1 && tok_seq[end] == seq) ++end;
     const int32_t* pages = block_table + (size_t)seq * bt_stride;
     const int hi = tok_pos[end - 1], lo = first_visible(tok_pos[seg], window, chunk);
-    const bool mine = t >= seg && t < end;
+    const bool mine = ONE ? on : t >= seg && t < end;
+    auto sees = [&](int key) { return mine && key <= my_pos && (key >= my_lo || key < keep_first); };
+    // A weight of 0 does not take an infinity or a NaN out of a matrix product.  One token's queries see the same keys: the values of
+    // others become zeros.
+    auto hidden = [&](int key) { return key > hi || (key < lo && key >= keep_first); };
+    f32x4_t acc[NB];
+#pragma unroll
+    for (int d = 0; d < NB; ++d) acc[d] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    float m_run = sig_bias ? 0.f : -INFINITY, l_run = 0.f;
     const int lo_unit = lo / 32;
     const int kept = keep_first > 0 ? (keep_first + 31) / 32 : 0;
     const int n_first = kept < lo_unit ? kept : lo_unit;
@@ -374,6 +387,16 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
             }
           }
         }
+      if (ONE && (key0 + 31 > hi || key0 < lo)) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (hidden(key0 + 16 * b + 4 * g + i)) {
+#pragma unroll
+              for (int d = 0; d < NB; ++d) vf[b][i][d] = 0.f;
+            }
+      }
       f32x4_t sc[2];
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
@@ -384,6 +407,7 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
           for (int i = 0; i < 4; ++i) sc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][c][i], qv[c][i], sc[b], 0, 0, 0);
       }
       float top = -INFINITY;
+      bool in_part = false;                   // some query of the sequence does not see one of these keys
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -391,7 +415,9 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
           const int key = key0 + 16 * b + 4 * g + i;
           float s = sc[b][i] * scale;
           if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-          s = mine && key <= my_pos && (key >= my_lo || key < keep_first) ? s : -INFINITY;
+          const bool seen = sees(key);
+          s = seen ? s : -INFINITY;
+          if (!ONE) in_part |= mine && !seen;
           sc[b][i] = s;
           top = fmaxf(top, s);
         }
@@ -412,61 +438,96 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
         }
 #pragma unroll
       for (int d = 0; d < NB; ++d) acc[d] *= corr;
+      // Several tokens': where a query does not see all of these keys and a value is an infinity or a NaN, every query adds up the
+      // keys that it sees, by itself.
+      bool bad = false;
+      if (!ONE && __any(in_part)) {
+        float zero = 0.f;
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int d = 0; d < NB; ++d) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][i][d], sc[b][i], acc[d], 0, 0, 0);
+            for (int d = 0; d < NB; ++d) zero = fmaf(vf[b][i][d], 0.f, zero);
+        bad = __any(zero != 0.f);
+      }
+      if (bad) {
+#pragma unroll 1
+        for (int kk = 0; kk < 32; ++kk) {
+          const f32x4_t four = kk < 16 ? sc[0] : sc[1];
+          const int i = kk & 3;
+          const float p = __shfl(i == 0 ? four[0] : i == 1 ? four[1] : i == 2 ? four[2] : four[3], (kk & 12) * 4 + col, RB_WAVE);
+          if (!sees(key0 + kk)) continue;
+          const float* vrow = v_pages + base + (size_t)kk * head_dim + 4 * NB * g;
+          const int left = here(head_dim) - 4 * NB * g;
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int d = 0; d < NB; d += VW)
+              if (NB * j + d < left) {
+                float v[VW];
+                if (VW == 4) *reinterpret_cast<f32x4_t*>(v) = *reinterpret_cast<const f32x4_t*>(vrow + NB * j + d);
+                else *reinterpret_cast<float2*>(v) = *reinterpret_cast<const float2*>(vrow + NB * j + d);
+#pragma unroll
+                for (int e = 0; e < VW; ++e) acc[d + e][j] = fmaf(p, v[e], acc[d + e][j]);
+              }
+        }
+      } else {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int d = 0; d < NB; ++d) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][i][d], sc[b][i], acc[d], 0, 0, 0);
+      }
     }
-    seg = end;
-  }
-  l_run += __shfl_xor(l_run, 16, RB_WAVE);
-  l_run += __shfl_xor(l_run, 32, RB_WAVE);
+    l_run += __shfl_xor(l_run, 16, RB_WAVE);
+    l_run += __shfl_xor(l_run, 32, RB_WAVE);
 
-  // lane holds, for query col, the numbers NB (4 g + j) + d of the head
-  if (n_waves == 1) {
-    if (!on) return;
-    if (sinks) l_run += expf(sinks[h] - m_run);
-    const float inv = sig_bias ? 1.0f : (l_run > 0.f ? 1.0f / l_run : 0.f);
-    float* orow = out + ((size_t)t * n_heads + h) * head_dim;
+    // lane holds, for query col, the numbers NB (4 g + j) + d of the head
+    if (n_waves == 1) {
+      if (!mine) continue;
+      if (sinks) l_run += expf(sinks[h] - m_run);
+      const float inv = sig_bias ? 1.0f : (l_run > 0.f ? 1.0f / l_run : 0.f);
+      float* orow = out + ((size_t)t * n_heads + h) * head_dim + 4 * NB * g;
+      const int left = here(head_dim) - 4 * NB * g;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int d = 0; d < NB; ++d)
+          if (NB * j + d < left) orow[NB * j + d] = acc[d][j] * inv;
+      continue;
+    }
+    if (seg > t0) __syncthreads();            // the sequence before has been read
+    float* row = merged + ((size_t)wave * 16 + col) * LD;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int d = 0; d < NB; ++d) {
-        const int at = NB * (4 * g + j) + d;
-        if (at < head_dim) orow[at] = acc[d][j] * inv;
-      }
-    return;
-  }
-  float* row = merged + ((size_t)wave * 16 + col) * LD;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int d = 0; d < NB; ++d) row[NB * (4 * g + j) + d] = acc[d][j];
-  if (g == 0) {
-    row[16 * NB] = m_run;
-    row[16 * NB + 1] = l_run;
-  }
-  __syncthreads();
-  // every thread finishes a few numbers of a query: the waves' sums under their common maximum, in the order of the waves
-  const int queries = (t1 - t0) * h_count;
-  for (int idx = threadIdx.x; idx < queries * head_dim; idx += blockDim.x) {
-    const int cc = idx / head_dim, d = idx - cc * head_dim;
-    const int hh = h0 + cc % h_count;
-    const float* src = merged + (size_t)cc * LD;
-    float mx = -INFINITY;
-    for (int w = 0; w < n_waves; ++w) mx = fmaxf(mx, src[(size_t)w * 16 * LD + 16 * NB]);
-    float l = 0.f, o = 0.f;
-    for (int w = 0; w < n_waves; ++w) {
-      const float mw = src[(size_t)w * 16 * LD + 16 * NB];
-      const float f = mw == -INFINITY ? 0.f : expf(mw - mx);
-      l += src[(size_t)w * 16 * LD + 16 * NB + 1] * f;
-      o += src[(size_t)w * 16 * LD + d] * f;
+      for (int d = 0; d < NB; ++d) row[NB * (4 * g + j) + d] = acc[d][j];
+    if (g == 0) {
+      row[16 * NB] = m_run;
+      row[16 * NB + 1] = l_run;
     }
-    if (sinks) l += expf(sinks[hh] - mx);
-    const float inv = sig_bias ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
-    out[((size_t)(t0 + cc / h_count) * n_heads + hh) * head_dim + d] = o * inv;
+    __syncthreads();
+    // every thread finishes a few numbers of a query: the waves' sums under their common maximum, in the order of the waves
+    const int first_col = (seg - t0) * h_count, queries = (end - seg) * h_count;
+    for (int idx = threadIdx.x; idx < queries * head_dim; idx += blockDim.x) {
+      const int q_of = idx / head_dim, d = idx - q_of * head_dim, cc = first_col + q_of;
+      const int hh = h0 + cc % h_count;
+      const float* src = merged + (size_t)cc * LD;
+      float mx = -INFINITY;
+      for (int w = 0; w < n_waves; ++w) mx = fmaxf(mx, src[(size_t)w * 16 * LD + 16 * NB]);
+      float l = 0.f, o = 0.f;
+      for (int w = 0; w < n_waves; ++w) {
+        const float mw = src[(size_t)w * 16 * LD + 16 * NB];
+        const float f = mw == -INFINITY ? 0.f : expf(mw - mx);
+        l += src[(size_t)w * 16 * LD + 16 * NB + 1] * f;
+        o += src[(size_t)w * 16 * LD + d] * f;
+      }
+      if (sinks) l += expf(sinks[hh] - mx);
+      const float inv = sig_bias ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
+      out[((size_t)(t0 + cc / h_count) * n_heads + hh) * head_dim + d] = o * inv;
+    }
   }
 }
 
@@ -484,19 +545,15 @@ struct AttentionF32 {
   const float* sig_bias;
 };
 
-template <int NB>
-static int launch_attention_f32(const AttentionF32& a, hipStream_t s) {
-  const int group = a.n_heads / a.n_kv, chunks = (group + 15) / 16;
-  // One token a block while that leaves the GPU room (single-token steps above all: a block of tokens of several sequences takes
-  // them one after another), as many as the 16 columns hold beyond.
+template <int NB, bool ONE>
+static int launch_attention_f32_blocks(const AttentionF32& a, int per_block, int chunks, hipStream_t s) {
   const long long cus = rb_compute_units();
-  const int per_block = (long long)a.n_tokens * a.n_kv * chunks >= 4 * cus && group < 16 ? 16 / group : 1;
   const long long blocks = ((long long)a.n_tokens + per_block - 1) / per_block;
   int n_waves = 1;
   while (n_waves < AG_MAX_WAVES && blocks * a.n_kv * chunks * n_waves < 8 * cus) n_waves *= 2;
   RB_REQUIRE((long long)a.n_kv * chunks <= 65535, "rb_attention_generic: too many heads %d", a.n_heads);
   const size_t lds = n_waves > 1 ? (size_t)n_waves * 16 * (16 * NB + 4) * sizeof(float) : 0;
-  auto kern = attention_f32_mfma_kernel<NB>;
+  auto kern = attention_f32_mfma_kernel<NB, ONE>;
   static bool configured = false;
   if (!configured) {
     const size_t most = (size_t)AG_MAX_WAVES * 16 * (16 * NB + 4) * sizeof(float);
@@ -508,6 +565,16 @@ static int launch_attention_f32(const AttentionF32& a, hipStream_t s) {
       a.q, a.k_pages, a.v_pages, a.out, a.tok_pos, a.tok_seq, a.block_table, a.bt_stride, a.n_tokens, a.n_heads, a.n_kv, a.head_dim,
       a.scale, a.window, a.sinks, a.keep_first, a.softcap, a.chunk, a.sig_bias, per_block, chunks);
   return 0;
+}
+
+template <int NB>
+static int launch_attention_f32(const AttentionF32& a, hipStream_t s) {
+  const int group = a.n_heads / a.n_kv, chunks = (group + 15) / 16;
+  // One token a block while that leaves the GPU room (single-token steps above all: a block of tokens of several sequences takes
+  // them one after another), as many as the 16 columns hold beyond.
+  const int per_block = (long long)a.n_tokens * a.n_kv * chunks >= 4 * rb_compute_units() && group < 16 ? 16 / group : 1;
+  if (per_block == 1) return launch_attention_f32_blocks<NB, true>(a, 1, chunks, s);
+  return launch_attention_f32_blocks<NB, false>(a, per_block, chunks, s);
 }
 
 static int g_attention_vec = 1;

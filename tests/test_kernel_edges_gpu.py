@@ -157,6 +157,60 @@ def test_float32_attention(lib, heads, kv, dim, past, new, more):
     _within(out.view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
 
 
+@pytest.mark.parametrize("heads,kv,dim", [(8, 8, 32), (6, 2, 32), (12, 4, 64), (24, 8, 128), (5, 5, 100)])
+@pytest.mark.parametrize("past,new", [([0, 40, 130, 0], [301, 7, 2, 303]), ([70, 3, 0], [1, 1, 1]), ([0], [90])])
+@pytest.mark.parametrize("more", [{}, {"window": 50, "keep": 9}, {"sig": True, "chunk": 48}])
+@pytest.mark.parametrize("bad", ["none", "values", "keys"])
+def test_float32_attention_keeps_tokens_apart(lib, heads, kv, dim, past, new, more, bad):
+    """Blocks over the boundaries of sequences, two and three in a block; an infinite or undefined key or value comes to the queries that
+    see it and to no other token's, of its sequence or the next, and an undefined value to its own number of a head alone."""
+    g = torch.Generator().manual_seed(heads * 7 + dim + sum(new))
+    more = dict(more)
+    lengths = [p + n for p, n in zip(past, new)]
+    kp, table, ks = _paged(lengths, kv, dim, g)
+    vp, vs = torch.full_like(kp, float("nan")), []
+    for b, n in enumerate(lengths):
+        x = torch.randn(n, kv, dim, generator=g)
+        for j in range(n):
+            vp[table[b, j // 64], :, j % 64] = x[j]
+        vs.append(x)
+    where = {}                                                    # sequence -> position, kv head and number of what is not finite
+    if bad != "none":
+        for b, n in enumerate(lengths):
+            if b % 2 == 0:
+                j, head, d = max(past[b], n - 1 - n // 3), b % kv, (5 * b) % dim
+                where[b] = (j, head, d)
+                (vp if bad == "values" else kp)[table[b, j // 64], head, j % 64, d] = float("inf") if b else float("nan")
+    q = torch.randn(sum(new), heads, dim, generator=g)
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip(past, new)])
+    seq = torch.repeat_interleave(torch.arange(len(new)), torch.tensor(new))
+    if more.get("sig"):
+        more["sig"] = torch.randn(heads, generator=g)
+    scale = dim ** -0.5
+    want = torch.cat([_attention64(q[seq == b], ks[b], vs[b], pos[seq == b], scale, **more) for b in range(len(new))])
+    out = torch.full((sum(new), heads * dim), float("nan"), device=DEV)
+    i32 = lambda x: x.to(torch.int32).to(DEV)
+    lib.attention_opts(q.to(DEV), kp.to(DEV), vp.to(DEV), out, i32(pos), i32(seq), table.to(DEV), heads, kv, dim, scale,
+                       more.get("window", 0), more.get("keep", 0), 0.0, None, more.get("chunk", 0),
+                       None if more.get("sig") is None else more["sig"].to(DEV))
+    got = out.view(want.shape).cpu()
+    touched = torch.zeros(want.shape, dtype=torch.bool)           # what may differ from the result with finite keys and values
+    for b, (j, head, d) in where.items():
+        seen = (seq == b) & (pos >= j)
+        if more.get("window"):
+            seen &= (pos - j < more["window"]) | (j < more["keep"])
+        if more.get("chunk"):
+            seen &= pos // more["chunk"] == j // more["chunk"]
+        mine = slice(head * (heads // kv), (head + 1) * (heads // kv))
+        assert seen.any()
+        if bad == "values":
+            touched[seen, mine, d] = True
+            assert not torch.isfinite(got[seen][:, mine, d]).any()
+        else:
+            touched[seen, mine] = True
+    _within(torch.where(touched, 0.0, got), torch.where(touched, 0.0, want), 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
+
+
 # ---------------------------------------------------------------- products per head on the matrix cores
 @pytest.mark.parametrize("tokens", [1, 4, 16, 17, 200])
 @pytest.mark.parametrize("heads,k,n,more", [(1, 32, 16, {}), (3, 64, 96, {"rot": 32, "pad": 128}), (16, 128, 128, {}),
