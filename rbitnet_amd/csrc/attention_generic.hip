@@ -333,12 +333,12 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
   }
   const float sb = sig_bias && on ? sig_bias[h] : 0.f;
 
-  // Sequence after sequence: almost always the whole block is one's.  Each starts anew and leaves with its own columns only, so that
-  // nothing of another sequence comes into a query's sums.
+  // Run after run of consecutive positions of one sequence: almost always the whole block is one.  Each starts anew and leaves with its
+  // own columns only, so that nothing of another sequence comes into a query's sums, and tokens may come in any order.
   for (int seg = t0, end; seg < t1; seg = end) {
     const int seq = tok_seq[seg];
     end = seg + 1;
-    while (!ONE && end < t1 && tok_seq[end] == seq) ++end;
+    while (!ONE && end < t1 && tok_seq[end] == seq && tok_pos[end] == tok_pos[end - 1] + 1) ++end;
     const int32_t* pages = block_table + (size_t)seq * bt_stride;
     const int hi = tok_pos[end - 1], lo = first_visible(tok_pos[seg], window, chunk);
     const bool mine = ONE ? on : t >= seg && t < end;
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
     const int lo_unit = lo / 32;
     const int kept = keep_first > 0 ? (keep_first + 31) / 32 : 0;
     const int n_first = kept < lo_unit ? kept : lo_unit;
-    const int n_walk = n_first + hi / 32 - lo_unit + 1;
+    const int n_walk = hi < 0 ? 0 : n_first + hi / 32 - lo_unit + 1;      // (without a position there are no keys)
     for (int walk = wave; walk < n_walk; walk += n_waves) {
       const int key0 = 32 * (walk < n_first ? walk : lo_unit + walk - n_first);
       const size_t base = ((size_t)pages[key0 / RB_PAGE] * n_kv + kvh) * RB_PAGE * head_dim + (size_t)(key0 % RB_PAGE) * head_dim;
@@ -407,7 +407,7 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
           for (int i = 0; i < 4; ++i) sc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][c][i], qv[c][i], sc[b], 0, 0, 0);
       }
       float top = -INFINITY;
-      bool in_part = false;                   // some query of the sequence does not see one of these keys
+      bool in_part = false;                   // some query of the run does not see one of these keys
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -498,7 +498,7 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
           if (NB * j + d < left) orow[NB * j + d] = acc[d][j] * inv;
       continue;
     }
-    if (seg > t0) __syncthreads();            // the sequence before has been read
+    if (seg > t0) __syncthreads();            // the run before has been read
     float* row = merged + ((size_t)wave * 16 + col) * LD;
 #pragma unroll
     for (int j = 0; j < 4; ++j)

@@ -211,6 +211,42 @@ def test_float32_attention_keeps_tokens_apart(lib, heads, kv, dim, past, new, mo
     _within(torch.where(touched, 0.0, got), torch.where(touched, 0.0, want), 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
 
 
+@pytest.mark.parametrize("heads,kv,dim", [(8, 8, 32), (12, 4, 64), (24, 8, 128)])
+@pytest.mark.parametrize("more", [{}, {"window": 50, "keep": 9}])
+@pytest.mark.parametrize("order", ["falling", "mixed", "twice", "without a position"])
+def test_float32_attention_of_tokens_in_any_order(lib, heads, kv, dim, more, order):
+    """Every token is answered from its own position and sequence, whatever its neighbours in the step are; a token without a position
+    (a negative one) sees nothing."""
+    g = torch.Generator().manual_seed(heads + dim)
+    lengths = [300, 90]
+    kp, table, ks = _paged(lengths, kv, dim, g)
+    vp, vs = torch.full_like(kp, float("nan")), []
+    for b, n in enumerate(lengths):
+        x = torch.randn(n, kv, dim, generator=g)
+        for j in range(n):
+            vp[table[b, j // 64], :, j % 64] = x[j]
+        vs.append(x)
+    pos, seq = torch.cat([torch.arange(n) for n in lengths]), torch.repeat_interleave(torch.arange(2), torch.tensor(lengths))
+    if order == "falling":
+        pos, seq = pos.flip(0), seq.flip(0)
+    elif order == "mixed":
+        at = torch.randperm(len(pos), generator=g)
+        pos, seq = pos[at], seq[at]
+    elif order == "twice":
+        pos, seq = pos.repeat_interleave(2), seq.repeat_interleave(2)
+    else:
+        pos = torch.where(torch.rand(len(pos), generator=g) < 0.3, -1, pos)
+    q = torch.randn(len(pos), heads, dim, generator=g)
+    want = torch.zeros(q.shape, dtype=torch.float64)
+    for b in range(2):
+        at = (seq == b) & (pos >= 0)
+        want[at] = _attention64(q[at], ks[b], vs[b], pos[at], dim ** -0.5, **more)
+    out = torch.full((len(pos), heads * dim), float("nan"), device=DEV)
+    lib.attention_opts(q.to(DEV), kp.to(DEV), vp.to(DEV), out, pos.int().to(DEV), seq.int().to(DEV), table.to(DEV), heads, kv, dim,
+                       dim ** -0.5, more.get("window", 0), more.get("keep", 0), 0.0, None)
+    _within(out.view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
+
+
 # ---------------------------------------------------------------- products per head on the matrix cores
 @pytest.mark.parametrize("tokens", [1, 4, 16, 17, 200])
 @pytest.mark.parametrize("heads,k,n,more", [(1, 32, 16, {}), (3, 64, 96, {"rot": 32, "pad": 128}), (16, 128, 128, {}),
