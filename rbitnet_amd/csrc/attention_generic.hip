@@ -295,6 +295,10 @@ __device__ __forceinline__ int here(int x) {
 // numbers NB r + dt of a head for its row r), so that they come with wide loads and leave as pieces of rows.  The waves of a workgroup
 // share the keys, 32 at a time, and merge through LDS at the end.  Softmax, its running maximum, caps, sinks, windows, kept first
 // keys, chunks and sigmoid weights as in the kernels above.
+// A score is four sums (of every fourth number), a unit of 32 keys has sums of its own, 16 / NB of them side by side, which are added up
+// as a tree before they meet the running ones, and so are its weights: one sum for everything had twice the error. Relative error of
+// the outputs, 24 heads of 128 at 131 to 512 keys / one token at 8,000: 3.2e-7 / 6.8e-7 with one sum, 1.5e-7 / 2.4e-7 now, 1.7e-7 / 4.4e-7 in
+// the kernel above; heads of 24: 1.7e-7 / 6.9e-7, 1.2e-7 / 2.3e-7 and 1.3e-7 / 2.8e-7.
 // Bound by the MFMAs for prompts (2 x 32 cycles for 16 keys, 16 queries and 4 numbers) and by a chain of loads in single-token
 // steps.  Measured beside the kernel above (a lane per key on the vector units), 24 heads of 128 on 8: four prompts of 131 to 512 tokens
 // 600 -> 130 us a layer, one token for each of four sequences at 131 to 520 keys 29 -> 24 us (32 workgroups,
@@ -307,6 +311,7 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
     int n_tokens, int n_heads, int n_kv, int head_dim, float scale, int window, const float* __restrict__ sinks, int keep_first,
     float softcap, int chunk, const float* __restrict__ sig_bias, int tokens_per_block, int head_chunks) {
   constexpr int VW = NB < 4 ? NB : 4;                  // floats of a load of V
+  constexpr int CHAINS = 16 / NB;                      // the shorter a head, the more sums a unit's values go into
   constexpr int LD = 16 * NB + 4;                      // a query's row in LDS: outputs, then maximum and sum
   extern __shared__ __attribute__((aligned(16))) float merged[];      // [waves][16][LD]
   const int lane = threadIdx.x & (RB_WAVE - 1);
@@ -400,11 +405,14 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
       f32x4_t sc[2];
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        sc[b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        f32x4_t part[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < NB; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) sc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][c][i], qv[c][i], sc[b], 0, 0, 0);
+          for (int i = 0; i < 4; ++i) part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][c][i], qv[c][i], part[i], 0, 0, 0);
+        sc[b] = (part[0] + part[1]) + (part[2] + part[3]);
       }
       float top = -INFINITY;
       bool in_part = false;                   // some query of the run does not see one of these keys
@@ -432,10 +440,9 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float s = sc[b][i];
-          const float p = s == -INFINITY ? 0.f : (sig_bias ? 1.0f / (1.0f + expf(-(s + sb))) : expf(s - m_new));
-          l_run += p;
-          sc[b][i] = p;
+          sc[b][i] = s == -INFINITY ? 0.f : (sig_bias ? 1.0f / (1.0f + expf(-(s + sb))) : expf(s - m_new));
         }
+      l_run += ((sc[0][0] + sc[0][1]) + (sc[0][2] + sc[0][3])) + ((sc[1][0] + sc[1][1]) + (sc[1][2] + sc[1][3]));
 #pragma unroll
       for (int d = 0; d < NB; ++d) acc[d] *= corr;
       // Several tokens': where a query does not see all of these keys and a value is an infinity or a NaN, every query adds up the
@@ -473,12 +480,28 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
               }
         }
       } else {
+        f32x4_t unit[CHAINS][NB];
+#pragma unroll
+        for (int n = 0; n < CHAINS; ++n)
+#pragma unroll
+          for (int d = 0; d < NB; ++d) unit[n][d] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int d = 0; d < NB; ++d) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][i][d], sc[b][i], acc[d], 0, 0, 0);
+            for (int d = 0; d < NB; ++d) {
+              f32x4_t& sum = unit[(4 * b + i) % CHAINS][d];
+              sum = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][i][d], sc[b][i], sum, 0, 0, 0);
+            }
+#pragma unroll
+        for (int n = CHAINS / 2; n > 0; n /= 2)
+#pragma unroll
+          for (int m = 0; m < n; ++m)
+#pragma unroll
+            for (int d = 0; d < NB; ++d) unit[m][d] += unit[m + n][d];
+#pragma unroll
+        for (int d = 0; d < NB; ++d) acc[d] += unit[0][d];
       }
     }
     l_run += __shfl_xor(l_run, 16, RB_WAVE);

@@ -247,6 +247,37 @@ def test_float32_attention_of_tokens_in_any_order(lib, heads, kv, dim, more, ord
     _within(out.view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
 
 
+@pytest.mark.parametrize("heads,kv,dim", [(24, 8, 128), (16, 4, 64), (8, 2, 32), (32, 16, 20)])
+@pytest.mark.parametrize("past,new", [([0, 0], [131, 387]), ([400, 131, 300, 520, 900, 77, 30, 2000], [1] * 8), ([500], [60])])
+def test_float32_attention_is_as_exact_as_on_the_vector_units(lib, heads, kv, dim, past, new):
+    """The error against float64 is not larger than that of the kernel that takes the keys one by one on the vector units.  The relative
+    errors of 2,000 numbers and more are random ones of the same size: their norms are known to a few hundredths."""
+    g = torch.Generator().manual_seed(dim + sum(new))
+    lengths = [p + n for p, n in zip(past, new)]
+    kp, table, ks = _paged(lengths, kv, dim, g)
+    vp, vs = torch.full_like(kp, float("nan")), []
+    for b, n in enumerate(lengths):
+        x = torch.randn(n, kv, dim, generator=g)
+        for j in range(n):
+            vp[table[b, j // 64], :, j % 64] = x[j]
+        vs.append(x)
+    q = torch.randn(sum(new), heads, dim, generator=g)
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip(past, new)])
+    seq = torch.repeat_interleave(torch.arange(len(new)), torch.tensor(new))
+    want = torch.cat([_attention64(q[seq == b], ks[b], vs[b], pos[seq == b], dim ** -0.5) for b in range(len(new))])
+    args = [q.to(DEV), kp.to(DEV), vp.to(DEV)], [pos.int().to(DEV), seq.int().to(DEV), table.to(DEV), heads, kv, dim, dim ** -0.5, 0, None]
+    error = {}
+    try:
+        for mode in (1, 2):
+            lib._lib.rb_tune_attention_vec(mode)
+            out = torch.full((sum(new), heads * dim), float("nan"), device=DEV)
+            lib.attention_sinks(*args[0], out, *args[1])
+            error[mode] = float((out.view(want.shape).double().cpu() - want).norm() / want.norm())
+    finally:
+        lib._lib.rb_tune_attention_vec(1)
+    assert error[1] <= 1.1 * error[2], error
+
+
 # ---------------------------------------------------------------- products per head on the matrix cores
 @pytest.mark.parametrize("tokens", [1, 4, 16, 17, 200])
 @pytest.mark.parametrize("heads,k,n,more", [(1, 32, 16, {}), (3, 64, 96, {"rot": 32, "pad": 128}), (16, 128, 128, {}),
