@@ -1,7 +1,8 @@
 // Causal attention of each token over its sequence's paged cache: any head_dim up to
 // 512, any number of heads and groups, float32 or bfloat16 storage, float32 arithmetic
-// throughout (scores, softmax, weighted sum).  One workgroup per (token, query head): one wave
-// when the step has many tokens, up to 8 waves that share the pages of the context and merge
+// throughout (scores, softmax, weighted sum).  Float32 heads of up to 128 numbers run on the
+// matrix cores but in small steps (the last kernel); the others below take one workgroup per
+// (token, query head): one wave when the step has many tokens, up to 8 waves that share the pages of the context and merge
 // their running softmax states through LDS when it has few (a decode step of 8 sequences and
 // 32 heads would otherwise leave three quarters of the GPU idle, each wave walking its whole
 // context alone).
@@ -299,10 +300,10 @@ __device__ __forceinline__ int here(int x) {
 // as a tree before they meet the running ones, and so are its weights: one sum for everything had twice the error. Relative error of
 // the outputs, 24 heads of 128 at 131 to 512 keys / one token at 8,000: 3.2e-7 / 6.8e-7 with one sum, 1.5e-7 / 2.4e-7 now, 1.7e-7 / 4.4e-7 in
 // the kernel above; heads of 24: 1.7e-7 / 6.9e-7, 1.2e-7 / 2.3e-7 and 1.3e-7 / 2.8e-7.
-// Bound by the MFMAs for prompts (2 x 32 cycles for 16 keys, 16 queries and 4 numbers) and by a chain of loads in single-token
-// steps.  Measured beside the kernel above (a lane per key on the vector units), 24 heads of 128 on 8: four prompts of 131 to 512 tokens
-// 600 -> 130 us a layer, one token for each of four sequences at 131 to 520 keys 29 -> 24 us (32 workgroups,
-// whose matrix cores three of sixteen columns keep busy: what bounds it now).
+// Bound by the MFMAs for prompts (2 x 32 cycles for 16 keys, 16 queries and 4 numbers) and by a chain of loads in single-token steps.
+// Measured beside the kernel above (a lane per key on the vector units), 24 heads of 128 on 8: four prompts of 131 to 512 tokens 608 -> 130 us
+// a layer, four of 100 tokens 66 -> 27, 16 and 64 single tokens at 1,001 keys 53 -> 40 and 211 -> 112 us.  32 heads on 32: 862 -> 132 us,
+// 110 -> 35, 124 -> 113 and 724 -> 383.
 // ONE: a block is one token's.
 template <int NB, bool ONE>
 __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_kernel(
@@ -326,7 +327,12 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
   const int t1 = ONE ? t0 + 1 : t0 + tokens_per_block < n_tokens ? t0 + tokens_per_block : n_tokens;
   const int t = ONE ? t0 : t0 + col / h_count, h = ONE ? h0 + col : h0 + col % h_count;
   const bool on = ONE ? col < h_count : t < t1;
-  const int my_pos = on ? tok_pos[t] : -1;
+  // The block's tokens, a lane each (one trip to memory), and where a run of consecutive positions of one sequence starts among them.
+  const int count = t1 - t0;
+  const int l_seq = lane < count ? tok_seq[t0 + lane] : -1, l_pos = lane < count ? tok_pos[t0 + lane] : -1;
+  const int seq_before = __shfl_up(l_seq, 1, RB_WAVE), pos_before = __shfl_up(l_pos, 1, RB_WAVE);
+  unsigned long long starts = __ballot(lane == 0 || lane == count || (lane < count && (l_seq != seq_before || l_pos != pos_before + 1)));
+  const int my_pos = ONE ? __builtin_amdgcn_readfirstlane(l_pos) : __shfl(l_pos, t - t0, RB_WAVE);      // (of a column in use)
   const int my_lo = on ? first_visible(my_pos, window, chunk) : 0;
 
   f32x4_t qv[NB];
@@ -338,14 +344,16 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
   }
   const float sb = sig_bias && on ? sig_bias[h] : 0.f;
 
-  // Run after run of consecutive positions of one sequence: almost always the whole block is one.  Each starts anew and leaves with its
-  // own columns only, so that nothing of another sequence comes into a query's sums, and tokens may come in any order.
+  // Run after run: almost always the whole block is one.  Each starts anew and leaves with its own columns only, so that nothing of
+  // another sequence comes into a query's sums, and tokens may come in any order.
+  bool in_use = false;                        // what the waves share in LDS
   for (int seg = t0, end; seg < t1; seg = end) {
-    const int seq = tok_seq[seg];
-    end = seg + 1;
-    while (!ONE && end < t1 && tok_seq[end] == seq && tok_pos[end] == tok_pos[end - 1] + 1) ++end;
+    starts &= starts - 1;
+    end = ONE ? t1 : t0 + __builtin_ctzll(starts);
+    const int seq = __builtin_amdgcn_readlane(l_seq, seg - t0);
     const int32_t* pages = block_table + (size_t)seq * bt_stride;
-    const int hi = tok_pos[end - 1], lo = first_visible(tok_pos[seg], window, chunk);
+    const int hi = __builtin_amdgcn_readlane(l_pos, end - 1 - t0);
+    const int lo = first_visible(__builtin_amdgcn_readlane(l_pos, seg - t0), window, chunk);
     const bool mine = ONE ? on : t >= seg && t < end;
     auto sees = [&](int key) { return mine && key <= my_pos && (key >= my_lo || key < keep_first); };
     // A weight of 0 does not take an infinity or a NaN out of a matrix product.  One token's queries see the same keys: the values of
@@ -508,8 +516,9 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
     l_run += __shfl_xor(l_run, 32, RB_WAVE);
 
     // lane holds, for query col, the numbers NB (4 g + j) + d of the head
-    if (n_waves == 1) {
-      if (!mine) continue;
+    const int at_work = n_walk > n_waves ? n_waves : n_walk;      // waves that had keys: the first ones
+    if (at_work <= 1) {
+      if (!mine || wave > 0) continue;
       if (sinks) l_run += expf(sinks[h] - m_run);
       const float inv = sig_bias ? 1.0f : (l_run > 0.f ? 1.0f / l_run : 0.f);
       float* orow = out + ((size_t)t * n_heads + h) * head_dim + 4 * NB * g;
@@ -521,7 +530,8 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
           if (NB * j + d < left) orow[NB * j + d] = acc[d][j] * inv;
       continue;
     }
-    if (seg > t0) __syncthreads();            // the run before has been read
+    if (in_use) __syncthreads();              // the run before has been read
+    in_use = true;
     float* row = merged + ((size_t)wave * 16 + col) * LD;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -539,9 +549,9 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
       const int hh = h0 + cc % h_count;
       const float* src = merged + (size_t)cc * LD;
       float mx = -INFINITY;
-      for (int w = 0; w < n_waves; ++w) mx = fmaxf(mx, src[(size_t)w * 16 * LD + 16 * NB]);
+      for (int w = 0; w < at_work; ++w) mx = fmaxf(mx, src[(size_t)w * 16 * LD + 16 * NB]);
       float l = 0.f, o = 0.f;
-      for (int w = 0; w < n_waves; ++w) {
+      for (int w = 0; w < at_work; ++w) {
         const float mw = src[(size_t)w * 16 * LD + 16 * NB];
         const float f = mw == -INFINITY ? 0.f : expf(mw - mx);
         l += src[(size_t)w * 16 * LD + 16 * NB + 1] * f;
@@ -566,6 +576,7 @@ struct AttentionF32 {
   float softcap;
   int chunk;
   const float* sig_bias;
+  int n_seqs;            // 0: not known
 };
 
 template <int NB, bool ONE>
@@ -593,9 +604,14 @@ static int launch_attention_f32_blocks(const AttentionF32& a, int per_block, int
 template <int NB>
 static int launch_attention_f32(const AttentionF32& a, hipStream_t s) {
   const int group = a.n_heads / a.n_kv, chunks = (group + 15) / 16;
-  // One token a block while that leaves the GPU room (single-token steps above all: a block of tokens of several sequences takes
-  // them one after another), as many as the 16 columns hold beyond.
-  const int per_block = (long long)a.n_tokens * a.n_kv * chunks >= 4 * rb_compute_units() && group < 16 ? 16 / group : 1;
+  // How many tokens share a block's 16 columns: as many as fit where one token a block (whose other columns are idle) would make more
+  // blocks than the GPU has room for.  A block over a boundary takes its sequences one after another, so with several of them that is
+  // four blocks a compute unit, with one sequence one (24 heads of 128 on 8, one prompt of 100 tokens: 20.9 us with one token a block,
+  // 12.5 with 5; four of 16: 7.8 and 13.0; four of 100: 27), and never in a single-token step (32 sequences at 151 keys, 32 heads of
+  // 128: 32 us with one token a block, 145 with 16).
+  const long long blocks_of_one = (long long)a.n_tokens * a.n_kv * chunks;
+  const bool share = a.n_seqs != a.n_tokens && blocks_of_one >= (a.n_seqs == 1 ? 1 : 4) * rb_compute_units();
+  const int per_block = share && group < 16 ? 16 / group : 1;
   if (per_block == 1) return launch_attention_f32_blocks<NB, true>(a, 1, chunks, s);
   return launch_attention_f32_blocks<NB, false>(a, per_block, chunks, s);
 }
@@ -648,6 +664,19 @@ extern "C" int rb_attention_generic_chunked(const void* q, const void* k_pages, 
   RB_RECORDED(rb_attention_generic_chunked(q, k_pages, v_pages, out, dtype, tok_pos, tok_seq, block_table, bt_stride, n_tokens,
                                            n_heads, n_kv_heads, head_dim, scale, window, keep_first, softcap, sinks, chunk, sig_bias,
                                            stream));
+  return rb_attention_generic_steps(q, k_pages, v_pages, out, dtype, tok_pos, tok_seq, block_table, bt_stride, n_tokens, n_heads,
+                                    n_kv_heads, head_dim, scale, window, keep_first, softcap, sinks, chunk, sig_bias, 0, stream);
+}
+
+// The same, told how many sequences the tokens are of (0: not known; it decides between kernels, not what is computed).
+extern "C" int rb_attention_generic_steps(const void* q, const void* k_pages, const void* v_pages, void* out, int dtype,
+                                          const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* block_table,
+                                          int bt_stride, int n_tokens, int n_heads, int n_kv_heads, int head_dim,
+                                          float scale, int window, int keep_first, float softcap, const float* sinks, int chunk,
+                                          const float* sig_bias, int n_seqs, void* stream) {
+  RB_RECORDED(rb_attention_generic_steps(q, k_pages, v_pages, out, dtype, tok_pos, tok_seq, block_table, bt_stride, n_tokens,
+                                         n_heads, n_kv_heads, head_dim, scale, window, keep_first, softcap, sinks, chunk, sig_bias,
+                                         n_seqs, stream));
   RB_REQUIRE(keep_first >= 0 && softcap >= 0.f && chunk >= 0, "rb_attention_generic: negative keep_first, softcap or chunk");
   RB_REQUIRE(sig_bias == nullptr || sinks == nullptr, "rb_attention_generic: a sink belongs to the softmax");
   RB_REQUIRE(n_tokens >= 0 && n_heads > 0 && n_kv_heads > 0 && n_heads % n_kv_heads == 0,
@@ -659,9 +688,16 @@ extern "C" int rb_attention_generic_chunked(const void* q, const void* k_pages, 
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool wide = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) & 15) == 0;
-  if (dtype == RB_F32 && head_dim % 4 == 0 && head_dim <= 128 && wide && g_attention_vec == 1) {
+  // Small steps are a chain of trips to memory, which is shorter on the vector units: a workgroup a head there, whose 8 waves take 64 keys at
+  // once.  Single tokens (vector units / matrix cores, us): 32 heads of 128, one sequence of 151 / 1,001 keys 10.4 and 28.6 / 11.4 and 37;
+  // four sequences on 32 kv heads 10.6 and 40.8 / 11.7 and 41.0, on 8 10.7 and 38.4 / 11.8 and 37.2; 16 on 8 12.5 and 66.7 / 11.9 and 41; 16 heads
+  // of 64 on 8, four sequences 7.8 and 18 / 8.0 and 20.5.  Prompts: 24 heads of 128 on 8, 8 tokens 5.9 / 7.4, 30 tokens 7.5 / 7.8, 60 tokens
+  // 11.2 / 10.6; 4 heads of 24 on 2, 30 tokens 5.9 / 5.2.
+  const bool single = n_seqs == n_tokens;
+  const bool few = (long long)n_tokens * n_heads * head_dim <= (single ? 64LL : n_seqs > 0 && head_dim > 32 ? 128LL : 0LL) * rb_compute_units();
+  if (dtype == RB_F32 && head_dim % 4 == 0 && head_dim <= 128 && wide && g_attention_vec == 1 && !few) {
     const AttentionF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, (float*)out, tok_pos, tok_seq, block_table,
-                            bt_stride, n_tokens, n_heads, n_kv_heads, head_dim, scale, window, sinks, keep_first, softcap, chunk, sig_bias};
+                            bt_stride, n_tokens, n_heads, n_kv_heads, head_dim, scale, window, sinks, keep_first, softcap, chunk, sig_bias, n_seqs};
     const int rc = head_dim <= 32 ? launch_attention_f32<2>(a, s) : head_dim <= 64 ? launch_attention_f32<4>(a, s) : launch_attention_f32<8>(a, s);
     if (rc) return rc;
     RB_LAUNCH_CHECK();

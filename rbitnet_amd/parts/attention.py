@@ -362,7 +362,7 @@ class Attention(Part):
         else:
             lib.attention_opts(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, view.block_table, hq, hk, d,
                                self.scale, window, self.keep_first, self.softcap or 0.0, self.sink, chunk=self.chunk or 0,
-                               sig_bias=self.score_bias)
+                               sig_bias=self.score_bias, n_seqs=ctx.n_seqs)
         return self._gate_and_project(attn, h, stream, next_norm)
 
     def _forward_mixed(self, h, ctx, view, stream, next_norm):
@@ -448,7 +448,7 @@ class Attention(Part):
                                        ctx.n_seqs, ctx.max_q_len, hq, hk, d, self.scale, window, sinks=self.sink)
         else:
             lib.attention_sinks(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, bt, hq, hk, d,
-                                self.scale, window, self.sink)
+                                self.scale, window, self.sink, n_seqs=ctx.n_seqs)
         return self._gate_and_project(attn, h, stream, next_norm)
 
 

@@ -180,7 +180,7 @@ class LatentAttention(Part):
                                        ctx.max_q_len, self.heads, 1, r, self.scale, None, sinks=self.sink)
         else:
             lib.attention_sinks(q3, pages, pages, ol, ctx.tok_pos, ctx.tok_seq, view.block_table, self.heads, 1, r,
-                                self.scale, None, self.sink)
+                                self.scale, None, self.sink, n_seqs=ctx.n_seqs)
         o = torch.empty((t, self.heads * self.vdim), dtype=dt, device=h.device)
         # the latent's part of every head's sum through the head's value matrix, the head's gate on the way out
         lib.heads_linear_part(ol, r, self.w_uv, o, self.vdim, gate=down if self.has_gate else None, gate_col=self.gate_col,

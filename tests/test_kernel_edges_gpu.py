@@ -247,6 +247,33 @@ def test_float32_attention_of_tokens_in_any_order(lib, heads, kv, dim, more, ord
     _within(out.view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
 
 
+@pytest.mark.parametrize("heads,kv,dim", [(32, 32, 128), (4, 2, 24), (24, 8, 128), (16, 16, 64)])
+@pytest.mark.parametrize("past,new", [([70] * 3, [1] * 3), ([70, 3, 129, 0] * 9, [1] * 36), ([0], [6]), ([100], [40]), ([0, 9, 0], [16, 16, 16]),
+                                      ([0], [130])])
+def test_float32_attention_by_how_many_sequences_a_step_has(lib, heads, kv, dim, past, new):
+    """Single-token steps, one prompt and several, on either side of the lines between the kernels and the splits; the count decides between
+    kernels and not what is computed."""
+    g = torch.Generator().manual_seed(heads + dim + sum(new))
+    lengths = [p + n for p, n in zip(past, new)]
+    kp, table, ks = _paged(lengths, kv, dim, g)
+    vp, vs = torch.full_like(kp, float("nan")), []
+    for b, n in enumerate(lengths):
+        x = torch.randn(n, kv, dim, generator=g)
+        for j in range(n):
+            vp[table[b, j // 64], :, j % 64] = x[j]
+        vs.append(x)
+    q, sinks = torch.randn(sum(new), heads, dim, generator=g), torch.randn(heads, generator=g)
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip(past, new)])
+    seq = torch.repeat_interleave(torch.arange(len(new)), torch.tensor(new))
+    want = torch.cat([_attention64(q[seq == b], ks[b], vs[b], pos[seq == b], dim ** -0.5, sinks=sinks) for b in range(len(new))])
+    for n_seqs in (0, len(new)):
+        for more in ({}, {"keep_first": 0, "softcap": 0.0}):
+            out = torch.full((sum(new), heads * dim), float("nan"), device=DEV)
+            args = [q.to(DEV), kp.to(DEV), vp.to(DEV), out, pos.int().to(DEV), seq.int().to(DEV), table.to(DEV), heads, kv, dim, dim ** -0.5, 0]
+            (lib.attention_opts if more else lib.attention_sinks)(*args, *more.values(), sinks.to(DEV), n_seqs=n_seqs)
+            _within(out.view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
+
+
 @pytest.mark.parametrize("heads,kv,dim", [(24, 8, 128), (16, 4, 64), (8, 2, 32), (32, 16, 20)])
 @pytest.mark.parametrize("past,new", [([0, 0], [131, 387]), ([400, 131, 300, 520, 900, 77, 30, 2000], [1] * 8), ([500], [60])])
 def test_float32_attention_is_as_exact_as_on_the_vector_units(lib, heads, kv, dim, past, new):
