@@ -343,9 +343,6 @@ int rb_latent_norm_store(const float* proj, long long stride, int q_rank, const 
                          int kv_rank, const float* kv_gain, void* pages, int dtype, const int32_t* tok_pos,
                          const int32_t* tok_seq, const int32_t* block_table, int bt_stride, float eps, int n_tokens,
                          void* stream);
-// y[t, h, n] = sum_k w[h, k, n] x[t, h, k]
-int rb_heads_linear(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype, int n_tokens, int n_heads,
-                    int n, int k, void* stream);
 
 // ---- a norm on the sublayer's output, limits in the gated unit, and what the mixers of such layers need
 // x <- (assign ? 0 : x) + y / sqrt(mean(y^2) + eps) * gain with y = sa * a + sb * b (b null: sa * a), rows of `width` float32
@@ -466,13 +463,11 @@ int rb_linear_recurrence_bonus(const float* q, const float* k, long long qk_stri
 int rb_gated_rmsnorm_heads(const float* o, const float* weight, long long weight_head_stride, const float* gate,
                            long long gate_stride, int act, float eps, void* out, int out_dtype, int n_tokens, int n_heads, int vdim,
                            void* stream);
-// rb_heads_linear on a part of every head: a head of x takes x_head_stride numbers (the first k are read), a head of y
-// y_head_stride (the first n are written).
-int rb_heads_linear_strided(const void* x, int x_dtype, long long x_head_stride, const void* w, int w_dtype, void* y, int y_dtype,
-                            long long y_head_stride, int n_tokens, int n_heads, int n, int k, void* stream);
-// rb_heads_linear_strided with two things in the same launch: a gate per head on the outputs (gate float32, rows gate_stride
-// apart, null: none: head h of token t times sigmoid(gate[t * gate_stride + h])), and (rot >= 0) the `rot` numbers at x_rot_col
-// of every head of x rotated by the token's position into y at y_rot_col >= n, with zeros behind them up to y_head_stride.
+// y[t, h, n] = sum_k w[h, k, n] x[t, h, k] on a part of every head: a head of x takes x_head_stride numbers (the first k are read), a
+// head of y y_head_stride (the first n are written).  Two things may ride in the launch: a gate per head on the outputs (gate float32, rows
+// gate_stride apart, null: none: head h of token t times sigmoid(gate[t * gate_stride + h])), and (rot >= 0) the `rot` numbers at x_rot_col
+// of every head of x rotated by the token's position into y at y_rot_col >= n, with zeros behind them up to y_head_stride.  w_layout 1: every
+// head's [N, K] fragment-major.
 int rb_heads_linear_more(const void* x, int x_dtype, long long x_head_stride, const void* w, int w_dtype, int w_layout, void* y, int y_dtype,
                          long long y_head_stride, int n_tokens, int n_heads, int n, int k, const float* gate, long long gate_stride,
                          int rot, int x_rot_col, int y_rot_col, const float* cos, const float* sin, int style,

@@ -324,23 +324,8 @@ static void launch_heads_mfma(const void* x, const void* w, void* y, int n_token
 #undef HM_GO
 }
 
-extern "C" int rb_heads_linear(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype, int n_tokens,
-                               int n_heads, int n, int k, void* stream) {
-  RB_RECORDED(rb_heads_linear(x, x_dtype, w, w_dtype, y, y_dtype, n_tokens, n_heads, n, k, stream));
-  return rb_heads_linear_strided(x, x_dtype, k, w, w_dtype, y, y_dtype, n, n_tokens, n_heads, n, k, stream);
-}
-
-// The same with a head of x taking x_head_stride numbers (the first k of them are read) and a head of y y_head_stride
-// (the first n are written): products on a part of every head, into a part of every head.
-extern "C" int rb_heads_linear_strided(const void* x, int x_dtype, long long x_head_stride, const void* w, int w_dtype, void* y,
-                                       int y_dtype, long long y_head_stride, int n_tokens, int n_heads, int n, int k, void* stream) {
-  RB_RECORDED(rb_heads_linear_strided(x, x_dtype, x_head_stride, w, w_dtype, y, y_dtype, y_head_stride, n_tokens, n_heads, n, k,
-                                      stream));
-  return rb_heads_linear_more(x, x_dtype, x_head_stride, w, w_dtype, 0, y, y_dtype, y_head_stride, n_tokens, n_heads, n, k, nullptr, 0,
-                              -1, 0, 0, nullptr, nullptr, 0, nullptr, stream);
-}
-
-// The same with two things in the same launch.  gate (float32, rows gate_stride apart; null: none): head h's outputs of token t
+// y[t, h, :n] = w[h]^T x[t, h, :k] (w [H, K, N]): a head of x takes x_head_stride numbers (the first k are read), a head of y
+// y_head_stride (the first n are written).  Two things may ride in the launch.  gate (float32, rows gate_stride apart; null: none): head h's outputs of token t
 // are multiplied by sigmoid(gate[t * gate_stride + h]).  rot >= 0 (rot < 0: none): the `rot` numbers at x_rot_col of every head
 // of x, rotated by the token's position (cos, sin [positions, rot / 2]; style 0: 2i with 2i + 1, 1: i with i + rot / 2), go to
 // y at y_rot_col, and what lies behind them in a head of y becomes zero.  w_layout 1: every head's [N, K] fragment-major (bfloat16, K 32,

@@ -12,7 +12,7 @@ A layer with `cache_from = j` has no Wdkv: it reads the latents that layer j sto
 The products with Wuk and Wuv are moved to the query's side, so that attention runs over the cached latents
 themselves, one key/value head of size kv_rank shared by all query heads:
     score = (Wuk_i^T q_i) . c_j,      sum_j w_j v_j = Wuv_i (sum_j w_j c_j)
-which costs a product per head on either side of attention (`heads_linear`) and never expands the cache, whatever
+which costs a product per head on either side of attention (`heads_linear_part`) and never expands the cache, whatever
 the step brings on top of whatever past.  Scores, softmax and norms in float32.
 
 With a rotated part (`rot_dim` > 0 and a `position` part whose rotation covers rot_dim numbers): a query head is
