@@ -420,8 +420,8 @@ class Attention(Part):
         tables = getattr(self.position, "rotation_tables", None)
         if decode and owns and tables is not None and self.same_sizes:
             # one kernel: rotation, cache write, attention over the pages
-            # (a window bounds the walk; heads with sinks stand in front of routed experts, whose choice a sum in another order
-            # may turn where two are as good as equal, and keep their order)
+            # (a window bounds the walk; heads with sinks are dealt as `decode_splits` says: the wider deal adds up in another order,
+            # which in a model whose routers stand behind such heads turned choices between experts that are as good as equal)
             cos, sin, style = tables()
             n_splits, workspace = ctx.decode_workspace(hq, d, hk, spread=window == 0 and self.sink is None)
             lib.attention_decode_fused_bf16(qkv, cos, sin, style, view.k_pages, view.v_pages, attn, ctx.tok_pos, bt,

@@ -442,6 +442,41 @@ def test_single_token_attention_over_many_pages(lib, dim, heads, kv, length, spl
         assert torch.equal(out, outs[0])
 
 
+@pytest.mark.parametrize("heads,kv,dim", [(32, 8, 128), (16, 1, 64), (8, 8, 128)])
+@pytest.mark.parametrize("splits", [1, 3, 8, 9, 16, 65])
+@pytest.mark.parametrize("sink", [False, True])
+def test_single_token_attention_dealt_to_many_workgroups(lib, heads, kv, dim, splits, sink):
+    """The kernel that rotates and stores, and the combination behind it: fewer and more workgroups than pages, than loads in flight and than
+    lanes, with sequences of one page beside longer ones."""
+    g = torch.Generator().manual_seed(heads + splits)
+    lengths = [1, 70, 1500]
+    kp, table, ks = _paged(lengths, kv, dim, g)
+    vp, vs = torch.full_like(kp, float("nan")), []
+    for b, n in enumerate(lengths):
+        x = torch.randn(n, kv, dim, generator=g)
+        for j in range(n):
+            vp[table[b, j // 64], :, j % 64] = x[j]
+        vs.append(x)
+    q = torch.randn(3, heads, dim, generator=g)
+    last = lambda rows: torch.stack([x[-1] for x in rows])
+    qkv = torch.cat([q.flatten(1), last(ks).flatten(1), last(vs).flatten(1)], 1)
+    sinks = torch.randn(heads, generator=g) if sink else None
+    pos = torch.tensor(lengths, dtype=torch.int32) - 1
+    r = lambda x: x.bfloat16().float()
+    want = torch.cat([_attention64(r(q[b:b + 1]), r(ks[b]), r(vs[b]), pos[b:b + 1].long(), 0.1, sinks=sinks) for b in range(3)])
+    kd, vd = kp.bfloat16().to(DEV), vp.bfloat16().to(DEV)
+    for b, n in enumerate(lengths):                               # the token itself is the kernel's to store
+        for pages in (kd, vd):
+            pages[table[b, (n - 1) // 64], :, (n - 1) % 64] = float("nan")
+    cos, sin = torch.ones(1600, dim // 2, device=DEV), torch.zeros(1600, dim // 2, device=DEV)
+    ws = torch.full((3 * heads * splits * (dim + 2),), float("nan"), device=DEV)
+    out = torch.full((3, heads * dim), float("nan"), dtype=torch.bfloat16, device=DEV)
+    lib.attention_decode_fused_bf16(qkv.to(DEV), cos, sin, 1, kd, vd, out, pos.to(DEV), table.to(DEV), heads, kv, dim, 0.1, None, splits, ws,
+                                    sinks=None if sinks is None else sinks.to(DEV))
+    # weights and outputs are rounded to 8 bits each
+    _within(out.view(want.shape), want, 2.0 ** -7 * float(max(x.abs().max() for x in vs)))
+
+
 # ---------------------------------------------------------------- float32 products of few tokens, any depth
 @pytest.mark.parametrize("m", [1, 4, 16])
 @pytest.mark.parametrize("n,k", [(1, 4), (15, 12), (16, 20), (17, 96), (33, 124), (48, 132), (96, 252), (40, 260), (144, 500), (10, 516), (5, 1348)])
