@@ -688,13 +688,12 @@ extern "C" int rb_attention_generic_steps(const void* q, const void* k_pages, co
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool wide = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) & 15) == 0;
-  // Small steps are a chain of trips to memory, which is shorter on the vector units: a workgroup a head there, whose 8 waves take 64 keys at
-  // once.  Single tokens (vector units / matrix cores, us): 32 heads of 128, one sequence of 151 / 1,001 keys 10.4 and 28.6 / 11.4 and 37;
-  // four sequences on 32 kv heads 10.6 and 40.8 / 11.7 and 41.0, on 8 10.7 and 38.4 / 11.8 and 37.2; 16 on 8 12.5 and 66.7 / 11.9 and 41; 16 heads
-  // of 64 on 8, four sequences 7.8 and 18 / 8.0 and 20.5.  Prompts: 24 heads of 128 on 8, 8 tokens 5.9 / 7.4, 30 tokens 7.5 / 7.8, 60 tokens
-  // 11.2 / 10.6; 4 heads of 24 on 2, 30 tokens 5.9 / 5.2.
-  const bool single = n_seqs == n_tokens;
-  const bool few = (long long)n_tokens * n_heads * head_dim <= (single ? 64LL : n_seqs > 0 && head_dim > 32 ? 128LL : 0LL) * rb_compute_units();
+  // Small steps of longer heads are a chain of trips to memory, which is shorter on the vector units: a workgroup a head there, whose 8 waves
+  // take 64 keys at once.  Single tokens (vector units / matrix cores, us): 32 heads of 128, one sequence of 81 / 151 / 1,001 keys 9.8, 10.4 and
+  // 28.6 / 8.3, 11.4 and 37; 16 heads of 64, four sequences of 151 / 1,001 keys 7.8 and 18 / 8.0 and 20.5.  Behind the line: 24 heads of 128 on 8, four
+  // sequences of 151 / 601 keys 10.6 and 32.4 / 11.8 and 23.1.  Prompts: 24 heads of 128 on 8, 8 tokens 5.9 / 7.4, 30 tokens 7.5 / 7.8,
+  // 60 tokens 11.2 / 10.6.  Heads of 24: 4 of them, four sequences of 81 / 301 keys 6.2 and 6.5 / 5.4 and 7.7, 30 tokens 5.9 / 5.2.
+  const bool few = n_seqs > 0 && head_dim > 32 && (long long)n_tokens * n_heads * head_dim <= (n_seqs == n_tokens ? 32LL : 128LL) * rb_compute_units();
   if (dtype == RB_F32 && head_dim % 4 == 0 && head_dim <= 128 && wide && g_attention_vec == 1 && !few) {
     const AttentionF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, (float*)out, tok_pos, tok_seq, block_table,
                             bt_stride, n_tokens, n_heads, n_kv_heads, head_dim, scale, window, sinks, keep_first, softcap, chunk, sig_bias, n_seqs};
