@@ -1,7 +1,7 @@
 // Causal attention of each token over its sequence's paged cache: any head_dim up to
 // 512, any number of heads and groups, float32 or bfloat16 storage, float32 arithmetic
 // throughout (scores, softmax, weighted sum).  Float32 heads of up to 128 numbers run on the
-// matrix cores but in small steps (the last kernel); the others below take one workgroup per
+// matrix cores (the last kernel); the others take one workgroup per
 // (token, query head): one wave when the step has many tokens, up to 8 waves that share the pages of the context and merge
 // their running softmax states through LDS when it has few (a decode step of 8 sequences and
 // 32 heads would otherwise leave three quarters of the GPU idle, each wave walking its whole
@@ -301,9 +301,10 @@ __device__ __forceinline__ int here(int x) {
 // the outputs, 24 heads of 128 at 131 to 512 keys / one token at 8,000: 3.2e-7 / 6.8e-7 with one sum, 1.5e-7 / 2.4e-7 now, 1.7e-7 / 4.4e-7 in
 // the kernel above; heads of 24: 1.7e-7 / 6.9e-7, 1.2e-7 / 2.3e-7 and 1.3e-7 / 2.8e-7.
 // Bound by the MFMAs for prompts (2 x 32 cycles for 16 keys, 16 queries and 4 numbers) and by a chain of loads in single-token steps.
-// Measured beside the kernel above (a lane per key on the vector units), 24 heads of 128 on 8: four prompts of 131 to 512 tokens 608 -> 130 us
-// a layer, four of 100 tokens 66 -> 27, 16 and 64 single tokens at 1,001 keys 53 -> 40 and 211 -> 112 us.  32 heads on 32: 862 -> 132 us,
-// 110 -> 35, 124 -> 113 and 724 -> 383.
+// Measured beside the kernel above (a lane per key on the vector units; caches as a step finds them: what the step wrote is not in a
+// workgroup's own, keys of earlier steps are in none), 24 heads of 128 on 8: four prompts of 131 to 512 tokens 608 -> 130 us a layer, one
+// of 8 / 30 / 100 tokens 7.0 / 10.1 / 28 -> 8.0 / 8.2 / 12.7; single tokens at 150 / 1,000 keys: one sequence 22 / 51 -> 13.5 / 42, 16 27 / 88 -> 16 / 70,
+// 64 55 / 246 -> 39 / 162.  32 heads on 32, 64 sequences 159 / 784 -> 133 / 418.
 // ONE: a block is one token's.
 template <int NB, bool ONE>
 __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_kernel(
@@ -606,9 +607,9 @@ static int launch_attention_f32(const AttentionF32& a, hipStream_t s) {
   const int group = a.n_heads / a.n_kv, chunks = (group + 15) / 16;
   // How many tokens share a block's 16 columns: as many as fit where one token a block (whose other columns are idle) would make more
   // blocks than the GPU has room for.  A block over a boundary takes its sequences one after another, so with several of them that is
-  // four blocks a compute unit, with one sequence one (24 heads of 128 on 8, one prompt of 100 tokens: 20.9 us with one token a block,
-  // 12.5 with 5; four of 16: 7.8 and 13.0; four of 100: 27), and never in a single-token step (32 sequences at 151 keys, 32 heads of
-  // 128: 32 us with one token a block, 145 with 16).
+  // four blocks a compute unit, with one sequence one (24 heads of 128 on 8, one prompt of 100 tokens: 21.4 us with one token a block,
+  // 12.7 with 5; four of 16: 8.7 and 13; four of 40: 14.0 and 10.6), and never in a single-token step (32 sequences at 150 / 1,000 keys, 32
+  // heads of 128: 66 / 240 us with one token a block, 177 / 630 with 16).
   const long long blocks_of_one = (long long)a.n_tokens * a.n_kv * chunks;
   const bool share = a.n_seqs != a.n_tokens && blocks_of_one >= (a.n_seqs == 1 ? 1 : 4) * rb_compute_units();
   const int per_block = share && group < 16 ? 16 / group : 1;
@@ -688,13 +689,7 @@ extern "C" int rb_attention_generic_steps(const void* q, const void* k_pages, co
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool wide = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) & 15) == 0;
-  // Small steps of longer heads are a chain of trips to memory, which is shorter on the vector units: a workgroup a head there, whose 8 waves
-  // take 64 keys at once.  Single tokens (vector units / matrix cores, us): 32 heads of 128, one sequence of 81 / 151 / 1,001 keys 9.8, 10.4 and
-  // 28.6 / 8.3, 11.4 and 37; 16 heads of 64, four sequences of 151 / 1,001 keys 7.8 and 18 / 8.0 and 20.5.  Behind the line: 24 heads of 128 on 8, four
-  // sequences of 151 / 601 keys 10.6 and 32.4 / 11.8 and 23.1.  Prompts: 24 heads of 128 on 8, 8 tokens 5.9 / 7.4, 30 tokens 7.5 / 7.8,
-  // 60 tokens 11.2 / 10.6.  Heads of 24: 4 of them, four sequences of 81 / 301 keys 6.2 and 6.5 / 5.4 and 7.7, 30 tokens 5.9 / 5.2.
-  const bool few = n_seqs > 0 && head_dim > 32 && (long long)n_tokens * n_heads * head_dim <= (n_seqs == n_tokens ? 32LL : 128LL) * rb_compute_units();
-  if (dtype == RB_F32 && head_dim % 4 == 0 && head_dim <= 128 && wide && g_attention_vec == 1 && !few) {
+  if (dtype == RB_F32 && head_dim % 4 == 0 && head_dim <= 128 && wide && g_attention_vec == 1) {
     const AttentionF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, (float*)out, tok_pos, tok_seq, block_table,
                             bt_stride, n_tokens, n_heads, n_kv_heads, head_dim, scale, window, sinks, keep_first, softcap, chunk, sig_bias, n_seqs};
     const int rc = head_dim <= 32 ? launch_attention_f32<2>(a, s) : head_dim <= 64 ? launch_attention_f32<4>(a, s) : launch_attention_f32<8>(a, s);
