@@ -187,6 +187,40 @@ def test_float32_tiles_in_parts(lib, tile, m, n, k):
         lib._lib.rb_tune_f32_tile(0)
 
 
+@pytest.mark.parametrize("frag", [False, True])
+def test_float32_product_with_an_undefined_token_costs_no_multiple(lib, frag):
+    """A token that is no number is computed again on the float32 matrix core: about three times the product's time where every
+    token is one; other tokens keep their bits."""
+    m, n, k = 1000, 4096, 3072
+    g = torch.Generator().manual_seed(3)
+    a, w = torch.randn(m, k, generator=g).to(DEV), torch.randn(n, k, generator=g).to(DEV)
+    if frag:
+        rows, w = w, torch.empty_like(w)
+        lib.place_rows(rows, w, frag=True)
+
+    def run(x):
+        c, times = torch.empty(m, n, device=DEV), []
+        for _ in range(5):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            lib.gemm_generic(x, w, c, w_frag=frag)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return c, min(times)
+
+    whole, finite = run(a)
+    bad = a.clone()
+    bad[37, 5] = float("nan")
+    c, with_one = run(bad)
+    assert torch.isnan(c[37]).all()
+    keep = torch.arange(m, device=DEV) != 37
+    assert torch.equal(c[keep], whole[keep])
+    c, with_all = run(torch.full_like(a, float("nan")))
+    assert torch.isnan(c).all()
+    assert with_one < 4 * finite and with_all < 8 * finite, (finite, with_one, with_all)
+
+
 @pytest.mark.parametrize("m,n", [(256, 2112), (250, 2100), (256, 4352)])
 def test_float32_product_in_two_launches(lib, m, n):
     """Whole rounds of a large tile (of 8 compute units, for small operands), and the rows that are left with another tile."""
