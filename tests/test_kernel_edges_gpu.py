@@ -187,6 +187,67 @@ def test_float32_tiles_in_parts(lib, tile, m, n, k):
         lib._lib.rb_tune_f32_tile(0)
 
 
+def _both_layouts(lib, w):
+    wf = torch.empty_like(w)
+    lib.place_rows(w, wf, frag=True)
+    return ((w, False), (wf, True))
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
+def test_float32_tiles_hold_every_bit_of_a_product(lib, tile):
+    """One depth value of a token is not zero, another one for every token, so that a result is one product and no bound grows with
+    K: 12 K tiles, those whose sums are turned among them, both layouts, numbers of 24 bits and the pair whose left-out
+    products of parts are largest."""
+    m, n, k = 131, 208, 384
+    g = torch.Generator().manual_seed(tile)
+    bits = lambda *size: (torch.randint(0, 1 << 22, size, generator=g) * 2 + (1 << 23) + 1).float() * 2.0 ** -23
+    a, w = torch.zeros(m, k), bits(n, k) * torch.randint(0, 2, (n, k), generator=g).mul(2).sub(1)
+    at = torch.arange(m) * 3 % k
+    a[torch.arange(m), at] = bits(m)
+    a[7, at[7]] = a[90, at[90]] = 1.0039138793945312
+    w[5, at[7]], w[6, at[90]] = 1.0039138793945312, -1.0039138793945312
+    want = a.double() @ w.double().T
+    # the last of six additions rounds down, 2^-23 of the result at most, the products left out are 2^-24, the other additions 2^-30 each
+    bound = (2.0 ** -23 + 2.0 ** -24 + 2.0 ** -27) * want.abs()
+    two = lambda x: x.bfloat16().double() + (x - x.bfloat16().float()).bfloat16().double()
+    assert ((two(a) @ two(w).T - want).abs() > bound).double().mean() > 0.5          # two parts would not pass
+    try:
+        lib._lib.rb_tune_f32_tile(tile)
+        for weights, frag in _both_layouts(lib, w.to(DEV)):
+            c = torch.full((m, n), float("nan"), device=DEV)
+            lib.gemm_generic(a.to(DEV), weights, c, w_frag=frag)
+            _within(c, want, bound)
+    finally:
+        lib._lib.rb_tune_f32_tile(0)
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("scale", [1e-30, 1e-36, 1e-40, 1e31])
+def test_float32_tiles_over_the_range_of_exponents(lib, tile, scale):
+    """Operands near the ends of the exponents' range, one side at a time: as close as float32 sums of them are, down to numbers
+    that are subnormal."""
+    m, n, k = 131, 208, 384
+    g = torch.Generator().manual_seed(tile)
+    for small in (0, 1):
+        a, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
+        if small:
+            a = a * scale
+        else:
+            w = w * scale
+        want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+        try:
+            lib._lib.rb_tune_f32_tile(tile)
+            for weights, frag in _both_layouts(lib, w.to(DEV)):
+                c = torch.full((m, n), float("nan"), device=DEV)
+                lib.gemm_generic(a.to(DEV), weights, c, w_frag=frag)
+                _within(c, want, 2.0 ** -24 * (k + 1) * size + 2.0 ** -149)
+                off = (c.double().cpu() - want).norm() / want.norm()
+                # K roundings, each to 24 bits or to a subnormal's last place, are as good as independent: a tenth of what they could add up to
+                assert off <= 0.1 * k * (2.0 ** -24 + 2.0 ** -149 / want.square().mean().sqrt()), (small, frag, float(off))
+        finally:
+            lib._lib.rb_tune_f32_tile(0)
+
+
 @pytest.mark.parametrize("frag", [False, True])
 def test_float32_product_with_an_undefined_token_costs_no_multiple(lib, frag):
     """A token that is no number is computed again on the float32 matrix core: about three times the product's time where every
