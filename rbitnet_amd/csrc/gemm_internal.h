@@ -45,8 +45,9 @@ bool gemm_resident_try(const GemmTokens& x, const bf16_t* w, void* c, int dtype_
                        int n, int k, hipStream_t s, int* rc);
 // more than 16 tokens (more than 64 when K is no multiple of 64): tiles through LDS
 // (gemm_tiled.hip).  gemm_tiled_parts: 0 when these sizes are not for it, else the number of K
-// slices it will use; more than 1 needs parts * m * n floats of workspace.
-int gemm_tiled_parts(int m, int n, int k, int epilogue);
+// slices it will use; more than 1 needs parts * m * n floats of workspace.  own_sum: the slices are added up by a launch
+// of the product's own, not by the kernel that reads them; a product that is one slice then is one for itself, too.
+int gemm_tiled_parts(int m, int n, int k, int epilogue, bool own_sum);
 int gemm_tiled_launch(const bf16_t* x, const bf16_t* w, bool w_frag, void* c, float* workspace, int dtype_out,
                       int epilogue, int m, int n, int k, hipStream_t s, const float* act = nullptr);
 // float32, more than 16 tokens, K % 32 == 0: tiles through LDS on the float32 MFMA (gemm_f32.hip); false: these operands are not

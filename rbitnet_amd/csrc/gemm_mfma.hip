@@ -17,9 +17,9 @@ extern "C" void rb_tune_use_resident(int on) {      // experiments only
 }
 extern "C" void rb_tune_use_stream(int on) { g_use_tiled_small = on; }     // experiments only: 0 = skinny up to 64 tokens
 
-static int tiled_parts(int m, int n, int k, int epilogue) {
+static int tiled_parts(int m, int n, int k, int epilogue, bool own_sum = true) {
   if (m <= 64 && !g_use_tiled_small) return 0;
-  return gemm_tiled_parts(m, n, k, epilogue);
+  return gemm_tiled_parts(m, n, k, epilogue, own_sum);
 }
 
 extern "C" long long rb_gemm_workspace_floats(int m, int n, int k, int epilogue) {
@@ -80,7 +80,7 @@ extern "C" int rb_gemm_bf16_act(const void* a, const void* w, int w_layout, void
 // The product as the terms its K slices computed, [terms, M, N] float32, for a caller that adds
 // them up with something else (rb_add_rmsnorm does).  One term: the product itself.
 extern "C" int rb_gemm_bf16_terms_count(int m, int n, int k) {
-  const int p = (m > 0 && n > 0 && k > 0 && k % 8 == 0) ? tiled_parts(m, n, k, 0) : 0;
+  const int p = (m > 0 && n > 0 && k > 0 && k % 8 == 0) ? tiled_parts(m, n, k, 0, false) : 0;
   return p > 1 ? p : 1;
 }
 

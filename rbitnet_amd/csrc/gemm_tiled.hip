@@ -330,54 +330,64 @@ extern "C" void rb_tune_tiles(int cfg, int parts) {       // experiments only; 0
 }
 
 // The choice among the tiles that are loaded straight into LDS and the number of K slices is the least of an estimate
-// of every candidate's time, a sum whose terms were fitted to measured products: for more than 64 tokens 609 products (the
-// products of a layer of six model shapes, hidden sizes 1,024 to 5,120, and others as the mixers have them, at 72 to 8,700
-// tokens, every tile with 1 to 8 slices forced in turn; `bench.py --planner-sweep` repeats such a sweep), for 17 to 64 tokens
-// 96 of six shapes at 24 to 64.
+// of every candidate's time, a sum whose terms were fitted to measured products: for more than 64 tokens 13,400 times of 580 products (29
+// sizes of W, K 512 to 14,336, at 65 to 8,192 tokens, every tile with 1 to 8 slices forced in turn, W rotated over copies beyond the
+// caches, the sums of slices apart; `bench.py --planner-sweep` repeats such a sweep), for 17 to 64 tokens 96 of six shapes at 24 to 64.
 //
 //   time [us] = c0 + K tiles of a slice x (what the compute units' tiles cost per K tile)
-//               + fixed x (tiles on the busiest compute unit)
-//               + slab x (MB of partial sums, when K is cut) + gate x (millions of gated outputs)
+//               + fixed x (tiles on the busiest compute unit) + w x MB of W
+//               + out x MB of float32 outputs, slices among them, or gate x millions of gated pairs
+//               + what adding up the slices takes
 //
-// A launch of w workgroups fills `slots` places at a time (the compute units, or twice as many for
-// the tiles of which two fit on one): w / slots full rounds at `full` each, and a last round of
+// A round is one tile on every compute unit (`per_unit` tiles where that many fit), and in K tiles
+// of 64 it costs `full`; a product's w workgroups are full rounds and a last one of
 // rem workgroups.  A last round is cheaper than a full one and the cheaper the emptier (the
 // compute units that have work share the memory system with fewer): `last + per_fill x rem / units`,
 // and for the tiles that fit twice, once every unit has one, `second + per_second x (rem - units) / units`.
-// The machine enters through the number of compute units alone.  The slabs are priced with what reading them again costs the
-// kernel that adds them up (0.11 us a MB to write, the rest to read).  The choice for more than 64 tokens is 1.3 % above the best
-// candidate in the mean and within 5 % of it in 550 of the 609 (the worst, 28 %, is a product of 25 us); for 17 to 64 tokens 0.8 %, within 5 %
-// in 90 of the 96.
+// The machine enters through the number of compute units alone.  For more than 64 tokens the choice is 0.4 % above the best candidate in the
+// mean, within 5 % of it in 570 of the 580 and 20 % above it at worst (72 tokens by 8,192 rows at K = 8192); fitted to two thirds of the sizes of W,
+// 0.3 to 0.8 % for the other third.  For 17 to 64 tokens 0.8 %, within 5 % in 90 of the 96.
 struct TileCost {
   int cfg, rows, tokens, bk, per_unit;
-  float full, last, per_fill, second, per_second, fixed;
+  float c0, full, last, per_fill, second, per_second, fixed, w, out, gate;
 };
 struct CostTable {
-  float c0, slab, gate;
+  float slab;       // 17 to 64 tokens: what a MB of slices costs, their sum included
   const TileCost* tiles;
   int n_tiles;
 };
 static const TileCost kCostMany[] = {
-    {4, 256, 256, 64, 1, 1.3121f, 0.8927f, 0.3633f, 0.f, 0.f, 6.6981f},
-    {5, 128, 128, 64, 2, 0.9120f, 0.4783f, 0.1449f, 0.7735f, 0.2201f, 1.7404f},
-    {6, 192, 256, 64, 1, 1.0788f, 0.7641f, 0.3037f, 0.f, 0.f, 5.1493f},
-    {7, 128, 64, 64, 2, 0.6827f, 0.3374f, 0.0978f, 0.5510f, 0.2018f, 1.0034f},
-    {8, 256, 128, 64, 1, 0.8634f, 0.6693f, 0.2196f, 0.f, 0.f, 3.9339f},
-    {9, 128, 256, 64, 1, 0.8336f, 0.5680f, 0.2405f, 0.f, 0.f, 3.6532f},
-    {10, 64, 64, 64, 2, 0.4382f, 0.2298f, 0.0403f, 0.3525f, 0.0814f, 0.5490f},
-    {11, 192, 128, 64, 2, 1.2206f, 0.6218f, 0.1553f, 1.0713f, 0.2635f, 2.6533f},
-    {13, 128, 64, 128, 1, 0.4429f, 0.3120f, 0.0987f, 0.f, 0.f, 2.0183f}};
-static const TileCost kCostFew[] = {{7, 128, 64, 64, 2, 1.2099f, 0.3352f, 0.2479f, 0.8967f, 0.3f, -0.4082f},
-                                    {10, 64, 64, 64, 2, 0.6268f, 0.191f, 0.1144f, 0.4995f, 0.1176f, -0.1f},
-                                    {13, 128, 64, 128, 1, 0.6506f, 0.3182f, 0.2568f, 0.f, 0.f, 0.2565f}};
-static const CostTable kMany = {2.674f, 0.25f, 0.f, kCostMany, 9};      // more than 64 tokens
-static const CostTable kFew = {5.522f, 0.6852f, 0.f, kCostFew, 3};            // 17 to 64 tokens
+    {4, 256, 256, 64, 1, 2.838f, 1.303f, 0.7147f, 0.5014f, 0.f, 0.f, 6.819f, 0.03584f, 0.0974f, 0.05812f},
+    {5, 128, 128, 64, 2, 3.569f, 0.8656f, 0.4617f, 0.07921f, 0.7067f, 0.1693f, 1.128f, 0.05974f, 0.1282f, 0.f},
+    {6, 192, 256, 64, 1, 2.987f, 1.037f, 0.7484f, 0.2013f, 0.f, 0.f, 3.817f, 0.04315f, 0.1525f, 0.2065f},
+    {7, 128, 64, 64, 2, 3.276f, 0.599f, 0.3345f, 0.02616f, 0.4611f, 0.1671f, 0.7892f, 0.08291f, 0.1237f, 1.662f},
+    {8, 256, 128, 64, 1, 2.261f, 0.7886f, 0.6168f, 0.1378f, 0.f, 0.f, 4.84f, 0.05987f, 0.1094f, 0.f},
+    {9, 128, 256, 64, 1, 2.529f, 0.7407f, 0.6354f, 0.0592f, 0.f, 0.f, 2.17f, 0.04335f, 0.2121f, 0.3667f},
+    {10, 64, 64, 64, 2, 2.772f, 0.3846f, 0.2352f, 0.f, 0.3132f, 0.08173f, 0.5103f, 0.06921f, 0.1375f, 1.562f},
+    {11, 192, 128, 64, 2, 4.905f, 1.237f, 0.5608f, 0.08948f, 0.9398f, 0.2723f, 0.8626f, 0.06783f, 0.1372f, 0.04604f},
+    {13, 128, 64, 128, 1, 1.95f, 0.3657f, 0.3025f, 0.05767f, 0.f, 0.f, 2.889f, 0.06945f, 0.1094f, 2.212f}};
+static const TileCost kCostFew[] = {{7, 128, 64, 64, 2, 5.522f, 1.2099f, 0.3352f, 0.2479f, 0.8967f, 0.3f, -0.4082f, 0.f, 0.f, 0.f},
+                                    {10, 64, 64, 64, 2, 5.522f, 0.6268f, 0.191f, 0.1144f, 0.4995f, 0.1176f, -0.1f, 0.f, 0.f, 0.f},
+                                    {13, 128, 64, 128, 1, 5.522f, 0.6506f, 0.3182f, 0.2568f, 0.f, 0.f, 0.2565f, 0.f, 0.f, 0.f}};
+static const CostTable kMany = {0.f, kCostMany, 9};          // more than 64 tokens
+static const CostTable kFew = {0.6852f, kCostFew, 3};        // 17 to 64 tokens
+
+// What adding up the slices of a product of more than 64 tokens costs.  A launch of its own (gemm_sum_slabs_kernel) takes 2.1 us and its bytes, 0.19 us
+// a MB it reads and 0.2 a MB it writes (2,133 pairs of times, with and without it).  A kernel that reads the terms anyway reads
+// more of them: 0.3 us and 0.165 a MB (a norm behind the product, over one term and over 2 to 8, 1,578 times).  One price for both, 0.25 us a
+// MB, cut products whose sum is a launch into slices that cost more than they gave: 700 tokens by 3,072 rows at K = 2048 20.0 -> 26.4 us.
+// (The first price is never below the second one: what is not cut for a reader is not cut for itself.)
+static double cost_of_slices(bool own_sum, int p, int m, int n) {
+  const double mb = 4e-6 * m * n;
+  return own_sum ? 2.1 + 0.19 * p * mb + 0.2 * mb : 0.3 + 0.165 * (p - 1) * mb;
+}
 
 // A product of more than 64 tokens may be two launches: as many whole rounds of a large tile as there are, and the rows behind them with
 // a tile that takes less than the round that would not be full: 2,048 tokens by 28,672 rows are 3.5 rounds of 256 x 256, or 3 and one of
 // 128 x 256 (362 -> 350 us); 3,781 tokens by 10,304 rows at K = 2048 151 -> 142; 3,000 by 22,016 gated, K = 4096, 423 -> 394.  Taken where the
 // estimate is better by 3 %: of two launches it is up to 5 % too low (8,600 tokens by 4,096 rows at K = 11,008, 2 % better by the estimate: 586 -> 605).
-static TilePlan plan_by_cost(int m, int n, int k, int epilogue) {
+// own_sum: a product cut into slices is added up by a launch of its own, and not by the kernel that reads it.
+static TilePlan plan_by_cost(int m, int n, int k, int epilogue, bool own_sum) {
   const CostTable& table = m > 64 ? kMany : kFew;
   const long long units = rb_compute_units();
   const int kt = k / 64;
@@ -387,9 +397,10 @@ static TilePlan plan_by_cost(int m, int n, int k, int epilogue) {
     double per_k = rounds * t.full;
     if (rem > 0 && rem <= units) per_k += t.last + t.per_fill * ((double)rem / units);
     if (rem > units) per_k += t.second + t.per_second * ((double)(rem - units) / units);
-    double cost = table.c0 + (double)kt / p * per_k + t.fixed * ((w + units - 1) / units);
-    if (p > 1) cost += table.slab * (4e-6 * p * m * rows);
-    if (epilogue) cost += table.gate * (1e-6 * m * rows);
+    double cost = t.c0 + (double)kt / p * per_k + t.fixed * ((w + units - 1) / units) + t.w * (2e-6 * rows * k);
+    if (epilogue) cost += t.gate * (1e-6 * m * rows);
+    else cost += t.out * (4e-6 * p * m * rows);
+    if (p > 1) cost += m > 64 ? cost_of_slices(own_sum, p, m, rows) : table.slab * (4e-6 * p * m * rows);
     return cost;
   };
   auto one = [&](int rows, int slices, double* least) {     // the best of all tiles in one launch
@@ -429,7 +440,7 @@ static TilePlan plan_by_cost(int m, int n, int k, int epilogue) {
   return best;
 }
 
-static TilePlan plan_tiles(int m, int n, int k, int epilogue) {
+static TilePlan plan_tiles(int m, int n, int k, int epilogue, bool own_sum) {
   const long long R = rb_compute_units();
   const bool dma = k % 64 == 0 && (long long)k * 512 < (1LL << 32);
   if (!dma) {
@@ -444,7 +455,7 @@ static TilePlan plan_tiles(int m, int n, int k, int epilogue) {
     const int p = (epilogue == 0 && g_tile_parts > 0 && (k / 64) % g_tile_parts == 0) ? g_tile_parts : 1;
     return {g_tile_cfg, p};
   }
-  return plan_by_cost(m, n, k, epilogue);
+  return plan_by_cost(m, n, k, epilogue, own_sum);
 }
 
 template <int EPI, typename TO, bool WF>
@@ -476,7 +487,7 @@ static int launch_tiles(int cfg, const bf16_t* x, const bf16_t* w, void* c, floa
 template <int EPI, typename TO, bool WF>
 static int launch_planned(const bf16_t* x, const bf16_t* w, void* c, float* workspace, int m, int n, int k,
                           hipStream_t s, const float* act) {
-  const TilePlan plan = plan_tiles(m, n, k, EPI);
+  const TilePlan plan = plan_tiles(m, n, k, EPI, c != nullptr);
   RB_REQUIRE(plan.cfg != 0, "rb_gemm_bf16: internal: M=%d N=%d K=%d is not a product for the tiled kernels", m, n, k);
   RB_REQUIRE(plan.parts == 1 || workspace != nullptr, "rb_gemm_bf16: M=%d N=%d K=%d needs a workspace of %lld floats",
              m, n, k, (long long)plan.parts * m * n);
@@ -492,12 +503,12 @@ static int launch_planned(const bf16_t* x, const bf16_t* w, void* c, float* work
 
 // what the planner picks for these sizes, as 10000 * (the tiles of a second launch) + 100 * cfg + parts (0: not a product for this file)
 extern "C" int rb_tune_plan(int m, int n, int k, int epilogue) {
-  const TilePlan plan = plan_tiles(m, n, k, epilogue);
+  const TilePlan plan = plan_tiles(m, n, k, epilogue, true);
   return plan.cfg == 0 ? 0 : 10000 * plan.rest + 100 * plan.cfg + plan.parts;
 }
 
-int gemm_tiled_parts(int m, int n, int k, int epilogue) {
-  const TilePlan plan = plan_tiles(m, n, k, epilogue);
+int gemm_tiled_parts(int m, int n, int k, int epilogue, bool own_sum) {
+  const TilePlan plan = plan_tiles(m, n, k, epilogue, own_sum);
   return plan.cfg == 0 ? 0 : plan.parts;
 }
 
