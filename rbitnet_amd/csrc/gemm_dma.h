@@ -110,8 +110,8 @@ template <int BN, int BM, int WN, int WM, int BK, int S, int EPI, typename TO, b
 __global__ __launch_bounds__(64 * (BN / WN) * (BM / WM)) void gemm_dma_kernel(const bf16_t* __restrict__ x,
                                                        const bf16_t* __restrict__ w, TO* __restrict__ c,
                                                        float* __restrict__ slabs, int m, int n, int k, int m_tiles,
-                                                       int n_tiles, int k_tiles, const float* __restrict__ act,
-                                                       GemmGroups groups, int n_first) {
+                                                       int n_tiles, int k_tiles, int n_first, const float* __restrict__ act,
+                                                       GemmGroups groups) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int TN = WN / 32, TM = WM / 32;
   constexpr int WAVES_N = BN / WN;

@@ -28,7 +28,7 @@ static int launch_grouped(const bf16_t* x, const bf16_t* w, TO* c, int m_tiles, 
     configured = true;
   }
   kern<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 64 * (BN / WN) * (BM / WM), lds, s>>>(x, w, c, nullptr, m_tiles * BM, n, k, m_tiles, n_tiles,
-                                                                                      k / BK, act, groups, 0);
+                                                                                      k / BK, 0, act, groups);
   return 0;
 }
 
@@ -47,7 +47,7 @@ static int launch_grouped_pingpong(const bf16_t* x, const bf16_t* w, TO* c, int 
     RB_REQUIRE(e == hipSuccess, "rb_routed_experts_tiled: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
     configured = true;
   }
-  kern<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 512, lds, s>>>(x, w, c, nullptr, m_tiles * BM, n, k, m_tiles, n_tiles, k / 64, act, groups, 0);
+  kern<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 512, lds, s>>>(x, w, c, nullptr, m_tiles * BM, n, k, m_tiles, n_tiles, k / 64, 0, act, groups);
   return 0;
 }
 

@@ -227,7 +227,7 @@ static int launch_dma_cfg(const bf16_t* x, const bf16_t* w, void* c, int m, int 
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)parts);
   RB_REQUIRE(act == nullptr || (EPI <= 1 && c != nullptr), "rb_gemm_bf16: internal: an activation or a gate's numbers go with epilogues 0 and 1 and an output");
   kern<<<grid, 64 * (BN / WN) * (BM / WM), lds, s>>>(x, w, (TO*)c, parts > 1 ? slabs : nullptr, m, n, k, m_tiles,
-                                                      n_tiles, k / BK / parts, act, GemmGroups{nullptr, nullptr, 1}, rows.first);
+                                                      n_tiles, k / BK / parts, rows.first, act, GemmGroups{nullptr, nullptr, 1});
   if (parts > 1 && c != nullptr) {      // without c the caller adds the slabs up itself
     const size_t count = (size_t)m * n;
     gemm_sum_slabs_kernel<TO><<<(unsigned)((count + 255) / 256), 256, 0, s>>>(slabs, (TO*)c, parts, count, EPI == 0 ? act : nullptr);
@@ -256,7 +256,7 @@ static int launch_pingpong_kernel(const bf16_t* x, const bf16_t* w, void* c, int
     configured = true;
   }
   kern<<<dim3((unsigned)((tiles + 7) / 8 * 8), (unsigned)parts), 512, lds, s>>>(x, w, (TO*)c, parts > 1 ? slabs : nullptr, m, n, k, m_tiles,
-                                                                                n_tiles, k / 64 / parts, act, GemmGroups{nullptr, nullptr, 1}, rows.first);
+                                                                                n_tiles, k / 64 / parts, rows.first, act, GemmGroups{nullptr, nullptr, 1});
   return 0;
 }
 
