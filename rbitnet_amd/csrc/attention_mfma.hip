@@ -455,11 +455,6 @@ extern "C" int rb_attention_prefill_bf16_chunked(const void* q, const void* k_pa
 // device-coherent stores, loads and a relaxed counter: correct, but the chain store
 // acknowledgement -> counter -> uncached loads takes as long as the second launch at 4
 // splits and much longer at 16 or more.)
-// Cross-lane moves without LDS traffic (data-parallel primitives of the vector unit).
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
 // ---------------------------------------------------------------------------------------
 // On the matrix cores, for any number of query heads per kv head up to
 // 16: scores S^T[key, head] = K q^T and outputs O^T[d, head] = V^T P^T as 16x16x32 MFMAs with
@@ -468,7 +463,9 @@ __device__ __forceinline__ float dpp_move(float v) {
 // ONE: a single query head per kv head.  All columns then hold its query, and three of them the weights' three bfloat16 parts (24
 // bits together: what float32 holds), so that the weighted sum has float32 weights; the parts' sums are added at the end.
 // A kernel on the vector units (dot products and float32 multiply-adds, a key's weight by lane reads) spent 1.2 us of a SIMD's time on a
-// page where this one spends 0.6: 16 sequences of 560 keys, 32 heads, 34.9 -> 31.0 us, of 64 to 1,024 keys 42.3 -> 33.7, 4 of 2,000 35.6 -> 29.4.
+// page where this one spends 0.6.  In turn, us: 16 sequences of 500 keys, 32 heads, 24.8 -> 23.1, of 64 to 1,024 keys 29.3 -> 25.4, 8 of 1,000
+// 26.7 -> 23.9, 16 heads of 64, 16 of 200 to 1,500 24.3 -> 16.2; contexts of one round of the waves' pages are slower: one sequence of
+// 200 keys 6.9 -> 7.5, 32 of 200, 16 heads of 64, 8.1 -> 9.6, one of 16 keys 4.1 -> 6.5.
 //
 // A wave takes a page at a time.  K rows go from memory straight into MFMA operands.  The
 // second product needs V^T (8 keys of one d per lane): the page of V is brought into the
@@ -500,6 +497,7 @@ __device__ __forceinline__ int v_swizzle(int key) {
   return D == 128 ? ((key & 7) << 1) : (((key >> 1) & 3) << 1);
 }
 
+constexpr int PAIRED_MOST = 32;       // sequences that are paired by length
 template <int D, int NW, bool FUSED, int ONCE, bool SIG, bool ONE>
 __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
     const float* __restrict__ qkv, const bf16_t* __restrict__ q_in, const float* __restrict__ cos_t,
@@ -508,8 +506,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
     int n_kv, float scale_log2, int window, int n_splits, float* __restrict__ ws, int qkv_terms, size_t qkv_stride,
     const float* __restrict__ sinks, int keep_first, float cap, float cap_pre, int kv_rep, int chunk,
     const float* __restrict__ sig_bias, int by_length) {
-  // by_length: the sequences are taken by rank, the longest first and then the shortest (at most 32 of them).  Workgroups that far
-  // apart share a compute unit where there are two for each, and the busiest one then has no two long sequences.
+  // by_length: the sequences are taken by rank, the longest first and then the shortest (at most PAIRED_MOST of them).  Workgroups that far
+  // apart share a compute unit where there are two for each, and the busiest one then has no two long sequences.  Where every
+  // sequence is done in one round of the waves' pages there is nothing to pair.
   // chunk > 0: the query sees the keys of its own chunk of positions only.  SIG: a visible key's weight is
   // sigmoid(score + sig_bias[head]); the waves' and the splits' outputs are then simply added.
   // kv_rep > 1: n_kv counts every key/value head kv_rep times (head kvh reads the pages of head kvh / kv_rep), so that more
@@ -538,19 +537,20 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
   const int c16 = lane & 15, grp = lane >> 4;
   const int split = blockIdx.x, kvh = blockIdx.y;
   const int G = ONE ? 1 : n_heads / n_kv;
-  int b = blockIdx.z;
-  int pos;
+  int b = blockIdx.z, pos;
   if (by_length) {
     const int n = gridDim.z, half = (n + 1) / 2;
     const int want = b < half ? b : n - 1 - (b - half);
-    const int mine = lane < n ? tok_pos[lane] : -1;
-    int rank = 0;                                        // how many sequences are longer (of equal ones, those before)
-#pragma unroll 8
-    for (int i = 0; i < n; ++i) {
-      const int other = __builtin_amdgcn_readlane(mine, i);
-      rank += other + (i < lane ? 1 : 0) > mine ? 1 : 0;
+    const int mine = lane < n ? tok_pos[lane] : -1;      // a lane behind the last sequence is longer than none
+    if (__ballot(mine >= NW * RB_PAGE * n_splits)) {
+      int rank = 0;                                      // how many sequences are longer (of equal ones, those before)
+#pragma unroll
+      for (int i = 0; i < PAIRED_MOST; ++i) {
+        const int other = __builtin_amdgcn_readlane(mine, i);
+        rank += other + (i < lane ? 1 : 0) > mine ? 1 : 0;
+      }
+      b = __builtin_ctzll(__ballot(lane < n && rank == want));
     }
-    b = __builtin_ctzll(__ballot(lane < n && rank == want));
     pos = __builtin_amdgcn_readlane(mine, b);
   } else {
     pos = tok_pos[b];
@@ -608,8 +608,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
     const float* src = qkv + (size_t)b * row_width;
     const float* cr = cos_t ? cos_t + (size_t)pos * HALF : nullptr;
     const float* sr = cos_t ? sin_t + (size_t)pos * HALF : nullptr;
-    for (int idx = tid; idx < 17 * HALF; idx += NT) {
-      const int gg = idx / HALF, i = idx - gg * HALF;
+    // (ONE reads the first row and the new key only: with rows of zeros between them the key's loads waited for a trip of their own)
+    for (int idx = tid; idx < (ONE ? 2 : 17) * HALF; idx += NT) {
+      const int row = idx / HALF, i = idx - row * HALF, gg = ONE && row == 1 ? 16 : row;
       const int i0 = style == 0 ? 2 * i : i, i1 = style == 0 ? 2 * i + 1 : i + HALF;
       uint16_t* dst = gg < 16 ? q_h + gg * D : knew_h;
       if (gg < 16 && gg >= G) {
@@ -813,20 +814,11 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
     page_cur = page_nx;
   }
 
-  if constexpr (ONE) {                     // the parts' sums into column 0 (an infinite value times a part that is zero is no number)
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float first = acc_o[dt][i], rest = dpp_move<0x101>(first) + dpp_move<0x102>(first);      // row_shl: of lanes c16 + 1, c16 + 2
-        acc_o[dt][i] = isfinite(first) ? first + rest : first;
-      }
-  }
   // ---- the waves' states into one (the pages' area is reused for the outputs): a thread four numbers of a head, so that the
   // waves' factors are computed once for them
   constexpr int LD = D + 4;                // the rows of a store hit different banks
   __syncthreads();
-  if (c16 < G) {
+  if (c16 < (ONE ? 3 : G)) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
       *reinterpret_cast<f32x4_t*>(red_acc + ((size_t)wave * 16 + c16) * LD + 16 * dt + 4 * grp) = acc_o[dt];
@@ -844,7 +836,13 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const float f = exp2f(red_m[w * 16 + gg] - m_safe);
-      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(red_acc + ((size_t)w * 16 + gg) * LD + d);
+      const float* of = red_acc + ((size_t)w * 16 + gg) * LD + d;
+      f32x4_t v = *reinterpret_cast<const f32x4_t*>(of);
+      if constexpr (ONE) {                 // the parts' sums (an infinite value times a part that is zero is no number)
+        const f32x4_t second = *reinterpret_cast<const f32x4_t*>(of + LD), third = *reinterpret_cast<const f32x4_t*>(of + 2 * LD);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = isfinite(v[e]) ? v[e] + (second[e] + third[e]) : v[e];
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) a[e] += SIG ? v[e] : v[e] * f;
       const float* lw = red_l + w * 64 + gg;
@@ -962,10 +960,11 @@ static int launch_decode_mfma_nw(const DecodeArgs& a, hipStream_t s) {
     configured = true;
   }
   dim3 grid(a.n_splits, a.n_kv, a.n_seqs);
-  // two workgroups a compute unit: those of long sequences beside those of short ones (finding a sequence's rank takes 0.7 us with 16
-  // sequences and 2.7 with 64, so up to 32 only)
+  // Two workgroups a compute unit: those of long sequences beside those of short ones, up to 32 sequences.  32 heads of their own, in turn without and with:
+  // 16 sequences of 64 to 1,024 keys 28.8 and 25.5 us, of 200 to 1,500 42.9 and 39.3, 12 of 64 to 1,024 24.2 and 23.8; where all are equally
+  // long the ranks cost 0.3 to 0.6 us (16 of 1,000 keys 42.6 and 43.3).
   const long long wgs = (long long)a.n_splits * a.n_kv * a.n_seqs;
-  const int by_length = a.n_seqs > 1 && a.n_seqs <= 32 && wgs > rb_compute_units() && wgs <= 2 * rb_compute_units() ? 1 : 0;
+  const int by_length = a.n_seqs > 1 && a.n_seqs <= PAIRED_MOST && wgs > rb_compute_units() && wgs <= 2 * rb_compute_units() ? 1 : 0;
   kern<<<grid, 64 * NW, lds, s>>>(a.qkv, a.q, a.cos_t, a.sin_t, a.style, a.k, a.v, a.out, a.tok_pos, a.bt,
                                   a.bt_stride, a.n_heads, a.n_kv, a.sl2, a.window, a.n_splits, a.ws, a.qkv_terms,
                                   a.qkv_stride, a.sinks, a.keep_first, a.cap, a.cap_pre, a.kv_rep, a.chunk, a.sig_bias, by_length);

@@ -1051,6 +1051,36 @@ def test_single_token_attention_of_heads_of_their_own(lib, dim, kv, lengths, win
     _within(out.view(want.shape), want, 2.0 ** -8 * want.abs() + 2.0 ** -14 * float(max(x.abs().max() for x in vs)))
 
 
+@pytest.mark.parametrize("length", [60, 200])
+def test_float32_weights_cost_a_short_context_little(lib, length):
+    """A step whose heads have a key head each, short contexts: beside the same heads with weights of 8 bits.  (Rows of zeros that
+    nothing read, a second trip to memory behind them and lane moves made it 1.2 to 1.25 of that.)"""
+    heads, dim = 32, 128
+    pages = (length + 63) // 64
+    kp = torch.randn(pages, heads, 64, dim, device=DEV).bfloat16()
+    vp = torch.randn_like(kp)
+    table = torch.arange(pages, dtype=torch.int32, device=DEV)[None]
+    pos = torch.tensor([length - 1], dtype=torch.int32, device=DEV)
+    qkv = torch.randn(1, 3 * heads * dim, device=DEV)
+    cos, sin = torch.ones(256, dim // 2, device=DEV), torch.zeros(256, dim // 2, device=DEV)
+    out, ws = torch.empty(1, heads * dim, dtype=torch.bfloat16, device=DEV), torch.empty(heads * (dim + 2), device=DEV)
+    run = lambda: lib.attention_decode_fused_bf16(qkv, cos, sin, 1, kp, vp, out, pos, table, heads, heads, dim, 0.1, 0, 1, ws)
+    times = []
+    try:
+        for mode in (0, 1):
+            lib._lib.rb_tune_decode_mfma(mode)
+            graph = torch.cuda.CUDAGraph()
+            run()
+            torch.cuda.synchronize()
+            with torch.cuda.graph(graph):
+                for _ in range(20):
+                    run()
+            times.append(_least_time(graph.replay, calls=3))
+    finally:
+        lib._lib.rb_tune_decode_mfma(0)
+    assert times[0] <= 1.1 * times[1], times
+
+
 def test_single_token_attention_of_an_infinite_value(lib):
     """An infinity among the visible values comes out in its own place, whatever the weights' parts are, and nowhere else."""
     kv, dim, n = 2, 128, 200
