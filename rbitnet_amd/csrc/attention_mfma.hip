@@ -1018,6 +1018,10 @@ static int dispatch_decode(DecodeArgs a, int head_dim, hipStream_t s, const char
   const int group = a.n_heads / a.n_kv;
   RB_REQUIRE(group <= 16, "%s: %d query heads per kv head not supported (at most 16; use rb_attention_generic)", who,
              group);
+  RB_REQUIRE(g_decode_waves == 0 || g_decode_waves == 2 || g_decode_waves == 4, "%s: workgroups of %d waves are not built (2 or 4)", who,
+             g_decode_waves);
+  RB_REQUIRE(g_decode_mfma == 0 || g_decode_mfma == 1, "%s: kernel choice %d is neither by group size (0) nor weights of 8 bits (1)", who,
+             g_decode_mfma);
   // one head: float32 weights, as long as nothing else is asked (kept first keys, capped scores, repeated kv heads, chunks, sigmoid weights)
   const bool opts = a.keep_first > 0 || a.cap > 0.f || a.kv_rep > 1 || a.chunk > 0 || a.sig_bias != nullptr;
   a.one = group == 1 && !opts && g_decode_mfma == 0;

@@ -1081,6 +1081,23 @@ def test_float32_weights_cost_a_short_context_little(lib, length):
     assert times[0] <= 1.1 * times[1], times
 
 
+@pytest.mark.parametrize("hook,value", [("rb_tune_decode_waves", 8), ("rb_tune_decode_waves", 3), ("rb_tune_decode_mfma", 2)])
+def test_forced_choices_of_single_token_attention_that_are_not_built_are_refused(lib, hook, value):
+    from rbitnet_amd.errors import KernelError
+    kp = torch.zeros(1, 2, 64, 64, dtype=torch.bfloat16, device=DEV)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    call = lambda: lib.attention_decode_bf16(torch.zeros(1, 4, 64, dtype=torch.bfloat16, device=DEV), kp, torch.zeros_like(kp),
+                                             torch.empty(1, 256, dtype=torch.bfloat16, device=DEV), i32(5), i32(0)[None], 4, 2, 64, 0.1, 0, 1,
+                                             torch.empty(4 * 66, device=DEV))
+    try:
+        getattr(lib._lib, hook)(value)
+        with pytest.raises(KernelError):
+            call()
+    finally:
+        getattr(lib._lib, hook)(0)
+    call()
+
+
 def test_single_token_attention_of_an_infinite_value(lib):
     """An infinity among the visible values comes out in its own place, whatever the weights' parts are, and nowhere else."""
     kv, dim, n = 2, 128, 200
