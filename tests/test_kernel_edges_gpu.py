@@ -60,7 +60,7 @@ def test_float32_tiles(lib, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(130, 208, 64), (257, 400, 128), (70, 272, 192), (300, 1000, 320), (259, 521, 448)])
 def test_turn_taking_tiles(lib, tile, m, n, k):
     """One K tile, two, odd numbers of them; row and token counts that end inside a tile, a wave's share and a piece of 16; rows that
-    begin at whole vectors and not; float32 and bfloat16 outputs, an activation on the way out, gated pairs, W as rows and
+    begin at whole vectors and not; float32 and bfloat16 outputs, an activation on the way out, W as rows and
     fragment-major (N a multiple of 16 only)."""
     g = torch.Generator().manual_seed(1000 * tile + m + n + k)
     a, w = torch.randn(m, k, generator=g).bfloat16(), (torch.randn(n, k, generator=g) * k ** -0.5).bfloat16()
@@ -91,14 +91,47 @@ def test_turn_taking_tiles(lib, tile, m, n, k):
                     got.append(c.cpu())
         for other in got[8:]:                              # either layout: the same bits
             assert any(torch.equal(other, first) for first in got[:8])
-        if n % 32 == 0:
-            gate, up = (want.view(m, n // 32, 2, 16)[:, :, i].reshape(m, n // 2) for i in (0, 1))
-            exact = gate * torch.sigmoid(gate) * up
-            for dtype in (torch.float32, torch.bfloat16):
-                c = torch.full((m, n // 2), float("nan"), device=DEV, dtype=dtype)
-                lib.gemm_bf16(ad, wd, c, 1)
-                bound = (1e-4 if dtype == torch.float32 else half) * (1 + exact.abs()) + 1e-4
-                assert ((c.double().cpu() - exact).abs() <= bound).all(), dtype
+    finally:
+        lib._lib.rb_tune_tiles(0, 0)
+
+
+@pytest.mark.parametrize("tile", [4, 5, 6, 7, 8, 9, 10, 11, 13])
+@pytest.mark.parametrize("m,n,k", [(70, 224, 128), (130, 416, 64), (259, 992, 320), (300, 1376, 384)])
+@pytest.mark.parametrize("limits", [None, (1.5, 1.702)])
+def test_gated_tiles(lib, tile, m, n, k, limits):
+    """Gated pairs for row counts that are multiples of 32 and fill no tile (with three pieces a half a pair's rows lie in two halves),
+    W as rows and fragment-major, outputs that begin at whole vectors and not, the plain gate and the one with limits."""
+    if tile == 13 and k % 128:
+        pytest.skip("K tiles of 128")
+    g = torch.Generator().manual_seed(100 * tile + m)
+    a, w = torch.randn(m, k, generator=g).bfloat16(), (torch.randn(n, k, generator=g) * 2 * k ** -0.5).bfloat16()
+    sums, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    gate, up = (sums.view(m, n // 32, 2, 16)[:, :, i].reshape(m, n // 2) for i in (0, 1))
+    off = 2.0 ** -24 * k * size.view(m, n // 32, 2, 16).amax(2).reshape(m, n // 2)      # the sums' rounding, either of a pair
+    act = None
+    if limits is None:
+        exact = gate * torch.sigmoid(gate) * up
+        slack = 1.1 * off * up.abs() + off * gate.abs() + 1.1 * off * off               # |silu'| <= 1.1, |silu(x)| <= |x|
+    else:
+        act = torch.tensor(limits, device=DEV)
+        lim, alpha = (float(x) for x in act.cpu())
+        cut, moved = gate.clamp(max=lim), up.clamp(-lim, lim) + 1
+        exact = cut * torch.sigmoid(alpha * cut) * moved
+        slack = 1.1 * off * moved.abs() + off * cut.abs() + 1.1 * off * off             # g sigmoid(alpha g) has the same slopes
+    slack = slack + 2.0 ** -20 * exact.abs()               # the hardware's exponential and reciprocal, 1 ulp each
+    ad, wd = a.to(DEV), w.to(DEV)
+    wf = torch.empty_like(wd)
+    lib.place_rows(wd, wf, frag=True)
+    try:
+        lib._lib.rb_tune_tiles(tile, 1)
+        for weights, frag in ((wd, False), (wf, True)):
+            for offset in (0, 1):
+                for dtype in (torch.float32, torch.bfloat16):
+                    room = torch.full((m * n // 2 + 1,), float("nan"), device=DEV, dtype=dtype)
+                    c = room[offset:offset + m * n // 2].view(m, n // 2)
+                    lib.gemm_bf16(ad, weights, c, 1, w_frag=frag, act=act)
+                    bound = slack if dtype == torch.float32 else slack + 2.0 ** -8 * (exact.abs() + slack)
+                    _within(c, exact, bound)
     finally:
         lib._lib.rb_tune_tiles(0, 0)
 
@@ -185,9 +218,9 @@ def test_planner_of_products_that_add_up_their_slices(lib, m, n, k):
 
 
 @pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
-@pytest.mark.parametrize("m,n,k", [(70, 160, 32), (131, 200, 64), (300, 333, 96)])
+@pytest.mark.parametrize("m,n,k", [(70, 160, 32), (131, 200, 64), (300, 333, 96), (131, 208, 128), (300, 400, 640)])
 def test_float32_tiles_forced(lib, tile, m, n, k):
-    """Every float32 tile: one, two and three K tiles, ends inside a tile, both layouts."""
+    """Every float32 tile: one, two, three, four and twenty K tiles, ends inside a tile, both layouts where K is a multiple of 128."""
     g = torch.Generator().manual_seed(100 * tile + m)
     a, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
     want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T

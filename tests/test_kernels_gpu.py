@@ -373,8 +373,8 @@ def test_attention_prefill_of_a_long_prompt(lib, waves, n_heads, n_kv, d, t, win
 
 @pytest.fixture
 def decode_kernel(lib, request):
-    """"auto": the kernel the library picks for the group size; "matrix": the matrix-core
-    decode kernel whatever the group size."""
+    """"auto": float32 weights for groups of one query head, weights of 8 bits for larger ones; "matrix": weights of 8 bits
+    whatever the group size."""
     lib._lib.rb_tune_decode_mfma(1 if request.param == "matrix" else 0)
     yield request.param
     lib._lib.rb_tune_decode_mfma(0)
@@ -425,7 +425,7 @@ def test_far_key_stands_out(lib):
                               bt.to(DEV), n_heads, n_kv, d, scale, 0)
         outs.append(out.clone())
         ws = torch.empty(n_heads * 4 * (d + 2), device=DEV)
-        for mode in (0, 1):             # the vector kernel, the matrix-core kernel
+        for mode in (0, 1):             # weights by group size, weights of 8 bits
             lib._lib.rb_tune_decode_mfma(mode)
             try:
                 lib.attention_decode_bf16(q.to(dtype).to(DEV), kp.to(DEV), vp.to(DEV), out, tok_pos.to(DEV),
@@ -739,7 +739,7 @@ def test_products_planned_for_another_number_of_compute_units(lib, units):
         lib._lib.rb_tune_compute_units(0)
 
 
-@pytest.mark.parametrize("cfg", [4, 5, 6, 7, 8, 9, 10, 13])
+@pytest.mark.parametrize("cfg", [4, 5, 6, 7, 8, 9, 10, 11, 13])
 def test_every_tile_of_the_direct_to_lds_product_at_sizes_that_fill_none(lib, cfg):
     """The planner picks a tile by the product's sizes, so sizes of a test reach only some of the
     tiles: here each is forced in turn (the hook that measurements use), with 1, 2 and 4 K slices,
@@ -799,7 +799,7 @@ def test_attention_long_context(lib):
     for n_splits, mode in ((1, 0), (3, 0), (16, 0), (1, 1), (5, 1), (16, 1)):
         out = torch.full((2, n_heads * d), float("nan"), dtype=dtype, device=DEV)
         ws = torch.empty(2 * n_heads * n_splits * (d + 2), device=DEV)
-        lib._lib.rb_tune_decode_mfma(mode)             # 1: the matrix-core kernel
+        lib._lib.rb_tune_decode_mfma(mode)             # 1: weights of 8 bits whatever the group size
         try:
             lib.attention_decode_bf16(q.to(DEV), kp, vp, out, tok_pos.to(DEV), bt.to(DEV), n_heads, n_kv, d, scale,
                                       0, n_splits, ws)
