@@ -324,7 +324,7 @@ struct TilePlan {
 };
 
 static int g_tile_cfg = 0, g_tile_parts = 0;
-extern "C" void rb_tune_tiles(int cfg, int parts) {       // experiments only; 0 = built-in choice
+extern "C" void rb_tune_tiles(int cfg, int parts) {       // experiments only; 0 = built-in choice; + 100 * (tiles of a second launch)
   g_tile_cfg = cfg;
   g_tile_parts = parts;
 }
@@ -382,6 +382,13 @@ static double cost_of_slices(bool own_sum, int p, int m, int n) {
   return own_sum ? 2.1 + 0.19 * p * mb + 0.2 * mb : 0.3 + 0.165 * (p - 1) * mb;
 }
 
+// How many of W's rows the whole rounds of a tile take (0: there are none, or nothing is left).
+static int whole_rounds(const TileCost& t, int m, int n) {
+  const long long m_tiles = (m + t.tokens - 1) / t.tokens, slots = (long long)rb_compute_units() * t.per_unit;
+  const int split = (int)(m_tiles * (n / t.rows) / slots * slots / m_tiles) * t.rows;
+  return split < n ? split : 0;
+}
+
 // A product of more than 64 tokens may be two launches: as many whole rounds of a large tile as there are, and the rows behind them with
 // a tile that takes less than the round that would not be full: 2,048 tokens by 28,672 rows are 3.5 rounds of 256 x 256, or 3 and one of
 // 128 x 256 (362 -> 350 us); 3,781 tokens by 10,304 rows at K = 2048 151 -> 142; 3,000 by 22,016 gated, K = 4096, 423 -> 394.  Taken where the
@@ -426,9 +433,8 @@ static TilePlan plan_by_cost(int m, int n, int k, int epilogue, bool own_sum) {
   for (int i = 0; i < table.n_tiles; ++i) {
     const TileCost& t = table.tiles[i];
     if (t.rows * t.tokens < 192 * 256 || k % t.bk != 0) continue;
-    const long long m_tiles = (m + t.tokens - 1) / t.tokens, slots = units * t.per_unit;
-    const int split = (int)(m_tiles * (n / t.rows) / slots * slots / m_tiles) * t.rows;
-    if (split == 0 || split >= n) continue;
+    const int split = whole_rounds(t, m, n);
+    if (split == 0) continue;
     double behind = 0.0;
     const TilePlan rest = one(n - split, 1, &behind);
     const double cost = cost_of(t, split, 1) + behind;
@@ -452,8 +458,15 @@ static TilePlan plan_tiles(int m, int n, int k, int epilogue, bool own_sum) {
   }
   if (m <= 16) return {0, 1};
   if (g_tile_cfg >= 4) {
+    const int cfg = g_tile_cfg % 100, rest = g_tile_cfg / 100;
+    if (rest > 0) {
+      for (const TileCost& t : kCostMany)
+        if (t.cfg == cfg && m > 64)
+          if (const int split = whole_rounds(t, m, n)) return {cfg, 1, rest, split};
+      return {cfg, 1};
+    }
     const int p = (epilogue == 0 && g_tile_parts > 0 && (k / 64) % g_tile_parts == 0) ? g_tile_parts : 1;
-    return {g_tile_cfg, p};
+    return {cfg, p};
   }
   return plan_by_cost(m, n, k, epilogue, own_sum);
 }

@@ -16,7 +16,7 @@ void rb_tune_f32_few(int on);                                   // float32 produ
 void rb_tune_f32_tile(int tile);                                // float32 product of many tokens: 1..7 = that tile, -1 = tiles staged through registers
 int rb_tune_f32_plan(int m, int n, int k);                      // float32 product of many tokens: the built-in choice, 10 * (tile of a second launch) + tile
 void rb_tune_use_stream(int on);                                // 0: the skinny product up to 64 tokens
-void rb_tune_tiles(int cfg, int parts);                         // tiled product: tile configuration and K slices
+void rb_tune_tiles(int cfg, int parts);                         // tiled product: tile configuration (+ 100 * that of a second launch) and K slices
 int rb_tune_plan(int m, int n, int k, int epilogue);            // tiled product: the built-in choice, 10000 * (tiles of a second launch) + 100 * cfg + parts
 void rb_tune_attention_vec(int on);                             // generic attention: 0 = the scalar kernel also for head sizes that are multiples of 4, 2 = the vector units for float32 too
 void rb_tune_prefill_waves(int waves);                          // prefill attention: 4 or 8

@@ -16,6 +16,7 @@ import sys
 from typing import Dict, List, Sequence, Tuple
 
 TILE_CFGS = (4, 5, 6, 7, 8, 9, 10, 11, 13)
+TWO_LAUNCH_CFGS = (4, 6)                # the tiles whose whole rounds may be a launch, the rows behind them another
 SMALL_TILE_CFGS = (7, 10, 13)           # the tiles for at most 64 tokens
 
 
@@ -81,7 +82,7 @@ def sweep(models: Sequence[Tuple[str, Dict]], token_counts: Sequence[int], out=s
     print("|---|---|---|---|---|---|---|---|---|", file=out)
     for label, cfg in models:
         for name, n, k, epi in products(cfg):
-            copies = max(2, min(8, (1 << 30) // (n * k * 2)))
+            copies = max(2, min(32, (5 << 27) // (n * k * 2) + 1))      # more than the caches hold
             ws = [(torch.randn(n, k, device=dev) * 0.02).to(torch.bfloat16) for _ in range(copies)]
             for m in token_counts:
                 a = (torch.randn(m, k, device=dev)).to(torch.bfloat16)
@@ -101,6 +102,12 @@ def sweep(models: Sequence[Tuple[str, Dict]], token_counts: Sequence[int], out=s
                                 continue
                             names.append(f"tile {cfg_id} x {parts}")
                             setups.append(tile(cfg_id, parts))
+                    for first in TWO_LAUNCH_CFGS if m > 64 else ():
+                        for rest in TILE_CFGS:
+                            L.rb_tune_tiles(first + 100 * rest, 1)
+                            if int(L.rb_tune_plan(m, n, k, epi)) >= 10000 and not (rest == 13 and k % 128):
+                                names.append(f"tile {first}, rest {rest}")
+                                setups.append(tile(first + 100 * rest, 1))
                     if m <= 64:
                         names.append("few-token kernels")
                         setups.append(lambda: (reset(), L.rb_tune_use_stream(0)))
