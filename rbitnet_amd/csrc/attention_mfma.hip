@@ -521,7 +521,6 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
   constexpr int CPR = D / 8;          // 16-byte chunks per row of V
   constexpr int RPI = 64 / CPR;       // rows one direct load instruction covers
   constexpr int VI = RB_PAGE / RPI;   // direct load instructions per page
-  constexpr int DL = D / 64;          // elements of a row per lane
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int NT = 64 * NW;
   uint16_t* vpages = reinterpret_cast<uint16_t*>(smem);                    // [NW waves][64 keys][D]
@@ -530,7 +529,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
   uint16_t* vnew_h = knew_h + D;
   float* red_m = reinterpret_cast<float*>(vnew_h + D);                     // [NW][16]
   float* red_l = red_m + NW * 16;                                          // [NW][64]
-  float* red_acc = reinterpret_cast<float*>(smem);                         // [NW][16][D], over the pages at the end
+  float* red_acc = reinterpret_cast<float*>(smem);                         // [NW][16][D + 4], over the pages at the end
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);      // the same for the whole wave: LDS addresses go to a scalar register
@@ -976,7 +975,9 @@ static int launch_decode_mfma_nw(const DecodeArgs& a, hipStream_t s) {
 // where there are more workgroups than that: four of them share a compute unit then, and a short context leaves no wave without a
 // page (us: 8 kv heads, 128 sequences of 300 keys 35.0 -> 31.3; a kv head per query head, 32 of them: 24 sequences of 300 keys 34.2 -> 25.5,
 // 64 of 100 42.4 -> 32.9, 64 of 600 112.6 -> 113.9).  8 waves for steps that leave compute units empty, which dealt 8 pages at a time, lost
-// to 4 (8 sequences of 450 to 900 keys on 8 kv heads: the whole step 0.7 to 1.3 %).
+// to 4 (8 sequences of 450 to 900 keys on 8 kv heads: the whole step 0.7 to 1.3 %; with a sink or a window and one workgroup for all pages, 1 to 16
+// sequences on 8 kv heads of 128, 200 keys 8.7 to 9.3 -> 7.5 to 8.2 us, 500 keys 10.3 to 11.8 -> 9.2 to 10.2; 32 sequences of 1,000 keys on 8 heads of 64
+// 13.7 -> 14.4, of 500 8.8 -> 8.2).
 static int g_decode_waves = 0;
 extern "C" void rb_tune_decode_waves(int nw) { g_decode_waves = nw; }      // experiments only; 0 = built-in
 template <int D, bool FUSED>

@@ -6,8 +6,9 @@
 
 Nothing of a step goes through the host: the router's product, one launch that chooses and sorts the (token, expert)
 pairs by expert in runs padded to tiles of 16 rows, one launch pair for all experts' products (on the matrix cores in
-bfloat16), and, with more than one expert a token, the sum of a token's pairs in a fixed order.  A token's result does
-not depend on what else the step holds.
+bfloat16), and, with more than one expert a token, the sum of a token's pairs in a fixed order.  Steps of many tokens run on the
+dense product's tiles (runs padded to 64 to 256 rows), which multiply the sums of the way up by s_e instead of rounding s_e * h.  A token's
+result does not depend on what else the step holds but for which of these kernels its number of tokens asks for.
 
 Experts' tensors are `e<i>.gate`, `e<i>.up` [ff, E] and `e<i>.down` [E, ff]; they are stacked at load time.
 Parameters: experts, top, intermediate_size, limit, alpha (1.702), names ({"router", "expert", "gate", "up", "down"}).
@@ -44,13 +45,16 @@ DEFAULT_NAMES = {"router": "router", "expert": "e{i}", "gate": "gate", "up": "up
 MAX_EXPERTS = 1024
 MAX_CHOSEN = 64            # of the softmax over the chosen logits
 TILED_FROM = 65            # tokens of a step from which experts without gates run on the dense product's tiles
-GATED_TILED_FROM = 112     # rows of an expert's run, in the mean, from which gated ones do
+GATED_TILED_FROM = 112     # rows of an expert's run, in the mean, from which gated ones do, whichever side their weights are on
 
 
 def tile_rows(n_pairs: int, n_experts: int) -> int:
     """How many rows every expert's run is padded to where it runs on the dense product's tiles: large tiles where the runs fill
-    them.  Gated experts of 2,048 units, width 2,048, 16 of them (us for runs padded to 64, 128, 256): 32 rows an expert 109, 116,
-    141; 64 rows 127, 117, 143; 375 rows 295, 210, 243; 512 rows 381, 266, 257; 945 rows 618, 460, 397."""
+    them.  Experts of 2,048 units, width 2,048, 16 of them, us for runs padded to 64, 128, 256.  Gated: 32 rows an expert 131, 121,
+    150; 88 rows 144, 134, 153; 350 rows 301, 220, 254; 500 rows 381, 278, 269; 946 rows 663, 482, 415; with weights on the inputs
+    32 rows 140, 123, 150; 88 rows 163, 135, 153.  Without a gate: 32 rows 94, 85, 108; 88 rows 111, 96, 111; 350 rows 210, 162, 214;
+    700 rows 349, 292, 237.  Where a run just passes a multiple of 128 the next tile is better: 150 rows 176, 180, 166, without a gate
+    132, 152, 121."""
     each = n_pairs / n_experts
     return 256 if each >= 512 else 128 if each >= 64 else 64
 
