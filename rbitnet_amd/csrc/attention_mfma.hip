@@ -464,8 +464,9 @@ extern "C" int rb_attention_prefill_bf16_chunked(const void* q, const void* k_pa
 // bits together: what float32 holds), so that the weighted sum has float32 weights; the parts' sums are added at the end.
 // A kernel on the vector units (dot products and float32 multiply-adds, a key's weight by lane reads) spent 1.2 us of a SIMD's time on a
 // page where this one spends 0.6.  In turn, us: 16 sequences of 500 keys, 32 heads, 24.8 -> 23.1, of 64 to 1,024 keys 29.3 -> 25.4, 8 of 1,000
-// 26.7 -> 23.9, 16 heads of 64, 16 of 200 to 1,500 24.3 -> 16.2; contexts of one round of the waves' pages are slower: one sequence of
-// 200 keys 6.9 -> 7.5, 32 of 200, 16 heads of 64, 8.1 -> 9.6, one of 16 keys 4.1 -> 6.5.
+// 26.7 -> 23.9, 16 heads of 64, 16 of 200 to 1,500 24.3 -> 16.2; contexts of one round of the waves' pages are slower, one sequence of
+// 200 keys 6.9 -> 7.5, 32 of 200, 16 heads of 64, 8.1 -> 9.6, one of 16 keys 4.1 -> 6.5, and 40 to 48 sequences of 130 to 300 keys, 32 heads,
+// which are 1.25 to 1.5 rounds of workgroups (48 of 200 35.0 -> 41.3; 64 of 200 44.3 -> 48.3, of 500 101.6 -> 84.8).
 //
 // A wave takes a page at a time.  K rows go from memory straight into MFMA operands.  The
 // second product needs V^T (8 keys of one d per lane): the page of V is brought into the
