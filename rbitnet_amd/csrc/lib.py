@@ -162,6 +162,7 @@ class Kernels:
             "rb_streams_update_layernorm": [_P, _I, _L, _P, _P, _P, _P, _P, _P, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_streams_update": [_P, _I, _L, _P, _P, _P, _P, _I, _I, _P],
             "rb_embed_streams_waves": [_P, _I, _P, _F, _P, _P, _P, _I, _L, _I, _I, _P],
+            "rb_embed_streams_layout": [_P, _I, _I, _P, _F, _P, _P, _P, _I, _L, _I, _I, _P],
             "rb_streams_rmsnorm": [_P, _I, _L, _P, _P, _P, _I, _L, _L, _P, _P, _I, _L, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_short_conv_biases": [_P, _L, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
             "rb_selective_scan": [_P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
@@ -594,20 +595,22 @@ class Kernels:
                                              self._stream()))
 
     def embed_streams_waves(self, table: torch.Tensor, ids: torch.Tensor, scale: float, inv: Optional[torch.Tensor],
-                            tok_pos: torch.Tensor, x: torch.Tensor) -> None:
+                            tok_pos: Optional[torch.Tensor], x: torch.Tensor, frag: bool = False) -> None:
         """`embed_streams` with table[ids[t]] * scale + wave(tok_pos[t]): numbers 2i and 2i + 1 of wave(p) are the sine and the
-        cosine of p inv[i] (inv float64 [(E + 1) // 2]; None: no wave)."""
+        cosine of p inv[i] (inv float64 [(E + 1) // 2]; None: no wave).  frag: the table is stored fragment-major (as `pack_rows`
+        stores a matrix)."""
         s_, n, width = x.shape
         _check(table, "table")
         _check(ids, "ids", torch.int32, (n,))
-        _check(tok_pos, "tok_pos", torch.int32, (n,))
+        if tok_pos is not None:
+            _check(tok_pos, "tok_pos", torch.int32, (n,))
         _check(x, "x", torch.float32)
         if table.shape[1] != width:
             raise KernelError("embedding width mismatch")
         if inv is not None:
             _check(inv, "inv", torch.float64, ((width + 1) // 2,))
-        self._ok(self._lib.rb_embed_streams_waves(_ptr(table), dtype_code(table.dtype), _ptr(ids), float(scale), _ptr(inv),
-                                                  _ptr(tok_pos), _ptr(x), s_, n * width, n, width, self._stream()))
+        self._ok(self._lib.rb_embed_streams_layout(_ptr(table), dtype_code(table.dtype), 1 if frag else 0, _ptr(ids), float(scale),
+                                                   _ptr(inv), _ptr(tok_pos), _ptr(x), s_, n * width, n, width, self._stream()))
 
     def streams_rmsnorm(self, x: torch.Tensor, coef: Optional[torch.Tensor], weight: torch.Tensor, eps: float,
                         rows: Optional[torch.Tensor], out: torch.Tensor, update=None) -> None:

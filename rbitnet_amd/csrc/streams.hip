@@ -357,13 +357,18 @@ extern "C" int rb_embed_streams(const void* table, int table_dtype, const int32_
 // The same with what a model may do to an embedding's row: x[s][t, :] = table[ids[t], :] * scale + wave(pos[t]), where number 2i of
 // wave(p) is sin(p inv[i]) and number 2i + 1 is cos(p inv[i]) (inv float64 [(width + 1) / 2]; null: no wave).  The angle is
 // made and brought into one turn in float64, so that a late position's sine is as good as an early one's.
-template <typename T>
+// FRAG: the table is stored fragment-major, as the output matrix that it is tied to wants it (gemm_internal.h; W for a product of 4 tokens
+// by 128,256 rows at K = 2048: 141 us as rows, 80 fragment-major).  A row is then width / E pieces of 16 bytes (E values) that lie 256
+// bytes apart, so a gather of T rows touches four times its bytes: 3,781 rows of 2,048 take as long as the stream they write.
+template <typename T, bool FRAG>
 __global__ void embed_streams_waves_kernel(const T* __restrict__ table, const int32_t* __restrict__ ids, float scale,
                                            const double* __restrict__ inv, const int32_t* __restrict__ tok_pos, float* __restrict__ x,
                                            int n_streams, size_t stream_stride, int width) {
   const int t = blockIdx.x;
-  const T* row = table + (size_t)ids[t] * width;
-  const double pos = (double)tok_pos[t];
+  constexpr int E = 16 / sizeof(T);
+  const int id = ids[t];
+  const T* row = FRAG ? table + (size_t)(id / 16) * 16 * width + (id % 16) * E : table + (size_t)id * width;
+  const double pos = inv ? (double)tok_pos[t] : 0.0;
   const int n_pairs = (width + 1) / 2;
   for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) {
     float sn = 0.f, cs = 0.f;
@@ -372,9 +377,10 @@ __global__ void embed_streams_waves_kernel(const T* __restrict__ table, const in
       const double turns = rint(angle * 0.15915494309189535);
       sincosf((float)fma(-turns, 6.283185307179586, angle), &sn, &cs);
     }
-    const float a = fmaf(Num<T>::load(row + 2 * i), scale, sn);
+    const T* at = FRAG ? row + (size_t)(2 * i / E) * 16 * E + 2 * i % E : row + 2 * i;      // (E is even: a pair is within a piece)
+    const float a = fmaf(Num<T>::load(at), scale, sn);
     const bool two = 2 * i + 1 < width;
-    const float b = two ? fmaf(Num<T>::load(row + 2 * i + 1), scale, cs) : 0.f;
+    const float b = two ? fmaf(Num<T>::load(at + 1), scale, cs) : 0.f;
     const bool pair = two && width % 2 == 0 && stream_stride % 2 == 0 && (reinterpret_cast<uintptr_t>(x) & 7) == 0;
     for (int s = 0; s < n_streams; ++s) {
       float* xr = x + (size_t)s * stream_stride + (size_t)t * width + 2 * i;
@@ -392,18 +398,32 @@ extern "C" int rb_embed_streams_waves(const void* table, int table_dtype, const 
                                       const int32_t* tok_pos, float* x, int n_streams, long long stream_stride, int n_tokens, int width,
                                       void* stream) {
   RB_RECORDED(rb_embed_streams_waves(table, table_dtype, ids, scale, inv, tok_pos, x, n_streams, stream_stride, n_tokens, width, stream));
+  return rb_embed_streams_layout(table, table_dtype, 0, ids, scale, inv, tok_pos, x, n_streams, stream_stride, n_tokens, width, stream);
+}
+
+// The same from a table of either layout (0: rows; 1: fragment-major).
+extern "C" int rb_embed_streams_layout(const void* table, int table_dtype, int table_layout, const int32_t* ids, float scale,
+                                       const double* inv, const int32_t* tok_pos, float* x, int n_streams, long long stream_stride,
+                                       int n_tokens, int width, void* stream) {
+  RB_RECORDED(rb_embed_streams_layout(table, table_dtype, table_layout, ids, scale, inv, tok_pos, x, n_streams, stream_stride, n_tokens,
+                                      width, stream));
   RB_REQUIRE(n_tokens >= 0 && width > 0 && n_streams >= 1 && stream_stride >= 0, "rb_embed_streams_waves: bad sizes");
   RB_REQUIRE(inv == nullptr || tok_pos != nullptr, "rb_embed_streams_waves: a wave needs the tokens' positions");
+  RB_REQUIRE(table_dtype == RB_F32 || table_dtype == RB_BF16, "rb_embed_streams_waves: unknown dtype %d", table_dtype);
+  RB_REQUIRE(table_layout == 0 || (table_layout == 1 && width % (table_dtype == RB_F32 ? 16 : 32) == 0),
+             "rb_embed_streams_waves: layout %d of a table of width %d", table_layout, width);
   if (n_tokens == 0) return 0;
-  hipStream_t s = (hipStream_t)stream;
-  if (table_dtype == RB_F32)
-    embed_streams_waves_kernel<float><<<n_tokens, 256, 0, s>>>((const float*)table, ids, scale, inv, tok_pos, x, n_streams,
-                                                               (size_t)stream_stride, width);
-  else if (table_dtype == RB_BF16)
-    embed_streams_waves_kernel<bf16_t><<<n_tokens, 256, 0, s>>>((const bf16_t*)table, ids, scale, inv, tok_pos, x, n_streams,
-                                                                (size_t)stream_stride, width);
-  else
-    RB_REQUIRE(false, "rb_embed_streams_waves: unknown dtype %d", table_dtype);
+#define ES_GO(T, FRAG)                                                                                                          \
+  embed_streams_waves_kernel<T, FRAG><<<n_tokens, 256, 0, (hipStream_t)stream>>>((const T*)table, ids, scale, inv, tok_pos, x, \
+                                                                                 n_streams, (size_t)stream_stride, width)
+  if (table_dtype == RB_F32) {
+    if (table_layout) ES_GO(float, true);
+    else ES_GO(float, false);
+  } else {
+    if (table_layout) ES_GO(bf16_t, true);
+    else ES_GO(bf16_t, false);
+  }
+#undef ES_GO
   RB_LAUNCH_CHECK();
   return 0;
 }

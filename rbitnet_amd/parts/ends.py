@@ -16,7 +16,8 @@ embedding "table" (crates/bitnet-core/src/llama/model.rs:229-232): x[t, :] = tab
     that offers `add_normed`) with norm_name (its tensor): the stream starts as norm(row), and the first block also gets
     these rows in the compute dtype (forward then returns the stream and a `StreamCopy`).
     Interface of an embedding: tensor_specs() / load(tensors) / forward(ctx) -> float32 [T, E]
-    (ctx.token_ids int32 [T]); `table` if a head may share it.
+    (ctx.token_ids int32 [T]); `table` if a head may share it, and `as_matrix()` if the embedding can read the
+    table the way the output product wants it stored.
 
 head "linear" (model.rs:309-315): logits = W norm(x), on the asked rows only; W is the
     embedding's table when the parameters name no matrix (tied).
@@ -38,7 +39,7 @@ import torch
 
 from ..errors import ConfigError
 from .base import BuildEnv, Part, TensorSpec, build_part, register_embedding, register_head
-from .linear import linear, pack_rows
+from .linear import Matrix, fragment_major_ok, linear, pack_rows
 from .stream import StreamCopy, normed_for
 
 
@@ -69,7 +70,7 @@ class TableEmbedding(Part):
             self.norm_name = str(params["norm_name"])
             if self.streams is not None or not hasattr(self.norm, "add_normed") or len(self.norm.tensor_specs()) != 1:
                 raise ConfigError("a norm behind the embedding: one copy of the stream, and a norm of one tensor that can stand on an output")
-        self.table: Optional[torch.Tensor] = None
+        self.table = None             # a tensor of rows, or, once a head shares it, a `Matrix`
         self.positions: Optional[torch.Tensor] = None
 
     def tensor_specs(self) -> Dict[str, TensorSpec]:
@@ -98,24 +99,33 @@ class TableEmbedding(Part):
     def step_bytes(self, element_size: int) -> int:
         return 0                      # the gather reads a few rows only
 
+    def as_matrix(self):
+        """The table as the output matrix of a head that shares it: stored fragment-major where the products read that, and from
+        then on gathered from as it is stored (no second copy is kept)."""
+        t = self.table
+        if (isinstance(t, torch.Tensor) and self.positions is None and not getattr(self.env, "generic_only", False)
+                and fragment_major_ok(t.dtype, *t.shape)):
+            self.table = pack_rows(self.env.lib, [(t, 0, None, None)], t.shape[0], t.shape[1], t.dtype, t.device)
+        return self.table
+
     def forward(self, ctx) -> torch.Tensor:
+        lib, table, frag = self.env.lib, self.table, isinstance(self.table, Matrix)
+        table = table.data if frag else table
+        scale = 1.0 if self.scale is None else self.scale
         if self.streams is not None:
-            x = torch.empty((self.streams, ctx.n_tokens, self.hidden), dtype=torch.float32, device=self.table.device)
-            if self.waves is not None or self.scale is not None:
-                self.env.lib.embed_streams_waves(self.table, ctx.token_ids, 1.0 if self.scale is None else self.scale, self.inv,
-                                                 ctx.tok_pos, x)
+            x = torch.empty((self.streams, ctx.n_tokens, self.hidden), dtype=torch.float32, device=table.device)
+            if self.waves is not None or self.scale is not None or frag:
+                lib.embed_streams_waves(table, ctx.token_ids, scale, self.inv, ctx.tok_pos, x, frag)
             else:
-                self.env.lib.embed_streams(self.table, ctx.token_ids, x)
+                lib.embed_streams(table, ctx.token_ids, x)
             return x
-        x = torch.empty((ctx.n_tokens, self.hidden), dtype=torch.float32, device=self.table.device)
-        if self.waves is not None:
-            self.env.lib.embed_streams_waves(self.table, ctx.token_ids, 1.0 if self.scale is None else self.scale, self.inv,
-                                             ctx.tok_pos, x.unsqueeze(0))
+        x = torch.empty((ctx.n_tokens, self.hidden), dtype=torch.float32, device=table.device)
+        if self.waves is not None or frag:
+            lib.embed_streams_waves(table, ctx.token_ids, scale, self.inv, ctx.tok_pos, x.unsqueeze(0), frag)
         elif self.scale is not None or self.positions is not None:
-            self.env.lib.embed_scaled_pos(self.table, ctx.token_ids, 1.0 if self.scale is None else self.scale,
-                                          self.positions, ctx.tok_pos, x)
+            lib.embed_scaled_pos(table, ctx.token_ids, scale, self.positions, ctx.tok_pos, x)
         else:
-            self.env.lib.embed_gather(self.table, ctx.token_ids, x)
+            lib.embed_gather(table, ctx.token_ids, x)
         if self.norm is not None:
             rows = torch.empty((ctx.n_tokens, self.hidden), dtype=torch.float32, device=x.device)
             h = rows if self.env.dtype == torch.float32 else torch.empty_like(rows, dtype=self.env.dtype)
@@ -172,10 +182,10 @@ class LinearHead(Part):
     def load(self, tensors: Dict[str, torch.Tensor], embedding=None) -> None:
         self.norm.load({name: tensors[full] for full, name in self._norm_names().items()})
         if self.name is None:
-            table = getattr(embedding, "table", None)
+            table = embedding.as_matrix() if hasattr(embedding, "as_matrix") else getattr(embedding, "table", None)
             if table is None or tuple(table.shape) != (self.vocab_size, self.hidden):
                 raise ConfigError("a head without a matrix of its own needs an embedding whose table it can share")
-            self.weight = table                 # tied: the table's rows are also read one by one, so it stays rows
+            self.weight = table
             return
         w = tensors[str(self.name)]
         self.weight = pack_rows(self.env.lib, [(w, 0, None, None)], w.shape[0], w.shape[1], w.dtype, w.device,

@@ -156,6 +156,32 @@ def test_the_two_ends_alone(lib, dtype, tol, tied):
             head.load({"final.weight": gain.to(DEV)}, embedding=None)
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-6), (torch.bfloat16, 8e-3)])
+@pytest.mark.parametrize("streams", [None, 3])
+@pytest.mark.parametrize("vocab,hidden,stored", [(336, 128, True), (16, 256, True), (336, 96, False), (330, 128, False)])
+def test_a_tied_table_is_gathered_from_as_the_output_matrix_stores_it(lib, dtype, tol, streams, vocab, hidden, stored):
+    """The rows of a table that a head shares, first and last ids and edges of blocks of 16 rows among them, and the head's logits
+    from the same memory; sizes that the products want as rows stay rows."""
+    env = _env(lib, hidden, dtype)
+    scale = None if streams is None else 2.5
+    emb = build_part("embedding", PartSpec("table", {"name": "e", "vocab_size": vocab, "streams": streams, "scale": scale}), env)
+    head = build_part("head", PartSpec("linear", {"norm": PartSpec("rmsnorm", {"size": hidden, "eps": 1e-4}), "norm_name": "g",
+                                                  "vocab_size": vocab}), env)
+    table = (torch.randn(vocab, hidden) * 0.5).to(dtype)
+    gain = 1 + 0.2 * torch.randn(hidden)
+    emb.load({"e": table.to(DEV)})
+    head.load({"g": gain.to(DEV)}, embedding=emb)
+    assert isinstance(head.weight, torch.Tensor) != stored and head.weight is emb.table
+    ids = [0, vocab - 1, 15 % vocab, 16 % vocab, 17 % vocab, vocab // 2]
+    ctx = StepContext.for_batch(DEV, StepBatch([0], [0], [ids], [0, 1, 5], {}), n_compute_units=lib.n_compute_units)
+    x = emb.forward(ctx)
+    want = table[ids].float() * (1.0 if scale is None else scale)
+    assert all(torch.equal(c, want) for c in (x.cpu() if streams else [x.cpu()]))
+    if streams is None:
+        want = P.linear(P.rmsnorm(want.double()[[0, 1, 5]], gain.double(), 1e-4), table.double())
+        assert _rel(head.forward(x, None, ctx.rows, ctx), want) < tol
+
+
 def _attention_params(hq, hk, d, window=None, theta=10000.0, style="interleaved", scaling=None):
     return {"num_heads": hq, "num_kv_heads": hk, "head_dim": d, "scale": 1 / math.sqrt(d), "window": window,
             "cache_from": None,
