@@ -42,6 +42,7 @@ from __future__ import annotations
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 
 from ..errors import CacheError, InferenceError
@@ -198,6 +199,8 @@ class Cache:
             r = reqs[key]
             g = _GROUP_KINDS[r.kind](r, layers, self.n_pages, self.n_slots, dtype, device)
             self.groups.append(g)
+            if getattr(g, "paged", False):
+                g.table.put(self.spare_slot, 0, g.spare_page)
             for l in layers:
                 self.layer_groups.setdefault(l, []).append((g, g.index[l]))
         for l, j in (readers or {}).items():
@@ -275,11 +278,21 @@ class Cache:
             for s, q in zip(slots, q_lens):
                 g.table.ensure(s, self.lens[s] + q)
 
+    def reserve_one(self, slots: Sequence[int], past: Sequence[int]) -> None:
+        """`reserve` for one token more of every sequence, `past` being their lengths: only a sequence whose pages are full
+        (its length is a multiple of the page's) can need another."""
+        if len(set(slots)) != len(slots):
+            raise InferenceError("a slot appears twice in one step")
+        full = [s for s, n in zip(slots, past) if n % PAGE_SIZE == 0]
+        if full:
+            self.reserve(full, [1] * len(full))
+
     def commit(self, slots: Sequence[int], q_lens: Sequence[int]) -> None:
         """The step has run: lengths grow, windowed groups give dead pages back."""
+        windowed = [g for g in self.kv_groups if g.table.window is not None]
         for s, q in zip(slots, q_lens):
             self.lens[s] += q
-            for g in self.kv_groups:
+            for g in windowed:
                 g.table.release_behind(s, self.lens[s])
 
     def group_keys(self) -> List[int]:
@@ -290,6 +303,11 @@ class Cache:
         window is never read; 0 stands in for it).  The spare slot holds the spare page."""
         return {id(g): [[g.spare_page] if s == self.spare_slot else [(p if p >= 0 else 0) for p in g.table.pages(s)]
                         for s in slots] for g in self.kv_groups}
+
+    def table_rows(self, slots: Sequence[int], width: int) -> Dict[int, np.ndarray]:
+        """`block_tables` as arrays [len(slots), at most `width`]: per paged group, the rows of the slots (the spare slot's among
+        them); what lies behind a sequence's pages means nothing."""
+        return {id(g): g.table.rows[slots, :width] for g in self.kv_groups}
 
     def view(self, layer: int, block_tables: Dict[int, torch.Tensor]) -> LayerCacheView:
         v = LayerCacheView()

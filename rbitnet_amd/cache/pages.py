@@ -14,6 +14,8 @@ from __future__ import annotations
 import heapq
 from typing import Dict, List, Optional
 
+import numpy as np
+
 from ..errors import CacheError
 
 PAGE_SIZE = 64
@@ -75,13 +77,26 @@ class PageTable:
     positions [i * PAGE_SIZE, (i + 1) * PAGE_SIZE).  With a window, pages that lie wholly
     behind every future query's reach are given back early; their entries stay in the
     table as -1 and are never read.  `keep_first` tokens at a sequence's start stay in reach
-    whatever the window: the pages that hold them are never given back early."""
+    whatever the window: the pages that hold them are never given back early.
+
+    `rows` is the same as an array, one row per slot, for steps that take the tables of many slots at once: entry i of a
+    row is the slot's page i, 0 for one that was given back; what lies behind a slot's pages means nothing."""
 
     def __init__(self, n_pages: int, window: Optional[int] = None, keep_first: int = 0):
         self.pool = FreeList(n_pages, "cache page")
         self.window = window
         self.keep_first = max(0, int(keep_first or 0))
         self.tables: Dict[int, List[int]] = {}
+        self.rows = np.zeros((0, 0), dtype=np.int32)
+
+    def put(self, slot: int, i: int, page: int) -> None:
+        """Entry i of the slot's row of `rows`, which grows as it has to."""
+        n, width = self.rows.shape
+        if slot >= n or i >= width:
+            more = np.zeros((max(n, 2 * slot if slot >= n else 0, slot + 1), max(width, 2 * i if i >= width else 0, i + 1)), dtype=np.int32)
+            more[:n, :width] = self.rows
+            self.rows = more
+        self.rows[slot, i] = page
 
     def open(self, slot: int) -> None:
         if slot in self.tables:
@@ -101,6 +116,7 @@ class PageTable:
                 f"{self.pool.n_free} of {self.pool.n} are free")
         for _ in range(need):
             table.append(self.pool.take())
+            self.put(slot, len(table) - 1, table[-1])
         return True
 
     def release_behind(self, slot: int, length: int) -> int:
@@ -115,6 +131,7 @@ class PageTable:
             if table[i] >= 0:
                 self.pool.give_back(table[i])
                 table[i] = -1
+                self.put(slot, i, 0)
                 n += 1
         return n
 
@@ -132,6 +149,8 @@ class PageTable:
         self.pool.check()
         seen = set()
         for slot, table in self.tables.items():
+            if table and self.rows[slot, :len(table)].tolist() != [max(p, 0) for p in table]:
+                raise CacheError(f"the pages of slot {slot} and its row of the array differ")
             for p in table:
                 if p < 0:
                     continue

@@ -149,6 +149,8 @@ class Kernels:
                                                _P, _P],
             "rb_attention_decode_fused_bf16_sinks": [_P, _I, ctypes.c_longlong, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
                                                      _F, _I, _I, _P, _P, _P],
+            "rb_fetch_words": [_P, _P, _L, _P],
+            "rb_stream_wait": [_P],
             "rb_sample": [_P, _I, _I, _P, _P, _P, _P, _P],
             "rb_fill_normal": [_P, _I, ctypes.c_longlong, ctypes.c_ulonglong, ctypes.c_double, ctypes.c_double, _P],
             "rb_place_rows": [_P, _I, _P, _I, _I] + [ctypes.c_longlong] * 6 + [_P],
@@ -523,7 +525,11 @@ class Kernels:
         if temperature is not None:
             _check(temperature, "temperature", torch.float32, (n,))
             _check(u, "u", torch.float32, (n,))
-        _check(tokens, "tokens", torch.int32, (n,))
+        if not tokens.is_cuda and tokens.is_pinned():       # pinned host memory: the kernel writes it where it is
+            if tokens.dtype != torch.int32 or tuple(tokens.shape) != (n,) or not tokens.is_contiguous():
+                raise KernelError(f"tokens must be int32 [{n}]")
+        else:
+            _check(tokens, "tokens", torch.int32, (n,))
         need = int(self._lib.rb_sample_workspace_bytes(n, vocab))
         if workspace is None:
             workspace = torch.empty((need + 7) // 8, dtype=torch.int64, device=logits.device)
@@ -532,6 +538,18 @@ class Kernels:
             raise KernelError("sampling workspace too small")
         self._ok(self._lib.rb_sample(_ptr(logits), n, vocab, _ptr(temperature), _ptr(u), _ptr(tokens),
                                      _ptr(workspace), self._stream()))
+
+    def fetch_words(self, host: torch.Tensor, out: torch.Tensor) -> None:
+        """int32 words from pinned host memory to the GPU, by a kernel that reads them where they are when it runs (a captured
+        step's own copy of what changes between its replays)."""
+        if not host.is_pinned() or host.dtype != torch.int32 or not host.is_contiguous():
+            raise KernelError("host must be contiguous int32 in pinned memory")
+        _check(out, "out", torch.int32, host.shape)
+        self._ok(self._lib.rb_fetch_words(_ptr(host), _ptr(out), out.numel(), self._stream()))
+
+    def wait(self) -> None:
+        """Until everything that was put on torch's current stream has run."""
+        self._ok(self._lib.rb_stream_wait(self._stream()))
 
     # ------------------------------------------------------------------ streams, layer norm, activations
     def embed_streams(self, table: torch.Tensor, ids: torch.Tensor, x: torch.Tensor) -> None:

@@ -270,3 +270,27 @@ extern "C" int rb_sample_static(const float* logits, int n_rows, int vocab, cons
   RB_LAUNCH_CHECK();
   return 0;
 }
+
+// ---------------------------------------------------------------- a captured step's inputs and its end
+// n words from pinned host memory: what changes between the replays of a captured step, read when the kernel runs.  Loads at the scope of
+// the whole system: no cache of the GPU may answer with the words of the replay before.  One launch at the head of the graph in place of
+// a copy in front of it (10 us a step between the call and the first kernel).
+__global__ __launch_bounds__(256) void fetch_words_kernel(const int32_t* host, int32_t* __restrict__ out, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    out[i] = __hip_atomic_load(host + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+extern "C" int rb_fetch_words(const int32_t* host, int32_t* out, long long n, void* stream) {
+  RB_RECORDED(rb_fetch_words(host, out, n, stream));
+  RB_REQUIRE(n >= 0, "rb_fetch_words: negative count");
+  if (n == 0) return 0;
+  const long long blocks = (n + 255) / 256;
+  fetch_words_kernel<<<(int)(blocks < 256 ? blocks : 256), 256, 0, (hipStream_t)stream>>>(host, out, (size_t)n);
+  RB_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int rb_stream_wait(void* stream) {
+  const hipError_t e = hipStreamSynchronize((hipStream_t)stream);
+  RB_REQUIRE(e == hipSuccess, "rb_stream_wait: %s", hipGetErrorString(e));
+  return 0;
+}

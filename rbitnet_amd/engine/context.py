@@ -162,8 +162,8 @@ class StepContext:
         ctx.fill(batch)
         return ctx
 
-    def fill(self, batch: StepBatch) -> None:
-        """Writes the batch into the layout and copies it to the GPU (one copy)."""
+    def fill(self, batch: StepBatch, copy: bool = True) -> None:
+        """Writes the batch into the layout and copies it to the GPU (one copy; copy False: a captured step does that itself)."""
         if self._copied is not None:
             self._copied.synchronize()        # the copy before this one has read the host buffer
         q_lens = [len(t) for t in batch.tokens]
@@ -200,11 +200,33 @@ class StepContext:
         self.host_past = list(batch.past_lens)
         if self.fixed_bucket is None:
             self.bucket = split_bucket(self.max_kv_len)
+        if not copy:
+            return
         self._dev.copy_(self._host, non_blocking=True)
         if self._host.is_pinned():
             if self._copied is None:
                 self._copied = torch.cuda.Event()
             self._copied.record()
+
+    def fetch(self, lib) -> None:
+        """The copy of the layout to the GPU as a launch of the step's own: the kernel reads what the host has written by then."""
+        lib.fetch_words(self._host, self._dev)
+
+    def refill_single(self, slots: Sequence[int], past: Sequence[int], tokens: Sequence[int], tables: Dict[int, np.ndarray],
+                      temperatures: Optional[Sequence[float]], uniforms: Optional[Sequence[float]]) -> None:
+        """What differs between two batches of one token per sequence, written into the layout (whose other arrays a `fill` wrote
+        before); a captured step copies it over itself.  tables: per storage group, an array of rows at most as wide as the layout's."""
+        h = self._h
+        h["token_ids"][:] = tokens
+        h["tok_pos"][:] = past
+        h["past_len"][:] = past
+        h["slots"][:] = slots
+        h["temperature"][:] = 0.0 if temperatures is None else temperatures
+        h["uniform"][:] = 0.0 if uniforms is None else uniforms
+        for key, rows in tables.items():
+            h[("table", key)][:, :rows.shape[1]] = rows
+        self.max_kv_len = max(past) + 1
+        self.host_slots, self.host_past = list(slots), list(past)
 
     def tile_split_workspace(self, n_heads: int, head_dim: int, pages_per_split: int = 1) -> Tuple:
         """Split count and scratch for an attention kernel whose workgroup takes ALL heads of a sequence and to which a

@@ -1,5 +1,5 @@
 """The decode step as a HIP graph: one token per sequence in, the next token per
-sequence out, replayed with nothing but one small host-to-device copy in between.
+sequence out, replayed with nothing but a few words of pinned host memory written in between.
 
 A decode step of a 32-layer model is some three hundred kernel launches; issued one by
 one from Python they cost more host time than the GPU needs to run them.  The launches of
@@ -7,8 +7,12 @@ one step depend only on the number of sequences, so they are captured once per b
 into a graph whose kernels read everything that changes (tokens, positions, page tables,
 temperatures, uniform numbers) from fixed device buffers.
 
-No memset is recorded into the graph (the buffers are written by a copy issued before
-each replay, outside the graph), and only this library's kernels run inside it.
+Only this library's kernels run inside the graph, no memset and no copy: its first kernel reads the
+step's layout from pinned host memory and its last one writes the chosen tokens there.  Between two
+replays the GPU waits for the host, so the host does little: it writes what differs from the step
+before into the pinned layout, launches, waits, and reads the tokens.  A sequence's pages are taken
+as a row of an array that the page tables keep up to date.  (4 sequences: 80 us between two replays
+with copies and lists, 64 sequences 300 us.)
 
 A batch whose sequences end one by one would need a capture for every size on the way down.
 Graphs are therefore captured for a ladder of sizes only (`graph_size`), and a batch runs in the
@@ -24,6 +28,7 @@ from typing import Optional
 
 import torch
 
+from ..cache import pages_for
 from .context import StepBatch, StepContext, bucket_max_pages
 
 GRAPH_SIZES = (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64)
@@ -52,41 +57,52 @@ class DecodeGraph:
         width = min(engine.cache.pages_per_sequence(engine.max_seq_len), engine.cache.n_pages)
         if bucket_max_pages(bucket) is not None:
             width = min(width, bucket_max_pages(bucket))
-        width = max(1, width)
+        self.width = width = max(1, width)
         self.ctx = StepContext(engine.device, n_seqs, n_seqs, n_seqs,
                                {key: width for key in engine.cache.group_keys()}, bucket=bucket,
                                n_compute_units=engine.lib.n_compute_units)
-        self.tokens_out = torch.zeros(n_seqs, dtype=torch.int32, device=engine.device)
+        self.tokens_out = torch.zeros(n_seqs, dtype=torch.int32).pin_memory()
+        self._tokens = self.tokens_out.numpy()
+        self._in_flight = False
         self.logits: Optional[torch.Tensor] = None           # of the captured launches: valid after a replay
         self.first_logits: Optional[torch.Tensor] = None     # of the step that ran before the capture
         self.graph: Optional[torch.cuda.CUDAGraph] = None
 
-    def _fill(self, slots, tokens, temperatures, uniforms) -> None:
-        cache = self.engine.cache
+    def _fill(self, slots, past, tokens, temperatures, uniforms) -> None:
+        cache, ctx = self.engine.cache, self.ctx
         idle = self.n_seqs - len(slots)
-        past = [cache.length(s) for s in slots] + [0] * idle
-        slots = list(slots) + [cache.spare_slot] * idle
-        pad = lambda values: None if values is None else list(values) + [0.0] * idle
-        self.ctx.fill(StepBatch(slots=slots, past_lens=past,
-                                tokens=[[t] for t in tokens] + [[0]] * idle, rows=list(range(self.n_seqs)),
-                                block_tables=cache.block_tables(slots), temperatures=pad(temperatures),
-                                uniforms=pad(uniforms)))
+        if idle:
+            rest = [0] * idle
+            slots, past, tokens = slots + [cache.spare_slot] * idle, past + rest, tokens + rest
+            temperatures = None if temperatures is None else list(temperatures) + rest
+            uniforms = None if uniforms is None else list(uniforms) + rest
+        if self.graph is None or ctx.extra:        # the first step, and parts with arrays of their own: the whole layout
+            ctx.fill(StepBatch(slots=slots, past_lens=past, tokens=[[t] for t in tokens], rows=list(range(self.n_seqs)),
+                               block_tables=cache.block_tables(slots), temperatures=temperatures, uniforms=uniforms), copy=False)
+            return
+        if pages_for(max(past) + 1) > self.width:
+            raise ValueError("a sequence holds more pages than the step layout has room for")
+        ctx.refill_single(slots, past, tokens, cache.table_rows(slots, self.width), temperatures, uniforms)
 
     def _launch(self) -> None:
         eng, c = self.engine, self.ctx
+        c.fetch(eng.lib)
         self.logits = eng.model.forward(c, eng.cache, c.rows)
         eng.lib.sample(self.logits, c.temperature, c.uniform, self.tokens_out)
 
-    def run(self, slots, tokens, temperatures=None, uniforms=None) -> list:
-        """The step for these sequences (at most as many as the graph was made for); returns their
+    def run(self, slots, past, tokens, temperatures=None, uniforms=None) -> list:
+        """The step for these sequences (at most as many as the graph was made for), `past` being their lengths; returns their
         next tokens.  `logits`/`first_logits` hold a row per row of the graph, the live ones first."""
         eng = self.engine
         n = len(slots)
         if not 1 <= n <= self.n_seqs:
             raise ValueError(f"a captured step for {self.n_seqs} sequences cannot run {n}")
-        q = [1] * n
-        eng.cache.reserve(slots, q)
-        self._fill(slots, tokens, temperatures, uniforms)
+        if len(tokens) != n:
+            raise ValueError(f"{len(tokens)} tokens for {n} sequences")
+        if self._in_flight:                      # a wait was interrupted: the kernels may still read the layout
+            torch.cuda.synchronize()
+        eng.cache.reserve_one(slots, past)
+        self._fill(slots, past, tokens, temperatures, uniforms)
         if self.graph is None:
             # The first step for this batch size is launched kernel by kernel, on a side stream so
             # that allocations settle, and its result is the step's result; then the same launches
@@ -98,17 +114,20 @@ class DecodeGraph:
                 self._launch()
             torch.cuda.current_stream().wait_stream(side)
             torch.cuda.synchronize()
-            out = self.tokens_out.tolist()[:n]
+            out = self._tokens[:n].tolist()
             first_logits = self.logits.clone()
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 self._launch()
             self.graph = graph
             self.first_logits = first_logits
-            eng.cache.commit(slots, q)
+            eng.cache.commit(slots, [1] * n)
             return out
         self.first_logits = None
+        self._in_flight = True
         self.graph.replay()
-        out = self.tokens_out.tolist()[:n]
-        eng.cache.commit(slots, q)
+        eng.lib.wait()
+        self._in_flight = False
+        out = self._tokens[:n].tolist()
+        eng.cache.commit(slots, [1] * n)
         return out

@@ -16,6 +16,7 @@ import sys
 from collections import OrderedDict
 from typing import Any, List, Optional, Sequence, Tuple, Union
 
+import numpy as np
 import torch
 
 from ..cache import PAGE_SIZE, Cache, pages_for
@@ -43,6 +44,19 @@ def parse_dtype(dtype: Any) -> torch.dtype:
     if dtype not in _DTYPES:
         raise ConfigError(f"dtype must be 'bfloat16' or 'float32', found {dtype!r}")
     return _DTYPES[dtype]
+
+
+def _token_array(tokens) -> np.ndarray:
+    """Token ids as an array: a prompt's thousands are checked and packed as one."""
+    tokens = tokens if isinstance(tokens, (list, np.ndarray)) else list(tokens)
+    try:
+        ids = np.asarray(tokens, dtype=np.int64)
+    except OverflowError:
+        bad = next(t for t in map(int, tokens) if not -1 << 63 <= t < 1 << 63)
+        raise InferenceError(f"token id out of range ({bad})") from None
+    if ids.ndim != 1:
+        raise InferenceError(f"a sequence's tokens are one row of ids, not an array of shape {ids.shape}")
+    return ids
 
 
 class Engine:
@@ -184,40 +198,40 @@ class Engine:
         if not entries:
             raise InferenceError("a step needs at least one sequence")
         slots = [int(s) for s, _ in entries]
-        tokens = [list(t) for _, t in entries]
+        tokens = [_token_array(t) for _, t in entries]
         vocab = self.spec.vocab_size
         past = []
         for s, toks in zip(slots, tokens):
-            if not toks:
+            if not len(toks):
                 raise InferenceError(f"slot {s}: a step brings at least one token per sequence")
             n = self.cache.length(s)
             if n + len(toks) > self.max_seq_len:
                 raise InferenceError(
                     f"slot {s}: sequence position >= max_seq ({n} + {len(toks)} tokens exceed {self.max_seq_len})")
-            for t in toks:
-                if not 0 <= int(t) < vocab:
-                    raise InferenceError(f"slot {s}: token id out of range ({t}, vocabulary {vocab})")
+            if toks.min() < 0 or toks.max() >= vocab:
+                t = next(t for t in toks.tolist() if not 0 <= t < vocab)
+                raise InferenceError(f"slot {s}: token id out of range ({t}, vocabulary {vocab})")
             past.append(n)
         rows: List[int] = []
         base = 0
         for i, toks in enumerate(tokens):
             if want == "last":
-                idx = [len(toks) - 1]
+                rows.append(base + len(toks) - 1)
             elif want == "all":
-                idx = range(len(toks))
+                rows.extend(range(base, base + len(toks)))
             else:
-                idx = want[i]
-            for j in idx:
-                if not 0 <= int(j) < len(toks):
-                    raise InferenceError(f"slot {slots[i]}: wanted place {j} is not among its {len(toks)} tokens")
-                rows.append(base + int(j))
+                for j in want[i]:
+                    if not 0 <= int(j) < len(toks):
+                        raise InferenceError(f"slot {slots[i]}: wanted place {j} is not among its {len(toks)} tokens")
+                    rows.append(base + int(j))
             base += len(toks)
         q_lens = [len(t) for t in tokens]
         if sum(q_lens) > 1024 and self.device.type == "cuda":
             # a long step's activations must fit beside the cache: say so before anything is reserved or launched
             need = self.model.activation_bytes(sum(q_lens), len(rows))
-            free = torch.cuda.mem_get_info(self.device)[0] + torch.cuda.memory_reserved(self.device) \
-                - torch.cuda.memory_allocated(self.device)
+            free = torch.cuda.mem_get_info(self.device)[0]
+            if need > free:                   # (what the allocator holds is asked for only where it matters)
+                free += torch.cuda.memory_reserved(self.device) - torch.cuda.memory_allocated(self.device)
             if need > free:
                 raise InferenceError(
                     f"a step of {sum(q_lens)} tokens needs about {need / 2**30:.1f} GiB for its activations and "
@@ -241,28 +255,30 @@ class Engine:
         sampling of its logits, replayed as a HIP graph (captured for a ladder of batch sizes, a
         batch running in the next size up with idle rows, see decode_graph.py);
         `use_graphs = False` runs the same kernels launch by launch."""
-        slots = [int(s) for s in slots]
-        tokens = [int(t) for t in tokens]
+        slots = list(map(int, slots))
+        tokens = list(map(int, tokens))
         vocab = self.spec.vocab_size
-        for s, t in zip(slots, tokens):
-            if not 0 <= t < vocab:
-                raise InferenceError(f"slot {s}: token id out of range ({t}, vocabulary {vocab})")
-            if self.cache.length(s) + 1 > self.max_seq_len:
-                raise InferenceError(f"slot {s}: sequence position >= max_seq ({self.max_seq_len})")
+        past = [self.cache.length(s) for s in slots]
+        if len(tokens) < len(slots) or min(tokens, default=0) < 0 or max(tokens, default=0) >= vocab or max(past, default=0) >= self.max_seq_len:
+            for s, t, n in zip(slots, tokens, past):
+                if not 0 <= t < vocab:
+                    raise InferenceError(f"slot {s}: token id out of range ({t}, vocabulary {vocab})")
+                if n + 1 > self.max_seq_len:
+                    raise InferenceError(f"slot {s}: sequence position >= max_seq ({self.max_seq_len})")
         if not self.use_graphs:
             logits = self.step([(s, [t]) for s, t in zip(slots, tokens)], "last")
             self.last_decode_logits = logits
             return self.sampler.sample(logits, temperatures, uniforms)
         from .decode_graph import DecodeGraph, graph_size
         n = len(slots)
-        key = (graph_size(n), split_bucket(max(self.cache.length(s) for s in slots) + 1))
+        key = (graph_size(n), split_bucket(max(past) + 1))
         if key not in self._graphs:
             if len(self._graphs) >= MAX_DECODE_GRAPHS:
                 self._graphs.popitem(last=False)           # the least recently used
             self._graphs[key] = DecodeGraph(self, key[0], key[1])
         self._graphs.move_to_end(key)
         graph = self._graphs[key]
-        out = graph.run(slots, tokens, temperatures, uniforms)
+        out = graph.run(slots, past, tokens, temperatures, uniforms)
         self.last_decode_logits = (graph.logits if graph.first_logits is None else graph.first_logits)[:n]
         self.stats["steps"] += 1
         self.stats["decode_tokens"] += n

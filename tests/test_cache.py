@@ -98,6 +98,39 @@ def test_random_traffic_never_loses_anything():
     assert c.kv_groups[0].table.pool.n_free == 40 and c.slots.n_free == 6
 
 
+@pytest.mark.parametrize("window", [None, 70, 200])
+def test_rows_of_page_tables_and_steps_of_one_token(window):
+    """The array of page tables beside the lists, and `reserve_one` beside `reserve`, over random traffic: prompts, single tokens
+    (across full pages, and where the pool runs out), slots given back and taken again."""
+    rng = random.Random(7)
+    c, plain = _cache(n_slots=5, max_tokens=64 * 12, window=window), _cache(n_slots=5, max_tokens=64 * 12, window=window)
+    g = c.kv_groups[0]
+    for _ in range(600):
+        live = c.live_slots
+        kind = rng.random()
+        if kind < 0.15 and len(live) < 5:
+            assert c.alloc_slot() == plain.alloc_slot()
+        elif kind < 0.2 and live:
+            slot = rng.choice(live)
+            c.free_slot(slot), plain.free_slot(slot)
+        elif live:
+            slots = rng.sample(live, rng.randint(1, len(live)))
+            q = [rng.randint(1, 90) for _ in slots] if kind < 0.3 else [1] * len(slots)
+            for one, cache in ((kind >= 0.3, c), (False, plain)):
+                try:
+                    cache.reserve_one(slots, [cache.length(s) for s in slots]) if one else cache.reserve(slots, q)
+                    cache.commit(slots, q)
+                except CacheError:
+                    pass
+        c.check()
+        assert c.lens == plain.lens and g.table.tables == plain.kv_groups[0].table.tables
+        slots = c.live_slots + [c.spare_slot]
+        lists, rows = c.block_tables(slots)[id(g)], c.table_rows(slots, 12)[id(g)]
+        assert len(rows) == len(slots) and all(r[:len(l)].tolist() == l for l, r in zip(lists, rows))
+    with pytest.raises(InferenceError, match="twice"):
+        c.reserve_one([0, 0], [0, 0])
+
+
 def test_groups_by_need_and_readers():
     reqs = [CacheRequest("kv", heads=2, head_dim=8), CacheRequest("kv", heads=2, head_dim=8, window=100),
             None, CacheRequest("kv", heads=2, head_dim=8), CacheRequest("kv", heads=1, head_dim=16),
