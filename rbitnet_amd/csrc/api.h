@@ -234,6 +234,35 @@ int rb_gated_rmsnorm_act(const float* o, const float* weight, const float* gate,
 int rb_short_conv_biases(const float* x, long long x_stride, const float* bias, const float* bias_out, const float* w, int taps, float* state,
                          const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* cu_seqlens, const int32_t* slots, void* out,
                          long long out_stride, int out_dtype, int residual, int act, int n_tokens, int n_seqs, int channels, void* stream);
+// A step of ONE token per sequence (token t is of slot slots[t]) through such a layer in one launch: convolution and silu (conv_w null:
+// none; the state moves on), unit vectors or the query's scale, decays, the recurrence, the read-out norm and its gate.
+//   mode 0: the delta rule (beta = sigmoid(b)); 1: the plain rule; 2: read before the write, with a bonus [H, dim]; 3: the selective scan,
+//   whose step size softplus(a + a_bias) also makes the decay, with d [H].   decay as in rb_recurrence_prep, a_per_head: one a head.
+//   norm_part 0: out = o / sqrt(mean over the head's vdim + eps) * norm[h * norm_head_stride + i] * act(gate); else the gate first, then
+//   the norm over parts of norm_part numbers, norm [H * vdim].  gate_act 0: sigmoid(gate), 1: silu(gate).
+// conv_q, conv_k, conv_v: the first channels of q, k and v among the convolution's conv_channels; q, k and v head-major from their pointers.
+struct RbRecurrenceStep {
+  const float *q, *k, *v;
+  long long q_stride, k_stride, v_stride;
+  const float *conv_w, *conv_bias;
+  float* conv_state;
+  const float* a;
+  long long a_stride;
+  const float *a_bias, *a_log, *b;
+  long long b_stride;
+  const float *bonus, *d;
+  float* state;
+  const int32_t* slots;
+  const float* gate;
+  long long gate_stride;
+  const float* norm;
+  void* out;
+  float tau, q_scale, unit_eps, eps;
+  int mode, unit, taps, conv_channels, conv_q, conv_k, conv_v, a_per_head, decay, gate_act, norm_head_stride, norm_part, out_dtype;
+  int n_tokens, n_heads, n_kv_heads, dim, vdim;
+};
+int rb_recurrence_step_ok(int n_heads, int n_kv_heads, int dim, int vdim, int taps, int norm_part);
+int rb_recurrence_step(const struct RbRecurrenceStep* args, void* stream);
 // A selective scan, token after token, on the state S kept column by column as [slots, H, vdim, dim]; with
 // dt = softplus(dt_in[t * dt_stride + h] + dt_bias[h]):
 //   S <- exp(-exp(a_log[h]) dt) S + dt k v^T;  out[t, h, :] = S^T q + d[h] v      (head h reads the q and k of group h / (H / G))

@@ -105,7 +105,7 @@ class KernelTimes:
         return "\n".join(lines)
 
 
-TIMED_OPS = ("routed_experts_tiled", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
+TIMED_OPS = ("routed_experts_tiled", "recurrence_step", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
              "route_top", "routed_experts", "pairs_sum", "embed_streams", "streams_layernorm", "streams_update", "xielu", "tanh_cap", "short_conv",
              "delta_prep", "delta_rule", "gated_rmsnorm", "latent_norm_store", "attention_sinks", "embed_gather", "add_rmsnorm", "rope_kv_write", "swiglu", "gemm_generic", "gemm_bf16", "gemm_bf16_terms",
              "gemm_bf16_few", "attention_generic", "attention_prefill_bf16", "attention_decode_bf16",
@@ -113,6 +113,20 @@ TIMED_OPS = ("routed_experts_tiled", "selective_chunks", "embed_streams_waves", 
 
 
 ROUTED_FEW_TOKENS = 64         # steps of up to so many tokens run their experts in the kernels for few tokens
+
+
+class RecurrenceStep(ctypes.Structure):
+    """RbRecurrenceStep of csrc/api.h."""
+    _fields_ = ([(n, _P) for n in ("q", "k", "v")] + [(n, _L) for n in ("q_stride", "k_stride", "v_stride")]
+                + [(n, _P) for n in ("conv_w", "conv_bias", "conv_state", "a")] + [("a_stride", _L)]
+                + [(n, _P) for n in ("a_bias", "a_log", "b")] + [("b_stride", _L)] + [(n, _P) for n in ("bonus", "d", "state", "slots", "gate")]
+                + [("gate_stride", _L), ("norm", _P), ("out", _P)] + [(n, _F) for n in ("tau", "q_scale", "unit_eps", "eps")]
+                + [(n, _I) for n in ("mode", "unit", "taps", "conv_channels", "conv_q", "conv_k", "conv_v", "a_per_head", "decay",
+                                     "gate_act", "norm_head_stride", "norm_part", "out_dtype", "n_tokens", "n_heads", "n_kv_heads",
+                                     "dim", "vdim")])
+
+
+STEP_MODES = {"delta": 0, "plain": 1, "bonus": 2, "selective": 3}
 
 
 class Kernels:
@@ -167,6 +181,8 @@ class Kernels:
             "rb_embed_streams_layout": [_P, _I, _I, _P, _F, _P, _P, _P, _I, _L, _I, _I, _P],
             "rb_streams_rmsnorm": [_P, _I, _L, _P, _P, _P, _I, _L, _L, _P, _P, _I, _L, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_short_conv_biases": [_P, _L, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
+            "rb_recurrence_step_ok": [_I, _I, _I, _I, _I, _I],
+            "rb_recurrence_step": [ctypes.POINTER(RecurrenceStep), _P],
             "rb_selective_scan": [_P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
             "rb_selective_chunks_ok": [_I, _I],
             "rb_selective_chunks": [_P, _P, _P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
@@ -760,6 +776,72 @@ class Kernels:
         _check(out, "out", None, (n, n_heads * vdim))
         self._ok(self._lib.rb_gated_rmsnorm(_ptr(o), _ptr(weight), gate.data_ptr() + 4 * gate_col, gate.shape[1], float(eps),
                                             _ptr(out), dtype_code(out.dtype), n, n_heads, vdim, self._stream()))
+
+    # ------------------------------------------------------------------ a step of single tokens, in one launch
+    def recurrence_step_ok(self, n_heads: int, n_kv: int, dim: int, vdim: int, taps: int = 0, norm_part: int = 0) -> bool:
+        return bool(self._lib.rb_recurrence_step_ok(n_heads, n_kv, dim, vdim, taps, norm_part))
+
+    def recurrence_step(self, mode: str, q, k, v, n_heads: int, n_kv: int, dim: int, vdim: int, a, a_per_head: bool, decay: int,
+                        state: torch.Tensor, ctx, gate, gate_act: int, norm: torch.Tensor, eps: float, out: torch.Tensor,
+                        conv=None, a_bias=None, a_log=None, tau: float = 1.0, b=None, bonus=None, d=None, unit: bool = False,
+                        q_scale: float = 1.0, unit_eps: float = 0.0, norm_part: int = 0) -> None:
+        """One token per sequence through a layer with a state per head (`RbRecurrenceStep` in csrc/api.h says what it computes).
+        q, k, v, a, b, gate: (matrix [T, W] float32, first column).  conv: None, or (w [channels, taps], bias or None, state, first
+        channel of q, of k, of v).  norm [vdim] or [heads * vdim]."""
+        n = out.shape[0]
+        if ctx.n_tokens != n or ctx.n_seqs != n:
+            raise KernelError("recurrence_step: a step of one token per sequence")
+
+        def part(pair, width, what):
+            m, col = pair
+            _check(m, what, torch.float32)
+            if m.shape[0] != n or col < 0 or col + width > m.shape[1]:
+                raise KernelError(f"recurrence_step: the columns of {what} lie outside the rows")
+            return m.data_ptr() + 4 * col, m.shape[1]
+
+        r = RecurrenceStep(mode=STEP_MODES[mode], unit=int(bool(unit)), a_per_head=int(bool(a_per_head)), decay=int(decay),
+                           gate_act=int(gate_act), norm_part=int(norm_part), out_dtype=dtype_code(out.dtype), n_tokens=n, n_heads=n_heads,
+                           n_kv_heads=n_kv, dim=dim, vdim=vdim, tau=float(tau), q_scale=float(q_scale), unit_eps=float(unit_eps),
+                           eps=float(eps))
+        r.q, r.q_stride = part(q, n_kv * dim, "q")
+        r.k, r.k_stride = part(k, n_kv * dim, "k")
+        r.v, r.v_stride = part(v, n_heads * vdim, "v")
+        r.gate, r.gate_stride = part(gate, n_heads * vdim, "gate")
+        per_head = a_per_head or mode == "selective"
+        n_a = n_heads if per_head else n_heads * dim
+        r.a, r.a_stride = part(a, n_a, "a")
+        if b is not None:
+            r.b, r.b_stride = part(b, n_heads, "b")
+        for name, t, shape in (("a_bias", a_bias, (n_a,)), ("a_log", a_log, (n_heads,)), ("bonus", bonus, (n_heads, dim)), ("d", d, (n_heads,))):
+            if t is not None:
+                _check(t, name, torch.float32, shape)
+                setattr(r, name, _ptr(t))
+        if conv is not None:
+            w, bias_out, conv_state, cq, ck, cv = conv
+            channels, taps = w.shape
+            _check(w, "w", torch.float32)
+            if bias_out is not None:
+                _check(bias_out, "bias_out", torch.float32, (channels,))
+            if taps > 1:
+                _check(conv_state, "conv state", torch.float32)
+                if tuple(conv_state.shape[1:]) != (taps - 1, channels):
+                    raise KernelError(f"recurrence_step: convolution state of shape {tuple(conv_state.shape)}")
+            if min(cq, ck, cv) < 0 or max(cq + n_kv * dim, ck + n_kv * dim, cv + n_heads * vdim) > channels:
+                raise KernelError("recurrence_step: q, k or v lie outside the convolution's channels")
+            r.conv_w, r.conv_bias, r.conv_state = _ptr(w), _ptr(bias_out), _ptr(conv_state) if taps > 1 else None
+            r.taps, r.conv_channels, r.conv_q, r.conv_k, r.conv_v = taps, channels, cq, ck, cv
+        _check(state, "state", torch.float32)
+        if tuple(state.shape[1:]) != (n_heads, vdim, dim):
+            raise KernelError(f"recurrence_step: state of shape {tuple(state.shape)}, expected [*, {n_heads}, {vdim}, {dim}]")
+        if norm_part == 0 and tuple(norm.shape) == (vdim,):
+            r.norm_head_stride = 0
+        else:
+            _check(norm, "norm", None, (n_heads * vdim,))
+            r.norm_head_stride = vdim
+        _check(norm, "norm", torch.float32)
+        _check(out, "out", None, (n, n_heads * vdim))
+        r.state, r.slots, r.norm, r.out = _ptr(state), _ptr(ctx.slots), _ptr(norm), _ptr(out)
+        self._ok(self._lib.rb_recurrence_step(ctypes.byref(r), self._stream()))
 
     # ------------------------------------------------------------------ recurrences with their choices spelled out
     def recurrence_prep(self, qkv: torch.Tensor, n_kv: int, dim: int, unit: bool, q_scale: float, unit_eps: float,

@@ -34,6 +34,12 @@ DEFAULT_NAMES = {"q": "q", "k": "k", "v": "v", "q_conv": "q.conv", "k_conv": "k.
                  "o": "o"}
 
 
+def step_in_one_launch(env: BuildEnv, heads: int, kv_heads: int, dim: int, vdim: int, taps: int = 0, norm_part: int = 0) -> bool:
+    """Whether steps of one token per sequence run as one launch between the projections (`recurrence_step`)."""
+    return (env.lib is not None and not getattr(env, "generic_only", False)
+            and env.lib.recurrence_step_ok(heads, kv_heads, dim, vdim, taps, norm_part))
+
+
 class ChannelDelta(Part):
     graph_safe = True
     plan_safe = True
@@ -56,6 +62,7 @@ class ChannelDelta(Part):
         self.n_qk, self.n_v = self.kv_heads * self.dim, self.heads * self.vdim
         self.n_conv = 2 * self.n_qk + self.n_v
         self.conv = ShortConv(self.n_conv, self.taps, env, residual=False, act=ACT_SILU)
+        self.one_launch = step_in_one_launch(env, self.heads, self.kv_heads, self.dim, self.vdim, self.taps)
         self.cache_from = None
 
     # ------------------------------------------------------------------ tensors
@@ -111,6 +118,14 @@ class ChannelDelta(Part):
         proj = linear(lib, h, self.w_in, torch.float32)                       # [T, q | k | v | b]
         low = linear(lib, h, self.w_low, self.env.dtype)                      # [T, a1 h | g1 h]
         up = linear(lib, low, self.w_up, torch.float32)                       # [T, a | gate]
+        if self.one_launch and ctx.max_q_len == 1:
+            on = torch.empty((t, self.n_v), dtype=self.env.dtype, device=h.device)
+            lib.recurrence_step("delta", (proj, 0), (proj, self.n_qk), (proj, 2 * self.n_qk), self.heads, self.kv_heads, self.dim, self.vdim,
+                                (up, 0), False, 0, view.states["delta"], ctx, (up, self.heads * self.dim), 0, self.norm, self.eps, on,
+                                conv=(self.conv.weight, None, view.states.get("conv"), 0, self.n_qk, 2 * self.n_qk),
+                                a_bias=self.dt_bias, a_log=self.a_log, b=(proj, self.b_col), unit=True, q_scale=self.dim ** -0.5,
+                                unit_eps=self.unit_eps)
+            return linear(lib, on, self.w_o, torch.float32)
         qkv = self.conv.forward(proj, ctx, view.states.get("conv"), torch.float32)
         n_a = self.heads * self.dim
         beta = torch.empty((t, self.heads), dtype=torch.float32, device=h.device)
@@ -154,6 +169,7 @@ class HeadDelta(Part):
         self.n_qk, self.n_v = self.kv_heads * self.dim, self.heads * self.vdim
         self.n_conv = 2 * self.n_qk + self.n_v
         self.conv = ShortConv(self.n_conv, self.taps, env, residual=False, act=ACT_SILU)
+        self.one_launch = step_in_one_launch(env, self.heads, self.kv_heads, self.dim, self.vdim, self.taps)
         self.cache_from = None
 
     def tensor_specs(self) -> Dict[str, TensorSpec]:
@@ -195,6 +211,14 @@ class HeadDelta(Part):
     def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None) -> torch.Tensor:
         lib, t, c = self.env.lib, h.shape[0], self.cols
         proj = linear(lib, h, self.w_in, torch.float32)
+        if self.one_launch and ctx.max_q_len == 1:
+            on = torch.empty((t, self.n_v), dtype=self.env.dtype, device=h.device)
+            lib.recurrence_step("delta", (proj, 0), (proj, self.n_qk), (proj, 2 * self.n_qk), self.heads, self.kv_heads, self.dim, self.vdim,
+                                (proj, c["a"]), True, 0, view.states["delta"], ctx, (proj, c["g"]), 1, self.norm, self.eps, on,
+                                conv=(self.conv.weight, None, view.states.get("conv"), 0, self.n_qk, 2 * self.n_qk),
+                                a_bias=self.dt_bias, a_log=self.a_log, b=(proj, c["b"]), unit=True, q_scale=self.dim ** -0.5,
+                                unit_eps=self.unit_eps)
+            return linear(lib, on, self.w_o, torch.float32)
         qkv = self.conv.forward(proj, ctx, view.states.get("conv"), torch.float32)
         beta = torch.empty((t, self.heads), dtype=torch.float32, device=h.device)
         lib.recurrence_prep(qkv, self.kv_heads, self.dim, True, self.dim ** -0.5, self.unit_eps, proj, c["a"], self.heads, 0,
@@ -233,6 +257,7 @@ class DecayAttention(Part):
         self.names = dict(self.NAMES, **(params.get("names") or {}))
         self.hidden = env.hidden_size
         self.n_qk, self.n_v = self.heads * self.dim, self.heads * self.vdim
+        self.one_launch = step_in_one_launch(env, self.heads, self.heads, self.dim, self.vdim)
         self.cache_from = None
 
     def tensor_specs(self) -> Dict[str, TensorSpec]:
@@ -273,6 +298,12 @@ class DecayAttention(Part):
         proj = linear(lib, h, self.w_in, torch.float32)                       # [T, q | k | v | gate]
         low = linear(lib, h, self.w_a1, dt)
         z = linear(lib, low, self.w_a2, torch.float32)                        # [T, heads * dim]
+        if self.one_launch and ctx.max_q_len == 1:
+            on = torch.empty((t, self.n_v), dtype=dt, device=h.device)
+            lib.recurrence_step("plain", (proj, 0), (proj, self.n_qk), (proj, 2 * self.n_qk), self.heads, self.heads, self.dim, self.vdim,
+                                (z, 0), False, 1, view.states["decay"], ctx, (proj, c["g"]), 1, self.norm, self.eps, on,
+                                a_bias=self.a_bias, tau=self.tau, q_scale=self.dim ** -0.5)
+            return linear(lib, on, self.w_o, torch.float32)
         lib.recurrence_prep(proj, self.heads, self.dim, False, self.dim ** -0.5, 0.0, z, 0, self.n_qk, 1, self.a_bias, None,
                             self.tau, self.heads)
         o = torch.empty((t, self.n_v), dtype=torch.float32, device=h.device)
@@ -310,6 +341,7 @@ class TimeMix(Part):
         self.names = dict(self.NAMES, **(params.get("names") or {}))
         self.hidden = env.hidden_size
         self.n = self.heads * self.dim
+        self.one_launch = step_in_one_launch(env, self.heads, self.heads, self.dim, self.dim)
         self.cache_from = None
 
     def tensor_specs(self) -> Dict[str, TensorSpec]:
@@ -345,6 +377,11 @@ class TimeMix(Part):
         low = torch.empty((t, self.decay_rank), dtype=dt, device=h.device)
         lib.tanh_cast(linear(lib, mixes[4], self.w_1, torch.float32), low)
         decay = linear(lib, low, self.w_2, torch.float32)
+        if self.one_launch and ctx.max_q_len == 1:
+            on = torch.empty((t, self.n), dtype=dt, device=h.device)
+            lib.recurrence_step("bonus", (r, 0), (k, 0), (v, 0), self.heads, self.heads, self.dim, self.dim, (decay, 0), False, 2,
+                                view.states["time_mix"], ctx, (g, 0), 1, self.norm, self.eps, on, a_bias=self.w0, bonus=self.u)
+            return linear(lib, on, self.w_o, torch.float32)
         lib.decay_exp_exp(decay, self.w0, self.heads, self.dim)
         o = torch.empty((t, self.n), dtype=torch.float32, device=h.device)
         lib.time_mix_recurrence(r, k, v, decay, self.u, view.states["time_mix"], ctx, o, self.heads, self.dim, self.dim)

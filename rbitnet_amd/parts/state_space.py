@@ -26,6 +26,7 @@ import torch
 
 from ..errors import ConfigError
 from .base import BuildEnv, CacheRequest, Part, TensorSpec, register_mixer
+from .delta import step_in_one_launch
 from .linear import linear, linear_to_stream, pack_rows
 from .short_conv import ACT_SILU, ShortConv
 
@@ -57,6 +58,8 @@ class StateSpace(Part):
         self.channels = self.inner + 2 * self.groups * self.state
         self.dt_col = self.inner + self.channels
         self.conv = ShortConv(self.channels, int(params["conv"]), env, residual=False, act=ACT_SILU)
+        self.one_launch = step_in_one_launch(env, self.heads, self.groups, self.state, self.vdim, int(params["conv"]),
+                                             self.inner // self.norm_groups)
         self.cache_from = None
         self.in_chunks = bool(env.dtype == torch.bfloat16 and env.lib is not None and not getattr(env, "generic_only", False)
                               and env.lib.selective_chunks_ok(self.state, self.vdim))
@@ -98,6 +101,15 @@ class StateSpace(Part):
     def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None) -> torch.Tensor:
         lib, t = self.env.lib, h.shape[0]
         proj = linear(lib, h, self.w_in, torch.float32)                       # [T, z | x | k | q | t]
+        if self.one_launch and ctx.max_q_len == 1:
+            k_col = 2 * self.inner                                            # the convolution's channels are [x | k | q]
+            q_col = k_col + self.groups * self.state
+            yn = torch.empty((t, self.inner), dtype=self.env.dtype, device=h.device)
+            lib.recurrence_step("selective", (proj, q_col), (proj, k_col), (proj, self.inner), self.heads, self.groups, self.state, self.vdim,
+                                (proj, self.dt_col), True, 0, view.states["scan"], ctx, (proj, 0), 1, self.norm, self.eps, yn,
+                                conv=(self.conv.weight, self.conv_bias, view.states.get("conv"), q_col - self.inner, k_col - self.inner, 0),
+                                a_bias=self.dt_bias, a_log=self.a_log, d=self.d, norm_part=self.inner // self.norm_groups)
+            return linear_to_stream(lib, yn, self.w_o, None, next_norm)
         chunks = self.in_chunks and ctx.max_q_len >= CHUNKS_FROM
         xkq = self.conv.forward(proj, ctx, view.states.get("conv"), torch.bfloat16 if chunks else torch.float32, col0=self.inner,
                                 bias_out=self.conv_bias)

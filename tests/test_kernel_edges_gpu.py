@@ -3,7 +3,11 @@ largest of their ranges, each against the same operation in float64."""
 import pytest
 import torch
 
+from rbitnet_amd.cache import Cache
+from rbitnet_amd.config.spec import PartSpec
 from rbitnet_amd.csrc.lib import kernels
+from rbitnet_amd.engine.context import StepBatch, StepContext
+from rbitnet_amd.parts.base import BuildEnv, build_part
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -1186,3 +1190,49 @@ def test_single_token_attention_of_many_sequences(lib, heads, kv, count, sink):
         _within(kd[page, :, at], k[n - 1].double(), 2.0 ** -7 * k[n - 1].abs().double() + 1e-6)
     want = torch.cat(want)
     _within(out.view(want.shape), want, 2.0 ** -6 * float(max(x.abs().max() for x in vs)))
+
+
+# ---------------------------------------------------------------------------- single tokens through a recurrence, in one launch
+ONE_LAUNCH = [("channel_delta", dict(heads=h, kv_heads=k, dim=d, vdim=v, conv=c, eps=1e-5, decay_rank=16, gate_rank=16))
+              for h, k, d, v, c in ((1, 1, 64, 64, 4), (3, 3, 128, 64, 2), (4, 2, 128, 128, 3), (4, 1, 64, 128, 1))]
+ONE_LAUNCH += [("gated_delta", dict(heads=h, kv_heads=k, dim=d, vdim=v, conv=c, eps=1e-5))
+               for h, k, d, v, c in ((2, 2, 64, 192, 4), (4, 1, 128, 128, 4), (7, 1, 64, 64, 3), (6, 2, 128, 64, 1))]
+ONE_LAUNCH += [("decay_attention", dict(heads=h, dim=d, vdim=v, tau=8.0, decay_rank=16, eps=1e-5)) for h, d, v in ((2, 64, 128), (1, 128, 448), (3, 128, 64))]
+ONE_LAUNCH += [("time_mix", dict(heads=h, dim=d, decay_rank=16, eps=1e-5)) for h, d in ((1, 64), (3, 128))]
+ONE_LAUNCH += [("state_space", dict(heads=h, vdim=v, state=d, groups=g, conv=c, norm_groups=n, eps=1e-5))
+               for h, v, d, g, c, n in ((8, 64, 128, 1, 4, 1), (4, 64, 64, 2, 2, 4), (2, 128, 128, 2, 3, 4), (5, 64, 128, 1, 1, 5))]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind,params", ONE_LAUNCH)
+def test_single_tokens_through_a_recurrence_in_one_launch_beside_launches_of_their_own(lib, kind, params, dtype):
+    """The same mixer, states and tokens both ways, three steps of three sequences.  Both compute in float32 and differ in the
+    order of sums of at most 512 numbers: 1e-5 of the largest value bounds that; bfloat16 outputs may round the other way once."""
+    gen = torch.Generator().manual_seed(11)
+    hidden = 64
+    part = build_part("mixer", PartSpec(kind, params), BuildEnv(hidden_size=hidden, dtype=dtype, device=torch.device(DEV), lib=lib))
+    assert part.one_launch
+    part.load({n: (torch.randn(ts.shape, generator=gen) * (0.5 if len(ts.shape) < 2 or min(ts.shape) < 8 else ts.shape[-1] ** -0.5))
+               .to(torch.float32 if ts.role == "gain" else dtype).to(DEV) for n, ts in part.tensor_specs().items()})
+    caches = [Cache([part.cache_requests()], 3, 64 * 4, dtype, DEV) for _ in range(2)]
+    slots = [2, 0, 1]
+    for c in caches:
+        assert sorted(c.alloc_slot() for _ in range(3)) == [0, 1, 2]
+    for g, other in zip(caches[0].state_groups, caches[1].state_groups):
+        g.data.copy_(torch.randn(g.data.shape, generator=gen) * 0.3)
+        other.data.copy_(g.data)
+    for step in range(3):
+        h = torch.randn(3, hidden, generator=gen).to(dtype).to(DEV)
+        outs = []
+        for one, c in zip((True, False), caches):
+            part.one_launch = one
+            c.reserve(slots, [1, 1, 1])
+            ctx = StepContext.for_batch(DEV, StepBatch(slots, [c.length(s) for s in slots], [[1]] * 3, [0, 1, 2], c.block_tables(slots)),
+                                        n_compute_units=lib.n_compute_units)
+            outs.append(part.forward(h, ctx, c.view(0, ctx.block_tables)).float())
+            c.commit(slots, [1, 1, 1])
+        worst = lambda got, want: float((got - want).abs().max() / want.abs().max())
+        assert worst(*outs) < (1e-5 if dtype == torch.float32 else 1e-2)
+        for g, other in zip(caches[0].state_groups, caches[1].state_groups):
+            assert worst(g.data[:, slots], other.data[:, slots]) < 1e-5
+    assert not lib.recurrence_step_ok(2, 2, 96, 64) and not lib.recurrence_step_ok(2, 2, 64, 96) and not lib.recurrence_step_ok(9, 1, 64, 64)
