@@ -458,6 +458,10 @@ int rb_route_choose_bias(const float* z, long long z_stride, const float* bias, 
                          const float* correction, int32_t* sel, float* weight, int32_t* row_pair, int32_t* tile_expert, int max_rows,
                          int n_tokens, void* stream);
 // The same with every expert's run padded to a multiple of `unit` rows instead of 16, row_pair and tile_expert counting tiles of so many.
+int rb_route_linear_ok(int n_tokens, int n_rows, int n_outputs, int k);
+int rb_route_linear(const void* h, const void* w, int w_layout, int k, int n_rows, float* z, const float* bias, int n_outputs, int n_experts,
+                    int top, int score, const float* correction, int32_t* sel, float* weight, int32_t* row_pair, int32_t* tile_expert,
+                    int max_rows, int unit, int n_tokens, void* stream);      // with z = h W^T in front, up to 16 tokens
 int rb_route_choose_units(const float* z, long long z_stride, const float* bias, int n_outputs, int n_experts, int top, int score,
                           const float* correction, int32_t* sel, float* weight, int32_t* row_pair, int32_t* tile_expert, int max_rows,
                           int unit, int n_tokens, void* stream);

@@ -105,7 +105,7 @@ class KernelTimes:
         return "\n".join(lines)
 
 
-TIMED_OPS = ("routed_experts_tiled", "recurrence_step", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
+TIMED_OPS = ("routed_experts_tiled", "recurrence_step", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
              "route_top", "routed_experts", "pairs_sum", "embed_streams", "streams_layernorm", "streams_update", "xielu", "tanh_cap", "short_conv",
              "delta_prep", "delta_rule", "gated_rmsnorm", "latent_norm_store", "attention_sinks", "embed_gather", "add_rmsnorm", "rope_kv_write", "swiglu", "gemm_generic", "gemm_bf16", "gemm_bf16_terms",
              "gemm_bf16_few", "attention_generic", "attention_prefill_bf16", "attention_decode_bf16",
@@ -234,6 +234,8 @@ class Kernels:
             "rb_lightning_chunks_ok": [_I, _I],
             "rb_lightning_chunks": [_P, _P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
             "rb_gated_rmsnorm_rows": [_P, _P, _P, _L, _I, _F, _P, _I, _I, _I, _P],
+            "rb_route_linear_ok": [_I, _I, _I, _I],
+            "rb_route_linear": [_P, _P, _I, _I, _I, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
             "rb_route_choose_units": [_P, _L, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P],
             "rb_routed_experts_tiled": [_P, _I, _I, _P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _P, _P],
             "rb_route_choose_bias": [_P, _L, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P],
@@ -1063,6 +1065,33 @@ class Kernels:
         self._ok(self._lib.rb_route_choose_units(_ptr(z), z.shape[1], _ptr(bias), n_outputs, n_experts, top, int(score),
                                                  _ptr(correction), _ptr(sel), _ptr(weight), _ptr(row_pair), _ptr(tile_expert), max_rows,
                                                  int(unit), n, self._stream()))
+
+    def route_linear_ok(self, h: torch.Tensor, n_rows: int, n_outputs: int) -> bool:
+        return h.dtype == torch.bfloat16 and bool(self._lib.rb_route_linear_ok(h.shape[0], n_rows, n_outputs, h.shape[1]))
+
+    def route_linear(self, h: torch.Tensor, w: torch.Tensor, w_frag: bool, z: torch.Tensor, n_outputs: int, n_experts: int, top: int,
+                     score: int, correction: Optional[torch.Tensor], sel: torch.Tensor, weight: torch.Tensor, row_pair: torch.Tensor,
+                     tile_expert: torch.Tensor, bias: Optional[torch.Tensor] = None, unit: int = 16) -> None:
+        """`route_choose` of z = h w^T (written as well) with the product in the same launch, for a step of few tokens."""
+        n, k = h.shape
+        n_rows = w.shape[0]
+        _check(h, "h", torch.bfloat16)
+        _check(w, "w", torch.bfloat16, (n_rows, k))
+        _check(z, "z", torch.float32, (n, n_rows))
+        max_rows = row_pair.shape[0]
+        if max_rows < self.routed_rows(n, top, n_experts, unit) or max_rows % unit:
+            raise KernelError("route_linear: too little room for the sorted pairs")
+        if correction is not None:
+            _check(correction, "correction", torch.float32, (n_outputs,))
+        if bias is not None:
+            _check(bias, "bias", torch.float32, (n_outputs,))
+        _check(sel, "sel", torch.int32, (n * top,))
+        _check(weight, "weight", torch.float32, (n * top,))
+        _check(row_pair, "row_pair", torch.int32, (max_rows,))
+        _check(tile_expert, "tile_expert", torch.int32, (2 * (max_rows // unit),))
+        self._ok(self._lib.rb_route_linear(_ptr(h), _ptr(w), 1 if w_frag else 0, k, n_rows, _ptr(z), _ptr(bias), n_outputs, n_experts, top,
+                                           int(score), _ptr(correction), _ptr(sel), _ptr(weight), _ptr(row_pair), _ptr(tile_expert),
+                                           max_rows, int(unit), n, self._stream()))
 
     def routed_experts_tiled(self, h: torch.Tensor, top: int, row_pair: torch.Tensor, tile_expert: torch.Tensor, unit: int,
                              w_up: torch.Tensor, w_down: torch.Tensor, gated: bool, act: Optional[torch.Tensor], y: torch.Tensor,

@@ -177,19 +177,20 @@ __global__ __launch_bounds__(1024) void route_few_kernel(const float* __restrict
 // pair in its expert's run comes with the count; the runs' starts are a scan over the lanes instead of one thread's walk through
 // the experts.  The choices, the order of the sums and so the weights are those of route_token.  (4 tokens, 16 experts, 4 chosen, in a
 // graph: 7.6 us with route_few_kernel, 3.4 here; after a softmax 10.3 and 3.7.)
-__global__ __launch_bounds__(1024) void route_few_small_kernel(const float* __restrict__ z, size_t z_stride, int n_outputs, int n_experts,
-                                                               int top, int score, const float* __restrict__ bias,
-                                                               const float* __restrict__ correction, int32_t* __restrict__ sel,
-                                                               float* __restrict__ weight, int n_tokens, int32_t* __restrict__ row_pair,
-                                                               int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_pos,
-                                                               int max_rows, int unit) {
+// `logit` says what token t's output `lane` is; the same numbers lie at z for the case that route_token decides.
+template <typename L>
+__device__ __forceinline__ void route_few_small(L logit, const float* __restrict__ z, size_t z_stride, int n_outputs, int n_experts, int top,
+                                                int score, const float* __restrict__ bias, const float* __restrict__ correction,
+                                                int32_t* __restrict__ sel, float* __restrict__ weight, int n_tokens,
+                                                int32_t* __restrict__ row_pair, int32_t* __restrict__ tile_expert,
+                                                int32_t* __restrict__ tile_pos, int max_rows, int unit) {
   __shared__ int counts[RB_WAVE], start[RB_WAVE];
   __shared__ int pair_at[RT_FEW_TOKENS * RB_WAVE];       // a pair's expert and its place in the expert's run: place * 64 + expert
   const int lane = threadIdx.x & (RB_WAVE - 1);
   if (threadIdx.x < RB_WAVE) counts[threadIdx.x] = 0;
   __syncthreads();
   for (int t = threadIdx.x / RB_WAVE; t < n_tokens; t += blockDim.x / RB_WAVE) {
-    float v = lane < n_outputs ? z[(size_t)t * z_stride + lane] + (bias ? bias[lane] : 0.f) : -INFINITY;
+    float v = lane < n_outputs ? logit(t, lane) + (bias ? bias[lane] : 0.f) : -INFINITY;
     const float corr = score == 1 && correction && lane < n_outputs ? correction[lane] : 0.f;
     if (v != v) v = -INFINITY;
     float own = 0.f;
@@ -261,6 +262,92 @@ __global__ __launch_bounds__(1024) void route_few_small_kernel(const float* __re
   }
 }
 
+__global__ __launch_bounds__(1024) void route_few_small_kernel(const float* __restrict__ z, size_t z_stride, int n_outputs, int n_experts,
+                                                               int top, int score, const float* __restrict__ bias,
+                                                               const float* __restrict__ correction, int32_t* __restrict__ sel,
+                                                               float* __restrict__ weight, int n_tokens, int32_t* __restrict__ row_pair,
+                                                               int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_pos,
+                                                               int max_rows, int unit) {
+  route_few_small([&](int t, int o) { return z[(size_t)t * z_stride + o]; }, z, z_stride, n_outputs, n_experts, top, score, bias, correction, sel,
+                  weight, n_tokens, row_pair, tile_expert, tile_pos, max_rows, unit);
+}
+
+// The router's product in front of that, in the same launch, for up to 16 tokens and 64 rows of W: one workgroup of 8 waves, which deal
+// themselves the depth as a product of that few rows does (gemm_skinny.hip: stages of 128 in a row, the waves' sums added in their order), so
+// the logits are the same bits, and a step has one launch of one workgroup in place of two that wait for each other.  (4 tokens, 16
+// experts, 4 chosen, K = 2048, in a captured step: 3.4 + 4.4 us in two launches, 5.4 to 6.3 in one.)
+constexpr int RL_WAVES = 8, RL_TOKENS = 16, RL_TILES = 4;
+template <bool WF, int NT>                                   // NT: row tiles of 16, 1 or up to RL_TILES
+__global__ __launch_bounds__(RL_WAVES * RB_WAVE) void route_linear_kernel(
+    const bf16_t* __restrict__ h, const bf16_t* __restrict__ w, int k, int n_rows, int n_tokens, float* __restrict__ z, int n_outputs,
+    int n_experts, int top, int score, const float* __restrict__ bias, const float* __restrict__ correction, int32_t* __restrict__ sel,
+    float* __restrict__ weight, int32_t* __restrict__ row_pair, int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_pos, int max_rows,
+    int unit) {
+  __shared__ __attribute__((aligned(16))) float red[RL_WAVES - 1][NT][4 * RB_WAVE];
+  __shared__ __attribute__((aligned(16))) float logits[RL_TOKENS][16 * NT + 4];
+  constexpr int AHEAD = NT == 1 ? 4 : 1;                     // stages that are asked for together (K = 2048 is two a wave, 4096 four)
+  const int lane = threadIdx.x & (RB_WAVE - 1), wave = threadIdx.x / RB_WAVE, r = lane & 15, kq = lane >> 4;
+  const int n_tiles = NT == 1 ? 1 : (n_rows + 15) / 16;
+  const int total = k / 128, base = total / RL_WAVES, extra = total % RL_WAVES;
+  const int stages = base + (wave < extra ? 1 : 0), begin = 128 * (wave * base + (wave < extra ? wave : extra));
+  const bf16_t* xrow = h + (size_t)(r < n_tokens ? r : 0) * k + 8 * kq;
+  f32x4_t acc[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) acc[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  for (int st0 = 0; st0 < stages; st0 += AHEAD) {
+    Frag8 x[AHEAD][4], f[AHEAD][NT][4];
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) {
+      if (a > 0 && st0 + a >= stages) continue;
+      const int ks = begin + 128 * (st0 + a);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[a][j].u = load16(xrow + ks + 32 * j);
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        if (i >= n_tiles) continue;
+        const int row = 16 * i + r;                          // rows behind the last are row 0's, and nobody reads their sums
+        const bf16_t* at = WF ? w + (size_t)16 * i * k + (size_t)ks * 16 + 8 * lane : w + (size_t)(row < n_rows ? row : 0) * k + ks + 8 * kq;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f[a][i][j].u = load16(at + 32 * j * (WF ? 16 : 1));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) {
+      if (a > 0 && st0 + a >= stages) continue;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        if (i >= n_tiles) continue;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i] = mfma16(f[a][i][j], x[a][j], acc[i]);
+      }
+    }
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+      if (i < n_tiles) *reinterpret_cast<f32x4_t*>(&red[wave - 1][i][4 * lane]) = acc[i];
+  }
+  __syncthreads();
+  if (wave == 0) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      if (i >= n_tiles) continue;
+#pragma unroll
+      for (int v = 0; v < RL_WAVES - 1; ++v) acc[i] += *reinterpret_cast<const f32x4_t*>(&red[v][i][4 * lane]);
+      // (token r, rows 16 i + 4 kq .. + 3)
+      *reinterpret_cast<f32x4_t*>(&logits[r][16 * i + 4 * kq]) = acc[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (r < n_tokens && 16 * i + 4 * kq + e < n_rows) z[(size_t)r * n_rows + 16 * i + 4 * kq + e] = acc[i][e];
+    }
+    __threadfence_block();
+  }
+  __syncthreads();
+  route_few_small([&](int t, int o) { return logits[t][o]; }, z, (size_t)n_rows, n_outputs, n_experts, top, score, bias, correction, sel, weight,
+                  n_tokens, row_pair, tile_expert, tile_pos, max_rows, unit);
+}
+
 extern "C" int rb_route_choose(const float* z, long long z_stride, int n_outputs, int n_experts, int top, int score,
                                const float* correction, int32_t* sel, float* weight, int32_t* row_pair, int32_t* tile_expert,
                                int max_rows, int n_tokens, void* stream) {
@@ -309,6 +396,41 @@ extern "C" int rb_route_choose_units(const float* z, long long z_stride, const f
   (n_outputs <= RB_WAVE ? route_kernel<1> : route_kernel<RT_MAX_EXPERTS / RB_WAVE>)<<<(n_tokens + 3) / 4, 256, 0, s>>>(
       z, (size_t)z_stride, n_outputs, top, score, bias, correction, sel, weight, n_tokens);
   route_sort_kernel<<<1, 1024, 0, s>>>(sel, (int)pairs, n_experts, row_pair, tile_expert, tile_expert + max_rows / unit, max_rows, unit);
+  RB_LAUNCH_CHECK();
+  return 0;
+}
+
+// Whether the router's product and the choice go in one launch: bfloat16 rows of a depth that 8 waves share in stages of 128.
+extern "C" int rb_route_linear_ok(int n_tokens, int n_rows, int n_outputs, int k) {
+  return n_tokens >= 1 && n_tokens <= RL_TOKENS && n_tokens <= RT_FEW_TOKENS && n_rows >= n_outputs && n_rows <= 16 * RL_TILES &&
+         n_outputs <= RB_WAVE && k % 128 == 0 && k >= 128 * RL_WAVES;
+}
+
+// rb_route_choose_units of z = h W^T (float32 [T, n_rows], written as well), h bfloat16 [T, K], W bfloat16 [n_rows, K], as rows or
+// (w_layout 1: n_rows % 16 == 0) fragment-major; rows of W behind the router's outputs go to z and are no choice.
+extern "C" int rb_route_linear(const void* h, const void* w, int w_layout, int k, int n_rows, float* z, const float* bias, int n_outputs,
+                               int n_experts, int top, int score, const float* correction, int32_t* sel, float* weight, int32_t* row_pair,
+                               int32_t* tile_expert, int max_rows, int unit, int n_tokens, void* stream) {
+  RB_RECORDED(rb_route_linear(h, w, w_layout, k, n_rows, z, bias, n_outputs, n_experts, top, score, correction, sel, weight, row_pair,
+                              tile_expert, max_rows, unit, n_tokens, stream));
+  RB_REQUIRE(rb_route_linear_ok(n_tokens, n_rows, n_outputs, k) && (w_layout == 0 || (w_layout == 1 && n_rows % 16 == 0)),
+             "rb_route_linear: T=%d rows=%d outputs=%d K=%d layout %d are not for it", n_tokens, n_rows, n_outputs, k, w_layout);
+  RB_REQUIRE(unit > 0 && n_experts >= 0 && n_outputs >= n_experts && top > 0 && top <= n_outputs, "rb_route_linear: bad sizes");
+  RB_REQUIRE(score >= 0 && score <= 2 && (correction == nullptr || score == 1), "rb_route_linear: bad score %d or correction", score);
+  const long long pairs = (long long)n_tokens * top;
+  RB_REQUIRE(max_rows % unit == 0 && max_rows >= (pairs + unit - 1) / unit * unit + (long long)unit * n_experts,
+             "rb_route_linear: room for %d rows, %lld pairs of %d experts may need more", max_rows, pairs, n_experts);
+  RB_REQUIRE(((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(w)) & 15) == 0, "rb_route_linear: rows are not aligned to 16 bytes");
+#define RL_GO(WF, NT)                                                                                                                    \
+  route_linear_kernel<WF, NT><<<1, RL_WAVES * RB_WAVE, 0, (hipStream_t)stream>>>((const bf16_t*)h, (const bf16_t*)w, k, n_rows, n_tokens, z, \
+                                                                                 n_outputs, n_experts, top, score, bias, correction, sel,  \
+                                                                                 weight, row_pair, tile_expert, tile_expert + max_rows / unit, \
+                                                                                 max_rows, unit)
+  if (w_layout && n_rows <= 16) RL_GO(true, 1);
+  else if (w_layout) RL_GO(true, RL_TILES);
+  else if (n_rows <= 16) RL_GO(false, 1);
+  else RL_GO(false, RL_TILES);
+#undef RL_GO
   RB_LAUNCH_CHECK();
   return 0;
 }

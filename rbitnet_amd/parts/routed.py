@@ -5,7 +5,7 @@
     expert(x):  g = min(Wg x, limit),  u = clamp(Wu x, -limit, limit),  Wd (g * sigmoid(alpha * g) * (u + 1))
 
 Nothing of a step goes through the host: the router's product, one launch that chooses and sorts the (token, expert)
-pairs by expert in runs padded to tiles of 16 rows, one launch pair for all experts' products (on the matrix cores in
+pairs by expert in runs padded to tiles of 16 rows (the product in front of it in the same launch where tokens are few), one launch pair for all experts' products (on the matrix cores in
 bfloat16), and, with more than one expert a token, the sum of a token's pairs in a fixed order.  Steps of many tokens run on the
 dense product's tiles (runs padded to 64 to 256 rows), which multiply the sums of the way up by s_e instead of rounding s_e * h.  A token's
 result does not depend on what else the step holds but for which of these kernels its number of tokens asks for.
@@ -183,7 +183,6 @@ class RoutedExperts(Part):
     def forward(self, h: torch.Tensor, ctx=None, stream: Optional[torch.Tensor] = None, next_norm=None, pairs: bool = False):
         """-> float32 [T, E], or, with pairs=True (where `leaves_pairs` or `leaves_shared_pairs`), the `ExpertPairs` of the step."""
         lib, t, dev = self.env.lib, h.shape[0], h.device
-        z = linear(lib, h, self.w_router, torch.float32)
         n_pairs = t * self.top
         # (gated experts have a kernel for runs of a few dozen rows that is as fast; a row's place is a 32-bit byte offset in the tiles)
         tiled = self.tiled and t >= (TILED_FROM if self.w_gate is None else GATED_TILED_FROM * self.n_experts / self.top) \
@@ -194,9 +193,16 @@ class RoutedExperts(Part):
         weight = torch.empty(n_pairs, dtype=torch.float32, device=dev)
         row_pair = torch.empty(max_rows, dtype=torch.int32, device=dev)
         tile_expert = torch.empty(2 * (max_rows // unit), dtype=torch.int32, device=dev)      # experts, then positions in their runs
-        if self.plain and not tiled:
+        n_rows = self.w_router.shape[0]
+        if not tiled and lib.route_linear_ok(h, n_rows, self.n_outputs) and not getattr(self.env, "generic_only", False):
+            z = torch.empty((t, n_rows), dtype=torch.float32, device=dev)
+            lib.route_linear(h, self.w_router.data, self.w_router.frag, z, self.n_outputs, self.n_experts, self.top, self.score,
+                             self.correction, sel, weight, row_pair, tile_expert, bias=self.bias, unit=unit)
+        elif self.plain and not tiled:
+            z = linear(lib, h, self.w_router, torch.float32)
             lib.route_top(z, self.n_experts, self.top, sel, weight, row_pair, tile_expert)
         else:
+            z = linear(lib, h, self.w_router, torch.float32)
             lib.route_choose(z, self.n_outputs, self.n_experts, self.top, self.score, self.correction, sel, weight, row_pair,
                              tile_expert, bias=self.bias, unit=unit)
         out = torch.empty((n_pairs, self.hidden), dtype=torch.float32, device=dev)

@@ -1236,3 +1236,41 @@ def test_single_tokens_through_a_recurrence_in_one_launch_beside_launches_of_the
         for g, other in zip(caches[0].state_groups, caches[1].state_groups):
             assert worst(g.data[:, slots], other.data[:, slots]) < 1e-5
     assert not lib.recurrence_step_ok(2, 2, 96, 64) and not lib.recurrence_step_ok(2, 2, 64, 96) and not lib.recurrence_step_ok(9, 1, 64, 64)
+
+
+# ---------------------------------------------------------------------------- the router's product and the choice in one launch
+@pytest.mark.parametrize("n", [1, 3, 16])
+@pytest.mark.parametrize("rows,outputs,experts,top,k", [(16, 16, 16, 4, 2048), (17, 16, 16, 2, 1024), (8, 8, 8, 8, 1152), (64, 64, 64, 6, 1280),
+                                                       (33, 32, 30, 5, 8192), (48, 48, 48, 1, 3200)])
+def test_router_product_and_choice_in_one_launch_beside_two(lib, n, rows, outputs, experts, top, k):
+    """The same bits as a product and a choice of their own: the product's sums are taken in the same order.  A token whose logits
+    are not numbers, every score, rows of W behind the outputs, W as rows and fragment-major.  (Which row of an expert's run a pair
+    gets is the waves' to say: a run is compared as a set.)"""
+    gen = torch.Generator().manual_seed(rows + k)
+    h = torch.randn(n, k, generator=gen).to(torch.bfloat16)
+    if n > 2:
+        h[1] = float("nan")
+    h, w = h.to(DEV), (torch.randn(rows, k, generator=gen) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    bias = (torch.randn(outputs, generator=gen) * 0.1).to(DEV)
+    correction = (torch.randn(outputs, generator=gen) * 0.1).to(DEV)
+    assert lib.route_linear_ok(h, rows, outputs)
+    for frag in (False, True) if rows % 16 == 0 and k % 64 == 0 else (False,):
+        wd = w
+        if frag:
+            wd = torch.empty_like(w)
+            lib.place_rows(w, wd, frag=True)
+        for score, corr, b in ((0, None, None), (1, correction, bias), (1, None, None), (2, None, bias)):
+            room = lib.routed_rows(n, top, experts)
+            got, want = ([torch.zeros(n, rows, device=DEV), torch.empty(n * top, dtype=torch.int32, device=DEV), torch.empty(n * top, device=DEV),
+                          torch.empty(room, dtype=torch.int32, device=DEV), torch.zeros(2 * (room // 16), dtype=torch.int32, device=DEV)]
+                         for _ in range(2))
+            lib.route_linear(h, wd, frag, got[0], outputs, experts, top, score, corr, got[1], got[2], got[3], got[4], bias=b)
+            lib.gemm_bf16(h, wd, want[0], 0, w_frag=frag)
+            lib.route_choose(want[0], outputs, experts, top, score, corr, want[1], want[2], want[3], want[4], bias=b)
+            for i, (x, y) in enumerate(zip(got, want)):
+                if i != 3:
+                    assert torch.equal(x.nan_to_num(7.0) if x.is_floating_point() else x, y.nan_to_num(7.0) if y.is_floating_point() else y), i
+            runs = lambda pair, tile: {e: sorted(p for t in range(room // 16) if tile[t] == e for p in pair[16 * t:16 * t + 16]) for e in set(tile[:room // 16])}
+            assert runs(got[3].tolist(), got[4].tolist()) == runs(want[3].tolist(), want[4].tolist())
+    assert not lib.route_linear_ok(h, 65, 65) and not lib.route_linear_ok(h[:, :k - 64].contiguous(), rows, outputs)
+    assert not lib.route_linear_ok(h.float(), rows, outputs)
