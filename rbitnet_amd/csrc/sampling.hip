@@ -1,4 +1,4 @@
-// Next-token choice on the device, in two kernels so that a 128k vocabulary is read by
+// Next-token choice on the device, in two kernels (one where the vocabulary is one chunk) so that a 128k vocabulary is read by
 // many workgroups: (1) per chunk of the vocabulary, the maximum with its lowest index and
 // the sum of exponentials relative to it; (2) per sequence, the chunks combined and, for
 // temperature sampling, the chunk that holds the target walked element by element.
@@ -28,18 +28,71 @@ struct ChunkStat {
 
 __device__ __forceinline__ float clean(float v) { return v != v ? -INFINITY : v; }
 
+// The chosen chunk c in index order: `before` is the sum over the chunks in front of it.  A thread adds up a segment of its own, the segments'
+// running sums are a scan over the workgroup, and the first segment that reaches the target is walked by its thread, which holds its values.
+// (One thread walking 256 segments' sums: 5 us of a step's last 6.)
+__device__ __forceinline__ void sample_walk(const float* __restrict__ row, int vocab, int c, float temp, float zmax, double before, double target,
+                                            int32_t* __restrict__ token) {
+  __shared__ double s_wave[SAMPLE_THREADS / RB_WAVE];
+  __shared__ int s_first;
+  const int tid = threadIdx.x, lane = tid & (RB_WAVE - 1), wave = tid / RB_WAVE;
+  const int i0 = c * SAMPLE_CHUNK + tid * SAMPLE_SEG;
+  const int cend = (c + 1) * SAMPLE_CHUNK < vocab ? (c + 1) * SAMPLE_CHUNK : vocab;
+  float v[SAMPLE_SEG];
+#pragma unroll
+  for (int k = 0; k < SAMPLE_SEG; ++k) v[k] = i0 + k < cend ? row[i0 + k] : 0.f;
+  double part = 0.0;
+#pragma unroll
+  for (int k = 0; k < SAMPLE_SEG; ++k) {
+    v[k] = i0 + k < cend ? expf(clean(v[k]) / temp - zmax) : 0.f;
+    part += (double)v[k];
+  }
+  double upto = part;
+#pragma unroll
+  for (int o = 1; o < RB_WAVE; o <<= 1) {
+    const double below = __shfl_up(upto, o, RB_WAVE);
+    if (lane >= o) upto += below;
+  }
+  if (lane == RB_WAVE - 1) s_wave[wave] = upto;
+  if (tid == 0) s_first = SAMPLE_THREADS;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) before += s_wave[w];
+  if (i0 < cend && before + upto >= target) atomicMin(&s_first, tid);
+  __syncthreads();
+  if (s_first == SAMPLE_THREADS) {                           // rounding kept the running sum just below the target
+    if (tid == 0) *token = cend - 1;
+    return;
+  }
+  if (tid != s_first) return;
+  double run = before + (upto - part);
+  int pick = i0 + SAMPLE_SEG < cend ? i0 + SAMPLE_SEG - 1 : cend - 1;
+  bool reached = false;
+#pragma unroll
+  for (int k = 0; k < SAMPLE_SEG; ++k) {
+    run += (double)v[k];
+    if (!reached && i0 + k < cend && run >= target) {
+      pick = i0 + k;
+      reached = true;
+    }
+  }
+  *token = pick;
+}
+
+// WHOLE: the vocabulary is one chunk, and the choice is made here, in one launch.
+template <bool WHOLE>
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_chunk_kernel(const float* __restrict__ logits, int vocab,
-                                                                      const float* __restrict__ temperature,
-                                                                      ChunkStat* __restrict__ stats, int n_chunks) {
+                                                                      const float* __restrict__ temperature, const float* __restrict__ u,
+                                                                      ChunkStat* __restrict__ stats, int n_chunks,
+                                                                      int32_t* __restrict__ tokens) {
   __shared__ float s_val[SAMPLE_THREADS / RB_WAVE];
   __shared__ int s_idx[SAMPLE_THREADS / RB_WAVE];
   __shared__ double s_sum[SAMPLE_THREADS / RB_WAVE];
-  __shared__ float s_max;
   const int c = blockIdx.x, r = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & (RB_WAVE - 1), wave = tid / RB_WAVE;
   const float* row = logits + (size_t)r * vocab;
   const int i0 = c * SAMPLE_CHUNK;
   const int i1 = i0 + SAMPLE_CHUNK < vocab ? i0 + SAMPLE_CHUNK : vocab;
+  const float temp = temperature ? temperature[r] : 0.f;
   float v[SAMPLE_SEG];
   float best = -INFINITY;
   int best_i = 0x7fffffff;
@@ -66,126 +119,126 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_chunk_kernel(const floa
     s_idx[wave] = best_i;
   }
   __syncthreads();
-  if (tid == 0) {
-    float b = s_val[0];
-    int bi = s_idx[0];
-    for (int w = 1; w < SAMPLE_THREADS / RB_WAVE; ++w)
-      if (s_val[w] > b || (s_val[w] == b && s_idx[w] < bi)) {
-        b = s_val[w];
-        bi = s_idx[w];
-      }
-    s_max = b;
-    stats[(size_t)r * n_chunks + c].max = b;
-    stats[(size_t)r * n_chunks + c].arg = bi;
-  }
-  __syncthreads();
-  const float temp = temperature ? temperature[r] : 0.f;
-  double sum = 0.0;
-  if (temp > 0.f && s_max > -INFINITY) {
-    const float zmax = s_max / temp;
 #pragma unroll
-    for (int k = 0; k < SAMPLE_SEG; ++k) sum += (double)expf(v[k] / temp - zmax);      // exp(-inf) = 0 beyond the end
+  for (int w = 0; w < SAMPLE_THREADS / RB_WAVE; ++w)         // every thread: the chunk's maximum and its lowest index
+    if (s_val[w] > best || (s_val[w] == best && s_idx[w] < best_i)) {
+      best = s_val[w];
+      best_i = s_idx[w];
+    }
+  const bool sums = temp > 0.f && best > -INFINITY;
+  const float zmax = sums ? best / temp : 0.f;
+  double total = 0.0;
+  if (sums) {
 #pragma unroll
-    for (int o = RB_WAVE / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, RB_WAVE);
+    for (int k = 0; k < SAMPLE_SEG; ++k) total += (double)expf(v[k] / temp - zmax);      // exp(-inf) = 0 beyond the end
+#pragma unroll
+    for (int o = RB_WAVE / 2; o > 0; o >>= 1) total += __shfl_xor(total, o, RB_WAVE);
+    if (lane == 0) s_sum[wave] = total;
+    __syncthreads();
+    total = 0.0;
+    for (int w = 0; w < SAMPLE_THREADS / RB_WAVE; ++w) total += s_sum[w];
   }
-  if (lane == 0) s_sum[wave] = sum;
-  __syncthreads();
-  if (tid == 0) {
-    double t = 0.0;
-    for (int w = 0; w < SAMPLE_THREADS / RB_WAVE; ++w) t += s_sum[w];
-    stats[(size_t)r * n_chunks + c].sum = t;
+  if (!WHOLE) {
+    if (tid == 0) stats[(size_t)r * n_chunks + c] = ChunkStat{best, best_i, total};
+    return;
   }
+  if (!sums) {
+    if (tid == 0) tokens[r] = best_i == 0x7fffffff ? 0 : best_i;      // every logit NaN or -inf: index 0
+    return;
+  }
+  sample_walk(row, vocab, 0, temp, zmax, 0.0, (double)u[r] * total, tokens + r);
 }
 
+// The chunks of a row combined by one wave, a lane a run of neighbouring chunks: their maximum; for temperature sampling, the running sums in
+// index order as a scan over the lanes, and the chunk in which they reach the target.  (A thread that walks the chunks alone has a trip to
+// memory for each: 4 rows of 128,256 logits 5.1 us, and 12 to 15 for both launches in a captured step with the cap on the logits in front of them; now 6.6.)
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(const float* __restrict__ logits, int vocab,
                                                                      const float* __restrict__ temperature,
                                                                      const float* __restrict__ u,
                                                                      const ChunkStat* __restrict__ stats, int n_chunks,
                                                                      int32_t* __restrict__ tokens) {
-  __shared__ double s_part[SAMPLE_THREADS];
   __shared__ int s_chunk;
-  __shared__ double s_before, s_target, s_factor;
+  __shared__ double s_before, s_target;
   __shared__ float s_gmax;
   const int r = blockIdx.x, tid = threadIdx.x;
-  const ChunkStat* st = stats + (size_t)r * n_chunks;
   const float temp = temperature ? temperature[r] : 0.f;
-  if (tid == 0) {
+  if (tid < RB_WAVE) {
+    const ChunkStat* st = stats + (size_t)r * n_chunks;
+    const int each = (n_chunks + RB_WAVE - 1) / RB_WAVE, c0 = tid * each, c1 = c0 + each < n_chunks ? c0 + each : n_chunks;
     float gmax = -INFINITY;
     int garg = 0x7fffffff;
-    for (int c = 0; c < n_chunks; ++c)
+    for (int c = c0; c < c1; ++c)
       if (st[c].max > gmax || (st[c].max == gmax && st[c].arg < garg)) {
         gmax = st[c].max;
         garg = st[c].arg;
       }
-    s_gmax = gmax;
-    s_chunk = -1;
-    if (!(temp > 0.f) || gmax == -INFINITY) {
-      tokens[r] = garg == 0x7fffffff ? 0 : garg;          // every logit NaN or -inf: index 0
-    } else {
-      double total = 0.0;
-      for (int c = 0; c < n_chunks; ++c)
-        if (st[c].max > -INFINITY) total += st[c].sum * exp((double)(st[c].max / temp) - (double)(gmax / temp));
-      const double target = (double)u[r] * total;
-      double run = 0.0;
-      int pick = -1;
-      for (int c = 0; c < n_chunks; ++c) {
-        if (!(st[c].max > -INFINITY)) continue;
-        const double f = exp((double)(st[c].max / temp) - (double)(gmax / temp));
-        if (run + st[c].sum * f >= target) {
-          pick = c;
-          s_factor = f;
-          break;
-        }
-        run += st[c].sum * f;
-      }
-      if (pick < 0) {
-        tokens[r] = vocab - 1;
-      } else {
-        s_chunk = pick;
-        s_before = run;
-        s_target = target;
+#pragma unroll
+    for (int o = RB_WAVE / 2; o > 0; o >>= 1) {
+      const float ov = __shfl_xor(gmax, o, RB_WAVE);
+      const int oi = __shfl_xor(garg, o, RB_WAVE);
+      if (ov > gmax || (ov == gmax && oi < garg)) {
+        gmax = ov;
+        garg = oi;
       }
     }
+    int pick = -1;
+    double before = 0.0, target = 0.0;
+    if (!(temp > 0.f) || gmax == -INFINITY) {
+      if (tid == 0) tokens[r] = garg == 0x7fffffff ? 0 : garg;          // every logit NaN or -inf: index 0
+    } else {
+      const double top = (double)(gmax / temp);
+      auto share = [&](const ChunkStat& s) { return s.max > -INFINITY ? s.sum * exp((double)(s.max / temp) - top) : 0.0; };
+      double mine = 0.0;
+      bool any = false;
+      for (int c = c0; c < c1; ++c) {
+        mine += share(st[c]);
+        any = any || st[c].max > -INFINITY;
+      }
+      double upto = mine;
+#pragma unroll
+      for (int o = 1; o < RB_WAVE; o <<= 1) {
+        const double below = __shfl_up(upto, o, RB_WAVE);
+        if (tid >= o) upto += below;
+      }
+      target = (double)u[r] * __shfl(upto, RB_WAVE - 1, RB_WAVE);
+      const unsigned long long reach = __ballot(any && upto >= target);
+      const int owner = reach ? __ffsll((long long)reach) - 1 : -1;
+      if (tid == owner) {
+        before = upto - mine;
+        double run = before;
+        for (int c = c0; c < c1; ++c) {
+          if (!(st[c].max > -INFINITY)) continue;
+          const double sum = share(st[c]);
+          pick = c;                                          // (the last of them, should rounding leave the sum below the target)
+          before = run;
+          if (run + sum >= target) break;
+          run += sum;
+        }
+        s_chunk = pick;
+        s_before = before;
+        s_target = target;
+        s_gmax = gmax;
+      }
+      if (owner < 0 && tid == 0) tokens[r] = vocab - 1;
+      if (owner >= 0) pick = 0;
+    }
+    if (pick < 0 && tid == 0) s_chunk = -1;
   }
   __syncthreads();
   const int c = s_chunk;
   if (c < 0) return;
-  // ---- walk the chosen chunk in index order: each thread a contiguous segment
-  const float* row = logits + (size_t)r * vocab;
-  const float zmax = s_gmax / temp;
-  const int i0 = c * SAMPLE_CHUNK + tid * SAMPLE_SEG;
-  const int cend = (c + 1) * SAMPLE_CHUNK < vocab ? (c + 1) * SAMPLE_CHUNK : vocab;
-  double part = 0.0;
-  for (int i = i0; i < i0 + SAMPLE_SEG && i < cend; ++i) part += (double)expf(clean(row[i]) / temp - zmax);
-  s_part[tid] = part;
-  __syncthreads();
-  if (tid == 0) {
-    double run = s_before;
-    const double target = s_target;
-    int owner = -1;
-    for (int w = 0; w < SAMPLE_THREADS; ++w) {
-      if (c * SAMPLE_CHUNK + w * SAMPLE_SEG >= cend) break;
-      if (run + s_part[w] >= target) {
-        owner = w;
-        break;
-      }
-      run += s_part[w];
-    }
-    int pick = cend - 1;            // rounding kept the running sum just below the target
-    if (owner >= 0) {
-      const int j0 = c * SAMPLE_CHUNK + owner * SAMPLE_SEG;
-      const int j1 = j0 + SAMPLE_SEG < cend ? j0 + SAMPLE_SEG : cend;
-      pick = j1 - 1;
-      for (int i = j0; i < j1; ++i) {
-        run += (double)expf(clean(row[i]) / temp - zmax);
-        if (run >= target) {
-          pick = i;
-          break;
-        }
-      }
-    }
-    tokens[r] = pick;
+  // sums inside the chunk are relative to the row's maximum, as the target is
+  sample_walk(logits + (size_t)r * vocab, vocab, c, temp, s_gmax / temp, s_before, s_target, tokens + r);
+}
+
+static void launch_sample(const float* logits, int n_rows, int vocab, const float* temperature, const float* u, ChunkStat* stats, int n_chunks,
+                          int32_t* tokens, hipStream_t s) {
+  if (n_chunks == 1) {
+    sample_chunk_kernel<true><<<dim3(1, n_rows), SAMPLE_THREADS, 0, s>>>(logits, vocab, temperature, u, stats, 1, tokens);
+    return;
   }
+  sample_chunk_kernel<false><<<dim3(n_chunks, n_rows), SAMPLE_THREADS, 0, s>>>(logits, vocab, temperature, u, stats, n_chunks, tokens);
+  sample_pick_kernel<<<n_rows, SAMPLE_THREADS, 0, s>>>(logits, vocab, temperature, u, stats, n_chunks, tokens);
 }
 
 extern "C" int rb_sample_workspace_bytes(int n_rows, int vocab) {
@@ -205,8 +258,7 @@ extern "C" int rb_sample(const float* logits, int n_rows, int vocab, const float
              n_rows);
   hipStream_t s = (hipStream_t)stream;
   ChunkStat* stats = (ChunkStat*)workspace;
-  sample_chunk_kernel<<<dim3(n_chunks, n_rows), SAMPLE_THREADS, 0, s>>>(logits, vocab, temperature, stats, n_chunks);
-  sample_pick_kernel<<<n_rows, SAMPLE_THREADS, 0, s>>>(logits, vocab, temperature, u, stats, n_chunks, tokens);
+  launch_sample(logits, n_rows, vocab, temperature, u, stats, n_chunks, tokens, s);
   RB_LAUNCH_CHECK();
   return 0;
 }
@@ -264,9 +316,7 @@ extern "C" int rb_sample_static(const float* logits, int n_rows, int vocab, cons
   if (int rc = scratch_of_current_device(&ptr)) return rc;
   hipStream_t s = (hipStream_t)stream;
   ChunkStat* stats = (ChunkStat*)ptr;
-  sample_chunk_kernel<<<dim3((int)n_chunks, n_rows), SAMPLE_THREADS, 0, s>>>(logits, vocab, temperature, stats,
-                                                                             (int)n_chunks);
-  sample_pick_kernel<<<n_rows, SAMPLE_THREADS, 0, s>>>(logits, vocab, temperature, u, stats, (int)n_chunks, tokens);
+  launch_sample(logits, n_rows, vocab, temperature, u, stats, (int)n_chunks, tokens, s);
   RB_LAUNCH_CHECK();
   return 0;
 }
