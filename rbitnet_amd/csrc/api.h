@@ -234,6 +234,16 @@ int rb_gated_rmsnorm_act(const float* o, const float* weight, const float* gate,
 int rb_short_conv_biases(const float* x, long long x_stride, const float* bias, const float* bias_out, const float* w, int taps, float* state,
                          const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* cu_seqlens, const int32_t* slots, void* out,
                          long long out_stride, int out_dtype, int residual, int act, int n_tokens, int n_seqs, int channels, void* stream);
+// Up to RB_GROUP_PRODUCTS products C_i = X_i W_i^T of 1 to 16 tokens (bfloat16 X_i [m, k] and W_i [n, k], all of one layout as in
+// rb_gemm_bf16) in one launch; end 0: C float32, 1: C bfloat16, 2: C = bfloat16(tanh(sum)).  Rows at 16 bytes.
+#define RB_GROUP_PRODUCTS 6
+struct RbGroupProduct {
+  const void *x, *w;
+  void* c;
+  int n, end;
+};
+int rb_gemm_bf16_group_ok(int m, int k);
+int rb_gemm_bf16_group(const struct RbGroupProduct* products, int count, int w_layout, int m, int k, void* stream);
 // A step of ONE token per sequence (token t is of slot slots[t]) through such a layer in one launch: convolution and silu (conv_w null:
 // none; the state moves on), unit vectors or the query's scale, decays, the recurrence, the read-out norm and its gate.
 //   mode 0: the delta rule (beta = sigmoid(b)); 1: the plain rule; 2: read before the write, with a bonus [H, dim]; 3: the selective scan,

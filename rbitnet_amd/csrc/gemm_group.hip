@@ -1,0 +1,120 @@
+// Several products of a few tokens in one launch: C_i = X_i W_i^T, bfloat16 operands of one depth K, each with inputs, a matrix, outputs
+// and an end of its own.  A layer's projections that do not wait for each other (the inputs of time mixing and what its decays are made
+// from; a large product and the low-rank one beside it) were launches one after the other, and a product of 16 to 1,024 rows with 4 tokens at
+// K = 2048 costs 3.8 to 5 us whatever it reads (4 MB: 0.6 us of memory's time): its boundary, two trips to memory, the waves' sums.
+// The same kernel as gemm_skinny_kernel with one row tile a wave: K / 128 stages dealt to the waves in a row, sums through LDS in their order.
+// Measured in captured steps of 4 tokens: 6,160 and 256 rows 6.8 + 4.3 us in two launches, 6.6 in one; five of 1,024 and 64 rows and the tanh behind the
+// last, 19 + 10 us in six launches, 4.2 in one.
+#include "api.h"
+#include "gemm_internal.h"
+
+namespace {
+
+constexpr int MOST = RB_GROUP_PRODUCTS;
+enum { END_F32 = 0, END_BF16 = 1, END_TANH = 2 };          // tanh: bfloat16(tanh(sum))
+struct Group {
+  RbGroupProduct p[MOST];
+  int end[MOST];                                            // row tiles up to and with this product
+  int count;
+};
+
+template <bool WF>
+__global__ __launch_bounds__(512) void gemm_group_kernel(const Group g, int m, int k) {
+  extern __shared__ __attribute__((aligned(16))) float red[];      // [waves - 1][64] pieces of four sums
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6, r = lane & 15, kq = lane >> 4;
+  int i = 0;
+  while (i + 1 < g.count && (int)blockIdx.x >= g.end[i]) ++i;
+  const RbGroupProduct p = g.p[i];
+  const int n0 = 16 * ((int)blockIdx.x - (i > 0 ? g.end[i - 1] : 0));
+  const bf16_t* w = (const bf16_t*)p.w;
+  const bf16_t* wrow = WF ? w + (size_t)n0 * k + 8 * lane : w + (size_t)(n0 + r < p.n ? n0 + r : 0) * k + 8 * kq;
+  const bf16_t* xrow = (const bf16_t*)p.x + (size_t)(r < m ? r : 0) * k + 8 * kq;
+  const int total = k / 128, base = total / n_waves, extra = total % n_waves;
+  const int stages = base + (wave < extra ? 1 : 0), begin = 128 * (wave * base + (wave < extra ? wave : extra));
+  f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  Frag8 a[4], b[4];
+  auto load_stage = [&](int st) {
+    const int ks = begin + 128 * st;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j].u = WF ? load16_stream(wrow + (size_t)(ks + 32 * j) * 16) : load16(wrow + ks + 32 * j);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b[j].u = load16(xrow + ks + 32 * j);
+  };
+  auto multiply_stage = [&]() {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = mfma16(a[j], b[j], acc);
+  };
+  load_stage(0);                                            // (the host launches no more waves than stages)
+  for (int st = 1; st < stages; ++st) {
+    multiply_stage();
+    load_stage(st);
+  }
+  multiply_stage();
+  if (n_waves > 1) {
+    if (wave > 0) *reinterpret_cast<f32x4_t*>(red + (wave - 1) * 256 + 4 * lane) = acc;
+    __syncthreads();
+    if (wave > 0) return;
+    for (int v = 0; v < n_waves - 1; ++v) acc += *reinterpret_cast<const f32x4_t*>(red + v * 256 + 4 * lane);
+  }
+  if (r >= m) return;
+  const int nn = n0 + 4 * kq;                               // token r, rows nn .. + 3
+  if (p.end == END_TANH) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = tanhf(acc[e]);
+  }
+  if (p.end == END_F32) {
+    float* c = (float*)p.c + (size_t)r * p.n + nn;
+    if (p.n % 4 == 0) {
+      if (nn < p.n) *reinterpret_cast<f32x4_t*>(c) = acc;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (nn + e < p.n) c[e] = acc[e];
+    }
+  } else {
+    bf16_t* c = (bf16_t*)p.c + (size_t)r * p.n + nn;
+    if (p.n % 4 == 0) {
+      if (nn < p.n) *reinterpret_cast<uint2*>(c) = make_uint2(pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (nn + e < p.n) c[e] = f32_to_bf16(acc[e]);
+    }
+  }
+}
+
+}  // namespace
+
+// Whether m tokens of depth k go in one launch (more tokens have kernels that deal a product's tiles out better).
+extern "C" int rb_gemm_bf16_group_ok(int m, int k) { return m >= 1 && m <= 16 && k >= 128 && k % 128 == 0; }
+
+extern "C" int rb_gemm_bf16_group(const RbGroupProduct* products, int count, int w_layout, int m, int k, void* stream) {
+  RB_REQUIRE(products != nullptr && count >= 1 && count <= MOST, "rb_gemm_bf16_group: %d products (1 to %d)", count, MOST);
+  Group g;
+  g.count = count;
+  for (int i = 0; i < count; ++i) g.p[i] = products[i];
+  RB_RECORDED(rb_gemm_bf16_group(g.p, count, w_layout, m, k, stream));
+  RB_REQUIRE(m == 0 || rb_gemm_bf16_group_ok(m, k), "rb_gemm_bf16_group: M=%d K=%d is not for it", m, k);
+  RB_REQUIRE(w_layout == 0 || w_layout == 1, "rb_gemm_bf16_group: W layout %d", w_layout);
+  long long tiles = 0;
+  for (int i = 0; i < count; ++i) {
+    const RbGroupProduct& p = g.p[i];
+    RB_REQUIRE(p.x && p.w && p.c && p.n > 0 && p.end >= END_F32 && p.end <= END_TANH && (w_layout == 0 || p.n % 16 == 0),
+               "rb_gemm_bf16_group: product %d of %d rows, layout %d, end %d", i, p.n, w_layout, p.end);
+    RB_REQUIRE(((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.w) | reinterpret_cast<uintptr_t>(p.c)) & 15) == 0,
+               "rb_gemm_bf16_group: product %d is not aligned to 16 bytes", i);
+    tiles += (p.n + 15) / 16;
+    RB_REQUIRE(tiles <= 1 << 24, "rb_gemm_bf16_group: too many rows");
+    g.end[i] = (int)tiles;
+  }
+  if (m == 0) return 0;
+  // as for a product alone (gemm_skinny.hip): 8 waves where a compute unit has about one workgroup, 4 where it has more (4 tokens, K = 2048,
+  // 256 tiles 5.7 us with 8 and 6.0 with 4; 385 tiles 8.0 and 7.3), and 8 where K is long
+  int waves = k >= 8192 || 4 * tiles <= 5LL * rb_compute_units() ? 8 : 4;
+  if (waves > k / 128) waves = k / 128;
+  const size_t lds = (size_t)(waves - 1) * 256 * sizeof(float);
+  if (w_layout) gemm_group_kernel<true><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
+  else gemm_group_kernel<false><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
+  RB_LAUNCH_CHECK();
+  return 0;
+}

@@ -105,7 +105,7 @@ class KernelTimes:
         return "\n".join(lines)
 
 
-TIMED_OPS = ("routed_experts_tiled", "recurrence_step", "recurrence_chunks", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
+TIMED_OPS = ("routed_experts_tiled", "recurrence_step", "recurrence_chunks", "gemm_bf16_group", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
              "route_top", "routed_experts", "pairs_sum", "embed_streams", "streams_layernorm", "streams_update", "xielu", "tanh_cap", "short_conv",
              "delta_prep", "delta_rule", "gated_rmsnorm", "latent_norm_store", "attention_sinks", "embed_gather", "add_rmsnorm", "rope_kv_write", "swiglu", "gemm_generic", "gemm_bf16", "gemm_bf16_terms",
              "gemm_bf16_few", "attention_generic", "attention_prefill_bf16", "attention_decode_bf16",
@@ -127,6 +127,13 @@ class RecurrenceStep(ctypes.Structure):
 
 
 RECURRENCE_WORKSPACE = 256 << 20         # bytes of a chunked recurrence's operands at a time
+class GroupProduct(ctypes.Structure):
+    """RbGroupProduct of csrc/api.h."""
+    _fields_ = [("x", _P), ("w", _P), ("c", _P), ("n", _I), ("end", _I)]
+
+
+GROUP_PRODUCTS = 6                       # RB_GROUP_PRODUCTS
+GROUP_ENDS = {"float32": 0, "bfloat16": 1, "tanh": 2}
 STEP_MODES = {"delta": 0, "plain": 1, "bonus": 2, "selective": 3}
 
 
@@ -182,6 +189,8 @@ class Kernels:
             "rb_embed_streams_layout": [_P, _I, _I, _P, _F, _P, _P, _P, _I, _L, _I, _I, _P],
             "rb_streams_rmsnorm": [_P, _I, _L, _P, _P, _P, _I, _L, _L, _P, _P, _I, _L, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_short_conv_biases": [_P, _L, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
+            "rb_gemm_bf16_group_ok": [_I, _I],
+            "rb_gemm_bf16_group": [ctypes.POINTER(GroupProduct), _I, _I, _I, _I, _P],
             "rb_recurrence_step_ok": [_I, _I, _I, _I, _I, _I],
             "rb_recurrence_step": [ctypes.POINTER(RecurrenceStep), _P],
             "rb_recurrence_chunks_ok": [_I, _I, _I, _I],
@@ -378,6 +387,23 @@ class Kernels:
                 raise KernelError("gemm_bf16: an activation goes with epilogue 0, a gate's numbers with epilogue 1")
         self._ok(self._lib.rb_gemm_bf16_act(_ptr(a), _ptr(w), int(bool(w_frag)), _ptr(c), dtype_code(c.dtype), int(epilogue),
                                             _ptr(act), m, n, k, _ptr(workspace), self._stream()))
+
+    def gemm_bf16_group(self, products, w_frag: bool) -> None:
+        """products: up to GROUP_PRODUCTS of (x [M, K], w [N, K], c [M, N], end), all of one M, K and layout of w; end: "float32",
+        "bfloat16" (the type of c), or "tanh": c = bfloat16(tanh(x w^T))."""
+        m, k = products[0][0].shape
+        if len(products) > GROUP_PRODUCTS:
+            raise KernelError(f"gemm_bf16_group: at most {GROUP_PRODUCTS} products")
+        args = (GroupProduct * len(products))()
+        for a, (x, w, c, end) in zip(args, products):
+            _check(x, "x", torch.bfloat16, (m, k))
+            _check(w, "w", torch.bfloat16, (w.shape[0], k))
+            _check(c, "c", torch.float32 if end == "float32" else torch.bfloat16, (m, w.shape[0]))
+            a.x, a.w, a.c, a.n, a.end = _ptr(x), _ptr(w), _ptr(c), w.shape[0], GROUP_ENDS[end]
+        self._ok(self._lib.rb_gemm_bf16_group(args, len(products), int(bool(w_frag)), m, k, self._stream()))
+
+    def gemm_bf16_group_ok(self, m: int, k: int) -> bool:
+        return bool(self._lib.rb_gemm_bf16_group_ok(int(m), int(k)))
 
     def gemm_bf16_terms_count(self, m: int, n: int, k: int) -> int:
         return int(self._lib.rb_gemm_bf16_terms_count(int(m), int(n), int(k)))

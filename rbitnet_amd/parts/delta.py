@@ -26,7 +26,7 @@ import torch
 
 from ..errors import ConfigError
 from .base import BuildEnv, CacheRequest, Part, TensorSpec, register_mixer
-from .linear import linear, linear_to_stream, pack_rows
+from .linear import linear, linear_group, linear_to_stream, pack_rows
 from .short_conv import ACT_SILU, ShortConv
 
 DEFAULT_NAMES = {"q": "q", "k": "k", "v": "v", "q_conv": "q.conv", "k_conv": "k.conv", "v_conv": "v.conv", "b": "b",
@@ -121,8 +121,8 @@ class ChannelDelta(Part):
     # ------------------------------------------------------------------ forward
     def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None) -> torch.Tensor:
         lib, t = self.env.lib, h.shape[0]
-        proj = linear(lib, h, self.w_in, torch.float32)                       # [T, q | k | v | b]
-        low = linear(lib, h, self.w_low, self.env.dtype)                      # [T, a1 h | g1 h]
+        # [T, q | k | v | b] and [T, a1 h | g1 h]
+        proj, low = linear_group(lib, [(h, self.w_in, "float32"), (h, self.w_low, "same")], self.env.dtype)
         up = linear(lib, low, self.w_up, torch.float32)                       # [T, a | gate]
         if self.one_launch and ctx.max_q_len == 1:
             on = torch.empty((t, self.n_v), dtype=self.env.dtype, device=h.device)
@@ -313,8 +313,7 @@ class DecayAttention(Part):
 
     def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None) -> torch.Tensor:
         lib, t, c, dt = self.env.lib, h.shape[0], self.cols, self.env.dtype
-        proj = linear(lib, h, self.w_in, torch.float32)                       # [T, q | k | v | gate]
-        low = linear(lib, h, self.w_a1, dt)
+        proj, low = linear_group(lib, [(h, self.w_in, "float32"), (h, self.w_a1, "same")], dt)      # [T, q | k | v | gate]
         z = linear(lib, low, self.w_a2, torch.float32)                        # [T, heads * dim]
         if self.one_launch and ctx.max_q_len == 1:
             on = torch.empty((t, self.n_v), dtype=dt, device=h.device)
@@ -396,9 +395,7 @@ class TimeMix(Part):
         lib, t, dt = self.env.lib, h.shape[0], self.env.dtype
         mixes = torch.empty((5, t, self.hidden), dtype=dt, device=h.device)
         lib.shift_mix(h, view.states["time_shift"], self.mu, ctx, mixes)
-        r, k, v, g = (linear(lib, mixes[i], self.w_in[i], torch.float32) for i in range(4))
-        low = torch.empty((t, self.decay_rank), dtype=dt, device=h.device)
-        lib.tanh_cast(linear(lib, mixes[4], self.w_1, torch.float32), low)
+        r, k, v, g, low = linear_group(lib, [(mixes[i], self.w_in[i], "float32") for i in range(4)] + [(mixes[4], self.w_1, "tanh")], dt)
         decay = linear(lib, low, self.w_2, torch.float32)
         if self.one_launch and ctx.max_q_len == 1:
             on = torch.empty((t, self.n), dtype=dt, device=h.device)

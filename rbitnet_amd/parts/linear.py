@@ -100,6 +100,28 @@ def linear(lib, x, w, out_dtype: torch.dtype) -> torch.Tensor:
     return out
 
 
+def linear_group(lib, products, dtype: torch.dtype):
+    """Products that do not wait for each other: [(x [M, K], w, end)], end "float32", "same" (the result in `dtype`) or "tanh" (tanh of
+    the result, in `dtype`) -> their results.  One launch where tokens are few and all matrices are stored alike; else one after another."""
+    m, k = products[0][0].shape
+    frags = {_data(w)[1] for _, w, _ in products}
+    if (dtype == torch.bfloat16 and len(frags) == 1 and m > 0 and all(x.shape == (m, k) and x.dtype == dtype for x, _, _ in products)
+            and lib.gemm_bf16_group_ok(m, k)):
+        args = [(x, _data(w)[0], torch.empty((m, w.shape[0]), dtype=torch.float32 if end == "float32" else dtype, device=x.device),
+                 "bfloat16" if end == "same" else end) for x, w, end in products]
+        if all(t.data_ptr() % 16 == 0 for x, w, _, _ in args for t in (x, w)):
+            lib.gemm_bf16_group(args, frags.pop())
+            return [c for _, _, c, _ in args]
+    out = []
+    for x, w, end in products:
+        c = linear(lib, x, w, dtype if end == "same" else torch.float32)
+        if end == "tanh":
+            z, c = c, torch.empty(c.shape, dtype=dtype, device=c.device)
+            lib.tanh_cast(z, c)
+        out.append(c)
+    return out
+
+
 def linear_or_terms(lib, x, w) -> torch.Tensor:
     """x W^T in float32 for a reader that adds up terms itself: [M, N], or [P, M, N] where the
     product's kernel cut K into P slices (their sums are then not added by a kernel of their own)."""

@@ -1370,3 +1370,31 @@ def test_recurrences_in_chunks(lib, mode, heads, kv, dim, vdim, per_head, decay,
                 rms = lambda t: float((f(t) - want_).square().mean().sqrt())
                 assert rms(got_) <= 2 * rms(walked_) + 1e-9 * float(want_.abs().max()), (rms(got_), rms(walked_))
                 print(mode, dim, lens, rms(got_), rms(walked_), flush=True)
+
+
+# ---------------------------------------------------------------------------- products of few tokens in one launch
+@pytest.mark.parametrize("m", [1, 4, 16])
+@pytest.mark.parametrize("k", [128, 384, 2048, 8192])
+@pytest.mark.parametrize("rows,frag", [((16, 64, 1024), True), ((1, 37, 16, 250, 3), False), ((4096, 1024, 16, 16, 16, 16), True), ((2050,), False)])
+def test_products_in_one_launch(lib, m, k, rows, frag):
+    """Products of inputs, matrices and ends of their own against each in float64: a float32 sum of K products of bfloat16 numbers is off
+    by K 2^-24 of the sum of their sizes at the most, and bfloat16 results by half a unit in their last place besides."""
+    gen = torch.Generator().manual_seed(k + m + len(rows))
+    ends = ["float32", "bfloat16", "tanh"]
+    products, wants = [], []
+    for i, n in enumerate(rows):
+        x = torch.randn(m, k, generator=gen).to(torch.bfloat16)
+        w = (torch.randn(n, k, generator=gen) * k ** -0.5).to(torch.bfloat16)
+        end, wd = ends[(i + m) % 3], w.to(DEV)
+        if frag:
+            rows_of, wd = wd, torch.empty_like(wd)
+            lib.place_rows(rows_of, wd, frag=True)
+        want, size = x.double() @ w.double().T, k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        if end == "tanh":
+            want = want.tanh()
+        wants.append((want, size + (0 if end == "float32" else 2.0 ** -8 * want.abs()) + 1e-7))
+        products.append((x.to(DEV), wd, torch.full((m, n), 9.0, dtype=torch.float32 if end == "float32" else torch.bfloat16, device=DEV), end))
+    lib.gemm_bf16_group(products, frag)
+    for (_, _, c, _), (want, bound) in zip(products, wants):
+        _within(c, want, bound)
+    assert not lib.gemm_bf16_group_ok(17, 128) and not lib.gemm_bf16_group_ok(4, 192)
