@@ -71,7 +71,7 @@ import torch
 
 from ..errors import ConfigError
 from .base import BuildEnv, CacheRequest, Part, TensorSpec, build_part, register_mixer
-from .linear import linear, linear_or_terms, linear_to_stream, pack_rows
+from .linear import linear, linear_group, linear_or_terms, linear_to_stream, pack_rows, products_in_one_launch
 from .short_conv import ACT_NONE, ShortConv
 
 DEFAULT_NAMES = {"q": "q_proj.weight", "k": "k_proj.weight", "v": "v_proj.weight", "o": "o_proj.weight", "sink": "sink",
@@ -312,22 +312,23 @@ class Attention(Part):
         return out + ([state] if state is not None else [])
 
     # ------------------------------------------------------------------ forward
-    def _gate_and_project(self, attn, h, stream, next_norm):
+    def _gate_and_project(self, attn, h, stream, next_norm, gate=None):
         lib = self.env.lib
         if self.gate_kind == "head":
-            logits = linear(lib, h, self.w_gate, torch.float32)
+            logits = linear(lib, h, self.w_gate, torch.float32) if gate is None else gate
             lib.head_gate(attn, logits, 0, self.n_heads, self.pad)
         elif self.gate_kind == "elementwise":
-            lib.sigmoid_gate(attn, linear(lib, h, self.w_gate, torch.float32))
+            lib.sigmoid_gate(attn, linear(lib, h, self.w_gate, torch.float32) if gate is None else gate)
         return linear_to_stream(lib, attn, self.w_o, stream, next_norm)
 
-    def _forward_prepared(self, h, ctx, view, stream, next_norm):
+    def _forward_prepared(self, h, ctx, view, stream, next_norm, qkv=None, gate=None):
         """Bias and convolution, norms with weights, rotation and the cache write by kernels of their own; attention with
         capped scores and kept first tokens; the gate."""
         lib = self.env.lib
         t, hq, hk, d = h.shape[0], self.n_heads, self.n_kv, self.pad
         owns = self.cache_from is None
-        qkv = linear(lib, h, self.w_qkv, torch.float32)
+        if qkv is None:
+            qkv = linear(lib, h, self.w_qkv, torch.float32)
         if self.conv is not None:
             qkv = self.conv.forward(qkv, ctx, view.states.get("qkv_conv"), torch.float32, bias=self.bias)
         q = torch.empty((t, hq, d), dtype=self.env.dtype, device=h.device)
@@ -363,14 +364,15 @@ class Attention(Part):
             lib.attention_opts(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, view.block_table, hq, hk, d,
                                self.scale, window, self.keep_first, self.softcap or 0.0, self.sink, chunk=self.chunk or 0,
                                sig_bias=self.score_bias, n_seqs=ctx.n_seqs)
-        return self._gate_and_project(attn, h, stream, next_norm)
+        return self._gate_and_project(attn, h, stream, next_norm, gate)
 
-    def _forward_mixed(self, h, ctx, view, stream, next_norm):
+    def _forward_mixed(self, h, ctx, view, stream, next_norm, qkv=None, gate=None):
         """Biases, unit heads, the cache write, and attention with all heads of a token together."""
         lib = self.env.lib
         t, hq, hk, d = h.shape[0], self.n_heads, self.n_kv, self.pad
         owns = self.cache_from is None
-        qkv = linear(lib, h, self.w_qkv, torch.float32)
+        if qkv is None:
+            qkv = linear(lib, h, self.w_qkv, torch.float32)
         q = torch.empty((t, hq, d), dtype=self.env.dtype, device=h.device)
         lib.bias_norm_store(qkv, self.bias, self.qk_eps is not None, self.qk_eps or 0.0, q, view.k_pages if owns else None,
                             view.v_pages if owns else None, ctx.tok_pos, ctx.tok_seq, view.block_table, hq, hk, self.head_dim,
@@ -391,23 +393,30 @@ class Attention(Part):
         else:
             lib.attention_mixed(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, view.block_table, hq, hk, d,
                                 self.scale, self.talk, self.chunk or 0, window)
-        return self._gate_and_project(attn, h, stream, next_norm)
+        return self._gate_and_project(attn, h, stream, next_norm, gate)
 
-    def forward(self, h, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None):
+    def early(self, h):
+        """The products that wait for nothing but the mixer's input (`linear_group`'s): `forward` takes their results as `ready`."""
+        return [(h, self.w_qkv, "float32")] + ([(h, self.w_gate, "float32")] if self.has_gate else [])
+
+    def forward(self, h, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None, ready=None):
+        if (self.prepared or self.mixed) and hasattr(h, "tensor") and not isinstance(h, torch.Tensor):
+            h = h.tensor()
+        if ready is None and self.has_gate and products_in_one_launch(self.env.lib, h):
+            ready = linear_group(self.env.lib, self.early(h), self.env.dtype)
+        qkv, gate = (list(ready or []) + [None, None])[:2]
         if self.prepared:
-            if hasattr(h, "tensor") and not isinstance(h, torch.Tensor):
-                h = h.tensor()
-            return self._forward_prepared(h, ctx, view, stream, next_norm)
+            return self._forward_prepared(h, ctx, view, stream, next_norm, qkv, gate)
         if self.mixed:
-            if hasattr(h, "tensor") and not isinstance(h, torch.Tensor):
-                h = h.tensor()
-            return self._forward_mixed(h, ctx, view, stream, next_norm)
+            return self._forward_mixed(h, ctx, view, stream, next_norm, qkv, gate)
         lib = self.env.lib
         t = h.shape[0]
         hq, hk, d = self.n_heads, self.n_kv, self.pad
         owns = self.cache_from is None
         # q, k and v of the step; as the terms of the product where the position part reads such
-        if self.same_sizes and getattr(self.position, "takes_terms", False):
+        if qkv is not None:
+            pass
+        elif self.same_sizes and getattr(self.position, "takes_terms", False):
             qkv = linear_or_terms(lib, h, self.w_qkv)
         else:
             qkv = linear(lib, h, self.w_qkv, torch.float32)
@@ -426,7 +435,7 @@ class Attention(Part):
             n_splits, workspace = ctx.decode_workspace(hq, d, hk, spread=window == 0 and self.sink is None)
             lib.attention_decode_fused_bf16(qkv, cos, sin, style, view.k_pages, view.v_pages, attn, ctx.tok_pos, bt,
                                             hq, hk, d, self.scale, window, n_splits, workspace, sinks=self.sink)
-            return self._gate_and_project(attn, h, stream, next_norm)
+            return self._gate_and_project(attn, h, stream, next_norm, gate)
         q = torch.empty((t, hq, d), dtype=self.env.dtype, device=h.device)
         if self.same_sizes:
             if owns:
@@ -449,7 +458,7 @@ class Attention(Part):
         else:
             lib.attention_sinks(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, bt, hq, hk, d,
                                 self.scale, window, self.sink, n_seqs=ctx.n_seqs)
-        return self._gate_and_project(attn, h, stream, next_norm)
+        return self._gate_and_project(attn, h, stream, next_norm, gate)
 
 
 register_mixer("attention", Attention)

@@ -311,9 +311,13 @@ class DecayAttention(Part):
     def cache_request(self) -> Optional[CacheRequest]:
         return self.cache_requests()[0]
 
-    def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None) -> torch.Tensor:
+    def early(self, h):
+        """The products that wait for nothing but the mixer's input (`linear_group`'s): `forward` takes their results as `ready`."""
+        return [(h, self.w_in, "float32"), (h, self.w_a1, "same")]
+
+    def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None, ready=None) -> torch.Tensor:
         lib, t, c, dt = self.env.lib, h.shape[0], self.cols, self.env.dtype
-        proj, low = linear_group(lib, [(h, self.w_in, "float32"), (h, self.w_a1, "same")], dt)      # [T, q | k | v | gate]
+        proj, low = linear_group(lib, self.early(h), dt) if ready is None else ready                # proj [T, q | k | v | gate]
         z = linear(lib, low, self.w_a2, torch.float32)                        # [T, heads * dim]
         if self.one_launch and ctx.max_q_len == 1:
             on = torch.empty((t, self.n_v), dtype=dt, device=h.device)

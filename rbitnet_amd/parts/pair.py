@@ -24,6 +24,7 @@ import torch
 
 from ..errors import ConfigError
 from .base import BuildEnv, CacheRequest, Part, TensorSpec, _REGISTRIES, register_mixer
+from .linear import GROUP_PRODUCTS, linear_group, products_in_one_launch
 from .stream import WeightedTerms
 
 DEFAULT_NAMES = {"left_out": "left.out", "right_out": "right.out"}
@@ -100,8 +101,15 @@ class MixerPair(Part):
 
     def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None,
                 weighted_terms: bool = False):
-        a = self.left.forward(h, ctx, view)
-        b = self.right.forward(h, ctx, view)
+        ready = [{}, {}]
+        if hasattr(self.left, "early") and hasattr(self.right, "early") and products_in_one_launch(self.env.lib, h):
+            # a step of few tokens: what either mixer starts with, in one launch
+            first, second = self.left.early(h), self.right.early(h)
+            if len(first) + len(second) <= GROUP_PRODUCTS:
+                done = linear_group(self.env.lib, first + second, self.env.dtype)
+                ready = [{"ready": done[:len(first)]}, {"ready": done[len(first):]}]
+        a = self.left.forward(h, ctx, view, **ready[0])
+        b = self.right.forward(h, ctx, view, **ready[1])
         if self.combine == "weighted":
             if not weighted_terms:
                 raise ConfigError("a pair of mixers combined as a weighted sum needs a block that adds up its two terms (outnorm)")
