@@ -427,10 +427,13 @@ int rb_attention_generic_chunked(const void* q, const void* k_pages, const void*
                                  int n_tokens, int n_heads, int n_kv_heads, int head_dim, float scale, int window, int keep_first,
                                  float softcap, const float* sinks, int chunk, const float* sig_bias, void* stream);
 // n_seqs: how many sequences the tokens are of (0: not known); the choice of the kernel goes by it, not what is computed.
+// n_splits: how many workgroups may share a token's keys; more than one (at most 8) need a workspace: n_tokens * n_heads counters of 4
+// bytes, zeros before and after, then n_tokens * n_heads * n_splits * (head_dim + 2) floats.
 int rb_attention_generic_steps(const void* q, const void* k_pages, const void* v_pages, void* out, int dtype,
                                const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* block_table, int bt_stride,
                                int n_tokens, int n_heads, int n_kv_heads, int head_dim, float scale, int window, int keep_first,
-                               float softcap, const float* sinks, int chunk, const float* sig_bias, int n_seqs, void* stream);
+                               float softcap, const float* sinks, int chunk, const float* sig_bias, int n_seqs, int n_splits,
+                               void* workspace, void* stream);
 int rb_attention_prefill_bf16_chunked(const void* q, const void* k_pages, const void* v_pages, void* out,
                                       const int32_t* cu_seqlens, const int32_t* past_len, const int32_t* block_table, int bt_stride,
                                       int n_seqs, int max_q_len, int n_heads, int n_kv_heads, int head_dim, float scale, int window,

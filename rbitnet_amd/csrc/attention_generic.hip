@@ -305,13 +305,18 @@ __device__ __forceinline__ int here(int x) {
 // workgroup's own, keys of earlier steps are in none), 24 heads of 128 on 8: four prompts of 131 to 512 tokens 608 -> 130 us a layer, one
 // of 8 / 30 / 100 tokens 7.0 / 10.1 / 28 -> 8.0 / 8.2 / 12.7; single tokens at 150 / 1,000 keys: one sequence 22 / 51 -> 13.5 / 42, 16 27 / 88 -> 16 / 70,
 // 64 55 / 246 -> 39 / 162.  32 heads on 32, 64 sequences 159 / 784 -> 133 / 418.
-// ONE: a block is one token's.
+// ONE: a block is one token's, and where tokens and kv heads leave the GPU empty up to MAX_SHARING workgroups share its keys: as many as
+// have a unit of 32 keys for each of their 8 waves, known from the token's position, so that short contexts stay with one and pay nothing.
+// Whoever of them is done last adds up (no second launch, no waiting).  24 heads of 128 on 8, one workgroup / shared by up to 4: one token at
+// 250 / 280 / 400 / 1,000 / 4,000 keys 15.0 / 17.3 / 21.5 / 42.9 / 139.7 -> 14.6 / 14.9 / 16.3 / 18.6 / 46.3 us (28.3 by 8), four at 1,000 44.5 -> 19.9.
+constexpr int MAX_SHARING = 8;      // workgroups of a token's keys
 template <int NB, bool ONE>
 __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_kernel(
     const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages, float* __restrict__ out,
     const int32_t* __restrict__ tok_pos, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ block_table, int bt_stride,
     int n_tokens, int n_heads, int n_kv, int head_dim, float scale, int window, const float* __restrict__ sinks, int keep_first,
-    float softcap, int chunk, const float* __restrict__ sig_bias, int tokens_per_block, int head_chunks) {
+    float softcap, int chunk, const float* __restrict__ sig_bias, int tokens_per_block, int head_chunks, int32_t* __restrict__ arrived,
+    float* __restrict__ parts) {
   constexpr int VW = NB < 4 ? NB : 4;                  // floats of a load of V
   constexpr int CHAINS = 16 / NB;                      // the shorter a head, the more sums a unit's values go into
   constexpr int LD = 16 * NB + 4;                      // a query's row in LDS: outputs, then maximum and sum
@@ -368,7 +373,12 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
     const int kept = keep_first > 0 ? (keep_first + 31) / 32 : 0;
     const int n_first = kept < lo_unit ? kept : lo_unit;
     const int n_walk = hi < 0 ? 0 : n_first + hi / 32 - lo_unit + 1;      // (without a position there are no keys)
-    for (int walk = wave; walk < n_walk; walk += n_waves) {
+    // One token's keys: as many workgroups as its waves have keys for share them, the others are done (all of a token know the same).
+    const int needed = (n_walk + n_waves - 1) / n_waves;
+    const int sharing = !ONE || needed <= 1 ? 1 : needed < (int)gridDim.z ? needed : (int)gridDim.z;
+    const int part = ONE ? blockIdx.z : 0;
+    if (part >= sharing) return;
+    for (int walk = wave * sharing + part; walk < n_walk; walk += n_waves * sharing) {
       const int key0 = 32 * (walk < n_first ? walk : lo_unit + walk - n_first);
       const size_t base = ((size_t)pages[key0 / RB_PAGE] * n_kv + kvh) * RB_PAGE * head_dim + (size_t)(key0 % RB_PAGE) * head_dim;
       // keys behind the last one are not written yet: the last one's numbers stand in for them, with weight 0
@@ -517,8 +527,9 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
     l_run += __shfl_xor(l_run, 32, RB_WAVE);
 
     // lane holds, for query col, the numbers NB (4 g + j) + d of the head
-    const int at_work = n_walk > n_waves ? n_waves : n_walk;      // waves that had keys: the first ones
-    if (at_work <= 1) {
+    const int mine_of = (n_walk - part + sharing - 1) / sharing;           // units of this workgroup
+    const int at_work = mine_of > n_waves ? n_waves : mine_of;    // waves that had keys: the first ones
+    if (at_work <= 1 && sharing == 1) {
       if (!mine || wave > 0) continue;
       if (sinks) l_run += expf(sinks[h] - m_run);
       const float inv = sig_bias ? 1.0f : (l_run > 0.f ? 1.0f / l_run : 0.f);
@@ -558,9 +569,60 @@ __global__ __launch_bounds__(RB_WAVE * AG_MAX_WAVES) void attention_f32_mfma_ker
         l += src[(size_t)w * 16 * LD + 16 * NB + 1] * f;
         o += src[(size_t)w * 16 * LD + d] * f;
       }
+      if (sharing > 1) {
+        float* dst = parts + (((size_t)t0 * n_heads + hh) * gridDim.z + part) * (head_dim + 2);
+        __hip_atomic_store(dst + d, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (d == 0) {
+          __hip_atomic_store(dst + head_dim, mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(dst + head_dim + 1, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        continue;
+      }
       if (sinks) l += expf(sinks[hh] - mx);
       const float inv = sig_bias ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
       out[((size_t)(t0 + cc / h_count) * n_heads + hh) * head_dim + d] = o * inv;
+    }
+    if (ONE && sharing > 1) {
+      // Whoever is done last adds up what all have left, in their order; nobody waits for another.  What they leave goes through to
+      // where every workgroup sees it (atomic stores and loads of the device's scope) and has arrived before its wave counts: a fence
+      // would write back the whole L2 instead, 10 to 20 us with 128 workgroups.
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      int32_t* count = arrived + (size_t)t0 * gridDim.y + blockIdx.y;
+      if (threadIdx.x == 0) {
+        const bool last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == sharing - 1;
+        if (last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch
+        merged[0] = last ? 1.f : 0.f;
+      }
+      __syncthreads();
+      if (merged[0] == 0.f) return;
+      asm volatile("" ::: "memory");
+      for (int idx = threadIdx.x; idx < h_count * head_dim; idx += blockDim.x) {
+        const int hh = h0 + idx / head_dim, d = idx % head_dim;
+        const float* src = parts + ((size_t)t0 * n_heads + hh) * gridDim.z * (head_dim + 2);
+        float top[MAX_SHARING], sum[MAX_SHARING], value[MAX_SHARING];
+#pragma unroll
+        for (int w = 0; w < MAX_SHARING; ++w) {
+          const float* from = src + (size_t)(w < sharing ? w : sharing - 1) * (head_dim + 2);
+          top[w] = __hip_atomic_load(from + head_dim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          sum[w] = __hip_atomic_load(from + head_dim + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          value[w] = __hip_atomic_load(from + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < MAX_SHARING; ++w) mx = fmaxf(mx, top[w]);
+        float l = 0.f, o = 0.f;
+#pragma unroll
+        for (int w = 0; w < MAX_SHARING; ++w)
+          if (w < sharing) {
+            const float f = top[w] == -INFINITY ? 0.f : expf(top[w] - mx);
+            l += sum[w] * f;
+            o += value[w] * f;
+          }
+        if (sinks) l += expf(sinks[hh] - mx);
+        const float inv = sig_bias ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
+        out[((size_t)t0 * n_heads + hh) * head_dim + d] = o * inv;
+      }
     }
   }
 }
@@ -578,6 +640,8 @@ struct AttentionF32 {
   int chunk;
   const float* sig_bias;
   int n_seqs;            // 0: not known
+  int n_splits;          // workgroups that may share a token's keys
+  void* workspace;
 };
 
 template <int NB, bool ONE>
@@ -596,9 +660,12 @@ static int launch_attention_f32_blocks(const AttentionF32& a, int per_block, int
     RB_REQUIRE(e == hipSuccess, "rb_attention_generic: cannot reserve %zu bytes of LDS: %s", most, hipGetErrorString(e));
     configured = true;
   }
-  kern<<<dim3((unsigned)blocks, (unsigned)(a.n_kv * chunks)), RB_WAVE * n_waves, lds, s>>>(
+  const int splits = ONE && n_waves > 1 ? a.n_splits : 1;
+  int32_t* arrived = (int32_t*)a.workspace;
+  float* parts = a.workspace ? (float*)a.workspace + (size_t)a.n_tokens * a.n_heads : nullptr;
+  kern<<<dim3((unsigned)blocks, (unsigned)(a.n_kv * chunks), (unsigned)splits), RB_WAVE * n_waves, lds, s>>>(
       a.q, a.k_pages, a.v_pages, a.out, a.tok_pos, a.tok_seq, a.block_table, a.bt_stride, a.n_tokens, a.n_heads, a.n_kv, a.head_dim,
-      a.scale, a.window, a.sinks, a.keep_first, a.softcap, a.chunk, a.sig_bias, per_block, chunks);
+      a.scale, a.window, a.sinks, a.keep_first, a.softcap, a.chunk, a.sig_bias, per_block, chunks, arrived, parts);
   return 0;
 }
 
@@ -666,18 +733,21 @@ extern "C" int rb_attention_generic_chunked(const void* q, const void* k_pages, 
                                            n_heads, n_kv_heads, head_dim, scale, window, keep_first, softcap, sinks, chunk, sig_bias,
                                            stream));
   return rb_attention_generic_steps(q, k_pages, v_pages, out, dtype, tok_pos, tok_seq, block_table, bt_stride, n_tokens, n_heads,
-                                    n_kv_heads, head_dim, scale, window, keep_first, softcap, sinks, chunk, sig_bias, 0, stream);
+                                    n_kv_heads, head_dim, scale, window, keep_first, softcap, sinks, chunk, sig_bias, 0, 1, nullptr,
+                                    stream);
 }
 
-// The same, told how many sequences the tokens are of (0: not known; it decides between kernels, not what is computed).
+// The same, told how many sequences the tokens are of (0: not known; it decides between kernels, not what is computed), and how many
+// workgroups may share the keys of a token where every sequence has one (1: none).  workspace, where that is more than one:
+// n_tokens * n_heads counters, zeros before and after, then n_tokens * n_heads * n_splits * (head_dim + 2) floats.
 extern "C" int rb_attention_generic_steps(const void* q, const void* k_pages, const void* v_pages, void* out, int dtype,
                                           const int32_t* tok_pos, const int32_t* tok_seq, const int32_t* block_table,
                                           int bt_stride, int n_tokens, int n_heads, int n_kv_heads, int head_dim,
                                           float scale, int window, int keep_first, float softcap, const float* sinks, int chunk,
-                                          const float* sig_bias, int n_seqs, void* stream) {
+                                          const float* sig_bias, int n_seqs, int n_splits, void* workspace, void* stream) {
   RB_RECORDED(rb_attention_generic_steps(q, k_pages, v_pages, out, dtype, tok_pos, tok_seq, block_table, bt_stride, n_tokens,
                                          n_heads, n_kv_heads, head_dim, scale, window, keep_first, softcap, sinks, chunk, sig_bias,
-                                         n_seqs, stream));
+                                         n_seqs, n_splits, workspace, stream));
   RB_REQUIRE(keep_first >= 0 && softcap >= 0.f && chunk >= 0, "rb_attention_generic: negative keep_first, softcap or chunk");
   RB_REQUIRE(sig_bias == nullptr || sinks == nullptr, "rb_attention_generic: a sink belongs to the softmax");
   RB_REQUIRE(n_tokens >= 0 && n_heads > 0 && n_kv_heads > 0 && n_heads % n_kv_heads == 0,
@@ -686,12 +756,15 @@ extern "C" int rb_attention_generic_steps(const void* q, const void* k_pages, co
              AG_MAX_D);
   RB_REQUIRE(n_heads <= 65535, "rb_attention_generic: too many heads %d", n_heads);
   RB_REQUIRE(window >= 0, "rb_attention_generic: negative window");
+  RB_REQUIRE(n_splits >= 1 && n_splits <= MAX_SHARING && (n_splits == 1 || workspace != nullptr),
+             "rb_attention_generic: %d workgroups for a token's keys need a workspace and are at most %d", n_splits, MAX_SHARING);
+  RB_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3) == 0, "rb_attention_generic: the workspace is not aligned");
   if (n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool wide = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) & 15) == 0;
   if (dtype == RB_F32 && head_dim % 4 == 0 && head_dim <= 128 && wide && g_attention_vec == 1) {
     const AttentionF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, (float*)out, tok_pos, tok_seq, block_table,
-                            bt_stride, n_tokens, n_heads, n_kv_heads, head_dim, scale, window, sinks, keep_first, softcap, chunk, sig_bias, n_seqs};
+                            bt_stride, n_tokens, n_heads, n_kv_heads, head_dim, scale, window, sinks, keep_first, softcap, chunk, sig_bias, n_seqs, n_splits, workspace};
     const int rc = head_dim <= 32 ? launch_attention_f32<2>(a, s) : head_dim <= 64 ? launch_attention_f32<4>(a, s) : launch_attention_f32<8>(a, s);
     if (rc) return rc;
     RB_LAUNCH_CHECK();

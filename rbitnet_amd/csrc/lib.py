@@ -237,7 +237,7 @@ class Kernels:
             "rb_heads_linear_more": [_P, _I, _L, _P, _I, _I, _P, _I, _L, _I, _I, _I, _I, _P, _L, _I, _I, _I, _P, _P, _I, _P, _P],
             "rb_latent_norm_rope_store": [_P, _L, _I, _P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _P, _I, _I, _P, _P, _P, _I, _F, _I, _P],
             "rb_attention_generic_chunked": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _F, _P, _I, _P, _P],
-            "rb_attention_generic_steps": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _F, _P, _I, _P, _I, _P],
+            "rb_attention_generic_steps": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _F, _P, _I, _P, _I, _I, _P, _P],
             "rb_attention_prefill_bf16_chunked": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _F, _P, _I, _P, _P],
             "rb_attention_decode_bf16_chunked": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _F, _I, _P, _P, _I, _P, _P],
             "rb_heads_prepare": [_P, _L, _P, _P, _I, _I, _P, _P, _I, _F, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
@@ -1345,10 +1345,24 @@ class Kernels:
                                                 _ptr(ctx.tok_seq), _ptr(block_table) if kv_rank else None,
                                                 block_table.shape[1] if kv_rank else 0, float(eps), n, self._stream()))
 
+    @staticmethod
+    def _shared_keys(q, shared):
+        """(n_splits, pointer) of `shared`, None or (n_splits, workspace): an int32 counter for each (token, head), zeros before and
+        after the call, then n_splits rows of head_dim + 2 floats for each."""
+        if shared is None:
+            return 1, None
+        n_splits, workspace = shared
+        n, heads, dim = q.shape
+        _check(workspace, "workspace", torch.float32)
+        if workspace.numel() < n * heads * (1 + n_splits * (dim + 2)):
+            raise KernelError("the workspace of shared keys is too small")
+        return int(n_splits), _ptr(workspace)
+
     def attention_sinks(self, q, k_pages, v_pages, out, tok_pos, tok_seq, block_table, n_heads, n_kv, head_dim,
-                        scale, window, sinks, n_seqs: int = 0) -> None:
+                        scale, window, sinks, n_seqs: int = 0, shared=None) -> None:
         """`attention_generic` with a sink per query head in the softmax's denominator (sinks float32 [Hq] or None);
-        v_pages may be k_pages itself.  n_seqs: how many sequences the tokens are of (0: not known); which kernel runs goes by it."""
+        v_pages may be k_pages itself.  n_seqs: how many sequences the tokens are of (0: not known); which kernel runs goes by it.
+        shared: how many workgroups may share a token's keys, and their workspace (`_shared_keys`)."""
         n = q.shape[0]
         _check(q, "q", None, (n, n_heads, head_dim))
         _check(k_pages, "k_pages", q.dtype)
@@ -1365,7 +1379,8 @@ class Kernels:
             self._ok(self._lib.rb_attention_generic_steps(_ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(out), dtype_code(q.dtype),
                                                           _ptr(tok_pos), _ptr(tok_seq), _ptr(block_table), block_table.shape[1],
                                                           n, n_heads, n_kv, head_dim, float(scale), int(window or 0), 0, 0.0,
-                                                          _ptr(sinks), 0, None, int(n_seqs), self._stream()))
+                                                          _ptr(sinks), 0, None, int(n_seqs), *self._shared_keys(q, shared),
+                                                          self._stream()))
             return
         self._ok(self._lib.rb_attention_generic_sinks(_ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(out), dtype_code(q.dtype),
                                                       _ptr(tok_pos), _ptr(tok_seq), _ptr(block_table), block_table.shape[1],
@@ -1401,9 +1416,9 @@ class Kernels:
         self._ok(self._lib.rb_tanh_cast(_ptr(z), _ptr(out), dtype_code(out.dtype), z.numel(), self._stream()))
 
     def attention_opts(self, q, k_pages, v_pages, out, tok_pos, tok_seq, block_table, n_heads, n_kv, head_dim, scale, window,
-                       keep_first, softcap, sinks, chunk: int = 0, sig_bias=None, n_seqs: int = 0) -> None:
+                       keep_first, softcap, sinks, chunk: int = 0, sig_bias=None, n_seqs: int = 0, shared=None) -> None:
         """`attention_sinks` with kept first keys behind the window, capped scores, chunks (a query sees the keys of its own
-        chunk of positions only) and sigmoid weights (sig_bias float32 [Hq]).  n_seqs: as in `attention_sinks`."""
+        chunk of positions only) and sigmoid weights (sig_bias float32 [Hq]).  n_seqs, shared: as in `attention_sinks`."""
         n = q.shape[0]
         _check(q, "q", None, (n, n_heads, head_dim))
         _check(k_pages, "k_pages", q.dtype)
@@ -1423,7 +1438,8 @@ class Kernels:
                                                           _ptr(tok_pos), _ptr(tok_seq), _ptr(block_table), block_table.shape[1],
                                                           n, n_heads, n_kv, head_dim, float(scale), int(window or 0),
                                                           int(keep_first or 0), float(softcap or 0.0), _ptr(sinks),
-                                                          int(chunk or 0), _ptr(sig_bias), int(n_seqs), self._stream()))
+                                                          int(chunk or 0), _ptr(sig_bias), int(n_seqs),
+                                                          *self._shared_keys(q, shared), self._stream()))
             return
         if chunk or sig_bias is not None:
             self._ok(self._lib.rb_attention_generic_chunked(_ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(out), dtype_code(q.dtype),

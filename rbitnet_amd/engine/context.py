@@ -251,3 +251,17 @@ class StepContext:
                              device=self.device)
             self._workspaces[key] = (n_splits, ws)
         return self._workspaces[key]
+
+    def shared_keys_workspace(self, n_heads: int, head_dim: int, n_kv_heads: int) -> Optional[Tuple]:
+        """How many workgroups of the float32 attention may share the keys of a single token, and their scratch with counters (zeros
+        between launches); None where tokens and heads alone fill the GPU.  Up to 8, one a compute unit: a token's keys are
+        in 8 waves of a workgroup, and workgroups without keys for 8 waves of their own leave at once."""
+        blocks = self.n_seqs * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)
+        n_splits = min(8, self.n_compute_units // blocks)
+        if n_splits < 2:
+            return None
+        key = ("shared keys", n_heads, head_dim, n_splits)
+        if key not in self._workspaces:
+            ws = torch.zeros(self.n_seqs * n_heads * (1 + n_splits * (head_dim + 2)), dtype=torch.float32, device=self.device)
+            self._workspaces[key] = (n_splits, ws)
+        return self._workspaces[key]

@@ -321,6 +321,10 @@ class Attention(Part):
             lib.sigmoid_gate(attn, linear(lib, h, self.w_gate, torch.float32) if gate is None else gate)
         return linear_to_stream(lib, attn, self.w_o, stream, next_norm)
 
+    def _shared_keys(self, ctx):
+        """What lets several workgroups share a token's keys in float32 steps of single tokens."""
+        return ctx.shared_keys_workspace(self.n_heads, self.pad, self.n_kv) if self.env.dtype == torch.float32 and ctx.max_q_len == 1 else None
+
     def _forward_prepared(self, h, ctx, view, stream, next_norm, qkv=None, gate=None):
         """Bias and convolution, norms with weights, rotation and the cache write by kernels of their own; attention with
         capped scores and kept first tokens; the gate."""
@@ -363,7 +367,7 @@ class Attention(Part):
         else:
             lib.attention_opts(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, view.block_table, hq, hk, d,
                                self.scale, window, self.keep_first, self.softcap or 0.0, self.sink, chunk=self.chunk or 0,
-                               sig_bias=self.score_bias, n_seqs=ctx.n_seqs)
+                               sig_bias=self.score_bias, n_seqs=ctx.n_seqs, shared=self._shared_keys(ctx))
         return self._gate_and_project(attn, h, stream, next_norm, gate)
 
     def _forward_mixed(self, h, ctx, view, stream, next_norm, qkv=None, gate=None):
@@ -457,7 +461,7 @@ class Attention(Part):
                                        ctx.n_seqs, ctx.max_q_len, hq, hk, d, self.scale, window, sinks=self.sink)
         else:
             lib.attention_sinks(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, bt, hq, hk, d,
-                                self.scale, window, self.sink, n_seqs=ctx.n_seqs)
+                                self.scale, window, self.sink, n_seqs=ctx.n_seqs, shared=self._shared_keys(ctx))
         return self._gate_and_project(attn, h, stream, next_norm, gate)
 
 

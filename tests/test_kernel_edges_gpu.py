@@ -7,6 +7,7 @@ from rbitnet_amd.cache import Cache
 from rbitnet_amd.config.spec import PartSpec
 from rbitnet_amd.csrc.lib import kernels
 from rbitnet_amd.engine.context import StepBatch, StepContext
+from rbitnet_amd.errors import KernelError
 from rbitnet_amd.parts.base import BuildEnv, build_part
 
 pytestmark = pytest.mark.gpu
@@ -615,6 +616,42 @@ def test_float32_attention_of_tokens_in_any_order(lib, heads, kv, dim, more, ord
     lib.attention_opts(q.to(DEV), kp.to(DEV), vp.to(DEV), out, pos.int().to(DEV), seq.int().to(DEV), table.to(DEV), heads, kv, dim,
                        dim ** -0.5, more.get("window", 0), more.get("keep", 0), 0.0, None)
     _within(out.view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
+
+
+@pytest.mark.parametrize("heads,kv,dim,n_splits", [(24, 8, 128, 8), (40, 2, 100, 3), (16, 1, 64, 4), (6, 2, 24, 2)])
+@pytest.mark.parametrize("more", [{}, {"window": 300, "keep": 9, "cap": 3.0, "sinks": True}, {"sig": True, "chunk": 512}])
+def test_float32_tokens_whose_keys_are_shared(lib, heads, kv, dim, n_splits, more):
+    """Contexts in which no, some and all workgroups have keys: 8 units of 32 keys are one workgroup's, 9 two's.  The counters are zeros
+    again after every launch."""
+    g = torch.Generator().manual_seed(heads + dim + n_splits)
+    more = dict(more)
+    lengths = [1, 256, 257, 700, 2081, 64]
+    kp, table, ks = _paged(lengths, kv, dim, g)
+    vp, vs = torch.full_like(kp, float("nan")), []
+    for b, n in enumerate(lengths):
+        x = torch.randn(n, kv, dim, generator=g)
+        for j in range(n):
+            vp[table[b, j // 64], :, j % 64] = x[j]
+        vs.append(x)
+    n = len(lengths)
+    q = torch.randn(n, heads, dim, generator=g)
+    pos, seq = torch.tensor(lengths) - 1, torch.arange(n)
+    for name in ("sinks", "sig"):
+        if more.get(name):
+            more[name] = torch.randn(heads, generator=g)
+    want = torch.cat([_attention64(q[b:b + 1], ks[b], vs[b], pos[b:b + 1], dim ** -0.5, **more) for b in range(n)])
+    i32 = lambda x: x.to(torch.int32).to(DEV)
+    dev = lambda x: None if x is None else x.to(DEV)
+    workspace = torch.zeros(n * heads * (1 + n_splits * (dim + 2)), device=DEV)
+    args = [q.to(DEV), kp.to(DEV), vp.to(DEV), None, i32(pos), i32(seq), table.to(DEV), heads, kv, dim, dim ** -0.5, more.get("window", 0),
+            more.get("keep", 0), more.get("cap", 0.0), dev(more.get("sinks")), more.get("chunk", 0), dev(more.get("sig"))]
+    for _ in range(3):
+        args[3] = torch.full((n, heads * dim), float("nan"), device=DEV)
+        lib.attention_opts(*args, n_seqs=n, shared=(n_splits, workspace))
+        _within(args[3].view(want.shape), want, 64 * 2.0 ** -24 * max(4.0, float(want.abs().max())) * 4)
+        assert not workspace[:n * heads].view(torch.int32).any()
+    with pytest.raises(KernelError):
+        lib.attention_opts(*args, n_seqs=n, shared=(n_splits + 1, workspace))
 
 
 @pytest.mark.parametrize("heads,kv,dim", [(32, 32, 128), (4, 2, 24), (24, 8, 128), (16, 16, 64)])
