@@ -177,7 +177,10 @@ static bool launch_add_rmsnorm_vec(float* x, const float* delta, int n_terms, si
                                    float eps, const int32_t* rows, int n_rows, int width, TO* out, hipStream_t s) {
   if (width % 4 != 0 || term_stride % 4 != 0) return false;
   const int n4 = width / 4;
-  if (delta && n_terms > 1 && n4 > 256 && n4 <= 2048) {
+  // Rows of several terms, and rows of which a compute unit has no more than one: what counts is the trip to memory, which four times the
+  // threads make with a quarter of the loads each.  In a chain of launches, float32 out, 4 / 128 / 256 rows of 3,072: 3.20 / 3.59 / 4.12 us
+  // with 256 threads, 2.56 / 3.10 / 3.61 with 1,024; of 8,192: 5.01 / 6.13 / 7.48 and 3.66 / 4.84 / 6.07.
+  if (((delta && n_terms > 1) || n_rows <= rb_compute_units()) && n4 > 256 && n4 <= 2048) {
     if (n4 <= 1024)
       add_rmsnorm_vec_kernel<TO, 1, 1024><<<n_rows, 1024, 0, s>>>(x, delta, n_terms, term_stride, gain, eps, rows, width, out);
     else
@@ -362,7 +365,10 @@ __global__ void rope_kv_write_vec_kernel(const float* __restrict__ qkv, int n_te
   }
   if (v_pages) {
     const float* vsrc = src + (size_t)(n_heads + n_kv) * head_dim;
-    for (int idx = 4 * threadIdx.x; idx < n_kv * head_dim; idx += 4 * blockDim.x) {
+    // the threads behind the last ones with heads first: they have nothing else to do
+    const int turn = ((n_heads + n_kv) * quads - first) % blockDim.x;
+    const int start = (int)threadIdx.x < turn ? threadIdx.x + blockDim.x - turn : threadIdx.x - turn;
+    for (int idx = 4 * start; idx < n_kv * head_dim; idx += 4 * blockDim.x) {
       const int h = idx / head_dim;
       const int d = idx - h * head_dim;
       const float4 v = sum_terms4(vsrc + idx, n_terms, term_stride);
@@ -390,13 +396,17 @@ extern "C" int rb_rope_kv_write(const float* qkv, int qkv_terms, long long qkv_t
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   const bool vec = head_dim % 8 == 0 && qkv_term_stride % 4 == 0 && aligned(qkv) && aligned(cos) && aligned(sin) &&
                    aligned(q_out) && aligned(k_pages) && aligned(v_pages);
+  // A step of few tokens waits for its loads: with four times the threads each has one trip to memory instead of three (24 heads of
+  // 128 on 8, float32, 4 / 32 / 256 tokens in a chain of launches: 3.06 / 3.30 / 3.80 us with 256 threads, 2.43 / 2.66 / 3.33 with 1,024; more tokens
+  // fill the GPU by themselves).
+  const int threads = n_tokens <= rb_compute_units() ? 1024 : 256;
   if (vec && cache_dtype == RB_F32)
-    rope_kv_write_vec_kernel<float><<<n_tokens, 256, 0, s>>>(qkv, qkv_terms, (size_t)qkv_term_stride, cos, sin, style,
+    rope_kv_write_vec_kernel<float><<<n_tokens, threads, 0, s>>>(qkv, qkv_terms, (size_t)qkv_term_stride, cos, sin, style,
                                                              (float*)q_out, (float*)k_pages, (float*)v_pages, tok_pos,
                                                              tok_seq, block_table, bt_stride, n_heads, n_kv_heads,
                                                              head_dim);
   else if (vec && cache_dtype == RB_BF16)
-    rope_kv_write_vec_kernel<bf16_t><<<n_tokens, 256, 0, s>>>(qkv, qkv_terms, (size_t)qkv_term_stride, cos, sin, style,
+    rope_kv_write_vec_kernel<bf16_t><<<n_tokens, threads, 0, s>>>(qkv, qkv_terms, (size_t)qkv_term_stride, cos, sin, style,
                                                               (bf16_t*)q_out, (bf16_t*)k_pages, (bf16_t*)v_pages,
                                                               tok_pos, tok_seq, block_table, bt_stride, n_heads,
                                                               n_kv_heads, head_dim);

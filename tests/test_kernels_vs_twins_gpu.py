@@ -81,6 +81,36 @@ def test_add_rmsnorm(lib, twin, out_dtype, width):
             _close(*res[0], what="stream")              # updated in place, or left alone with chosen rows
 
 
+@pytest.mark.parametrize("out_dtype", [F32, BF])
+@pytest.mark.parametrize("width", [1024, 1028, 4100, 8192])
+def test_add_rmsnorm_by_rows(lib, twin, out_dtype, width):
+    """On either side of as many rows as compute units, where the number of threads a row changes."""
+    g, units = _gen(width), torch.cuda.get_device_properties(0).multi_processor_count
+    gain = 1 + 0.1 * torch.randn(width, generator=g)
+    for n in (1, units, units + 1):
+        x, delta = torch.randn(n, width, generator=g), torch.randn(n, width, generator=g)
+        res = _both(lib, twin, "add_rmsnorm", [x, delta, gain, 1e-5, None, torch.empty(n, width, dtype=out_dtype)], [0, 5])
+        _close(*res[5], what=f"norm of {n}")
+        _close(*res[0], what="stream")
+
+
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("hq,hk,d", [(24, 8, 128), (6, 2, 24), (64, 64, 64)])
+def test_rope_kv_write_by_tokens(lib, twin, dtype, hq, hk, d):
+    """On either side of as many tokens as compute units, where the number of threads a token changes."""
+    g, units = _gen(hq + d), torch.cuda.get_device_properties(0).multi_processor_count
+    angles = torch.arange(64, dtype=torch.float64)[:, None] * (10000.0 ** (-2.0 * torch.arange(d // 2) / d))[None, :]
+    for n in (1, units + 1):
+        cos, sin = torch.cos(angles).float(), torch.sin(angles).float()
+        qkv = torch.randn(n, (hq + 2 * hk) * d, generator=g)
+        pages = torch.zeros(n + 1, hk, 64, d, dtype=dtype)
+        pos = (torch.arange(n) % 64).to(I32)
+        args = [qkv, cos, sin, 1, torch.empty(n, hq, d, dtype=dtype), pages, pages.clone(), pos, torch.arange(n).to(I32),
+                (1 + torch.arange(n)).to(I32).view(n, 1), hq, hk, d]
+        for i, pair in _both(lib, twin, "rope_kv_write", args, [4, 5, 6]).items():
+            assert torch.equal(pair[0].cpu(), pair[1]), f"argument {i} of {n}"
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 @pytest.mark.parametrize("style", [0, 1])
 def test_rope_kv_write(lib, twin, dtype, style):
