@@ -366,8 +366,8 @@ __global__ void rope_kv_write_vec_kernel(const float* __restrict__ qkv, int n_te
   if (v_pages) {
     const float* vsrc = src + (size_t)(n_heads + n_kv) * head_dim;
     // the threads behind the last ones with heads first: they have nothing else to do
-    const int turn = ((n_heads + n_kv) * quads - first) % blockDim.x;
-    const int start = (int)threadIdx.x < turn ? threadIdx.x + blockDim.x - turn : threadIdx.x - turn;
+    const int busy = (n_heads + n_kv) * quads - first, n_threads = blockDim.x;
+    const int start = busy > n_threads ? threadIdx.x : (int)threadIdx.x < busy ? threadIdx.x + n_threads - busy : threadIdx.x - busy;
     for (int idx = 4 * start; idx < n_kv * head_dim; idx += 4 * blockDim.x) {
       const int h = idx / head_dim;
       const int d = idx - h * head_dim;
@@ -399,7 +399,7 @@ extern "C" int rb_rope_kv_write(const float* qkv, int qkv_terms, long long qkv_t
   // A step of few tokens waits for its loads: with four times the threads each has one trip to memory instead of three (24 heads of
   // 128 on 8, float32, 4 / 32 / 256 tokens in a chain of launches: 3.06 / 3.30 / 3.80 us with 256 threads, 2.43 / 2.66 / 3.33 with 1,024; more tokens
   // fill the GPU by themselves).
-  const int threads = n_tokens <= rb_compute_units() ? 1024 : 256;
+  const int threads = n_tokens <= rb_compute_units() && (n_heads + n_kv_heads) * head_dim / 8 + n_kv_heads * head_dim / 4 > 256 ? 1024 : 256;
   if (vec && cache_dtype == RB_F32)
     rope_kv_write_vec_kernel<float><<<n_tokens, threads, 0, s>>>(qkv, qkv_terms, (size_t)qkv_term_stride, cos, sin, style,
                                                              (float*)q_out, (float*)k_pages, (float*)v_pages, tok_pos,
