@@ -1406,7 +1406,6 @@ def test_recurrences_in_chunks(lib, mode, heads, kv, dim, vdim, per_head, decay,
             for got_, walked_, want_ in ((got, walked, want.reshape(n, -1)), (got_state[slots], walked_state[slots], want_state)):
                 rms = lambda t: float((f(t) - want_).square().mean().sqrt())
                 assert rms(got_) <= 2 * rms(walked_) + 1e-9 * float(want_.abs().max()), (rms(got_), rms(walked_))
-                print(mode, dim, lens, rms(got_), rms(walked_), flush=True)
 
 
 # ---------------------------------------------------------------------------- products of few tokens in one launch
