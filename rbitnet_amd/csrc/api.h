@@ -540,6 +540,7 @@ int rb_latent_norm_rope_store(const float* proj, long long stride, int q_rank, c
 int rb_sample_workspace_bytes(int n_rows, int vocab);
 int rb_fetch_words(const int32_t* host, int32_t* out, long long n, void* stream);      // from pinned host memory, as it is when the kernel runs
 int rb_stream_wait(void* stream);
+int rb_zero_words(void* out, long long n, void* stream);      // n words of 4 bytes, by a launch that a recorded step repeats
 int rb_sample(const float* logits, int n_rows, int vocab, const float* temperature, const float* u,
               int32_t* tokens, void* workspace, void* stream);
 

@@ -34,6 +34,21 @@ int rb_compute_units(void) {
   return known[dev];
 }
 
+// ---------------------------------------------------------------- zeros
+// Clearing that a recorded or captured step has to repeat: a launch like any other (a memset is none).
+__global__ __launch_bounds__(256) void zero_words_kernel(int32_t* __restrict__ out, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) out[i] = 0;
+}
+extern "C" int rb_zero_words(void* out, long long n, void* stream) {
+  RB_RECORDED(rb_zero_words(out, n, stream));
+  RB_REQUIRE(n >= 0 && (reinterpret_cast<uintptr_t>(out) & 3) == 0, "rb_zero_words: %lld words, or not at a word's address", n);
+  if (n == 0) return 0;
+  const long long blocks = (n + 255) / 256;
+  zero_words_kernel<<<(int)(blocks < 1024 ? blocks : 1024), 256, 0, (hipStream_t)stream>>>((int32_t*)out, (size_t)n);
+  RB_LAUNCH_CHECK();
+  return 0;
+}
+
 // ---------------------------------------------------------------- embedding
 // Reference: x[j] = token_embd[j + tok * n_embd] (llama/model.rs:229-232).
 template <typename T>

@@ -173,6 +173,7 @@ class Kernels:
                                                      _F, _I, _I, _P, _P, _P],
             "rb_fetch_words": [_P, _P, _L, _P],
             "rb_stream_wait": [_P],
+            "rb_zero_words": [_P, _L, _P],
             "rb_sample": [_P, _I, _I, _P, _P, _P, _P, _P],
             "rb_fill_normal": [_P, _I, ctypes.c_longlong, ctypes.c_ulonglong, ctypes.c_double, ctypes.c_double, _P],
             "rb_place_rows": [_P, _I, _P, _I, _I] + [ctypes.c_longlong] * 6 + [_P],
@@ -595,6 +596,13 @@ class Kernels:
             raise KernelError("host must be contiguous int32 in pinned memory")
         _check(out, "out", torch.int32, host.shape)
         self._ok(self._lib.rb_fetch_words(_ptr(host), _ptr(out), out.numel(), self._stream()))
+
+    def zero_words(self, words: torch.Tensor) -> None:
+        """Zeros in a tensor of 4-byte numbers, by a launch of the library's own: a recorded step repeats it, a `zero_()` it would not."""
+        if words.dtype not in (torch.int32, torch.float32):
+            raise KernelError("words must be int32 or float32")
+        _check(words, "words", None, words.shape)
+        self._ok(self._lib.rb_zero_words(_ptr(words), words.numel(), self._stream()))
 
     def wait(self) -> None:
         """Until everything that was put on torch's current stream has run."""

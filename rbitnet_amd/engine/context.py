@@ -252,16 +252,21 @@ class StepContext:
             self._workspaces[key] = (n_splits, ws)
         return self._workspaces[key]
 
-    def shared_keys_workspace(self, n_heads: int, head_dim: int, n_kv_heads: int) -> Optional[Tuple]:
+    def shared_keys_workspace(self, lib, n_heads: int, head_dim: int, n_kv_heads: int) -> Optional[Tuple]:
         """How many workgroups of the float32 attention may share the keys of a single token, and their scratch with counters (zeros
         between launches); None where tokens and heads alone fill the GPU.  Up to 8, one a compute unit: a token's keys are
-        in 8 waves of a workgroup, and workgroups without keys for 8 waves of their own leave at once."""
+        in 8 waves of a workgroup, and workgroups without keys for 8 waves of their own leave at once.
+
+        The counters are cleared by a launch of the step that makes the scratch.  A recorded step repeats that launch before the first
+        use, and has to: the memory may be what a temporary of an earlier layer held, which every replay writes again."""
         blocks = self.n_seqs * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)
         n_splits = min(8, self.n_compute_units // blocks)
         if n_splits < 2:
             return None
         key = ("shared keys", n_heads, head_dim, n_splits)
         if key not in self._workspaces:
-            ws = torch.zeros(self.n_seqs * n_heads * (1 + n_splits * (head_dim + 2)), dtype=torch.float32, device=self.device)
+            counters = self.n_seqs * n_heads
+            ws = torch.empty(counters * (1 + n_splits * (head_dim + 2)), dtype=torch.float32, device=self.device)
+            lib.zero_words(ws[:counters])
             self._workspaces[key] = (n_splits, ws)
         return self._workspaces[key]

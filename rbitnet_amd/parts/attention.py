@@ -323,7 +323,9 @@ class Attention(Part):
 
     def _shared_keys(self, ctx):
         """What lets several workgroups share a token's keys in float32 steps of single tokens."""
-        return ctx.shared_keys_workspace(self.n_heads, self.pad, self.n_kv) if self.env.dtype == torch.float32 and ctx.max_q_len == 1 else None
+        if self.env.dtype != torch.float32 or ctx.max_q_len != 1:
+            return None
+        return ctx.shared_keys_workspace(self.env.lib, self.n_heads, self.pad, self.n_kv)
 
     def _forward_prepared(self, h, ctx, view, stream, next_norm, qkv=None, gate=None):
         """Bias and convolution, norms with weights, rotation and the cache write by kernels of their own; attention with

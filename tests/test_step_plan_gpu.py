@@ -57,6 +57,33 @@ def test_replayed_steps_equal_steps_launched_from_python(name, dtype):
     planned.cache.check()
 
 
+def test_replayed_single_tokens_whose_keys_are_shared_start_from_zero_counters():
+    """Float32 steps of one token per sequence with more than 256 keys: workgroups share a token's keys and count who is done.  A replay
+    gives the eager step's bits whatever its scratch memory holds when it starts: in the plan's pool that may be what a temporary
+    of an earlier layer was in."""
+    eager, planned = _engine("D", "float32", max_batch=2), _engine("D", "float32", max_batch=2)
+    eager.use_plans = False
+    lengths, new = (300, 700), 6
+    reqs = [tokens_for("D", n + new, n) for n in lengths]
+    outs = []
+    for eng in (eager, planned):
+        slots = [eng.alloc_slot() for _ in reqs]
+        eng.step([(s, r[:n]) for s, r, n in zip(slots, reqs, lengths)], "last")
+        got = []
+        for j in range(new):
+            for plan in eng.plans.plans.values():
+                for _, scratch in plan.ctx._workspaces.values():
+                    scratch.view(torch.int32).fill_(5)
+            got.append(eng.step([(s, [r[n + j]]) for s, r, n in zip(slots, reqs, lengths)], "last"))
+        outs.append(torch.stack(got))
+        for s in slots:
+            eng.free_slot(s)
+    assert planned.plans.stats["replayed"] >= 2 and any(k[0] == "shared keys" for p in planned.plans.plans.values() for k in p.ctx._workspaces)
+    assert torch.equal(outs[0], outs[1])
+    for i, (r, n) in enumerate(zip(reqs, lengths)):
+        assert max_err(outs[1][:, i], plain_logits("D", tuple(r))[n:n + new]) < TOL["float32"]
+
+
 def test_a_shape_seen_once_is_not_recorded_and_old_plans_make_room():
     from rbitnet_amd.engine import step_plan
     eng = _engine("A", "float32", max_batch=1, max_tokens=256)
