@@ -21,6 +21,8 @@ from typing import Callable, Dict, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
+from ..cache.pages import pages_for
+
 # tests may force a number of splits of decode attention (None: the built-in choice)
 FORCED_DECODE_SPLITS: Optional[int] = None
 
@@ -215,8 +217,12 @@ class StepContext:
     def refill_single(self, slots: Sequence[int], past: Sequence[int], tokens: Sequence[int], tables: Dict[int, np.ndarray],
                       temperatures: Optional[Sequence[float]], uniforms: Optional[Sequence[float]]) -> None:
         """What differs between two batches of one token per sequence, written into the layout (whose other arrays a `fill` wrote
-        before); a captured step copies it over itself.  tables: per storage group, an array of rows at most as wide as the layout's."""
+        before); a captured step copies it over itself.  tables: per storage group, an array of rows at most as wide as the layout's.
+        Only tables bound a sequence: layers with states alone have none."""
         h = self._h
+        pages = pages_for(max(past) + 1)
+        if any(pages > h[("table", key)].shape[1] for key in tables):
+            raise ValueError("a sequence holds more pages than the step layout has room for")
         h["token_ids"][:] = tokens
         h["tok_pos"][:] = past
         h["past_len"][:] = past

@@ -28,7 +28,6 @@ from typing import Optional
 
 import torch
 
-from ..cache import pages_for
 from .context import StepBatch, StepContext, bucket_max_pages
 
 GRAPH_SIZES = (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64)
@@ -80,8 +79,6 @@ class DecodeGraph:
             ctx.fill(StepBatch(slots=slots, past_lens=past, tokens=[[t] for t in tokens], rows=list(range(self.n_seqs)),
                                block_tables=cache.block_tables(slots), temperatures=temperatures, uniforms=uniforms), copy=False)
             return
-        if pages_for(max(past) + 1) > self.width:
-            raise ValueError("a sequence holds more pages than the step layout has room for")
         ctx.refill_single(slots, past, tokens, cache.table_rows(slots, self.width), temperatures, uniforms)
 
     def _launch(self) -> None:

@@ -131,6 +131,48 @@ def test_rows_of_page_tables_and_steps_of_one_token(window):
         c.reserve_one([0, 0], [0, 0])
 
 
+def test_a_captured_steps_layout_has_room_to_check_only_where_pages_are():
+    """`StepContext.refill_single` across the end of the pages: a cache of states alone has no tables and so no limit; with pages,
+    windowed ones too, a sequence that holds more of them than the layout has columns for is refused before anything is written."""
+    from rbitnet_amd.engine.context import StepContext
+
+    def refill(cache, past):
+        slot = cache.alloc_slot()
+        cache.reserve([slot], [past])
+        cache.commit([slot], [past])
+        ctx = StepContext("cpu", 1, 1, 1, {key: cache.n_pages for key in cache.group_keys()}, bucket=1, n_compute_units=256)
+        ctx._h["past_len"][:] = -1
+        try:
+            cache.reserve_one([slot], [past])
+            ctx.refill_single([slot], [past], [3], cache.table_rows([slot], cache.n_pages), None, None)
+        finally:
+            cache.free_slot(slot)
+        return ctx
+
+    states = Cache([CacheRequest("state", state_shape=(2, 3))], 2, 64, torch.float32, "cpu")
+    for past in (0, 63, 64, 65, 5000):
+        ctx = refill(states, past)
+        assert ctx._h["past_len"][0] == past and ctx.max_kv_len == past + 1 and ctx.host_past == [past]
+    both = Cache([CacheRequest("state", state_shape=(2, 3)), CacheRequest("kv", heads=1, head_dim=8)], 2, 128, torch.float32, "cpu")
+    assert refill(both, 127)._h["past_len"][0] == 127
+    with pytest.raises(CacheError, match="cache full"):
+        refill(both, 128)
+    windowed = _cache(max_tokens=64 * 4, window=70)
+    slot = windowed.alloc_slot()
+    ctx = StepContext("cpu", 1, 1, 1, {key: windowed.n_pages for key in windowed.group_keys()}, bucket=1, n_compute_units=256)
+    for past in range(300):
+        windowed.reserve_one([slot], [past])
+        rows = windowed.table_rows([slot], windowed.n_pages)
+        if past < 256:
+            ctx.refill_single([slot], [past], [3], rows, None, None)
+            windowed.commit([slot], [1])
+        else:
+            with pytest.raises(ValueError, match="more pages"):
+                ctx.refill_single([slot], [past], [3], rows, None, None)
+            assert ctx._h["past_len"][0] == 255
+            break
+
+
 def test_groups_by_need_and_readers():
     reqs = [CacheRequest("kv", heads=2, head_dim=8), CacheRequest("kv", heads=2, head_dim=8, window=100),
             None, CacheRequest("kv", heads=2, head_dim=8), CacheRequest("kv", heads=1, head_dim=16),

@@ -551,6 +551,27 @@ def test_experts_on_the_dense_products_tiles_give_what_the_routed_kernels_give(l
 
 
 # ---------------------------------------------------------------------------- whole models
+def test_a_model_of_states_alone_decodes_past_its_cache_of_pages():
+    """Layers with states and none with keys: `max_tokens` sizes pages that nobody has, and captured steps go on behind it as steps
+    launched one by one do."""
+    import rbitnet_amd
+    config = {"architecture": "Goperax", "vocab": 90, "width": 64, "streams": 2, "embedding": {"scale": 8.0}, "norm": {"eps": 1e-5},
+              "layers": [{"type": "mamba2", "mixer": _scan(4, 32, 32, 2, 4, 2), "mlp": {"kind": "dense", "ff": 96}} for _ in range(2)]}
+    outs = []
+    for graphs in (True, False):
+        eng = rbitnet_amd.Engine.random(config, std=0.1, dtype="float32", max_tokens=64, max_batch=2, max_seq_len=200)
+        eng.use_graphs, eng.use_plans = graphs, False
+        assert not eng.cache.kv_groups
+        slots, logits = [eng.alloc_slot(), eng.alloc_slot()], []
+        eng.step([(slots[0], list(range(60))), (slots[1], [5, 6, 7])])
+        for j in range(70):
+            eng.decode_step(slots, [j, 2 * j % 90])
+            logits.append(eng.last_decode_logits.clone())
+        assert eng.length(slots[0]) == 130
+        outs.append(torch.stack(logits))
+    assert torch.equal(outs[0], outs[1])
+
+
 def _moe(ff, experts, top, shared=None):
     out = {"kind": "moe", "expert": {"ff": ff}, "router": {"experts": experts, "top": top}}
     if shared:
