@@ -105,12 +105,14 @@ class DecodeGraph:
             # that allocations settle, and its result is the step's result; then the same launches
             # are captured for the steps after it.  Capturing executes nothing, so a mixer that
             # updates a state of its own has updated it once.
+            self._in_flight = True
             side = torch.cuda.Stream(device=eng.device)
             side.wait_stream(torch.cuda.current_stream())
             with torch.cuda.stream(side):
                 self._launch()
             torch.cuda.current_stream().wait_stream(side)
             torch.cuda.synchronize()
+            self._in_flight = False
             out = self._tokens[:n].tolist()
             first_logits = self.logits.clone()
             graph = torch.cuda.CUDAGraph()
