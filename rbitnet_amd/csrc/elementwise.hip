@@ -124,13 +124,16 @@ __device__ __forceinline__ void add4(float4& d, const float4& e) {
   d.w += e.w;
 }
 
-template <typename TO, int VPT, int THREADS>          // VPT float4 per thread
+// AS_FEW: a thousand threads add the squares up in the order of 256 of them, so that a row's norm is the same bits whether the step has few rows or
+// many: the sums of four squares meet in LDS, and 256 threads take every 256th of them in turn.
+template <typename TO, int VPT, int THREADS, bool AS_FEW = false>          // VPT float4 per thread
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restrict__ x, const float* __restrict__ delta,
                                                               int n_terms, size_t term_stride,
                                                               const float* __restrict__ gain, float eps,
                                                               const int32_t* __restrict__ rows, int width,
                                                               TO* __restrict__ out) {
-  __shared__ float scratch[16];
+  constexpr int FEW = 256;
+  __shared__ float scratch[16], quads[AS_FEW ? VPT * THREADS : 1];
   const int r = blockIdx.x;
   const size_t src = rows ? (size_t)rows[r] : (size_t)r;
   float4* xr = reinterpret_cast<float4*>(x + src * width);
@@ -170,9 +173,25 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restr
   for (int i = 0; i < VPT; ++i) {
     const int c = threadIdx.x + i * THREADS;
     if (write_back && c < n4) xr[c] = v[i];
-    ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+    const float four = v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+    if (AS_FEW) quads[c] = four;
+    else ss += four;
   }
-  ss = block_sum(ss, scratch);
+  if (AS_FEW) {
+    __syncthreads();
+    if (threadIdx.x < FEW) {
+#pragma unroll
+      for (int i = 0; i < VPT * THREADS / FEW; ++i) ss += quads[threadIdx.x + i * FEW];
+      ss = wave_sum(ss);
+      if (threadIdx.x % RB_WAVE == 0) scratch[threadIdx.x / RB_WAVE] = ss;
+    }
+    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < FEW / RB_WAVE; ++i) ss += scratch[i];
+  } else {
+    ss = block_sum(ss, scratch);
+  }
   const float scale = 1.0f / sqrtf(ss / (float)width + eps);
   TO* orow = out + (size_t)r * width;
 #pragma unroll
@@ -194,14 +213,17 @@ static bool launch_add_rmsnorm_vec(float* x, const float* delta, int n_terms, si
   const int n4 = width / 4;
   // Rows of several terms, and rows of which a compute unit has no more than one: what counts is the trip to memory, which four times the
   // threads make with a quarter of the loads each.  In a chain of launches, float32 out, 4 / 128 / 256 rows of 3,072: 3.20 / 3.59 / 4.12 us
-  // with 256 threads, 2.56 / 3.10 / 3.61 with 1,024; of 8,192: 5.01 / 6.13 / 7.48 and 3.66 / 4.84 / 6.07.
-  if (((delta && n_terms > 1) || n_rows <= rb_compute_units()) && n4 > 256 && n4 <= 2048) {
-    if (n4 <= 1024)
-      add_rmsnorm_vec_kernel<TO, 1, 1024><<<n_rows, 1024, 0, s>>>(x, delta, n_terms, term_stride, gain, eps, rows, width, out);
-    else
-      add_rmsnorm_vec_kernel<TO, 2, 1024><<<n_rows, 1024, 0, s>>>(x, delta, n_terms, term_stride, gain, eps, rows, width, out);
+  // with 256 threads, 2.53 / 3.05 / 3.62 with 1,024; of 8,192: 5.07 / 6.17 / 7.45 and 3.46 / 4.60 / 5.83.
+#define AN_GO(VPT, ...) add_rmsnorm_vec_kernel<TO, VPT, __VA_ARGS__><<<n_rows, 1024, 0, s>>>(x, delta, n_terms, term_stride, gain, eps, rows, width, out)
+  const bool terms = delta && n_terms > 1;
+  if ((terms || n_rows <= rb_compute_units()) && n4 > 256 && n4 <= 2048) {
+    if (terms && n4 <= 1024) AN_GO(1, 1024);
+    else if (terms) AN_GO(2, 1024);
+    else if (n4 <= 1024) AN_GO(1, 1024, true);
+    else AN_GO(2, 1024, true);
     return true;
   }
+#undef AN_GO
   if (n4 <= 256)
     add_rmsnorm_vec_kernel<TO, 1, 256><<<n_rows, 256, 0, s>>>(x, delta, n_terms, term_stride, gain, eps, rows, width, out);
   else if (n4 <= 512)

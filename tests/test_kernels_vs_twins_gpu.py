@@ -94,6 +94,21 @@ def test_add_rmsnorm_by_rows(lib, twin, out_dtype, width):
         _close(*res[0], what="stream")
 
 
+@pytest.mark.parametrize("width", [1024, 1028, 2048, 4096, 4100, 8192])
+def test_a_rows_norm_is_the_same_bits_among_few_rows_and_among_many(lib, width):
+    """The squares are added up in the same order by either number of threads, with and without one term to add to the row first."""
+    g, units = _gen(width), torch.cuda.get_device_properties(0).multi_processor_count
+    gain, rows = (1 + 0.1 * torch.randn(width, generator=g)).cuda(), 3 * units + 1
+    x, delta = torch.randn(rows, width, generator=g).cuda(), torch.randn(rows, width, generator=g).cuda()
+    for d in (None, delta):
+        many, streams = torch.empty(rows, width, device="cuda"), x.clone()
+        lib.add_rmsnorm(streams, d, gain, 1e-5, None, many)
+        for n in (1, units):
+            few, stream = torch.empty(n, width, device="cuda"), x[-n:].clone()
+            lib.add_rmsnorm(stream, None if d is None else d[-n:].contiguous(), gain, 1e-5, None, few)
+            assert torch.equal(few, many[-n:]) and torch.equal(stream, streams[-n:])
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 @pytest.mark.parametrize("hq,hk,d", [(24, 8, 128), (6, 2, 24), (64, 64, 64)])
 def test_rope_kv_write_by_tokens(lib, twin, dtype, hq, hk, d):
