@@ -854,6 +854,14 @@ class Kernels:
     def recurrence_step_ok(self, n_heads: int, n_kv: int, dim: int, vdim: int, taps: int = 0, norm_part: int = 0) -> bool:
         return bool(self._lib.rb_recurrence_step_ok(n_heads, n_kv, dim, vdim, taps, norm_part))
 
+    @staticmethod
+    def recurrence_step_pays(mode: str, n_heads: int, n_kv: int, dim: int, vdim: int, n_seqs: int) -> bool:
+        """Whether a step of single tokens is faster in one launch than in those it stands for (the bits are the same): us of a layer in one /
+        in several, heads of 128 x 64 in 8 groups, selective.  64 heads, 256 KB of state a workgroup, 1, 2, 3, 4, 8 and 24 sequences: 16.5/15.1, 18.4/18.1,
+        20.7/20.4, 21.3/21.6, 23.7/26.4, 38.5/54.4; 32 heads 12.6/13.9 with one sequence.  The delta rule replaces a launch more: 32 heads
+        of 128 x 128 on 8 (256 KB as well) 16.2/17.7 with one sequence."""
+        return mode != "selective" or n_heads // n_kv * vdim * dim < 1 << 16 or n_seqs * n_kv >= 32
+
     def recurrence_step(self, mode: str, q, k, v, n_heads: int, n_kv: int, dim: int, vdim: int, a, a_per_head: bool, decay: int,
                         state: torch.Tensor, ctx, gate, gate_act: int, norm: torch.Tensor, eps: float, out: torch.Tensor,
                         conv=None, a_bias=None, a_log=None, tau: float = 1.0, b=None, bonus=None, d=None, unit: bool = False,

@@ -101,7 +101,7 @@ class StateSpace(Part):
     def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None) -> torch.Tensor:
         lib, t = self.env.lib, h.shape[0]
         proj = linear(lib, h, self.w_in, torch.float32)                       # [T, z | x | k | q | t]
-        if self.one_launch and ctx.max_q_len == 1:
+        if self.one_launch and ctx.max_q_len == 1 and lib.recurrence_step_pays("selective", self.heads, self.groups, self.state, self.vdim, ctx.n_seqs):
             k_col = 2 * self.inner                                            # the convolution's channels are [x | k | q]
             q_col = k_col + self.groups * self.state
             yn = torch.empty((t, self.inner), dtype=self.env.dtype, device=h.device)

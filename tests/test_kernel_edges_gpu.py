@@ -1275,6 +1275,34 @@ def test_single_tokens_through_a_recurrence_in_one_launch_beside_launches_of_the
     assert not lib.recurrence_step_ok(2, 2, 96, 64) and not lib.recurrence_step_ok(2, 2, 64, 96) and not lib.recurrence_step_ok(9, 1, 64, 64)
 
 
+@pytest.mark.parametrize("units", [0, 1])
+@pytest.mark.parametrize("kind,params", ONE_LAUNCH + [("state_space", dict(heads=8, vdim=64, state=128, groups=1, conv=4, norm_groups=n, eps=1e-5)) for n in (2, 8)])
+def test_single_tokens_through_a_recurrence_in_one_launch_give_the_same_bits(lib, kind, params, units, monkeypatch):
+    """Sums are taken in the order of the launches that this one stands for, by whichever number of lanes those deal a column to (units:
+    how many compute units decide that; 1: as if the sequences filled the GPU)."""
+    gen = torch.Generator().manual_seed(5)
+    monkeypatch.setattr(type(lib), "recurrence_step_pays", staticmethod(lambda *a: True))
+    part = build_part("mixer", PartSpec(kind, params), BuildEnv(hidden_size=64, dtype=torch.float32, device=torch.device(DEV), lib=lib))
+    part.load({n: (torch.randn(ts.shape, generator=gen) * (0.5 if len(ts.shape) < 2 or min(ts.shape) < 8 else ts.shape[-1] ** -0.5)).to(DEV)
+               for n, ts in part.tensor_specs().items()})
+    cache = Cache([part.cache_requests()], 3, 64, torch.float32, DEV)
+    slots, h = [cache.alloc_slot() for _ in range(3)], torch.randn(3, 64, generator=gen).to(DEV)
+    states = [torch.randn(g.data.shape, generator=gen).to(DEV) * 0.3 for g in cache.state_groups]
+    ctx = StepContext.for_batch(DEV, StepBatch(slots, [0] * 3, [[1]] * 3, [0, 1, 2], {}), n_compute_units=lib.n_compute_units)
+    got = []
+    try:
+        lib._lib.rb_tune_compute_units(units)
+        for one in (True, False):
+            part.one_launch = one
+            for g, s in zip(cache.state_groups, states):
+                g.data.copy_(s)
+            got.append([part.forward(h, ctx, cache.view(0, {}))] + [g.data[:, slots].clone() for g in cache.state_groups])
+    finally:
+        lib._lib.rb_tune_compute_units(0)
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 # ---------------------------------------------------------------------------- the router's product and the choice in one launch
 @pytest.mark.parametrize("n", [1, 3, 16])
 @pytest.mark.parametrize("rows,outputs,experts,top,k", [(16, 16, 16, 4, 2048), (17, 16, 16, 2, 1024), (8, 8, 8, 8, 1152), (64, 64, 64, 6, 1280),
