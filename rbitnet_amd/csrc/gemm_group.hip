@@ -3,8 +3,9 @@
 // from; a large product and the low-rank one beside it) were launches one after the other, and a product of 16 to 1,024 rows with 4 tokens at
 // K = 2048 costs 3.8 to 5 us whatever it reads (4 MB: 0.6 us of memory's time): its boundary, two trips to memory, the waves' sums.
 // The same kernel as gemm_skinny_kernel with one row tile a wave: K / 128 stages dealt to the waves in a row, sums through LDS in their order.
+// Sums are those of a product alone: each has the waves that it would have by itself.
 // Measured in captured steps of 4 tokens: 6,160 and 256 rows 6.8 + 4.3 us in two launches, 6.6 in one; five of 1,024 and 64 rows and the tanh behind the
-// last, 19 + 10 us in six launches, 4.2 in one.
+// last, 19 + 10 us in six launches, 4.2 in one.  In a chain of launches that read W from memory, 4 tokens, K = 2048: 7.2 for 10.4, 6.8 for 20.2.
 #include "api.h"
 #include "gemm_internal.h"
 
@@ -15,15 +16,17 @@ enum { END_F32 = 0, END_BF16 = 1, END_TANH = 2 };          // tanh: bfloat16(tan
 struct Group {
   RbGroupProduct p[MOST];
   int end[MOST];                                            // row tiles up to and with this product
+  int waves[MOST];                                          // of a workgroup of it, as if it were alone
   int count;
 };
 
 template <bool WF>
 __global__ __launch_bounds__(512) void gemm_group_kernel(const Group g, int m, int k) {
   extern __shared__ __attribute__((aligned(16))) float red[];      // [waves - 1][64] pieces of four sums
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6, r = lane & 15, kq = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, kq = lane >> 4;
   int i = 0;
   while (i + 1 < g.count && (int)blockIdx.x >= g.end[i]) ++i;
+  const int n_waves = g.waves[i];
   const RbGroupProduct p = g.p[i];
   const int n0 = 16 * ((int)blockIdx.x - (i > 0 ? g.end[i - 1] : 0));
   const bf16_t* w = (const bf16_t*)p.w;
@@ -44,14 +47,16 @@ __global__ __launch_bounds__(512) void gemm_group_kernel(const Group g, int m, i
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc = mfma16(a[j], b[j], acc);
   };
-  load_stage(0);                                            // (the host launches no more waves than stages)
-  for (int st = 1; st < stages; ++st) {
+  if (wave < n_waves) {                                     // (the host gives a product no more waves than stages)
+    load_stage(0);
+    for (int st = 1; st < stages; ++st) {
+      multiply_stage();
+      load_stage(st);
+    }
     multiply_stage();
-    load_stage(st);
   }
-  multiply_stage();
-  if (n_waves > 1) {
-    if (wave > 0) *reinterpret_cast<f32x4_t*>(red + (wave - 1) * 256 + 4 * lane) = acc;
+  if (blockDim.x > 64) {
+    if (wave > 0 && wave < n_waves) *reinterpret_cast<f32x4_t*>(red + (wave - 1) * 256 + 4 * lane) = acc;
     __syncthreads();
     if (wave > 0) return;
     for (int v = 0; v < n_waves - 1; ++v) acc += *reinterpret_cast<const f32x4_t*>(red + v * 256 + 4 * lane);
@@ -85,8 +90,15 @@ __global__ __launch_bounds__(512) void gemm_group_kernel(const Group g, int m, i
 
 }  // namespace
 
-// Whether m tokens of depth k go in one launch (more tokens have kernels that deal a product's tiles out better).
+// Whether m tokens of depth k can go in one launch (more tokens have kernels that deal a product's tiles out better).
 extern "C" int rb_gemm_bf16_group_ok(int m, int k) { return m >= 1 && m <= 16 && k >= 128 && k % 128 == 0; }
+
+// Whether a product of n rows is as fast among others as alone, and the same bits: where it has one row tile a wave alone as well, or as many
+// waves with more of them.  Groups / their products one after another, 1 and 16 tokens: K = 4096, 6,160 and 256 rows 11.6/15.0 and 13.7/20.4 us, 4,096 twice
+// 13.5/15.0 and 14.6/16.9, 64 twice 5.5/10.0 and 7.3/13.6; K = 8192, 8,192 and 1,024 rows 30.9/41.0 and 36.6/44.6; K = 256, five of 1,024 and 64 3.4/11.4 and
+// 3.6/12.5.  Left out: K = 5120 with 16,384 rows twice (four row tiles a wave alone) 54.5/55.5 and 69.0/56.1, and 3584 or 4096 with more than
+// 8,192 rows (resident tokens: other sums) 43.8/47.6 and 52.4/52.3.
+extern "C" int rb_gemm_bf16_group_pays(int m, int n, int k) { return rb_gemm_bf16_group_ok(m, k) && n > 0 && gemm_sums_alone_alike(m, n, k); }
 
 extern "C" int rb_gemm_bf16_group(const RbGroupProduct* products, int count, int w_layout, int m, int k, void* stream) {
   RB_REQUIRE(products != nullptr && count >= 1 && count <= MOST, "rb_gemm_bf16_group: %d products (1 to %d)", count, MOST);
@@ -108,10 +120,12 @@ extern "C" int rb_gemm_bf16_group(const RbGroupProduct* products, int count, int
     g.end[i] = (int)tiles;
   }
   if (m == 0) return 0;
-  // as for a product alone (gemm_skinny.hip): 8 waves where a compute unit has about one workgroup, 4 where it has more (4 tokens, K = 2048,
-  // 256 tiles 5.7 us with 8 and 6.0 with 4; 385 tiles 8.0 and 7.3), and 8 where K is long
-  int waves = k >= 8192 || 4 * tiles <= 5LL * rb_compute_units() ? 8 : 4;
-  if (waves > k / 128) waves = k / 128;
+  // every product has the waves that it has alone with one row tile a wave; the others of its workgroups wait at the barrier
+  int waves = 1;
+  for (int i = 0; i < count; ++i) {
+    g.waves[i] = gemm_skinny_waves(g.p[i].n, k);
+    if (g.waves[i] > waves) waves = g.waves[i];
+  }
   const size_t lds = (size_t)(waves - 1) * 256 * sizeof(float);
   if (w_layout) gemm_group_kernel<true><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
   else gemm_group_kernel<false><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);

@@ -43,6 +43,12 @@ int gemm_skinny_launch(const GemmTokens& x, const bf16_t* w, void* c, int dtype_
 // sizes are not for it and nothing was launched
 bool gemm_resident_try(const GemmTokens& x, const bf16_t* w, void* c, int dtype_out, const GemmAfter& after, int m,
                        int n, int k, hipStream_t s, int* rc);
+bool gemm_resident_takes(int m, int k, int parts);
+// For several products in one launch (gemm_group.hip), K % 128 == 0: the waves that share K with one row tile a wave, and whether a product
+// alone takes its sums in that order (the same waves, whatever row tiles each has, and not the kernel with resident tokens).
+int gemm_skinny_waves(int n, int k);
+bool gemm_skinny_waves_alone(int n, int k);
+bool gemm_sums_alone_alike(int m, int n, int k);
 // more than 16 tokens (more than 64 when K is no multiple of 64): tiles through LDS
 // (gemm_tiled.hip).  gemm_tiled_parts: 0 when these sizes are not for it, else the number of K
 // slices it will use; more than 1 needs parts * m * n floats of workspace.  own_sum: the slices are added up by a launch

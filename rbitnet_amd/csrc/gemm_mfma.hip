@@ -27,11 +27,17 @@ extern "C" long long rb_gemm_workspace_floats(int m, int n, int k, int epilogue)
   return p > 1 ? (long long)p * m * n : 0;
 }
 
+static bool resident_first(int m, int n) { return g_use_resident && m <= 16 && (n > 8192 || g_use_resident == 2); }
+
+bool gemm_sums_alone_alike(int m, int n, int k) {
+  return m <= 16 && k % 128 == 0 && gemm_skinny_waves_alone(n, k) && !(resident_first(m, n) && gemm_resident_takes(m, k, 1));
+}
+
 // products that no tiled kernel takes: the two kernels of gemm_skinny.hip
 static int launch_few_tokens(const GemmTokens& x, const bf16_t* w, void* c, int dtype_out, const GemmAfter& after,
                              int m, int n, int k, hipStream_t s) {
   int rc = 0;
-  if (g_use_resident && m <= 16 && (n > 8192 || g_use_resident == 2) &&
+  if (resident_first(m, n) &&
       gemm_resident_try(x, w, c, dtype_out, after, m, n, k, s, &rc))
     return rc;
   return gemm_skinny_launch(x, w, c, dtype_out, after, m, n, k, s);

@@ -398,19 +398,21 @@ static int launch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const Ge
 // waves beat 8 at K = 4096, 8 beat 4 at K = 14336.  (With W fragment-major again: launched alone, products
 // with K = 8192 and more gain up to 10 % from two or four stages in flight; the decode steps they belong to
 // lose 4-6 % at the 8B and 70B shapes and gain 1-2 % at hidden sizes of 2,048 and 3,072.  One stage it stays.)
+static int skinny_waves(int n, int k, int r, int max_waves) {
+  const long long wgs = (n + 16 * r - 1) / (16 * r);
+  // 8 waves where K is long, or where every compute unit gets one workgroup at most and so needs
+  // more loads in flight of its own (4,096 rows at K = 4096: 8.1-8.3 us against 8.6-9.0 with 4);
+  // 4 where several workgroups share a compute unit (6,144 rows: 10.7 against 11.6 with 8)
+  int nw = g_tune_waves ? g_tune_waves : ((k >= 8192 || wgs <= rb_compute_units() || max_waves < 4) ? max_waves : 4);
+  if (nw > max_waves) nw = max_waves;
+  return nw > k / 128 ? k / 128 : nw;
+}
 template <int MB, int R, int EPI, typename TO, bool SCALED>
 static int launch_skinny_u(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
                            hipStream_t s) {
   constexpr int max_waves = (R * MB <= 4) ? 8 : (R * MB <= 8 ? 4 : 3);      // bounds the reduction buffer
   if (k % 128 == 0) {
-    const int t = k / 128;
-    // 8 waves where K is long, or where every compute unit gets one workgroup at most and so needs
-    // more loads in flight of its own (4,096 rows at K = 4096: 8.1-8.3 us against 8.6-9.0 with 4);
-    // 4 where several workgroups share a compute unit (6,144 rows: 10.7 against 11.6 with 8)
-    const long long wgs = (n + 16 * R - 1) / (16 * R);
-    int nw = g_tune_waves ? g_tune_waves : ((k >= 8192 || wgs <= rb_compute_units() || max_waves < 4) ? max_waves : 4);
-    if (nw > max_waves) nw = max_waves;
-    if (nw > t) nw = t;
+    const int nw = skinny_waves(n, k, R, max_waves);
     return launch_skinny<MB, R, true, EPI, TO, SCALED>(x, w, c, after, m, n, k, nw, 0, s);
   }
   int n_waves = k / 256;
@@ -421,31 +423,25 @@ static int launch_skinny_u(const GemmTokens& x, const bf16_t* w, void* c, const 
   return launch_skinny<MB, R, false, EPI, TO, SCALED>(x, w, c, after, m, n, k, n_waves, k_per_wave, s);
 }
 
-template <int EPI, typename TO, bool SCALED>
-static int dispatch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
-                           hipStream_t s) {
-  constexpr bool FOLDS = SCALED || EPI == 2 || EPI == 3;      // compiled for up to 16 tokens only
-  const int mb = (m + 15) / 16;
-  RB_REQUIRE(!FOLDS || mb == 1, "rb_gemm_bf16: a product that folds its neighbours in takes at most 16 tokens, not %d",
-             m);
-  // Row tiles of W per wave (16 R rows per workgroup).  Up to K = 4096 (workgroups of 4 waves, several
-  // of which share a compute unit) one tile per wave is the fastest at every N from 1024 to 16384
-  // (measured with 8 tokens, W fragment-major; N = 6144: 11.1 us against 13.5 with two).  From
-  // K = 8192 on (8 waves) more tiles reuse the token operand better and fewer deal the rows to the 256
-  // compute units more evenly: the time goes with the rows that the busiest compute unit gets, at
-  // a price per row that falls with R (about 15 % / R).  57344 rows at K = 8192: R = 4 gives 896
-  // workgroups, 4 on some compute units and 3 on others, 194 us; R = 2 gives every one 7: 175 us.
-  // 10240 rows at K = 8192 with one token: R = 1 35 us, R = 2 42; R = 4 takes 31 us by itself (160
-  // workgroups), but the decode step of that shape is no faster with it (+0.3 % at batch 1, +0.5 % at
-  // 8, -1.1 % at 16, each the mean of four runs in alternating order), so it is not taken.
-  // Between K = 4096 and 8192 the same estimate holds: 15,360 rows at K = 5120 with 16 tokens 26.6 us
-  // with R = 4 against 33.6 with R = 1 (8 tokens: 26.4 against 27.5, one token 26.9 against 26.5),
-  // 5,120 rows 13.6 with R = 2 against 16.8 (8 tokens: 12.1 against 13.4).
+// Row tiles of W per wave (16 R rows per workgroup).  Up to K = 4096 (workgroups of 4 waves, several
+// of which share a compute unit) one tile per wave is the fastest at every N from 1024 to 16384
+// (measured with 8 tokens, W fragment-major; N = 6144: 11.1 us against 13.5 with two).  From
+// K = 8192 on (8 waves) more tiles reuse the token operand better and fewer deal the rows to the 256
+// compute units more evenly: the time goes with the rows that the busiest compute unit gets, at
+// a price per row that falls with R (about 15 % / R).  57344 rows at K = 8192: R = 4 gives 896
+// workgroups, 4 on some compute units and 3 on others, 194 us; R = 2 gives every one 7: 175 us.
+// 10240 rows at K = 8192 with one token: R = 1 35 us, R = 2 42; R = 4 takes 31 us by itself (160
+// workgroups), but the decode step of that shape is no faster with it (+0.3 % at batch 1, +0.5 % at
+// 8, -1.1 % at 16, each the mean of four runs in alternating order), so it is not taken.
+// Between K = 4096 and 8192 the same estimate holds: 15,360 rows at K = 5120 with 16 tokens 26.6 us
+// with R = 4 against 33.6 with R = 1 (8 tokens: 26.4 against 27.5, one token 26.9 against 26.5),
+// 5,120 rows 13.6 with R = 2 against 16.8 (8 tokens: 12.1 against 13.4).
+static int skinny_rows(int n, int k, bool pairs) {
   int r = 1;
   if (k > 4096) {
     double best = 0.0;
     const long long cus = rb_compute_units();
-    for (int cand = (EPI == 1 ? 2 : 1); cand <= 4; cand *= 2) {
+    for (int cand = (pairs ? 2 : 1); cand <= 4; cand *= 2) {
       const long long wgs = (n + 16 * cand - 1) / (16 * cand);
       const double cost = (double)((wgs + cus - 1) / cus * 16 * cand) * (1.0 + 0.15 / cand);
       if (best == 0.0 || cost <= best) {
@@ -455,7 +451,20 @@ static int dispatch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const 
     }
   }
   if (g_tune_r) r = g_tune_r;
-  if (EPI == 1 && r < 2) r = 2;
+  return pairs && r < 2 ? 2 : r;
+}
+
+int gemm_skinny_waves(int n, int k) { return skinny_waves(n, k, 1, 8); }
+bool gemm_skinny_waves_alone(int n, int k) { return skinny_waves(n, k, skinny_rows(n, k, false), 8) == skinny_waves(n, k, 1, 8); }
+
+template <int EPI, typename TO, bool SCALED>
+static int dispatch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
+                           hipStream_t s) {
+  constexpr bool FOLDS = SCALED || EPI == 2 || EPI == 3;      // compiled for up to 16 tokens only
+  const int mb = (m + 15) / 16;
+  RB_REQUIRE(!FOLDS || mb == 1, "rb_gemm_bf16: a product that folds its neighbours in takes at most 16 tokens, not %d",
+             m);
+  const int r = skinny_rows(n, k, EPI == 1);
 #define RB_SK(MBV, RV) return launch_skinny_u<MBV, RV, EPI, TO, SCALED>(x, w, c, after, m, n, k, s)
   if (mb == 1) {
     if (r == 4) RB_SK(1, 4);
@@ -684,23 +693,26 @@ static int launch_resident(const GemmTokens& x, const bf16_t* w, void* c, const 
   return 0;
 }
 
+static int resident_depth(int m) { return m <= 16 ? 16 : (m <= 32 ? 8 : 4); }      // XQ
+
+bool gemm_resident_takes(int m, int k, int parts) {
+  const int each = 32 * resident_depth(m);
+  if (k % each != 0 || parts < 1 || k / each % parts != 0) return false;
+  const int n_waves = k / each / parts;
+  // With fewer than 7 waves a workgroup has too few loads in flight for the one compute unit it has to
+  // itself, and the skinny kernel, several workgroups to a compute unit, is faster (32,768 gated rows at
+  // K = 2048: 12.4 us against 13.8 with 4 waves; at K = 3072: 17.3 against 18.4 with 6); forced on
+  // (rb_tune_use_resident(2)) it still takes them.
+  return n_waves <= 8 && (n_waves >= 7 || g_res_forced != 0);
+}
+
 // true if the resident kernel takes these sizes
 template <int EPI, typename TO, bool SCALED>
 static bool try_resident(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
                          int parts, hipStream_t s, int* rc) {
   constexpr bool FOLDS = SCALED || EPI == 2 || EPI == 3;      // compiled for up to 16 tokens and all of K in one workgroup
   const int mb = (m + 15) / 16;
-  const int xq = mb == 1 ? 16 : (mb == 2 ? 8 : 4);
-  if (k % (32 * xq) != 0) return false;
-  const int slices = k / (32 * xq);
-  if (parts < 1 || slices % parts != 0) return false;
-  const int n_waves = slices / parts;
-  if (n_waves > 8) return false;
-  // With fewer than 7 waves a workgroup has too few loads in flight for the one compute unit it has to
-  // itself, and the skinny kernel, several workgroups to a compute unit, is faster (32,768 gated rows at
-  // K = 2048: 12.4 us against 13.8 with 4 waves; at K = 3072: 17.3 against 18.4 with 6); forced on
-  // (rb_tune_use_resident(2)) it still takes them.
-  if (n_waves < 7 && g_res_forced == 0) return false;
+  if (!gemm_resident_takes(m, k, parts)) return false;
   if (EPI == 1 && (n % 32 != 0)) return false;
   if (FOLDS && (mb != 1 || parts != 1)) return false;
   if (mb == 1) {

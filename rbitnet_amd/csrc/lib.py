@@ -191,6 +191,7 @@ class Kernels:
             "rb_streams_rmsnorm": [_P, _I, _L, _P, _P, _P, _I, _L, _L, _P, _P, _I, _L, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_short_conv_biases": [_P, _L, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
             "rb_gemm_bf16_group_ok": [_I, _I],
+            "rb_gemm_bf16_group_pays": [_I, _I, _I],
             "rb_gemm_bf16_group": [ctypes.POINTER(GroupProduct), _I, _I, _I, _I, _P],
             "rb_recurrence_step_ok": [_I, _I, _I, _I, _I, _I],
             "rb_recurrence_step": [ctypes.POINTER(RecurrenceStep), _P],
@@ -405,6 +406,9 @@ class Kernels:
 
     def gemm_bf16_group_ok(self, m: int, k: int) -> bool:
         return bool(self._lib.rb_gemm_bf16_group_ok(int(m), int(k)))
+
+    def gemm_bf16_group_pays(self, m: int, n: int, k: int) -> bool:
+        return bool(self._lib.rb_gemm_bf16_group_pays(int(m), int(n), int(k)))
 
     def gemm_bf16_terms_count(self, m: int, n: int, k: int) -> int:
         return int(self._lib.rb_gemm_bf16_terms_count(int(m), int(n), int(k)))

@@ -1462,3 +1462,34 @@ def test_products_in_one_launch(lib, m, k, rows, frag):
     for (_, _, c, _), (want, bound) in zip(products, wants):
         _within(c, want, bound)
     assert not lib.gemm_bf16_group_ok(17, 128) and not lib.gemm_bf16_group_ok(4, 192)
+
+
+@pytest.mark.parametrize("m", [1, 16])
+@pytest.mark.parametrize("k,rows", [(128, (16, 4112)), (2048, (6160, 256, 1024)), (4096, (4096, 4112, 64)), (4096, (8192, 8208)), (5120, (5120, 1024)),
+                                    (8192, (4112, 16))])
+def test_products_in_one_launch_give_the_bits_of_each_alone(lib, m, k, rows):
+    """Wherever a product is said to gain among others its sums are those it has alone, on either side of as many row tiles as compute
+    units; what is left out (other row tiles a wave, resident tokens) goes alone."""
+    gen = torch.Generator(device=DEV).manual_seed(k + m)
+    x = torch.randn(m, k, generator=gen, device=DEV).bfloat16()
+    ws = [torch.randn(n, k, generator=gen, device=DEV).bfloat16() for n in rows]
+    pays = [lib.gemm_bf16_group_pays(m, n, k) for n in rows]
+    if k in (128, 2048, 8192):
+        assert all(pays)
+    assert lib.gemm_bf16_group_pays(m, 8192, 4096) and not lib.gemm_bf16_group_pays(m, 8208, 4096)
+    assert not lib.gemm_bf16_group_pays(17, 64, 2048) and not lib.gemm_bf16_group_pays(m, 64, 192)
+    alone, ends = [], ["float32", "bfloat16", "tanh"]
+    for w in ws:
+        c = torch.empty(m, w.shape[0], device=DEV)
+        lib.gemm_bf16(x, w, c, 0)
+        alone.append(c)
+    end = lambda i: "float32" if not pays[i] else ends[i % 3]
+    got = [torch.empty(m, w.shape[0], dtype=torch.float32 if end(i) == "float32" else torch.bfloat16, device=DEV) for i, w in enumerate(ws)]
+    lib.gemm_bf16_group([(x, w, c, end(i)) for i, (w, c) in enumerate(zip(ws, got))], False)
+    for i, (c, a) in enumerate(zip(got, alone)):
+        if not pays[i]:
+            continue
+        if end(i) == "tanh":
+            z, a = a, torch.empty_like(c)
+            lib.tanh_cast(z, a)
+        assert torch.equal(c, a.to(c.dtype)), rows[i]
