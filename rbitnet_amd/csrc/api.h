@@ -274,12 +274,6 @@ struct RbRecurrenceStep {
 };
 int rb_recurrence_step_ok(int n_heads, int n_kv_heads, int dim, int vdim, int taps, int norm_part);
 int rb_recurrence_step(const struct RbRecurrenceStep* args, void* stream);
-// Steps of many tokens through the same recurrence (modes 0, 1, 2; q, k, v behind the convolution, a and b as they come from the
-// projections) in chunks of 16 tokens, `window` chunks of every sequence at a time; its outputs [T, H, vdim] float32 to o.
-int rb_recurrence_chunks_ok(int n_heads, int n_kv_heads, int dim, int vdim);
-long long rb_recurrence_chunks_floats(int n_seqs, int n_heads, int dim, int vdim, int chunks);
-int rb_recurrence_chunks(const struct RbRecurrenceStep* args, const int32_t* cu_seqlens, int n_seqs, int chunks, int window, float* ws, float* o,
-                         void* stream);
 // A selective scan, token after token, on the state S kept column by column as [slots, H, vdim, dim]; with
 // dt = softplus(dt_in[t * dt_stride + h] + dt_bias[h]):
 //   S <- exp(-exp(a_log[h]) dt) S + dt k v^T;  out[t, h, :] = S^T q + d[h] v      (head h reads the q and k of group h / (H / G))

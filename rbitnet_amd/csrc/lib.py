@@ -105,7 +105,7 @@ class KernelTimes:
         return "\n".join(lines)
 
 
-TIMED_OPS = ("routed_experts_tiled", "recurrence_step", "recurrence_chunks", "gemm_bf16_group", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
+TIMED_OPS = ("routed_experts_tiled", "recurrence_step", "gemm_bf16_group", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
              "route_top", "routed_experts", "pairs_sum", "embed_streams", "streams_layernorm", "streams_update", "xielu", "tanh_cap", "short_conv",
              "delta_prep", "delta_rule", "gated_rmsnorm", "latent_norm_store", "attention_sinks", "embed_gather", "add_rmsnorm", "rope_kv_write", "swiglu", "gemm_generic", "gemm_bf16", "gemm_bf16_terms",
              "gemm_bf16_few", "attention_generic", "attention_prefill_bf16", "attention_decode_bf16",
@@ -126,7 +126,6 @@ class RecurrenceStep(ctypes.Structure):
                                      "dim", "vdim")])
 
 
-RECURRENCE_WORKSPACE = 256 << 20         # bytes of a chunked recurrence's operands at a time
 class GroupProduct(ctypes.Structure):
     """RbGroupProduct of csrc/api.h."""
     _fields_ = [("x", _P), ("w", _P), ("c", _P), ("n", _I), ("end", _I)]
@@ -195,8 +194,6 @@ class Kernels:
             "rb_gemm_bf16_group": [ctypes.POINTER(GroupProduct), _I, _I, _I, _I, _P],
             "rb_recurrence_step_ok": [_I, _I, _I, _I, _I, _I],
             "rb_recurrence_step": [ctypes.POINTER(RecurrenceStep), _P],
-            "rb_recurrence_chunks_ok": [_I, _I, _I, _I],
-            "rb_recurrence_chunks": [ctypes.POINTER(RecurrenceStep), _P, _I, _I, _I, _P, _P, _P],
             "rb_selective_scan": [_P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
             "rb_selective_chunks_ok": [_I, _I],
             "rb_selective_chunks": [_P, _P, _P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
@@ -267,8 +264,6 @@ class Kernels:
         L.rb_plan_free.argtypes, L.rb_plan_free.restype = [_P], None
         L.rb_selective_chunks_floats.argtypes = [_I, _I, _I, _I, _I]
         L.rb_selective_chunks_floats.restype = ctypes.c_longlong
-        L.rb_recurrence_chunks_floats.argtypes = [_I, _I, _I, _I, _I]
-        L.rb_recurrence_chunks_floats.restype = ctypes.c_longlong
         L.rb_gemm_workspace_floats.argtypes = [_I, _I, _I, _I]
         L.rb_gemm_workspace_floats.restype = ctypes.c_longlong
         L.rb_sample_workspace_bytes.argtypes = [_I, _I]
@@ -822,39 +817,7 @@ class Kernels:
         self._ok(self._lib.rb_gated_rmsnorm(_ptr(o), _ptr(weight), gate.data_ptr() + 4 * gate_col, gate.shape[1], float(eps),
                                             _ptr(out), dtype_code(out.dtype), n, n_heads, vdim, self._stream()))
 
-    # ------------------------------------------------------------------ recurrences with what enters them
-    def _recurrence(self, mode: str, q, k, v, n_heads: int, n_kv: int, dim: int, vdim: int, a, a_per_head: bool, decay: int,
-                    state: torch.Tensor, ctx, a_bias, a_log, tau, b, bonus, d, unit: bool, q_scale: float, unit_eps: float):
-        """The arguments that a step of single tokens and one in chunks share, checked, and the function that checks a part of a row."""
-        n = ctx.n_tokens
-
-        def part(pair, width, what):
-            m, col = pair
-            _check(m, what, torch.float32)
-            if m.shape[0] != n or col < 0 or col + width > m.shape[1]:
-                raise KernelError(f"recurrence: the columns of {what} lie outside the rows")
-            return m.data_ptr() + 4 * col, m.shape[1]
-
-        r = RecurrenceStep(mode=STEP_MODES[mode], unit=int(bool(unit)), a_per_head=int(bool(a_per_head)), decay=int(decay), n_tokens=n,
-                           n_heads=n_heads, n_kv_heads=n_kv, dim=dim, vdim=vdim, tau=float(tau), q_scale=float(q_scale),
-                           unit_eps=float(unit_eps))
-        r.q, r.q_stride = part(q, n_kv * dim, "q")
-        r.k, r.k_stride = part(k, n_kv * dim, "k")
-        r.v, r.v_stride = part(v, n_heads * vdim, "v")
-        n_a = n_heads if a_per_head or mode == "selective" else n_heads * dim
-        r.a, r.a_stride = part(a, n_a, "a")
-        if b is not None:
-            r.b, r.b_stride = part(b, n_heads, "b")
-        for name, t, shape in (("a_bias", a_bias, (n_a,)), ("a_log", a_log, (n_heads,)), ("bonus", bonus, (n_heads, dim)), ("d", d, (n_heads,))):
-            if t is not None:
-                _check(t, name, torch.float32, shape)
-                setattr(r, name, _ptr(t))
-        _check(state, "state", torch.float32)
-        if tuple(state.shape[1:]) != (n_heads, vdim, dim):
-            raise KernelError(f"recurrence: state of shape {tuple(state.shape)}, expected [*, {n_heads}, {vdim}, {dim}]")
-        r.state, r.slots = _ptr(state), _ptr(ctx.slots)
-        return r, part
-
+    # ------------------------------------------------------------------ a step of single tokens, in one launch
     def recurrence_step_ok(self, n_heads: int, n_kv: int, dim: int, vdim: int, taps: int = 0, norm_part: int = 0) -> bool:
         return bool(self._lib.rb_recurrence_step_ok(n_heads, n_kv, dim, vdim, taps, norm_part))
 
@@ -876,10 +839,31 @@ class Kernels:
         n = out.shape[0]
         if ctx.n_tokens != n or ctx.n_seqs != n:
             raise KernelError("recurrence_step: a step of one token per sequence")
-        r, part = self._recurrence(mode, q, k, v, n_heads, n_kv, dim, vdim, a, a_per_head, decay, state, ctx, a_bias, a_log, tau, b, bonus, d,
-                                   unit, q_scale, unit_eps)
-        r.gate_act, r.norm_part, r.out_dtype, r.eps = int(gate_act), int(norm_part), dtype_code(out.dtype), float(eps)
+
+        def part(pair, width, what):
+            m, col = pair
+            _check(m, what, torch.float32)
+            if m.shape[0] != n or col < 0 or col + width > m.shape[1]:
+                raise KernelError(f"recurrence_step: the columns of {what} lie outside the rows")
+            return m.data_ptr() + 4 * col, m.shape[1]
+
+        r = RecurrenceStep(mode=STEP_MODES[mode], unit=int(bool(unit)), a_per_head=int(bool(a_per_head)), decay=int(decay),
+                           gate_act=int(gate_act), norm_part=int(norm_part), out_dtype=dtype_code(out.dtype), n_tokens=n, n_heads=n_heads,
+                           n_kv_heads=n_kv, dim=dim, vdim=vdim, tau=float(tau), q_scale=float(q_scale), unit_eps=float(unit_eps),
+                           eps=float(eps))
+        r.q, r.q_stride = part(q, n_kv * dim, "q")
+        r.k, r.k_stride = part(k, n_kv * dim, "k")
+        r.v, r.v_stride = part(v, n_heads * vdim, "v")
         r.gate, r.gate_stride = part(gate, n_heads * vdim, "gate")
+        per_head = a_per_head or mode == "selective"
+        n_a = n_heads if per_head else n_heads * dim
+        r.a, r.a_stride = part(a, n_a, "a")
+        if b is not None:
+            r.b, r.b_stride = part(b, n_heads, "b")
+        for name, t, shape in (("a_bias", a_bias, (n_a,)), ("a_log", a_log, (n_heads,)), ("bonus", bonus, (n_heads, dim)), ("d", d, (n_heads,))):
+            if t is not None:
+                _check(t, name, torch.float32, shape)
+                setattr(r, name, _ptr(t))
         if conv is not None:
             w, bias_out, conv_state, cq, ck, cv = conv
             channels, taps = w.shape
@@ -894,6 +878,9 @@ class Kernels:
                 raise KernelError("recurrence_step: q, k or v lie outside the convolution's channels")
             r.conv_w, r.conv_bias, r.conv_state = _ptr(w), _ptr(bias_out), _ptr(conv_state) if taps > 1 else None
             r.taps, r.conv_channels, r.conv_q, r.conv_k, r.conv_v = taps, channels, cq, ck, cv
+        _check(state, "state", torch.float32)
+        if tuple(state.shape[1:]) != (n_heads, vdim, dim):
+            raise KernelError(f"recurrence_step: state of shape {tuple(state.shape)}, expected [*, {n_heads}, {vdim}, {dim}]")
         if norm_part == 0 and tuple(norm.shape) == (vdim,):
             r.norm_head_stride = 0
         else:
@@ -901,39 +888,8 @@ class Kernels:
             r.norm_head_stride = vdim
         _check(norm, "norm", torch.float32)
         _check(out, "out", None, (n, n_heads * vdim))
-        r.norm, r.out = _ptr(norm), _ptr(out)
+        r.state, r.slots, r.norm, r.out = _ptr(state), _ptr(ctx.slots), _ptr(norm), _ptr(out)
         self._ok(self._lib.rb_recurrence_step(ctypes.byref(r), self._stream()))
-
-    def recurrence_chunks_ok(self, n_heads: int, n_kv: int, dim: int, vdim: int) -> bool:
-        return bool(self._lib.rb_recurrence_chunks_ok(n_heads, n_kv, dim, vdim))
-
-    def recurrence_chunks_pay(self, mode: str, n_heads: int, dim: int, vdim: int, ctx) -> bool:
-        """Whether a step's recurrence is faster in chunks than walked (with the launch that makes its inputs): us walked / in chunks,
-        16 heads, longest piece 32, 48, 64, 128 and 1,000 tokens.  128 x 128, delta: 4 sequences 20/23, 26/24, 31/30, 55/39, 352/167;
-        16: 58/50, 80/52, 103/72, 188/114, 1372/806.  64 x 64, read before write: 4 sequences 11/12, 13/12, 16/14, 27/19, 192/81; 16
-        16/20, 21/23, 26/31, 45/43, 338/317.  64 x 64, delta: 4 sequences 13/17, 17/18, 20/21, 36/28, 238/142, but 16 sequences, whose
-        waves fill the GPU when they walk, 24/31, 32/34, 39/50, 60/74, 465/573: the chunks' operands then cost what the walk does."""
-        if mode == "delta" and dim == 64:
-            return ctx.max_q_len >= 96 and ctx.n_seqs * n_heads * vdim <= 8 * 4 * self.n_compute_units
-        return ctx.max_q_len >= 48
-
-    def recurrence_chunks(self, mode: str, q, k, v, n_heads: int, n_kv: int, dim: int, vdim: int, a, a_per_head: bool, decay: int,
-                          state: torch.Tensor, ctx, out: torch.Tensor, a_bias=None, a_log=None, tau: float = 1.0, b=None, bonus=None,
-                          unit: bool = False, q_scale: float = 1.0, unit_eps: float = 0.0, window: Optional[int] = None) -> None:
-        """Any number of tokens per sequence through the recurrence, with what enters it, in chunks of 16 tokens: out [T, heads * vdim]
-        float32.  q, k, v, a, b: (matrix [T, W] float32, first column), as they are before unit vectors, decays and beta.  window:
-        chunks of every sequence that the workspace holds at a time (None: as many as `RECURRENCE_WORKSPACE` bytes hold)."""
-        n = ctx.n_tokens
-        _check(out, "out", torch.float32, (n, n_heads * vdim))
-        _check(ctx.cu_seqlens, "cu_seqlens", torch.int32, (ctx.n_seqs + 1,))
-        r, _ = self._recurrence(mode, q, k, v, n_heads, n_kv, dim, vdim, a, a_per_head, decay, state, ctx, a_bias, a_log, tau, b, bonus, None,
-                                unit, q_scale, unit_eps)
-        chunks = (int(ctx.max_q_len) + 15) // 16
-        each = int(self._lib.rb_recurrence_chunks_floats(ctx.n_seqs, n_heads, dim, vdim, 1))
-        window = max(1, min(chunks, RECURRENCE_WORKSPACE // (4 * each) if window is None else int(window)))
-        ws = torch.empty(each * window, dtype=torch.float32, device=out.device)
-        self._ok(self._lib.rb_recurrence_chunks(ctypes.byref(r), _ptr(ctx.cu_seqlens), ctx.n_seqs, chunks, window, _ptr(ws), _ptr(out),
-                                                self._stream()))
 
     # ------------------------------------------------------------------ recurrences with their choices spelled out
     def recurrence_prep(self, qkv: torch.Tensor, n_kv: int, dim: int, unit: bool, q_scale: float, unit_eps: float,

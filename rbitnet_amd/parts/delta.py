@@ -40,11 +40,6 @@ def step_in_one_launch(env: BuildEnv, heads: int, kv_heads: int, dim: int, vdim:
             and env.lib.recurrence_step_ok(heads, kv_heads, dim, vdim, taps, norm_part))
 
 
-def steps_in_chunks(env: BuildEnv, heads: int, kv_heads: int, dim: int, vdim: int) -> bool:
-    """Whether steps of many tokens run in chunks (`recurrence_chunks`), with what enters the recurrence made on the way."""
-    return (env.lib is not None and not getattr(env, "generic_only", False) and env.lib.recurrence_chunks_ok(heads, kv_heads, dim, vdim))
-
-
 class ChannelDelta(Part):
     graph_safe = True
     plan_safe = True
@@ -68,7 +63,6 @@ class ChannelDelta(Part):
         self.n_conv = 2 * self.n_qk + self.n_v
         self.conv = ShortConv(self.n_conv, self.taps, env, residual=False, act=ACT_SILU)
         self.one_launch = step_in_one_launch(env, self.heads, self.kv_heads, self.dim, self.vdim, self.taps)
-        self.in_chunks = steps_in_chunks(env, self.heads, self.kv_heads, self.dim, self.vdim)
         self.cache_from = None
 
     # ------------------------------------------------------------------ tensors
@@ -134,16 +128,11 @@ class ChannelDelta(Part):
             return linear(lib, on, self.w_o, torch.float32)
         qkv = self.conv.forward(proj, ctx, view.states.get("conv"), torch.float32)
         n_a = self.heads * self.dim
+        beta = torch.empty((t, self.heads), dtype=torch.float32, device=h.device)
+        lib.delta_prep(qkv, self.kv_heads, self.dim, up, self.dt_bias, self.a_log, self.heads, proj, self.b_col, beta,
+                       self.dim ** -0.5, self.unit_eps)
         o = torch.empty((t, self.n_v), dtype=torch.float32, device=h.device)
-        if self.in_chunks and lib.recurrence_chunks_pay("delta", self.heads, self.dim, self.vdim, ctx):
-            lib.recurrence_chunks("delta", (qkv, 0), (qkv, self.n_qk), (qkv, 2 * self.n_qk), self.heads, self.kv_heads, self.dim, self.vdim,
-                                  (up, 0), False, 0, view.states["delta"], ctx, o, a_bias=self.dt_bias, a_log=self.a_log, b=(proj, self.b_col),
-                                  unit=True, q_scale=self.dim ** -0.5, unit_eps=self.unit_eps)
-        else:
-            beta = torch.empty((t, self.heads), dtype=torch.float32, device=h.device)
-            lib.delta_prep(qkv, self.kv_heads, self.dim, up, self.dt_bias, self.a_log, self.heads, proj, self.b_col, beta,
-                           self.dim ** -0.5, self.unit_eps)
-            lib.delta_rule(qkv, self.kv_heads, self.dim, self.heads, self.vdim, up, beta, view.states["delta"], ctx, o)
+        lib.delta_rule(qkv, self.kv_heads, self.dim, self.heads, self.vdim, up, beta, view.states["delta"], ctx, o)
         on = torch.empty((t, self.n_v), dtype=self.env.dtype, device=h.device)
         lib.gated_rmsnorm(o, self.norm, up, n_a, self.eps, self.heads, self.vdim, on)
         return linear(lib, on, self.w_o, torch.float32)
@@ -181,7 +170,6 @@ class HeadDelta(Part):
         self.n_conv = 2 * self.n_qk + self.n_v
         self.conv = ShortConv(self.n_conv, self.taps, env, residual=False, act=ACT_SILU)
         self.one_launch = step_in_one_launch(env, self.heads, self.kv_heads, self.dim, self.vdim, self.taps)
-        self.in_chunks = steps_in_chunks(env, self.heads, self.kv_heads, self.dim, self.vdim)
         self.cache_from = None
 
     def tensor_specs(self) -> Dict[str, TensorSpec]:
@@ -232,17 +220,12 @@ class HeadDelta(Part):
                                 unit_eps=self.unit_eps)
             return linear(lib, on, self.w_o, torch.float32)
         qkv = self.conv.forward(proj, ctx, view.states.get("conv"), torch.float32)
+        beta = torch.empty((t, self.heads), dtype=torch.float32, device=h.device)
+        lib.recurrence_prep(qkv, self.kv_heads, self.dim, True, self.dim ** -0.5, self.unit_eps, proj, c["a"], self.heads, 0,
+                            self.dt_bias, self.a_log, 1.0, self.heads, b_in=proj, b_col=c["b"], beta=beta)
         o = torch.empty((t, self.n_v), dtype=torch.float32, device=h.device)
-        if self.in_chunks and lib.recurrence_chunks_pay("delta", self.heads, self.dim, self.vdim, ctx):
-            lib.recurrence_chunks("delta", (qkv, 0), (qkv, self.n_qk), (qkv, 2 * self.n_qk), self.heads, self.kv_heads, self.dim, self.vdim,
-                                  (proj, c["a"]), True, 0, view.states["delta"], ctx, o, a_bias=self.dt_bias, a_log=self.a_log,
-                                  b=(proj, c["b"]), unit=True, q_scale=self.dim ** -0.5, unit_eps=self.unit_eps)
-        else:
-            beta = torch.empty((t, self.heads), dtype=torch.float32, device=h.device)
-            lib.recurrence_prep(qkv, self.kv_heads, self.dim, True, self.dim ** -0.5, self.unit_eps, proj, c["a"], self.heads, 0,
-                                self.dt_bias, self.a_log, 1.0, self.heads, b_in=proj, b_col=c["b"], beta=beta)
-            lib.linear_recurrence(qkv, self.kv_heads, self.dim, self.heads, self.vdim, proj, c["a"], True, beta,
-                                  view.states["delta"], ctx, o)
+        lib.linear_recurrence(qkv, self.kv_heads, self.dim, self.heads, self.vdim, proj, c["a"], True, beta,
+                              view.states["delta"], ctx, o)
         on = torch.empty((t, self.n_v), dtype=self.env.dtype, device=h.device)
         lib.gated_rmsnorm_act(o, self.norm, proj, c["g"], 1, self.eps, self.heads, self.vdim, on)
         return linear(lib, on, self.w_o, torch.float32)
@@ -275,7 +258,6 @@ class DecayAttention(Part):
         self.hidden = env.hidden_size
         self.n_qk, self.n_v = self.heads * self.dim, self.heads * self.vdim
         self.one_launch = step_in_one_launch(env, self.heads, self.heads, self.dim, self.vdim)
-        self.in_chunks = steps_in_chunks(env, self.heads, self.heads, self.dim, self.vdim)
         self.cache_from = None
 
     def tensor_specs(self) -> Dict[str, TensorSpec]:
@@ -325,14 +307,10 @@ class DecayAttention(Part):
                                 (z, 0), False, 1, view.states["decay"], ctx, (proj, c["g"]), 1, self.norm, self.eps, on,
                                 a_bias=self.a_bias, tau=self.tau, q_scale=self.dim ** -0.5)
             return linear(lib, on, self.w_o, torch.float32)
+        lib.recurrence_prep(proj, self.heads, self.dim, False, self.dim ** -0.5, 0.0, z, 0, self.n_qk, 1, self.a_bias, None,
+                            self.tau, self.heads)
         o = torch.empty((t, self.n_v), dtype=torch.float32, device=h.device)
-        if self.in_chunks and lib.recurrence_chunks_pay("plain", self.heads, self.dim, self.vdim, ctx):
-            lib.recurrence_chunks("plain", (proj, 0), (proj, self.n_qk), (proj, 2 * self.n_qk), self.heads, self.heads, self.dim, self.vdim,
-                                  (z, 0), False, 1, view.states["decay"], ctx, o, a_bias=self.a_bias, tau=self.tau, q_scale=self.dim ** -0.5)
-        else:
-            lib.recurrence_prep(proj, self.heads, self.dim, False, self.dim ** -0.5, 0.0, z, 0, self.n_qk, 1, self.a_bias, None,
-                                self.tau, self.heads)
-            lib.linear_recurrence(proj, self.heads, self.dim, self.heads, self.vdim, z, 0, False, None, view.states["decay"], ctx, o)
+        lib.linear_recurrence(proj, self.heads, self.dim, self.heads, self.vdim, z, 0, False, None, view.states["decay"], ctx, o)
         on = torch.empty((t, self.n_v), dtype=dt, device=h.device)
         lib.gated_rmsnorm_act(o, self.norm, proj, c["g"], 1, self.eps, self.heads, self.vdim, on)
         return linear(lib, on, self.w_o, torch.float32)
@@ -367,7 +345,6 @@ class TimeMix(Part):
         self.hidden = env.hidden_size
         self.n = self.heads * self.dim
         self.one_launch = step_in_one_launch(env, self.heads, self.heads, self.dim, self.dim)
-        self.in_chunks = steps_in_chunks(env, self.heads, self.heads, self.dim, self.dim)
         self.cache_from = None
 
     def tensor_specs(self) -> Dict[str, TensorSpec]:
@@ -406,13 +383,9 @@ class TimeMix(Part):
             lib.recurrence_step("bonus", (r, 0), (k, 0), (v, 0), self.heads, self.heads, self.dim, self.dim, (decay, 0), False, 2,
                                 view.states["time_mix"], ctx, (g, 0), 1, self.norm, self.eps, on, a_bias=self.w0, bonus=self.u)
             return linear(lib, on, self.w_o, torch.float32)
+        lib.decay_exp_exp(decay, self.w0, self.heads, self.dim)
         o = torch.empty((t, self.n), dtype=torch.float32, device=h.device)
-        if self.in_chunks and lib.recurrence_chunks_pay("bonus", self.heads, self.dim, self.dim, ctx):
-            lib.recurrence_chunks("bonus", (r, 0), (k, 0), (v, 0), self.heads, self.heads, self.dim, self.dim, (decay, 0), False, 2,
-                                  view.states["time_mix"], ctx, o, a_bias=self.w0, bonus=self.u)
-        else:
-            lib.decay_exp_exp(decay, self.w0, self.heads, self.dim)
-            lib.time_mix_recurrence(r, k, v, decay, self.u, view.states["time_mix"], ctx, o, self.heads, self.dim, self.dim)
+        lib.time_mix_recurrence(r, k, v, decay, self.u, view.states["time_mix"], ctx, o, self.heads, self.dim, self.dim)
         on = torch.empty((t, self.n), dtype=dt, device=h.device)
         lib.gated_rmsnorm_heads(o, self.norm, g, 1, self.eps, self.heads, self.dim, on)
         return linear(lib, on, self.w_o, torch.float32)

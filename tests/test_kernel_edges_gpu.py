@@ -1341,100 +1341,6 @@ def test_router_product_and_choice_in_one_launch_beside_two(lib, n, rows, output
     assert not lib.route_linear_ok(h.float(), rows, outputs)
 
 
-# ---------------------------------------------------------------------------- recurrences in chunks of 16 tokens
-def _recurrence_in_64_bits(mode, q, k, v, g, beta, bonus, state, lens):
-    """Token after token: q, k [T, H, d], v [T, H, e], g [T, H, d], beta [T, H], state [B, H, e, d]."""
-    out, at = torch.empty(v.shape, dtype=torch.float64), 0
-    state = state.clone()
-    for b, n in enumerate(lens):
-        s = state[b].transpose(1, 2)                          # [H, d, e]
-        for t in range(at, at + n):
-            kt, qt, vt = k[t].unsqueeze(2), q[t].unsqueeze(1), v[t].unsqueeze(1)
-            if mode == "bonus":
-                out[t] = (qt @ (s + bonus.unsqueeze(2) * (kt @ vt))).squeeze(1)
-            s = g[t].unsqueeze(2) * s
-            u = vt if mode != "delta" else beta[t].view(-1, 1, 1) * (vt - kt.transpose(1, 2) @ s)
-            s = s + kt @ u
-            if mode != "bonus":
-                out[t] = (qt @ s).squeeze(1)
-        state[b], at = s.transpose(1, 2), at + n
-    return out, state
-
-
-@pytest.mark.parametrize("lens", [[1], [15, 16, 17], [40, 1, 130], [300]])
-@pytest.mark.parametrize("mode,heads,kv,dim,vdim,per_head,decay", [
-    ("delta", 2, 2, 64, 16, False, 0), ("delta", 2, 1, 128, 80, True, 0), ("delta", 3, 3, 128, 128, False, 0), ("plain", 2, 2, 64, 128, False, 1),
-    ("plain", 1, 1, 128, 48, False, 0), ("bonus", 3, 3, 64, 64, False, 2), ("bonus", 1, 1, 128, 128, False, 2)])
-def test_recurrences_in_chunks(lib, mode, heads, kv, dim, vdim, per_head, decay, lens):
-    """Against the same in 64 bits, and no further from it than twice what the kernel that walks the tokens is: strong and weak
-    decays, a state to start from, pieces of a chunk, a window of a few chunks, and tokens that are not finite, which reach the
-    outputs that they reach when the tokens are walked and no others."""
-    gen = torch.Generator().manual_seed(sum(lens) + dim)
-    n, b = sum(lens), len(lens)
-    rnd = lambda *shape: torch.randn(*shape, generator=gen)
-    n_a = heads if per_head else heads * dim
-    for poison in (None, "v", "k", "a"):
-        qkv = rnd(n, 2 * kv * dim + heads * vdim)
-        raw, b_in = rnd(n, n_a) * 3 - 1, rnd(n, heads)
-        if poison and n > 20:
-            t = n // 2 + 1
-            if poison == "v":
-                qkv[t, 2 * kv * dim + 3], qkv[t - 3, 2 * kv * dim + 5] = float("inf"), float("nan")
-            elif poison == "k":
-                qkv[t, kv * dim + 1] = float("nan")
-            else:
-                raw[t, -1] = float("nan")
-        elif poison:
-            continue
-        a_bias, a_log = rnd(n_a), rnd(heads) * 0.5
-        bonus = rnd(heads, dim) if mode == "bonus" else None
-        state = rnd(b + 1, heads, vdim, dim)
-        unit, q_scale, tau = mode == "delta", dim ** -0.5, 8.0
-        slots = list(range(b, 0, -1))
-        ctx = StepContext.for_batch(DEV, StepBatch(slots, [0] * b, [[0] * m for m in lens], [0], {}), n_compute_units=lib.n_compute_units)
-        n_qk, dev = kv * dim, lambda t: None if t is None else t.clone().to(DEV)
-
-        def chunks(window):
-            x, st, o = dev(qkv), dev(state), torch.full((n, heads * vdim), 7.0, device=DEV)
-            lib.recurrence_chunks(mode, (x, 0), (x, n_qk), (x, 2 * n_qk), heads, kv, dim, vdim, (dev(raw), 0), per_head, decay, st, ctx, o,
-                                  a_bias=dev(a_bias), a_log=dev(a_log) if decay == 0 else None, tau=tau,
-                                  b=(dev(b_in), 0) if mode == "delta" else None, bonus=dev(bonus), unit=unit, q_scale=q_scale, unit_eps=1e-6,
-                                  window=window)
-            return o.cpu(), st.cpu()
-
-        x, st, o = dev(qkv), dev(state), torch.empty((n, heads * vdim), device=DEV)
-        z, beta = dev(raw), torch.empty((n, heads), device=DEV) if mode == "delta" else None
-        lib.recurrence_prep(x, kv, dim, unit, q_scale, 1e-6, z, 0, n_a, decay, dev(a_bias), dev(a_log) if decay == 0 else None, tau, heads,
-                            b_in=dev(b_in) if mode == "delta" else None, beta=beta)
-        if mode == "bonus":
-            parts = [x[:, i * n_qk:(i + 1) * n_qk].contiguous() for i in range(2)] + [x[:, 2 * n_qk:].contiguous()]
-            lib.time_mix_recurrence(*parts, z, dev(bonus), st, ctx, o, heads, dim, vdim)
-        else:
-            lib.linear_recurrence(x, kv, dim, heads, vdim, z, 0, per_head, beta, st, ctx, o)
-        walked, walked_state = o.cpu(), st.cpu()
-        got, got_state = chunks(None)
-        again, again_state = chunks(2)
-        assert torch.equal(got.nan_to_num(3.0), again.nan_to_num(3.0)) and torch.equal(got_state.nan_to_num(3.0), again_state.nan_to_num(3.0))
-        assert torch.equal(got_state[0], state[0])                                  # a slot of nobody's
-        assert torch.equal(got.isfinite(), walked.isfinite()) and torch.equal(got_state.isfinite(), walked_state.isfinite())
-        ok, ok_state = got.isfinite(), got_state.isfinite()
-        bound = lambda w: 1e-5 * float(w.abs().max())
-        assert float((got - walked)[ok].abs().max()) <= bound(walked[ok]) and float((got_state - walked_state)[ok_state].abs().max()) <= bound(walked_state[ok_state])
-        if poison is None:
-            f = lambda t: t.double().cpu()
-            each = lambda t, h, e: f(t).reshape(n, h, e).repeat_interleave(heads // h, dim=1)
-            q64, k64 = each(qkv[:, :n_qk], kv, dim), each(qkv[:, n_qk:2 * n_qk], kv, dim)
-            norm = lambda t: t / (t.square().sum(-1, keepdim=True) + 1e-6).sqrt() if unit else t
-            zb = f(raw) + f(a_bias)
-            zb = zb.view(n, heads, 1).expand(n, heads, dim) if per_head else zb.view(n, heads, dim)
-            sp = torch.nn.functional.softplus
-            g64 = torch.exp(-f(a_log).exp().view(1, heads, 1) * sp(zb)) if decay == 0 else torch.exp(-sp(-zb) / tau) if decay == 1 else torch.exp(-zb.exp())
-            want, want_state = _recurrence_in_64_bits(mode, norm(q64) * q_scale, norm(k64), each(qkv[:, 2 * n_qk:], heads, vdim), g64,
-                                                      torch.sigmoid(f(b_in)), None if bonus is None else f(bonus), f(state[slots]), lens)
-            for got_, walked_, want_ in ((got, walked, want.reshape(n, -1)), (got_state[slots], walked_state[slots], want_state)):
-                rms = lambda t: float((f(t) - want_).square().mean().sqrt())
-                assert rms(got_) <= 2 * rms(walked_) + 1e-9 * float(want_.abs().max()), (rms(got_), rms(walked_))
-
 
 # ---------------------------------------------------------------------------- products of few tokens in one launch
 @pytest.mark.parametrize("m", [1, 4, 16])
