@@ -166,13 +166,11 @@ int rb_streams_update_layernorm(float* x, int n_streams, long long stream_stride
                                 const float* bias, float eps, const int32_t* rows, int n_rows, int width, void* out,
                                 int out_dtype, void* stream);      // rb_streams_update (mix null: none), then the norm, in one pass
 // rb_embed_streams with x[s][t, :] = table[ids[t], :] * scale + wave(tok_pos[t]): number 2i of wave(p) is sin(p inv[i]), number 2i + 1
-// cos(p inv[i]); inv float64 [(width + 1) / 2], null: no wave.
-int rb_embed_streams_waves(const void* table, int table_dtype, const int32_t* ids, float scale, const double* inv, const int32_t* tok_pos,
-                           float* x, int n_streams, long long stream_stride, int n_tokens, int width, void* stream);
-// the same from a table stored as rows (table_layout 0) or fragment-major (1: a table that is the output matrix as well)
-int rb_embed_streams_layout(const void* table, int table_dtype, int table_layout, const int32_t* ids, float scale, const double* inv,
-                            const int32_t* tok_pos, float* x, int n_streams, long long stream_stride, int n_tokens, int width,
-                            void* stream);
+// cos(p inv[i]); inv float64 [(width + 1) / 2], null: no wave.  table_layout 0: rows, 1: fragment-major (a table that is the output
+// matrix as well).
+int rb_embed_streams_waves(const void* table, int table_dtype, int table_layout, const int32_t* ids, float scale, const double* inv,
+                           const int32_t* tok_pos, float* x, int n_streams, long long stream_stride, int n_tokens, int width,
+                           void* stream);
 // RMS norm of a stream in several copies, behind the update that may still be to be done (mix null: none), in one pass:
 //   x'[t] = sum_s mix[s, t] x[s] + out_coef[t] * y;  u = sum_s coef[s] x'[s][src];  out[r] = u / sqrt(mean(u^2) + eps) * gain,
 // src = rows ? rows[r] : r; with rows the copies stay as they are.  y of row src is the sum over k < n_terms of

@@ -185,8 +185,7 @@ class Kernels:
             "rb_streams_layernorm": [_P, _I, _L, _P, _P, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_streams_update_layernorm": [_P, _I, _L, _P, _P, _P, _P, _P, _P, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_streams_update": [_P, _I, _L, _P, _P, _P, _P, _I, _I, _P],
-            "rb_embed_streams_waves": [_P, _I, _P, _F, _P, _P, _P, _I, _L, _I, _I, _P],
-            "rb_embed_streams_layout": [_P, _I, _I, _P, _F, _P, _P, _P, _I, _L, _I, _I, _P],
+            "rb_embed_streams_waves": [_P, _I, _I, _P, _F, _P, _P, _P, _I, _L, _I, _I, _P],
             "rb_streams_rmsnorm": [_P, _I, _L, _P, _P, _P, _I, _L, _L, _P, _P, _I, _L, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_short_conv_biases": [_P, _L, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
             "rb_gemm_bf16_group_ok": [_I, _I],
@@ -683,8 +682,8 @@ class Kernels:
             raise KernelError("embedding width mismatch")
         if inv is not None:
             _check(inv, "inv", torch.float64, ((width + 1) // 2,))
-        self._ok(self._lib.rb_embed_streams_layout(_ptr(table), dtype_code(table.dtype), 1 if frag else 0, _ptr(ids), float(scale),
-                                                   _ptr(inv), _ptr(tok_pos), _ptr(x), s_, n * width, n, width, self._stream()))
+        self._ok(self._lib.rb_embed_streams_waves(_ptr(table), dtype_code(table.dtype), 1 if frag else 0, _ptr(ids), float(scale),
+                                                  _ptr(inv), _ptr(tok_pos), _ptr(x), s_, n * width, n, width, self._stream()))
 
     def streams_rmsnorm(self, x: torch.Tensor, coef: Optional[torch.Tensor], weight: torch.Tensor, eps: float,
                         rows: Optional[torch.Tensor], out: torch.Tensor, update=None) -> None:

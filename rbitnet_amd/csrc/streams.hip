@@ -394,19 +394,12 @@ __global__ void embed_streams_waves_kernel(const T* __restrict__ table, const in
   }
 }
 
-extern "C" int rb_embed_streams_waves(const void* table, int table_dtype, const int32_t* ids, float scale, const double* inv,
-                                      const int32_t* tok_pos, float* x, int n_streams, long long stream_stride, int n_tokens, int width,
-                                      void* stream) {
-  RB_RECORDED(rb_embed_streams_waves(table, table_dtype, ids, scale, inv, tok_pos, x, n_streams, stream_stride, n_tokens, width, stream));
-  return rb_embed_streams_layout(table, table_dtype, 0, ids, scale, inv, tok_pos, x, n_streams, stream_stride, n_tokens, width, stream);
-}
-
-// The same from a table of either layout (0: rows; 1: fragment-major).
-extern "C" int rb_embed_streams_layout(const void* table, int table_dtype, int table_layout, const int32_t* ids, float scale,
-                                       const double* inv, const int32_t* tok_pos, float* x, int n_streams, long long stream_stride,
-                                       int n_tokens, int width, void* stream) {
-  RB_RECORDED(rb_embed_streams_layout(table, table_dtype, table_layout, ids, scale, inv, tok_pos, x, n_streams, stream_stride, n_tokens,
-                                      width, stream));
+// table_layout 0: rows; 1: fragment-major
+extern "C" int rb_embed_streams_waves(const void* table, int table_dtype, int table_layout, const int32_t* ids, float scale,
+                                      const double* inv, const int32_t* tok_pos, float* x, int n_streams, long long stream_stride,
+                                      int n_tokens, int width, void* stream) {
+  RB_RECORDED(rb_embed_streams_waves(table, table_dtype, table_layout, ids, scale, inv, tok_pos, x, n_streams, stream_stride, n_tokens,
+                                     width, stream));
   RB_REQUIRE(n_tokens >= 0 && width > 0 && n_streams >= 1 && stream_stride >= 0, "rb_embed_streams_waves: bad sizes");
   RB_REQUIRE(inv == nullptr || tok_pos != nullptr, "rb_embed_streams_waves: a wave needs the tokens' positions");
   RB_REQUIRE(table_dtype == RB_F32 || table_dtype == RB_BF16, "rb_embed_streams_waves: unknown dtype %d", table_dtype);

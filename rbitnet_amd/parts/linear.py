@@ -16,10 +16,10 @@ from typing import Optional
 
 import torch
 
+from ..csrc.lib import GROUP_PRODUCTS
 from ..errors import KernelError
 from .stream import GainedRows, norm_adds_terms, norm_folds
 
-GROUP_PRODUCTS = 6  # of one launch (rb_gemm_bf16_group)
 GATE_BLOCK = 16     # rows per block when gate and up rows are interleaved for the fused epilogue
 
 
