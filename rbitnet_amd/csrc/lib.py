@@ -1114,6 +1114,14 @@ class Kernels:
     def route_linear_ok(self, h: torch.Tensor, n_rows: int, n_outputs: int) -> bool:
         return h.dtype == torch.bfloat16 and bool(self._lib.rb_route_linear_ok(h.shape[0], n_rows, n_outputs, h.shape[1]))
 
+    @staticmethod
+    def route_linear_pays(n_tokens: int, n_rows: int) -> bool:
+        """Whether one workgroup that multiplies and chooses is faster than a product on several compute units and a choice (the bits are the
+        same): us in one launch / in two, K = 2048 and 8192, 1, 4, 8 and 16 tokens.  16 rows 5.2/6.4 5.7/6.8 6.1/7.1 8.1/8.4 and 8.3/9.9 9.7/10.9
+        10.9/12.0 14.9/15.2; 32 rows 6.8/7.5 7.3/8.2 7.6/8.4 10.4/10.1 and 11.0/12.2 12.4/13.0 13.5/13.7 18.2/17.3; 64 rows 10.3/9.4 10.6/9.8 10.9/10.0
+        14.8/11.8 and 17.1/13.6 18.3/14.4 19.4/15.2 25.0/19.2."""
+        return n_rows <= 16 or (n_rows <= 32 and n_tokens <= 8)
+
     def route_linear(self, h: torch.Tensor, w: torch.Tensor, w_frag: bool, z: torch.Tensor, n_outputs: int, n_experts: int, top: int,
                      score: int, correction: Optional[torch.Tensor], sel: torch.Tensor, weight: torch.Tensor, row_pair: torch.Tensor,
                      tile_expert: torch.Tensor, bias: Optional[torch.Tensor] = None, unit: int = 16) -> None:

@@ -275,7 +275,7 @@ __global__ __launch_bounds__(1024) void route_few_small_kernel(const float* __re
 // The router's product in front of that, in the same launch, for up to 16 tokens and 64 rows of W: one workgroup of 8 waves, which deal
 // themselves the depth as a product of that few rows does (gemm_skinny.hip: stages of 128 in a row, the waves' sums added in their order), so
 // the logits are the same bits, and a step has one launch of one workgroup in place of two that wait for each other.  (4 tokens, 16
-// experts, 4 chosen, K = 2048, in a captured step: 3.4 + 4.4 us in two launches, 5.4 to 6.3 in one.)
+// experts, 4 chosen, K = 2048, in a captured step: 3.4 + 4.4 us in two launches, 5.4 to 6.3 in one; with more rows: Kernels.route_linear_pays.)
 constexpr int RL_WAVES = 8, RL_TOKENS = 16, RL_TILES = 4;
 template <bool WF, int NT>                                   // NT: row tiles of 16, 1 or up to RL_TILES
 __global__ __launch_bounds__(RL_WAVES * RB_WAVE) void route_linear_kernel(

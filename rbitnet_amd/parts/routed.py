@@ -194,7 +194,8 @@ class RoutedExperts(Part):
         row_pair = torch.empty(max_rows, dtype=torch.int32, device=dev)
         tile_expert = torch.empty(2 * (max_rows // unit), dtype=torch.int32, device=dev)      # experts, then positions in their runs
         n_rows = self.w_router.shape[0]
-        if not tiled and lib.route_linear_ok(h, n_rows, self.n_outputs) and not getattr(self.env, "generic_only", False):
+        if (not tiled and lib.route_linear_ok(h, n_rows, self.n_outputs) and lib.route_linear_pays(t, n_rows)
+                and not getattr(self.env, "generic_only", False)):
             z = torch.empty((t, n_rows), dtype=torch.float32, device=dev)
             lib.route_linear(h, self.w_router.data, self.w_router.frag, z, self.n_outputs, self.n_experts, self.top, self.score,
                              self.correction, sel, weight, row_pair, tile_expert, bias=self.bias, unit=unit)

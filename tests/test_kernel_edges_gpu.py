@@ -1342,6 +1342,23 @@ def test_router_product_and_choice_in_one_launch_beside_two(lib, n, rows, output
 
 
 
+@pytest.mark.parametrize("experts,n,one", [(16, 16, True), (17, 8, True), (32, 8, True), (32, 9, False), (33, 1, False), (64, 4, False)])
+def test_routers_of_many_rows_keep_a_product_of_their_own(lib, monkeypatch, experts, n, one):
+    """On either side of where one workgroup is no faster any more; the outputs are the same bits."""
+    gen = torch.Generator().manual_seed(experts + n)
+    params = {"experts": experts, "top": 2, "intermediate_size": 32, "limit": 7.0}
+    part = build_part("feed_forward", PartSpec("routed_experts", params), BuildEnv(hidden_size=1024, dtype=torch.bfloat16, device=torch.device(DEV), lib=lib))
+    part.load({name: (torch.randn(ts.shape, generator=gen) * 0.03).to(torch.float32 if ts.role == "gain" else torch.bfloat16).to(DEV)
+               for name, ts in part.tensor_specs().items()})
+    h = torch.randn(n, 1024, generator=gen).bfloat16().to(DEV)
+    calls, real = [], lib.route_linear
+    monkeypatch.setattr(lib, "route_linear", lambda *a, **kw: (calls.append(1), real(*a, **kw)))
+    got = part.forward(h)
+    assert bool(calls) == one
+    monkeypatch.setattr(type(lib), "route_linear_pays", staticmethod(lambda *a: not one))
+    assert torch.equal(part.forward(h), got)
+
+
 # ---------------------------------------------------------------------------- products of few tokens in one launch
 @pytest.mark.parametrize("m", [1, 4, 16])
 @pytest.mark.parametrize("k", [128, 384, 2048, 8192])
