@@ -1243,8 +1243,8 @@ ONE_LAUNCH += [("state_space", dict(heads=h, vdim=v, state=d, groups=g, conv=c, 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("kind,params", ONE_LAUNCH)
 def test_single_tokens_through_a_recurrence_in_one_launch_beside_launches_of_their_own(lib, kind, params, dtype):
-    """The same mixer, states and tokens both ways, three steps of three sequences.  Both compute in float32 and differ in the
-    order of sums of at most 512 numbers: 1e-5 of the largest value bounds that; bfloat16 outputs may round the other way once."""
+    """The same mixer, states and tokens both ways, three steps of three sequences, by formula: 1e-5 of the largest value bounds any order
+    of float32 sums of at most 512 numbers, and bfloat16 outputs may round the other way once.  (That the order is the same: below.)"""
     gen = torch.Generator().manual_seed(11)
     hidden = 64
     part = build_part("mixer", PartSpec(kind, params), BuildEnv(hidden_size=hidden, dtype=dtype, device=torch.device(DEV), lib=lib))
