@@ -84,6 +84,32 @@ def test_replayed_single_tokens_whose_keys_are_shared_start_from_zero_counters()
         assert max_err(outs[1][:, i], plain_logits("D", tuple(r))[n:n + new]) < TOL["float32"]
 
 
+def test_replayed_single_tokens_of_layers_behind_others_equal_eager_ones():
+    """The same without a hand on the scratch memory, where the first attention with shared keys follows layers whose temporaries the
+    plan's pool has taken back by then: attention through latents, then windowed attention beside time mixing."""
+    import rbitnet_amd
+    latent = {"heads": 4, "dim": 32, "rot_dim": 16, "vdim": 32, "q_rank": 64, "kv_rank": 48, "scale": 48 ** -0.5, "rot": {"base": 10000.0, "dims": 16}}
+    left = {"heads": 4, "kv_heads": 2, "dim": 32, "vdim": 32, "conv": 4, "rot": {"base": 10000.0, "dims": 16}, "scale": 32 ** -0.5, "softcap": 50.0,
+            "mask": {"size": 512, "keep_first": 64}}
+    right = {"heads": 2, "dim": 32, "decay_rank": 16}
+    mlp = {"kind": "dense", "ff": 192, "limit": 7.0}
+    pair = {"type": "parallel", "mlp": mlp, "mixer": {"left": left, "right": right, "left_scale": 0.5, "right_scale": 1.0}}
+    config = {"architecture": "Menerax", "vocab": 160, "width": 128, "norm": {"eps": 1e-5},
+              "layers": [{"type": "latent_attention", "mixer": latent, "mlp": mlp}] * 2 + [pair] * 2}
+    outs = []
+    for plans in (False, True):
+        eng = rbitnet_amd.Engine.random(config, std=0.1, dtype="float32", max_tokens=2048, max_batch=2, max_seq_len=1000)
+        eng.use_plans = plans and eng.use_plans
+        slots, got = [eng.alloc_slot(), eng.alloc_slot()], []
+        eng.step([(slots[0], [i * 7 % 160 for i in range(650)]), (slots[1], [i * 11 % 160 for i in range(330)])])
+        for j in range(6):
+            got.append(eng.step([(s, [(j + 5 * s) % 160]) for s in slots]))
+        outs.append(torch.stack(got))
+        assert eng.use_plans == plans and (not plans or eng.plans.stats["replayed"] >= 2)
+    assert any(k[0] == "shared keys" for p in eng.plans.plans.values() for k in p.ctx._workspaces)
+    assert torch.equal(outs[0], outs[1])
+
+
 def test_a_shape_seen_once_is_not_recorded_and_old_plans_make_room():
     from rbitnet_amd.engine import step_plan
     eng = _engine("A", "float32", max_batch=1, max_tokens=256)
