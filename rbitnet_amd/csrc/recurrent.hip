@@ -8,6 +8,8 @@
 #include "api.h"
 #include "common.h"
 
+#include <type_traits>
+
 __device__ __forceinline__ float rb_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
 __device__ __forceinline__ float rb_softplus(float v) { return v > 20.0f ? v : log1pf(expf(v)); }
 
@@ -383,9 +385,9 @@ extern "C" int rb_delta_prep(float* qk, long long qk_stride, int n_kv_heads, int
 //   S <- diag(g) S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
 // The columns of S (one per value channel) do not meet: a column is held by RG lanes, each with DKL of its rows in
 // registers; the dot products over the rows are finished among the RG lanes by moves inside a row of lanes.  A workgroup is one wave
-// and holds 64 / RG columns.  Tokens go by in chunks of CH: q, k, g, v and beta of a chunk lie in LDS for all lanes, and
+// and holds P columns a lane, 64 / RG * P in all (two of them share what the lane reads from LDS, and the product of k and q).  Tokens go by in chunks of CH: q, k, g, v and beta of a chunk lie in LDS for all lanes, and
 // the next chunk's loads are in flight (in registers) while the current one is computed, so that a token costs its
-// arithmetic and no trip to memory; the chunk's outputs leave through LDS as whole rows.  The state is read once and
+// arithmetic and no trip to memory; the chunk's outputs leave from registers.  The state is read once and
 // written once.
 // The sum over each group of RG neighbouring lanes (RG = 4, 8 or 16), in every lane of the group, by moves inside a
 // row of 16 lanes (no trip through LDS): the two swaps inside a quad, then the mirror of a half row, then of a row.
@@ -403,19 +405,22 @@ __device__ __forceinline__ float lanes_sum(float v) {
 // 3: a selective scan: every token has a step size dt = softplus(dt_in + dt_bias[h]) per head, from which the decay and the
 // weight of the write come, and its value passes to the read-out with a weight of the head:
 //   S <- exp(-exp(a_log[h]) dt) S + dt k v^T;  o = S^T q + d[h] v
+// 4: without beta, the plain rule S <- diag(g) S + k v^T.
 struct SelectiveArgs {
   const float* dt_in;
   size_t dt_stride;
   const float *dt_bias, *a_log, *d;
 };
-template <int DKL, int RG, int CH, int MODE, bool WIDE>
+// ONE_G: one decay a head and token (g_per_head), which the lanes read as one number.
+template <int DKL, int RG, int P, int CH, int MODE, bool ONE_G, bool WIDE>
 __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
     const float* __restrict__ q, const float* __restrict__ k, size_t qk_stride, const float* __restrict__ v,
     size_t v_stride, const float* __restrict__ g, size_t g_stride, const float* __restrict__ beta, float* __restrict__ state,
     const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slots, float* __restrict__ out, int n_heads,
-    int n_kv, int dim, int vdim, int g_per_head, const float* __restrict__ bonus, SelectiveArgs sel) {
-  constexpr bool BONUS = MODE == 1, SELECTIVE = MODE == 3;
-  constexpr int COLS = RB_WAVE / RG;
+    int n_kv, int dim, int vdim, int n_parts, const float* __restrict__ bonus, SelectiveArgs sel) {
+  constexpr bool DELTA = MODE == 0, BONUS = MODE == 1, SILU = MODE == 2, SELECTIVE = MODE == 3;
+  static_assert(ONE_G || !SELECTIVE, "a selective scan has one decay a head");
+  constexpr int COLS = RB_WAVE / RG * P;
   constexpr int DK = DKL * RG;               // rows held, >= dim; rows beyond dim stay zero
   constexpr int NQ = DK * CH / RB_WAVE;      // q (or k, or g) values of a chunk per lane
   constexpr int NV = (COLS * CH + RB_WAVE - 1) / RB_WAVE;
@@ -424,36 +429,39 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
   // 512, 2,662 and 1,415.  Up to dim 128 the gap gives nothing: 464 and 467 us.)
   constexpr int STEP = DK > 128 ? DKL + 4 : DKL, LD = STEP * RG;
   auto pos = [](int i) { return i + (STEP - DKL) * (i / DKL); };
-  __shared__ __attribute__((aligned(16))) float sq[CH][LD], sk[CH][LD], sg[SELECTIVE ? 1 : CH][SELECTIVE ? CH : LD];
-  __shared__ float sv[CH][COLS], so[CH][COLS], sb[CH];
-  const int b = blockIdx.x, h = blockIdx.y;
+  __shared__ __attribute__((aligned(16))) float sq[CH][LD], sk[CH][LD], sg[ONE_G ? 1 : CH][ONE_G ? CH : LD];
+  __shared__ __attribute__((aligned(16))) float sv[CH][COLS], sb[CH];
+  // heads are dealt first, then a head's columns, then sequences: neighbouring workgroups go to different XCDs, so one sequence's are spread
+  // over the whole GPU and those of a long one have it to themselves once the short ones are done
+  const int h = blockIdx.x % n_heads, b = blockIdx.x / n_heads / n_parts;
   const int lane = threadIdx.x;
-  const int col0 = blockIdx.z * COLS;
-  const int col = col0 + lane / RG;
-  const int rg = lane % RG;
-  const bool on = col < vdim;
+  const int col0 = blockIdx.x / n_heads % n_parts * COLS;
+  const int rg = lane % RG, mine = lane / RG * P, col = col0 + mine;      // this lane's columns: col .. col + P - 1
   const int kvh = h / (n_heads / n_kv);
   const int row0 = cu_seqlens[b], n = cu_seqlens[b + 1] - row0;
   // the state is kept column by column, [slots, H, vdim, dim]: a lane's rows are DKL numbers in a row and a wave's
   // columns one piece of memory (with S as rows a wave of four columns used a quarter of every line it touched)
-  float* S = state + (((size_t)slots[b] * n_heads + h) * vdim + (on ? col : 0)) * dim;
-  float s[DKL];
+  float* S = state + (((size_t)slots[b] * n_heads + h) * vdim + col) * dim;
+  float s[P][DKL];
   const bool quads = dim % 4 == 0 && DKL % 4 == 0 && (reinterpret_cast<uintptr_t>(state) & 15) == 0;
-  if (quads) {
 #pragma unroll
-    for (int i = 0; i < DKL; i += 4) {
-      const int r = rg * DKL + i;
-      const float4 v4 = (on && r < dim) ? *reinterpret_cast<const float4*>(S + r) : make_float4(0.f, 0.f, 0.f, 0.f);
-      s[i] = v4.x;
-      s[i + 1] = v4.y;
-      s[i + 2] = v4.z;
-      s[i + 3] = v4.w;
-    }
-  } else {
+  for (int p = 0; p < P; ++p) {
+    if (quads) {
 #pragma unroll
-    for (int i = 0; i < DKL; ++i) {
-      const int r = rg * DKL + i;
-      s[i] = (on && r < dim) ? S[r] : 0.f;
+      for (int i = 0; i < DKL; i += 4) {
+        const int r = rg * DKL + i;
+        const float4 v4 = (col + p < vdim && r < dim) ? *reinterpret_cast<const float4*>(S + (size_t)p * dim + r) : make_float4(0.f, 0.f, 0.f, 0.f);
+        s[p][i] = v4.x;
+        s[p][i + 1] = v4.y;
+        s[p][i + 2] = v4.z;
+        s[p][i + 3] = v4.w;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < DKL; ++i) {
+        const int r = rg * DKL + i;
+        s[p][i] = (col + p < vdim && r < dim) ? S[(size_t)p * dim + r] : 0.f;
+      }
     }
   }
   // BONUS: the read-out sees the state as it was before the token, and the token's own k v^T times a weight per key
@@ -464,8 +472,8 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
     const int r = rg * DKL + i;
     ub[i] = (BONUS && r < dim) ? bonus[(size_t)h * dim + r] : 0.f;
   }
-  float rq[WIDE ? 1 : NQ], rk[WIDE ? 1 : NQ], rgt[SELECTIVE || WIDE ? 1 : NQ], rv[NV], rb = 0.f;
-  float4 wq[WIDE ? NQ / 4 : 1], wk[WIDE ? NQ / 4 : 1], wg[WIDE && !SELECTIVE ? NQ / 4 : 1];
+  float rq[WIDE ? 1 : NQ], rk[WIDE ? 1 : NQ], rgt[ONE_G || WIDE ? 1 : NQ], rv[NV], rb = 0.f, rg1 = 0.f;
+  float4 wq[WIDE ? NQ / 4 : 1], wk[WIDE ? NQ / 4 : 1], wg[WIDE && !ONE_G ? NQ / 4 : 1];
   const float rate = SELECTIVE ? expf(sel.a_log[h]) : 0.f, dt_bias = SELECTIVE ? sel.dt_bias[h] : 0.f, pass = SELECTIVE ? sel.d[h] : 0.f;
   // WIDE (rows and strides of 16 bytes): a chunk's values reach a lane four in a row, and what lies beyond the tokens or the key's rows is
   // taken out on the way to LDS and not before the next chunk's loads have come.  Values one by one were as many instructions, masks and addresses, as
@@ -473,7 +481,48 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
   // now; dim 128 464 and 343; dim 256 1,624 and 860; 8 heads of dim 512 2,664 and 792).  Fetch j: token wide_t(j) of the chunk, rows wide_i(j) .. + 3.
   auto wide_t = [&](int j) { return DK <= 256 ? lane / (DK / 4) + j * (DK <= 256 ? 256 / DK : 1) : j / (DK > 256 ? DK / 256 : 1); };
   auto wide_i = [&](int j) { return DK <= 256 ? 4 * (lane % (DK / 4)) : 4 * lane + 256 * (j % (DK > 256 ? DK / 256 : 1)); };
-  auto fetch = [&](int t0) {
+  // Whole chunks of keys without padding: every place is an offset of the lane's from a place that moves on by a chunk, and nothing is masked.
+  // A wave has its SIMD to itself and takes an instruction every 5 cycles whatever it waits for, so instructions are the time: with places and
+  // masks made anew a chunk of 16 tokens was 500 of them (51 multiplications at a quarter of the rate) beside the 1,900 of its tokens, now 150.
+  // us for 4 sequences of 390 to 1,500 tokens, before this, the dealing of sequences over the GPU, outputs that leave late and a plain rule without the
+  // delta rule's sums, and with them: 16 heads of 128 x 128 537 and 423; 8 heads of 64 x 128, plain, 247 and 145; with two columns a lane as well, 64
+  // sequences of 64 tokens, 16 heads of 128 x 128, 397 and 229, 8 heads of 64 x 128 115 and 65.  Tried: LDS read piece by piece among the
+  // arithmetic (a seventh slower), a token's read-out beside the next token (no change).
+  const bool no_pad = WIDE && dim == DK && col0 + COLS <= vdim;
+  uint32_t qk_off[WIDE ? NQ / 4 : 1], g_off[WIDE && !ONE_G ? NQ / 4 : 1], v_off[WIDE ? NV : 1];
+  if (WIDE) {
+#pragma unroll
+    for (int j = 0; j < NQ / 4; ++j) {
+      qk_off[j] = (uint32_t)wide_t(j) * (uint32_t)qk_stride + wide_i(j);
+      if (!ONE_G) g_off[ONE_G ? 0 : j] = (uint32_t)wide_t(j) * (uint32_t)g_stride + wide_i(j);
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int e = lane + RB_WAVE * j < COLS * CH ? lane + RB_WAVE * j : 0;
+      v_off[j] = (uint32_t)(e / COLS) * (uint32_t)v_stride + e % COLS;
+    }
+  }
+  // WHOLE: a whole chunk of keys without padding, CH tokens
+  auto fetch = [&](auto is_whole, int t0) __attribute__((always_inline)) {
+    constexpr bool WHOLE = decltype(is_whole)::value;
+    if constexpr (WHOLE) {
+      const size_t t = (size_t)(row0 + t0);
+      const float *qt = q + t * qk_stride + (size_t)kvh * dim, *kt = k + t * qk_stride + (size_t)kvh * dim;
+      const float *gt = ONE_G ? nullptr : g + t * g_stride + (size_t)h * dim, *vt = v + t * v_stride + (size_t)h * vdim + col0;
+#pragma unroll
+      for (int j = 0; j < NQ / 4; ++j) {
+        wq[j] = *reinterpret_cast<const float4*>(qt + qk_off[j]);
+        wk[j] = *reinterpret_cast<const float4*>(kt + qk_off[j]);
+        if (!ONE_G) wg[ONE_G ? 0 : j] = *reinterpret_cast<const float4*>(gt + g_off[ONE_G ? 0 : j]);
+      }
+#pragma unroll
+      for (int j = 0; j < NV; ++j) rv[j] = vt[v_off[j]];
+      const size_t own = t + lane % CH;
+      if (SELECTIVE) rb = sel.dt_in[own * sel.dt_stride + h];
+      if (DELTA) rb = beta[own * n_heads + h];
+      if (ONE_G && !SELECTIVE) rg1 = g[own * g_stride + h];
+      return;
+    }
     const int nt = n - t0 < CH ? n - t0 : CH;
     if (WIDE) {
 #pragma unroll
@@ -483,9 +532,7 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
         const size_t t = (size_t)(row0 + t0 + tt);
         wq[j] = *reinterpret_cast<const float4*>(q + t * qk_stride + (size_t)kvh * dim + i);
         wk[j] = *reinterpret_cast<const float4*>(k + t * qk_stride + (size_t)kvh * dim + i);
-        if (SELECTIVE) continue;
-        if (g_per_head) wg[j].x = g[t * g_stride + h];
-        else wg[j] = *reinterpret_cast<const float4*>(g + t * g_stride + (size_t)h * dim + i);
+        if (!ONE_G) wg[ONE_G ? 0 : j] = *reinterpret_cast<const float4*>(g + t * g_stride + (size_t)h * dim + i);
       }
     }
 #pragma unroll
@@ -495,116 +542,128 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
       const size_t t = (size_t)(row0 + t0 + tt);
       rq[j] = in ? q[t * qk_stride + (size_t)kvh * dim + i] : 0.f;
       rk[j] = in ? k[t * qk_stride + (size_t)kvh * dim + i] : 0.f;
-      if (!SELECTIVE) rgt[j] = in ? (g_per_head ? g[t * g_stride + h] : g[t * g_stride + (size_t)h * dim + i]) : 0.f;
-      if (MODE == 2) {
-        rq[j] *= rb_sigmoid(rq[j]);
-        rk[j] *= rb_sigmoid(rk[j]);
-      }
+      if (!ONE_G) rgt[ONE_G ? 0 : j] = in ? g[t * g_stride + (size_t)h * dim + i] : 0.f;
     }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int e = lane + RB_WAVE * j, tt = e / COLS, c = e - tt * COLS;
       rv[j] = (tt < nt && col0 + c < vdim) ? v[(size_t)(row0 + t0 + tt) * v_stride + (size_t)h * vdim + col0 + c] : 0.f;
-      if (MODE == 2) rv[j] *= rb_sigmoid(rv[j]);
     }
     if (SELECTIVE)                                     // the step's raw number: what it becomes is made when the chunk goes to LDS
       rb = lane < nt ? sel.dt_in[(size_t)(row0 + t0 + lane) * sel.dt_stride + h] : 0.f;
-    else
-      rb = (beta && lane < nt) ? beta[(size_t)(row0 + t0 + lane) * n_heads + h] : 0.f;
+    if (DELTA) rb = lane < nt ? beta[(size_t)(row0 + t0 + lane) * n_heads + h] : 0.f;
+    if (ONE_G && !SELECTIVE) rg1 = lane < nt ? g[(size_t)(row0 + t0 + lane) * g_stride + h] : 0.f;
   };
-  if (n > 0) fetch(0);
-  for (int t0 = 0; t0 < n; t0 += CH) {
-    const int nt = n - t0 < CH ? n - t0 : CH;
-    __syncthreads();                                   // the chunk before has been read and its outputs are out
+  // what was fetched goes to LDS
+  auto place = [&](auto is_whole, int nt) __attribute__((always_inline)) {
+    constexpr bool WHOLE = decltype(is_whole)::value;
     if (WIDE) {
 #pragma unroll
       for (int j = 0; j < NQ / 4; ++j) {
         const int tt = wide_t(j), i = wide_i(j), at = pos(i);
-        float4 fq = wq[j], fk = wk[j], fg = wg[SELECTIVE ? 0 : j];
-        if (!SELECTIVE && g_per_head) fg.y = fg.z = fg.w = fg.x;
-        if (MODE == 2) {
+        float4 fq = wq[j], fk = wk[j], fg = wg[ONE_G ? 0 : j];
+        if (SILU) {
           fq = make_float4(fq.x * rb_sigmoid(fq.x), fq.y * rb_sigmoid(fq.y), fq.z * rb_sigmoid(fq.z), fq.w * rb_sigmoid(fq.w));
           fk = make_float4(fk.x * rb_sigmoid(fk.x), fk.y * rb_sigmoid(fk.y), fk.z * rb_sigmoid(fk.z), fk.w * rb_sigmoid(fk.w));
         }
-        if (tt >= nt || i >= dim) fq = fk = fg = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (!WHOLE && (tt >= nt || i >= dim)) fq = fk = fg = make_float4(0.f, 0.f, 0.f, 0.f);
         *reinterpret_cast<float4*>(&sq[tt][at]) = fq;
         *reinterpret_cast<float4*>(&sk[tt][at]) = fk;
-        if (!SELECTIVE) *reinterpret_cast<float4*>(&sg[SELECTIVE ? 0 : tt][SELECTIVE ? 0 : at]) = fg;
+        if (!ONE_G) *reinterpret_cast<float4*>(&sg[ONE_G ? 0 : tt][ONE_G ? 0 : at]) = fg;
       }
     }
 #pragma unroll
     for (int j = 0; j < (WIDE ? 0 : NQ); ++j) {
       const int e = lane + RB_WAVE * j, tt = e / DK, i = e - tt * DK;
-      sq[tt][pos(i)] = rq[j];
-      sk[tt][pos(i)] = rk[j];
-      if (!SELECTIVE) sg[tt][pos(i)] = rgt[j];
+      sq[tt][pos(i)] = SILU ? rq[j] * rb_sigmoid(rq[j]) : rq[j];
+      sk[tt][pos(i)] = SILU ? rk[j] * rb_sigmoid(rk[j]) : rk[j];
+      if (!ONE_G) sg[ONE_G ? 0 : tt][ONE_G ? 0 : pos(i)] = rgt[ONE_G ? 0 : j];
     }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int e = lane + RB_WAVE * j;
-      if (e < COLS * CH) sv[e / COLS][e % COLS] = rv[j];
+      if (e < COLS * CH) sv[e / COLS][e % COLS] = SILU ? rv[j] * rb_sigmoid(rv[j]) : rv[j];
     }
-    if (SELECTIVE) {
-      if (lane < CH) {
+    if (lane < CH) {
+      if (SELECTIVE) {
         const float dt = rb_softplus(rb + dt_bias);
         sb[lane] = dt;
         sg[0][lane] = expf(-rate * dt);
+      } else {
+        sb[lane] = rb;
+        if (ONE_G) sg[0][lane] = rg1;
       }
-    } else if (lane < CH) {
-      sb[lane] = rb;
     }
-    __syncthreads();
-    if (t0 + CH < n) fetch(t0 + CH);                   // in flight while this chunk is computed
-    __builtin_amdgcn_sched_barrier(0);                 // (issued here, not where the scheduler would sink them: at their use)
-    // One token: with D = diag(g) S and u = beta (v - D^T k), the read-out of the updated state is
-    // (D + k u^T)^T q = D^T q + u (k . q): one pass over the decayed column gives both dot products, and a token has
-    // one reduction among the RG lanes on its way instead of two.  Two partial sums each: shorter chains of additions.
-    struct Token {
-      float k[DKL], q[DKL], g[SELECTIVE ? 1 : DKL], v, b;
-    };
-    auto read = [&](Token& r, int tt) __attribute__((always_inline)) {
+  };
+  // Lane tt % RG of a column's lanes keeps the outputs of a chunk's token tt.  They leave once the next chunk is in LDS: in front of the wait for
+  // its values, that wait was for the stores as well.
+  constexpr int KEPT = (CH + RG - 1) / RG;
+  float o[KEPT][P];
 #pragma unroll
-      for (int i = 0; i < DKL; ++i) {
-        r.k[i] = sk[tt][rg * STEP + i];
-        r.q[i] = sq[tt][rg * STEP + i];
-        if (!SELECTIVE) r.g[i] = sg[tt][rg * STEP + i];
+  for (int j = 0; j < KEPT; ++j)
+#pragma unroll
+    for (int p = 0; p < P; ++p) o[j][p] = 0.f;
+  auto leave = [&](auto is_whole, int t0) __attribute__((always_inline)) {
+    constexpr bool WHOLE = decltype(is_whole)::value;
+#pragma unroll
+    for (int j = 0; j < KEPT; ++j) {
+      const int tt = rg + j * RG;
+      if (WHOLE ? CH % RG == 0 || tt < CH : tt < (n - t0 < CH ? n - t0 : CH)) {
+        float* to = out + ((size_t)(row0 + t0 + tt) * n_heads + h) * vdim + col;
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          if (WHOLE || col + p < vdim) to[p] = o[j][p];
       }
-      if (SELECTIVE) r.g[0] = sg[0][tt];
-      r.v = sv[tt][lane / RG];
-      r.b = sb[tt];
-    };
-    auto token = [&](const Token& r, int tt) __attribute__((always_inline)) {
-      const float vv = r.v, bt = r.b, gt = r.g[0];
-      float kv0 = 0.f, kv1 = 0.f, dq0 = 0.f, dq1 = 0.f, kq0 = 0.f, kq1 = 0.f;
+    }
+  };
+      // One token: with D = diag(g) S and u = beta (v - D^T k), the read-out of the updated state is
+      // (D + k u^T)^T q = D^T q + u (k . q): one pass over the decayed column gives both dot products, and a token has
+      // one reduction among the RG lanes on its way instead of two.  Two partial sums each: shorter chains of additions.
+      struct Token {
+        float k[DKL], q[DKL], g[ONE_G ? 1 : DKL], v[P], b;
+      };
+      auto read = [&](Token& r, int tt) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < DKL; i += 2) {
-        const float k0 = r.k[i], q0 = r.q[i];
-        const float k1 = r.k[i + 1], q1 = r.q[i + 1];
-        kq0 = fmaf(BONUS ? ub[i] * k0 : k0, q0, kq0);
-        kq1 = fmaf(BONUS ? ub[i + 1] * k1 : k1, q1, kq1);
-        if (BONUS) {
-          dq0 = fmaf(s[i], q0, dq0);
-          dq1 = fmaf(s[i + 1], q1, dq1);
+        for (int i = 0; i < DKL; ++i) {
+          r.k[i] = sk[tt][rg * STEP + i];
+          r.q[i] = sq[tt][rg * STEP + i];
+          if (!ONE_G) r.g[ONE_G ? 0 : i] = sg[ONE_G ? 0 : tt][ONE_G ? 0 : rg * STEP + i];
         }
-        s[i] *= SELECTIVE ? gt : r.g[SELECTIVE ? 0 : i];
-        s[i + 1] *= SELECTIVE ? gt : r.g[SELECTIVE ? 0 : i + 1];
-        if (BONUS) continue;
-        if (!SELECTIVE) {
-          kv0 = fmaf(s[i], k0, kv0);
-          kv1 = fmaf(s[i + 1], k1, kv1);
-        }
-        dq0 = fmaf(s[i], q0, dq0);
-        dq1 = fmaf(s[i + 1], q1, dq1);
-      }
-      const float kv = (BONUS || SELECTIVE) ? 0.f : lanes_sum<RG>(kv0 + kv1);
-      const float dq = lanes_sum<RG>(dq0 + dq1);
-      const float kq = lanes_sum<RG>(kq0 + kq1);
-      // without beta: the plain rule, S <- diag(g) S + k v^T
-      const float u = SELECTIVE ? bt * vv : (!BONUS && beta) ? bt * (vv - kv) : vv;
+        if (ONE_G) r.g[0] = sg[0][ONE_G ? tt : 0];
 #pragma unroll
-      for (int i = 0; i < DKL; ++i) s[i] = fmaf(r.k[i], u, s[i]);
-      if (rg == 0) so[tt][lane / RG] = SELECTIVE ? fmaf(pass, vv, fmaf(u, kq, dq)) : fmaf(u, kq, dq);
-    };
+        for (int p = 0; p < P; ++p) r.v[p] = sv[tt][mine + p];
+        r.b = DELTA || SELECTIVE ? sb[tt] : 0.f;
+      };
+      auto token = [&](const Token& r, int tt) __attribute__((always_inline)) {
+        float kv[P][2], dq[P][2], kq[2] = {0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < P; ++p) kv[p][0] = kv[p][1] = dq[p][0] = dq[p][1] = 0.f;
+#pragma unroll
+        for (int i = 0; i < DKL; ++i) {
+          kq[i & 1] = fmaf(BONUS ? ub[i] * r.k[i] : r.k[i], r.q[i], kq[i & 1]);
+#pragma unroll
+          for (int p = 0; p < P; ++p) {
+            if (BONUS) dq[p][i & 1] = fmaf(s[p][i], r.q[i], dq[p][i & 1]);
+            s[p][i] *= r.g[ONE_G ? 0 : i];
+            if (BONUS) continue;
+            if (DELTA) kv[p][i & 1] = fmaf(s[p][i], r.k[i], kv[p][i & 1]);
+            dq[p][i & 1] = fmaf(s[p][i], r.q[i], dq[p][i & 1]);
+          }
+        }
+        const float kqs = lanes_sum<RG>(kq[0] + kq[1]);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const float kvs = DELTA ? lanes_sum<RG>(kv[p][0] + kv[p][1]) : 0.f;
+      const float dqs = lanes_sum<RG>(dq[p][0] + dq[p][1]);
+      const float u = SELECTIVE ? r.b * r.v[p] : DELTA ? r.b * (r.v[p] - kvs) : r.v[p];
+#pragma unroll
+      for (int i = 0; i < DKL; ++i) s[p][i] = fmaf(r.k[i], u, s[p][i]);
+      const float y = SELECTIVE ? fmaf(pass, r.v[p], fmaf(u, kqs, dqs)) : fmaf(u, kqs, dqs);
+#pragma unroll
+      for (int j = 0; j < KEPT; ++j) o[j][p] = rg + j * RG == tt ? y : o[j][p];
+    }
+  };
+  auto tokens = [&](int nt) __attribute__((always_inline)) {
     if (nt == CH && CH > 1 && DKL <= 16) {
       // a whole chunk as straight code, each token read from LDS while the one before is computed
       Token even, odd;
@@ -632,41 +691,75 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
         token(r, tt);
       }
     }
-    __syncthreads();
-    for (int e = lane; e < nt * COLS; e += RB_WAVE) {
-      const int tt = e / COLS, c = e - tt * COLS;
-      if (col0 + c < vdim) out[((size_t)(row0 + t0 + tt) * n_heads + h) * vdim + col0 + c] = so[tt][c];
+  };
+  using Whole = std::integral_constant<bool, WIDE>;
+  using Any = std::false_type;
+  int t0 = 0;
+  if (no_pad && n >= CH) {
+    fetch(Whole{}, 0);
+    // the state is in registers now: a wait for it at its first use in the loop would be one for every chunk's values as well
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int i = 0; i < DKL; ++i) asm volatile("" : "+v"(s[p][i]));
+    for (; t0 + CH <= n; t0 += CH) {
+      __syncthreads();                                 // the chunk before has been read
+      place(Whole{}, CH);
+      __syncthreads();
+      if (t0 > 0) leave(Whole{}, t0 - CH);
+      if (t0 + 2 * CH <= n) fetch(Whole{}, t0 + CH);   // in flight while this chunk is computed
+      __builtin_amdgcn_sched_barrier(0);               // (issued here, not where the scheduler would sink them: at their use)
+      tokens(CH);
     }
+    leave(Whole{}, t0 - CH);
   }
-  if (quads) {
+  if (t0 < n) fetch(Any{}, t0);
+  for (; t0 < n; t0 += CH) {
+    const int nt = n - t0 < CH ? n - t0 : CH;
+    __syncthreads();
+    place(Any{}, nt);
+    __syncthreads();
+    if (t0 + CH < n) fetch(Any{}, t0 + CH);
+    __builtin_amdgcn_sched_barrier(0);
+    tokens(nt);
+    leave(Any{}, t0);
+  }
 #pragma unroll
-    for (int i = 0; i < DKL; i += 4) {
-      const int r = rg * DKL + i;
-      if (on && r < dim) *reinterpret_cast<float4*>(S + r) = make_float4(s[i], s[i + 1], s[i + 2], s[i + 3]);
-    }
-  } else {
+  for (int p = 0; p < P; ++p) {
+    if (quads) {
 #pragma unroll
-    for (int i = 0; i < DKL; ++i) {
-      const int r = rg * DKL + i;
-      if (on && r < dim) S[r] = s[i];
+      for (int i = 0; i < DKL; i += 4) {
+        const int r = rg * DKL + i;
+        if (col + p < vdim && r < dim) *reinterpret_cast<float4*>(S + (size_t)p * dim + r) = make_float4(s[p][i], s[p][i + 1], s[p][i + 2], s[p][i + 3]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < DKL; ++i) {
+        const int r = rg * DKL + i;
+        if (col + p < vdim && r < dim) S[(size_t)p * dim + r] = s[p][i];
+      }
     }
   }
 }
 
-template <int DKL, int RG, int CH, int MODE>
-static void launch_delta_rule(const float* q, const float* k, size_t qk_stride, const float* v, size_t v_stride,
-                              const float* g, size_t g_stride, const float* beta, float* state, const int32_t* cu_seqlens,
-                              const int32_t* slots, float* out, int n_seqs, int n_heads, int n_kv, int dim, int vdim,
-                              int g_per_head, const float* bonus, const SelectiveArgs& sel, hipStream_t s) {
-  constexpr int COLS = RB_WAVE / RG;
+// P: columns of a lane, where the values come wide (else 1).
+template <int DKL, int RG, int P, int CH, int MODE, bool ONE_G>
+static int launch_delta_rule(const float* q, const float* k, size_t qk_stride, const float* v, size_t v_stride,
+                             const float* g, size_t g_stride, const float* beta, float* state, const int32_t* cu_seqlens,
+                             const int32_t* slots, float* out, int n_seqs, int n_heads, int n_kv, int dim, int vdim,
+                             const float* bonus, const SelectiveArgs& sel, hipStream_t s) {
   static_assert((DKL * RG * CH) % RB_WAVE == 0 && CH <= RB_WAVE && DKL % 4 == 0, "a chunk's values are dealt evenly to the lanes");
-  dim3 grid(n_seqs, n_heads, (vdim + COLS - 1) / COLS);
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   constexpr bool MAY = CH > 1 && DKL * RG * CH / RB_WAVE % 4 == 0;
-  const bool wide = MAY && dim % 4 == 0 && qk_stride % 4 == 0 && aligned(q) && aligned(k) &&
-                    (MODE == 3 || g_per_head || (g_stride % 4 == 0 && aligned(g)));
-  (wide ? delta_rule_kernel<DKL, RG, CH, MODE, MAY> : delta_rule_kernel<DKL, RG, CH, MODE, false>)<<<grid, RB_WAVE, 0, s>>>(
-      q, k, qk_stride, v, v_stride, g, g_stride, beta, state, cu_seqlens, slots, out, n_heads, n_kv, dim, vdim, g_per_head, bonus, sel);
+  const bool wide = MAY && dim % 4 == 0 && qk_stride % 4 == 0 && aligned(q) && aligned(k) && (ONE_G || (g_stride % 4 == 0 && aligned(g))) &&
+                    (qk_stride | v_stride | (ONE_G ? 0 : g_stride)) < (1u << 24);      // (a chunk's places are offsets of 32 bits)
+  const int cols = RB_WAVE / RG * (wide ? P : 1), parts = (vdim + cols - 1) / cols;
+  RB_REQUIRE((long long)n_seqs * n_heads * parts <= 0x7fffffffLL, "rb_linear_recurrence: too many sequences, heads and value channels");
+  const int grid = n_seqs * n_heads * parts;
+  (wide ? delta_rule_kernel<DKL, RG, MAY ? P : 1, CH, MODE, ONE_G, MAY> : delta_rule_kernel<DKL, RG, 1, CH, MODE, ONE_G, false>)<<<grid, RB_WAVE, 0, s>>>(
+      q, k, qk_stride, v, v_stride, g, g_stride, beta, state, cu_seqlens, slots, out, n_heads, n_kv, dim, vdim, parts, bonus, sel);
+  RB_LAUNCH_CHECK();
+  return 0;
 }
 
 extern "C" int rb_delta_rule(const float* q, const float* k, long long qk_stride, const float* v, long long v_stride,
@@ -754,57 +847,53 @@ static int linear_recurrence_launch(const float* q, const float* k, long long qk
   // a step of one token per sequence (n_tokens == n_seqs) stages chunks of as few tokens as deal evenly to the lanes:
   // the machinery of a chunk of 16 would cost it several times its arithmetic
   const bool single = n_tokens <= n_seqs;
-#define DR_GO(DKL, RG, CH)                                                                                                  \
-  do {                                                                                                                      \
-    constexpr int CH1 = (DKL * RG >= RB_WAVE) ? 1 : RB_WAVE / (DKL * RG);                                                   \
-    if (single && selective)                                                                                                \
-      launch_delta_rule<DKL, RG, CH1, 3>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, out,        \
-                                         n_seqs, n_heads, n_kv_heads, dim, vdim, g_per_head, bonus, sel, s);                \
-    else if (selective)                                                                                                     \
-      launch_delta_rule<DKL, RG, CH, 3>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, out,         \
-                                        n_seqs, n_heads, n_kv_heads, dim, vdim, g_per_head, bonus, sel, s);                 \
-    else if (single && silu_in)                                                                                                  \
-      launch_delta_rule<DKL, RG, CH1, 2>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, out,        \
-                                         n_seqs, n_heads, n_kv_heads, dim, vdim, g_per_head, bonus, sel, s);                   \
-    else if (silu_in)                                                                                                       \
-      launch_delta_rule<DKL, RG, CH, 2>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, out,         \
-                                        n_seqs, n_heads, n_kv_heads, dim, vdim, g_per_head, bonus, sel, s);                    \
-    else if (single && bonus)                                                                                               \
-      launch_delta_rule<DKL, RG, CH1, 1>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, out,     \
-                                            n_seqs, n_heads, n_kv_heads, dim, vdim, g_per_head, bonus, sel, s);                \
-    else if (single)                                                                                                        \
-      launch_delta_rule<DKL, RG, CH1, 0>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, out,    \
-                                             n_seqs, n_heads, n_kv_heads, dim, vdim, g_per_head, bonus, sel, s);               \
-    else if (bonus)                                                                                                         \
-      launch_delta_rule<DKL, RG, CH, 1>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, out,      \
-                                           n_seqs, n_heads, n_kv_heads, dim, vdim, g_per_head, bonus, sel, s);                 \
-    else                                                                                                                    \
-      launch_delta_rule<DKL, RG, CH, 0>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, out,     \
-                                            n_seqs, n_heads, n_kv_heads, dim, vdim, g_per_head, bonus, sel, s);                \
+#define DR_MODE(DKL, RG, P, CH, MODE, ONE_G)                                                                                 \
+  return launch_delta_rule<DKL, RG, P, CH, MODE, ONE_G>(q, k, qs, v, vs, g, (size_t)g_stride, beta, state, cu_seqlens, slots, \
+                                                        out, n_seqs, n_heads, n_kv_heads, dim, vdim, bonus, sel, s)
+#define DR_LENGTH(DKL, RG, P, CH)                                   \
+  do {                                                              \
+    if (selective) DR_MODE(DKL, RG, P, CH, 3, true);                \
+    if (silu_in) DR_MODE(DKL, RG, P, CH, 2, true);                  \
+    if (bonus && g_per_head) DR_MODE(DKL, RG, 1, CH, 1, true);      \
+    if (bonus) DR_MODE(DKL, RG, P, CH, 1, false);                   \
+    if (beta && g_per_head) DR_MODE(DKL, RG, P, CH, 0, true);       \
+    if (beta) DR_MODE(DKL, RG, P, CH, 0, false);                    \
+    if (g_per_head) DR_MODE(DKL, RG, P, CH, 4, true);               \
+    DR_MODE(DKL, RG, P, CH, 4, false);                              \
+  } while (0)
+#define DR_GO(DKL, RG, P, CH)                                                             \
+  do {                                                                                    \
+    constexpr int CH1 = (DKL * RG >= RB_WAVE) ? 1 : RB_WAVE / (DKL * RG);                 \
+    if (single) DR_LENGTH(DKL, RG, 1, CH1);                                               \
+    DR_LENGTH(DKL, RG, P, CH);                                                            \
   } while (0)
   // Rows of a column over RG lanes, chunks as long as the registers that hold the next one allow.  A token's time is
   // its lane's share of the column, so while the waves do not fill the GPU's SIMDs a column goes to more lanes
-  // (more and shorter waves); once they do, fewer lanes per column save the moves between them.
+  // (more and shorter waves); once they do, fewer lanes per column save the moves between them.  Where they still do with two columns a
+  // lane, it has two: they share what the lane reads from LDS and the product of k and q, and the sums stay as they are (16 sequences of 400 tokens,
+  // 16 heads of 128 x 128, 437 us with one column a lane of 16, 325 with two of 8).
   const long long simds = 4LL * rb_compute_units();
-  auto waves = [&](int rg) { return (long long)n_seqs * n_heads * ((vdim + RB_WAVE / rg - 1) / (RB_WAVE / rg)); };
+  auto waves = [&](int cols) { return (long long)n_seqs * n_heads * ((vdim + cols - 1) / cols); };
   if (dim <= 16)
-    DR_GO(4, 4, 16);
+    DR_GO(4, 4, 1, 16);
   else if (dim <= 32) {
-    if (waves(4) >= simds) DR_GO(8, 4, 16);
-    else DR_GO(4, 8, 16);
+    if (waves(16) >= simds) DR_GO(8, 4, 1, 16);
+    else DR_GO(4, 8, 1, 16);
   } else if (dim <= 64) {
-    if (waves(8) >= simds) DR_GO(8, 8, 16);
-    else DR_GO(4, 16, 16);
+    if (waves(16) >= simds) DR_GO(8, 8, 2, 16);
+    else if (waves(8) >= simds) DR_GO(8, 8, 1, 16);
+    else DR_GO(4, 16, 1, 16);
   } else if (dim <= 128) {
-    if (waves(8) >= simds) DR_GO(16, 8, 16);
-    else DR_GO(8, 16, 16);
+    if (waves(16) >= simds) DR_GO(16, 8, 2, 16);
+    else if (waves(8) >= simds) DR_GO(16, 8, 1, 16);
+    else DR_GO(8, 16, 1, 16);
   } else if (dim <= 256)
-    DR_GO(16, 16, 8);
+    DR_GO(16, 16, 1, 8);
   else
-    DR_GO(32, 16, 4);
+    DR_GO(32, 16, 1, 4);
 #undef DR_GO
-  RB_LAUNCH_CHECK();
-  return 0;
+#undef DR_LENGTH
+#undef DR_MODE
 }
 
 // ---------------------------------------------------------------- read-out norm with gate

@@ -1,5 +1,7 @@
 """Kernels and branches of dispatches at the sizes where they can go wrong: edges of tiles, remainders, the smallest and the
 largest of their ranges, each against the same operation in float64."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -1301,6 +1303,63 @@ def test_single_tokens_through_a_recurrence_in_one_launch_give_the_same_bits(lib
         lib._lib.rb_tune_compute_units(0)
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+# ---------------------------------------------------------------------------- recurrences: whole chunks of 16 tokens and what is left
+@pytest.mark.parametrize("dim,vdim", [(64, 12), (64, 36), (128, 12), (128, 24), (128, 33), (96, 36)])
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("delta", [False, True])
+def test_recurrences_of_whole_and_partial_chunks_with_one_and_two_columns_a_lane(lib, dim, vdim, per_head, delta):
+    """Against the equations in float64 (1e-5 of the largest value bounds any order of float32 sums of 128 numbers over 50 tokens whose
+    decays shrink what came before).  How many compute units there are decides about two columns a lane of 8, one, and one of 16 lanes: the
+    first two give the same bits, and so does a step in two pieces."""
+    gen = torch.Generator().manual_seed(dim + vdim)
+    heads, kv, lengths, cuts = 4, 2, [1, 15, 16, 17, 31, 32, 33, 50], [1, 7, 16, 1, 16, 31, 17, 33]
+    n, cu = sum(lengths), [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    q, k = (torch.nn.functional.normalize(torch.randn(n, kv, dim, generator=gen), dim=-1) for _ in range(2))
+    v, beta = torch.randn(n, heads, vdim, generator=gen), torch.rand(n, heads, generator=gen)
+    g = 0.5 + 0.5 * torch.rand(n, heads, 1 if per_head else dim, generator=gen)
+    start = torch.randn(len(lengths), heads, vdim, dim, generator=gen) * 0.3
+
+    def run(units, steps):
+        state, out = start.to(DEV), torch.full((n, heads * vdim), float("nan"), device=DEV)
+        try:
+            lib._lib.rb_tune_compute_units(units)
+            for spans in steps:
+                pick = torch.cat([torch.arange(cu[b] + lo, cu[b] + hi) for b, (lo, hi) in enumerate(spans)])
+                seqs = [hi - lo for lo, hi in spans]
+                ctx = SimpleNamespace(n_tokens=len(pick), n_seqs=len(seqs), slots=torch.arange(len(seqs), dtype=torch.int32, device=DEV),
+                                      cu_seqlens=torch.tensor([sum(seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32, device=DEV))
+                qkv = torch.cat([t[pick].reshape(len(pick), -1) for t in (q, k, v)], 1).to(DEV)
+                part = torch.full((len(pick), heads * vdim), float("nan"), device=DEV)
+                lib.linear_recurrence(qkv, kv, dim, heads, vdim, g[pick].reshape(len(pick), -1).to(DEV), 0, per_head,
+                                      beta[pick].to(DEV) if delta else None, state, ctx, part)
+                out[pick.to(DEV)] = part
+        finally:
+            lib._lib.rb_tune_compute_units(0)
+        return out, state
+
+    whole = [[(0, m) for m in lengths]]
+    waves = lambda cols: len(lengths) * heads * -(-vdim // cols)
+    between = (waves(16) + waves(8)) // 2 // 4               # four SIMDs a compute unit
+    assert waves(16) < 4 * between <= waves(8) < 4 * 256
+    out, state = run(1, whole)
+    for other in (run(between, whole), run(1, [[(0, c) for c in cuts], [(c, m) for c, m in zip(cuts, lengths)]])):
+        assert torch.equal(out, other[0]) and torch.equal(state, other[1])
+    more_lanes = run(0, whole)
+    want, wanted = torch.empty(n, heads, vdim, dtype=torch.float64), start.double().clone()
+    for b, m in enumerate(lengths):
+        s = wanted[b]                                          # [H, vdim, dim]
+        for t in range(cu[b], cu[b] + m):
+            kk, qq = (x[t].double().repeat_interleave(heads // kv, 0)[:, None] for x in (k, q))
+            s *= g[t].double()[:, None]
+            u = v[t].double()
+            if delta:
+                u = beta[t].double()[:, None] * (u - (s * kk).sum(-1))
+            s += u[..., None] * kk
+            want[t] = (s * qq).sum(-1)
+    for got, ref in ((out, want), (state, wanted), (more_lanes[0], want), (more_lanes[1], wanted)):
+        _within(got.view(ref.shape), ref, 1e-5 * float(ref.abs().max()))
 
 
 # ---------------------------------------------------------------------------- the router's product and the choice in one launch
