@@ -330,11 +330,14 @@ int rb_route_top(const float* z, long long z_stride, int n_experts, int top, int
 int rb_routed_experts(const void* h, int dtype, const float* weight, int top, const int32_t* row_pair, const int32_t* tile_expert,
                       int max_rows, const void* w_gate, const void* w_up, const void* w_down, int w_layout, void* y, float* out,
                       int n_experts, int width, int ff, float limit, float alpha, void* stream);
-// The same for a step of at most 64 tokens with fragment-major experts: the same sums, bit for bit, in two launches.
+// The same for a step of at most 64 tokens with fragment-major experts: the same sums, bit for bit, in two launches.  Where
+// rb_routed_shared_ok says so an expert that every token uses goes with them: shared_out [T, width] float32 = act(h shared_up^T) shared_down^T, bfloat16
+// matrices [shared_ff, width] and [width, shared_ff] fragment-major, shared_units [T, shared_ff] scratch (shared_up null: none; no gate, no weight).
+int rb_routed_shared_ok(int n_tokens, int width, int expert_ff, int shared_ff);
 int rb_routed_experts_few(const void* h, const float* weight, int top, const int32_t* row_pair, const int32_t* tile_expert, int max_rows,
-                          int w_layout,
-                          const void* w_gate, const void* w_up, const void* w_down, void* y, float* out, int n_tokens, int n_experts,
-                          int width, int ff, float limit, float alpha, void* stream);
+                                 int w_layout, const void* w_gate, const void* w_up, const void* w_down, void* y, float* out, int n_tokens,
+                                 int n_experts, int width, int ff, float limit, float alpha, const void* shared_up, const void* shared_down,
+                                 const float* shared_act, void* shared_units, float* shared_out, int shared_ff, void* stream);
 // rb_route_top with its choices spelled out.  The router has n_outputs outputs, of which the first n_experts are experts
 // with matrices; a pair whose output lies behind them belongs to no run (rb_experts_combine gives it the token's input).
 // score 0: weight = sigmoid(z) of the chosen, chosen by z.  score 1: weight = softmax(z) over all outputs, chosen by

@@ -213,7 +213,8 @@ class Kernels:
             "rb_pair_norm_mean": [_P, _P, _P, _P, _F, _P, _I, _I, _P],
             "rb_route_top": [_P, _L, _I, _I, _P, _P, _P, _P, _I, _I, _P],
             "rb_routed_experts": [_P, _I, _P, _I, _P, _P, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _F, _F, _P],
-            "rb_routed_experts_few": [_P, _P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _F, _P],
+            "rb_routed_shared_ok": [_I, _I, _I, _I],
+            "rb_routed_experts_few": [_P, _P, _I, _P, _P, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _F, _P, _P, _P, _P, _P, _I, _P],
             "rb_pairs_sum": [_P, _I, _P, _I, _I, _P],
             "rb_route_choose": [_P, _L, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P],
             "rb_experts_combine": [_P, _P, _P, _I, _I, _P, _I, _P, _P, _L, _P, _I, _I, _P],
@@ -1057,10 +1058,11 @@ class Kernels:
 
     def routed_experts(self, h: torch.Tensor, weight: torch.Tensor, top: int, row_pair: torch.Tensor, tile_expert: torch.Tensor,
                        w_gate: Optional[torch.Tensor], w_up: Optional[torch.Tensor], w_down: torch.Tensor, y: torch.Tensor, out: torch.Tensor,
-                       limit: float, alpha: float, w_frag: bool = False) -> None:
+                       limit: float, alpha: float, w_frag: bool = False, shared=None) -> None:
         """w_frag: every expert's matrices are stored fragment-major (`place_rows(..., frag=True)` on each).  w_gate None: experts
         without a gate, Wd max(Wu x, 0)^2.  w_up None (w_frag): w_gate [experts, 2 ff, width] holds gate and up rows interleaved in
-        blocks of 16."""
+        blocks of 16.  shared (where `routed_shared_ok`): (up [shared ff, width] and down [width, shared ff] fragment-major, act float32 [2],
+        units [T, shared ff] as scratch, out [T, width] float32): an expert without a gate that every token uses, in the same launches."""
         n, width = h.shape
         n_experts, _, ff = w_down.shape
         layout = 0 if not w_frag else 1 if w_up is not None else 2
@@ -1077,14 +1079,32 @@ class Kernels:
         _check(w_down, "w_down", h.dtype, (n_experts, width, ff))
         _check(y, "y", h.dtype, (max_rows, ff + width))
         _check(out, "out", torch.float32, (n * top, width))
+        if shared is not None:
+            s_up, s_down, s_act, s_units, s_out = shared
+            s_ff = s_up.shape[0]
+            if not w_frag or not self.routed_shared_ok(n, width, ff, s_ff):
+                raise KernelError("routed_experts: this shared expert goes in launches of its own")
+            _check(s_up, "shared up", h.dtype, (s_ff, width))
+            _check(s_down, "shared down", h.dtype, (width, s_ff))
+            _check(s_act, "shared act", torch.float32, (2,))
+            _check(s_units, "shared units", h.dtype, (n, s_ff))
+            _check(s_out, "shared out", torch.float32, (n, width))
+        else:
+            s_up = s_down = s_act = s_units = s_out = None
+            s_ff = 0
         if w_frag and n <= ROUTED_FEW_TOKENS:
-            self._ok(self._lib.rb_routed_experts_few(_ptr(h), _ptr(weight), top, _ptr(row_pair), _ptr(tile_expert), max_rows, layout, _ptr(w_gate),
-                                                     _ptr(w_up), _ptr(w_down), _ptr(y), _ptr(out), n, n_experts, width, ff, float(limit),
-                                                     float(alpha), self._stream()))
+            self._ok(self._lib.rb_routed_experts_few(_ptr(h), _ptr(weight), top, _ptr(row_pair), _ptr(tile_expert), max_rows, layout,
+                                                            _ptr(w_gate), _ptr(w_up), _ptr(w_down), _ptr(y), _ptr(out), n, n_experts, width, ff,
+                                                            float(limit), float(alpha), _ptr(s_up), _ptr(s_down), _ptr(s_act), _ptr(s_units),
+                                                            _ptr(s_out), s_ff, self._stream()))
             return
         self._ok(self._lib.rb_routed_experts(_ptr(h), dtype_code(h.dtype), _ptr(weight), top, _ptr(row_pair), _ptr(tile_expert),
                                              max_rows, _ptr(w_gate), _ptr(w_up), _ptr(w_down), layout, _ptr(y), _ptr(out),
                                              n_experts, width, ff, float(limit), float(alpha), self._stream()))
+
+    def routed_shared_ok(self, n_tokens: int, width: int, expert_ff: int, shared_ff: int) -> bool:
+        """Whether `routed_experts` takes a shared expert of `shared_ff` units along (bfloat16, matrices fragment-major)."""
+        return bool(self._lib.rb_routed_shared_ok(n_tokens, width, expert_ff, shared_ff))
 
     def route_choose(self, z: torch.Tensor, n_outputs: int, n_experts: int, top: int, score: int,
                      correction: Optional[torch.Tensor], sel: torch.Tensor, weight: torch.Tensor, row_pair: torch.Tensor,

@@ -19,6 +19,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "gemm_internal.h"
 #include "mfma.h"
 
 #define RT_TILE 16
@@ -581,13 +582,78 @@ __device__ __forceinline__ void walk_ahead(int n_steps, const Load& load, const 
   }
 }
 
-template <int NT, bool WEIGHTED, bool GATED>
+// A shared expert's product C = X W^T beside the chosen experts' (at most 16 tokens, W fragment-major, K a multiple of 128): it waits for
+// nothing that they do, and as two launches of its own it was 64 and 128 workgroups between kernels that wait for each other.  16 rows of
+// W by one wave, which takes the shares of depth of the `waves` that the product alone has one after another and adds up their sums in the
+// same order: the same bits.  Bound by the chosen experts' matrices, which take longer than this wave's walk.  (A captured step of 4 tokens through 15
+// layers of 16 experts of 2,048 and a shared one of 1,024 at width 2,048 took 148 us longer with four launches a layer than with two: 4.9 us a launch.)
+struct SharedProduct {
+  const bf16_t *x, *w;
+  void* c;                   // bfloat16 with act, else float32
+  const float* act;          // xIELU's two numbers (see xielu_pair); null: the sums as they are
+  int n, k, m, waves;
+};
+__device__ __forceinline__ void shared_product(const SharedProduct& p, int tile) {
+  const int lane = threadIdx.x, r = lane & 15, kq = lane >> 4, n0 = 16 * tile;
+  if (n0 >= p.n) return;
+  const bf16_t* wr = p.w + (size_t)n0 * p.k + 8 * lane;
+  const bf16_t* xr = p.x + (size_t)(r < p.m ? r : 0) * p.k + 8 * kq;
+  const int total = p.k / 128, base = total / p.waves, extra = total % p.waves;
+  int wave = 0, left = base + (extra > 0 ? 1 : 0);         // stages of 128 that this share still has
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, sum = acc;
+  struct Ahead {
+    Frag8 w[RT_AHEAD], x[RT_AHEAD];
+  };
+  static_assert(RT_AHEAD % 4 == 0, "a trip is whole stages");
+  auto load = [&](Ahead& f, int s0, int cnt) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < RT_AHEAD; ++u) {
+      const size_t s = (size_t)(s0 + (u < cnt ? u : 0));
+      f.w[u].u = load16_stream(wr + 512 * s);
+      f.x[u].u = load16(xr + 32 * s);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](Ahead& f, int cnt) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < RT_AHEAD; ++u) {
+      if (u >= cnt) break;
+      acc = mfma16(f.w[u], f.x[u], acc);
+      if (u % 4 == 3 && --left == 0) {
+        sum = wave == 0 ? acc : sum + acc;
+        acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        ++wave;
+        left = base + (wave < extra ? 1 : 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  walk_ahead<true, Ahead>(p.k / 32, load, multiply);
+  if (r >= p.m) return;
+  const size_t to = (size_t)r * p.n + n0 + 4 * kq;
+  if (p.act) {
+    const XieluPair xa = xielu_pair(p.act);
+    *reinterpret_cast<uint2*>((bf16_t*)p.c + to) =
+        make_uint2(pack_bf16x2(xielu_value(sum[0], xa.ap, xa.an), xielu_value(sum[1], xa.ap, xa.an)),
+                   pack_bf16x2(xielu_value(sum[2], xa.ap, xa.an), xielu_value(sum[3], xa.ap, xa.an)));
+  } else {
+    *reinterpret_cast<f32x4_t*>((float*)p.c + to) = sum;
+  }
+}
+
+// SHARED: the first shared_y rows of the grid are a shared expert's product
+template <int NT, bool WEIGHTED, bool GATED, bool SHARED>
 __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __restrict__ h, const float* __restrict__ weight, int top,
                                                             const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
                                                             const int32_t* __restrict__ tile_pos, const bf16_t* __restrict__ w_gate,
                                                             const bf16_t* __restrict__ w_up, bf16_t* __restrict__ y, int width, int ff,
-                                                            float limit, float alpha, int n_tiles, int rows) {
-  const int t0 = blockIdx.y, e = tile_expert[t0];
+                                                            float limit, float alpha, int n_tiles, int rows, int shared_y,
+                                                            const SharedProduct shared) {
+  if (SHARED && (int)blockIdx.y < shared_y) {
+    shared_product(shared, blockIdx.y * gridDim.x + blockIdx.x);
+    return;
+  }
+  const int t0 = blockIdx.y - (SHARED ? shared_y : 0), e = tile_expert[t0];
   if (e < 0 || tile_pos[t0] % NT != 0) return;
   const int lane = threadIdx.x;
   const int c0 = blockIdx.x * 16;
@@ -650,12 +716,16 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
   }
 }
 
-template <int NT>
+template <int NT, bool SHARED>
 __global__ __launch_bounds__(RB_WAVE) void routed_down_few_kernel(const bf16_t* __restrict__ y, const int32_t* __restrict__ row_pair,
                                                               const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_pos,
                                                               const bf16_t* __restrict__ w_down, float* __restrict__ out, int width, int ff,
-                                                              int n_tiles) {
-  const int t0 = blockIdx.y, e = tile_expert[t0];
+                                                              int n_tiles, int shared_y, const SharedProduct shared) {
+  if (SHARED && (int)blockIdx.y < shared_y) {
+    shared_product(shared, blockIdx.y * gridDim.x + blockIdx.x);
+    return;
+  }
+  const int t0 = blockIdx.y - (SHARED ? shared_y : 0), e = tile_expert[t0];
   if (e < 0 || tile_pos[t0] % NT != 0) return;
   const int lane = threadIdx.x;
   const int c0 = blockIdx.x * 16;
@@ -886,13 +956,24 @@ extern "C" int rb_routed_experts(const void* h, int dtype, const float* weight, 
   return 0;
 }
 
+// Whether a shared expert of `ff` units goes into those two launches: at most 16 tokens, sums that a product of its sizes alone takes in the same
+// order, and a walk along the depth no longer than the experts' own.
+extern "C" int rb_routed_shared_ok(int n_tokens, int width, int expert_ff, int shared_ff) {
+  return n_tokens >= 1 && n_tokens <= RT_TILE && width % 128 == 0 && shared_ff > 0 && shared_ff % 128 == 0 && shared_ff <= expert_ff &&
+         gemm_sums_alone_alike(n_tokens, shared_ff, width) && gemm_sums_alone_alike(n_tokens, width, shared_ff);
+}
+
 // rb_routed_experts for a step of at most 64 tokens with fragment-major experts (bfloat16, sizes that are multiples of 32): the
 // same sums in the same order, two launches whose waves keep more of the experts' matrices on their way.  n_tokens: rows of h.
+// Beside them, an expert that every token uses (no gate; shared_up [shared_ff, width] and shared_down [width, shared_ff] bfloat16, fragment-major):
+// shared_out [T, width] float32 = act(h shared_up^T) shared_down^T, shared_units [T, shared_ff] bfloat16 in between; shared_up null: without.
 extern "C" int rb_routed_experts_few(const void* h, const float* weight, int top, const int32_t* row_pair, const int32_t* tile_expert,
-                                     int max_rows, int w_layout, const void* w_gate, const void* w_up, const void* w_down, void* y, float* out,
-                                     int n_tokens, int n_experts, int width, int ff, float limit, float alpha, void* stream) {
+                                            int max_rows, int w_layout, const void* w_gate, const void* w_up, const void* w_down, void* y,
+                                            float* out, int n_tokens, int n_experts, int width, int ff, float limit, float alpha,
+                                            const void* shared_up, const void* shared_down, const float* shared_act, void* shared_units,
+                                            float* shared_out, int shared_ff, void* stream) {
   RB_RECORDED(rb_routed_experts_few(h, weight, top, row_pair, tile_expert, max_rows, w_layout, w_gate, w_up, w_down, y, out, n_tokens, n_experts, width,
-                                    ff, limit, alpha, stream));
+                                           ff, limit, alpha, shared_up, shared_down, shared_act, shared_units, shared_out, shared_ff, stream));
   const int rows = w_layout == 2 ? 2 : 1;
   RB_REQUIRE(w_layout == 1 || (w_layout == 2 && w_gate && !w_up), "rb_routed_experts_few: layout %d of the experts", w_layout);
   if (w_layout == 2) w_up = (const bf16_t*)w_gate + (size_t)16 * width;
@@ -903,16 +984,36 @@ extern "C" int rb_routed_experts_few(const void* h, const float* weight, int top
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   RB_REQUIRE(aligned(h) && aligned(w_gate) && aligned(w_up) && aligned(w_down) && aligned(y) && aligned(out),
              "rb_routed_experts_few: operands must be 16-byte aligned");
+  RB_REQUIRE(!shared_up || (shared_down && shared_act && shared_units && shared_out && !w_gate && !weight &&
+                            rb_routed_shared_ok(n_tokens, width, ff, shared_ff)),
+             "rb_routed_experts_few: a shared expert of %d units beside experts of %d is not for it", shared_ff, ff);
+  RB_REQUIRE(aligned(shared_up) && aligned(shared_down) && aligned(shared_units) && aligned(shared_out),
+             "rb_routed_experts_few: the shared expert's operands must be 16-byte aligned");
   if (max_rows == 0 || n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const int tiles = max_rows / RT_TILE;
+  if (shared_up) {
+    const SharedProduct up = {(const bf16_t*)h, (const bf16_t*)shared_up, shared_units, shared_act, shared_ff, width, n_tokens,
+                              gemm_skinny_waves(shared_ff, width)};
+    const SharedProduct down = {(const bf16_t*)shared_units, (const bf16_t*)shared_down, shared_out, nullptr, width, shared_ff, n_tokens,
+                                gemm_skinny_waves(width, shared_ff)};
+    const int uy = (shared_ff / 16 + ff / 16 - 1) / (ff / 16);       // its tiles in rows of the experts' grid; down: one row
+    RB_REQUIRE(tiles + uy <= 65535, "rb_routed_experts_few: too many rows");
+    routed_up_few_kernel<1, false, false, true><<<dim3(ff / 16, tiles + uy), RB_WAVE, 0, s>>>(
+        (const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles, nullptr, (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha,
+        tiles, rows, uy, up);
+    routed_down_few_kernel<1, true><<<dim3(width / 16, tiles + 1), RB_WAVE, 0, s>>>(
+        (const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles, (const bf16_t*)w_down, out, width, ff, tiles, 1, down);
+    RB_LAUNCH_CHECK();
+    return 0;
+  }
   const dim3 gu(ff / 16, tiles), gd(width / 16, tiles);      // (both are multiples of 32)
 #define RT_UP(NT, WEIGHTED)                                                                                                           \
-  (w_gate ? routed_up_few_kernel<NT, WEIGHTED, true> : routed_up_few_kernel<NT, WEIGHTED, false>)<<<gu, RB_WAVE, 0, s>>>((const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles,    \
-                                                        (const bf16_t*)w_gate, (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha, tiles, rows)
+  (w_gate ? routed_up_few_kernel<NT, WEIGHTED, true, false> : routed_up_few_kernel<NT, WEIGHTED, false, false>)<<<gu, RB_WAVE, 0, s>>>((const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles,    \
+                                                        (const bf16_t*)w_gate, (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha, tiles, rows, 0, SharedProduct{})
 #define RT_DOWN(NT)                                                                                                       \
-  routed_down_few_kernel<NT><<<gd, RB_WAVE, 0, s>>>((const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles,             \
-                                                (const bf16_t*)w_down, out, width, ff, tiles)
+  routed_down_few_kernel<NT, false><<<gd, RB_WAVE, 0, s>>>((const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles,             \
+                                                (const bf16_t*)w_down, out, width, ff, tiles, 0, SharedProduct{})
   if (n_tokens <= RT_TILE) {                  // a token chooses an expert once: no run is longer than the step's tokens
     if (weight) RT_UP(1, true);
     else RT_UP(1, false);

@@ -166,6 +166,8 @@ class RoutedExperts(Part):
                     lib.place_rows(tensors[self._name(i, what)].contiguous(), out[i], row0, GATE_BLOCK, 2 * GATE_BLOCK, frag=True)
             return out
 
+        # few tokens: a shared expert without a gate goes in the chosen experts' launches
+        self.shared_along = bool(self.frag and isinstance(self.shared, DenseAct) and self.shared.w_up.frag and self.shared.w_down.frag)
         # a step of many tokens runs on the dense product's tiles
         gated = self.unit == "gated"
         self.tiled = bool(self.frag and self.hidden % 64 == 0 and self.ff % 64 == 0)
@@ -207,6 +209,7 @@ class RoutedExperts(Part):
             lib.route_choose(z, self.n_outputs, self.n_experts, self.top, self.score, self.correction, sel, weight, row_pair,
                              tile_expert, bias=self.bias, unit=unit)
         out = torch.empty((n_pairs, self.hidden), dtype=torch.float32, device=dev)
+        both = None                                           # what the shared expert gives
         if tiled:
             gated = self.w_gate is not None
             y = torch.empty((max_rows, self.ff), dtype=h.dtype, device=dev)
@@ -214,15 +217,20 @@ class RoutedExperts(Part):
                                      self.act, y, out, weight if self.weight_on == "input" else None)
         else:
             y = torch.empty((max_rows, self.ff + self.hidden), dtype=h.dtype, device=dev)     # scratch: gated units, scaled inputs
+            along = None
+            if self.shared_along and lib.routed_shared_ok(t, self.hidden, self.ff, self.shared.ff):
+                s, both = self.shared, torch.empty((t, self.hidden), dtype=torch.float32, device=dev)
+                along = (s.w_up.data, s.w_down.data, s.act, torch.empty((t, s.ff), dtype=h.dtype, device=dev), both)
             lib.routed_experts(h, weight if self.weight_on == "input" else None, self.top, row_pair, tile_expert, self.w_gate,
-                               self.w_up, self.w_down, y, out, self.limit or 0.0, self.alpha, w_frag=self.frag)
+                               self.w_up, self.w_down, y, out, self.limit or 0.0, self.alpha, w_frag=self.frag, shared=along)
+        if self.shared is not None and both is None:
+            both = self.shared.forward(h, ctx)
         if pairs:
             if not (self.leaves_pairs or self.leaves_shared_pairs):
                 raise ConfigError("routed experts: only a plain weighted sum of the experts' outputs can be left to its reader")
-            return ExpertPairs(out, weight, None if self.shared is None else self.shared.forward(h, ctx))
+            return ExpertPairs(out, weight, both)
         if self.weight_on == "output":
             total = torch.empty((t, self.hidden), dtype=torch.float32, device=dev)
-            both = None if self.shared is None else self.shared.forward(h, ctx)
             lib.experts_combine(out, sel, weight, self.top, self.n_experts, h, both, z if self.shared_gate else None,
                                 self.n_outputs, total)
             return total

@@ -1418,6 +1418,27 @@ def test_routers_of_many_rows_keep_a_product_of_their_own(lib, monkeypatch, expe
     assert torch.equal(part.forward(h), got)
 
 
+# ---------------------------------------------------------------------------- a shared expert in the chosen experts' launches
+@pytest.mark.parametrize("n", [1, 4, 16, 17])
+@pytest.mark.parametrize("hidden,ff,shared,along", [(128, 128, 128, True), (384, 256, 128, True), (2048, 1024, 1024, True), (1152, 640, 640, True),
+                                                    (256, 128, 256, False), (256, 192, 160, False)])
+def test_a_shared_expert_in_the_chosen_experts_launches_gives_the_bits_of_its_own(lib, n, hidden, ff, shared, along):
+    gen = torch.Generator().manual_seed(hidden + n)
+    params = {"experts": 4, "top": 2, "intermediate_size": ff, "score": "softmax", "weight_on": "output", "unit": "squared_relu",
+              "shared": {"intermediate_size": shared, "gate": False}}
+    part = build_part("feed_forward", PartSpec("routed_experts", params), BuildEnv(hidden_size=hidden, dtype=torch.bfloat16, device=torch.device(DEV), lib=lib))
+    part.load({name: (torch.randn(ts.shape, generator=gen) * ts.shape[-1] ** -0.5).to(torch.float32 if ts.role == "gain" else torch.bfloat16).to(DEV)
+               for name, ts in part.tensor_specs().items()})
+    h = torch.randn(n, hidden, generator=gen).bfloat16().to(DEV)
+    assert part.shared_along == (shared % 64 == 0)
+    assert lib.routed_shared_ok(n, hidden, ff, shared) == (along and n <= 16)
+    got = part.forward(h, pairs=True)
+    part.shared_along = False
+    want = part.forward(h, pairs=True)
+    for a, b in ((got.outputs, want.outputs), (got.weights, want.weights), (got.shared, want.shared)):
+        assert torch.equal(a, b)
+
+
 # ---------------------------------------------------------------------------- products of few tokens in one launch
 @pytest.mark.parametrize("m", [1, 4, 16])
 @pytest.mark.parametrize("k", [128, 384, 2048, 8192])
