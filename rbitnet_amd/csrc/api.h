@@ -165,6 +165,13 @@ int rb_streams_update_layernorm(float* x, int n_streams, long long stream_stride
                                 const float* y, const float* scale, const float* coef, const float* delta, const float* weight,
                                 const float* bias, float eps, const int32_t* rows, int n_rows, int width, void* out,
                                 int out_dtype, void* stream);      // rb_streams_update (mix null: none), then the norm, in one pass
+// The same for single tokens, the result then going through rb_short_conv with the residual (conv_w [E, taps], conv_state [slots, taps - 1, E], row r
+// in slots[r]): the same numbers.  rb_streams_conv_ok: whether these sizes are for it.
+int rb_streams_conv_ok(int width, int taps);
+int rb_streams_update_layernorm_conv(float* x, int n_streams, long long stream_stride, const float* mix, const float* out_coef,
+                                     const float* y, const float* scale, const float* coef, const float* weight, const float* bias, float eps,
+                                     const float* conv_w, int taps, float* conv_state, const int32_t* slots, int n_rows, int width, void* out,
+                                     int out_dtype, void* stream);
 // rb_embed_streams with x[s][t, :] = table[ids[t], :] * scale + wave(tok_pos[t]): number 2i of wave(p) is sin(p inv[i]), number 2i + 1
 // cos(p inv[i]); inv float64 [(width + 1) / 2], null: no wave.  table_layout 0: rows, 1: fragment-major (a table that is the output
 // matrix as well).

@@ -184,6 +184,8 @@ class Kernels:
             "rb_embed_streams": [_P, _I, _P, _P, _I, _L, _I, _I, _P],
             "rb_streams_layernorm": [_P, _I, _L, _P, _P, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_streams_update_layernorm": [_P, _I, _L, _P, _P, _P, _P, _P, _P, _P, _P, _F, _P, _I, _I, _P, _I, _P],
+            "rb_streams_conv_ok": [_I, _I],
+            "rb_streams_update_layernorm_conv": [_P, _I, _L, _P, _P, _P, _P, _P, _P, _P, _F, _P, _I, _P, _P, _I, _I, _P, _I, _P],
             "rb_streams_update": [_P, _I, _L, _P, _P, _P, _P, _I, _I, _P],
             "rb_embed_streams_waves": [_P, _I, _I, _P, _F, _P, _P, _P, _I, _L, _I, _I, _P],
             "rb_streams_rmsnorm": [_P, _I, _L, _P, _P, _P, _I, _L, _L, _P, _P, _I, _L, _P, _P, _F, _P, _I, _I, _P, _I, _P],
@@ -621,10 +623,11 @@ class Kernels:
 
     def streams_layernorm(self, x: torch.Tensor, coef: Optional[torch.Tensor], weight: torch.Tensor,
                           bias: Optional[torch.Tensor], eps: float, rows: Optional[torch.Tensor], out: torch.Tensor,
-                          delta: Optional[torch.Tensor] = None, update=None) -> None:
+                          delta: Optional[torch.Tensor] = None, update=None, conv=None) -> None:
         """x [S, T, E] (or [T, E]: one stream) float32; out [rows or T, E]: the layer norm of sum_s coef[s] x[s].
         update (mix [S, S], out_coef [S], y [T, E], scale [E] or None): `streams_update` with these first, in the same
-        pass (every row, so rows must be None)."""
+        pass (every row, so rows must be None).  conv (w [E, taps], state [slots, taps - 1, E], ctx; a step of one token per sequence, sizes that
+        `streams_conv_ok`): the float32 result goes through `short_conv` with the residual, in the same pass."""
         if x.dim() == 2:
             x = x.unsqueeze(0)
         s_, n, width = x.shape
@@ -651,9 +654,30 @@ class Kernels:
             _check(y, "y", torch.float32, (n, width))
             if scale is not None:
                 _check(scale, "scale", torch.float32, (width,))
+        if conv is not None:
+            w, state, ctx = conv
+            if rows is not None or delta is not None or ctx.n_tokens != n or ctx.n_seqs != n or ctx.max_q_len != 1:
+                raise KernelError("streams_layernorm: a convolution goes with steps of one token per sequence, all rows")
+            _check(w, "w", torch.float32, (width, w.shape[1]))
+            _check(state, "conv state", torch.float32)
+            if tuple(state.shape[1:]) != (w.shape[1] - 1, width):
+                raise KernelError(f"streams_layernorm: convolution state of shape {tuple(state.shape)}")
+            if any(p is not None and p.data_ptr() % 16 for p in (x, y, scale, weight, bias, w, state, out)):      # rows that are not whole pieces of 16 bytes
+                row = torch.empty((n, width), dtype=torch.float32, device=x.device)
+                self.streams_layernorm(x, coef, weight, bias, eps, None, row, update=update)
+                self.short_conv(row, 0, width, w, state, ctx, out, True, 0)
+                return
+            self._ok(self._lib.rb_streams_update_layernorm_conv(_ptr(x), s_, n * width, _ptr(mix), _ptr(out_coef), _ptr(y), _ptr(scale),
+                                                                _ptr(coef), _ptr(weight), _ptr(bias), float(eps), _ptr(w), w.shape[1],
+                                                                _ptr(state), _ptr(ctx.slots), n, width, _ptr(out), dtype_code(out.dtype),
+                                                                self._stream()))
+            return
         self._ok(self._lib.rb_streams_update_layernorm(_ptr(x), s_, n * width, _ptr(mix), _ptr(out_coef), _ptr(y), _ptr(scale),
                                                        _ptr(coef), _ptr(delta), _ptr(weight), _ptr(bias), float(eps), _ptr(rows),
                                                        n_rows, width, _ptr(out), dtype_code(out.dtype), self._stream()))
+
+    def streams_conv_ok(self, width: int, taps: int) -> bool:
+        return bool(self._lib.rb_streams_conv_ok(width, taps))
 
     def streams_update(self, x: torch.Tensor, mix: torch.Tensor, out_coef: torch.Tensor, y: torch.Tensor,
                        scale: Optional[torch.Tensor]) -> None:

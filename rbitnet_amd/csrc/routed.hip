@@ -586,7 +586,7 @@ __device__ __forceinline__ void walk_ahead(int n_steps, const Load& load, const 
 // nothing that they do, and as two launches of its own it was 64 and 128 workgroups between kernels that wait for each other.  16 rows of
 // W by one wave, which takes the shares of depth of the `waves` that the product alone has one after another and adds up their sums in the
 // same order: the same bits.  Bound by the chosen experts' matrices, which take longer than this wave's walk.  (A captured step of 4 tokens through 15
-// layers of 16 experts of 2,048 and a shared one of 1,024 at width 2,048 took 148 us longer with four launches a layer than with two: 4.9 us a launch.)
+// layers of 16 experts of 2,048 and a shared one of 1,024 at width 2,048 took 120 us longer with four launches a layer than with two: 4 us a launch.)
 struct SharedProduct {
   const bf16_t *x, *w;
   void* c;                   // bfloat16 with act, else float32

@@ -93,12 +93,22 @@ __device__ __forceinline__ void st4(bf16_t* p, float a, float b, float c, float 
 // more, which stay in registers.  A step of few tokens pays for every barrier and for code that comes from memory: the copies'
 // coefficients are scalar loads, and the two reductions have scratch of their own.  (4 rows of 2,048, four copies updated: 7.2 us for any
 // number of copies by way of LDS, 3.8 here, one copy 5.5 and 3.3; 3,781 rows: four copies 70 and 44, one 46 and 21.)
-template <typename TO, int NS, bool ONE>
+//
+// KEEP > 0 (with ONE, single tokens): what leaves is h + conv(h), h the normalised row and conv the causal convolution of KEEP + 1 taps of rb_short_conv,
+// whose last inputs move on; the same numbers as with a launch of its own, which cost a captured step of
+// 4 tokens at width 2,048 2.4 us a layer (16 layers: 1,035 -> 997).
+struct StreamConv {
+  const float* w;              // [width, KEEP + 1]
+  float* state;                // [slots, KEEP, width]
+  const int32_t* slots;        // row r's
+};
+template <typename TO, int NS, bool ONE, int KEEP = 0>
 __global__ __launch_bounds__(1024) void streams_layernorm_vec_kernel(
     float* __restrict__ x, int n_copies, size_t stream_stride, const float* __restrict__ coef, const float* __restrict__ delta,
     const float* __restrict__ weight, const float* __restrict__ bias, float eps, const int32_t* __restrict__ rows, int width,
     TO* __restrict__ out, const float* __restrict__ mix, const float* __restrict__ out_coef, const float* __restrict__ y,
-    const float* __restrict__ scale, const float* __restrict__ delta2, float dscale) {
+    const float* __restrict__ scale, const float* __restrict__ delta2, float dscale, const StreamConv conv) {
+  static_assert(KEEP == 0 || ONE, "a convolution behind the norm is for rows that stay in registers");
   extern __shared__ float u[];
   __shared__ float sums[2][16];
   constexpr int MOST = NS > 0 ? NS : ST_MAX_STREAMS;
@@ -176,6 +186,19 @@ __global__ __launch_bounds__(1024) void streams_layernorm_vec_kernel(
     w0 = ld4(weight + j0);
     if (bias) b0 = ld4(bias + j0);
   }
+  float taps[KEEP > 0 ? 4 * (KEEP + 1) : 1];
+  float4 win[KEEP > 0 ? KEEP : 1];
+  float* st = nullptr;
+  if (KEEP > 0 && j0 < width) {
+    st = conv.state + (size_t)conv.slots[r] * KEEP * width + j0;
+#pragma unroll
+    for (int i = 0; i <= KEEP; ++i) {
+      const float4 v = ld4(conv.w + (size_t)j0 * (KEEP + 1) + 4 * i);
+      taps[4 * i] = v.x, taps[4 * i + 1] = v.y, taps[4 * i + 2] = v.z, taps[4 * i + 3] = v.w;
+    }
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) win[i] = ld4(st + (size_t)i * width);
+  }
   __builtin_amdgcn_sched_barrier(0);
   const float mean = total(sum, sums[0]) / (float)width;
   float ss = 0.f;
@@ -195,6 +218,20 @@ __global__ __launch_bounds__(1024) void streams_layernorm_vec_kernel(
       const float4 bv = j == j0 ? b0 : ld4(bias + j);
       o = make_float4(o.x + bv.x, o.y + bv.y, o.z + bv.z, o.w + bv.w);
     }
+    if constexpr (KEEP > 0) {
+      const float cur[4] = {o.x + 0.f, o.y + 0.f, o.z + 0.f, o.w + 0.f};      // (as rb_short_conv, whose inputs have a bias of zero)
+      float y4[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        y4[i] = fmaf(taps[i * (KEEP + 1) + KEEP], cur[i], cur[i]);
+#pragma unroll
+        for (int q = 0; q < KEEP; ++q) y4[i] = fmaf(taps[i * (KEEP + 1) + q], i == 0 ? win[q].x : i == 1 ? win[q].y : i == 2 ? win[q].z : win[q].w, y4[i]);
+      }
+      o = make_float4(y4[0], y4[1], y4[2], y4[3]);
+#pragma unroll
+      for (int q = 0; q + 1 < KEEP; ++q) *reinterpret_cast<float4*>(st + (size_t)q * width) = win[q + 1];
+      *reinterpret_cast<float4*>(st + (size_t)(KEEP - 1) * width) = make_float4(cur[0], cur[1], cur[2], cur[3]);
+    }
     st4(orow + j, o.x, o.y, o.z, o.w);
     if (ONE) break;
   }
@@ -213,7 +250,7 @@ extern "C" int rb_streams_layernorm(float* x, int n_streams, long long stream_st
 static int layernorm_launch(float* x, int n_streams, long long stream_stride, const float* mix, const float* out_coef, const float* y,
                             const float* scale, const float* coef, const float* delta, const float* delta2, float dscale,
                             const float* weight, const float* bias, float eps, const int32_t* rows, int n_rows, int width, void* out,
-                            int out_dtype, void* stream);
+                            int out_dtype, void* stream, const StreamConv& conv = StreamConv{nullptr, nullptr, nullptr}, int taps = 0);
 
 extern "C" int rb_streams_update_layernorm(float* x, int n_streams, long long stream_stride, const float* mix,
                                            const float* out_coef, const float* y, const float* scale, const float* coef,
@@ -224,6 +261,24 @@ extern "C" int rb_streams_update_layernorm(float* x, int n_streams, long long st
                                           rows, n_rows, width, out, out_dtype, stream));
   return layernorm_launch(x, n_streams, stream_stride, mix, out_coef, y, scale, coef, delta, nullptr, 1.0f, weight, bias, eps, rows,
                           n_rows, width, out, out_dtype, stream);
+}
+
+// Whether a norm of rows of `width` takes the convolution of so many taps behind it along.
+extern "C" int rb_streams_conv_ok(int width, int taps) { return width > 0 && width % 4 == 0 && width <= 4096 && taps >= 2 && taps <= 4; }
+
+// rb_streams_update_layernorm of single tokens, then out[r] = h + conv(h) as rb_short_conv with the residual makes it of h, the normalised float32
+// row: conv_w [width, taps], conv_state [slots, taps - 1, width], row r being the one token of the sequence in slots[r].
+extern "C" int rb_streams_update_layernorm_conv(float* x, int n_streams, long long stream_stride, const float* mix, const float* out_coef,
+                                                const float* y, const float* scale, const float* coef, const float* weight, const float* bias,
+                                                float eps, const float* conv_w, int taps, float* conv_state, const int32_t* slots, int n_rows,
+                                                int width, void* out, int out_dtype, void* stream) {
+  RB_RECORDED(rb_streams_update_layernorm_conv(x, n_streams, stream_stride, mix, out_coef, y, scale, coef, weight, bias, eps, conv_w, taps,
+                                               conv_state, slots, n_rows, width, out, out_dtype, stream));
+  auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  RB_REQUIRE(rb_streams_conv_ok(width, taps) && conv_w && conv_state && slots && aligned(conv_w) && aligned(conv_state),
+             "rb_streams_update_layernorm_conv: %d taps behind rows of %d are not for it", taps, width);
+  return layernorm_launch(x, n_streams, stream_stride, mix, out_coef, y, scale, coef, nullptr, nullptr, 1.0f, weight, bias, eps, nullptr, n_rows,
+                          width, out, out_dtype, stream, StreamConv{conv_w, conv_state, slots}, taps);
 }
 
 // Layer norm of a plain stream x [T, E] with the residual sum that was still to be done, in one pass:
@@ -241,7 +296,7 @@ extern "C" int rb_layernorm_residual(float* x, const float* delta, const float* 
 static int layernorm_launch(float* x, int n_streams, long long stream_stride, const float* mix, const float* out_coef, const float* y,
                             const float* scale, const float* coef, const float* delta, const float* delta2, float dscale,
                             const float* weight, const float* bias, float eps, const int32_t* rows, int n_rows, int width, void* out,
-                            int out_dtype, void* stream) {
+                            int out_dtype, void* stream, const StreamConv& conv, int taps) {
   RB_REQUIRE(mix == nullptr || (rows == nullptr && out_coef != nullptr && y != nullptr),
              "rb_streams_update_layernorm: an update takes every row and needs out_coef and y");
   RB_REQUIRE(n_rows >= 0 && width > 0 && width <= 16384, "rb_streams_layernorm: bad sizes %d x %d (width at most 16384)", n_rows, width);
@@ -255,12 +310,22 @@ static int layernorm_launch(float* x, int n_streams, long long stream_stride, co
       aligned(y) && aligned(scale) && (out_dtype == RB_F32 || out_dtype == RB_BF16)) {
     int threads = ((width / 4 + RB_WAVE - 1) / RB_WAVE) * RB_WAVE;
     if (threads > 1024) threads = 1024;
-#define ST_GO(TO, NS, ONE)                                                                                                              \
-  streams_layernorm_vec_kernel<TO, NS, ONE><<<n_rows, threads, (ONE) ? 0 : lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight, bias, \
-                                                                                    eps, rows, width, (TO*)out, mix, out_coef, y, scale, delta2, dscale)
+#define ST_CONV(TO, NS, ONE, KEEP)                                                                                                                  \
+  streams_layernorm_vec_kernel<TO, NS, ONE, KEEP><<<n_rows, threads, (ONE) ? 0 : lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight,  \
+                                                                                          bias, eps, rows, width, (TO*)out, mix, out_coef, y, scale, \
+                                                                                          delta2, dscale, conv)
+#define ST_GO(TO, NS, ONE) ST_CONV(TO, NS, ONE, 0)
+#define ST_BY_TAPS(TO, NS)                        \
+  do {                                            \
+    if (taps == 2) ST_CONV(TO, NS, true, 1);      \
+    else if (taps == 3) ST_CONV(TO, NS, true, 2); \
+    else ST_CONV(TO, NS, true, 3);                \
+  } while (0)
 #define ST_BY_COPIES(TO)                                \
   do {                                                  \
-    if (width > 4 * threads) ST_GO(TO, 0, false);       \
+    if (taps && n_streams == 2) ST_BY_TAPS(TO, 2);      \
+    else if (taps) ST_BY_TAPS(TO, 0);                   \
+    else if (width > 4 * threads) ST_GO(TO, 0, false);  \
     else if (n_streams == 1) ST_GO(TO, 1, true);        \
     else if (n_streams == 2) ST_GO(TO, 2, true);        \
     else if (n_streams == 4) ST_GO(TO, 4, true);        \
@@ -269,10 +334,13 @@ static int layernorm_launch(float* x, int n_streams, long long stream_stride, co
     if (out_dtype == RB_F32) ST_BY_COPIES(float);
     else ST_BY_COPIES(bf16_t);
 #undef ST_BY_COPIES
+#undef ST_BY_TAPS
 #undef ST_GO
+#undef ST_CONV
     RB_LAUNCH_CHECK();
     return 0;
   }
+  RB_REQUIRE(taps == 0, "rb_streams_update_layernorm_conv: rows of 16 bytes only");
   if (out_dtype == RB_F32)
     streams_layernorm_kernel<float><<<n_rows, 256, lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight, bias, eps,
                                                              rows, width, (float*)out, mix, out_coef, y, scale, delta2, dscale);

@@ -84,6 +84,9 @@ class HyperBlock:
         self.sublayers = (1, 2) if self.feed_forward is not None else (1,)
         conv = params.get("input_conv")
         self.conv = ShortConv(self.hidden, int(conv["taps"]), env, residual=True, act=ACT_NONE) if conv else None
+        # steps of one token per sequence: norm and convolution in one launch
+        self.conv_in_norm = (conv is not None and getattr(self.norm1, "takes_conv", False) and not getattr(env, "generic_only", False)
+                             and env.lib is not None and env.lib.streams_conv_ok(self.hidden, self.conv.taps))
         self.conv_name = str(conv.get("name", "input_conv")) if conv else None
         self.own = _OwnTensors(self)
         self.coef: Dict[int, Dict[str, torch.Tensor]] = {}
@@ -151,7 +154,9 @@ class HyperBlock:
             raise ConfigError("a layer with the stream in several copies cannot follow one that leaves a plain term to be added")
         dt = self.env.dtype
         c = self.coef[1]
-        if self.conv is not None:
+        if self.conv is not None and self.conv_in_norm and ctx.max_q_len == 1:
+            h = self.norm1.forward(x, pending, None, coef=c["in"], out_dtype=dt, conv=(self.conv.weight, view.states["input_conv"], ctx))
+        elif self.conv is not None:
             hn = self._norm(self.norm1, x, pending, c["in"], torch.float32)
             h = self.conv.forward(hn, ctx, view.states.get("input_conv"), dt)
         else:

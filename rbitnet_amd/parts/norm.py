@@ -93,6 +93,7 @@ class LayerNorm(Part):
     graph_safe = True
     plan_safe = True
     reads_copies = True
+    takes_conv = True             # forward takes conv: what `short_conv` makes of the result, for single tokens
     adds_scaled_sum = True        # delta may be a ScaledSum: scale * (a + b), added in the norm's own pass
 
     def __init__(self, params: Dict, env: BuildEnv):
@@ -119,7 +120,7 @@ class LayerNorm(Part):
         self.bias = tensors[self.names["bias"]] if self.has_bias else None
 
     def forward(self, x: torch.Tensor, delta: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None,
-                coef: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+                coef: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None, conv=None) -> torch.Tensor:
         t = x.shape[-2]
         n = t if rows is None else rows.shape[0]
         out = torch.empty((n, self.size), dtype=out_dtype or self.env.dtype, device=x.device)
@@ -134,7 +135,7 @@ class LayerNorm(Part):
             else:
                 delta.apply(x)                            # only some rows are normalised: all are updated first
                 delta = None
-        self.env.lib.streams_layernorm(x, coef, self.weight, self.bias, self.eps, rows, out, delta=delta, update=update)
+        self.env.lib.streams_layernorm(x, coef, self.weight, self.bias, self.eps, rows, out, delta=delta, update=update, conv=conv)
         return out
 
 

@@ -1418,6 +1418,33 @@ def test_routers_of_many_rows_keep_a_product_of_their_own(lib, monkeypatch, expe
     assert torch.equal(part.forward(h), got)
 
 
+# ---------------------------------------------------------------------------- a norm with the convolution behind it
+@pytest.mark.parametrize("width", [4, 260, 2048, 4096])
+@pytest.mark.parametrize("taps,copies,update,biased,dtype", [(2, 1, False, True, torch.bfloat16), (3, 2, True, True, torch.float32),
+                                                             (4, 2, True, False, torch.bfloat16), (4, 3, True, True, torch.bfloat16), (4, 4, False, True, torch.bfloat16)])
+def test_a_norm_with_the_convolution_behind_it_gives_the_bits_of_two_launches(lib, width, taps, copies, update, biased, dtype):
+    gen = torch.Generator().manual_seed(width + taps)
+    n, r = 5, lambda *shape: torch.randn(*shape, generator=gen).to(DEV)
+    x, coef, weight, bias, w = r(copies, n, width), r(copies), r(width), r(width) if biased else None, r(width, taps)
+    todo = (r(copies, copies), r(copies), r(n, width), r(width)) if update else None
+    state, slots = r(7, taps - 1, width), torch.tensor([3, 0, 6, 1, 4], dtype=torch.int32, device=DEV)
+    ctx = SimpleNamespace(n_tokens=n, n_seqs=n, max_q_len=1, slots=slots, tok_pos=torch.zeros(n, dtype=torch.int32, device=DEV),
+                          tok_seq=torch.arange(n, dtype=torch.int32, device=DEV), cu_seqlens=torch.arange(n + 1, dtype=torch.int32, device=DEV))
+    assert lib.streams_conv_ok(width, taps) and not lib.streams_conv_ok(4100, taps) and not lib.streams_conv_ok(width, 5)
+    one, two = (tuple(t.clone() for t in (x, state)) for _ in range(2))
+    got, want, row = torch.empty(n, width, dtype=dtype, device=DEV), torch.empty(n, width, dtype=dtype, device=DEV), torch.empty(n, width, device=DEV)
+    lib.streams_layernorm(one[0], coef, weight, bias, 1e-5, None, got, update=todo, conv=(w, one[1], ctx))
+    lib.streams_layernorm(two[0], coef, weight, bias, 1e-5, None, row, update=todo)
+    lib.short_conv(row, 0, width, w, two[1], ctx, want, True, 0)
+    for a, b in ((got, want), (one[0], two[0]), (one[1], two[1])):
+        assert torch.equal(a, b)
+    odd = torch.empty(width * taps + 1, device=DEV)[1:].view(width, taps)      # weights at an odd address go in two launches
+    odd.copy_(w)
+    x2, s2 = x.clone(), state.clone()
+    lib.streams_layernorm(x2, coef, weight, bias, 1e-5, None, got, update=todo, conv=(odd, s2, ctx))
+    assert torch.equal(got, want) and torch.equal(s2, two[1])
+
+
 # ---------------------------------------------------------------------------- a shared expert in the chosen experts' launches
 @pytest.mark.parametrize("n", [1, 4, 16, 17])
 @pytest.mark.parametrize("hidden,ff,shared,along", [(128, 128, 128, True), (384, 256, 128, True), (2048, 1024, 1024, True), (1152, 640, 640, True),
