@@ -531,6 +531,11 @@ int rb_heads_linear_more(const void* x, int x_dtype, long long x_head_stride, co
                          long long y_head_stride, int n_tokens, int n_heads, int n, int k, const float* gate, long long gate_stride,
                          int rot, int x_rot_col, int y_rot_col, const float* cos, const float* sin, int style,
                          const int32_t* tok_pos, void* stream);
+// y[t, h, :n] = w[h]^T x[t, h, :k] for x [T, H, width] bfloat16, the result of single-token attention that lies in ws as n_splits > 1 splits
+// (rb_attention_decode_bf16_opts without an output leaves it so); sinks as there, w fragment-major bfloat16, y bfloat16, gate as above.
+int rb_heads_combined_ok(int n_tokens, int width, int n, int k);
+int rb_heads_combined(const float* ws, int n_splits, const float* sinks, int width, const void* w, void* y, long long y_head_stride, int n_tokens,
+                      int n_heads, int n, int k, const float* gate, long long gate_stride, void* stream);
 // rb_latent_norm_store into pages [n_pages, 1, 64, page_width] with, behind the latent, the `rot` numbers at rot_col of the
 // row rotated by the token's position (style 0: 2i with 2i + 1; 1: i with i + rot / 2) and zeros up to page_width.
 int rb_latent_norm_rope_store(const float* proj, long long stride, int q_rank, const float* q_gain, void* cq, int kv_col,

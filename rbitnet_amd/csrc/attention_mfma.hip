@@ -18,6 +18,7 @@
 #include <math.h>
 
 #include "api.h"
+#include "decode_combine.h"
 #include "tune.h"
 #include "mfma.h"
 
@@ -864,57 +865,15 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_mfma_kernel(
   }
 }
 
-// The splits of a (sequence, head) into one: a thread a number of the head, the splits' maxima and sums a lane each, so that all
-// of them are one trip to memory (a loop over the splits, once for the maximum and once for the sums, took 6.2 us for 8 splits
-// of 32 heads, 4.7 this way with 16 splits of 32 heads).
-// sum_only: the splits' outputs are added as they are (sigmoid weights), without maxima and denominators
+// The splits of a (sequence, head) into one: a thread a number of the head.  sum_only: sigmoid weights.
 template <int D>
 __global__ void attn_decode_combine_kernel(const float* __restrict__ ws, bf16_t* __restrict__ out, int n_splits,
                                            const float* __restrict__ sinks, int n_heads, int sum_only) {
-  constexpr int AHEAD = 8;
   __shared__ float2 factors[D / RB_WAVE][RB_WAVE];
   const size_t row = blockIdx.x;            // sequence * heads + head
-  const int d = threadIdx.x, lane = threadIdx.x & (RB_WAVE - 1);
-  const float* src = ws + row * n_splits * (D + 2);
-  float2* mine = factors[threadIdx.x / RB_WAVE];     // every wave keeps its own, so that none waits for another
-  float mx = -INFINITY;
-  if (!sum_only) {
-    for (int s = lane; s < n_splits; s += RB_WAVE) mx = fmaxf(mx, src[(size_t)s * (D + 2) + D]);
-    mx = wave_max(mx);
-  }
-  const float m_safe = (mx == -INFINITY) ? 0.f : mx;
-  float a = 0.f, l = 0.f;
-  for (int s0 = 0; s0 < n_splits; s0 += RB_WAVE) {
-    const int here = n_splits - s0 < RB_WAVE ? n_splits - s0 : RB_WAVE;
-    if (!sum_only && lane < here) {
-      const float* of = src + (size_t)(s0 + lane) * (D + 2);
-      mine[lane] = make_float2(exp2f(of[D] - m_safe), of[D + 1]);      // this wave's alone; a wave's LDS accesses complete in order
-    }
-    __builtin_amdgcn_wave_barrier();
-    for (int s1 = 0; s1 < here; s1 += AHEAD) {
-      float v[AHEAD];
-#pragma unroll
-      for (int u = 0; u < AHEAD; ++u) v[u] = src[(size_t)(s0 + (s1 + u < here ? s1 + u : s1)) * (D + 2) + d];
-#pragma unroll
-      for (int u = 0; u < AHEAD; ++u)
-        if (s1 + u < here) {                            // in the order of the splits
-          if (sum_only) {
-            a += v[u];
-          } else {
-            const float2 f = mine[s1 + u];
-            a = fmaf(v[u], f.x, a);
-            l = fmaf(f.y, f.x, l);
-          }
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-  if (sum_only) {
-    out[row * D + d] = f32_to_bf16(a);
-    return;
-  }
-  if (sinks) l += exp2f(fmaf(sinks[row % n_heads], LOG2E, -m_safe));          // the sink: in the denominator only
-  out[row * D + d] = f32_to_bf16(l > 0.f ? a / l : 0.f);
+  const int d = threadIdx.x;
+  out[row * D + d] = f32_to_bf16(combined_split<D>(ws + row * n_splits * (D + 2), n_splits, sinks ? sinks + row % n_heads : nullptr, sum_only != 0,
+                                                   factors[d / RB_WAVE], d & (RB_WAVE - 1), d));
 }
 
 struct DecodeArgs {
@@ -968,7 +927,7 @@ static int launch_decode_mfma_nw(const DecodeArgs& a, hipStream_t s) {
   kern<<<grid, 64 * NW, lds, s>>>(a.qkv, a.q, a.cos_t, a.sin_t, a.style, a.k, a.v, a.out, a.tok_pos, a.bt,
                                   a.bt_stride, a.n_heads, a.n_kv, a.sl2, a.window, a.n_splits, a.ws, a.qkv_terms,
                                   a.qkv_stride, a.sinks, a.keep_first, a.cap, a.cap_pre, a.kv_rep, a.chunk, a.sig_bias, by_length);
-  if (a.n_splits > 1) attn_decode_combine_kernel<D><<<a.n_seqs * a.n_heads, D, 0, s>>>(a.ws, a.out, a.n_splits, a.sinks, a.n_heads, a.sig_bias != nullptr);
+  if (a.n_splits > 1 && a.out) attn_decode_combine_kernel<D><<<a.n_seqs * a.n_heads, D, 0, s>>>(a.ws, a.out, a.n_splits, a.sinks, a.n_heads, a.sig_bias != nullptr);
   return 0;
 }
 
@@ -1017,6 +976,7 @@ static int dispatch_decode(DecodeArgs a, int head_dim, hipStream_t s, const char
   RB_REQUIRE(a.n_kv <= 65535 && a.n_seqs <= 65535, "%s: batch or head count too large", who);
   RB_REQUIRE(a.window >= 0, "%s: negative window", who);
   RB_REQUIRE(a.n_splits == 1 || a.ws != nullptr, "%s: splits need a workspace", who);
+  RB_REQUIRE(a.n_splits > 1 || a.out != nullptr, "%s: only splits can be left to their reader", who);
   const int group = a.n_heads / a.n_kv;
   RB_REQUIRE(group <= 16, "%s: %d query heads per kv head not supported (at most 16; use rb_attention_generic)", who,
              group);

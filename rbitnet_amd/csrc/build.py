@@ -33,7 +33,7 @@ ARCH = "gfx950"
 SOURCES = ["elementwise.hip", "gemm_generic.hip", "gemm_mfma.hip", "gemm_skinny.hip", "gemm_tiled.hip", "gemm_grouped.hip", "gemm_group.hip", "gemm_f32.hip",
            "attention_generic.hip", "attention_mfma.hip", "sampling.hip", "weights_init.hip", "probe.hip", "plan.hip", "streams.hip", "recurrent.hip", "recurrent_step.hip", "lightning.hip", "scan_chunks.hip",
            "latent.hip", "mixers.hip", "routed.hip", "talking.hip", "talking_mfma.hip"]
-HEADERS = ["api.h", "tune.h", "common.h", "mfma.h", "gemm_internal.h", "gemm_dma.h", "gemm_pingpong.h"]
+HEADERS = ["api.h", "tune.h", "common.h", "decode_combine.h", "mfma.h", "gemm_internal.h", "gemm_dma.h", "gemm_pingpong.h"]
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16", "-Wno-unused-result", "-Wno-unknown-warning-option"]
 

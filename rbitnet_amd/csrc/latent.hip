@@ -8,6 +8,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "decode_combine.h"
 #include "mfma.h"
 
 // proj [T, stride] float32 holds, per token, q_rank numbers at column 0 and kv_rank numbers at column kv_col.
@@ -382,6 +383,85 @@ extern "C" int rb_heads_linear_more(const void* x, int x_dtype, long long x_head
     case 2: launch_heads_linear<float, bf16_t, float>(x, w, y, n_tokens, n_heads, n, k, xs, ys, s, more); break;
     default: RB_REQUIRE(false, "rb_heads_linear: this combination of types is not built (x %d, w %d, y %d)", x_dtype, w_dtype, y_dtype);
   }
+  RB_LAUNCH_CHECK();
+  return 0;
+}
+
+// The product per head behind single-token attention whose splits are still to be put together (n_splits > 1; ws as rb_attention_decode_bf16_opts
+// leaves it without an output, sinks as there): the result of a (sequence, head) goes to LDS as the bfloat16 numbers that attention would
+// write, and through the head's matrix from there.  Bound by its trips to memory (maxima and sums, the splits, the weights beside them), as
+// either launch was that it stands for; a workgroup a head, a wave 16 outputs.  Attention and product, us in a graph
+// with the launch between them and without: 16 heads of 128 x 128, 1,500 keys in 16 splits, 1, 4 and 8 tokens 11.6 -> 9.8, 11.9 -> 10.2 and 12.2 ->
+// 10.9; 12 and 16 tokens, which are two rounds of the workgroup's waves, 12.6 -> 12.9 and 12.8 -> 14.0.  So at most 8, where a wave has one row.
+#define HC_THREADS 1024
+#define HC_TOKENS 8
+template <int D, int KS>
+__global__ __launch_bounds__(HC_THREADS) void heads_combined_kernel(const float* __restrict__ ws, int n_splits, const float* __restrict__ sinks,
+                                                                    const bf16_t* __restrict__ w, bf16_t* __restrict__ y, int n_tokens,
+                                                                    int n_heads, int n, size_t y_hs, const float* __restrict__ gate,
+                                                                    size_t gate_stride) {
+  constexpr int LD = D + 8;                                // rows of the operand on different banks
+  __shared__ __attribute__((aligned(16))) bf16_t xs[HC_TOKENS][LD];
+  __shared__ float2 factors[HC_THREADS / RB_WAVE][RB_WAVE];
+  const int h = blockIdx.x, lane = threadIdx.x & (RB_WAVE - 1), wave = threadIdx.x / RB_WAVE, r = lane & 15, kq = lane >> 4;
+  const int n_tiles = n / 16;
+  const bf16_t* wt = w + ((size_t)h * n_tiles + (wave < n_tiles ? wave : 0)) * (KS * 512) + 8 * lane;
+  Frag8 a[KS], b[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) a[ks].u = load16(wt + 512 * ks);
+  const int t = r < n_tokens ? r : n_tokens - 1;           // a token behind the last: the last one's numbers, never stored
+  const float g = gate ? 1.0f / (1.0f + expf(-gate[(size_t)t * gate_stride + h])) : 1.0f;
+  __builtin_amdgcn_sched_barrier(0);
+  const int d = threadIdx.x % D;
+  for (int row = threadIdx.x / D; row < n_tokens; row += HC_THREADS / D)
+    xs[row][d] = f32_to_bf16(combined_split<D>(ws + ((size_t)row * n_heads + h) * n_splits * (D + 2), n_splits, sinks ? sinks + h : nullptr, false,
+                                               factors[wave], lane, d));
+  __syncthreads();
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) b[ks].u = *reinterpret_cast<const uint4*>(&xs[t][32 * ks + 8 * kq]);
+  bf16_t* yr = y + ((size_t)t * n_heads + h) * y_hs + 4 * kq;
+  for (int tile = wave; tile < n_tiles; tile += HC_THREADS / RB_WAVE) {
+    if (tile != wave) {
+      wt += (size_t)(HC_THREADS / RB_WAVE) * (KS * 512);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) a[ks].u = load16(wt + 512 * ks);
+    }
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) acc = mfma16(a[ks], b[ks], acc);
+    acc *= g;
+    if (r < n_tokens) *reinterpret_cast<uint2*>(yr + 16 * tile) = make_uint2(pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]));
+  }
+}
+
+// Whether the kernel takes these sizes: latents of 64 or 128 numbers, of which the first k are read, and few tokens.
+extern "C" int rb_heads_combined_ok(int n_tokens, int width, int n, int k) {
+  return n_tokens >= 1 && n_tokens <= HC_TOKENS && (width == 64 || width == 128) && k > 0 && k % 32 == 0 && k <= width && n > 0 && n % 16 == 0;
+}
+
+// y[t, h, :n] = w[h]^T x[t, h, :k], x [T, H, width] the bfloat16 result of attention that lies as splits in ws; w fragment-major, y bfloat16, gate as in
+// rb_heads_linear_more.
+extern "C" int rb_heads_combined(const float* ws, int n_splits, const float* sinks, int width, const void* w, void* y, long long y_head_stride,
+                                 int n_tokens, int n_heads, int n, int k, const float* gate, long long gate_stride, void* stream) {
+  RB_RECORDED(rb_heads_combined(ws, n_splits, sinks, width, w, y, y_head_stride, n_tokens, n_heads, n, k, gate, gate_stride, stream));
+  RB_REQUIRE(n_tokens == 0 || rb_heads_combined_ok(n_tokens, width, n, k), "rb_heads_combined: %d tokens, %d of %d numbers to %d are not for it",
+             n_tokens, k, width, n);
+  RB_REQUIRE(ws && w && y && n_splits > 1 && n_heads > 0 && n_heads <= 65535 && y_head_stride >= n && y_head_stride % 8 == 0,
+             "rb_heads_combined: bad sizes");
+  RB_REQUIRE(gate == nullptr || gate_stride >= n_heads, "rb_heads_combined: the gate's rows are shorter than the heads");
+  RB_REQUIRE(((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y)) & 15) == 0, "rb_heads_combined: operands must be 16-byte aligned");
+  if (n_tokens == 0) return 0;
+#define HC_GO(D, KS)                                                                                                                           heads_combined_kernel<D, KS><<<n_heads, HC_THREADS, 0, (hipStream_t)stream>>>(ws, n_splits, sinks, (const bf16_t*)w, (bf16_t*)y, n_tokens,                                                                                 n_heads, n, (size_t)y_head_stride, gate, (size_t)gate_stride)
+  if (width == 64) {
+    if (k == 32) HC_GO(64, 1);
+    else HC_GO(64, 2);
+  } else {
+    if (k == 32) HC_GO(128, 1);
+    else if (k == 64) HC_GO(128, 2);
+    else if (k == 96) HC_GO(128, 3);
+    else HC_GO(128, 4);
+  }
+#undef HC_GO
   RB_LAUNCH_CHECK();
   return 0;
 }

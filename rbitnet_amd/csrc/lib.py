@@ -235,6 +235,8 @@ class Kernels:
             "rb_short_conv_bias": [_P, _L, _P, _P, _I, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
             "rb_linear_recurrence_bonus": [_P, _P, _L, _P, _L, _P, _L, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
             "rb_gated_rmsnorm_heads": [_P, _P, _L, _P, _L, _I, _F, _P, _I, _I, _I, _I, _P],
+            "rb_heads_combined_ok": [_I, _I, _I, _I],
+            "rb_heads_combined": [_P, _I, _P, _I, _P, _P, _L, _I, _I, _I, _I, _P, _L, _P],
             "rb_heads_linear_more": [_P, _I, _L, _P, _I, _I, _P, _I, _L, _I, _I, _I, _I, _P, _L, _I, _I, _I, _P, _P, _I, _P, _P],
             "rb_latent_norm_rope_store": [_P, _L, _I, _P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _P, _I, _I, _P, _P, _P, _I, _F, _I, _P],
             "rb_attention_generic_chunked": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _F, _P, _I, _P, _P],
@@ -507,14 +509,16 @@ class Kernels:
     def attention_decode_bf16(self, q, k_pages, v_pages, out, tok_pos, block_table, n_heads, n_kv, head_dim,
                               scale, window, n_splits, workspace, sinks=None, keep_first: int = 0, softcap: float = 0.0,
                               chunk: int = 0, sig_bias=None) -> None:
-        """chunk > 0: a query sees the keys of its own chunk of positions only; sig_bias float32 [Hq]: sigmoid weights."""
+        """chunk > 0: a query sees the keys of its own chunk of positions only; sig_bias float32 [Hq]: sigmoid weights.  out None (n_splits >
+        1): the splits stay in the workspace, for `heads_combined`."""
         n = q.shape[0]
         _check(q, "q", torch.bfloat16, (n, n_heads, head_dim))
         _check(k_pages, "k_pages", torch.bfloat16)
         _check(v_pages, "v_pages", torch.bfloat16, k_pages.shape)
         if tuple(k_pages.shape[1:]) != (n_kv, self.page_size, head_dim):
             raise KernelError("cache pages do not match the head counts")
-        _check(out, "out", torch.bfloat16, (n, n_heads * head_dim))
+        if out is not None or n_splits < 2:
+            _check(out, "out", torch.bfloat16, (n, n_heads * head_dim))
         _check(tok_pos, "tok_pos", torch.int32, (n,))
         _check(block_table, "block_table", torch.int32)
         _check(workspace, "workspace", torch.float32)
@@ -1642,6 +1646,34 @@ class Kernels:
                                                 dtype_code(y.dtype), y_head, n, h, n_out, k, g_ptr, g_stride, int(rot), int(x_col),
                                                 int(y_col), _ptr(cos) if rot > 0 else None, _ptr(sin) if rot > 0 else None, int(style),
                                                 _ptr(tok_pos), self._stream()))
+
+    def heads_combined_ok(self, n_tokens: int, n_splits: int, width: int, n_out: int, k: int, w_frag: bool) -> bool:
+        """Whether `heads_combined` takes the splits of single-token attention through a product per head."""
+        return w_frag and n_splits > 1 and bool(self._lib.rb_heads_combined_ok(n_tokens, width, n_out, k))
+
+    def heads_combined(self, workspace: torch.Tensor, n_splits: int, sinks, width: int, w: torch.Tensor, y: torch.Tensor, y_head: int,
+                       gate: Optional[torch.Tensor] = None, gate_col: int = 0) -> None:
+        """`heads_linear_part` of the result that `attention_decode_bf16` with out None left as splits: w [H, N, K] fragment-major, y
+        [T, H y_head] bfloat16, gate as there."""
+        h, n_out, k = w.shape
+        n = y.shape[0]
+        _check(workspace, "workspace", torch.float32)
+        if workspace.numel() < n * h * n_splits * (width + 2):
+            raise KernelError("heads_combined: workspace too small")
+        _check(w, "w", torch.bfloat16)
+        _check(y, "y", torch.bfloat16, (n, h * y_head))
+        if y_head < n_out:
+            raise KernelError("heads_combined: a head is shorter than the product's outputs")
+        if sinks is not None:
+            _check(sinks, "sinks", torch.float32, (h,))
+        g_ptr, g_stride = None, 0
+        if gate is not None:
+            _check(gate, "gate", torch.float32)
+            if gate.shape[0] != n or gate_col < 0 or gate_col + h > gate.shape[1]:
+                raise KernelError("heads_combined: the gate's columns lie outside the rows")
+            g_ptr, g_stride = gate.data_ptr() + 4 * gate_col, gate.shape[1]
+        self._ok(self._lib.rb_heads_combined(_ptr(workspace), int(n_splits), _ptr(sinks), width, _ptr(w), _ptr(y), y_head, n, h, n_out, k, g_ptr,
+                                             g_stride, self._stream()))
 
     def latent_norm_rope_store(self, proj: torch.Tensor, q_rank: int, q_gain, cq, kv_rank: int, kv_gain, pages, rot: int, cos, sin,
                                style: int, ctx, block_table, eps: float, dtype: torch.dtype) -> None:

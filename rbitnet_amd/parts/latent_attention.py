@@ -168,11 +168,19 @@ class LatentAttention(Part):
                                   rope=(self.dim, self.rot, cos, sin, style, self.kv_rank, ctx.tok_pos), w_frag=self.uk_frag)
         else:
             lib.heads_linear_part(q, self.dim, self.w_uk, ql, r, w_frag=self.uk_frag)      # the queries in the latent's space
-        ol = torch.empty((t, self.heads * r), dtype=dt, device=h.device)
+        o = torch.empty((t, self.heads * self.vdim), dtype=dt, device=h.device)
         q3, pages = ql.view(t, self.heads, r), view.k_pages
         fast = dt == torch.bfloat16 and r in _MATRIX_CORE_RANKS and not getattr(self.env, "generic_only", False)
         if fast and ctx.max_q_len == 1:      # more than 16 heads on the latent run as several groups of at most 16
             n_splits, workspace = ctx.decode_workspace(self.heads, r, 1, spread=True)
+            if lib.heads_combined_ok(t, n_splits, r, self.vdim, self.kv_rank, self.uv_frag):      # the product that reads the splits puts them together
+                lib.attention_decode_bf16(q3, pages, pages, None, ctx.tok_pos, view.block_table, self.heads, 1, r, self.scale, None,
+                                          n_splits, workspace, sinks=self.sink)
+                lib.heads_combined(workspace, n_splits, self.sink, r, self.w_uv, o, self.vdim, gate=down if self.has_gate else None,
+                                   gate_col=self.gate_col)
+                return linear_to_stream(lib, o, self.w_o, None, next_norm)
+        ol = torch.empty((t, self.heads * r), dtype=dt, device=h.device)
+        if fast and ctx.max_q_len == 1:
             lib.attention_decode_bf16(q3, pages, pages, ol, ctx.tok_pos, view.block_table, self.heads, 1, r, self.scale, None,
                                       n_splits, workspace, sinks=self.sink)
         elif fast:
@@ -181,7 +189,6 @@ class LatentAttention(Part):
         else:
             lib.attention_sinks(q3, pages, pages, ol, ctx.tok_pos, ctx.tok_seq, view.block_table, self.heads, 1, r,
                                 self.scale, None, self.sink, n_seqs=ctx.n_seqs)
-        o = torch.empty((t, self.heads * self.vdim), dtype=dt, device=h.device)
         # the latent's part of every head's sum through the head's value matrix, the head's gate on the way out
         lib.heads_linear_part(ol, r, self.w_uv, o, self.vdim, gate=down if self.has_gate else None, gate_col=self.gate_col,
                               w_frag=self.uv_frag)

@@ -1418,6 +1418,34 @@ def test_routers_of_many_rows_keep_a_product_of_their_own(lib, monkeypatch, expe
     assert torch.equal(part.forward(h), got)
 
 
+# ---------------------------------------------------------------------------- splits of attention put together by the product that reads them
+@pytest.mark.parametrize("n", [1, 4, 7, 8])
+@pytest.mark.parametrize("heads,width,k,n_out,splits,sink,gated", [(16, 128, 128, 128, 2, True, False), (32, 128, 96, 64, 16, False, True),
+                                                                   (3, 64, 64, 16, 5, False, False), (2, 128, 32, 272, 70, True, True), (1, 64, 32, 64, 9, False, True)])
+def test_splits_put_together_by_the_product_per_head_give_the_bits_of_two_launches(lib, n, heads, width, k, n_out, splits, sink, gated):
+    gen = torch.Generator().manual_seed(heads + n)
+    lengths = [(97 * i) % 400 + 1 for i in range(n)]         # fewer pages than splits: some are empty
+    pages, table, _ = _paged(lengths, 1, width, gen)
+    pos = torch.tensor([m - 1 for m in lengths], dtype=torch.int32, device=DEV)
+    q = torch.randn(n, heads, width, generator=gen).bfloat16().to(DEV)
+    rows = (torch.randn(heads * n_out, k, generator=gen) * k ** -0.5).bfloat16().to(DEV)
+    w = torch.empty(heads, n_out, k, dtype=torch.bfloat16, device=DEV)
+    lib.place_rows(rows, w.view(-1, k), frag=True)
+    sinks = torch.randn(heads, generator=gen).to(DEV) if sink else None
+    gate = torch.randn(n, heads + 3, generator=gen).to(DEV) if gated else None
+    assert lib.heads_combined_ok(n, splits, width, n_out, k, True)
+    assert not lib.heads_combined_ok(9, splits, width, n_out, k, True) and not lib.heads_combined_ok(n, 1, width, n_out, k, True)
+    ws = [torch.full((n * heads * splits * (width + 2),), float("nan"), device=DEV) for _ in range(2)]
+    attend = lambda out, scratch: lib.attention_decode_bf16(q, pages.bfloat16().to(DEV), pages.bfloat16().to(DEV), out, pos, table.to(DEV), heads, 1, width, 0.1,
+                                                            None, splits, scratch, sinks=sinks)
+    x, want, got = torch.empty(n, heads * width, dtype=torch.bfloat16, device=DEV), *(torch.empty(n, heads * n_out, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    attend(x, ws[0])
+    lib.heads_linear_part(x, width, w, want, n_out, gate=gate, gate_col=2, w_frag=True)
+    attend(None, ws[1])
+    lib.heads_combined(ws[1], splits, sinks, width, w, got, n_out, gate=gate, gate_col=2)
+    assert torch.isfinite(want.float()).all() and torch.equal(got, want)
+
+
 # ---------------------------------------------------------------------------- a norm with the convolution behind it
 @pytest.mark.parametrize("width", [4, 260, 2048, 4096])
 @pytest.mark.parametrize("taps,copies,update,biased,dtype", [(2, 1, False, True, torch.bfloat16), (3, 2, True, True, torch.float32),
