@@ -20,7 +20,7 @@ struct Group {
   int count;
 };
 
-template <bool WF>
+template <bool WF, int XP>                                 // XP: see RowPack
 __global__ __launch_bounds__(512) void gemm_group_kernel(const Group g, int m, int k) {
   extern __shared__ __attribute__((aligned(16))) float red[];      // [waves - 1][64] pieces of four sums
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, kq = lane >> 4;
@@ -31,21 +31,22 @@ __global__ __launch_bounds__(512) void gemm_group_kernel(const Group g, int m, i
   const int n0 = 16 * ((int)blockIdx.x - (i > 0 ? g.end[i - 1] : 0));
   const bf16_t* w = (const bf16_t*)p.w;
   const bf16_t* wrow = WF ? w + (size_t)n0 * k + 8 * lane : w + (size_t)(n0 + r < p.n ? n0 + r : 0) * k + 8 * kq;
-  const bf16_t* xrow = (const bf16_t*)p.x + (size_t)(r < m ? r : 0) * k + 8 * kq;
+  const int row = RowPack<XP>::row(r);
+  const bf16_t* xrow = (const bf16_t*)p.x + (size_t)(row < m ? row : 0) * k + RowPack<XP>::depth(r) + 8 * kq;
   const int total = k / 128, base = total / n_waves, extra = total % n_waves;
   const int stages = base + (wave < extra ? 1 : 0), begin = 128 * (wave * base + (wave < extra ? wave : extra));
   f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  Frag8 a[4], b[4];
+  Frag8 a[4], b[4 / XP];
   auto load_stage = [&](int st) {
     const int ks = begin + 128 * st;
 #pragma unroll
     for (int j = 0; j < 4; ++j) a[j].u = WF ? load16_stream(wrow + (size_t)(ks + 32 * j) * 16) : load16(wrow + ks + 32 * j);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) b[j].u = load16(xrow + ks + 32 * j);
+    for (int j = 0; j < 4 / XP; ++j) b[j].u = load16(xrow + ks + 32 * XP * j);
   };
   auto multiply_stage = [&]() {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc = mfma16(a[j], b[j], acc);
+    for (int j = 0; j < 4; ++j) acc = mfma16(a[j], RowPack<XP>::block(b, j), acc);
   };
   if (wave < n_waves) {                                     // (the host gives a product no more waves than stages)
     load_stage(0);
@@ -127,8 +128,9 @@ extern "C" int rb_gemm_bf16_group(const RbGroupProduct* products, int count, int
     if (g.waves[i] > waves) waves = g.waves[i];
   }
   const size_t lds = (size_t)(waves - 1) * 256 * sizeof(float);
-  if (w_layout) gemm_group_kernel<true><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
-  else gemm_group_kernel<false><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
+  if (w_layout)
+    (m <= 4 ? gemm_group_kernel<true, 4> : m <= 8 ? gemm_group_kernel<true, 2> : gemm_group_kernel<true, 1>)<<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
+  else gemm_group_kernel<false, 1><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
   RB_LAUNCH_CHECK();
   return 0;
 }

@@ -128,7 +128,10 @@ __device__ __forceinline__ float squares_sum(const SquaresShare& s) {
 // before is multiplied; else any K % 8 == 0, with bounds checks.  WF (up to 16 tokens): W is stored fragment-major.
 // (All of a wave's stages asked for at once instead, W's first, for up to four stages a wave: no faster at K = 128 to 4096 with any
 // number of waves, 2,048 rows at K = 2048 4.5 us either way, 8,192 rows 7.6 -> 8.3.)
-template <int MB, int R, bool FAST, bool WF, int EPI, typename TO, bool SCALED>
+//
+// XP: blocks of 32 depth values that a load of the tokens brings (see RowPack in gemm_internal.h).
+// WP: blocks of depth that a load of W brings (one row tile a wave, W fragment-major): a workgroup then has 16 / WP of the tile's rows.
+template <int MB, int R, bool FAST, bool WF, int EPI, typename TO, bool SCALED, int XP, int WP = 1>
 __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restrict__ x,
                                                           const bf16_t* __restrict__ w, TO* __restrict__ c,
                                                           int m, int n, int k, int k_per_wave, FoldArgs fa) {
@@ -140,7 +143,9 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
   const int n_waves = blockDim.x >> 6;
   const int r = lane & 15;
   const int kq = lane >> 4;
-  const int n0 = blockIdx.x * (16 * R);
+  static_assert(WP == 1 || (R == 1 && MB == 1 && FAST && WF && EPI != 1 && EPI != 3), "parts of a tile: one row tile a wave, ends that know no tile");
+  const int n0 = WP > 1 ? blockIdx.x / WP * 16 : blockIdx.x * (16 * R);
+  const int part0 = WP > 1 ? blockIdx.x % WP * (16 / WP) : 0;      // this workgroup's rows of the tile
 
   f32x4_t acc[R][MB];
 #pragma unroll
@@ -159,16 +164,18 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
   for (int rt = 0; rt < R; ++rt) {
     const int row = n0 + 16 * rt + r;
     wok[rt] = row < n;
-    if (frag) wrow[rt] = w + (size_t)(n0 + 16 * rt < n ? n0 + 16 * rt : 0) * k + 8 * lane;
+    if (WP > 1) wrow[rt] = w + (size_t)n0 * k + 16 * RowPack<WP>::depth(r) + 8 * (16 * kq + part0 + RowPack<WP>::row(r));
+    else if (frag) wrow[rt] = w + (size_t)(n0 + 16 * rt < n ? n0 + 16 * rt : 0) * k + 8 * lane;
     else wrow[rt] = w + (size_t)(wok[rt] ? row : 0) * k + 8 * kq;
   }
-  Frag8 a[R][4], b[MB][4];
+  static_assert(XP == 1 || (MB == 1 && FAST), "packed tokens: at most 8, whole stages");
+  Frag8 a[R][4 / WP], b[MB][4 / XP];
   auto load_w = [&](int ks) {                         // depth values ks..ks + 127 of the wave's rows
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4 / WP; ++j)
 #pragma unroll
       for (int rt = 0; rt < R; ++rt) {
-        const bf16_t* src = wrow[rt] + (size_t)(ks + 32 * j) * wk;
+        const bf16_t* src = wrow[rt] + (size_t)(ks + 32 * WP * j) * wk;
         if (frag) a[rt][j].u = load16_stream(src);      // read once, whole lines at a time: past the caches
         else a[rt][j].u = load16(src);
       }
@@ -184,6 +191,10 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
     size_t src = xok[cb] ? row : 0;
     if (fa.rows) src = (size_t)fa.rows[src];
     xrow[cb] = x + src * k;
+    if (XP > 1) {
+      const int packed = RowPack<XP>::row(r) < m ? RowPack<XP>::row(r) : 0;
+      xrow[cb] = x + (size_t)(fa.rows ? fa.rows[packed] : packed) * k + RowPack<XP>::depth(r);
+    }
     ss[cb] = 0.f;
     if (SCALED) {
       const int n_sq = (k + 15) / 16;
@@ -196,7 +207,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
   f32x4_t before[R][MB], gain[R];
 #pragma unroll
   for (int rt = 0; rt < R; ++rt) {
-    const int nn = n0 + 16 * rt + 4 * kq;
+    const int nn = n0 + part0 + 16 * rt + 4 * kq;
     gain[rt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     if (EPI == 3 && wave == 0) {
       if (fa.wide) {
@@ -229,7 +240,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
 #pragma unroll
       for (int rt = 0; rt < R; ++rt)
 #pragma unroll
-        for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = mfma16(a[rt][j], b[cb][j], acc[rt][cb]);
+        for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = mfma16(RowPack<WP>::block(a[rt], j), RowPack<XP>::block(b[cb], j), acc[rt][cb]);
   };
   if constexpr (FAST) {
     // K and every wave's range are multiples of 128: no bounds checks.  Rows beyond N or M
@@ -244,9 +255,9 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
       const int ks = k_begin + 128 * st;
       load_w(ks);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 4 / XP; ++j)
 #pragma unroll
-        for (int cb = 0; cb < MB; ++cb) b[cb][j].u = load16(xrow[cb] + ks + 8 * kq + 32 * j);
+        for (int cb = 0; cb < MB; ++cb) b[cb][j].u = load16(xrow[cb] + ks + 8 * kq + 32 * XP * j);
     };
     load_stage(0);
     // the sums of squares were asked for before the first stage and arrive before it: added up
@@ -273,9 +284,9 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
         const bool in = kk < k_end;
 #pragma unroll
         for (int rt = 0; rt < R; ++rt)
-          a[rt][j].u = (in && wok[rt]) ? load16(wrow[rt] + (size_t)(k0 + 32 * j) * wk) : zero16();
+          a[rt][j / WP].u = (in && wok[rt]) ? load16(wrow[rt] + (size_t)(k0 + 32 * j) * wk) : zero16();
 #pragma unroll
-        for (int cb = 0; cb < MB; ++cb) b[cb][j].u = (in && xok[cb]) ? load16(xrow[cb] + kk) : zero16();
+        for (int cb = 0; cb < MB; ++cb) b[cb][j / XP].u = (in && xok[cb]) ? load16(xrow[cb] + kk) : zero16();
       }
       multiply_stage();
     }
@@ -333,12 +344,13 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
   }
 
   // ---- lane holds, per (rt, cb): token 16*cb + r, W rows n0 + 16*rt + 4*kq + 0..3
+  if (WP > 1 && kq >= 4 / WP) return;
   if (EPI != 1) {
 #pragma unroll
     for (int rt = 0; rt < R; ++rt)
 #pragma unroll
       for (int cb = 0; cb < MB; ++cb)
-        store_sums<EPI, true, TO>(c, acc[rt][cb], before[rt][cb], gain[rt], 16 * cb + r, n0 + 16 * rt + 4 * kq, m, n,
+        store_sums<EPI, true, TO>(c, acc[rt][cb], before[rt][cb], gain[rt], 16 * cb + r, n0 + part0 + 16 * rt + 4 * kq, m, n,
                             n0 / 16 + rt, kq, fa);
   } else {
     const int half_n = n / 2;
@@ -365,6 +377,8 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
   }
 }
 
+static int g_tune_parts = 0;
+extern "C" void rb_tune_parts(int parts) { g_tune_parts = parts; }      // experiments and tests only: 1 or 2 workgroups for a tile of 16 rows; 0 = the built-in choice
 static int g_tune_r = 0, g_tune_waves = 0;
 extern "C" void rb_tune(int r, int waves) {       // experiments only; 0 = the built-in choice
   g_tune_r = r;
@@ -377,17 +391,40 @@ static FoldArgs fold_args(const GemmTokens& x, const GemmAfter& after, const voi
                   after.epilogue <= 1 ? after.act : nullptr};
 }
 
+// Two workgroups for a tile of 16 rows where that still is at most one a compute unit.  A compute unit has so many requests under way and no more, so a
+// product of few rows takes as long as the units that have any of them need for their share, whatever is asked for ahead (two or four stages in
+// flight a wave: no change at any of 12 sizes); the two halves of a 1 KB block, loaded with the lanes of the other half for the next
+// block of depth, halve that share.  us with whole tiles and with halves, 4 tokens: 2,048 rows at K = 2048 4.17 and 3.89, 4096 5.75 and 5.42, 8192 10.2 and 8.8,
+// 11008 14.0 and 11.8; 896 rows at 2048 3.87 and 3.61; 16 tokens, 2,048 at 8192 12.6 and 11.4.  More than one a unit lose (2,304 rows at 2048 4.28 and
+// 4.57), and so do quarters, whose 64 bytes are half a line (2,048 rows at 2048 5.25, 896 4.01).
+static int skinny_parts(int n) {
+  if (g_tune_parts) return g_tune_parts;
+  return 2 * ((n + 15) / 16) <= rb_compute_units() ? 2 : 1;
+}
+
 template <int MB, int R, bool FAST, int EPI, typename TO, bool SCALED>
 static int launch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
                          int n_waves, int k_per_wave, hipStream_t s) {
   const size_t lds = (size_t)(n_waves - 1) * (R * MB * 4 + (SCALED ? MB : 0)) * 64 * sizeof(float);
   RB_REQUIRE(lds <= 64 * 1024, "rb_gemm_bf16: internal: reduction buffer of %zu bytes", lds);
   const int grid = (n + 16 * R - 1) / (16 * R);
-  if (MB == 1 && after.w_frag)
-    gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED>
+  if constexpr (MB == 1 && R == 1 && FAST && !SCALED && (EPI == 0 || EPI == 2 || EPI == EPI_ACT)) {
+    if (after.w_frag && skinny_parts(n) == 2) {
+      (m <= 4   ? gemm_skinny_kernel<1, 1, true, true, EPI, TO, false, 4, 2>
+       : m <= 8 ? gemm_skinny_kernel<1, 1, true, true, EPI, TO, false, 2, 2>
+                : gemm_skinny_kernel<1, 1, true, true, EPI, TO, false, 1, 2>)<<<2 * grid, n_waves * 64, lds, s>>>(
+          x.x, w, (TO*)c, m, n, k, k_per_wave, fold_args(x, after, c, n));
+      return 0;
+    }
+  }
+  if (MB == 1 && after.w_frag) {
+    constexpr bool MAY = MB == 1 && FAST;
+    (MAY && m <= 4   ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 4 : 1>
+     : MAY && m <= 8 ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 2 : 1>
+                     : gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, 1>)
         <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, k_per_wave, fold_args(x, after, c, n));
-  else
-    gemm_skinny_kernel<MB, R, FAST, false, EPI, TO, SCALED>
+  } else
+    gemm_skinny_kernel<MB, R, FAST, false, EPI, TO, SCALED, 1>
         <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, k_per_wave, fold_args(x, after, c, n));
   return 0;
 }

@@ -1418,6 +1418,51 @@ def test_routers_of_many_rows_keep_a_product_of_their_own(lib, monkeypatch, expe
     assert torch.equal(part.forward(h), got)
 
 
+# ---------------------------------------------------------------------------- products of few tokens: packed loads, halves of tiles
+@pytest.mark.parametrize("n,k", [(16, 128), (48, 384), (2048, 1024), (2064, 256), (1040, 2048), (96, 8192), (544, 5120), (4112, 128)])
+def test_a_row_of_a_product_has_the_same_bits_however_its_operands_are_loaded(lib, n, k):
+    """4, 2 or 1 blocks of the tokens a load by how many tokens there are, whole tiles of W and halves: 16 tokens with whole tiles, a block a load, and
+    the same rows among fewer, for every end.  (That those are right: the tests against float64 above and in test_kernels_gpu.py.)"""
+    gen = torch.Generator().manual_seed(n + k)
+    x = torch.randn(16, k, generator=gen).bfloat16().to(DEV)
+    rows = (torch.randn(n, k, generator=gen) * k ** -0.5).bfloat16().to(DEV)
+    w = torch.empty_like(rows)
+    lib.place_rows(rows, w, frag=True)
+    act, gain = torch.tensor([0.3, -0.2], device=DEV), torch.randn(n, generator=gen).to(DEV)
+    before, squares = torch.randn(16, n, generator=gen).to(DEV), torch.rand(16, (k + 15) // 16, generator=gen).to(DEV) * 16
+
+    def all_ends(m, pick=None):
+        at = slice(0, m) if pick is None else pick
+        outs = []
+        for dtype, epilogue, a in ((torch.float32, 0, None), (torch.bfloat16, 0, act), (torch.bfloat16, 1, None)):
+            if epilogue == 1 and n % 32:
+                continue
+            out = torch.empty(m, n // 2 if epilogue == 1 else n, dtype=dtype, device=DEV)
+            lib.gemm_bf16(x[at].contiguous(), w, out, epilogue, w_frag=True, act=a)
+            outs.append(out)
+        if lib.gemm_bf16_few_ok(m, n, k):
+            for epilogue in (2, 3):
+                out, g, s = before[at].clone(), torch.zeros(m, n, dtype=torch.bfloat16, device=DEV), torch.zeros(m, (n + 15) // 16, device=DEV)
+                lib.gemm_bf16_few(x[at].contiguous(), w, out, epilogue, w_frag=True, **(dict(gain=gain, gained=g, squares_out=s) if epilogue == 3 else {}))
+                outs += [out, g, s]
+            out = torch.empty(m, n, device=DEV)
+            chosen = None if pick is None else torch.tensor(pick, dtype=torch.int32, device=DEV)
+            lib.gemm_bf16_few(x if pick is not None else x[at].contiguous(), w, out, 0, squares=squares if pick is not None else squares[at].contiguous(), eps=1e-5,
+                              rows=chosen, w_frag=True)
+            outs.append(out)
+        return outs
+    try:
+        lib._lib.rb_tune_parts(1)
+        whole = all_ends(16)
+        for parts in (0, 1, 2):
+            lib._lib.rb_tune_parts(parts)
+            for m, pick in ((16, None), (9, None), (8, None), (5, None), (4, None), (3, None), (1, None), (3, [7, 2, 11]), (6, [15, 0, 3, 3, 9, 1])):
+                for got, want in zip(all_ends(m, pick), whole):
+                    assert torch.equal(got, want[:m] if pick is None else want[pick]), (parts, m, pick)
+    finally:
+        lib._lib.rb_tune_parts(0)
+
+
 # ---------------------------------------------------------------------------- splits of attention put together by the product that reads them
 @pytest.mark.parametrize("n", [1, 4, 7, 8])
 @pytest.mark.parametrize("heads,width,k,n_out,splits,sink,gated", [(16, 128, 128, 128, 2, True, False), (32, 128, 96, 64, 16, False, True),
