@@ -46,10 +46,9 @@ struct RowPack {
   static_assert(XP == 1 || XP == 2 || XP == 4, "a stage is four blocks");
   static __device__ __forceinline__ int row(int r) { return r % (16 / XP); }
   static __device__ __forceinline__ int depth(int r) { return 32 * (r / (16 / XP)); }
-  // block j of a stage from what its 4 / XP loads brought
-  template <typename F, int N>
-  static __device__ __forceinline__ Frag8 block(const F (&b)[N], int j) {
-    static_assert(N * XP == 4, "the loads of a stage");
+  // block j of those that these loads brought
+  template <int N>
+  static __device__ __forceinline__ Frag8 block(const Frag8 (&b)[N], int j) {
     Frag8 f = b[j / XP];
     const int turn = j % XP;
     if (XP == 1 || turn == 0) return f;

@@ -587,22 +587,24 @@ __device__ __forceinline__ void walk_ahead(int n_steps, const Load& load, const 
 // W by one wave, which takes the shares of depth of the `waves` that the product alone has one after another and adds up their sums in the
 // same order: the same bits.  Bound by the chosen experts' matrices, which take longer than this wave's walk.  (A captured step of 4 tokens through 15
 // layers of 16 experts of 2,048 and a shared one of 1,024 at width 2,048 took 120 us longer with four launches a layer than with two: 4 us a launch.)
+// XP: blocks of depth that a load of the tokens brings (see RowPack), here and below: an expert's run has no more rows than the step has tokens.
 struct SharedProduct {
   const bf16_t *x, *w;
   void* c;                   // bfloat16 with act, else float32
   const float* act;          // xIELU's two numbers (see xielu_pair); null: the sums as they are
   int n, k, m, waves;
 };
+template <int XP>
 __device__ __forceinline__ void shared_product(const SharedProduct& p, int tile) {
   const int lane = threadIdx.x, r = lane & 15, kq = lane >> 4, n0 = 16 * tile;
   if (n0 >= p.n) return;
   const bf16_t* wr = p.w + (size_t)n0 * p.k + 8 * lane;
-  const bf16_t* xr = p.x + (size_t)(r < p.m ? r : 0) * p.k + 8 * kq;
+  const bf16_t* xr = p.x + (size_t)(RowPack<XP>::row(r) < p.m ? RowPack<XP>::row(r) : 0) * p.k + RowPack<XP>::depth(r) + 8 * kq;
   const int total = p.k / 128, base = total / p.waves, extra = total % p.waves;
   int wave = 0, left = base + (extra > 0 ? 1 : 0);         // stages of 128 that this share still has
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, sum = acc;
   struct Ahead {
-    Frag8 w[RT_AHEAD], x[RT_AHEAD];
+    Frag8 w[RT_AHEAD], x[RT_AHEAD / XP];
   };
   static_assert(RT_AHEAD % 4 == 0, "a trip is whole stages");
   auto load = [&](Ahead& f, int s0, int cnt) __attribute__((always_inline)) {
@@ -610,7 +612,7 @@ __device__ __forceinline__ void shared_product(const SharedProduct& p, int tile)
     for (int u = 0; u < RT_AHEAD; ++u) {
       const size_t s = (size_t)(s0 + (u < cnt ? u : 0));
       f.w[u].u = load16_stream(wr + 512 * s);
-      f.x[u].u = load16(xr + 32 * s);
+      if (u % XP == 0) f.x[u / XP].u = load16(xr + 32 * s);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -618,7 +620,7 @@ __device__ __forceinline__ void shared_product(const SharedProduct& p, int tile)
 #pragma unroll
     for (int u = 0; u < RT_AHEAD; ++u) {
       if (u >= cnt) break;
-      acc = mfma16(f.w[u], f.x[u], acc);
+      acc = mfma16(f.w[u], RowPack<XP>::block(f.x, u), acc);
       if (u % 4 == 3 && --left == 0) {
         sum = wave == 0 ? acc : sum + acc;
         acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -642,7 +644,7 @@ __device__ __forceinline__ void shared_product(const SharedProduct& p, int tile)
 }
 
 // SHARED: the first shared_y rows of the grid are a shared expert's product
-template <int NT, bool WEIGHTED, bool GATED, bool SHARED>
+template <int NT, bool WEIGHTED, bool GATED, bool SHARED, int XP>
 __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __restrict__ h, const float* __restrict__ weight, int top,
                                                             const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
                                                             const int32_t* __restrict__ tile_pos, const bf16_t* __restrict__ w_gate,
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
                                                             float limit, float alpha, int n_tiles, int rows, int shared_y,
                                                             const SharedProduct shared) {
   if (SHARED && (int)blockIdx.y < shared_y) {
-    shared_product(shared, blockIdx.y * gridDim.x + blockIdx.x);
+    shared_product<XP>(shared, blockIdx.y * gridDim.x + blockIdx.x);
     return;
   }
   const int t0 = blockIdx.y - (SHARED ? shared_y : 0), e = tile_expert[t0];
@@ -660,15 +662,17 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
   int nt = 1;
   while (nt < NT && t0 + nt < n_tiles && tile_expert[t0 + nt] == e) ++nt;
   const int r = lane & 15, grp = lane >> 4;
+  static_assert(XP == 1 || NT == 1, "packed rows: runs of one tile");
   const bf16_t* xr[NT];
   float wt[NT];
   bool on[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
-    const int p = j < nt ? row_pair[(t0 + j) * RT_TILE + r] : -1;
-    on[j] = p >= 0;
+    const int at = (t0 + j) * RT_TILE;
+    const int p = j < nt ? row_pair[at + RowPack<XP>::row(r)] : -1;      // the row that this lane loads
+    on[j] = XP == 1 ? p >= 0 : row_pair[at + r] >= 0;
     wt[j] = (WEIGHTED && p >= 0) ? weight[p] : 1.0f;
-    xr[j] = h + (size_t)(p >= 0 ? p / top : 0) * width + 8 * grp;
+    xr[j] = h + (size_t)(p >= 0 ? p / top : 0) * width + RowPack<XP>::depth(r) + 8 * grp;
   }
   const bf16_t* gr = GATED ? w_gate + ((size_t)e * ff + c0) * rows * width + 8 * lane : nullptr;
   const bf16_t* ur = w_up + ((size_t)e * ff + c0) * rows * width + 8 * lane;
@@ -677,7 +681,7 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
   for (int j = 0; j < NT; ++j) ag[j] = au[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int n_steps = width / 32;
   struct Ahead {
-    Frag8 g[GATED ? RT_AHEAD : 1], u[RT_AHEAD], x[RT_AHEAD][NT];
+    Frag8 g[GATED ? RT_AHEAD : 1], u[RT_AHEAD], x[NT][RT_AHEAD / XP];
   };
   auto load = [&](Ahead& f, int s0, int cnt) __attribute__((always_inline)) {
 #pragma unroll
@@ -686,7 +690,8 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
       if (GATED) f.g[u].u = load16_stream(gr + 512 * s);
       f.u[u].u = load16_stream(ur + 512 * s);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) f.x[u][j].u = load16(xr[j] + 32 * s);
+      for (int j = 0; j < NT; ++j)
+        if (u % XP == 0) f.x[j][u / XP].u = load16(xr[j] + 32 * s);
     }
     __builtin_amdgcn_sched_barrier(0);            // all of them are on their way before anything is waited for
   };
@@ -696,9 +701,10 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
       if (u >= cnt) break;
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        if (WEIGHTED) f.x[u][j].u = scaled16(f.x[u][j].u, wt[j]);
-        if (GATED) ag[j] = mfma16(f.g[u], f.x[u][j], ag[j]);
-        au[j] = mfma16(f.u[u], f.x[u][j], au[j]);
+        if (WEIGHTED && u % XP == 0) f.x[j][u / XP].u = scaled16(f.x[j][u / XP].u, wt[j]);
+        const Frag8 x = RowPack<XP>::block(f.x[j], u);
+        if (GATED) ag[j] = mfma16(f.g[u], x, ag[j]);
+        au[j] = mfma16(f.u[u], x, au[j]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -716,13 +722,13 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
   }
 }
 
-template <int NT, bool SHARED>
+template <int NT, bool SHARED, int XP>
 __global__ __launch_bounds__(RB_WAVE) void routed_down_few_kernel(const bf16_t* __restrict__ y, const int32_t* __restrict__ row_pair,
                                                               const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_pos,
                                                               const bf16_t* __restrict__ w_down, float* __restrict__ out, int width, int ff,
                                                               int n_tiles, int shared_y, const SharedProduct shared) {
   if (SHARED && (int)blockIdx.y < shared_y) {
-    shared_product(shared, blockIdx.y * gridDim.x + blockIdx.x);
+    shared_product<XP>(shared, blockIdx.y * gridDim.x + blockIdx.x);
     return;
   }
   const int t0 = blockIdx.y - (SHARED ? shared_y : 0), e = tile_expert[t0];
@@ -736,13 +742,13 @@ __global__ __launch_bounds__(RB_WAVE) void routed_down_few_kernel(const bf16_t* 
 #pragma unroll
   for (int j = 0; j < NT; ++j) pair[j] = j < nt ? row_pair[(t0 + j) * RT_TILE + r] : -1;
   const bf16_t* dr = w_down + ((size_t)e * width + c0) * ff + 8 * lane;
-  const bf16_t* yr = y + (size_t)t0 * RT_TILE * ff + 8 * lane;
+  const bf16_t* yr = y + (size_t)t0 * RT_TILE * ff + 16 * RowPack<XP>::depth(r) + 8 * (16 * grp + RowPack<XP>::row(r));
   f32x4_t acc[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int n_steps = ff / 32;
   struct Ahead {
-    Frag8 d[RT_AHEAD], y[RT_AHEAD][NT];
+    Frag8 d[RT_AHEAD], y[NT][RT_AHEAD / XP];
   };
   auto load = [&](Ahead& f, int s0, int cnt) __attribute__((always_inline)) {
 #pragma unroll
@@ -750,7 +756,8 @@ __global__ __launch_bounds__(RB_WAVE) void routed_down_few_kernel(const bf16_t* 
       const size_t s = (size_t)(s0 + (u < cnt ? u : 0));
       f.d[u].u = load16_stream(dr + 512 * s);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) f.y[u][j].u = load16(yr + (size_t)(j < nt ? j : 0) * RT_TILE * ff + 512 * s);
+      for (int j = 0; j < NT; ++j)
+        if (u % XP == 0) f.y[j][u / XP].u = load16(yr + (size_t)(j < nt ? j : 0) * RT_TILE * ff + 512 * s);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -759,7 +766,7 @@ __global__ __launch_bounds__(RB_WAVE) void routed_down_few_kernel(const bf16_t* 
     for (int u = 0; u < RT_AHEAD; ++u) {
       if (u >= cnt) break;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j] = mfma16(f.d[u], f.y[u][j], acc[j]);
+      for (int j = 0; j < NT; ++j) acc[j] = mfma16(f.d[u], RowPack<XP>::block(f.y[j], u), acc[j]);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -992,37 +999,53 @@ extern "C" int rb_routed_experts_few(const void* h, const float* weight, int top
   if (max_rows == 0 || n_tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const int tiles = max_rows / RT_TILE;
-  if (shared_up) {
+  // Blocks of the rows a load: as many as the step's tokens leave room for, in whole trips of depth.  us of a layer's router and experts with one block
+  // a load and so, 4 of 16 experts, width and units 2,048: 4 tokens 48.8 and 45.4 (no gates), 65.1 and 63.6 (gates), 58.4 and 55.1 (gates, weighted
+  // inputs); 8 tokens 58.7 and 54.9, 76.2 and 74.3, 68.6 and 65.7.
+  const int deep = width % 128 == 0 && ff % 128 == 0 ? 4 : width % 64 == 0 && ff % 64 == 0 ? 2 : 1;
+  const int pack = n_tokens <= 4 ? deep : n_tokens <= 8 && deep >= 2 ? 2 : 1;
+#define RT_UP(NT, WEIGHTED, GATED, SHARED, XP, UP_Y, PRODUCT)                                                                                \
+  routed_up_few_kernel<NT, WEIGHTED, GATED, SHARED, XP><<<dim3(ff / 16, tiles + UP_Y), RB_WAVE, 0, s>>>(                                     \
+      (const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles, (const bf16_t*)w_gate, (const bf16_t*)w_up, (bf16_t*)y, width, ff, \
+      limit, alpha, tiles, rows, UP_Y, PRODUCT)
+#define RT_DOWN(NT, SHARED, XP, DOWN_Y, PRODUCT)                                                                                             \
+  routed_down_few_kernel<NT, SHARED, XP><<<dim3(width / 16, tiles + DOWN_Y), RB_WAVE, 0, s>>>(                                               \
+      (const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles, (const bf16_t*)w_down, out, width, ff, tiles, DOWN_Y, PRODUCT)
+#define RT_SHARED(XP)                              \
+  do {                                             \
+    RT_UP(1, false, false, true, XP, uy, up);      \
+    RT_DOWN(1, true, XP, 1, down);                 \
+  } while (0)
+#define RT_ALONE(NT, XP)                                                    \
+  do {                                                                      \
+    if (w_gate && weight) RT_UP(NT, true, true, false, XP, 0, none);        \
+    else if (w_gate) RT_UP(NT, false, true, false, XP, 0, none);            \
+    else if (weight) RT_UP(NT, true, false, false, XP, 0, none);            \
+    else RT_UP(NT, false, false, false, XP, 0, none);                       \
+    RT_DOWN(NT, false, XP, 0, none);                                        \
+  } while (0)
+  const SharedProduct none = {};
+  if (shared_up) {                            // (few tokens; its depths are multiples of 128)
     const SharedProduct up = {(const bf16_t*)h, (const bf16_t*)shared_up, shared_units, shared_act, shared_ff, width, n_tokens,
                               gemm_skinny_waves(shared_ff, width)};
     const SharedProduct down = {(const bf16_t*)shared_units, (const bf16_t*)shared_down, shared_out, nullptr, width, shared_ff, n_tokens,
                                 gemm_skinny_waves(width, shared_ff)};
     const int uy = (shared_ff / 16 + ff / 16 - 1) / (ff / 16);       // its tiles in rows of the experts' grid; down: one row
     RB_REQUIRE(tiles + uy <= 65535, "rb_routed_experts_few: too many rows");
-    routed_up_few_kernel<1, false, false, true><<<dim3(ff / 16, tiles + uy), RB_WAVE, 0, s>>>(
-        (const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles, nullptr, (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha,
-        tiles, rows, uy, up);
-    routed_down_few_kernel<1, true><<<dim3(width / 16, tiles + 1), RB_WAVE, 0, s>>>(
-        (const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles, (const bf16_t*)w_down, out, width, ff, tiles, 1, down);
-    RB_LAUNCH_CHECK();
-    return 0;
-  }
-  const dim3 gu(ff / 16, tiles), gd(width / 16, tiles);      // (both are multiples of 32)
-#define RT_UP(NT, WEIGHTED)                                                                                                           \
-  (w_gate ? routed_up_few_kernel<NT, WEIGHTED, true, false> : routed_up_few_kernel<NT, WEIGHTED, false, false>)<<<gu, RB_WAVE, 0, s>>>((const bf16_t*)h, weight, top, row_pair, tile_expert, tile_expert + tiles,    \
-                                                        (const bf16_t*)w_gate, (const bf16_t*)w_up, (bf16_t*)y, width, ff, limit, alpha, tiles, rows, 0, SharedProduct{})
-#define RT_DOWN(NT)                                                                                                       \
-  routed_down_few_kernel<NT, false><<<gd, RB_WAVE, 0, s>>>((const bf16_t*)y, row_pair, tile_expert, tile_expert + tiles,             \
-                                                (const bf16_t*)w_down, out, width, ff, tiles, 0, SharedProduct{})
-  if (n_tokens <= RT_TILE) {                  // a token chooses an expert once: no run is longer than the step's tokens
-    if (weight) RT_UP(1, true);
-    else RT_UP(1, false);
-    RT_DOWN(1);
+    if (pack == 4) RT_SHARED(4);
+    else if (pack == 2) RT_SHARED(2);
+    else RT_SHARED(1);
+  } else if (n_tokens > RT_TILE) {            // a token chooses an expert once: no run is longer than the step's tokens
+    RT_ALONE(4, 1);
+  } else if (pack == 4) {
+    RT_ALONE(1, 4);
+  } else if (pack == 2) {
+    RT_ALONE(1, 2);
   } else {
-    if (weight) RT_UP(4, true);
-    else RT_UP(4, false);
-    RT_DOWN(4);
+    RT_ALONE(1, 1);
   }
+#undef RT_ALONE
+#undef RT_SHARED
 #undef RT_UP
 #undef RT_DOWN
   RB_LAUNCH_CHECK();

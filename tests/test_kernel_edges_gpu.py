@@ -1491,6 +1491,26 @@ def test_splits_put_together_by_the_product_per_head_give_the_bits_of_two_launch
     assert torch.isfinite(want.float()).all() and torch.equal(got, want)
 
 
+# ---------------------------------------------------------------------------- experts of few tokens: packed loads
+@pytest.mark.parametrize("hidden,ff", [(96, 64), (64, 192), (128, 128), (384, 640), (2048, 256)])
+@pytest.mark.parametrize("params", [dict(score="softmax", weight_on="output", unit="squared_relu"), dict(score="chosen", weight_on="output"),
+                                    dict(limit=7.0), dict(score="softmax", weight_on="output", unit="squared_relu", shared={"intermediate_size": 128, "gate": False})])
+def test_a_tokens_experts_give_the_same_bits_however_many_tokens_a_load_brings(lib, hidden, ff, params):
+    """4, 2 or 1 blocks of depth a load by how many tokens there are: 16 tokens in a step, a block a load, and the same tokens in smaller ones."""
+    if params.get("shared") and (hidden % 128 or ff < 128):
+        params = dict(params, shared=None)
+    gen = torch.Generator().manual_seed(hidden + ff)
+    part = build_part("feed_forward", PartSpec("routed_experts", dict(params, experts=4, top=2, intermediate_size=ff)),
+                      BuildEnv(hidden_size=hidden, dtype=torch.bfloat16, device=torch.device(DEV), lib=lib))
+    part.load({name: (torch.randn(ts.shape, generator=gen) * ts.shape[-1] ** -0.5).to(torch.float32 if ts.role == "gain" else torch.bfloat16).to(DEV)
+               for name, ts in part.tensor_specs().items()})
+    h = torch.randn(16, hidden, generator=gen).bfloat16().to(DEV)
+    want = part.forward(h)
+    assert torch.isfinite(want).all()
+    for at in (slice(0, 1), slice(3, 6), slice(8, 12), slice(0, 5), slice(8, 16), slice(2, 11)):
+        assert torch.equal(part.forward(h[at].contiguous()), want[at])
+
+
 # ---------------------------------------------------------------------------- a norm with the convolution behind it
 @pytest.mark.parametrize("width", [4, 260, 2048, 4096])
 @pytest.mark.parametrize("taps,copies,update,biased,dtype", [(2, 1, False, True, torch.bfloat16), (3, 2, True, True, torch.float32),
