@@ -198,14 +198,22 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __rest
       if (n0 + 4 * kq + i < n) c[(size_t)r * n + n0 + 4 * kq + i] = sum[i];
 }
 
-template <int MB, int R, bool WF>
+//
+// At most 16 tokens, W fragment-major: XP blocks of 16 depth values that a load of the tokens brings, at most 16 / XP of them, and WP blocks
+// that a load of W brings, a workgroup then having 16 / WP of the tile's rows (RowPack in gemm_internal.h; the same sums).  U: stages a wave has
+// in registers.  A stage's 32 MFMAs add to one accumulator, 0.4 us one after the other, and behind them the next stage's loads took a trip to memory: with
+// two sets of registers they are under way meanwhile.  Where workgroups share a compute unit they do that for each other, and a wave
+// with more registers is slower (5,120 rows at K = 3072, 4 tokens: 14.9 us with one set, 15.9 with two).
+template <int MB, int R, bool WF, int XP = 1, int WP = 1, int U = 1>
 __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                           float* __restrict__ c, int m, int n, int k) {
   extern __shared__ float red[];      // [waves - 1][R * MB * 4][64]
   constexpr int ACC = R * MB * 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
   const int r = lane & 15, kq = lane >> 4;
-  const int n0 = blockIdx.x * (16 * R);
+  static_assert((XP == 1 || MB == 1) && (WP == 1 || (MB == 1 && R == 1 && WF)), "packed operands: one tile of tokens");
+  const int n0 = WP > 1 ? blockIdx.x / WP * 16 : blockIdx.x * (16 * R);
+  const int part0 = WP > 1 ? blockIdx.x % WP * (16 / WP) : 0;      // WP > 1: this workgroup has 16 / WP of the tile's rows
   gf_f32x4_t acc[R][MB];
 #pragma unroll
   for (int rt = 0; rt < R; ++rt)
@@ -220,50 +228,81 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
 #pragma unroll
   for (int rt = 0; rt < R; ++rt) {
     const int row = n0 + 16 * rt + r;
-    if (WF) wrow[rt] = w + (size_t)(n0 + 16 * rt < n ? n0 + 16 * rt : 0) * k + 4 * lane;
+    if (WP > 1) wrow[rt] = w + (size_t)n0 * k + 256 * (r / (16 / WP)) + 4 * (16 * kq + part0 + r % (16 / WP));
+    else if (WF) wrow[rt] = w + (size_t)(n0 + 16 * rt < n ? n0 + 16 * rt : 0) * k + 4 * lane;
     else wrow[rt] = w + (size_t)(row < n ? row : 0) * k + 4 * kq;        // rows beyond N: row 0, never stored
   }
   const float* xrow[MB];
 #pragma unroll
   for (int cb = 0; cb < MB; ++cb) {
-    const int row = 16 * cb + r;
-    xrow[cb] = x + (size_t)(row < m ? row : 0) * k + 4 * kq;
+    const int row = 16 * cb + r % (16 / XP);
+    xrow[cb] = x + (size_t)(row < m ? row : 0) * k + 16 * (r / (16 / XP)) + 4 * kq;
   }
   // the K / 128 stages dealt to the waves as evenly as they go (the host launches no more waves than stages)
   const int total = k / 128, base = total / n_waves, extra = total % n_waves;
   const int stages = base + (wave < extra ? 1 : 0);
   const int k_begin = 128 * (wave * base + (wave < extra ? wave : extra));
-  gf_f32x4_t a[R][8], b[MB][8];
-  auto load_stage = [&](int st) {
+  static_assert(U == 1 || (U == 2 && MB == 1 && R == 1), "two stages in registers: one tile of tokens and of rows");
+  gf_f32x4_t as[U][R][8 / WP], bs[U][MB][8 / XP];
+  auto load_stage = [&](int u, int st) __attribute__((always_inline)) {
+    auto &a = as[u];
+    auto &b = bs[u];
     const int ks = k_begin + 128 * st;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < 8 / WP; ++j)
 #pragma unroll
       for (int rt = 0; rt < R; ++rt)
-        a[rt][j] = WF ? __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + (size_t)(ks + 16 * j) * WK))
-                      : *reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + ks + 16 * j);
+        a[rt][j] = WF ? __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + (size_t)(ks + 16 * WP * j) * WK))
+                      : *reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + ks + 16 * WP * j);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < 8 / XP; ++j)
 #pragma unroll
-      for (int cb = 0; cb < MB; ++cb) b[cb][j] = *reinterpret_cast<const gf_f32x4_t*>(xrow[cb] + ks + 16 * j);
+      for (int cb = 0; cb < MB; ++cb) b[cb][j] = *reinterpret_cast<const gf_f32x4_t*>(xrow[cb] + ks + 16 * XP * j);
   };
-  auto multiply_stage = [&]() {
+  auto multiply_stage = [&](int u) __attribute__((always_inline)) {
+    auto &a = as[u];
+    auto &b = bs[u];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < 8; ++j) {
+      gf_f32x4_t aj[R], bj[MB];
+#pragma unroll
+      for (int rt = 0; rt < R; ++rt) aj[rt] = RowPack<WP>::turned(a[rt][j / WP], j % WP);
+#pragma unroll
+      for (int cb = 0; cb < MB; ++cb) bj[cb] = RowPack<XP>::turned(b[cb][j / XP], j % XP);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int rt = 0; rt < R; ++rt)
 #pragma unroll
-          for (int cb = 0; cb < MB; ++cb)
-            acc[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][j][i], b[cb][j][i], acc[rt][cb], 0, 0, 0);
+          for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aj[rt][i], bj[cb][i], acc[rt][cb], 0, 0, 0);
+    }
   };
-  load_stage(0);
-  for (int st = 1; st < stages; ++st) {
-    multiply_stage();
-    load_stage(st);
+  load_stage(0, 0);
+  if constexpr (U == 2) {
+    int st = 0;
+    for (; st + 2 < stages; st += 2) {
+      load_stage(1, st + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply_stage(0);
+      load_stage(0, st + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply_stage(1);
+    }
+    if (st + 1 < stages) {
+      load_stage(1, st + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply_stage(0);
+      multiply_stage(1);
+    } else {
+      multiply_stage(0);
+    }
+  } else {
+    for (int st = 1; st < stages; ++st) {
+      multiply_stage(0);
+      load_stage(0, st);
+    }
+    multiply_stage(0);
   }
-  multiply_stage();
 
   if (n_waves > 1) {
     if (wave > 0) {
@@ -288,11 +327,12 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
     }
   }
   // lane l holds, for token 16 cb + l % 16, the rows n0 + 16 rt + 4 (l / 16) + i
+  if (WP > 1 && kq >= 4 / WP) return;
 #pragma unroll
   for (int rt = 0; rt < R; ++rt)
 #pragma unroll
     for (int cb = 0; cb < MB; ++cb) {
-      const int mm = 16 * cb + r, nn = n0 + 16 * rt + 4 * kq;
+      const int mm = 16 * cb + r, nn = n0 + part0 + 16 * rt + 4 * kq;
       if (mm >= m) continue;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -303,6 +343,9 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
 static int g_f32_few = 1;
 // experiments only: 0 = the float32 product of few tokens (W as rows) on the vector units; 3 = one row tile a wave whatever the sizes
 extern "C" void rb_tune_f32_few(int on) { g_f32_few = on; }
+
+static int g_f32_parts = 0;
+extern "C" void rb_tune_f32_parts(int parts) { g_f32_parts = parts; }      // experiments and tests only: 1 or 2 workgroups for a tile of 16 rows; 0 = the built-in choice
 
 // One row tile per wave and at most 4 waves: measured at 1 to 16 tokens on the products of the 8B shape with W
 // fragment-major, two row tiles a wave lose everywhere but in the output matrix at 16 tokens (28,672 rows at
@@ -329,6 +372,20 @@ static void launch_f32_few(const float* x, const float* w, bool w_frag, float* c
   }
   const size_t lds = (size_t)(n_waves - 1) * MB * 4 * 64 * sizeof(float);
   const int grid = (n + 15) / 16;
+  if constexpr (MB == 1) {
+    // us, 4 tokens, as the kernel was (one stage, a block a load, whole tiles) and so: 3,072 rows at K = 3072 9.75 and 8.8, at 8192 24.3 and 21.3; 2,048 at 2048
+    // 7.2 and 5.9, 1,024 at 4096 10.8 and 8.3 (halves of tiles); more workgroups than compute units: 5,120 at 3072 17.4 and 14.9, 16,384 38.0 and 35.0,
+    // 128,256 260 and 239, 6,144 at 4096 23.4 and 20.7.  Halves of more tiles than half the units lose (3,072 rows at 3072 11.9).
+    if (w_frag) {
+      const int cus = rb_compute_units(), parts = g_f32_parts ? g_f32_parts : 2 * grid <= cus ? 2 : 1, pack = m <= 4 ? 4 : m <= 8 ? 2 : 1;
+      auto by = [&](auto four, auto two, auto one) { return pack == 4 ? four : pack == 2 ? two : one; };
+      (parts == 2    ? by(gemm_f32_few_kernel<1, 1, true, 4, 2, 2>, gemm_f32_few_kernel<1, 1, true, 2, 2, 2>, gemm_f32_few_kernel<1, 1, true, 1, 2, 2>)
+       : grid <= cus ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2>      // (packed tokens: 4,096 rows at K = 4096 14.2 for 13.9, the others the same)
+                     : by(gemm_f32_few_kernel<1, 1, true, 4>, gemm_f32_few_kernel<1, 1, true, 2>, gemm_f32_few_kernel<1, 1, true>))<<<
+          parts * grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
+      return;
+    }
+  }
   if (w_frag) gemm_f32_few_kernel<MB, 1, true><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
   else gemm_f32_few_kernel<MB, 1, false><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
 }

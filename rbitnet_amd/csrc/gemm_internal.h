@@ -46,22 +46,27 @@ struct RowPack {
   static_assert(XP == 1 || XP == 2 || XP == 4, "a stage is four blocks");
   static __device__ __forceinline__ int row(int r) { return r % (16 / XP); }
   static __device__ __forceinline__ int depth(int r) { return 32 * (r / (16 / XP)); }
+  // 16 bytes of block `turn` (a constant) of those that a load brought, in the lanes of the operand's rows
+  template <typename V>
+  static __device__ __forceinline__ V turned(const V& of, int turn) {
+    static_assert(sizeof(V) == 16, "16 bytes a lane");
+    if (XP == 1 || turn == 0) return of;
+    struct Words {
+      int v[4];
+    };
+    Words w = __builtin_bit_cast(Words, of);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)                             // row_ror: lane r gets what lane (r - n) % 16 holds
+      w.v[i] = 16 / XP * turn == 4   ? __builtin_amdgcn_update_dpp(w.v[i], w.v[i], 0x12C, 0xF, 0xF, true)
+               : 16 / XP * turn == 8 ? __builtin_amdgcn_update_dpp(w.v[i], w.v[i], 0x128, 0xF, 0xF, true)
+                                     : __builtin_amdgcn_update_dpp(w.v[i], w.v[i], 0x124, 0xF, 0xF, true);
+    return __builtin_bit_cast(V, w);
+  }
   // block j of those that these loads brought
   template <int N>
   static __device__ __forceinline__ Frag8 block(const Frag8 (&b)[N], int j) {
-    Frag8 f = b[j / XP];
-    const int turn = j % XP;
-    if (XP == 1 || turn == 0) return f;
-    uint32_t v[4] = {f.u.x, f.u.y, f.u.z, f.u.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int old = (int)v[i];
-      // row_ror: lane r gets what lane (r - n) % 16 holds
-      v[i] = (uint32_t)(16 / XP * turn == 4    ? __builtin_amdgcn_update_dpp(old, old, 0x12C, 0xF, 0xF, true)
-                        : 16 / XP * turn == 8  ? __builtin_amdgcn_update_dpp(old, old, 0x128, 0xF, 0xF, true)
-                                               : __builtin_amdgcn_update_dpp(old, old, 0x124, 0xF, 0xF, true));
-    }
-    f.u = make_uint4(v[0], v[1], v[2], v[3]);
+    Frag8 f;
+    f.u = turned(b[j / XP].u, j % XP);
     return f;
   }
 };

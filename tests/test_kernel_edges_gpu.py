@@ -1491,6 +1491,34 @@ def test_splits_put_together_by_the_product_per_head_give_the_bits_of_two_launch
     assert torch.isfinite(want.float()).all() and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("n,k", [(16, 128), (48, 384), (2048, 256), (2064, 512), (1040, 2048), (96, 8192), (4096, 640), (4112, 128), (6144, 384)])
+def test_a_row_of_a_float32_product_has_the_same_bits_however_its_operands_are_loaded(lib, n, k):
+    """As above, with one and two stages in registers besides (up to and beyond a workgroup a compute unit); against float64 as well: a sum of K products
+    is off by K 2^-24 of the sum of their sizes at the most."""
+    gen = torch.Generator().manual_seed(n + k)
+    x, rows = torch.randn(16, k, generator=gen), torch.randn(n, k, generator=gen) * k ** -0.5
+    w = torch.empty(n, k, device=DEV)
+    lib.place_rows(rows.to(DEV), w, frag=True)
+
+    def product(m):
+        out = torch.full((m, n), float("nan"), device=DEV)
+        lib.gemm_generic(x[:m].contiguous().to(DEV), w, out, w_frag=True)
+        return out
+    try:
+        lib._lib.rb_tune_f32_parts(1)
+        whole = product(16)
+        _within(whole, x.double() @ rows.double().T, k * 2.0 ** -24 * (x.double().abs() @ rows.double().abs().T))
+        for parts in (0, 1, 2):
+            lib._lib.rb_tune_f32_parts(parts)
+            for units in (0, 1, 1024):                       # workgroups that share a compute unit, and none that do
+                lib._lib.rb_tune_compute_units(units)
+                for m in (16, 9, 8, 5, 4, 1):
+                    assert torch.equal(product(m), whole[:m]), (parts, units, m)
+    finally:
+        lib._lib.rb_tune_f32_parts(0)
+        lib._lib.rb_tune_compute_units(0)
+
+
 # ---------------------------------------------------------------------------- experts of few tokens: packed loads
 @pytest.mark.parametrize("hidden,ff", [(96, 64), (64, 192), (128, 128), (384, 640), (2048, 256)])
 @pytest.mark.parametrize("params", [dict(score="softmax", weight_on="output", unit="squared_relu"), dict(score="chosen", weight_on="output"),
