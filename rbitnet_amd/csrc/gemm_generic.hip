@@ -142,6 +142,18 @@ __global__ __launch_bounds__(256) void gemm_f32_skinny_kernel(const float* __res
 // meet in LDS in a fixed order.
 typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
 
+// The gate's sums times those of the way up: which 0: the wave that has the gate's, 1: that has the others, -1: any other wave (all waves come here).
+// silu as rb_swiglu computes it.
+__device__ __forceinline__ gf_f32x4_t gated_end(gf_f32x4_t sum, float* __restrict__ lds, int lane, int which) {
+  if (which == 1) *reinterpret_cast<gf_f32x4_t*>(lds + 4 * lane) = sum;
+  __syncthreads();
+  if (which != 0) return sum;
+  const gf_f32x4_t u = *reinterpret_cast<const gf_f32x4_t*>(lds + 4 * lane);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sum[i] = sum[i] / (1.0f + expf(-sum[i])) * u[i];
+  return sum;
+}
+
 // At most 16 tokens and a depth of at most 1,024 that is no multiple of 128 (K a multiple of 4, W as rows): a launch that is
 // little more than its trips to memory.  Fragments as in the kernel below, a stage of 128 depth values per wave and trip, what lies
 // behind K counts as zeros.  Every one of a stage's 32 products has an accumulator of its own, and they meet as a tree: no chain
@@ -150,12 +162,19 @@ typedef __attribute__((ext_vector_type(4))) float gf_f32x4_t;
 // 144 rows at K = 96, 4 / 16 tokens: 6.0 / 18.3 us in the kernel above, 3.0 / 3.1 here; 32,000 rows at K = 100 17.0 / 74.8 and 7.7 / 8.7.
 // Its loads take 64 bytes of a row, the kernel above 1 KB: with many rows and K > 128 that one is the better for few tokens (32,000 rows
 // at K = 500: 22.6 against 29.3 us with 4 tokens, 80 against 36 with 16; 4,096 rows at K = 1,000: 9.3 against 7.5).
-__global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ c,
+// GATED: W is the gate's n rows and then n rows of the way up (n % 16 == 0), c [m, n] = silu(gate) up.  Twice the waves: the first half takes a tile of the
+// gate, the other half the same rows of the way up, whose sums go to the first through LDS (gated_end).  The launch of 1 to 128 workgroups that
+// did this behind the product cost a step 2 us; every sum and the gate are as they are in two launches.
+template <bool GATED>
+__global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ c,
                                                             int m, int n, int k) {
-  extern __shared__ float red[];      // [waves - 1][4][64]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+  extern __shared__ float lds[];      // [waves - 1][4][64] for each of gate and way up, then, gated, [4][64]
+  const int lane = threadIdx.x & 63, n_waves = (blockDim.x >> 6) / (GATED ? 2 : 1);
+  const int up = GATED && (int)(threadIdx.x >> 6) >= n_waves ? 1 : 0, wave = (threadIdx.x >> 6) - up * n_waves;
+  float* red = lds + up * (n_waves - 1) * 256;
   const int r = lane & 15, kq = lane >> 4;
   const int n0 = blockIdx.x * 16;
+  if (up) w += (size_t)n * k;
   // rows beyond N and tokens beyond M: row 0 and token 0, never stored
   const float* wrow = w + (size_t)(n0 + r < n ? n0 + r : 0) * k + 4 * kq;
   const float* xrow = x + (size_t)(r < m ? r : 0) * k + 4 * kq;
@@ -186,10 +205,15 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __rest
 #pragma unroll
       for (int i = 0; i < 4; ++i) red[((wave - 1) * 4 + i) * 64 + lane] = sum[i];
     __syncthreads();
-    if (wave > 0) return;
-    for (int o = 1; o < n_waves; ++o)
+    if (!GATED && wave > 0) return;
+    if (wave == 0)
+      for (int o = 1; o < n_waves; ++o)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sum[i] += red[((o - 1) * 4 + i) * 64 + lane];
+        for (int i = 0; i < 4; ++i) sum[i] += red[((o - 1) * 4 + i) * 64 + lane];
+  }
+  if (GATED) {
+    sum = gated_end(sum, lds + 2 * (n_waves - 1) * 256, lane, wave == 0 ? up : -1);
+    if (wave > 0 || up) return;
   }
   // lane l holds rows 4 (l / 16) + i of token l % 16
   if (r < m)
@@ -204,12 +228,17 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __rest
 // in registers.  A stage's 32 MFMAs add to one accumulator, 0.4 us one after the other, and behind them the next stage's loads took a trip to memory: with
 // two sets of registers they are under way meanwhile.  Where workgroups share a compute unit they do that for each other, and a wave
 // with more registers is slower (5,120 rows at K = 3072, 4 tokens: 14.9 us with one set, 15.9 with two).
-template <int MB, int R, bool WF, int XP = 1, int WP = 1, int U = 1>
-__global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
+// GATED: as in the kernel above.
+template <int MB, int R, bool WF, int XP = 1, int WP = 1, int U = 1, bool GATED = false>
+__global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                           float* __restrict__ c, int m, int n, int k) {
-  extern __shared__ float red[];      // [waves - 1][R * MB * 4][64]
+  extern __shared__ float lds[];      // [waves - 1][R * MB * 4][64] (for each of gate and way up, then [4][64])
+  static_assert(!GATED || (MB == 1 && R == 1 && WP == 1), "gated: one tile of tokens, one of gate rows");
   constexpr int ACC = R * MB * 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, n_waves = (blockDim.x >> 6) / (GATED ? 2 : 1);
+  const int up = GATED && (int)(threadIdx.x >> 6) >= n_waves ? 1 : 0, wave = (threadIdx.x >> 6) - up * n_waves;
+  float* red = lds + up * (n_waves - 1) * ACC * 64;
+  if (up) w += (size_t)n * k;
   const int r = lane & 15, kq = lane >> 4;
   static_assert((XP == 1 || MB == 1) && (WP == 1 || (MB == 1 && R == 1 && WF)), "packed operands: one tile of tokens");
   const int n0 = WP > 1 ? blockIdx.x / WP * 16 : blockIdx.x * (16 * R);
@@ -315,8 +344,8 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
           for (int i = 0; i < 4; ++i) dst[((rt * MB + cb) * 4 + i) * 64] = acc[rt][cb][i];
     }
     __syncthreads();
-    if (wave != 0) return;
-    for (int ww = 0; ww < n_waves - 1; ++ww) {
+    if (!GATED && wave != 0) return;
+    for (int ww = 0; ww < (wave == 0 ? n_waves - 1 : 0); ++ww) {
       const float* src = red + (size_t)ww * ACC * 64 + lane;
 #pragma unroll
       for (int rt = 0; rt < R; ++rt)
@@ -325,6 +354,10 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc[rt][cb][i] += src[((rt * MB + cb) * 4 + i) * 64];
     }
+  }
+  if constexpr (GATED) {
+    acc[0][0] = gated_end(acc[0][0], lds + 2 * (n_waves - 1) * ACC * 64, lane, wave == 0 ? up : -1);
+    if (wave > 0 || up) return;
   }
   // lane l holds, for token 16 cb + l % 16, the rows n0 + 16 rt + 4 (l / 16) + i
   if (WP > 1 && kq >= 4 / WP) return;
@@ -351,11 +384,16 @@ extern "C" void rb_tune_f32_parts(int parts) { g_f32_parts = parts; }      // ex
 // fragment-major, two row tiles a wave lose everywhere but in the output matrix at 16 tokens (28,672 rows at
 // K = 4096, 8 tokens: 78 us against 93; 4,096 rows at K = 14336: 38 against 54), and 4 waves are as fast as 8
 // or faster (4,096 rows at K = 4096: 13.2 us against 14.4).  The kernel is never launched with more.
+static int f32_few_waves(int k) { return k < 512 ? 1 : k < 1024 ? k / 256 : 4; }
+// K = 96 of a step's few tokens and the like: see gemm_f32_short_kernel
+static int f32_short_waves(int k) { return k <= 128 ? 1 : k <= 256 ? 2 : k <= 384 ? 3 : 4; }
+static bool f32_short_takes(int m, int n, int k) {
+  return m <= 16 && k % 4 == 0 && k <= 1024 && (k <= 128 || m > 8 || (long long)n * k <= 1 << 22) && g_f32_few;
+}
+
 template <int MB>
 static void launch_f32_few(const float* x, const float* w, bool w_frag, float* c, int m, int n, int k, hipStream_t s) {
-  int n_waves = k / 256;
-  if (n_waves < 1) n_waves = 1;
-  if (n_waves > 4) n_waves = 4;
+  const int n_waves = f32_few_waves(k);
   // From 33 tokens on a wave reads three to four times as many bytes of tokens as of W for every stage: two row
   // tiles a wave halve that (28,672 rows at K = 4096 with 64 tokens: 220 us against 305; 128,256 rows: 868
   // against 1,335; with 33 tokens 227 against 262).
@@ -507,6 +545,31 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
     }
 }
 
+// Whether gate and way up of ff units each go in one launch with the gate on their sums (float32, W [2 ff, K] the gate's rows and then the others):
+// at most 16 tokens, sizes that a product of them alone takes on the two kernels for few tokens.
+extern "C" int rb_gemm_f32_gated_ok(int m, int ff, int k, int w_layout) {
+  if (m < 1 || m > 16 || ff < 16 || ff % 16 != 0 || ff > 1 << 26 || k < 4 || !g_f32_few) return 0;
+  if (w_layout == 1) return k % 128 == 0;
+  return w_layout == 0 && k % 128 != 0 && f32_short_takes(m, 2 * ff, k);
+}
+
+extern "C" int rb_gemm_f32_gated(const float* a, const float* w, int w_layout, float* c, int m, int ff, int k, void* stream) {
+  RB_RECORDED(rb_gemm_f32_gated(a, w, w_layout, c, m, ff, k, stream));
+  RB_REQUIRE(m == 0 || rb_gemm_f32_gated_ok(m, ff, k, w_layout), "rb_gemm_f32_gated: M=%d ff=%d K=%d, layout %d are not for it", m, ff, k, w_layout);
+  if (m == 0) return 0;
+  hipStream_t s = (hipStream_t)stream;
+  const int grid = ff / 16, n_waves = w_layout ? f32_few_waves(k) : f32_short_waves(k);
+  const size_t lds = ((size_t)2 * (n_waves - 1) * 256 + 256) * sizeof(float);
+  auto kern = !w_layout                        ? gemm_f32_short_kernel<true>
+              : 2 * grid <= rb_compute_units() ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2, true>      // (8 waves a workgroup: as two workgroups above)
+              : m <= 4                         ? gemm_f32_few_kernel<1, 1, true, 4, 1, 1, true>
+              : m <= 8                         ? gemm_f32_few_kernel<1, 1, true, 2, 1, 1, true>
+                                               : gemm_f32_few_kernel<1, 1, true, 1, 1, 1, true>;
+  kern<<<grid, 2 * 64 * n_waves, lds, s>>>(a, w, c, m, ff, k);
+  RB_LAUNCH_CHECK();
+  return 0;
+}
+
 extern "C" int rb_gemm_generic(const void* a, const void* w, int w_layout, void* c, int dtype_in, int dtype_out, int m,
                                int n, int k, void* stream) {
   RB_RECORDED(rb_gemm_generic(a, w, w_layout, c, dtype_in, dtype_out, m, n, k, stream));
@@ -528,9 +591,9 @@ extern "C" int rb_gemm_generic(const void* a, const void* w, int w_layout, void*
     RB_LAUNCH_CHECK();
     return 0;
   }
-  if (dtype_in == RB_F32 && dtype_out == RB_F32 && m <= 16 && k % 4 == 0 && k <= 1024 && (k <= 128 || m > 8 || (long long)n * k <= 1 << 22) && g_f32_few) {
-    const int n_waves = k <= 128 ? 1 : k <= 256 ? 2 : k <= 384 ? 3 : 4;
-    gemm_f32_short_kernel<<<(n + 15) / 16, 64 * n_waves, (size_t)(n_waves - 1) * 4 * 64 * sizeof(float), s>>>((const float*)a, (const float*)w,
+  if (dtype_in == RB_F32 && dtype_out == RB_F32 && f32_short_takes(m, n, k)) {
+    const int n_waves = f32_short_waves(k);
+    gemm_f32_short_kernel<false><<<(n + 15) / 16, 64 * n_waves, (size_t)(n_waves - 1) * 4 * 64 * sizeof(float), s>>>((const float*)a, (const float*)w,
                                                                                                      (float*)c, m, n, k);
     RB_LAUNCH_CHECK();
     return 0;

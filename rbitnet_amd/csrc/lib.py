@@ -105,7 +105,7 @@ class KernelTimes:
         return "\n".join(lines)
 
 
-TIMED_OPS = ("routed_experts_tiled", "recurrence_step", "gemm_bf16_group", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
+TIMED_OPS = ("gemm_f32_gated", "heads_combined", "routed_experts_tiled", "recurrence_step", "gemm_bf16_group", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
              "route_top", "routed_experts", "pairs_sum", "embed_streams", "streams_layernorm", "streams_update", "xielu", "tanh_cap", "short_conv",
              "delta_prep", "delta_rule", "gated_rmsnorm", "latent_norm_store", "attention_sinks", "embed_gather", "add_rmsnorm", "rope_kv_write", "swiglu", "gemm_generic", "gemm_bf16", "gemm_bf16_terms",
              "gemm_bf16_few", "attention_generic", "attention_prefill_bf16", "attention_decode_bf16",
@@ -157,6 +157,8 @@ class Kernels:
             "rb_rope_kv_write": [_P, _I, ctypes.c_longlong, _P, _P, _I, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _P],
             "rb_swiglu": [_P, _P, _I, _I, _I, _P],
             "rb_gemm_generic": [_P, _P, _I, _P, _I, _I, _I, _I, _I, _P],
+            "rb_gemm_f32_gated_ok": [_I, _I, _I, _I],
+            "rb_gemm_f32_gated": [_P, _P, _I, _P, _I, _I, _I, _P],
             "rb_gemm_bf16": [_P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _P],
             "rb_gemm_bf16_act": [_P, _P, _I, _P, _I, _I, _P, _I, _I, _I, _P, _P],
             "rb_gemm_bf16_few": [_P, _P, _F, _P, _P, _I, _P, _I, _I, _P, _P, _P, _I, _I, _I, _P],
@@ -369,6 +371,18 @@ class Kernels:
         _check(c, "c", None, (m, n))
         self._ok(self._lib.rb_gemm_generic(_ptr(a), _ptr(w), int(bool(w_frag)), _ptr(c), dtype_code(a.dtype),
                                            dtype_code(c.dtype), m, n, k, self._stream()))
+
+    def gemm_f32_gated_ok(self, m: int, ff: int, k: int, w_frag: bool) -> bool:
+        return bool(self._lib.rb_gemm_f32_gated_ok(m, ff, k, int(bool(w_frag))))
+
+    def gemm_f32_gated(self, a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, w_frag: bool = False) -> None:
+        """`gemm_generic` with w [2 ff, K] (the gate's rows, then those of the way up) and `swiglu` in one launch (sizes that `gemm_f32_gated_ok`)."""
+        m, k = a.shape
+        ff = c.shape[1]
+        _check(a, "a", torch.float32)
+        _check(w, "w", torch.float32, (2 * ff, k))
+        _check(c, "c", torch.float32, (m, ff))
+        self._ok(self._lib.rb_gemm_f32_gated(_ptr(a), _ptr(w), int(bool(w_frag)), _ptr(c), m, ff, k, self._stream()))
 
     def gemm_bf16(self, a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, epilogue: int = 0,
                   w_frag: bool = False, act: Optional[torch.Tensor] = None) -> None:

@@ -211,6 +211,9 @@ def gated_linear(lib, x, w_packed, ff: int, fused: bool, gate: Optional[torch.Te
     if fused:
         wd, frag = _data(w_packed)
         lib.gemm_bf16(x, wd, out, 1, w_frag=frag, act=gate)
+    elif x.dtype == torch.float32 and lib.gemm_f32_gated_ok(m, ff, x.shape[1], _data(w_packed)[1]):
+        wd, frag = _data(w_packed)
+        lib.gemm_f32_gated(x, wd, out, w_frag=frag)
     else:
         gu = linear(lib, x, w_packed, torch.float32)
         lib.swiglu(gu, out)

@@ -1519,6 +1519,29 @@ def test_a_row_of_a_float32_product_has_the_same_bits_however_its_operands_are_l
         lib._lib.rb_tune_compute_units(0)
 
 
+@pytest.mark.parametrize("ff,k,frag", [(16, 128, True), (256, 96, False), (48, 500, False), (4096, 100, False), (2048, 512, True), (4112, 768, True), (1024, 3072, True),
+                                       (80, 8192, True)])
+def test_a_float32_gate_on_its_products_sums_gives_the_bits_of_two_launches(lib, ff, k, frag):
+    gen = torch.Generator().manual_seed(ff + k)
+    rows = torch.randn(2 * ff, k, generator=gen) * k ** -0.5
+    rows[:8] *= 300.0                                        # gates whose exponentials are none
+    w = rows.to(DEV)
+    if frag:
+        w = torch.empty(2 * ff, k, device=DEV)
+        lib.place_rows(rows.to(DEV), w, frag=True)
+    for m in (1, 4, 5, 8, 9, 16):
+        x = torch.randn(m, k, generator=gen).to(DEV)
+        got, gu, want = torch.full((m, ff), float("nan"), device=DEV), torch.empty(m, 2 * ff, device=DEV), torch.empty(m, ff, device=DEV)
+        if not lib.gemm_f32_gated_ok(m, ff, k, frag):
+            assert not frag and k > 128 and m <= 8           # (many rows of a longer depth: another kernel's)
+            continue
+        lib.gemm_f32_gated(x, w, got, w_frag=frag)
+        lib.gemm_generic(x, w, gu, w_frag=frag)
+        lib.swiglu(gu, want)
+        assert torch.isfinite(want).all() and torch.equal(got, want)
+    assert not lib.gemm_f32_gated_ok(17, ff, k, frag) and not lib.gemm_f32_gated_ok(4, ff + 8, k, frag)
+
+
 # ---------------------------------------------------------------------------- experts of few tokens: packed loads
 @pytest.mark.parametrize("hidden,ff", [(96, 64), (64, 192), (128, 128), (384, 640), (2048, 256)])
 @pytest.mark.parametrize("params", [dict(score="softmax", weight_on="output", unit="squared_relu"), dict(score="chosen", weight_on="output"),
