@@ -99,6 +99,12 @@ int rb_gemm_bf16_few(const void* a, const float* squares_in, float eps, const in
                      int w_layout, void* c, int dtype_out, int epilogue, const float* gain, void* gained,
                      float* squares_out, int m, int n, int k, void* stream);
 
+// The same in float32 (W rows, or fragment-major as rb_gemm_generic takes it).  Sums of squares over every 8 columns: squares_in [*, ceil(K / 8)],
+// squares_out [M, ceil(N / 8)]; gained float32.  epilogue 1: W has the gate's N / 2 rows and then those of the way up, C [M, N / 2].
+int rb_gemm_f32_few_ok(int m, int n, int k, int w_layout, int epilogue);
+int rb_gemm_f32_few(const float* a, const float* squares_in, float eps, const int32_t* rows, const float* w, int w_layout, float* c, int epilogue,
+                    const float* gain, float* gained, float* squares_out, int m, int n, int k, void* stream);
+
 // Causal attention of every token over its sequence's cache (keys 0..pos, or the last
 // `window` of them), any head_dim up to 512 (a rotation in front of it needs an even one).
 //   q [T, Hq, D], out [T, Hq * D], both of dtype; pages as in rb_rope_kv_write.

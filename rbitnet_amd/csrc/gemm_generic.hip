@@ -154,6 +154,77 @@ __device__ __forceinline__ gf_f32x4_t gated_end(gf_f32x4_t sum, float* __restric
   return sum;
 }
 
+// What stands before and after a product of at most 16 tokens in a step, done by the product (FOLD): the tokens are rows times a norm's gain, of which
+// squares_in has the sums of squares over every 8 columns, and the sums are multiplied by the norm's factor; they are added to C and leave
+// the same of C for the norm that follows.  Eight columns because a workgroup may have half of a tile's 16 rows.
+// A norm of 4 rows as a launch of its own is 4 workgroups that wait twice for memory behind every product that ends a sublayer; what it leaves to the
+// products is 384 sums of squares a token at width 3,072, asked for with the first stage, and one more number a lane to load and store.  Captured steps of
+// 4 sequences, with such launches and so: width 3,072, 28 layers 3,126 and 3,049 us, width 96, 3 layers 124 and 122.
+struct F32Fold {
+  const float* squares_in;      // null: the tokens as they are; else [*, ceil(K / 8)]
+  const int32_t* rows;          // which rows of x (and of squares_in) the tokens are; null: 0..M-1
+  float eps;
+  int add;                      // C += the sums
+  const float* gain;            // null: nothing for a norm; else [N], and
+  float* gained;                //   [M, N] = C gain
+  float* squares_out;           //   [M, ceil(N / 8)] = sums of C^2
+  int wide;                     // C, the gain and the prepared rows can be read and written four columns at a time
+};
+constexpr int F32_SQ_WIDE = 8;
+
+__device__ __forceinline__ gf_f32x4_t four_of(const float* __restrict__ at, int left, int wide) {
+  if (wide) return *reinterpret_cast<const gf_f32x4_t*>(at);
+  gf_f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i < left) v[i] = at[i];
+  return v;
+}
+__device__ __forceinline__ void put_four(float* __restrict__ at, gf_f32x4_t v, int left, int wide) {
+  if (wide) {
+    *reinterpret_cast<gf_f32x4_t*>(at) = v;
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i < left) at[i] = v[i];
+}
+// The four lanes of a wave that share token r hold their shares of its squares: `lds` [waves][16] takes the waves' sums, before the barrier ...
+__device__ __forceinline__ float squares_meet(float ss, float* __restrict__ lds, int wave, int lane) {
+  ss += __shfl_xor(ss, 16, RB_WAVE);
+  ss += __shfl_xor(ss, 32, RB_WAVE);
+  if (lane < 16) lds[wave * 16 + lane] = ss;
+  return ss;
+}
+// ... and behind it (with one wave there is none: its own sum) they make the norm's factor
+__device__ __forceinline__ float squares_factor(float own, const float* __restrict__ lds, int n_waves, int lane, int k, float eps) {
+  float ss = own;
+  if (n_waves > 1) {
+    ss = 0.f;
+    for (int ww = 0; ww < n_waves; ++ww) ss += lds[ww * 16 + (lane & 15)];
+  }
+  return 1.0f / sqrtf(ss / (float)k + eps);
+}
+// The end of such a product: a lane's four sums of token mm, columns nn.. (both in range); lanes 16 apart have the two halves of 8 columns
+__device__ __forceinline__ void fold_end(gf_f32x4_t v, gf_f32x4_t before, gf_f32x4_t gain, float* __restrict__ c, int mm, int nn, int n, bool in,
+                                         int kq, const F32Fold& fa) {
+  float sq = 0.f;
+  if (in) {
+    const int left = n - nn;
+    if (fa.add) v += before;
+    put_four(c + (size_t)mm * n + nn, v, left, fa.wide);
+    if (fa.gain) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i < left) sq = fmaf(v[i], v[i], sq);
+      put_four(fa.gained + (size_t)mm * n + nn, v * gain, left, fa.wide);
+    }
+  }
+  if (!fa.gain) return;
+  sq += __shfl_xor(sq, 16, RB_WAVE);
+  if (in && kq % 2 == 0) fa.squares_out[(size_t)mm * ((n + 7) / 8) + nn / 8] = sq;
+}
+
 // At most 16 tokens and a depth of at most 1,024 that is no multiple of 128 (K a multiple of 4, W as rows): a launch that is
 // little more than its trips to memory.  Fragments as in the kernel below, a stage of 128 depth values per wave and trip, what lies
 // behind K counts as zeros.  Every one of a stage's 32 products has an accumulator of its own, and they meet as a tree: no chain
@@ -165,10 +236,10 @@ __device__ __forceinline__ gf_f32x4_t gated_end(gf_f32x4_t sum, float* __restric
 // GATED: W is the gate's n rows and then n rows of the way up (n % 16 == 0), c [m, n] = silu(gate) up.  Twice the waves: the first half takes a tile of the
 // gate, the other half the same rows of the way up, whose sums go to the first through LDS (gated_end).  The launch of 1 to 128 workgroups that
 // did this behind the product cost a step 2 us; every sum and the gate are as they are in two launches.
-template <bool GATED>
+template <bool GATED, bool FOLD = false>
 __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ c,
-                                                            int m, int n, int k) {
-  extern __shared__ float lds[];      // [waves - 1][4][64] for each of gate and way up, then, gated, [4][64]
+                                                            int m, int n, int k, const F32Fold fa) {
+  extern __shared__ float lds[];      // [waves - 1][4][64] for each of gate and way up, then, gated, [4][64], then, folded, [waves][16] for each
   const int lane = threadIdx.x & 63, n_waves = (blockDim.x >> 6) / (GATED ? 2 : 1);
   const int up = GATED && (int)(threadIdx.x >> 6) >= n_waves ? 1 : 0, wave = (threadIdx.x >> 6) - up * n_waves;
   float* red = lds + up * (n_waves - 1) * 256;
@@ -177,8 +248,20 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const
   if (up) w += (size_t)n * k;
   // rows beyond N and tokens beyond M: row 0 and token 0, never stored
   const float* wrow = w + (size_t)(n0 + r < n ? n0 + r : 0) * k + 4 * kq;
-  const float* xrow = x + (size_t)(r < m ? r : 0) * k + 4 * kq;
+  int from = r < m ? r : 0;
+  if (FOLD && fa.rows) from = fa.rows[from];
+  const float* xrow = x + (size_t)from * k + 4 * kq;
   const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  float* sq_lds = lds + (GATED ? 2 : 1) * (n_waves - 1) * 256 + (GATED ? 256 : 0) + up * n_waves * 16;
+  SquaresShare<F32_SQ_WIDE> asked;
+  gf_f32x4_t before = zero, gain = zero;
+  const int nn = n0 + 4 * kq;
+  const bool mine = r < m && nn < n;
+  if (FOLD) {
+    if (fa.squares_in) asked = squares_ask<F32_SQ_WIDE>(fa.squares_in + (size_t)from * ((k + 7) / 8), (k + 7) / 8, wave * 4 + kq, n_waves * 4);
+    if (wave == 0 && mine && fa.add) before = four_of(c + (size_t)r * n + nn, n - nn, fa.wide);
+    if (wave == 0 && mine && fa.gain) gain = four_of(fa.gain + nn, n - nn, fa.wide);
+  }
   gf_f32x4_t acc[8][4];
 #pragma unroll
   for (int j = 0; j < 8; ++j)
@@ -200,6 +283,8 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j][0] = (acc[j][0] + acc[j][1]) + (acc[j][2] + acc[j][3]);
   gf_f32x4_t sum = ((acc[0][0] + acc[1][0]) + (acc[2][0] + acc[3][0])) + ((acc[4][0] + acc[5][0]) + (acc[6][0] + acc[7][0]));
+  float ss = 0.f;
+  if (FOLD && fa.squares_in) ss = squares_meet(squares_sum(asked), sq_lds, wave, lane);
   if (n_waves > 1) {
     if (wave > 0)
 #pragma unroll
@@ -211,9 +296,14 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const
 #pragma unroll
         for (int i = 0; i < 4; ++i) sum[i] += red[((o - 1) * 4 + i) * 64 + lane];
   }
+  if (FOLD && fa.squares_in && wave == 0) sum *= squares_factor(ss, sq_lds, n_waves, lane, k, fa.eps);
   if (GATED) {
     sum = gated_end(sum, lds + 2 * (n_waves - 1) * 256, lane, wave == 0 ? up : -1);
     if (wave > 0 || up) return;
+  }
+  if (FOLD && !GATED) {
+    fold_end(sum, before, gain, c, r, nn, n, mine, kq, fa);
+    return;
   }
   // lane l holds rows 4 (l / 16) + i of token l % 16
   if (r < m)
@@ -229,10 +319,12 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const
 // two sets of registers they are under way meanwhile.  Where workgroups share a compute unit they do that for each other, and a wave
 // with more registers is slower (5,120 rows at K = 3072, 4 tokens: 14.9 us with one set, 15.9 with two).
 // GATED: as in the kernel above.
-template <int MB, int R, bool WF, int XP = 1, int WP = 1, int U = 1, bool GATED = false>
+// FOLD: see F32Fold.
+template <int MB, int R, bool WF, int XP = 1, int WP = 1, int U = 1, bool GATED = false, bool FOLD = false>
 __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                          float* __restrict__ c, int m, int n, int k) {
-  extern __shared__ float lds[];      // [waves - 1][R * MB * 4][64] (for each of gate and way up, then [4][64])
+                                                          float* __restrict__ c, int m, int n, int k, const F32Fold fa) {
+  extern __shared__ float lds[];      // [waves - 1][R * MB * 4][64] (for each of gate and way up, then [4][64]), then, folded, [waves][16] (for each)
+  static_assert(!FOLD || (MB == 1 && R == 1), "folded: one tile of tokens and of rows");
   static_assert(!GATED || (MB == 1 && R == 1 && WP == 1), "gated: one tile of tokens, one of gate rows");
   constexpr int ACC = R * MB * 4;
   const int lane = threadIdx.x & 63, n_waves = (blockDim.x >> 6) / (GATED ? 2 : 1);
@@ -265,7 +357,23 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const f
 #pragma unroll
   for (int cb = 0; cb < MB; ++cb) {
     const int row = 16 * cb + r % (16 / XP);
-    xrow[cb] = x + (size_t)(row < m ? row : 0) * k + 16 * (r / (16 / XP)) + 4 * kq;
+    int from = row < m ? row : 0;
+    if (FOLD && fa.rows) from = fa.rows[from];
+    xrow[cb] = x + (size_t)from * k + 16 * (r / (16 / XP)) + 4 * kq;
+  }
+  float* sq_lds = lds + (GATED ? 2 : 1) * (n_waves - 1) * ACC * 64 + (GATED ? 256 : 0) + up * n_waves * 16;
+  SquaresShare<F32_SQ_WIDE> asked;
+  gf_f32x4_t before = {0.f, 0.f, 0.f, 0.f}, gain = before;
+  const int nn_own = n0 + part0 + 4 * kq;
+  const bool mine = r < m && nn_own < n && kq < 4 / WP;
+  if (FOLD) {
+    if (fa.squares_in) {
+      int from = r < m ? r : 0;
+      if (fa.rows) from = fa.rows[from];
+      asked = squares_ask<F32_SQ_WIDE>(fa.squares_in + (size_t)from * ((k + 7) / 8), (k + 7) / 8, wave * 4 + kq, n_waves * 4);
+    }
+    if (wave == 0 && mine && fa.add) before = four_of(c + (size_t)r * n + nn_own, n - nn_own, fa.wide);
+    if (wave == 0 && mine && fa.gain) gain = four_of(fa.gain + nn_own, n - nn_own, fa.wide);
   }
   // the K / 128 stages dealt to the waves as evenly as they go (the host launches no more waves than stages)
   const int total = k / 128, base = total / n_waves, extra = total % n_waves;
@@ -307,6 +415,11 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const f
     }
   };
   load_stage(0, 0);
+  float ss = 0.f;
+  if (FOLD) {                          // the squares were asked for before the first stage and are added up before it arrives
+    __builtin_amdgcn_sched_barrier(0);
+    if (fa.squares_in) ss = squares_sum(asked);
+  }
   if constexpr (U == 2) {
     int st = 0;
     for (; st + 2 < stages; st += 2) {
@@ -333,6 +446,7 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const f
     multiply_stage(0);
   }
 
+  if (FOLD && fa.squares_in) ss = squares_meet(ss, sq_lds, wave, lane);
   if (n_waves > 1) {
     if (wave > 0) {
       float* dst = red + (size_t)(wave - 1) * ACC * 64 + lane;
@@ -355,12 +469,17 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const f
           for (int i = 0; i < 4; ++i) acc[rt][cb][i] += src[((rt * MB + cb) * 4 + i) * 64];
     }
   }
+  if (FOLD && fa.squares_in && wave == 0) acc[0][0] *= squares_factor(ss, sq_lds, n_waves, lane, k, fa.eps);
   if constexpr (GATED) {
     acc[0][0] = gated_end(acc[0][0], lds + 2 * (n_waves - 1) * ACC * 64, lane, wave == 0 ? up : -1);
     if (wave > 0 || up) return;
   }
   // lane l holds, for token 16 cb + l % 16, the rows n0 + 16 rt + 4 (l / 16) + i
   if (WP > 1 && kq >= 4 / WP) return;
+  if (FOLD && !GATED) {
+    fold_end(acc[0][0], before, gain, c, r, nn_own, n, mine, kq, fa);
+    return;
+  }
 #pragma unroll
   for (int rt = 0; rt < R; ++rt)
 #pragma unroll
@@ -391,6 +510,47 @@ static bool f32_short_takes(int m, int n, int k) {
   return m <= 16 && k % 4 == 0 && k <= 1024 && (k <= 128 || m > 8 || (long long)n * k <= 1 << 22) && g_f32_few;
 }
 
+// At most 16 tokens: one tile of them
+template <bool FOLD>
+static void launch_f32_16(const float* x, const float* w, bool w_frag, float* c, int m, int n, int k, const F32Fold& fa, hipStream_t s) {
+  const int n_waves = f32_few_waves(k), grid = (n + 15) / 16;
+  const size_t lds = ((size_t)(n_waves - 1) * 256 + (FOLD ? n_waves * 16 : 0)) * sizeof(float);
+  // us, 4 tokens, as the kernel was (one stage, a block a load, whole tiles) and so: 3,072 rows at K = 3072 9.75 and 8.8, at 8192 24.3 and 21.3; 2,048 at 2048
+  // 7.2 and 5.9, 1,024 at 4096 10.8 and 8.3 (halves of tiles); more workgroups than compute units: 5,120 at 3072 17.4 and 14.9, 16,384 38.0 and 35.0,
+  // 128,256 260 and 239, 6,144 at 4096 23.4 and 20.7.  Halves of more tiles than half the units lose (3,072 rows at 3072 11.9).
+  if (w_frag) {
+    const int cus = rb_compute_units(), parts = g_f32_parts ? g_f32_parts : 2 * grid <= cus ? 2 : 1, pack = m <= 4 ? 4 : m <= 8 ? 2 : 1;
+    auto by = [&](auto four, auto two, auto one) { return pack == 4 ? four : pack == 2 ? two : one; };
+    (parts == 2    ? by(gemm_f32_few_kernel<1, 1, true, 4, 2, 2, false, FOLD>, gemm_f32_few_kernel<1, 1, true, 2, 2, 2, false, FOLD>,
+                        gemm_f32_few_kernel<1, 1, true, 1, 2, 2, false, FOLD>)
+     : grid <= cus ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2, false, FOLD>      // (packed tokens: 4,096 rows at K = 4096 14.2 for 13.9, the others the same)
+                   : by(gemm_f32_few_kernel<1, 1, true, 4, 1, 1, false, FOLD>, gemm_f32_few_kernel<1, 1, true, 2, 1, 1, false, FOLD>,
+                        gemm_f32_few_kernel<1, 1, true, 1, 1, 1, false, FOLD>))<<<parts * grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, fa);
+    return;
+  }
+  gemm_f32_few_kernel<1, 1, false, 1, 1, 1, false, FOLD><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, fa);
+}
+
+template <bool FOLD>
+static void launch_f32_short(const float* x, const float* w, float* c, int m, int n, int k, const F32Fold& fa, hipStream_t s) {
+  const int n_waves = f32_short_waves(k);
+  const size_t lds = ((size_t)(n_waves - 1) * 256 + (FOLD ? n_waves * 16 : 0)) * sizeof(float);
+  gemm_f32_short_kernel<false, FOLD><<<(n + 15) / 16, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, fa);
+}
+
+// gate and way up, and the gate (rb_gemm_f32_gated_ok)
+template <bool FOLD>
+static void launch_f32_gated(const float* x, const float* w, bool w_frag, float* c, int m, int ff, int k, const F32Fold& fa, hipStream_t s) {
+  const int grid = ff / 16, n_waves = w_frag ? f32_few_waves(k) : f32_short_waves(k);
+  const size_t lds = ((size_t)2 * (n_waves - 1) * 256 + 256 + (FOLD ? 2 * n_waves * 16 : 0)) * sizeof(float);
+  auto kern = !w_frag                          ? gemm_f32_short_kernel<true, FOLD>
+              : 2 * grid <= rb_compute_units() ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2, true, FOLD>      // (8 waves a workgroup: as two workgroups above)
+              : m <= 4                         ? gemm_f32_few_kernel<1, 1, true, 4, 1, 1, true, FOLD>
+              : m <= 8                         ? gemm_f32_few_kernel<1, 1, true, 2, 1, 1, true, FOLD>
+                                               : gemm_f32_few_kernel<1, 1, true, 1, 1, 1, true, FOLD>;
+  kern<<<grid, 2 * 64 * n_waves, lds, s>>>(x, w, c, m, ff, k, fa);
+}
+
 template <int MB>
 static void launch_f32_few(const float* x, const float* w, bool w_frag, float* c, int m, int n, int k, hipStream_t s) {
   const int n_waves = f32_few_waves(k);
@@ -403,29 +563,15 @@ static void launch_f32_few(const float* x, const float* w, bool w_frag, float* c
     if (g_f32_few != 3 && (n + 31) / 32 >= 2 * rb_compute_units()) {
       const size_t lds2 = (size_t)(n_waves - 1) * 2 * MB * 4 * 64 * sizeof(float);
       const int grid2 = (n + 31) / 32;
-      if (w_frag) gemm_f32_few_kernel<MB, 2, true><<<grid2, 64 * n_waves, lds2, s>>>(x, w, c, m, n, k);
-      else gemm_f32_few_kernel<MB, 2, false><<<grid2, 64 * n_waves, lds2, s>>>(x, w, c, m, n, k);
+      if (w_frag) gemm_f32_few_kernel<MB, 2, true><<<grid2, 64 * n_waves, lds2, s>>>(x, w, c, m, n, k, F32Fold{});
+      else gemm_f32_few_kernel<MB, 2, false><<<grid2, 64 * n_waves, lds2, s>>>(x, w, c, m, n, k, F32Fold{});
       return;
     }
   }
   const size_t lds = (size_t)(n_waves - 1) * MB * 4 * 64 * sizeof(float);
   const int grid = (n + 15) / 16;
-  if constexpr (MB == 1) {
-    // us, 4 tokens, as the kernel was (one stage, a block a load, whole tiles) and so: 3,072 rows at K = 3072 9.75 and 8.8, at 8192 24.3 and 21.3; 2,048 at 2048
-    // 7.2 and 5.9, 1,024 at 4096 10.8 and 8.3 (halves of tiles); more workgroups than compute units: 5,120 at 3072 17.4 and 14.9, 16,384 38.0 and 35.0,
-    // 128,256 260 and 239, 6,144 at 4096 23.4 and 20.7.  Halves of more tiles than half the units lose (3,072 rows at 3072 11.9).
-    if (w_frag) {
-      const int cus = rb_compute_units(), parts = g_f32_parts ? g_f32_parts : 2 * grid <= cus ? 2 : 1, pack = m <= 4 ? 4 : m <= 8 ? 2 : 1;
-      auto by = [&](auto four, auto two, auto one) { return pack == 4 ? four : pack == 2 ? two : one; };
-      (parts == 2    ? by(gemm_f32_few_kernel<1, 1, true, 4, 2, 2>, gemm_f32_few_kernel<1, 1, true, 2, 2, 2>, gemm_f32_few_kernel<1, 1, true, 1, 2, 2>)
-       : grid <= cus ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2>      // (packed tokens: 4,096 rows at K = 4096 14.2 for 13.9, the others the same)
-                     : by(gemm_f32_few_kernel<1, 1, true, 4>, gemm_f32_few_kernel<1, 1, true, 2>, gemm_f32_few_kernel<1, 1, true>))<<<
-          parts * grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
-      return;
-    }
-  }
-  if (w_frag) gemm_f32_few_kernel<MB, 1, true><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
-  else gemm_f32_few_kernel<MB, 1, false><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
+  if (w_frag) gemm_f32_few_kernel<MB, 1, true><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, F32Fold{});
+  else gemm_f32_few_kernel<MB, 1, false><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, F32Fold{});
 }
 
 // Float32 operands and more than 16 tokens with K a multiple of 16 that is not one of 32, or operands
@@ -557,15 +703,33 @@ extern "C" int rb_gemm_f32_gated(const float* a, const float* w, int w_layout, f
   RB_RECORDED(rb_gemm_f32_gated(a, w, w_layout, c, m, ff, k, stream));
   RB_REQUIRE(m == 0 || rb_gemm_f32_gated_ok(m, ff, k, w_layout), "rb_gemm_f32_gated: M=%d ff=%d K=%d, layout %d are not for it", m, ff, k, w_layout);
   if (m == 0) return 0;
+  launch_f32_gated<false>(a, w, w_layout == 1, c, m, ff, k, F32Fold{}, (hipStream_t)stream);
+  RB_LAUNCH_CHECK();
+  return 0;
+}
+
+// Whether a product of 1..16 float32 tokens takes its neighbours along (epilogue as in rb_gemm_f32_few): the sizes of the two kernels for few tokens.
+extern "C" int rb_gemm_f32_few_ok(int m, int n, int k, int w_layout, int epilogue) {
+  if (m < 1 || m > 16 || n < 1 || k < 4 || epilogue < 0 || epilogue > 3 || !g_f32_few) return 0;
+  if (epilogue == 1) return n % 2 == 0 && rb_gemm_f32_gated_ok(m, n / 2, k, w_layout);
+  if (w_layout == 1) return n % 16 == 0 && k % 128 == 0;
+  return w_layout == 0 && (k % 128 == 0 || f32_short_takes(m, n, k));
+}
+
+extern "C" int rb_gemm_f32_few(const float* a, const float* squares_in, float eps, const int32_t* rows, const float* w, int w_layout, float* c,
+                               int epilogue, const float* gain, float* gained, float* squares_out, int m, int n, int k, void* stream) {
+  RB_RECORDED(rb_gemm_f32_few(a, squares_in, eps, rows, w, w_layout, c, epilogue, gain, gained, squares_out, m, n, k, stream));
+  RB_REQUIRE(rb_gemm_f32_few_ok(m, n, k, w_layout, epilogue), "rb_gemm_f32_few: M=%d N=%d K=%d, layout %d, epilogue %d are not for it", m, n, k,
+             w_layout, epilogue);
+  RB_REQUIRE(!squares_in || epilogue <= 1, "rb_gemm_f32_few: prepared rows go with epilogues 0 and 1, not %d", epilogue);
+  RB_REQUIRE(epilogue != 3 || (gain && gained && squares_out), "rb_gemm_f32_few: epilogue 3 needs the gain and room for the prepared rows");
+  if (epilogue != 3) gain = nullptr, gained = squares_out = nullptr;
+  const uintptr_t all = reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(gain) | reinterpret_cast<uintptr_t>(gained);
+  const F32Fold fa = {squares_in, rows, eps, epilogue >= 2 ? 1 : 0, gain, gained, squares_out, n % 4 == 0 && (all & 15) == 0 ? 1 : 0};
   hipStream_t s = (hipStream_t)stream;
-  const int grid = ff / 16, n_waves = w_layout ? f32_few_waves(k) : f32_short_waves(k);
-  const size_t lds = ((size_t)2 * (n_waves - 1) * 256 + 256) * sizeof(float);
-  auto kern = !w_layout                        ? gemm_f32_short_kernel<true>
-              : 2 * grid <= rb_compute_units() ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2, true>      // (8 waves a workgroup: as two workgroups above)
-              : m <= 4                         ? gemm_f32_few_kernel<1, 1, true, 4, 1, 1, true>
-              : m <= 8                         ? gemm_f32_few_kernel<1, 1, true, 2, 1, 1, true>
-                                               : gemm_f32_few_kernel<1, 1, true, 1, 1, 1, true>;
-  kern<<<grid, 2 * 64 * n_waves, lds, s>>>(a, w, c, m, ff, k);
+  if (epilogue == 1) launch_f32_gated<true>(a, w, w_layout == 1, c, m, n / 2, k, fa, s);
+  else if (k % 128 == 0) launch_f32_16<true>(a, w, w_layout == 1, c, m, n, k, fa, s);
+  else launch_f32_short<true>(a, w, c, m, n, k, fa, s);
   RB_LAUNCH_CHECK();
   return 0;
 }
@@ -585,16 +749,14 @@ extern "C" int rb_gemm_generic(const void* a, const void* w, int w_layout, void*
     const float* af = (const float*)a;
     const float* wf = (const float*)w;
     const int mb = (m + 15) / 16;
-    if (mb == 1) launch_f32_few<1>(af, wf, w_frag, (float*)c, m, n, k, s);
+    if (mb == 1) launch_f32_16<false>(af, wf, w_frag, (float*)c, m, n, k, F32Fold{}, s);
     else if (mb == 2) launch_f32_few<2>(af, wf, w_frag, (float*)c, m, n, k, s);
     else launch_f32_few<4>(af, wf, w_frag, (float*)c, m, n, k, s);
     RB_LAUNCH_CHECK();
     return 0;
   }
   if (dtype_in == RB_F32 && dtype_out == RB_F32 && f32_short_takes(m, n, k)) {
-    const int n_waves = f32_short_waves(k);
-    gemm_f32_short_kernel<false><<<(n + 15) / 16, 64 * n_waves, (size_t)(n_waves - 1) * 4 * 64 * sizeof(float), s>>>((const float*)a, (const float*)w,
-                                                                                                     (float*)c, m, n, k);
+    launch_f32_short<false>((const float*)a, (const float*)w, (float*)c, m, n, k, F32Fold{}, s);
     RB_LAUNCH_CHECK();
     return 0;
   }

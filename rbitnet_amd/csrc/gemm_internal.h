@@ -71,6 +71,42 @@ struct RowPack {
   }
 };
 
+// A lane's share of a row's n_sq sums of squares: `share` of `shares` (4 lanes of every wave work
+// on one row).  With n_sq a multiple of 4 the first 16 * shares * SQ_WIDE of them are asked for
+// with 16-byte loads that are all in flight together, and added up by squares_sum() when they
+// are needed; the rest, if any, one by one.
+template <int SQ_WIDE = 4>
+struct SquaresShare {
+  float4 wide[SQ_WIDE];
+  float rest;
+};
+template <int SQ_WIDE = 4>
+__device__ __forceinline__ SquaresShare<SQ_WIDE> squares_ask(const float* __restrict__ sq, int n_sq, int share, int shares) {
+  SquaresShare<SQ_WIDE> out;
+  out.rest = 0.f;
+  int done = 0;
+  if (n_sq % 4 == 0) {
+#pragma unroll
+    for (int j = 0; j < SQ_WIDE; ++j) {
+      const int at = 4 * (share + j * shares);
+      out.wide[j] = at < n_sq ? *reinterpret_cast<const float4*>(sq + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    done = 4 * shares * SQ_WIDE;
+  } else {
+#pragma unroll
+    for (int j = 0; j < SQ_WIDE; ++j) out.wide[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  for (int i = done + share; i < n_sq; i += shares) out.rest += sq[i];
+  return out;
+}
+template <int SQ_WIDE>
+__device__ __forceinline__ float squares_sum(const SquaresShare<SQ_WIDE>& s) {
+  float t = s.rest;
+#pragma unroll
+  for (int j = 0; j < SQ_WIDE; ++j) t += (s.wide[j].x + s.wide[j].y) + (s.wide[j].z + s.wide[j].w);
+  return t;
+}
+
 // at most 64 tokens, any K % 8 == 0: W streamed straight into MFMA operands (gemm_skinny.hip);
 // prepared tokens and epilogues 2 and 3: at most 16 tokens
 int gemm_skinny_launch(const GemmTokens& x, const bf16_t* w, void* c, int dtype_out, const GemmAfter& after, int m,

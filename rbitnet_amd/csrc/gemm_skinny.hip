@@ -90,40 +90,6 @@ __device__ __forceinline__ void store_sums(TO* __restrict__ c, const f32x4_t& su
   }
 }
 
-// A lane's share of a row's n_sq sums of squares: `share` of `shares` (4 lanes of every wave work
-// on one row).  With n_sq a multiple of 4 the first 16 * shares * SQ_WIDE of them are asked for
-// with 16-byte loads that are all in flight together, and added up by squares_sum() when they
-// are needed; the rest, if any, one by one.
-constexpr int SQ_WIDE = 4;
-struct SquaresShare {
-  float4 wide[SQ_WIDE];
-  float rest;
-};
-__device__ __forceinline__ SquaresShare squares_ask(const float* __restrict__ sq, int n_sq, int share, int shares) {
-  SquaresShare out;
-  out.rest = 0.f;
-  int done = 0;
-  if (n_sq % 4 == 0) {
-#pragma unroll
-    for (int j = 0; j < SQ_WIDE; ++j) {
-      const int at = 4 * (share + j * shares);
-      out.wide[j] = at < n_sq ? *reinterpret_cast<const float4*>(sq + at) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    done = 4 * shares * SQ_WIDE;
-  } else {
-#pragma unroll
-    for (int j = 0; j < SQ_WIDE; ++j) out.wide[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  for (int i = done + share; i < n_sq; i += shares) out.rest += sq[i];
-  return out;
-}
-__device__ __forceinline__ float squares_sum(const SquaresShare& s) {
-  float t = s.rest;
-#pragma unroll
-  for (int j = 0; j < SQ_WIDE; ++j) t += (s.wide[j].x + s.wide[j].y) + (s.wide[j].z + s.wide[j].w);
-  return t;
-}
-
 // FAST: K % 128 == 0, the K / 128 stages of 128 depth values dealt to the waves as evenly as they go, one stage in flight while the one
 // before is multiplied; else any K % 8 == 0, with bounds checks.  WF (up to 16 tokens): W is stored fragment-major.
 // (All of a wave's stages asked for at once instead, W's first, for up to four stages a wave: no faster at K = 128 to 4096 with any
@@ -183,7 +149,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
   const bf16_t* xrow[MB];
   bool xok[MB];
   float ss[MB];
-  SquaresShare asked[MB];
+  SquaresShare<> asked[MB];
 #pragma unroll
   for (int cb = 0; cb < MB; ++cb) {
     const int row = 16 * cb + r;

@@ -105,7 +105,7 @@ class KernelTimes:
         return "\n".join(lines)
 
 
-TIMED_OPS = ("gemm_f32_gated", "heads_combined", "routed_experts_tiled", "recurrence_step", "gemm_bf16_group", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
+TIMED_OPS = ("gemm_f32_few", "gemm_f32_gated", "heads_combined", "routed_experts_tiled", "recurrence_step", "gemm_bf16_group", "route_linear", "selective_chunks", "embed_streams_waves", "streams_rmsnorm", "selective_scan", "gate_rmsnorm_parts", "tanh_norm", "heads_prepare", "lightning_recurrence", "lightning_chunks", "gated_rmsnorm_rows", "short_conv_bias", "decay_exp_exp", "gated_rmsnorm_heads", "outnorm_residual", "clamped_glu", "tanh_cast", "attention_opts", "norm_rope_store", "sigmoid_gate", "shift_mix", "time_mix_recurrence", "latent_norm_rope_store", "heads_linear_part", "route_choose", "experts_combine", "embed_scaled_pos", "scale", "bias_norm_store", "attention_mixed", "attention_mixed_bf16", "recurrence_prep", "linear_recurrence", "layernorm_residual", "rope_store", "head_gate", "pair_norm_mean",
              "route_top", "routed_experts", "pairs_sum", "embed_streams", "streams_layernorm", "streams_update", "xielu", "tanh_cap", "short_conv",
              "delta_prep", "delta_rule", "gated_rmsnorm", "latent_norm_store", "attention_sinks", "embed_gather", "add_rmsnorm", "rope_kv_write", "swiglu", "gemm_generic", "gemm_bf16", "gemm_bf16_terms",
              "gemm_bf16_few", "attention_generic", "attention_prefill_bf16", "attention_decode_bf16",
@@ -163,6 +163,8 @@ class Kernels:
             "rb_gemm_bf16_act": [_P, _P, _I, _P, _I, _I, _P, _I, _I, _I, _P, _P],
             "rb_gemm_bf16_few": [_P, _P, _F, _P, _P, _I, _P, _I, _I, _P, _P, _P, _I, _I, _I, _P],
             "rb_gemm_bf16_few_ok": [_I, _I, _I],
+            "rb_gemm_f32_few_ok": [_I, _I, _I, _I, _I],
+            "rb_gemm_f32_few": [_P, _P, _F, _P, _P, _I, _P, _I, _P, _P, _P, _I, _I, _I, _P],
             "rb_gemm_bf16_terms_count": [_I, _I, _I],
             "rb_gemm_bf16_terms": [_P, _P, _I, _P, _I, _I, _I, _P],
             "rb_attention_generic": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P],
@@ -383,6 +385,32 @@ class Kernels:
         _check(w, "w", torch.float32, (2 * ff, k))
         _check(c, "c", torch.float32, (m, ff))
         self._ok(self._lib.rb_gemm_f32_gated(_ptr(a), _ptr(w), int(bool(w_frag)), _ptr(c), m, ff, k, self._stream()))
+
+    def gemm_f32_few_ok(self, m: int, n: int, k: int, w_frag: bool, epilogue: int) -> bool:
+        return bool(self._lib.rb_gemm_f32_few_ok(int(m), int(n), int(k), int(bool(w_frag)), int(epilogue)))
+
+    def gemm_f32_few(self, a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, epilogue: int = 0, squares: Optional[torch.Tensor] = None,
+                     eps: float = 0.0, rows: Optional[torch.Tensor] = None, gain: Optional[torch.Tensor] = None,
+                     gained: Optional[torch.Tensor] = None, squares_out: Optional[torch.Tensor] = None, w_frag: bool = False) -> None:
+        """`gemm_bf16_few` in float32 (sizes that `gemm_f32_few_ok`): sums of squares over every 8 columns, gained rows in float32, and for
+        epilogue 1 w as for `gemm_f32_gated`."""
+        n, k = w.shape
+        _check(a, "a", torch.float32)
+        if a.dim() != 2 or a.shape[1] != k:
+            raise KernelError(f"a must have rows of {k} values, found {tuple(a.shape)}")
+        m = a.shape[0] if rows is None else rows.shape[0]
+        if rows is not None:
+            _check(rows, "rows", torch.int32, (m,))
+        if squares is not None:
+            _check(squares, "squares", torch.float32, (a.shape[0], (k + 7) // 8))
+        _check(w, "w", torch.float32, (n, k))
+        _check(c, "c", torch.float32, (m, n // 2 if epilogue == 1 else n))
+        if epilogue == 3:
+            _check(gain, "gain", torch.float32, (n,))
+            _check(gained, "gained", torch.float32, (m, n))
+            _check(squares_out, "squares_out", torch.float32, (m, (n + 7) // 8))
+        self._ok(self._lib.rb_gemm_f32_few(_ptr(a), _ptr(squares), float(eps), _ptr(rows), _ptr(w), int(bool(w_frag)), _ptr(c), int(epilogue),
+                                           _ptr(gain), _ptr(gained), _ptr(squares_out), m, n, k, self._stream()))
 
     def gemm_bf16(self, a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, epilogue: int = 0,
                   w_frag: bool = False, act: Optional[torch.Tensor] = None) -> None:

@@ -66,15 +66,23 @@ def uses_matrix_cores(dtype: torch.dtype, k: int) -> bool:
 FOLD_INTO_PRODUCTS = True
 
 
-def _few(lib, x, w) -> bool:
+def _few(lib, x, w, epilogue: int = 0) -> bool:
     """Whether the kernel for a few tokens, which folds its neighbours in, takes this product."""
     m, k = x.shape
-    return FOLD_INTO_PRODUCTS and uses_matrix_cores(x.dtype, k) and lib.gemm_bf16_few_ok(m, w.shape[0], k)
+    if not FOLD_INTO_PRODUCTS:
+        return False
+    if x.dtype == torch.float32:
+        return lib.gemm_f32_few_ok(m, w.shape[0], k, _data(w)[1], epilogue)
+    return uses_matrix_cores(x.dtype, k) and lib.gemm_bf16_few_ok(m, w.shape[0], k)
+
+
+def _few_product(lib, dtype: torch.dtype):
+    return lib.gemm_f32_few if dtype == torch.float32 else lib.gemm_bf16_few
 
 
 def _from_gained(lib, x: GainedRows, w, out: torch.Tensor, epilogue: int) -> None:
     wd, frag = _data(w)
-    lib.gemm_bf16_few(x.gained, wd, out, epilogue, squares=x.squares, eps=x.eps, rows=x.rows, w_frag=frag)
+    _few_product(lib, x.dtype)(x.gained, wd, out, epilogue, squares=x.squares, eps=x.eps, rows=x.rows, w_frag=frag)
 
 
 def linear(lib, x, w, out_dtype: torch.dtype) -> torch.Tensor:
@@ -85,7 +93,7 @@ def linear(lib, x, w, out_dtype: torch.dtype) -> torch.Tensor:
     if m == 0:
         return out
     if isinstance(x, GainedRows):
-        if _few(lib, x, w):
+        if _few(lib, x, w) and (x.dtype != torch.float32 or out_dtype == torch.float32):
             _from_gained(lib, x, w, out, 0)
             return out
         x = x.tensor()
@@ -146,19 +154,20 @@ def linear_to_stream(lib, x: torch.Tensor, w, stream: Optional[torch.Tensor], ne
     the product is added, and what comes back is None, or, if the norm that follows folds into
     products, the `GainedRows` for it."""
     wd, frag = _data(w)
-    if stream is None or x.shape[0] == 0 or not _few(lib, x, w):
+    if stream is None or x.shape[0] == 0 or not _few(lib, x, w, 2):
         m, k = x.shape
         if (norm_adds_terms(next_norm) and uses_matrix_cores(x.dtype, k)
                 and lib.gemm_bf16_terms_count(m, w.shape[0], k) > 1):
             return lib.gemm_bf16_terms(x, wd, w_frag=frag)        # [P, M, N]: the norm adds them up with the stream
         return linear(lib, x, w, torch.float32)
     if not norm_folds(next_norm):
-        lib.gemm_bf16_few(x, wd, stream, 2, w_frag=frag)
+        _few_product(lib, x.dtype)(x, wd, stream, 2, w_frag=frag)
         return None
     m, n = stream.shape
-    gained = torch.empty((m, n), dtype=torch.bfloat16, device=stream.device)
-    squares = torch.empty((m, (n + 15) // 16), dtype=torch.float32, device=stream.device)
-    lib.gemm_bf16_few(x, wd, stream, 3, gain=next_norm.weight, gained=gained, squares_out=squares, w_frag=frag)
+    gained = torch.empty((m, n), dtype=x.dtype, device=stream.device)
+    over = 8 if x.dtype == torch.float32 else 16          # columns of a sum of squares
+    squares = torch.empty((m, (n + over - 1) // over), dtype=torch.float32, device=stream.device)
+    _few_product(lib, x.dtype)(x, wd, stream, 3, gain=next_norm.weight, gained=gained, squares_out=squares, w_frag=frag)
     return GainedRows(next_norm, stream, gained, squares)
 
 
@@ -204,7 +213,7 @@ def gated_linear(lib, x, w_packed, ff: int, fused: bool, gate: Optional[torch.Te
     if m == 0:
         return out
     if isinstance(x, GainedRows):
-        if fused and _few(lib, x, w_packed):
+        if _few(lib, x, w_packed, 1) and (fused or x.dtype == torch.float32):
             _from_gained(lib, x, w_packed, out, 1)
             return out
         x = x.tensor()

@@ -14,7 +14,7 @@ Interface of a norm: forward(x, delta=None, rows=None) -> h
 
 A norm that says `folds_into_products` (with weight, eps and size as here) lets the product
 before it and the product after it do its work when a step has few tokens: the first, which
-adds to the stream, also leaves bf16(x * gain) and the sums of x^2 (`GainedRows`); the second
+adds to the stream, also leaves x * gain and the sums of x^2 (`GainedRows`); the second
 takes these as its tokens and multiplies its result by 1 / sqrt(mean(x^2) + eps).
 """
 from __future__ import annotations

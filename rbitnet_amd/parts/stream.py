@@ -58,8 +58,8 @@ import torch
 
 class GainedRows:
     """Rows of the float32 stream `x` (all, or those `rows` names) as a product left them for
-    `norm`: gained [T, E] = bf16(x * gain) and squares [T, ceil(E / 16)], the sums of x^2 over
-    every 16 columns.  What is left of the norm is one factor per row.  `linear` takes them as
+    `norm`: gained [T, E] = x * gain in the compute dtype and squares, the sums of x^2 over every 16 columns (in
+    float32 every 8).  What is left of the norm is one factor per row.  `linear` takes them as
     tokens; tensor() normalises the rows with the norm's own kernel instead.  shape, dtype and
     device are those of the normalised rows."""
 

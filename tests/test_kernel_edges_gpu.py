@@ -1667,3 +1667,69 @@ def test_products_in_one_launch_give_the_bits_of_each_alone(lib, m, k, rows):
             z, a = a, torch.empty_like(c)
             lib.tanh_cast(z, a)
         assert torch.equal(c, a.to(c.dtype)), rows[i]
+
+
+# ---------------------------------------------------------------------------- float32 products of few tokens: sums and norms in their launches
+@pytest.mark.parametrize("n,k,frag", [(16, 128, True), (96, 96, False), (257, 96, False), (90, 500, False), (384, 1000, False), (130, 384, False), (2048, 512, True),
+                                      (4096, 768, True), (4112, 1280, True), (3072, 3072, True), (256, 8192, True)])
+def test_float32_products_of_few_tokens_take_sum_and_norm_along(lib, n, k, frag):
+    """Against the same in 64 bits.  A product's error is at most (K + 3) units of 2^-24 of its sum of magnitudes, a random walk of them in fact:
+    2^-24 sqrt(K) times that sum covers it and the few more roundings (residual sum, gain, factor)."""
+    gen = torch.Generator().manual_seed(n + k)
+    rows = torch.randn(n, k, generator=gen) * k ** -0.5
+    w = rows.to(DEV)
+    if frag:
+        w = torch.empty(n, k, device=DEV)
+        lib.place_rows(rows.to(DEV), w, frag=True)
+    unit, eps = 2.0 ** -24 * max(4.0, k ** 0.5), 1e-5
+    nan = float("nan")
+
+    def close(got, want, size):
+        assert torch.isfinite(got).all()
+        assert ((got.double().cpu() - want).abs() <= unit * size).all()
+
+    for m in (1, 4, 5, 8, 9, 16):
+        if not lib.gemm_f32_few_ok(m, n, k, frag, 0):
+            assert not frag and k > 128 and m <= 8           # (many rows of a longer depth: another kernel's)
+            continue
+        x, gain, before = torch.randn(m + 2, k, generator=gen) * 3.0, torch.randn(k, generator=gen), torch.randn(m, n, generator=gen)
+        x[0] *= 1e-4                                         # (a row that eps decides)
+        gained = (x * gain).to(DEV)
+        padded = torch.zeros(m + 2, (k + 7) // 8 * 8)
+        padded[:, :k] = x * x
+        squares = padded.view(m + 2, -1, 8).sum(-1).to(DEV)
+        pick = torch.randperm(m + 2, generator=gen)[:m].to(torch.int32)
+        # rows that a norm prepared, all of the step's or some of them
+        for rows_of, src in ((None, torch.arange(m)), (pick, pick.long())):
+            normed = (x.double() * gain.double() / (x.double().square().mean(-1, keepdim=True) + eps).sqrt())[src]
+            got = torch.full((m, n), nan, device=DEV)
+            a = gained if rows_of is not None else gained[:m].contiguous()
+            lib.gemm_f32_few(a, w, got, 0, squares=squares if rows_of is not None else squares[:m].contiguous(), eps=eps,
+                             rows=None if rows_of is None else rows_of.to(DEV), w_frag=frag)
+            close(got, normed @ rows.double().T, normed.abs() @ rows.double().abs().T)
+        # the residual sum, and what the next norm needs; columns at whole vectors and not
+        g2 = torch.randn(n, generator=gen)
+        want = before.double() + x[:m].double() @ rows.double().T
+        size = before.double().abs() + x[:m].double().abs() @ rows.double().abs().T
+        for off in (0, 1):
+            c = torch.empty(m * n + off, device=DEV)[off:].view(m, n)
+            c.copy_(before)
+            alone = c.clone()
+            out, sq = torch.full((m, n), nan, device=DEV), torch.full((m, (n + 7) // 8), nan, device=DEV)
+            lib.gemm_f32_few(x[:m].contiguous().to(DEV), w, c, 3, gain=g2.to(DEV), gained=out, squares_out=sq, w_frag=frag)
+            close(c, want, size)
+            assert torch.equal(out, c * g2.to(DEV))
+            full = torch.zeros(m, (n + 7) // 8 * 8, dtype=torch.float64)
+            full[:, :n] = c.double().cpu().square()
+            torch.testing.assert_close(sq.double().cpu(), full.view(m, -1, 8).sum(-1), rtol=8 * 2.0 ** -24, atol=0.0)
+            lib.gemm_f32_few(x[:m].contiguous().to(DEV), w, alone, 2, w_frag=frag)
+            assert torch.equal(alone, c)
+        # the gate on prepared rows
+        if n % 32 == 0 and lib.gemm_f32_few_ok(m, n, k, frag, 1):
+            got = torch.full((m, n // 2), nan, device=DEV)
+            normed = x[:m].double() * gain.double() / (x[:m].double().square().mean(-1, keepdim=True) + eps).sqrt()
+            lib.gemm_f32_few(gained[:m].contiguous(), w, got, 1, squares=squares[:m].contiguous(), eps=eps, w_frag=frag)
+            g, u = (normed @ rows.double().T).split(n // 2, dim=1)
+            sg, su = (normed.abs() @ rows.double().abs().T).split(n // 2, dim=1)
+            close(got, g * torch.sigmoid(g) * u, 1.1 * sg * u.abs() + (g.abs() + 1.0) * su)
+    assert not lib.gemm_f32_few_ok(17, n, k, frag, 0) and not lib.gemm_f32_few_ok(4, n, k + 2, frag, 2)
