@@ -587,7 +587,9 @@ __device__ __forceinline__ void walk_ahead(int n_steps, const Load& load, const 
 // W by one wave, which takes the shares of depth of the `waves` that the product alone has one after another and adds up their sums in the
 // same order: the same bits.  Bound by the chosen experts' matrices, which take longer than this wave's walk.  (A captured step of 4 tokens through 15
 // layers of 16 experts of 2,048 and a shared one of 1,024 at width 2,048 took 120 us longer with four launches a layer than with two: 4 us a launch.)
-// XP: blocks of depth that a load of the tokens brings (see RowPack), here and below: an expert's run has no more rows than the step has tokens.
+// XP: blocks of depth that a load of the tokens brings (see RowPack), here and below: a run has at most 16 / XP rows as long as every token chooses an expert
+// once.  A token with fewer scores than choices (infinities or NaN among its logits) chooses one again and again: the rows behind follow in a walk of
+// their own, a block a load.  (As another turn of the same walk it took a wave's registers over 128, and a compute unit had 3 waves a SIMD for 4.)
 struct SharedProduct {
   const bf16_t *x, *w;
   void* c;                   // bfloat16 with act, else float32
@@ -663,6 +665,7 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
   while (nt < NT && t0 + nt < n_tiles && tile_expert[t0 + nt] == e) ++nt;
   const int r = lane & 15, grp = lane >> 4;
   static_assert(XP == 1 || NT == 1, "packed rows: runs of one tile");
+  const int behind = XP == 1 ? -1 : row_pair[t0 * RT_TILE + 16 / XP];
   const bf16_t* xr[NT];
   float wt[NT];
   bool on[NT];
@@ -670,7 +673,7 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
   for (int j = 0; j < NT; ++j) {
     const int at = (t0 + j) * RT_TILE;
     const int p = j < nt ? row_pair[at + RowPack<XP>::row(r)] : -1;      // the row that this lane loads
-    on[j] = XP == 1 ? p >= 0 : row_pair[at + r] >= 0;
+    on[j] = p >= 0 && r < 16 / XP;
     wt[j] = (WEIGHTED && p >= 0) ? weight[p] : 1.0f;
     xr[j] = h + (size_t)(p >= 0 ? p / top : 0) * width + RowPack<XP>::depth(r) + 8 * grp;
   }
@@ -720,6 +723,27 @@ __global__ __launch_bounds__(RB_WAVE) void routed_up_few_kernel(const bf16_t* __
         make_uint2(pack_bf16x2(expert_unit<GATED>(g[0], u[0], limit, alpha), expert_unit<GATED>(g[1], u[1], limit, alpha)),
                    pack_bf16x2(expert_unit<GATED>(g[2], u[2], limit, alpha), expert_unit<GATED>(g[3], u[3], limit, alpha)));
   }
+  if (behind < 0) return;
+  const int p = row_pair[t0 * RT_TILE + r], c = c0 + 4 * grp;
+  const float scale = WEIGHTED && p >= 0 ? weight[p] : 1.0f;
+  const bf16_t* xb = h + (size_t)(p >= 0 ? p / top : 0) * width + 8 * grp;
+  f32x4_t g = {0.f, 0.f, 0.f, 0.f}, u = g;
+#pragma unroll 1
+  for (int s = 0; s < n_steps; ++s) {
+    Frag8 fg, fu, fx;
+    fx.u = load16(xb + 32 * (size_t)s);
+    if (WEIGHTED) fx.u = scaled16(fx.u, scale);
+    fu.u = load16(ur + 512 * (size_t)s);
+    if (GATED) {
+      fg.u = load16(gr + 512 * (size_t)s);
+      g = mfma16(fg, fx, g);
+    }
+    u = mfma16(fu, fx, u);
+  }
+  if (p < 0 || r < 16 / XP) return;
+  *reinterpret_cast<uint2*>(y + (size_t)t0 * RT_TILE * ff + (size_t)(c / 32) * 512 + 8 * (16 * ((c % 32) / 8) + r) + c % 8) =
+      make_uint2(pack_bf16x2(expert_unit<GATED>(g[0], u[0], limit, alpha), expert_unit<GATED>(g[1], u[1], limit, alpha)),
+                 pack_bf16x2(expert_unit<GATED>(g[2], u[2], limit, alpha), expert_unit<GATED>(g[3], u[3], limit, alpha)));
 }
 
 template <int NT, bool SHARED, int XP>
@@ -740,7 +764,8 @@ __global__ __launch_bounds__(RB_WAVE) void routed_down_few_kernel(const bf16_t* 
   const int r = lane & 15, grp = lane >> 4;
   int pair[NT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) pair[j] = j < nt ? row_pair[(t0 + j) * RT_TILE + r] : -1;
+  for (int j = 0; j < NT; ++j) pair[j] = j < nt && r < 16 / XP ? row_pair[(t0 + j) * RT_TILE + r] : -1;
+  const int behind = XP == 1 ? -1 : row_pair[t0 * RT_TILE + 16 / XP];
   const bf16_t* dr = w_down + ((size_t)e * width + c0) * ff + 8 * lane;
   const bf16_t* yr = y + (size_t)t0 * RT_TILE * ff + 16 * RowPack<XP>::depth(r) + 8 * (16 * grp + RowPack<XP>::row(r));
   f32x4_t acc[NT];
@@ -775,6 +800,18 @@ __global__ __launch_bounds__(RB_WAVE) void routed_down_few_kernel(const bf16_t* 
   for (int j = 0; j < NT; ++j)
     if (pair[j] >= 0)
       *reinterpret_cast<float4*>(out + (size_t)pair[j] * width + c0 + 4 * grp) = make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
+  if (behind < 0) return;
+  const int p = row_pair[t0 * RT_TILE + r];
+  const bf16_t* yb = y + (size_t)t0 * RT_TILE * ff + 8 * lane;
+  f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int s = 0; s < n_steps; ++s) {
+    Frag8 fd, fy;
+    fd.u = load16(dr + 512 * (size_t)s);
+    fy.u = load16(yb + 512 * (size_t)s);
+    sum = mfma16(fd, fy, sum);
+  }
+  if (p >= 0 && r >= 16 / XP) *reinterpret_cast<float4*>(out + (size_t)p * width + c0 + 4 * grp) = make_float4(sum[0], sum[1], sum[2], sum[3]);
 }
 
 // A workgroup of 8 waves takes up to RT_SPAN tiles of 16 rows that follow one another in an expert's run (the

@@ -1562,6 +1562,28 @@ def test_a_tokens_experts_give_the_same_bits_however_many_tokens_a_load_brings(l
         assert torch.equal(part.forward(h[at].contiguous()), want[at])
 
 
+@pytest.mark.parametrize("hidden,ff", [(96, 64), (64, 192), (384, 640)])
+@pytest.mark.parametrize("params", [dict(score="softmax", weight_on="output", unit="squared_relu"), dict(score="chosen", weight_on="output"),
+                                    dict(limit=7.0), dict(score="softmax", weight_on="output", unit="squared_relu", shared={"intermediate_size": 128, "gate": False})])
+def test_a_token_of_nan_changes_nothing_in_the_tokens_beside_it(lib, hidden, ff, params):
+    """Its router's logits are none, and it chooses the first expert every time: a run with more rows than the step has tokens."""
+    if params.get("shared") and (hidden % 128 or ff < 128):
+        params = dict(params, shared=None)
+    gen = torch.Generator().manual_seed(hidden + ff)
+    part = build_part("feed_forward", PartSpec("routed_experts", dict(params, experts=4, top=4, intermediate_size=ff)),
+                      BuildEnv(hidden_size=hidden, dtype=torch.bfloat16, device=torch.device(DEV), lib=lib))
+    part.load({name: (torch.randn(ts.shape, generator=gen) * ts.shape[-1] ** -0.5).to(torch.float32 if ts.role == "gain" else torch.bfloat16).to(DEV)
+               for name, ts in part.tensor_specs().items()})
+    h = torch.randn(16, hidden, generator=gen).bfloat16().to(DEV)
+    want = part.forward(h)
+    for n in (3, 4, 7, 8, 16):
+        for bad in (0, 1, n - 1):
+            some = h[:n].clone()
+            some[bad] = float("nan")
+            got, others = part.forward(some), [i for i in range(n) if i != bad]
+            assert torch.equal(got[others], want[others])
+
+
 # ---------------------------------------------------------------------------- a norm with the convolution behind it
 @pytest.mark.parametrize("width", [4, 260, 2048, 4096])
 @pytest.mark.parametrize("taps,copies,update,biased,dtype", [(2, 1, False, True, torch.bfloat16), (3, 2, True, True, torch.float32),
