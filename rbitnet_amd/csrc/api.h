@@ -316,6 +316,9 @@ int rb_gate_rmsnorm_parts(const float* o, const float* weight, const float* gate
 // out[r] = (v - mean) / sqrt(var + eps) * weight + bias.  delta null: the norm alone.
 int rb_layernorm_residual(float* x, const float* delta, const float* delta2, float dscale, const float* weight, const float* bias,
                           float eps, const int32_t* rows, int n_rows, int width, void* out, int out_dtype, void* stream);
+// the same, delta2 being terms [T, terms2, E] that are added up in their order first
+int rb_layernorm_residual_terms(float* x, const float* delta, const float* delta2, int terms2, float dscale, const float* weight, const float* bias,
+                                float eps, const int32_t* rows, int n_rows, int width, void* out, int out_dtype, void* stream);
 
 // ---- around the mixers (mixers.hip)
 // rb_rope_kv_write for heads whose keys and values differ in size and of which only the first `rot` numbers are rotated

@@ -213,6 +213,7 @@ class Kernels:
             "rb_recurrence_prep": [_P, _L, _I, _I, _I, _F, _F, _P, _L, _I, _I, _P, _P, _F, _I, _P, _L, _P, _I, _P],
             "rb_linear_recurrence": [_P, _P, _L, _P, _L, _P, _L, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
             "rb_gated_rmsnorm_act": [_P, _P, _P, _L, _I, _F, _P, _I, _I, _I, _I, _P],
+            "rb_layernorm_residual_terms": [_P, _P, _P, _I, _F, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_layernorm_residual": [_P, _P, _P, _F, _P, _P, _F, _P, _I, _I, _P, _I, _P],
             "rb_rope_store": [_P, _L, _P, _P, _I, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
             "rb_head_gate": [_P, _I, _P, _L, _I, _I, _I, _P],
@@ -1032,12 +1033,13 @@ class Kernels:
     def layernorm_residual(self, x: torch.Tensor, delta: Optional[torch.Tensor], delta2: Optional[torch.Tensor], dscale: float,
                            weight: torch.Tensor, bias: Optional[torch.Tensor], eps: float, rows: Optional[torch.Tensor],
                            out: torch.Tensor) -> None:
-        """Layer norm of x [T, E] + dscale * (delta + delta2); without rows the sum is written back to x."""
+        """Layer norm of x [T, E] + dscale * (delta + delta2); without rows the sum is written back to x.  delta2 may be terms
+        [T, P, E] that are added up in their order first."""
         n, width = x.shape
         _check(x, "x", torch.float32)
         for name, d in (("delta", delta), ("delta2", delta2)):
             if d is not None:
-                _check(d, name, torch.float32, (n, width))
+                _check(d, name, torch.float32, (n, d.shape[1], width) if name == "delta2" and d.dim() == 3 else (n, width))
         if delta is None and delta2 is not None:
             raise KernelError("layernorm_residual: a second term without a first")
         _check(weight, "weight", torch.float32, (width,))
@@ -1048,6 +1050,11 @@ class Kernels:
             n_rows = rows.shape[0]
             _check(rows, "rows", torch.int32, (n_rows,))
         _check(out, "out", None, (n_rows, width))
+        if delta2 is not None and delta2.dim() == 3:
+            self._ok(self._lib.rb_layernorm_residual_terms(_ptr(x), _ptr(delta), _ptr(delta2), delta2.shape[1], float(dscale), _ptr(weight),
+                                                           _ptr(bias), float(eps), _ptr(rows), n_rows, width, _ptr(out), dtype_code(out.dtype),
+                                                           self._stream()))
+            return
         self._ok(self._lib.rb_layernorm_residual(_ptr(x), _ptr(delta), _ptr(delta2), float(dscale), _ptr(weight), _ptr(bias),
                                                  float(eps), _ptr(rows), n_rows, width, _ptr(out), dtype_code(out.dtype),
                                                  self._stream()))

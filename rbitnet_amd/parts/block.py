@@ -171,7 +171,10 @@ class ParallelBlock:
             raise ConfigError("what follows a parallel layer must begin with a norm that adds a scaled sum (layernorm)")
         h = self.norm1.forward(x, pending, None)
         a = self.mixer.forward(h, ctx, view)
-        b = self.feed_forward.forward(h, ctx) if self.feed_forward is not None else None
+        if getattr(self.feed_forward, "leaves_sum", False) and getattr(next_norm, "adds_scaled_terms", False):
+            b = self.feed_forward.forward(h, ctx, terms=True)
+        else:
+            b = self.feed_forward.forward(h, ctx) if self.feed_forward is not None else None
         return ScaledSum(a, b, self.scale)
 
 

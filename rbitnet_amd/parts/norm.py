@@ -95,6 +95,7 @@ class LayerNorm(Part):
     reads_copies = True
     takes_conv = True             # forward takes conv: what `short_conv` makes of the result, for single tokens
     adds_scaled_sum = True        # delta may be a ScaledSum: scale * (a + b), added in the norm's own pass
+    adds_scaled_terms = True      # whose b may be terms [T, P, E]
 
     def __init__(self, params: Dict, env: BuildEnv):
         self.size = int(params["size"])

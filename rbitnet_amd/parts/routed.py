@@ -113,6 +113,7 @@ class RoutedExperts(Part):
                       and not self.has_bias and self.unit == "gated")
         # the sum over a token's experts may be left to whoever reads it, where it is nothing but that
         self.leaves_pairs = self.weight_on == "output" and not self.identity and self.shared is None
+        self.leaves_sum = self.weight_on == "input" and self.top > 1
         self.leaves_shared_pairs = self.weight_on == "output" and not self.identity and not self.shared_gate
         self.kinds = ("gate", "up") if self.unit == "gated" else ("up",)
 
@@ -182,8 +183,10 @@ class RoutedExperts(Part):
         else:
             self.w_gate, self.w_up = stack("gate") if gated else None, stack("up")
 
-    def forward(self, h: torch.Tensor, ctx=None, stream: Optional[torch.Tensor] = None, next_norm=None, pairs: bool = False):
-        """-> float32 [T, E], or, with pairs=True (where `leaves_pairs` or `leaves_shared_pairs`), the `ExpertPairs` of the step."""
+    def forward(self, h: torch.Tensor, ctx=None, stream: Optional[torch.Tensor] = None, next_norm=None, pairs: bool = False,
+                terms: bool = False):
+        """-> float32 [T, E], or, with pairs=True (where `leaves_pairs` or `leaves_shared_pairs`), the `ExpertPairs` of the step, or, with
+        terms=True (where `leaves_sum`), the outputs of every token's experts [T, top, E], whose sum is still to be done."""
         lib, t, dev = self.env.lib, h.shape[0], h.device
         n_pairs = t * self.top
         # (gated experts have a kernel for runs of a few dozen rows that is as fast; a row's place is a 32-bit byte offset in the tiles)
@@ -236,6 +239,8 @@ class RoutedExperts(Part):
             return total
         if self.top == 1:
             return out
+        if terms:
+            return out.view(t, self.top, self.hidden)
         total = torch.empty((t, self.hidden), dtype=torch.float32, device=dev)
         lib.pairs_sum(out, self.top, total)
         return total

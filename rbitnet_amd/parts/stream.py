@@ -16,7 +16,8 @@ prepared for the norm that follows, `GainedRows`).  What a sublayer has not yet 
                     is still to be done; a norm that reads such a stream does it in its own pass over the rows.  The result may
                     be terms [P, T, E] or `ExpertPairs` where that norm says `adds_update_terms`
     ScaledSum       scale * (a + b) still to be added: the two sublayers of a layer whose mixer and feed-forward read
-                    the same norm, and the layer's residual factor; a norm that says `adds_scaled_sum` takes it as delta
+                    the same norm, and the layer's residual factor; a norm that says `adds_scaled_sum` takes it as delta, and with
+                    b as terms [T, P, E] where it says `adds_scaled_terms`
     StreamCopy      nothing to add, and the stream's rows as they are in the compute dtype: what the sublayers of a layer
                     whose norms stand on the sublayers' outputs read; only a block that says `takes_stream_copy` gets it
                     (`run_blocks` drops it before any other block and before the head)
@@ -38,6 +39,7 @@ returns plain tensors, a norm without any does every sum and every normalisation
     norm.reads_copies         forward takes a stream in several copies [S, T, E] with coef, and a StreamsUpdate as delta
     norm.adds_update_terms    that update's result may be terms [P, T, E] or `ExpertPairs` (with a shared expert's output)
     part.leaves_terms         forward takes next_norm (stream None) and may return [P, T, E] to one that `adds_terms`
+    part.leaves_sum           forward takes terms=True and then may return its result as terms [T, P, E]
     part.leaves_pairs         forward takes pairs=True and then returns `ExpertPairs`
     part.leaves_shared_pairs  the same, and the pairs may come with a shared expert's output
     norm.folds_into_products  the norm is x * weight / sqrt(mean x^2 + eps) with `weight`, `eps`
@@ -110,7 +112,7 @@ class StreamsUpdate:
 
 
 class ScaledSum:
-    """scale * (a + b) that is still to be added to the stream x [T, E]; b may be None."""
+    """scale * (a + b) that is still to be added to the stream x [T, E]; b may be None, or terms [T, P, E] to be added up in their order."""
 
     def __init__(self, a: torch.Tensor, b: Optional[torch.Tensor], scale: float):
         self.a, self.b, self.scale = a, b, float(scale)

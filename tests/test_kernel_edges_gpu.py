@@ -1755,3 +1755,26 @@ def test_float32_products_of_few_tokens_take_sum_and_norm_along(lib, n, k, frag)
             sg, su = (normed.abs() @ rows.double().abs().T).split(n // 2, dim=1)
             close(got, g * torch.sigmoid(g) * u, 1.1 * sg * u.abs() + (g.abs() + 1.0) * su)
     assert not lib.gemm_f32_few_ok(17, n, k, frag, 0) and not lib.gemm_f32_few_ok(4, n, k + 2, frag, 2)
+
+
+# ---------------------------------------------------------------------------- a norm that adds up the outputs of a token's experts
+@pytest.mark.parametrize("width", [4, 101, 2048, 4104])
+@pytest.mark.parametrize("terms", [1, 2, 3, 4, 5, 9])
+def test_a_norm_adds_up_the_outputs_of_a_tokens_experts_to_the_bits_of_two_launches(lib, width, terms):
+    gen = torch.Generator().manual_seed(width + terms)
+    r = lambda *shape: torch.randn(*shape, generator=gen).to(DEV)
+    n, rows = 5, torch.tensor([4, 0, 3], dtype=torch.int32, device=DEV)
+    x, a, pairs, weight, bias = r(n, width), r(n, width), r(n * terms, width), r(width), r(width)
+    total = torch.empty(n, width, device=DEV)
+    if terms > 1:
+        lib.pairs_sum(pairs, terms, total)
+    else:
+        total.copy_(pairs)
+    for some in (None, rows):
+        for dtype in (torch.float32, torch.bfloat16):
+            one, two = x.clone(), x.clone()
+            got, want = (torch.full((n if some is None else 3, width), float("nan"), dtype=dtype, device=DEV) for _ in range(2))
+            lib.layernorm_residual(one, a, pairs.view(n, terms, width), 0.6, weight, bias, 1e-5, some, got)
+            lib.layernorm_residual(two, a, total, 0.6, weight, bias, 1e-5, some, want)
+            assert torch.isfinite(want.float()).all() and torch.equal(got, want) and torch.equal(one, two)
+            assert torch.equal(one, x) == (some is not None)
