@@ -255,11 +255,11 @@ int rb_short_conv_biases(const float* x, long long x_stride, const float* bias, 
 struct RbGroupProduct {
   const void *x, *w;
   void* c;
-  int n, end;
+  int n, end, k;
 };
 int rb_gemm_bf16_group_ok(int m, int k);
 int rb_gemm_bf16_group_pays(int m, int n, int k);      // whether a product of n rows gains among others, its bits being the same
-int rb_gemm_bf16_group(const struct RbGroupProduct* products, int count, int w_layout, int m, int k, void* stream);
+int rb_gemm_bf16_group(const struct RbGroupProduct* products, int count, int w_layout, int m, void* stream);
 // A step of ONE token per sequence (token t is of slot slots[t]) through such a layer in one launch: convolution and silu (conv_w null:
 // none; the state moves on), unit vectors or the query's scale, decays, the recurrence, the read-out norm and its gate.
 //   mode 0: the delta rule (beta = sigmoid(b)); 1: the plain rule; 2: read before the write, with a bonus [H, dim]; 3: the selective scan,

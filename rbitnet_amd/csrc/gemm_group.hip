@@ -1,4 +1,4 @@
-// Several products of a few tokens in one launch: C_i = X_i W_i^T, bfloat16 operands of one depth K, each with inputs, a matrix, outputs
+// Several products of a few tokens in one launch: C_i = X_i W_i^T, bfloat16 operands, each with inputs, a depth, a matrix, outputs
 // and an end of its own.  A layer's projections that do not wait for each other (the inputs of time mixing and what its decays are made
 // from; a large product and the low-rank one beside it) were launches one after the other, and a product of 16 to 1,024 rows with 4 tokens at
 // K = 2048 costs 3.8 to 5 us whatever it reads (4 MB: 0.6 us of memory's time): its boundary, two trips to memory, the waves' sums.
@@ -21,13 +21,14 @@ struct Group {
 };
 
 template <bool WF, int XP>                                 // XP: see RowPack
-__global__ __launch_bounds__(512) void gemm_group_kernel(const Group g, int m, int k) {
+__global__ __launch_bounds__(512) void gemm_group_kernel(const Group g, int m) {
   extern __shared__ __attribute__((aligned(16))) float red[];      // [waves - 1][64] pieces of four sums
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, kq = lane >> 4;
   int i = 0;
   while (i + 1 < g.count && (int)blockIdx.x >= g.end[i]) ++i;
   const int n_waves = g.waves[i];
   const RbGroupProduct p = g.p[i];
+  const int k = p.k;
   const int n0 = 16 * ((int)blockIdx.x - (i > 0 ? g.end[i - 1] : 0));
   const bf16_t* w = (const bf16_t*)p.w;
   const bf16_t* wrow = WF ? w + (size_t)n0 * k + 8 * lane : w + (size_t)(n0 + r < p.n ? n0 + r : 0) * k + 8 * kq;
@@ -101,17 +102,17 @@ extern "C" int rb_gemm_bf16_group_ok(int m, int k) { return m >= 1 && m <= 16 &&
 // 8,192 rows (resident tokens: other sums) 43.8/47.6 and 52.4/52.3.
 extern "C" int rb_gemm_bf16_group_pays(int m, int n, int k) { return rb_gemm_bf16_group_ok(m, k) && n > 0 && gemm_sums_alone_alike(m, n, k); }
 
-extern "C" int rb_gemm_bf16_group(const RbGroupProduct* products, int count, int w_layout, int m, int k, void* stream) {
+extern "C" int rb_gemm_bf16_group(const RbGroupProduct* products, int count, int w_layout, int m, void* stream) {
   RB_REQUIRE(products != nullptr && count >= 1 && count <= MOST, "rb_gemm_bf16_group: %d products (1 to %d)", count, MOST);
   Group g;
   g.count = count;
   for (int i = 0; i < count; ++i) g.p[i] = products[i];
-  RB_RECORDED(rb_gemm_bf16_group(g.p, count, w_layout, m, k, stream));
-  RB_REQUIRE(m == 0 || rb_gemm_bf16_group_ok(m, k), "rb_gemm_bf16_group: M=%d K=%d is not for it", m, k);
+  RB_RECORDED(rb_gemm_bf16_group(g.p, count, w_layout, m, stream));
   RB_REQUIRE(w_layout == 0 || w_layout == 1, "rb_gemm_bf16_group: W layout %d", w_layout);
   long long tiles = 0;
   for (int i = 0; i < count; ++i) {
     const RbGroupProduct& p = g.p[i];
+    RB_REQUIRE(m == 0 || rb_gemm_bf16_group_ok(m, p.k), "rb_gemm_bf16_group: M=%d K=%d is not for it", m, p.k);
     RB_REQUIRE(p.x && p.w && p.c && p.n > 0 && p.end >= END_F32 && p.end <= END_TANH && (w_layout == 0 || p.n % 16 == 0),
                "rb_gemm_bf16_group: product %d of %d rows, layout %d, end %d", i, p.n, w_layout, p.end);
     RB_REQUIRE(((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.w) | reinterpret_cast<uintptr_t>(p.c)) & 15) == 0,
@@ -124,13 +125,13 @@ extern "C" int rb_gemm_bf16_group(const RbGroupProduct* products, int count, int
   // every product has the waves that it has alone with one row tile a wave; the others of its workgroups wait at the barrier
   int waves = 1;
   for (int i = 0; i < count; ++i) {
-    g.waves[i] = gemm_skinny_waves(g.p[i].n, k);
+    g.waves[i] = gemm_skinny_waves(g.p[i].n, g.p[i].k);
     if (g.waves[i] > waves) waves = g.waves[i];
   }
   const size_t lds = (size_t)(waves - 1) * 256 * sizeof(float);
   if (w_layout)
-    (m <= 4 ? gemm_group_kernel<true, 4> : m <= 8 ? gemm_group_kernel<true, 2> : gemm_group_kernel<true, 1>)<<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
-  else gemm_group_kernel<false, 1><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m, k);
+    (m <= 4 ? gemm_group_kernel<true, 4> : m <= 8 ? gemm_group_kernel<true, 2> : gemm_group_kernel<true, 1>)<<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m);
+  else gemm_group_kernel<false, 1><<<(int)tiles, waves * 64, lds, (hipStream_t)stream>>>(g, m);
   RB_LAUNCH_CHECK();
   return 0;
 }

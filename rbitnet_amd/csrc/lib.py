@@ -128,7 +128,7 @@ class RecurrenceStep(ctypes.Structure):
 
 class GroupProduct(ctypes.Structure):
     """RbGroupProduct of csrc/api.h."""
-    _fields_ = [("x", _P), ("w", _P), ("c", _P), ("n", _I), ("end", _I)]
+    _fields_ = [("x", _P), ("w", _P), ("c", _P), ("n", _I), ("end", _I), ("k", _I)]
 
 
 GROUP_PRODUCTS = 6                       # RB_GROUP_PRODUCTS
@@ -196,7 +196,7 @@ class Kernels:
             "rb_short_conv_biases": [_P, _L, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P],
             "rb_gemm_bf16_group_ok": [_I, _I],
             "rb_gemm_bf16_group_pays": [_I, _I, _I],
-            "rb_gemm_bf16_group": [ctypes.POINTER(GroupProduct), _I, _I, _I, _I, _P],
+            "rb_gemm_bf16_group": [ctypes.POINTER(GroupProduct), _I, _I, _I, _P],
             "rb_recurrence_step_ok": [_I, _I, _I, _I, _I, _I],
             "rb_recurrence_step": [ctypes.POINTER(RecurrenceStep), _P],
             "rb_selective_scan": [_P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
@@ -433,18 +433,19 @@ class Kernels:
                                             _ptr(act), m, n, k, _ptr(workspace), self._stream()))
 
     def gemm_bf16_group(self, products, w_frag: bool) -> None:
-        """products: up to GROUP_PRODUCTS of (x [M, K], w [N, K], c [M, N], end), all of one M, K and layout of w; end: "float32",
+        """products: up to GROUP_PRODUCTS of (x [M, K], w [N, K], c [M, N], end), all of one M and layout of w; end: "float32",
         "bfloat16" (the type of c), or "tanh": c = bfloat16(tanh(x w^T))."""
-        m, k = products[0][0].shape
+        m = products[0][0].shape[0]
         if len(products) > GROUP_PRODUCTS:
             raise KernelError(f"gemm_bf16_group: at most {GROUP_PRODUCTS} products")
         args = (GroupProduct * len(products))()
         for a, (x, w, c, end) in zip(args, products):
+            k = x.shape[1]
             _check(x, "x", torch.bfloat16, (m, k))
             _check(w, "w", torch.bfloat16, (w.shape[0], k))
             _check(c, "c", torch.float32 if end == "float32" else torch.bfloat16, (m, w.shape[0]))
-            a.x, a.w, a.c, a.n, a.end = _ptr(x), _ptr(w), _ptr(c), w.shape[0], GROUP_ENDS[end]
-        self._ok(self._lib.rb_gemm_bf16_group(args, len(products), int(bool(w_frag)), m, k, self._stream()))
+            a.x, a.w, a.c, a.n, a.end, a.k = _ptr(x), _ptr(w), _ptr(c), w.shape[0], GROUP_ENDS[end], k
+        self._ok(self._lib.rb_gemm_bf16_group(args, len(products), int(bool(w_frag)), m, self._stream()))
 
     def gemm_bf16_group_ok(self, m: int, k: int) -> bool:
         return bool(self._lib.rb_gemm_bf16_group_ok(int(m), int(k)))

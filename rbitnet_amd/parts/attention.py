@@ -88,6 +88,7 @@ class Attention(Part):
     graph_safe = True
     plan_safe = True
     takes_gained_rows = True
+    leaves_product = True
     adds_to_stream = True
     leaves_terms = True
 
@@ -312,14 +313,14 @@ class Attention(Part):
         return out + ([state] if state is not None else [])
 
     # ------------------------------------------------------------------ forward
-    def _gate_and_project(self, attn, h, stream, next_norm, gate=None):
+    def _gate_and_project(self, attn, h, stream, next_norm, gate=None, product=False):
         lib = self.env.lib
         if self.gate_kind == "head":
             logits = linear(lib, h, self.w_gate, torch.float32) if gate is None else gate
             lib.head_gate(attn, logits, 0, self.n_heads, self.pad)
         elif self.gate_kind == "elementwise":
             lib.sigmoid_gate(attn, linear(lib, h, self.w_gate, torch.float32) if gate is None else gate)
-        return linear_to_stream(lib, attn, self.w_o, stream, next_norm)
+        return (attn, self.w_o) if product else linear_to_stream(lib, attn, self.w_o, stream, next_norm)
 
     def _shared_keys(self, ctx):
         """What lets several workgroups share a token's keys in float32 steps of single tokens."""
@@ -327,7 +328,7 @@ class Attention(Part):
             return None
         return ctx.shared_keys_workspace(self.env.lib, self.n_heads, self.pad, self.n_kv)
 
-    def _forward_prepared(self, h, ctx, view, stream, next_norm, qkv=None, gate=None):
+    def _forward_prepared(self, h, ctx, view, stream, next_norm, qkv=None, gate=None, product=False):
         """Bias and convolution, norms with weights, rotation and the cache write by kernels of their own; attention with
         capped scores and kept first tokens; the gate."""
         lib = self.env.lib
@@ -370,9 +371,9 @@ class Attention(Part):
             lib.attention_opts(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, view.block_table, hq, hk, d,
                                self.scale, window, self.keep_first, self.softcap or 0.0, self.sink, chunk=self.chunk or 0,
                                sig_bias=self.score_bias, n_seqs=ctx.n_seqs, shared=self._shared_keys(ctx))
-        return self._gate_and_project(attn, h, stream, next_norm, gate)
+        return self._gate_and_project(attn, h, stream, next_norm, gate, product)
 
-    def _forward_mixed(self, h, ctx, view, stream, next_norm, qkv=None, gate=None):
+    def _forward_mixed(self, h, ctx, view, stream, next_norm, qkv=None, gate=None, product=False):
         """Biases, unit heads, the cache write, and attention with all heads of a token together."""
         lib = self.env.lib
         t, hq, hk, d = h.shape[0], self.n_heads, self.n_kv, self.pad
@@ -399,22 +400,22 @@ class Attention(Part):
         else:
             lib.attention_mixed(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, view.block_table, hq, hk, d,
                                 self.scale, self.talk, self.chunk or 0, window)
-        return self._gate_and_project(attn, h, stream, next_norm, gate)
+        return self._gate_and_project(attn, h, stream, next_norm, gate, product)
 
     def early(self, h):
         """The products that wait for nothing but the mixer's input (`linear_group`'s): `forward` takes their results as `ready`."""
         return [(h, self.w_qkv, "float32")] + ([(h, self.w_gate, "float32")] if self.has_gate else [])
 
-    def forward(self, h, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None, ready=None):
+    def forward(self, h, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None, ready=None, product: bool = False):
         if (self.prepared or self.mixed) and hasattr(h, "tensor") and not isinstance(h, torch.Tensor):
             h = h.tensor()
         if ready is None and self.has_gate and products_in_one_launch(self.env.lib, h):
             ready = linear_group(self.env.lib, self.early(h), self.env.dtype)
         qkv, gate = (list(ready or []) + [None, None])[:2]
         if self.prepared:
-            return self._forward_prepared(h, ctx, view, stream, next_norm, qkv, gate)
+            return self._forward_prepared(h, ctx, view, stream, next_norm, qkv, gate, product)
         if self.mixed:
-            return self._forward_mixed(h, ctx, view, stream, next_norm, qkv, gate)
+            return self._forward_mixed(h, ctx, view, stream, next_norm, qkv, gate, product)
         lib = self.env.lib
         t = h.shape[0]
         hq, hk, d = self.n_heads, self.n_kv, self.pad
@@ -441,7 +442,7 @@ class Attention(Part):
             n_splits, workspace = ctx.decode_workspace(hq, d, hk, spread=window == 0 and self.sink is None)
             lib.attention_decode_fused_bf16(qkv, cos, sin, style, view.k_pages, view.v_pages, attn, ctx.tok_pos, bt,
                                             hq, hk, d, self.scale, window, n_splits, workspace, sinks=self.sink)
-            return self._gate_and_project(attn, h, stream, next_norm, gate)
+            return self._gate_and_project(attn, h, stream, next_norm, gate, product)
         q = torch.empty((t, hq, d), dtype=self.env.dtype, device=h.device)
         if self.same_sizes:
             if owns:
@@ -464,7 +465,7 @@ class Attention(Part):
         else:
             lib.attention_sinks(q, view.k_pages, view.v_pages, attn, ctx.tok_pos, ctx.tok_seq, bt, hq, hk, d,
                                 self.scale, window, self.sink, n_seqs=ctx.n_seqs, shared=self._shared_keys(ctx))
-        return self._gate_and_project(attn, h, stream, next_norm, gate)
+        return self._gate_and_project(attn, h, stream, next_norm, gate, product)
 
 
 register_mixer("attention", Attention)

@@ -241,6 +241,7 @@ class DecayAttention(Part):
     Parameters: heads, dim, vdim, tau, decay_rank (the inner size of the decay's two matrices), eps, names."""
     graph_safe = True
     plan_safe = True
+    leaves_product = True
 
     NAMES = {"q": "q", "k": "k", "v": "v", "g": "g", "o": "o", "norm": "norm", "a1": "a1", "a2": "a2", "a_bias": "a2.b"}
 
@@ -297,7 +298,8 @@ class DecayAttention(Part):
         """The products that wait for nothing but the mixer's input (`linear_group`'s): `forward` takes their results as `ready`."""
         return [(h, self.w_in, "float32"), (h, self.w_a1, "same")]
 
-    def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None, ready=None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None, ready=None,
+                product: bool = False) -> torch.Tensor:
         lib, t, c, dt = self.env.lib, h.shape[0], self.cols, self.env.dtype
         proj, low = linear_group(lib, self.early(h), dt) if ready is None else ready                # proj [T, q | k | v | gate]
         z = linear(lib, low, self.w_a2, torch.float32)                        # [T, heads * dim]
@@ -306,14 +308,14 @@ class DecayAttention(Part):
             lib.recurrence_step("plain", (proj, 0), (proj, self.n_qk), (proj, 2 * self.n_qk), self.heads, self.heads, self.dim, self.vdim,
                                 (z, 0), False, 1, view.states["decay"], ctx, (proj, c["g"]), 1, self.norm, self.eps, on,
                                 a_bias=self.a_bias, tau=self.tau, q_scale=self.dim ** -0.5)
-            return linear(lib, on, self.w_o, torch.float32)
+            return (on, self.w_o) if product else linear(lib, on, self.w_o, torch.float32)
         lib.recurrence_prep(proj, self.heads, self.dim, False, self.dim ** -0.5, 0.0, z, 0, self.n_qk, 1, self.a_bias, None,
                             self.tau, self.heads)
         o = torch.empty((t, self.n_v), dtype=torch.float32, device=h.device)
         lib.linear_recurrence(proj, self.heads, self.dim, self.heads, self.vdim, z, 0, False, None, view.states["decay"], ctx, o)
         on = torch.empty((t, self.n_v), dtype=dt, device=h.device)
         lib.gated_rmsnorm_act(o, self.norm, proj, c["g"], 1, self.eps, self.heads, self.vdim, on)
-        return linear(lib, on, self.w_o, torch.float32)
+        return (on, self.w_o) if product else linear(lib, on, self.w_o, torch.float32)
 
 
 class TimeMix(Part):
@@ -330,6 +332,7 @@ class TimeMix(Part):
     Parameters: heads, dim, decay_rank (the inner size of the decay's two matrices), eps, names."""
     graph_safe = True
     plan_safe = True
+    leaves_product = True
 
     NAMES = {"mu_r": "mu.r", "mu_k": "mu.k", "mu_v": "mu.v", "mu_g": "mu.g", "mu_w": "mu.w", "r": "r", "k": "k", "v": "v", "g": "g",
              "w1": "w1", "w2": "w2", "w0": "w0", "u": "u", "norm": "norm", "o": "o"}
@@ -372,7 +375,8 @@ class TimeMix(Part):
     def cache_request(self) -> Optional[CacheRequest]:
         return self.cache_requests()[0]
 
-    def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, ctx, view, stream: Optional[torch.Tensor] = None, next_norm=None,
+                product: bool = False) -> torch.Tensor:
         lib, t, dt = self.env.lib, h.shape[0], self.env.dtype
         mixes = torch.empty((5, t, self.hidden), dtype=dt, device=h.device)
         lib.shift_mix(h, view.states["time_shift"], self.mu, ctx, mixes)
@@ -382,13 +386,13 @@ class TimeMix(Part):
             on = torch.empty((t, self.n), dtype=dt, device=h.device)
             lib.recurrence_step("bonus", (r, 0), (k, 0), (v, 0), self.heads, self.heads, self.dim, self.dim, (decay, 0), False, 2,
                                 view.states["time_mix"], ctx, (g, 0), 1, self.norm, self.eps, on, a_bias=self.w0, bonus=self.u)
-            return linear(lib, on, self.w_o, torch.float32)
+            return (on, self.w_o) if product else linear(lib, on, self.w_o, torch.float32)
         lib.decay_exp_exp(decay, self.w0, self.heads, self.dim)
         o = torch.empty((t, self.n), dtype=torch.float32, device=h.device)
         lib.time_mix_recurrence(r, k, v, decay, self.u, view.states["time_mix"], ctx, o, self.heads, self.dim, self.dim)
         on = torch.empty((t, self.n), dtype=dt, device=h.device)
         lib.gated_rmsnorm_heads(o, self.norm, g, 1, self.eps, self.heads, self.dim, on)
-        return linear(lib, on, self.w_o, torch.float32)
+        return (on, self.w_o) if product else linear(lib, on, self.w_o, torch.float32)
 
 
 class LightningAttention(Part):

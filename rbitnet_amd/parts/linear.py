@@ -118,10 +118,10 @@ def linear_group(lib, products, dtype: torch.dtype):
     """Products that do not wait for each other: [(x [M, K], w, end)], end "float32", "same" (the result in `dtype`) or "tanh" (tanh of
     the result, in `dtype`) -> their results, the same bits either way.  One launch where tokens are few, all matrices are stored alike and
     each product gains by it; else one after another."""
-    m, k = products[0][0].shape
+    m = products[0][0].shape[0]
     frags = {_data(w)[1] for _, w, _ in products}
     if (dtype == torch.bfloat16 and len(frags) == 1 and len(products) <= GROUP_PRODUCTS
-            and all(x.shape == (m, k) and products_in_one_launch(lib, x) and lib.gemm_bf16_group_pays(m, w.shape[0], k) for x, w, _ in products)):
+            and all(x.shape[0] == m and products_in_one_launch(lib, x) and lib.gemm_bf16_group_pays(m, w.shape[0], x.shape[1]) for x, w, _ in products)):
         args = [(x, _data(w)[0], torch.empty((m, w.shape[0]), dtype=torch.float32 if end == "float32" else dtype, device=x.device),
                  "bfloat16" if end == "same" else end) for x, w, end in products]
         if all(t.data_ptr() % 16 == 0 for x, w, _, _ in args for t in (x, w)):

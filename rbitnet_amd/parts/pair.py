@@ -108,8 +108,14 @@ class MixerPair(Part):
             if len(first) + len(second) <= GROUP_PRODUCTS:
                 done = linear_group(self.env.lib, first + second, self.env.dtype)
                 ready = [{"ready": done[:len(first)]}, {"ready": done[len(first):]}]
-        a = self.left.forward(h, ctx, view, **ready[0])
-        b = self.right.forward(h, ctx, view, **ready[1])
+        if (getattr(self.left, "leaves_product", False) and getattr(self.right, "leaves_product", False)
+                and products_in_one_launch(self.env.lib, h)):
+            # and what they end with, in another
+            ends = [part.forward(h, ctx, view, product=True, **early) for part, early in ((self.left, ready[0]), (self.right, ready[1]))]
+            a, b = linear_group(self.env.lib, [(x, w, "float32") for x, w in ends], self.env.dtype)
+        else:
+            a = self.left.forward(h, ctx, view, **ready[0])
+            b = self.right.forward(h, ctx, view, **ready[1])
         if self.combine == "weighted":
             if not weighted_terms:
                 raise ConfigError("a pair of mixers combined as a weighted sum needs a block that adds up its two terms (outnorm)")

@@ -39,6 +39,7 @@ returns plain tensors, a norm without any does every sum and every normalisation
     norm.reads_copies         forward takes a stream in several copies [S, T, E] with coef, and a StreamsUpdate as delta
     norm.adds_update_terms    that update's result may be terms [P, T, E] or `ExpertPairs` (with a shared expert's output)
     part.leaves_terms         forward takes next_norm (stream None) and may return [P, T, E] to one that `adds_terms`
+    part.leaves_product       forward takes product=True and then returns its last product's operands (x, w) instead of the result
     part.leaves_sum           forward takes terms=True and then may return its result as terms [T, P, E]
     part.leaves_pairs         forward takes pairs=True and then returns `ExpertPairs`
     part.leaves_shared_pairs  the same, and the pairs may come with a shared expert's output

@@ -1778,3 +1778,24 @@ def test_a_norm_adds_up_the_outputs_of_a_tokens_experts_to_the_bits_of_two_launc
             lib.layernorm_residual(two, a, total, 0.6, weight, bias, 1e-5, some, want)
             assert torch.isfinite(want.float()).all() and torch.equal(got, want) and torch.equal(one, two)
             assert torch.equal(one, x) == (some is not None)
+
+
+# ---------------------------------------------------------------------------- products of several depths in one launch
+@pytest.mark.parametrize("m", [1, 4, 7, 16])
+@pytest.mark.parametrize("sizes", [((2048, 2048), (2048, 1024)), ((16, 128), (4112, 4096), (64, 384)), ((1024, 8192), (1024, 128))])
+def test_products_of_several_depths_in_one_launch_give_the_bits_of_each_alone(lib, m, sizes):
+    gen = torch.Generator(device=DEV).manual_seed(m + sizes[0][1])
+    products, alone = [], []
+    for n, k in sizes:
+        x, rows = torch.randn(m, k, generator=gen, device=DEV).bfloat16(), (torch.randn(n, k, generator=gen, device=DEV) * k ** -0.5).bfloat16()
+        w, c = torch.empty_like(rows), torch.empty(m, n, device=DEV)
+        lib.place_rows(rows, w, frag=True)
+        lib.gemm_bf16(x, w, c, 0, w_frag=True)
+        alone.append(c if lib.gemm_bf16_group_pays(m, n, k) else None)
+        products.append((x, w, torch.full((m, n), float("nan"), device=DEV), "float32"))
+    assert any(c is not None for c in alone)
+    lib.gemm_bf16_group(products, True)
+    for (_, _, got, _), want in zip(products, alone):
+        assert want is None or torch.equal(got, want)
+    with pytest.raises(KernelError):
+        lib.gemm_bf16_group([products[0], (products[0][0][:, :96].contiguous(), products[0][1][:, :96].contiguous(), products[0][2], "float32")], True)
