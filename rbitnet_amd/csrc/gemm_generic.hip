@@ -171,6 +171,10 @@ struct F32Fold {
   int wide;                     // C, the gain and the prepared rows can be read and written four columns at a time
 };
 constexpr int F32_SQ_WIDE = 8;
+// A kernel that folds has one more argument.  The others have none: behind it the workgroup's size would no longer lie among the arguments that
+// are there when a wave starts (28,672 rows at K = 4096, 22 tokens: 142.2 us with it, 140.5 without).
+__device__ __forceinline__ F32Fold fold_of() { return F32Fold{}; }
+__device__ __forceinline__ F32Fold fold_of(const F32Fold& fa) { return fa; }
 
 __device__ __forceinline__ gf_f32x4_t four_of(const float* __restrict__ at, int left, int wide) {
   if (wide) return *reinterpret_cast<const gf_f32x4_t*>(at);
@@ -236,9 +240,11 @@ __device__ __forceinline__ void fold_end(gf_f32x4_t v, gf_f32x4_t before, gf_f32
 // GATED: W is the gate's n rows and then n rows of the way up (n % 16 == 0), c [m, n] = silu(gate) up.  Twice the waves: the first half takes a tile of the
 // gate, the other half the same rows of the way up, whose sums go to the first through LDS (gated_end).  The launch of 1 to 128 workgroups that
 // did this behind the product cost a step 2 us; every sum and the gate are as they are in two launches.
-template <bool GATED, bool FOLD = false>
+template <bool GATED, typename... FOLDS>
 __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ c,
-                                                            int m, int n, int k, const F32Fold fa) {
+                                                            int m, int n, int k, const FOLDS... folds) {
+  constexpr bool FOLD = sizeof...(FOLDS) > 0;
+  const F32Fold fa = fold_of(folds...);
   extern __shared__ float lds[];      // [waves - 1][4][64] for each of gate and way up, then, gated, [4][64], then, folded, [waves][16] for each
   const int lane = threadIdx.x & 63, n_waves = (blockDim.x >> 6) / (GATED ? 2 : 1);
   const int up = GATED && (int)(threadIdx.x >> 6) >= n_waves ? 1 : 0, wave = (threadIdx.x >> 6) - up * n_waves;
@@ -318,11 +324,15 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const
 // in registers.  A stage's 32 MFMAs add to one accumulator, 0.4 us one after the other, and behind them the next stage's loads took a trip to memory: with
 // two sets of registers they are under way meanwhile.  Where workgroups share a compute unit they do that for each other, and a wave
 // with more registers is slower (5,120 rows at K = 3072, 4 tokens: 14.9 us with one set, 15.9 with two).
+// U = 0: one set, its loads among the multiplications as the compiler places them; U = 1 keeps a block a load's tokens in front of W (4,096 rows at K = 4096, a workgroup
+// a compute unit, 4 / 12 tokens: 12.5 / 13.4 us with U = 0, 14.7 / 14.8 with 1; 28,672 rows, 12 / 16 tokens: 89 / 96 and 78 / 88).
 // GATED: as in the kernel above.
 // FOLD: see F32Fold.
-template <int MB, int R, bool WF, int XP = 1, int WP = 1, int U = 1, bool GATED = false, bool FOLD = false>
+template <int MB, int R, bool WF, int XP = 1, int WP = 1, int U = 1, bool GATED = false, typename... FOLDS>
 __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                          float* __restrict__ c, int m, int n, int k, const F32Fold fa) {
+                                                          float* __restrict__ c, int m, int n, int k, const FOLDS... folds) {
+  constexpr bool FOLD = sizeof...(FOLDS) > 0;
+  const F32Fold fa = fold_of(folds...);
   extern __shared__ float lds[];      // [waves - 1][R * MB * 4][64] (for each of gate and way up, then [4][64]), then, folded, [waves][16] (for each)
   static_assert(!FOLD || (MB == 1 && R == 1), "folded: one tile of tokens and of rows");
   static_assert(!GATED || (MB == 1 && R == 1 && WP == 1), "gated: one tile of tokens, one of gate rows");
@@ -379,18 +389,24 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const f
   const int total = k / 128, base = total / n_waves, extra = total % n_waves;
   const int stages = base + (wave < extra ? 1 : 0);
   const int k_begin = 128 * (wave * base + (wave < extra ? wave : extra));
-  static_assert(U == 1 || (U == 2 && MB == 1 && R == 1), "two stages in registers: one tile of tokens and of rows");
-  gf_f32x4_t as[U][R][8 / WP], bs[U][MB][8 / XP];
+  static_assert(U == 1 || (MB == 1 && R == 1), "two stages in registers: one tile of tokens and of rows");
+  gf_f32x4_t as[U == 2 ? 2 : 1][R][8 / WP], bs[U == 2 ? 2 : 1][MB][8 / XP];
   auto load_stage = [&](int u, int st) __attribute__((always_inline)) {
     auto &a = as[u];
     auto &b = bs[u];
     const int ks = k_begin + 128 * st;
+    if constexpr (MB == 1 && U < 2 && XP == 1) {           // the tokens, which the caches hold, in front of W
+#pragma unroll
+      for (int j = 0; j < 8; ++j) b[0][j] = *reinterpret_cast<const gf_f32x4_t*>(xrow[0] + ks + 16 * j);
+      if constexpr (U == 1) __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int j = 0; j < 8 / WP; ++j)
 #pragma unroll
       for (int rt = 0; rt < R; ++rt)
         a[rt][j] = WF ? __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + (size_t)(ks + 16 * WP * j) * WK))
                       : *reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + ks + 16 * WP * j);
+    if constexpr (MB == 1 && U < 2 && XP == 1) return;
 #pragma unroll
     for (int j = 0; j < 8 / XP; ++j)
 #pragma unroll
@@ -511,44 +527,51 @@ static bool f32_short_takes(int m, int n, int k) {
 }
 
 // At most 16 tokens: one tile of them
-template <bool FOLD>
-static void launch_f32_16(const float* x, const float* w, bool w_frag, float* c, int m, int n, int k, const F32Fold& fa, hipStream_t s) {
+template <typename... FOLDS>
+static void launch_f32_16(const float* x, const float* w, bool w_frag, float* c, int m, int n, int k, hipStream_t s, const FOLDS&... folds) {
+  constexpr bool FOLD = sizeof...(FOLDS) > 0;
   const int n_waves = f32_few_waves(k), grid = (n + 15) / 16;
   const size_t lds = ((size_t)(n_waves - 1) * 256 + (FOLD ? n_waves * 16 : 0)) * sizeof(float);
   // us, 4 tokens, as the kernel was (one stage, a block a load, whole tiles) and so: 3,072 rows at K = 3072 9.75 and 8.8, at 8192 24.3 and 21.3; 2,048 at 2048
   // 7.2 and 5.9, 1,024 at 4096 10.8 and 8.3 (halves of tiles); more workgroups than compute units: 5,120 at 3072 17.4 and 14.9, 16,384 38.0 and 35.0,
   // 128,256 260 and 239, 6,144 at 4096 23.4 and 20.7.  Halves of more tiles than half the units lose (3,072 rows at 3072 11.9).
+  // A second stage under way pays up to three tiles for four units and 12 tokens: with a tile a unit, 4,096 rows at K = 4096, 4 / 8 / 12 / 16 tokens, 12.6 / 12.6 /
+  // 12.9 / 13.6 without it and 13.1 / 13.4 / 14.3 / 15.4 with it; 3,072 rows at K = 8192 22.2 / 22.5 / 23.3 / 24.6 and 20.1 / 21.3 / 23.4 / 25.5.
   if (w_frag) {
+    const bool ahead = 4 * grid <= 3 * rb_compute_units() && m <= 12;
     const int cus = rb_compute_units(), parts = g_f32_parts ? g_f32_parts : 2 * grid <= cus ? 2 : 1, pack = m <= 4 ? 4 : m <= 8 ? 2 : 1;
     auto by = [&](auto four, auto two, auto one) { return pack == 4 ? four : pack == 2 ? two : one; };
-    (parts == 2    ? by(gemm_f32_few_kernel<1, 1, true, 4, 2, 2, false, FOLD>, gemm_f32_few_kernel<1, 1, true, 2, 2, 2, false, FOLD>,
-                        gemm_f32_few_kernel<1, 1, true, 1, 2, 2, false, FOLD>)
-     : grid <= cus ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2, false, FOLD>      // (packed tokens: 4,096 rows at K = 4096 14.2 for 13.9, the others the same)
-                   : by(gemm_f32_few_kernel<1, 1, true, 4, 1, 1, false, FOLD>, gemm_f32_few_kernel<1, 1, true, 2, 1, 1, false, FOLD>,
-                        gemm_f32_few_kernel<1, 1, true, 1, 1, 1, false, FOLD>))<<<parts * grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, fa);
+    (parts == 2    ? by(gemm_f32_few_kernel<1, 1, true, 4, 2, 2, false, FOLDS...>, gemm_f32_few_kernel<1, 1, true, 2, 2, 2, false, FOLDS...>,
+                        gemm_f32_few_kernel<1, 1, true, 1, 2, 2, false, FOLDS...>)
+     : ahead       ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2, false, FOLDS...>
+     : grid <= cus ? gemm_f32_few_kernel<1, 1, true, 1, 1, 0, false, FOLDS...>      // (packed tokens: 4,096 rows at K = 4096 14.2 for 13.9)
+                   : by(gemm_f32_few_kernel<1, 1, true, 4, 1, 1, false, FOLDS...>, gemm_f32_few_kernel<1, 1, true, 2, 1, 1, false, FOLDS...>,
+                        gemm_f32_few_kernel<1, 1, true, 1, 1, 1, false, FOLDS...>))<<<parts * grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, folds...);
     return;
   }
-  gemm_f32_few_kernel<1, 1, false, 1, 1, 1, false, FOLD><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, fa);
+  gemm_f32_few_kernel<1, 1, false, 1, 1, 1, false, FOLDS...><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, folds...);
 }
 
-template <bool FOLD>
-static void launch_f32_short(const float* x, const float* w, float* c, int m, int n, int k, const F32Fold& fa, hipStream_t s) {
+template <typename... FOLDS>
+static void launch_f32_short(const float* x, const float* w, float* c, int m, int n, int k, hipStream_t s, const FOLDS&... folds) {
+  constexpr bool FOLD = sizeof...(FOLDS) > 0;
   const int n_waves = f32_short_waves(k);
   const size_t lds = ((size_t)(n_waves - 1) * 256 + (FOLD ? n_waves * 16 : 0)) * sizeof(float);
-  gemm_f32_short_kernel<false, FOLD><<<(n + 15) / 16, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, fa);
+  gemm_f32_short_kernel<false, FOLDS...><<<(n + 15) / 16, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, folds...);
 }
 
 // gate and way up, and the gate (rb_gemm_f32_gated_ok)
-template <bool FOLD>
-static void launch_f32_gated(const float* x, const float* w, bool w_frag, float* c, int m, int ff, int k, const F32Fold& fa, hipStream_t s) {
+template <typename... FOLDS>
+static void launch_f32_gated(const float* x, const float* w, bool w_frag, float* c, int m, int ff, int k, hipStream_t s, const FOLDS&... folds) {
+  constexpr bool FOLD = sizeof...(FOLDS) > 0;
   const int grid = ff / 16, n_waves = w_frag ? f32_few_waves(k) : f32_short_waves(k);
   const size_t lds = ((size_t)2 * (n_waves - 1) * 256 + 256 + (FOLD ? 2 * n_waves * 16 : 0)) * sizeof(float);
-  auto kern = !w_frag                          ? gemm_f32_short_kernel<true, FOLD>
-              : 2 * grid <= rb_compute_units() ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2, true, FOLD>      // (8 waves a workgroup: as two workgroups above)
-              : m <= 4                         ? gemm_f32_few_kernel<1, 1, true, 4, 1, 1, true, FOLD>
-              : m <= 8                         ? gemm_f32_few_kernel<1, 1, true, 2, 1, 1, true, FOLD>
-                                               : gemm_f32_few_kernel<1, 1, true, 1, 1, 1, true, FOLD>;
-  kern<<<grid, 2 * 64 * n_waves, lds, s>>>(x, w, c, m, ff, k, fa);
+  auto kern = !w_frag                          ? gemm_f32_short_kernel<true, FOLDS...>
+              : 2 * grid <= rb_compute_units() ? gemm_f32_few_kernel<1, 1, true, 1, 1, 2, true, FOLDS...>      // (8 waves a workgroup: as two workgroups above)
+              : m <= 4                         ? gemm_f32_few_kernel<1, 1, true, 4, 1, 1, true, FOLDS...>
+              : m <= 8                         ? gemm_f32_few_kernel<1, 1, true, 2, 1, 1, true, FOLDS...>
+                                               : gemm_f32_few_kernel<1, 1, true, 1, 1, 1, true, FOLDS...>;
+  kern<<<grid, 2 * 64 * n_waves, lds, s>>>(x, w, c, m, ff, k, folds...);
 }
 
 template <int MB>
@@ -563,15 +586,15 @@ static void launch_f32_few(const float* x, const float* w, bool w_frag, float* c
     if (g_f32_few != 3 && (n + 31) / 32 >= 2 * rb_compute_units()) {
       const size_t lds2 = (size_t)(n_waves - 1) * 2 * MB * 4 * 64 * sizeof(float);
       const int grid2 = (n + 31) / 32;
-      if (w_frag) gemm_f32_few_kernel<MB, 2, true><<<grid2, 64 * n_waves, lds2, s>>>(x, w, c, m, n, k, F32Fold{});
-      else gemm_f32_few_kernel<MB, 2, false><<<grid2, 64 * n_waves, lds2, s>>>(x, w, c, m, n, k, F32Fold{});
+      if (w_frag) gemm_f32_few_kernel<MB, 2, true><<<grid2, 64 * n_waves, lds2, s>>>(x, w, c, m, n, k);
+      else gemm_f32_few_kernel<MB, 2, false><<<grid2, 64 * n_waves, lds2, s>>>(x, w, c, m, n, k);
       return;
     }
   }
   const size_t lds = (size_t)(n_waves - 1) * MB * 4 * 64 * sizeof(float);
   const int grid = (n + 15) / 16;
-  if (w_frag) gemm_f32_few_kernel<MB, 1, true><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, F32Fold{});
-  else gemm_f32_few_kernel<MB, 1, false><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k, F32Fold{});
+  if (w_frag) gemm_f32_few_kernel<MB, 1, true><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
+  else gemm_f32_few_kernel<MB, 1, false><<<grid, 64 * n_waves, lds, s>>>(x, w, c, m, n, k);
 }
 
 // Float32 operands and more than 16 tokens with K a multiple of 16 that is not one of 32, or operands
@@ -703,7 +726,7 @@ extern "C" int rb_gemm_f32_gated(const float* a, const float* w, int w_layout, f
   RB_RECORDED(rb_gemm_f32_gated(a, w, w_layout, c, m, ff, k, stream));
   RB_REQUIRE(m == 0 || rb_gemm_f32_gated_ok(m, ff, k, w_layout), "rb_gemm_f32_gated: M=%d ff=%d K=%d, layout %d are not for it", m, ff, k, w_layout);
   if (m == 0) return 0;
-  launch_f32_gated<false>(a, w, w_layout == 1, c, m, ff, k, F32Fold{}, (hipStream_t)stream);
+  launch_f32_gated(a, w, w_layout == 1, c, m, ff, k, (hipStream_t)stream);
   RB_LAUNCH_CHECK();
   return 0;
 }
@@ -727,9 +750,9 @@ extern "C" int rb_gemm_f32_few(const float* a, const float* squares_in, float ep
   const uintptr_t all = reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(gain) | reinterpret_cast<uintptr_t>(gained);
   const F32Fold fa = {squares_in, rows, eps, epilogue >= 2 ? 1 : 0, gain, gained, squares_out, n % 4 == 0 && (all & 15) == 0 ? 1 : 0};
   hipStream_t s = (hipStream_t)stream;
-  if (epilogue == 1) launch_f32_gated<true>(a, w, w_layout == 1, c, m, n / 2, k, fa, s);
-  else if (k % 128 == 0) launch_f32_16<true>(a, w, w_layout == 1, c, m, n, k, fa, s);
-  else launch_f32_short<true>(a, w, c, m, n, k, fa, s);
+  if (epilogue == 1) launch_f32_gated(a, w, w_layout == 1, c, m, n / 2, k, s, fa);
+  else if (k % 128 == 0) launch_f32_16(a, w, w_layout == 1, c, m, n, k, s, fa);
+  else launch_f32_short(a, w, c, m, n, k, s, fa);
   RB_LAUNCH_CHECK();
   return 0;
 }
@@ -749,14 +772,14 @@ extern "C" int rb_gemm_generic(const void* a, const void* w, int w_layout, void*
     const float* af = (const float*)a;
     const float* wf = (const float*)w;
     const int mb = (m + 15) / 16;
-    if (mb == 1) launch_f32_16<false>(af, wf, w_frag, (float*)c, m, n, k, F32Fold{}, s);
+    if (mb == 1) launch_f32_16(af, wf, w_frag, (float*)c, m, n, k, s);
     else if (mb == 2) launch_f32_few<2>(af, wf, w_frag, (float*)c, m, n, k, s);
     else launch_f32_few<4>(af, wf, w_frag, (float*)c, m, n, k, s);
     RB_LAUNCH_CHECK();
     return 0;
   }
   if (dtype_in == RB_F32 && dtype_out == RB_F32 && f32_short_takes(m, n, k)) {
-    launch_f32_short<false>((const float*)a, (const float*)w, (float*)c, m, n, k, F32Fold{}, s);
+    launch_f32_short((const float*)a, (const float*)w, (float*)c, m, n, k, s);
     RB_LAUNCH_CHECK();
     return 0;
   }
