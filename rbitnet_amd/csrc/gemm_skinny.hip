@@ -97,7 +97,9 @@ __device__ __forceinline__ void store_sums(TO* __restrict__ c, const f32x4_t& su
 //
 // XP: blocks of 32 depth values that a load of the tokens brings (see RowPack in gemm_internal.h).
 // WP: blocks of depth that a load of W brings (one row tile a wave, W fragment-major): a workgroup then has 16 / WP of the tile's rows.
-template <int MB, int R, bool FAST, bool WF, int EPI, typename TO, bool SCALED, int XP, int WP = 1>
+// ASIDE (a block a load): what was loaded is moved out of the way before it is multiplied, so that the next stage's W is asked for while the tokens of this
+// one are waited for.  It costs registers, 2 to 48 a lane; see set_aside for who gains.
+template <int MB, int R, bool FAST, bool WF, int EPI, typename TO, bool SCALED, int XP, int WP = 1, bool ASIDE = false>
 __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restrict__ x,
                                                           const bf16_t* __restrict__ w, TO* __restrict__ c,
                                                           int m, int n, int k, int k_per_wave, FoldArgs fa) {
@@ -206,7 +208,10 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
 #pragma unroll
       for (int rt = 0; rt < R; ++rt)
 #pragma unroll
-        for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = mfma16(RowPack<WP>::block(a[rt], j), RowPack<XP>::block(b[cb], j), acc[rt][cb]);
+        for (int cb = 0; cb < MB; ++cb) {
+          if constexpr (XP == 1 && WP == 1 && !ASIDE) acc[rt][cb] = mfma16(a[rt][j], b[cb][j], acc[rt][cb]);
+          else acc[rt][cb] = mfma16(RowPack<WP>::block(a[rt], j), RowPack<XP>::block(b[cb], j), acc[rt][cb]);
+        }
   };
   if constexpr (FAST) {
     // K and every wave's range are multiples of 128: no bounds checks.  Rows beyond N or M
@@ -368,6 +373,17 @@ static int skinny_parts(int n) {
   return 2 * ((n + 15) / 16) <= rb_compute_units() ? 2 : 1;
 }
 
+// Whether a product of 9 to 16 tokens (fragment-major W, tokens as they are) sets its operands aside: with two row tiles a wave at K > 4096, and with one
+// where the sums are added to C and nothing else.  us without and with, 9 / 16 tokens: 8,192 rows at K = 8192 31.0 / 31.5 and 27.3 / 27.3, with the next norm's
+// rows 30.2 / 30.3 and 27.8 / 27.6; 5,120 at 5120 with those 12.87 / 14.3 and 12.5 / 14.0; the gate, 10,240 at 8192, 31.6 / 32.4 and 30.2 / 31.8; added to C, 4,096 at 14336
+// 22.8 / 25.2 and 19.8 / 23.1, 6,144 at 4096 12.05 / 13.7 and 11.0 / 13.0.  The others lose: 6,144 at 4096 10.7 / 12.7 and 11.2 / 13.4; with the next norm's rows 4,096 at 14336
+// 23.0 / 23.4 and 23.2 / 23.8, 3,072 at 2048 5.3 / 5.6 and 5.4 / 5.8; the gate, 10,304 at 2048, 10.24 and 10.69 (9); four tiles, 16,384 at 8192 with the next norm's rows,
+// 45.3 / 44.5 and 54.5 / 55.3, for which there are not enough registers.  Captured steps of 12 sequences, 8 layers of the 8B shape 823 and 829 us, 5 of
+// the 70B shape 1,700 and 1,669.  (Two whole stages in registers, or W a stage ahead of the tokens, both spelled out: slower than either.)
+constexpr bool set_aside(int r, int epilogue, int k) {
+  return r == 2 ? epilogue != 1 || k > 4096 : r == 1 && epilogue == 2;
+}
+
 template <int MB, int R, bool FAST, int EPI, typename TO, bool SCALED>
 static int launch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const GemmAfter& after, int m, int n, int k,
                          int n_waves, int k_per_wave, hipStream_t s) {
@@ -384,9 +400,11 @@ static int launch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const Ge
     }
   }
   if (MB == 1 && after.w_frag) {
-    constexpr bool MAY = MB == 1 && FAST;
+    constexpr bool MAY = MB == 1 && FAST, MAY_ASIDE = MAY && !SCALED && set_aside(R, EPI, 8192);
+    const bool aside = MAY_ASIDE && set_aside(R, EPI, k);
     (MAY && m <= 4   ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 4 : 1>
      : MAY && m <= 8 ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 2 : 1>
+     : aside         ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, 1, 1, MAY_ASIDE>
                      : gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, 1>)
         <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, k_per_wave, fold_args(x, after, c, n));
   } else
