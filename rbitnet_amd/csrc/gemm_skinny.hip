@@ -348,6 +348,8 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restri
   }
 }
 
+static int skinny_rows(int n, int k, bool pairs);
+
 static int g_tune_parts = 0;
 extern "C" void rb_tune_parts(int parts) { g_tune_parts = parts; }      // experiments and tests only: 1 or 2 workgroups for a tile of 16 rows; 0 = the built-in choice
 static int g_tune_r = 0, g_tune_waves = 0;
@@ -380,8 +382,44 @@ static int skinny_parts(int n) {
 // 23.0 / 23.4 and 23.2 / 23.8, 3,072 at 2048 5.3 / 5.6 and 5.4 / 5.8; the gate, 10,304 at 2048, 10.24 and 10.69 (9); four tiles, 16,384 at 8192 with the next norm's rows,
 // 45.3 / 44.5 and 54.5 / 55.3, for which there are not enough registers.  Captured steps of 12 sequences, 8 layers of the 8B shape 823 and 829 us, 5 of
 // the 70B shape 1,700 and 1,669.  (Two whole stages in registers, or W a stage ahead of the tokens, both spelled out: slower than either.)
-constexpr bool set_aside(int r, int epilogue, int k) {
-  return r == 2 ? epilogue != 1 || k > 4096 : r == 1 && epilogue == 2;
+// (At K < 2048 a wave has no more than four stages: with at most a tile a compute unit there is nothing to gain, 3,584 rows at K = 1024 3.77 and 4.0, 8 tokens.)
+constexpr bool set_aside(int r, int epilogue, int k, bool many) {
+  return r == 2 ? epilogue != 1 || k > 4096 : r == 1 && epilogue == 2 && (k >= 2048 || many);
+}
+
+// Blocks of depth that a load of the tokens brings, where a tile of rows is one workgroup's: as many as there is room for, except
+//  - tokens that a norm prepared: their sums of squares are waited for first, and what is saved behind that seldom makes up for two rows' addresses and the
+//    rotations.  us with a block a load and packed, 4 tokens: 2,048 rows at K = 2048 4.61 and 4.73, 8,192 at 8192 28.4 and 29.4; of gate and way up
+//    8,192 at 8192 28.5 and 29.7, 8,192 at 2048 7.87 and 8.02.  It pays above K = 4096 with more tiles than compute units (5,120 at 5120 1 to 5 %), and for
+//    the gate from K = 3072 on with few tiles (4,096 at 14336 4 %) or, with 5 to 8 tokens, many (57,344 at 8192 2 %);
+//  - rows of 16 KB or a multiple: where workgroups share a compute unit, the few lines of tokens that packed loads ask for lie in too few channels of the
+//    caches (12,288 rows at K = 8192 5 to 7 %; at 7168, 9216 and 10240 nothing is lost);
+//  - four row tiles a wave on nearly every compute unit (15,360 rows at K = 5120 26.2 and 26.7 us; the gate on 192 units, 12,288 at 7168, gains 3 to 5 %);
+//  - 5 to 8 tokens at K < 2048 while the tiles are few (3,072 rows at K = 1024 4 to 5 %) and, with the next norm's rows, while they are many (2 to 3 %).
+// Added to C alone the packed loads gain otherwise, up to 30 %.
+static int packed_blocks(int m, int n, int k, int r, int epilogue, bool scaled) {
+  if (m > 8) return 1;
+  const long long tiles = (n + 15) / 16, cus = rb_compute_units();
+  const bool whole16k = k % 8192 == 0, short_of_eight = m > 4 && k < 2048;
+  bool pays;
+  if (scaled && epilogue == 1)
+    pays = (k >= 3072 && 4 * tiles <= (whole16k ? 3 : k > 4096 ? 5 : 4) * cus) || (m > 4 && k > 4096 && tiles > 2 * cus);
+  else if (scaled)
+    pays = k > 4096 && tiles > (whole16k ? 2 : 1) * cus;
+  else if (epilogue == 2)
+    pays = !(short_of_eight && tiles <= cus);
+  else if (r == 4)
+    pays = epilogue == 3 ? !(whole16k && tiles <= 4 * cus) : epilogue == 1 && tiles <= 3 * cus;
+  else if (epilogue == 3)
+    pays = !(whole16k && r == 1 && tiles > 2 * cus) && !(short_of_eight && tiles > 2 * cus && tiles <= 4 * cus);
+  else
+    pays = !(whole16k && r == 1 && tiles > 2 * cus) && !(short_of_eight && tiles < 2 * cus);
+  return !pays ? 1 : m <= 4 ? 4 : 2;
+}
+
+// For tests: the choice for a fragment-major product, tokens as they are or prepared by a norm
+extern "C" int rb_tune_few_blocks(int m, int n, int k, int epilogue, int prepared) {
+  return k % 128 != 0 || m > 16 ? 1 : packed_blocks(m, n, k, skinny_rows(n, k, epilogue == 1), epilogue, prepared != 0);
 }
 
 template <int MB, int R, bool FAST, int EPI, typename TO, bool SCALED>
@@ -400,12 +438,13 @@ static int launch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const Ge
     }
   }
   if (MB == 1 && after.w_frag) {
-    constexpr bool MAY = MB == 1 && FAST, MAY_ASIDE = MAY && !SCALED && set_aside(R, EPI, 8192);
-    const bool aside = MAY_ASIDE && set_aside(R, EPI, k);
-    (MAY && m <= 4   ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 4 : 1>
-     : MAY && m <= 8 ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 2 : 1>
-     : aside         ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, 1, 1, MAY_ASIDE>
-                     : gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, 1>)
+    constexpr bool MAY = MB == 1 && FAST, MAY_ASIDE = MAY && !SCALED && set_aside(R, EPI, 8192, true);
+    const int blocks = MAY ? packed_blocks(m, n, k, R, EPI, SCALED) : 1;
+    const bool aside = MAY_ASIDE && set_aside(R, EPI, k, grid > rb_compute_units());
+    (blocks == 4   ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 4 : 1>
+     : blocks == 2 ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 2 : 1>
+     : aside       ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, 1, 1, MAY_ASIDE>
+                   : gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, 1>)
         <<<grid, n_waves * 64, lds, s>>>(x.x, w, (TO*)c, m, n, k, k_per_wave, fold_args(x, after, c, n));
   } else
     gemm_skinny_kernel<MB, R, FAST, false, EPI, TO, SCALED, 1>

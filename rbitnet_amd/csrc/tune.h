@@ -10,9 +10,12 @@ extern "C" {
 
 void rb_tune_compute_units(int n);                              // every planner: pretend the GPU has n compute units
 void rb_tune(int rows_per_wave, int waves);                     // skinny product
+void rb_tune_parts(int parts);                                  // skinny product: 1 or 2 workgroups for a tile of 16 rows
+int rb_tune_few_blocks(int m, int n, int k, int epilogue, int prepared);      // skinny product: the built-in choice of blocks of depth a load of the tokens
 void rb_tune_resident(int tiles);                               // skinny product with resident tokens: row tiles per workgroup
 void rb_tune_use_resident(int on);                              // 0: never the resident variant, 2: also below 8192 rows
 void rb_tune_f32_few(int on);                                   // float32 product of few tokens: 0 = on the vector units, not the float32 MFMA; 3 = one row tile a wave always
+void rb_tune_f32_parts(int parts);                              // the same: 1 or 2 workgroups for a tile of 16 rows
 void rb_tune_f32_tile(int tile);                                // float32 product of many tokens: 1..7 = that tile, -1 = tiles staged through registers
 int rb_tune_f32_plan(int m, int n, int k);                      // float32 product of many tokens: the built-in choice, 10 * (tile of a second launch) + tile
 void rb_tune_use_stream(int on);                                // 0: the skinny product up to 64 tokens

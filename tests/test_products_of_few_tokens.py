@@ -1,0 +1,31 @@
+"""Which kernels the products of a step's few tokens go to, over sizes: rules that no result shows, for a GPU of 256 compute units."""
+import ctypes
+
+import pytest
+
+from rbitnet_amd.csrc import build
+
+
+@pytest.fixture(scope="module")
+def lib():
+    lib = ctypes.CDLL(build.ensure_built())
+    lib.rb_tune_compute_units(256)
+    yield lib
+    lib.rb_tune_compute_units(0)
+
+
+# rows, K, end, prepared by a norm -> blocks of depth a load of 4 and of 8 tokens, and what a load of the other kind took longer where that was timed
+@pytest.mark.parametrize("n,k,end,prepared,four,eight", [
+    (3072, 3072, 0, 0, 4, 2), (6144, 4096, 2, 0, 4, 2), (4096, 14336, 3, 0, 4, 2), (8192, 8192, 1, 0, 4, 2),
+    (2048, 2048, 0, 1, 1, 1), (6144, 4096, 0, 1, 1, 1), (8192, 8192, 0, 1, 1, 1),          # 2, 1 and 5 %
+    (5120, 5120, 0, 1, 4, 2), (10240, 8192, 0, 1, 4, 2),                                  # 5 and 1 %
+    (8192, 2048, 1, 1, 1, 1), (8192, 8192, 1, 1, 1, 1), (57344, 8192, 1, 1, 1, 2),         # 2, 5 and 2 %
+    (4096, 4096, 1, 1, 4, 2), (4096, 14336, 1, 1, 4, 2),                                  # 4 and 5 %
+    (12288, 8192, 0, 0, 1, 1), (10240, 8192, 3, 0, 1, 1), (12288, 7168, 0, 0, 4, 2),       # 5, 3 and 4 %
+    (16384, 8192, 3, 0, 1, 1), (16384, 6144, 3, 0, 4, 2), (15360, 5120, 0, 0, 1, 1),       # 4, 1 and 2 %
+    (12288, 6144, 1, 0, 4, 2), (16384, 6144, 1, 0, 1, 1),                                 # 4 and 1 %
+    (3072, 1024, 0, 0, 4, 1), (3072, 1024, 2, 0, 4, 1), (3072, 1024, 1, 0, 4, 1),          # 5, 4 and 4 % (8 tokens)
+])
+def test_tokens_are_packed_where_that_was_the_faster_load(lib, n, k, end, prepared, four, eight):
+    blocks = [lib.rb_tune_few_blocks(m, n, k, end, prepared) for m in (1, 4, 5, 8, 9, 16)]
+    assert blocks == [four, four, eight, eight, 1, 1]
