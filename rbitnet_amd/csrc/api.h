@@ -51,6 +51,7 @@ int rb_gemm_generic(const void* a, const void* w, int w_layout, void* c, int dty
 // c [m, ff] = silu(a Wg^T) * (a Wu^T) in one launch, float32, w [2 ff, k] the gate's rows and then those of the way up (layout as above); the same bits
 // as the product and rb_swiglu.  rb_gemm_f32_gated_ok: whether these sizes are for it (at most 16 tokens).
 int rb_gemm_f32_gated_ok(int m, int ff, int k, int w_layout);
+int rb_gemm_f32_gated_pays(int m, int ff, int k, int w_layout);      // and whether that is faster than the two launches
 int rb_gemm_f32_gated(const float* a, const float* w, int w_layout, float* c, int m, int ff, int k, void* stream);
 
 // C[M, N] = A[M, K] * W[N, K]^T, bfloat16 inputs on the matrix cores.

@@ -722,6 +722,22 @@ extern "C" int rb_gemm_f32_gated_ok(int m, int ff, int k, int w_layout) {
   return w_layout == 0 && k % 128 != 0 && f32_short_takes(m, 2 * ff, k);
 }
 
+// Whether that is also faster than the product and the gate in a launch each.  A compute unit that has one of these workgroups more has two tiles of rows more,
+// where the product alone deals tile by tile (and halves of tiles where there are few): the launch pays where no unit gets more rows for it.
+// us in two launches and in one, 4 tokens: 4,096 units of width 4096 (a tile of 16 a compute unit) 25.3 and 23.7, 8,192 45.8 and 44.1; 1,024 and 2,048 units, on which half of
+// the GPU is idle, 11.4 and 19.5, 14.8 and 20.3; 5,120 (1.25 tiles a unit) 32.9 and 36.0; 14,336 (3.5) with 16 tokens 93.3 and 100.
+// Depths of up to 512 are one trip to memory either way and the launch is what counts (1,024 units of 512 5.6 and 4.6), up to 1024 it still is with up to
+// 8 tokens and more than a tile a unit (6,144 units 12.4 and 11.2); rows (the kernel for short depths) go by the first half of the rule alone (2,048 units of 1000 9.3 and
+// 9.7, 5,120 with 16 tokens 24.5 and 23.1).
+extern "C" int rb_gemm_f32_gated_pays(int m, int ff, int k, int w_layout) {
+  if (!rb_gemm_f32_gated_ok(m, ff, k, w_layout)) return 0;
+  const long long tiles = ff / 16, cus = rb_compute_units();
+  if (k <= 512) return 1;
+  if (2 * tiles <= cus) return 0;
+  if (w_layout == 0 || (k <= 1024 && m <= 8 && tiles > cus)) return 1;
+  return 2 * ((tiles + cus - 1) / cus) == (2 * tiles + cus - 1) / cus;
+}
+
 extern "C" int rb_gemm_f32_gated(const float* a, const float* w, int w_layout, float* c, int m, int ff, int k, void* stream) {
   RB_RECORDED(rb_gemm_f32_gated(a, w, w_layout, c, m, ff, k, stream));
   RB_REQUIRE(m == 0 || rb_gemm_f32_gated_ok(m, ff, k, w_layout), "rb_gemm_f32_gated: M=%d ff=%d K=%d, layout %d are not for it", m, ff, k, w_layout);

@@ -158,6 +158,7 @@ class Kernels:
             "rb_swiglu": [_P, _P, _I, _I, _I, _P],
             "rb_gemm_generic": [_P, _P, _I, _P, _I, _I, _I, _I, _I, _P],
             "rb_gemm_f32_gated_ok": [_I, _I, _I, _I],
+            "rb_gemm_f32_gated_pays": [_I, _I, _I, _I],
             "rb_gemm_f32_gated": [_P, _P, _I, _P, _I, _I, _I, _P],
             "rb_gemm_bf16": [_P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _P],
             "rb_gemm_bf16_act": [_P, _P, _I, _P, _I, _I, _P, _I, _I, _I, _P, _P],
@@ -377,6 +378,9 @@ class Kernels:
 
     def gemm_f32_gated_ok(self, m: int, ff: int, k: int, w_frag: bool) -> bool:
         return bool(self._lib.rb_gemm_f32_gated_ok(m, ff, k, int(bool(w_frag))))
+
+    def gemm_f32_gated_pays(self, m: int, ff: int, k: int, w_frag: bool) -> bool:
+        return bool(self._lib.rb_gemm_f32_gated_pays(m, ff, k, int(bool(w_frag))))
 
     def gemm_f32_gated(self, a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, w_frag: bool = False) -> None:
         """`gemm_generic` with w [2 ff, K] (the gate's rows, then those of the way up) and `swiglu` in one launch (sizes that `gemm_f32_gated_ok`)."""

@@ -212,15 +212,17 @@ def gated_linear(lib, x, w_packed, ff: int, fused: bool, gate: Optional[torch.Te
     out = torch.empty((m, ff), dtype=x.dtype, device=x.device)
     if m == 0:
         return out
+    in_one = x.dtype == torch.float32 and not fused and lib.gemm_f32_gated_pays(m, ff, x.shape[1], _data(w_packed)[1])
     if isinstance(x, GainedRows):
-        if _few(lib, x, w_packed, 1) and (fused or x.dtype == torch.float32):
+        if (fused or in_one) and _few(lib, x, w_packed, 1):
             _from_gained(lib, x, w_packed, out, 1)
             return out
-        x = x.tensor()
+        if fused or in_one:
+            x = x.tensor()
     if fused:
         wd, frag = _data(w_packed)
         lib.gemm_bf16(x, wd, out, 1, w_frag=frag, act=gate)
-    elif x.dtype == torch.float32 and lib.gemm_f32_gated_ok(m, ff, x.shape[1], _data(w_packed)[1]):
+    elif in_one:
         wd, frag = _data(w_packed)
         lib.gemm_f32_gated(x, wd, out, w_frag=frag)
     else:

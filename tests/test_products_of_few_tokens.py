@@ -29,3 +29,16 @@ def lib():
 def test_tokens_are_packed_where_that_was_the_faster_load(lib, n, k, end, prepared, four, eight):
     blocks = [lib.rb_tune_few_blocks(m, n, k, end, prepared) for m in (1, 4, 5, 8, 9, 16)]
     assert blocks == [four, four, eight, eight, 1, 1]
+
+
+# units, K, stored fragment-major -> whether 1, 8, 9 and 16 float32 tokens go through gate, way up and the gate in one launch, and what the other way took longer
+@pytest.mark.parametrize("ff,k,frag,one", [
+    (1024, 512, 1, (1, 1, 1, 1)), (256, 96, 0, (1, 1, 1, 1)), (5120, 500, 0, (0, 0, 1, 1)),            # 22, 50 and 24 % (9 tokens)
+    (1024, 1024, 1, (0, 0, 0, 0)), (1024, 4096, 1, (0, 0, 0, 0)), (2048, 8192, 1, (0, 0, 0, 0)), (2048, 1000, 0, (0, 0, 0, 0)),      # 18, 70, 40 and 4 %
+    (3072, 4096, 1, (1, 1, 1, 1)), (4096, 3072, 1, (1, 1, 1, 1)), (8192, 3072, 1, (1, 1, 1, 1)),       # 12, 9 and 5 %
+    (5120, 3072, 1, (0, 0, 0, 0)), (6144, 8192, 1, (0, 0, 0, 0)), (14336, 4096, 1, (0, 0, 0, 0)),      # 7 to 20, 9 to 20, 0 to 8 %
+    (5120, 1024, 1, (1, 1, 0, 0)), (16384, 4096, 1, (1, 1, 1, 1)),
+])
+def test_the_float32_gate_is_in_its_products_launch_where_no_unit_gets_more_rows(lib, ff, k, frag, one):
+    assert tuple(lib.rb_gemm_f32_gated_pays(m, ff, k, frag) for m in (1, 8, 9, 16)) == one
+    assert lib.rb_gemm_f32_gated_pays(17, ff, k, frag) == 0
