@@ -324,7 +324,9 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_short_kernel(const
 // in registers.  A stage's 32 MFMAs add to one accumulator, 0.4 us one after the other, and behind them the next stage's loads took a trip to memory: with
 // two sets of registers they are under way meanwhile.  Where workgroups share a compute unit they do that for each other, and a wave
 // with more registers is slower (5,120 rows at K = 3072, 4 tokens: 14.9 us with one set, 15.9 with two).
-// U = 0: one set, its loads among the multiplications as the compiler places them; U = 1 keeps a block a load's tokens in front of W (4,096 rows at K = 4096, a workgroup
+// U = 0: one set as well, a stage's loads behind the multiplications of the one before, without FOLD in statements of its own: through the arrays and functions of the others, which say
+// the same, the compiler asks for one load of W in front of the tokens, and 200 to 256 tiles of rows took 2 to 5 % more (4,096 rows at K = 4096, 16 tokens, 14.1 and 14.8 us); with
+// barriers that fix the order of the loads 3 to 15 % more.  U = 1 keeps a block a load's tokens in front of W (4,096 rows at K = 4096, a workgroup
 // a compute unit, 4 / 12 tokens: 12.5 / 13.4 us with U = 0, 14.7 / 14.8 with 1; 28,672 rows, 12 / 16 tokens: 89 / 96 and 78 / 88).
 // GATED: as in the kernel above.
 // FOLD: see F32Fold.
@@ -389,77 +391,100 @@ __global__ __launch_bounds__(GATED ? 512 : 256) void gemm_f32_few_kernel(const f
   const int total = k / 128, base = total / n_waves, extra = total % n_waves;
   const int stages = base + (wave < extra ? 1 : 0);
   const int k_begin = 128 * (wave * base + (wave < extra ? wave : extra));
-  static_assert(U == 1 || (MB == 1 && R == 1), "two stages in registers: one tile of tokens and of rows");
-  gf_f32x4_t as[U == 2 ? 2 : 1][R][8 / WP], bs[U == 2 ? 2 : 1][MB][8 / XP];
-  auto load_stage = [&](int u, int st) __attribute__((always_inline)) {
-    auto &a = as[u];
-    auto &b = bs[u];
-    const int ks = k_begin + 128 * st;
-    if constexpr (MB == 1 && U < 2 && XP == 1) {           // the tokens, which the caches hold, in front of W
+  static_assert(U == 1 || (MB == 1 && R == 1 && WF), "no or two stages ahead: one tile of tokens and of rows, fragment-major");
+  float ss = 0.f;
+  if constexpr (U == 0 && !FOLD) {
+    gf_f32x4_t a[R][8], b[MB][8];
+    auto load_stage = [&](int st) {
+      const int ks = k_begin + 128 * st;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[0][j] = __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4_t*>(wrow[0] + (size_t)(ks + 16 * j) * WK));
 #pragma unroll
       for (int j = 0; j < 8; ++j) b[0][j] = *reinterpret_cast<const gf_f32x4_t*>(xrow[0] + ks + 16 * j);
-      if constexpr (U == 1) __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply_stage = [&]() {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0][j][i], b[0][j][i], acc[0][0], 0, 0, 0);
+    };
+    load_stage(0);
+    for (int st = 1; st < stages; ++st) {
+      multiply_stage();
+      load_stage(st);
     }
+    multiply_stage();
+  } else {
+    gf_f32x4_t as[U == 2 ? 2 : 1][R][8 / WP], bs[U == 2 ? 2 : 1][MB][8 / XP];
+    auto load_stage = [&](int u, int st) __attribute__((always_inline)) {
+      auto &a = as[u];
+      auto &b = bs[u];
+      const int ks = k_begin + 128 * st;
+      if constexpr (MB == 1 && U < 2 && XP == 1) {           // the tokens, which the caches hold, in front of W
 #pragma unroll
-    for (int j = 0; j < 8 / WP; ++j)
+        for (int j = 0; j < 8; ++j) b[0][j] = *reinterpret_cast<const gf_f32x4_t*>(xrow[0] + ks + 16 * j);
+        if constexpr (U == 1) __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
-      for (int rt = 0; rt < R; ++rt)
-        a[rt][j] = WF ? __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + (size_t)(ks + 16 * WP * j) * WK))
-                      : *reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + ks + 16 * WP * j);
-    if constexpr (MB == 1 && U < 2 && XP == 1) return;
-#pragma unroll
-    for (int j = 0; j < 8 / XP; ++j)
-#pragma unroll
-      for (int cb = 0; cb < MB; ++cb) b[cb][j] = *reinterpret_cast<const gf_f32x4_t*>(xrow[cb] + ks + 16 * XP * j);
-  };
-  auto multiply_stage = [&](int u) __attribute__((always_inline)) {
-    auto &a = as[u];
-    auto &b = bs[u];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      gf_f32x4_t aj[R], bj[MB];
-#pragma unroll
-      for (int rt = 0; rt < R; ++rt) aj[rt] = RowPack<WP>::turned(a[rt][j / WP], j % WP);
-#pragma unroll
-      for (int cb = 0; cb < MB; ++cb) bj[cb] = RowPack<XP>::turned(b[cb][j / XP], j % XP);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int j = 0; j < 8 / WP; ++j)
 #pragma unroll
         for (int rt = 0; rt < R; ++rt)
+          a[rt][j] = WF ? __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + (size_t)(ks + 16 * WP * j) * WK))
+                        : *reinterpret_cast<const gf_f32x4_t*>(wrow[rt] + ks + 16 * WP * j);
+      if constexpr (MB == 1 && U < 2 && XP == 1) return;
 #pragma unroll
-          for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aj[rt][i], bj[cb][i], acc[rt][cb], 0, 0, 0);
+      for (int j = 0; j < 8 / XP; ++j)
+#pragma unroll
+        for (int cb = 0; cb < MB; ++cb) b[cb][j] = *reinterpret_cast<const gf_f32x4_t*>(xrow[cb] + ks + 16 * XP * j);
+    };
+    auto multiply_stage = [&](int u) __attribute__((always_inline)) {
+      auto &a = as[u];
+      auto &b = bs[u];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        gf_f32x4_t aj[R], bj[MB];
+#pragma unroll
+        for (int rt = 0; rt < R; ++rt) aj[rt] = RowPack<WP>::turned(a[rt][j / WP], j % WP);
+#pragma unroll
+        for (int cb = 0; cb < MB; ++cb) bj[cb] = RowPack<XP>::turned(b[cb][j / XP], j % XP);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int rt = 0; rt < R; ++rt)
+#pragma unroll
+            for (int cb = 0; cb < MB; ++cb) acc[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aj[rt][i], bj[cb][i], acc[rt][cb], 0, 0, 0);
+      }
+    };
+    load_stage(0, 0);
+    if (FOLD) {                          // the squares were asked for before the first stage and are added up before it arrives
+      __builtin_amdgcn_sched_barrier(0);
+      if (fa.squares_in) ss = squares_sum(asked);
     }
-  };
-  load_stage(0, 0);
-  float ss = 0.f;
-  if (FOLD) {                          // the squares were asked for before the first stage and are added up before it arrives
-    __builtin_amdgcn_sched_barrier(0);
-    if (fa.squares_in) ss = squares_sum(asked);
-  }
-  if constexpr (U == 2) {
-    int st = 0;
-    for (; st + 2 < stages; st += 2) {
-      load_stage(1, st + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply_stage(0);
-      load_stage(0, st + 2);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply_stage(1);
-    }
-    if (st + 1 < stages) {
-      load_stage(1, st + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply_stage(0);
-      multiply_stage(1);
+    if constexpr (U == 2) {
+      int st = 0;
+      for (; st + 2 < stages; st += 2) {
+        load_stage(1, st + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply_stage(0);
+        load_stage(0, st + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply_stage(1);
+      }
+      if (st + 1 < stages) {
+        load_stage(1, st + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply_stage(0);
+        multiply_stage(1);
+      } else {
+        multiply_stage(0);
+      }
     } else {
+      for (int st = 1; st < stages; ++st) {
+        multiply_stage(0);
+        load_stage(0, st);
+      }
       multiply_stage(0);
     }
-  } else {
-    for (int st = 1; st < stages; ++st) {
-      multiply_stage(0);
-      load_stage(0, st);
-    }
-    multiply_stage(0);
   }
 
   if (FOLD && fa.squares_in) ss = squares_meet(ss, sq_lds, wave, lane);
@@ -526,6 +551,16 @@ static bool f32_short_takes(int m, int n, int k) {
   return m <= 16 && k % 4 == 0 && k <= 1024 && (k <= 128 || m > 8 || (long long)n * k <= 1 << 22) && g_f32_few;
 }
 
+// Whether a second stage under way pays where every tile has a workgroup (fragment-major W, at most a tile a compute unit): up to three tiles for four units and 12
+// tokens, up to seven for eight and 8 tokens.  us without and with, of 256 units: 176 tiles, K = 4096, 4 / 8 / 12 / 13 tokens 11.5 / 12.0 / 12.5 / 12.6 and 10.3 / 11.3 / 12.5 / 12.9;
+// 200 tiles 11.7 / 12.0 / 12.7 and 10.9 / 11.7 / 12.8; 224 11.8 / 12.3 / 12.7 and 11.6 / 12.1 / 13.4, K = 8192 22.3 / 22.9 / 23.4 and 21.2 / 22.2 / 24.1; 240 12.1 / 12.4 and 12.2 / 12.4; 256
+// 12.6 / 12.7 and 13.1 / 13.1.
+static bool f32_few_ahead(int m, int n) {
+  const long long tiles = (n + 15) / 16, cus = rb_compute_units();
+  return m <= 8 ? 8 * tiles <= 7 * cus : m <= 12 && 4 * tiles <= 3 * cus;
+}
+extern "C" int rb_tune_f32_ahead(int m, int n) { return f32_few_ahead(m, n); }      // for tests: the choice
+
 // At most 16 tokens: one tile of them
 template <typename... FOLDS>
 static void launch_f32_16(const float* x, const float* w, bool w_frag, float* c, int m, int n, int k, hipStream_t s, const FOLDS&... folds) {
@@ -535,10 +570,8 @@ static void launch_f32_16(const float* x, const float* w, bool w_frag, float* c,
   // us, 4 tokens, as the kernel was (one stage, a block a load, whole tiles) and so: 3,072 rows at K = 3072 9.75 and 8.8, at 8192 24.3 and 21.3; 2,048 at 2048
   // 7.2 and 5.9, 1,024 at 4096 10.8 and 8.3 (halves of tiles); more workgroups than compute units: 5,120 at 3072 17.4 and 14.9, 16,384 38.0 and 35.0,
   // 128,256 260 and 239, 6,144 at 4096 23.4 and 20.7.  Halves of more tiles than half the units lose (3,072 rows at 3072 11.9).
-  // A second stage under way pays up to three tiles for four units and 12 tokens: with a tile a unit, 4,096 rows at K = 4096, 4 / 8 / 12 / 16 tokens, 12.6 / 12.6 /
-  // 12.9 / 13.6 without it and 13.1 / 13.4 / 14.3 / 15.4 with it; 3,072 rows at K = 8192 22.2 / 22.5 / 23.3 / 24.6 and 20.1 / 21.3 / 23.4 / 25.5.
   if (w_frag) {
-    const bool ahead = 4 * grid <= 3 * rb_compute_units() && m <= 12;
+    const bool ahead = f32_few_ahead(m, n);
     const int cus = rb_compute_units(), parts = g_f32_parts ? g_f32_parts : 2 * grid <= cus ? 2 : 1, pack = m <= 4 ? 4 : m <= 8 ? 2 : 1;
     auto by = [&](auto four, auto two, auto one) { return pack == 4 ? four : pack == 2 ? two : one; };
     (parts == 2    ? by(gemm_f32_few_kernel<1, 1, true, 4, 2, 2, false, FOLDS...>, gemm_f32_few_kernel<1, 1, true, 2, 2, 2, false, FOLDS...>,

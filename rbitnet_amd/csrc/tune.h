@@ -16,6 +16,7 @@ void rb_tune_resident(int tiles);                               // skinny produc
 void rb_tune_use_resident(int on);                              // 0: never the resident variant, 2: also below 8192 rows
 void rb_tune_f32_few(int on);                                   // float32 product of few tokens: 0 = on the vector units, not the float32 MFMA; 3 = one row tile a wave always
 void rb_tune_f32_parts(int parts);                              // the same: 1 or 2 workgroups for a tile of 16 rows
+int rb_tune_f32_ahead(int m, int n);                            // the same: the built-in choice, 1 = a second stage in registers
 void rb_tune_f32_tile(int tile);                                // float32 product of many tokens: 1..7 = that tile, -1 = tiles staged through registers
 int rb_tune_f32_plan(int m, int n, int k);                      // float32 product of many tokens: the built-in choice, 10 * (tile of a second launch) + tile
 void rb_tune_use_stream(int on);                                // 0: the skinny product up to 64 tokens

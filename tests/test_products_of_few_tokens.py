@@ -42,3 +42,10 @@ def test_tokens_are_packed_where_that_was_the_faster_load(lib, n, k, end, prepar
 def test_the_float32_gate_is_in_its_products_launch_where_no_unit_gets_more_rows(lib, ff, k, frag, one):
     assert tuple(lib.rb_gemm_f32_gated_pays(m, ff, k, frag) for m in (1, 8, 9, 16)) == one
     assert lib.rb_gemm_f32_gated_pays(17, ff, k, frag) == 0
+
+
+def test_a_second_float32_stage_is_under_way_where_that_was_the_faster(lib):
+    """By tiles of 16 rows: up to which number of tokens (3 to 11 % at 200 tiles and 1 to 6 % at 224 with up to 8; 240 and 256 gain nothing)."""
+    for tiles, most in ((1, 12), (136, 12), (192, 12), (200, 8), (208, 8), (224, 8), (225, 0), (240, 0), (256, 0), (1024, 0)):
+        for n in (16 * tiles, 16 * tiles - 15):
+            assert [m for m in range(1, 17) if lib.rb_tune_f32_ahead(m, n)] == list(range(1, most + 1)), tiles
