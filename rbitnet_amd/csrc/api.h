@@ -103,6 +103,7 @@ int rb_gemm_bf16_few(const void* a, const float* squares_in, float eps, const in
 // The same in float32 (W rows, or fragment-major as rb_gemm_generic takes it).  Sums of squares over every 8 columns: squares_in [*, ceil(K / 8)],
 // squares_out [M, ceil(N / 8)]; gained float32.  epilogue 1: W has the gate's N / 2 rows and then those of the way up, C [M, N / 2].
 int rb_gemm_f32_few_ok(int m, int n, int k, int w_layout, int epilogue);
+int rb_gemm_f32_fold_pays(int m, int width);      // whether a norm of rows of so many columns between two such products is faster that way than as a launch
 int rb_gemm_f32_few(const float* a, const float* squares_in, float eps, const int32_t* rows, const float* w, int w_layout, float* c, int epilogue,
                     const float* gain, float* gained, float* squares_out, int m, int n, int k, void* stream);
 

@@ -788,6 +788,13 @@ extern "C" int rb_gemm_f32_few_ok(int m, int n, int k, int w_layout, int epilogu
   return w_layout == 0 && (k % 128 == 0 || f32_short_takes(m, n, k));
 }
 
+// Whether a norm of rows of `width` is better done by the products around it than by a launch of its own: every workgroup of a product behind it reads all the sums
+// of squares, which at more than 8 tokens or 3,072 columns takes longer than the launch.  Captured steps with launches and without, 1 / 4 / 8 / 9 / 16 sequences: width
+// 2,048, 16 layers, 1,316 / 1,294 / 1,318 / 1,447 / 1,577 and 1,309 / 1,278 / 1,289 / 1,425 / 1,558 us; 3,072, 12 layers, 1,393 / 1,411 / 1,474 / 1,641 / 1,783 and 1,362 / 1,380 / 1,461 / 1,649 / 1,805; 4,096, 8
+// layers, two shapes, 1,421 / 1,432 / 1,463 / 1,580 / 1,743 and 1,432 / 1,418 / 1,454 / 1,628 / 1,784, 1,402 / 1,368 / 1,413 / 1,594 / 1,736 and 1,415 / 1,377 / 1,423 / 1,627 / 1,769; 5,120, 6
+// layers, 1,594 / 1,559 / 1,724 / 1,921 / 2,122 and 1,596 / 1,571 / 1,762 / 2,036 / 2,261.
+extern "C" int rb_gemm_f32_fold_pays(int m, int width) { return m >= 1 && m <= 16 && width <= (m <= 8 ? 3072 : 2048); }
+
 extern "C" int rb_gemm_f32_few(const float* a, const float* squares_in, float eps, const int32_t* rows, const float* w, int w_layout, float* c,
                                int epilogue, const float* gain, float* gained, float* squares_out, int m, int n, int k, void* stream) {
   RB_RECORDED(rb_gemm_f32_few(a, squares_in, eps, rows, w, w_layout, c, epilogue, gain, gained, squares_out, m, n, k, stream));

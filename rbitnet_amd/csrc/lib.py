@@ -165,6 +165,7 @@ class Kernels:
             "rb_gemm_bf16_few": [_P, _P, _F, _P, _P, _I, _P, _I, _I, _P, _P, _P, _I, _I, _I, _P],
             "rb_gemm_bf16_few_ok": [_I, _I, _I],
             "rb_gemm_f32_few_ok": [_I, _I, _I, _I, _I],
+            "rb_gemm_f32_fold_pays": [_I, _I],
             "rb_gemm_f32_few": [_P, _P, _F, _P, _P, _I, _P, _I, _P, _P, _P, _I, _I, _I, _P],
             "rb_gemm_bf16_terms_count": [_I, _I, _I],
             "rb_gemm_bf16_terms": [_P, _P, _I, _P, _I, _I, _I, _P],
@@ -393,6 +394,9 @@ class Kernels:
 
     def gemm_f32_few_ok(self, m: int, n: int, k: int, w_frag: bool, epilogue: int) -> bool:
         return bool(self._lib.rb_gemm_f32_few_ok(int(m), int(n), int(k), int(bool(w_frag)), int(epilogue)))
+
+    def gemm_f32_fold_pays(self, m: int, width: int) -> bool:
+        return bool(self._lib.rb_gemm_f32_fold_pays(int(m), int(width)))
 
     def gemm_f32_few(self, a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, epilogue: int = 0, squares: Optional[torch.Tensor] = None,
                      eps: float = 0.0, rows: Optional[torch.Tensor] = None, gain: Optional[torch.Tensor] = None,

@@ -154,7 +154,10 @@ def linear_to_stream(lib, x: torch.Tensor, w, stream: Optional[torch.Tensor], ne
     the product is added, and what comes back is None, or, if the norm that follows folds into
     products, the `GainedRows` for it."""
     wd, frag = _data(w)
-    if stream is None or x.shape[0] == 0 or not _few(lib, x, w, 2):
+    folds = stream is not None and x.shape[0] > 0 and _few(lib, x, w, 2)
+    if folds and x.dtype == torch.float32:
+        folds = lib.gemm_f32_fold_pays(x.shape[0], w.shape[0])
+    if not folds:
         m, k = x.shape
         if (norm_adds_terms(next_norm) and uses_matrix_cores(x.dtype, k)
                 and lib.gemm_bf16_terms_count(m, w.shape[0], k) > 1):

@@ -49,3 +49,8 @@ def test_a_second_float32_stage_is_under_way_where_that_was_the_faster(lib):
     for tiles, most in ((1, 12), (136, 12), (192, 12), (200, 8), (208, 8), (224, 8), (225, 0), (240, 0), (256, 0), (1024, 0)):
         for n in (16 * tiles, 16 * tiles - 15):
             assert [m for m in range(1, 17) if lib.rb_tune_f32_ahead(m, n)] == list(range(1, most + 1)), tiles
+
+
+def test_a_float32_norm_is_left_to_its_products_where_that_was_the_faster(lib):
+    for width, most in ((96, 16), (2048, 16), (2052, 8), (3072, 8), (3076, 0), (4096, 0), (5120, 0)):
+        assert [m for m in range(0, 18) if lib.rb_gemm_f32_fold_pays(m, width)] == list(range(1, most + 1)), width
