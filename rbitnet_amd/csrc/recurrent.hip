@@ -754,10 +754,14 @@ static int launch_delta_rule(const float* q, const float* k, size_t qk_stride, c
   const bool wide = MAY && dim % 4 == 0 && qk_stride % 4 == 0 && aligned(q) && aligned(k) && (ONE_G || (g_stride % 4 == 0 && aligned(g))) &&
                     (qk_stride | v_stride | (ONE_G ? 0 : g_stride)) < (1u << 24);      // (a chunk's places are offsets of 32 bits)
   const int cols = RB_WAVE / RG * (wide ? P : 1), parts = (vdim + cols - 1) / cols;
-  RB_REQUIRE((long long)n_seqs * n_heads * parts <= 0x7fffffffLL, "rb_linear_recurrence: too many sequences, heads and value channels");
-  const int grid = n_seqs * n_heads * parts;
-  (wide ? delta_rule_kernel<DKL, RG, MAY ? P : 1, CH, MODE, ONE_G, MAY> : delta_rule_kernel<DKL, RG, 1, CH, MODE, ONE_G, false>)<<<grid, RB_WAVE, 0, s>>>(
-      q, k, qk_stride, v, v_stride, g, g_stride, beta, state, cu_seqlens, slots, out, n_heads, n_kv, dim, vdim, parts, bonus, sel);
+  // a launch has fewer than 2^32 threads: more sequences than that go in several
+  const long long most = 0xffffffffLL / RB_WAVE / ((long long)n_heads * parts);
+  RB_REQUIRE(most > 0, "rb_linear_recurrence: too many heads and value channels");
+  for (long long b0 = 0; b0 < n_seqs; b0 += most) {
+    const int grid = (int)((n_seqs - b0 < most ? n_seqs - b0 : most) * n_heads * parts);
+    (wide ? delta_rule_kernel<DKL, RG, MAY ? P : 1, CH, MODE, ONE_G, MAY> : delta_rule_kernel<DKL, RG, 1, CH, MODE, ONE_G, false>)<<<grid, RB_WAVE, 0, s>>>(
+        q, k, qk_stride, v, v_stride, g, g_stride, beta, state, cu_seqlens + b0, slots + b0, out, n_heads, n_kv, dim, vdim, parts, bonus, sel);
+  }
   RB_LAUNCH_CHECK();
   return 0;
 }

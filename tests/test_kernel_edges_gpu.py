@@ -1362,6 +1362,24 @@ def test_recurrences_of_whole_and_partial_chunks_with_one_and_two_columns_a_lane
         _within(got.view(ref.shape), ref, 1e-5 * float(ref.abs().max()))
 
 
+def test_a_recurrence_of_more_workgroups_than_a_launch_takes(lib):
+    """A launch has fewer than 2^32 threads, here a wave a (sequence, head).  States of one number, against the rule in float64: the state is off by two roundings of
+    numbers up to 5, and what is read by those of g S q (2 and 2), of k q times v (8) and of the sum (10), 2^-24 of each."""
+    seqs, heads = 16400, 4096
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    qkv = torch.randn(seqs, 2 + heads, generator=gen, device=DEV).clamp_(-2.0, 2.0)
+    g = torch.rand(seqs, heads, generator=gen, device=DEV)
+    state = torch.rand(seqs, heads, 1, 1, generator=gen, device=DEV)
+    out = torch.empty(seqs, heads, device=DEV)
+    ctx = SimpleNamespace(n_tokens=seqs, n_seqs=seqs, slots=torch.arange(seqs, dtype=torch.int32, device=DEV),
+                          cu_seqlens=torch.arange(seqs + 1, dtype=torch.int32, device=DEV))
+    kept = state.clone()
+    lib.linear_recurrence(qkv, 1, 1, heads, 1, g, 0, True, None, state, ctx, out)
+    want = g.double() * kept.view(seqs, heads) + qkv[:, 1:2].double() * qkv[:, 2:]
+    assert float((state.view(seqs, heads) - want).abs().max()) <= 10 * 2.0 ** -24
+    assert float((out - want * qkv[:, :1]).abs().max()) <= 22 * 2.0 ** -24
+
+
 # ---------------------------------------------------------------------------- the router's product and the choice in one launch
 @pytest.mark.parametrize("n", [1, 3, 16])
 @pytest.mark.parametrize("rows,outputs,experts,top,k", [(16, 16, 16, 4, 2048), (17, 16, 16, 2, 1024), (8, 8, 8, 8, 1152), (64, 64, 64, 6, 1280),
