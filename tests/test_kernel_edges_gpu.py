@@ -1362,6 +1362,77 @@ def test_recurrences_of_whole_and_partial_chunks_with_one_and_two_columns_a_lane
         _within(got.view(ref.shape), ref, 1e-5 * float(ref.abs().max()))
 
 
+@pytest.mark.parametrize("dim,vdim", [(64, 12), (64, 36), (128, 24), (128, 33), (96, 36)])
+@pytest.mark.parametrize("kind", ["bonus", "silu", "selective"])
+def test_other_recurrences_of_whole_and_partial_chunks_with_one_and_two_columns_a_lane(lib, dim, vdim, kind):
+    """As above for time mixing, silu on the inputs and the selective scan, against the equations in float64.  Sums: as above.  A decay made in float32 is off by a few
+    2^-24 of itself and what it multiplies shrinks by it, so that a state that has forgotten half of a value after 14 tokens (x = 0.05) is off by
+    2 / x of these: 5e-6."""
+    gen = torch.Generator().manual_seed(dim + vdim)
+    heads, lengths, cuts = 4, [1, 15, 16, 17, 31, 32, 33, 50], [1, 7, 16, 1, 16, 31, 17, 33]
+    n, cu = sum(lengths), [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    kv = 2 if kind == "selective" else heads
+    q, k = (torch.nn.functional.normalize(torch.randn(n, kv, dim, generator=gen), dim=-1) * (3.0 if kind == "silu" else 1.0) for _ in range(2))
+    v, start = torch.randn(n, heads, vdim, generator=gen), torch.randn(len(lengths), heads, vdim, dim, generator=gen) * 0.3
+    g, u = 0.5 + 0.5 * torch.rand(n, heads, dim, generator=gen), torch.randn(heads, dim, generator=gen)
+    constant = 0.5 + 0.45 * torch.rand(heads, generator=gen)
+    dt, dt_bias, a_log, d = (torch.randn(*shape, generator=gen) for shape in ((n, heads), (heads,), (heads,), (heads,)))
+
+    def run(units, steps):
+        state, out = start.to(DEV), torch.full((n, heads * vdim), float("nan"), device=DEV)
+        try:
+            lib._lib.rb_tune_compute_units(units)
+            for spans in steps:
+                pick = torch.cat([torch.arange(cu[b] + lo, cu[b] + hi) for b, (lo, hi) in enumerate(spans)])
+                seqs = [hi - lo for lo, hi in spans]
+                ctx = SimpleNamespace(n_tokens=len(pick), n_seqs=len(seqs), slots=torch.arange(len(seqs), dtype=torch.int32, device=DEV),
+                                      cu_seqlens=torch.tensor([sum(seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32, device=DEV))
+                rows = lambda *ts: torch.cat([t[pick].reshape(len(pick), -1) for t in ts], 1).to(DEV)
+                part = torch.full((len(pick), heads * vdim), float("nan"), device=DEV)
+                if kind == "bonus":
+                    lib.time_mix_recurrence(rows(q), rows(k), rows(v), rows(g), u.to(DEV), state, ctx, part, heads, dim, vdim)
+                elif kind == "silu":
+                    lib.lightning_recurrence(rows(q, k, v), dim, heads, vdim, constant.to(DEV), state, ctx, part)
+                else:
+                    lib.selective_scan(rows(v, k, q), dim, kv, heads, vdim, rows(dt), 0, dt_bias.to(DEV), a_log.to(DEV), d.to(DEV), state, ctx, part)
+                out[pick.to(DEV)] = part
+        finally:
+            lib._lib.rb_tune_compute_units(0)
+        return out, state
+
+    whole = [[(0, m) for m in lengths]]
+    waves = lambda cols: len(lengths) * heads * -(-vdim // cols)
+    between = (waves(16) + waves(8)) // 2 // 4               # four SIMDs a compute unit
+    assert waves(16) < 4 * between <= waves(8) < 4 * 256
+    out, state = run(1, whole)
+    for other in (run(between, whole), run(1, [[(0, c) for c in cuts], [(c, m) for c, m in zip(cuts, lengths)]])):
+        assert torch.equal(out, other[0]) and torch.equal(state, other[1])
+    want, wanted = torch.empty(n, heads, vdim, dtype=torch.float64), start.double().clone()
+    silu = torch.nn.functional.silu
+    for b, m in enumerate(lengths):
+        s = wanted[b]                                          # [H, vdim, dim]
+        for t in range(cu[b], cu[b] + m):
+            qq, kk = (x[t].double().repeat_interleave(heads // kv, 0)[:, None] for x in (q, k))
+            vv = v[t].double()
+            if kind == "bonus":
+                write = vv[..., None] * kk
+                want[t] = ((s + u.double()[:, None] * write) * qq).sum(-1)
+                s *= g[t].double()[:, None]
+                s += write
+            elif kind == "silu":
+                s *= constant.double()[:, None, None]
+                s += silu(vv)[..., None] * silu(kk)
+                want[t] = (s * silu(qq)).sum(-1)
+            else:
+                step = torch.nn.functional.softplus(dt[t].double() + dt_bias.double())
+                s *= torch.exp(-torch.exp(a_log.double()) * step)[:, None, None]
+                s += (step[:, None] * vv)[..., None] * kk
+                want[t] = (s * qq).sum(-1) + d.double()[:, None] * vv
+    more_lanes = run(0, whole)
+    for got, ref in ((out, want), (state, wanted), (more_lanes[0], want), (more_lanes[1], wanted)):
+        _within(got.view(ref.shape), ref, 1e-5 * float(ref.abs().max()))
+
+
 def test_a_recurrence_of_more_workgroups_than_a_launch_takes(lib):
     """A launch has fewer than 2^32 threads, here a wave a (sequence, head).  States of one number, against the rule in float64: the state is off by two roundings of
     numbers up to 5, and what is read by those of g S q (2 and 2), of k q times v (8) and of the sum (10), 2^-24 of each."""
