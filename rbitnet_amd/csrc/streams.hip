@@ -17,7 +17,7 @@
 // src = rows ? rows[r] : r.  With one stream, a delta and no rows the sum is written back to x (the residual sum of
 // a plain pre-norm layer).  coef null: every coefficient is 1.  bias null: none.  The row is held in LDS between
 // the passes: mean first, then the squared deviations.
-template <typename TO>
+template <typename TO, bool TERMS>
 __global__ void streams_layernorm_kernel(float* __restrict__ x, int n_streams, size_t stream_stride,
                                          const float* __restrict__ coef, const float* __restrict__ delta,
                                          const float* __restrict__ weight, const float* __restrict__ bias, float eps,
@@ -61,8 +61,8 @@ __global__ void streams_layernorm_kernel(float* __restrict__ x, int n_streams, s
     if (delta) {
       float d = delta[src * width + j];
       if (delta2) {
-        float e = delta2[src * terms2 * width + j];
-        for (int k = 1; k < terms2; ++k) e += delta2[(src * terms2 + k) * width + j];
+        float e = delta2[TERMS ? src * terms2 * width + j : src * width + j];
+        for (int k = 1; TERMS && k < terms2; ++k) e += delta2[(src * terms2 + k) * width + j];
         d += e;
       }
       v = fmaf(dscale, d, v);
@@ -110,7 +110,9 @@ struct StreamConv {
   float* state;                // [slots, KEEP, width]
   const int32_t* slots;        // row r's
 };
-template <typename TO, int NS, bool ONE, int KEEP = 0>
+// TERMS: delta2 is terms2 terms a row, added up in their order first (else one).  The loop over them cost norms that have none 2 to 5 % up to width 4,096 and 5 to 8 beyond
+// (4 rows of 8,192 with two terms 9.0 and 9.85 us).
+template <typename TO, int NS, bool ONE, int KEEP = 0, bool TERMS = false>
 __global__ __launch_bounds__(1024) void streams_layernorm_vec_kernel(
     float* __restrict__ x, int n_copies, size_t stream_stride, const float* __restrict__ coef, const float* __restrict__ delta,
     const float* __restrict__ weight, const float* __restrict__ bias, float eps, const int32_t* __restrict__ rows, int width,
@@ -156,18 +158,21 @@ __global__ __launch_bounds__(1024) void streams_layernorm_vec_kernel(
     if (delta) {
       float4 d = ld4(delta + src * width + j);
       if (delta2) {
-        // in their order, four on their way at a time
-        const float* at = delta2 + src * terms2 * width + j;
         float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int k = 0; k < terms2; k += 4) {
-          float4 q[4];
+        if constexpr (TERMS) {                              // four on their way at a time
+          const float* at = delta2 + src * terms2 * width + j;
+          for (int k = 0; k < terms2; k += 4) {
+            float4 q[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (i == 0 || k + i < terms2) q[i] = ld4(at + (size_t)(k + i) * width);
+            for (int i = 0; i < 4; ++i)
+              if (i == 0 || k + i < terms2) q[i] = ld4(at + (size_t)(k + i) * width);
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (k + i == 0) e = q[i];
-            else if (k + i < terms2) e = make_float4(e.x + q[i].x, e.y + q[i].y, e.z + q[i].z, e.w + q[i].w);
+            for (int i = 0; i < 4; ++i)
+              if (k + i == 0) e = q[i];
+              else if (k + i < terms2) e = make_float4(e.x + q[i].x, e.y + q[i].y, e.z + q[i].z, e.w + q[i].w);
+          }
+        } else {
+          e = ld4(delta2 + src * width + j);
         }
         d = make_float4(d.x + e.x, d.y + e.y, d.z + e.z, d.w + e.w);
       }
@@ -342,42 +347,45 @@ static int layernorm_launch(float* x, int n_streams, long long stream_stride, co
       aligned(y) && aligned(scale) && (out_dtype == RB_F32 || out_dtype == RB_BF16)) {
     int threads = ((width / 4 + RB_WAVE - 1) / RB_WAVE) * RB_WAVE;
     if (threads > 1024) threads = 1024;
-#define ST_CONV(TO, NS, ONE, KEEP)                                                                                                                  \
-  streams_layernorm_vec_kernel<TO, NS, ONE, KEEP><<<n_rows, threads, (ONE) ? 0 : lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight,  \
-                                                                                          bias, eps, rows, width, (TO*)out, mix, out_coef, y, scale, \
-                                                                                          delta2, dscale, terms2, conv)
-#define ST_GO(TO, NS, ONE) ST_CONV(TO, NS, ONE, 0)
-#define ST_BY_TAPS(TO, NS)                        \
-  do {                                            \
-    if (taps == 2) ST_CONV(TO, NS, true, 1);      \
-    else if (taps == 3) ST_CONV(TO, NS, true, 2); \
-    else ST_CONV(TO, NS, true, 3);                \
-  } while (0)
-#define ST_BY_COPIES(TO)                                \
+#define ST_ANY(TO, NS, ONE, KEEP, TERMS)                                                                                                              \
+  streams_layernorm_vec_kernel<TO, NS, ONE, KEEP, TERMS><<<n_rows, threads, (ONE) ? 0 : lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta,  \
+                                                                                                 weight, bias, eps, rows, width, (TO*)out, mix,    \
+                                                                                                 out_coef, y, scale, delta2, dscale, terms2, conv)
+#define ST_GO(TO, NS, ONE) ST_ANY(TO, NS, ONE, 0, false)
+#define ST_BY_TAPS(TO, NS)                              \
   do {                                                  \
-    if (taps && n_streams == 2) ST_BY_TAPS(TO, 2);      \
-    else if (taps) ST_BY_TAPS(TO, 0);                   \
-    else if (width > 4 * threads) ST_GO(TO, 0, false);  \
-    else if (n_streams == 1) ST_GO(TO, 1, true);        \
-    else if (n_streams == 2) ST_GO(TO, 2, true);        \
-    else if (n_streams == 4) ST_GO(TO, 4, true);        \
-    else ST_GO(TO, 0, true);                            \
+    if (taps == 2) ST_ANY(TO, NS, true, 1, false);      \
+    else if (taps == 3) ST_ANY(TO, NS, true, 2, false); \
+    else ST_ANY(TO, NS, true, 3, false);                \
+  } while (0)
+#define ST_BY_COPIES(TO)                                                   \
+  do {                                                                     \
+    if (taps && n_streams == 2) ST_BY_TAPS(TO, 2);                         \
+    else if (taps && n_streams == 4) ST_BY_TAPS(TO, 4);                    \
+    else if (taps) ST_BY_TAPS(TO, 0);                                      \
+    else if (terms2 > 1 && width > 4 * threads) ST_ANY(TO, 0, false, 0, true); \
+    else if (terms2 > 1) ST_ANY(TO, 1, true, 0, true);                     \
+    else if (width > 4 * threads) ST_GO(TO, 0, false);                     \
+    else if (n_streams == 1) ST_GO(TO, 1, true);                           \
+    else if (n_streams == 2) ST_GO(TO, 2, true);                           \
+    else if (n_streams == 4) ST_GO(TO, 4, true);                           \
+    else ST_GO(TO, 0, true);                                               \
   } while (0)
     if (out_dtype == RB_F32) ST_BY_COPIES(float);
     else ST_BY_COPIES(bf16_t);
 #undef ST_BY_COPIES
 #undef ST_BY_TAPS
 #undef ST_GO
-#undef ST_CONV
+#undef ST_ANY
     RB_LAUNCH_CHECK();
     return 0;
   }
   RB_REQUIRE(taps == 0, "rb_streams_update_layernorm_conv: rows of 16 bytes only");
   if (out_dtype == RB_F32)
-    streams_layernorm_kernel<float><<<n_rows, 256, lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight, bias, eps,
+    (terms2 > 1 ? streams_layernorm_kernel<float, true> : streams_layernorm_kernel<float, false>)<<<n_rows, 256, lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight, bias, eps,
                                                              rows, width, (float*)out, mix, out_coef, y, scale, delta2, dscale, terms2);
   else if (out_dtype == RB_BF16)
-    streams_layernorm_kernel<bf16_t><<<n_rows, 256, lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight, bias, eps,
+    (terms2 > 1 ? streams_layernorm_kernel<bf16_t, true> : streams_layernorm_kernel<bf16_t, false>)<<<n_rows, 256, lds, s>>>(x, n_streams, (size_t)stream_stride, coef, delta, weight, bias, eps,
                                                               rows, width, (bf16_t*)out, mix, out_coef, y, scale, delta2, dscale, terms2);
   else
     RB_REQUIRE(false, "rb_streams_layernorm: unknown dtype %d", out_dtype);
