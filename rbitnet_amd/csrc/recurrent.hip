@@ -411,8 +411,11 @@ struct SelectiveArgs {
   size_t dt_stride;
   const float *dt_bias, *a_log, *d;
 };
+// tokens of a chunk in a step of one token a sequence: as few as deal evenly to the lanes
+constexpr int single_chunk(int rows) { return rows >= RB_WAVE ? 1 : RB_WAVE / rows; }
 // ONE_G: one decay a head and token (g_per_head), which the lanes read as one number.
-template <int DKL, int RG, int P, int CH, int MODE, bool ONE_G, bool WIDE>
+// BY_SEQ: a grid of sequences, heads and a head's columns.
+template <int DKL, int RG, int P, int CH, int MODE, bool ONE_G, bool WIDE, bool BY_SEQ>
 __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
     const float* __restrict__ q, const float* __restrict__ k, size_t qk_stride, const float* __restrict__ v,
     size_t v_stride, const float* __restrict__ g, size_t g_stride, const float* __restrict__ beta, float* __restrict__ state,
@@ -431,11 +434,11 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
   auto pos = [](int i) { return i + (STEP - DKL) * (i / DKL); };
   __shared__ __attribute__((aligned(16))) float sq[CH][LD], sk[CH][LD], sg[ONE_G ? 1 : CH][ONE_G ? CH : LD];
   __shared__ __attribute__((aligned(16))) float sv[CH][COLS], sb[CH];
-  // heads are dealt first, then a head's columns, then sequences: neighbouring workgroups go to different XCDs, so one sequence's are spread
+  // Not BY_SEQ: heads are dealt first, then a head's columns, then sequences: neighbouring workgroups go to different XCDs, so one sequence's are spread
   // over the whole GPU and those of a long one have it to themselves once the short ones are done
-  const int h = blockIdx.x % n_heads, b = blockIdx.x / n_heads / n_parts;
+  const int h = BY_SEQ ? blockIdx.y : blockIdx.x % n_heads, b = BY_SEQ ? blockIdx.x : blockIdx.x / n_heads / n_parts;
   const int lane = threadIdx.x;
-  const int col0 = blockIdx.x / n_heads % n_parts * COLS;
+  const int col0 = (BY_SEQ ? blockIdx.z : blockIdx.x / n_heads % n_parts) * COLS;
   const int rg = lane % RG, mine = lane / RG * P, col = col0 + mine;      // this lane's columns: col .. col + P - 1
   const int kvh = h / (n_heads / n_kv);
   const int row0 = cu_seqlens[b], n = cu_seqlens[b + 1] - row0;
@@ -748,18 +751,27 @@ static int launch_delta_rule(const float* q, const float* k, size_t qk_stride, c
                              const float* g, size_t g_stride, const float* beta, float* state, const int32_t* cu_seqlens,
                              const int32_t* slots, float* out, int n_seqs, int n_heads, int n_kv, int dim, int vdim,
                              const float* bonus, const SelectiveArgs& sel, hipStream_t s) {
+  static_assert(CH > single_chunk(DKL * RG) || P == 1, "single tokens: one column a lane");
   static_assert((DKL * RG * CH) % RB_WAVE == 0 && CH <= RB_WAVE && DKL % 4 == 0, "a chunk's values are dealt evenly to the lanes");
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   constexpr bool MAY = CH > 1 && DKL * RG * CH / RB_WAVE % 4 == 0;
   const bool wide = MAY && dim % 4 == 0 && qk_stride % 4 == 0 && aligned(q) && aligned(k) && (ONE_G || (g_stride % 4 == 0 && aligned(g))) &&
                     (qk_stride | v_stride | (ONE_G ? 0 : g_stride)) < (1u << 24);      // (a chunk's places are offsets of 32 bits)
   const int cols = RB_WAVE / RG * (wide ? P : 1), parts = (vdim + cols - 1) / cols;
+  // Single tokens are bound by the state's way from memory and back, and go sequence by sequence while the XCDs' caches hold all states together.  us in the
+  // order of prompts and so: 16 heads of 128 x 128, 4 tokens 4.82 and 4.63, 16 tokens 15.6 and 13.6; 8 heads of 64 x 64, 8 tokens, 3.04 and 2.82.  Larger ones gain by the other:
+  // 64 tokens, 64 heads of 128 x 64 69 and 137, 32 heads of 64 x 64 17.8 and 21.7, 16 heads of 128 x 128 45.7 and 45.0, 128 tokens 82 and 110.
+  constexpr bool SINGLE = CH == single_chunk(DKL * RG);
+  const bool by_seq = SINGLE && (long long)n_seqs * n_heads * vdim * dim < 1LL << 23;
   // a launch has fewer than 2^32 threads: more sequences than that go in several
-  const long long most = 0xffffffffLL / RB_WAVE / ((long long)n_heads * parts);
+  const long long most = 0xffffffffLL / RB_WAVE / (by_seq ? 1 : (long long)n_heads * parts);
   RB_REQUIRE(most > 0, "rb_linear_recurrence: too many heads and value channels");
   for (long long b0 = 0; b0 < n_seqs; b0 += most) {
-    const int grid = (int)((n_seqs - b0 < most ? n_seqs - b0 : most) * n_heads * parts);
-    (wide ? delta_rule_kernel<DKL, RG, MAY ? P : 1, CH, MODE, ONE_G, MAY> : delta_rule_kernel<DKL, RG, 1, CH, MODE, ONE_G, false>)<<<grid, RB_WAVE, 0, s>>>(
+    const int here = (int)(n_seqs - b0 < most ? n_seqs - b0 : most);
+    const dim3 grid = by_seq ? dim3(here, n_heads, parts) : dim3((unsigned)((long long)here * n_heads * parts));
+    (by_seq ? delta_rule_kernel<DKL, RG, 1, CH, MODE, ONE_G, false, SINGLE>
+     : wide ? delta_rule_kernel<DKL, RG, MAY ? P : 1, CH, MODE, ONE_G, MAY, false>
+            : delta_rule_kernel<DKL, RG, 1, CH, MODE, ONE_G, false, false>)<<<grid, RB_WAVE, 0, s>>>(
         q, k, qk_stride, v, v_stride, g, g_stride, beta, state, cu_seqlens + b0, slots + b0, out, n_heads, n_kv, dim, vdim, parts, bonus, sel);
   }
   RB_LAUNCH_CHECK();
@@ -867,8 +879,7 @@ static int linear_recurrence_launch(const float* q, const float* k, long long qk
   } while (0)
 #define DR_GO(DKL, RG, P, CH)                                                             \
   do {                                                                                    \
-    constexpr int CH1 = (DKL * RG >= RB_WAVE) ? 1 : RB_WAVE / (DKL * RG);                 \
-    if (single) DR_LENGTH(DKL, RG, 1, CH1);                                               \
+    if (single) DR_LENGTH(DKL, RG, 1, single_chunk(DKL * RG));                                            \
     DR_LENGTH(DKL, RG, P, CH);                                                            \
   } while (0)
   // Rows of a column over RG lanes, chunks as long as the registers that hold the next one allow.  A token's time is
