@@ -126,6 +126,8 @@ class LayerNorm(Part):
         n = t if rows is None else rows.shape[0]
         out = torch.empty((n, self.size), dtype=out_dtype or self.env.dtype, device=x.device)
         if isinstance(delta, ScaledSum):                  # a plain stream [T, E] and the residual sum that is still to be done
+            if conv is not None:
+                raise ConfigError("a layer norm that adds a scaled sum takes no convolution along")
             a, b, scale = delta.parts()
             self.env.lib.layernorm_residual(x, a, b, scale, self.weight, self.bias, self.eps, rows, out)
             return out

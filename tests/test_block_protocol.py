@@ -1,8 +1,11 @@
 """How a block hands a norm's input on (no GPU: the parts here are stand-ins that record calls)."""
+import pytest
 import torch
 
+from rbitnet_amd.errors import ConfigError
 from rbitnet_amd.parts.block import normed_for
-from rbitnet_amd.parts.norm import GainedRows
+from rbitnet_amd.parts.norm import GainedRows, LayerNorm
+from rbitnet_amd.parts.stream import ScaledSum
 
 
 class _Env:
@@ -62,3 +65,9 @@ def test_rows_are_chosen_once():
     picked = normed_for(_Takes(), norm, x, _gained(norm, x), rows)
     assert picked.rows is rows and picked.shape == (2, 4) and picked.gained.shape == (3, 4)
     assert picked.tensor() == "normalised" and norm.calls == [(None, rows)]
+
+
+def test_a_layer_norm_that_adds_a_scaled_sum_leaves_out_no_convolution():
+    norm, x = LayerNorm({"size": 4, "eps": 1e-5}, _Env()), torch.zeros(3, 4)
+    with pytest.raises(ConfigError, match="convolution"):
+        norm.forward(x, ScaledSum(x, None, 1.0), conv=("weight", "state", "ctx"))
