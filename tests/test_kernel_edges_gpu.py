@@ -1846,6 +1846,33 @@ def test_float32_products_of_few_tokens_take_sum_and_norm_along(lib, n, k, frag)
     assert not lib.gemm_f32_few_ok(17, n, k, frag, 0) and not lib.gemm_f32_few_ok(4, n, k + 2, frag, 2)
 
 
+@pytest.mark.parametrize("k,frag", [(96, False), (128, True), (1000, False), (1024, True), (2048, True)])
+def test_float32_products_multiply_by_a_norms_factor_as_64_bits_have_it(lib, k, frag):
+    """Rows of W that pick a column each, sums of squares that float32 adds up exactly: what is left is the rounding of the result, half a unit of 2^-23, and
+    what one step from the root's estimate of 2^-23 leaves (2^-45).  An infinite sum of squares makes zeros, as the norm's own launch does."""
+    gen = torch.Generator().manual_seed(k)
+    pick = torch.randperm(k, generator=gen)[:64]
+    rows = torch.zeros(64, k)
+    rows[torch.arange(64), pick] = 1.0
+    w = rows.to(DEV)
+    if frag:
+        w = torch.empty(64, k, device=DEV)
+        lib.place_rows(rows.to(DEV), w, frag=True)
+    for m in (1, 4, 8, 16):
+        if not lib.gemm_f32_few_ok(m, 64, k, frag, 0):
+            continue
+        for eps in (1e-5, 0.0):
+            gained = torch.randn(m, k, generator=gen)
+            squares = torch.randint(1, 4096, (m, (k + 7) // 8), generator=gen).float()
+            want = gained[:, pick].double() / (squares.double().sum(-1, keepdim=True) / k + torch.tensor(eps).double()).sqrt()
+            if m == 4:
+                squares[2] = float("inf")
+                want[2] = 0.0
+            got = torch.full((m, 64), float("nan"), device=DEV)
+            lib.gemm_f32_few(gained.to(DEV), w, got, 0, squares=squares.to(DEV), eps=eps, w_frag=frag)
+            assert ((got.double().cpu() - want).abs() <= 2.0 ** -24 * 1.00001 * want.abs()).all()
+
+
 # ---------------------------------------------------------------------------- a norm that adds up the outputs of a token's experts
 @pytest.mark.parametrize("width", [4, 101, 2048, 4104])
 @pytest.mark.parametrize("terms", [1, 2, 3, 4, 5, 9])
