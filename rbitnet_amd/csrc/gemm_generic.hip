@@ -783,6 +783,7 @@ extern "C" int rb_gemm_f32_gated_pays(int m, int ff, int k, int w_layout) {
 extern "C" int rb_gemm_f32_gated(const float* a, const float* w, int w_layout, float* c, int m, int ff, int k, void* stream) {
   RB_RECORDED(rb_gemm_f32_gated(a, w, w_layout, c, m, ff, k, stream));
   RB_REQUIRE(m == 0 || rb_gemm_f32_gated_ok(m, ff, k, w_layout), "rb_gemm_f32_gated: M=%d ff=%d K=%d, layout %d are not for it", m, ff, k, w_layout);
+  RB_REQUIRE(((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15) == 0, "rb_gemm_f32_gated: operands must be 16-byte aligned");
   if (m == 0) return 0;
   launch_f32_gated(a, w, w_layout == 1, c, m, ff, k, (hipStream_t)stream);
   RB_LAUNCH_CHECK();
@@ -809,6 +810,8 @@ extern "C" int rb_gemm_f32_few(const float* a, const float* squares_in, float ep
   RB_RECORDED(rb_gemm_f32_few(a, squares_in, eps, rows, w, w_layout, c, epilogue, gain, gained, squares_out, m, n, k, stream));
   RB_REQUIRE(rb_gemm_f32_few_ok(m, n, k, w_layout, epilogue), "rb_gemm_f32_few: M=%d N=%d K=%d, layout %d, epilogue %d are not for it", m, n, k,
              w_layout, epilogue);
+  RB_REQUIRE(((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(squares_in)) & 15) == 0,
+             "rb_gemm_f32_few: operands must be 16-byte aligned");
   RB_REQUIRE(!squares_in || epilogue <= 1, "rb_gemm_f32_few: prepared rows go with epilogues 0 and 1, not %d", epilogue);
   RB_REQUIRE(epilogue != 3 || (gain && gained && squares_out), "rb_gemm_f32_few: epilogue 3 needs the gain and room for the prepared rows");
   if (epilogue != 3) gain = nullptr, gained = squares_out = nullptr;

@@ -72,8 +72,13 @@ def _few(lib, x, w, epilogue: int = 0) -> bool:
     if not FOLD_INTO_PRODUCTS:
         return False
     if x.dtype == torch.float32:
-        return lib.gemm_f32_few_ok(m, w.shape[0], k, _data(w)[1], epilogue)
+        return lib.gemm_f32_few_ok(m, w.shape[0], k, _data(w)[1], epilogue) and _wide_loads(x, w)
     return uses_matrix_cores(x.dtype, k) and lib.gemm_bf16_few_ok(m, w.shape[0], k)
+
+
+def _wide_loads(x, w) -> bool:
+    """Whether tokens and matrix lie at whole pieces of 16 bytes, as torch allocates them (views of other tensors may not)."""
+    return _data(w)[0].data_ptr() % 16 == 0 and (isinstance(x, GainedRows) or x.data_ptr() % 16 == 0)
 
 
 def _few_product(lib, dtype: torch.dtype):
@@ -215,7 +220,8 @@ def gated_linear(lib, x, w_packed, ff: int, fused: bool, gate: Optional[torch.Te
     out = torch.empty((m, ff), dtype=x.dtype, device=x.device)
     if m == 0:
         return out
-    in_one = x.dtype == torch.float32 and not fused and lib.gemm_f32_gated_pays(m, ff, x.shape[1], _data(w_packed)[1])
+    in_one = (x.dtype == torch.float32 and not fused and lib.gemm_f32_gated_pays(m, ff, x.shape[1], _data(w_packed)[1])
+              and _wide_loads(x, w_packed))
     if isinstance(x, GainedRows):
         if (fused or in_one) and _few(lib, x, w_packed, 1):
             _from_gained(lib, x, w_packed, out, 1)

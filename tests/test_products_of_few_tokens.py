@@ -2,8 +2,10 @@
 import ctypes
 
 import pytest
+import torch
 
 from rbitnet_amd.csrc import build
+from rbitnet_amd.parts import linear
 
 
 @pytest.fixture(scope="module")
@@ -54,3 +56,36 @@ def test_a_second_float32_stage_is_under_way_where_that_was_the_faster(lib):
 def test_a_float32_norm_is_left_to_its_products_where_that_was_the_faster(lib):
     for width, most in ((96, 16), (2048, 16), (2052, 8), (3072, 8), (3076, 0), (4096, 0), (5120, 0)):
         assert [m for m in range(0, 18) if lib.rb_gemm_f32_fold_pays(m, width)] == list(range(1, most + 1)), width
+
+
+def test_float32_products_with_their_neighbours_refuse_operands_between_whole_pieces_of_16_bytes(lib):
+    """Host checks in front of the launch (addresses that nothing reads)."""
+    lib.rb_last_error.restype = ctypes.c_char_p
+    at, p, f = 1 << 20, ctypes.c_void_p, ctypes.c_float
+    for a, w, squares in ((at + 4, at, at), (at, at + 8, at), (at, at, at + 4)):
+        assert lib.rb_gemm_f32_few(p(a), p(squares), f(1e-5), None, p(w), 1, p(at), 0, None, None, None, 4, 128, 128, None) != 0
+        assert b"16-byte aligned" in lib.rb_last_error()
+    for a, w in ((at + 4, at), (at, at + 8)):
+        assert lib.rb_gemm_f32_gated(p(a), p(w), 1, p(at), 4, 128, 128, None) != 0
+        assert b"16-byte aligned" in lib.rb_last_error()
+
+
+def test_float32_operands_between_whole_pieces_of_16_bytes_go_to_the_products_that_take_any(lib):
+    class Products:
+        calls = []
+        gemm_f32_few_ok = staticmethod(lambda *sizes: True)
+        gemm_f32_gated_pays = staticmethod(lambda *sizes: True)
+        gemm_f32_fold_pays = staticmethod(lambda *sizes: True)
+
+        def __getattr__(self, name):
+            return lambda *args, **kwargs: self.calls.append(name)
+
+    aligned, between = torch.zeros(4, 128), torch.zeros(4 * 128 + 1)[1:].view(4, 128)
+    w, w_between, kernels = torch.zeros(128, 128), torch.zeros(128 * 128 + 1)[1:].view(128, 128), Products()
+    assert aligned.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    for x, m, calls in ((aligned, w, ["gemm_f32_gated", "gemm_f32_few"]), (between, w, ["gemm_generic", "swiglu", "gemm_generic"]),
+                        (aligned, w_between, ["gemm_generic", "swiglu", "gemm_generic"])):
+        kernels.calls.clear()
+        linear.gated_linear(kernels, x, m, 64, fused=False)
+        linear.linear_to_stream(kernels, x, m, torch.zeros(4, 128))
+        assert kernels.calls == calls
