@@ -451,7 +451,10 @@ extern "C" int rb_heads_combined(const float* ws, int n_splits, const float* sin
   RB_REQUIRE(gate == nullptr || gate_stride >= n_heads, "rb_heads_combined: the gate's rows are shorter than the heads");
   RB_REQUIRE(((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y)) & 15) == 0, "rb_heads_combined: operands must be 16-byte aligned");
   if (n_tokens == 0) return 0;
-#define HC_GO(D, KS)                                                                                                                           heads_combined_kernel<D, KS><<<n_heads, HC_THREADS, 0, (hipStream_t)stream>>>(ws, n_splits, sinks, (const bf16_t*)w, (bf16_t*)y, n_tokens,                                                                                 n_heads, n, (size_t)y_head_stride, gate, (size_t)gate_stride)
+#define HC_GO(D, KS)                                                                                                              \
+  heads_combined_kernel<D, KS><<<n_heads, HC_THREADS, 0, (hipStream_t)stream>>>(ws, n_splits, sinks, (const bf16_t*)w, (bf16_t*)y, \
+                                                                                n_tokens, n_heads, n, (size_t)y_head_stride, gate, \
+                                                                                (size_t)gate_stride)
   if (width == 64) {
     if (k == 32) HC_GO(64, 1);
     else HC_GO(64, 2);

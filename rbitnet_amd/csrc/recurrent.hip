@@ -619,41 +619,41 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
       }
     }
   };
-      // One token: with D = diag(g) S and u = beta (v - D^T k), the read-out of the updated state is
-      // (D + k u^T)^T q = D^T q + u (k . q): one pass over the decayed column gives both dot products, and a token has
-      // one reduction among the RG lanes on its way instead of two.  Two partial sums each: shorter chains of additions.
-      struct Token {
-        float k[DKL], q[DKL], g[ONE_G ? 1 : DKL], v[P], b;
-      };
-      auto read = [&](Token& r, int tt) __attribute__((always_inline)) {
+  // One token: with D = diag(g) S and u = beta (v - D^T k), the read-out of the updated state is
+  // (D + k u^T)^T q = D^T q + u (k . q): one pass over the decayed column gives both dot products, and a token has
+  // one reduction among the RG lanes on its way instead of two.  Two partial sums each: shorter chains of additions.
+  struct Token {
+    float k[DKL], q[DKL], g[ONE_G ? 1 : DKL], v[P], b;
+  };
+  auto read = [&](Token& r, int tt) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < DKL; ++i) {
-          r.k[i] = sk[tt][rg * STEP + i];
-          r.q[i] = sq[tt][rg * STEP + i];
-          if (!ONE_G) r.g[ONE_G ? 0 : i] = sg[ONE_G ? 0 : tt][ONE_G ? 0 : rg * STEP + i];
-        }
-        if (ONE_G) r.g[0] = sg[0][ONE_G ? tt : 0];
+    for (int i = 0; i < DKL; ++i) {
+      r.k[i] = sk[tt][rg * STEP + i];
+      r.q[i] = sq[tt][rg * STEP + i];
+      if (!ONE_G) r.g[ONE_G ? 0 : i] = sg[ONE_G ? 0 : tt][ONE_G ? 0 : rg * STEP + i];
+    }
+    if (ONE_G) r.g[0] = sg[0][ONE_G ? tt : 0];
 #pragma unroll
-        for (int p = 0; p < P; ++p) r.v[p] = sv[tt][mine + p];
-        r.b = DELTA || SELECTIVE ? sb[tt] : 0.f;
-      };
-      auto token = [&](const Token& r, int tt) __attribute__((always_inline)) {
-        float kv[P][2], dq[P][2], kq[2] = {0.f, 0.f};
+    for (int p = 0; p < P; ++p) r.v[p] = sv[tt][mine + p];
+    r.b = DELTA || SELECTIVE ? sb[tt] : 0.f;
+  };
+  auto token = [&](const Token& r, int tt) __attribute__((always_inline)) {
+    float kv[P][2], dq[P][2], kq[2] = {0.f, 0.f};
 #pragma unroll
-        for (int p = 0; p < P; ++p) kv[p][0] = kv[p][1] = dq[p][0] = dq[p][1] = 0.f;
+    for (int p = 0; p < P; ++p) kv[p][0] = kv[p][1] = dq[p][0] = dq[p][1] = 0.f;
 #pragma unroll
-        for (int i = 0; i < DKL; ++i) {
-          kq[i & 1] = fmaf(BONUS ? ub[i] * r.k[i] : r.k[i], r.q[i], kq[i & 1]);
+    for (int i = 0; i < DKL; ++i) {
+      kq[i & 1] = fmaf(BONUS ? ub[i] * r.k[i] : r.k[i], r.q[i], kq[i & 1]);
 #pragma unroll
-          for (int p = 0; p < P; ++p) {
-            if (BONUS) dq[p][i & 1] = fmaf(s[p][i], r.q[i], dq[p][i & 1]);
-            s[p][i] *= r.g[ONE_G ? 0 : i];
-            if (BONUS) continue;
-            if (DELTA) kv[p][i & 1] = fmaf(s[p][i], r.k[i], kv[p][i & 1]);
-            dq[p][i & 1] = fmaf(s[p][i], r.q[i], dq[p][i & 1]);
-          }
-        }
-        const float kqs = lanes_sum<RG>(kq[0] + kq[1]);
+      for (int p = 0; p < P; ++p) {
+        if (BONUS) dq[p][i & 1] = fmaf(s[p][i], r.q[i], dq[p][i & 1]);
+        s[p][i] *= r.g[ONE_G ? 0 : i];
+        if (BONUS) continue;
+        if (DELTA) kv[p][i & 1] = fmaf(s[p][i], r.k[i], kv[p][i & 1]);
+        dq[p][i & 1] = fmaf(s[p][i], r.q[i], dq[p][i & 1]);
+      }
+    }
+    const float kqs = lanes_sum<RG>(kq[0] + kq[1]);
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const float kvs = DELTA ? lanes_sum<RG>(kv[p][0] + kv[p][1]) : 0.f;

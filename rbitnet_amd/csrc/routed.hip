@@ -1072,7 +1072,7 @@ extern "C" int rb_routed_experts_few(const void* h, const float* weight, int top
     if (pack == 4) RT_SHARED(4);
     else if (pack == 2) RT_SHARED(2);
     else RT_SHARED(1);
-  } else if (n_tokens > RT_TILE) {            // a token chooses an expert once: no run is longer than the step's tokens
+  } else if (n_tokens > RT_TILE) {            // up to 4 tiles of a run a workgroup; what a run has beyond them is another's (tile_pos)
     RT_ALONE(4, 1);
   } else if (pack == 4) {
     RT_ALONE(1, 4);
