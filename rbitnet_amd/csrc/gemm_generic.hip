@@ -203,7 +203,8 @@ __device__ __forceinline__ float squares_meet(float ss, float* __restrict__ lds,
 }
 // ... and behind it (with one wave there is none: its own sum) they make the norm's factor, in 64 bits.  The four roundings that it has in float32 (a mean,
 // eps, a root, a quotient) meet all of a row's numbers alike: with them a model of width 96 was 2 % further off 64 bits than with norms in
-// launches of their own (1.040e-7 for 1.021e-7), without them it is at 0.953e-7, in the same time.  One step from the root's estimate; infinity and 0, where the step is not a number, keep the estimate (0 and infinity).
+// launches of their own (1.040e-7 for 1.021e-7), without them it is at 0.953e-7, in the same time.  One step from the root's estimate; infinity and 0,
+// where the step is not a number, keep the estimate (0 and infinity).
 __device__ __forceinline__ double squares_factor(float own, const float* __restrict__ lds, int n_waves, int lane, const F32Fold& fa) {
   float ss = own;
   if (n_waves > 1) {
