@@ -12,6 +12,7 @@ void rb_tune_compute_units(int n);                              // every planner
 void rb_tune(int rows_per_wave, int waves);                     // skinny product
 void rb_tune_parts(int parts);                                  // skinny product: 1 or 2 workgroups for a tile of 16 rows
 int rb_tune_few_blocks(int m, int n, int k, int epilogue, int prepared);      // skinny product: the built-in choice of blocks of depth a load of the tokens
+int rb_tune_group_form(int m, int k, int tiles);                // products in one launch: the built-in choice of how the tokens are loaded
 void rb_tune_resident(int tiles);                               // skinny product with resident tokens: row tiles per workgroup
 void rb_tune_use_resident(int on);                              // 0: never the resident variant, 2: also below 8192 rows
 void rb_tune_f32_few(int on);                                   // float32 product of few tokens: 0 = on the vector units, not the float32 MFMA; 3 = one row tile a wave always

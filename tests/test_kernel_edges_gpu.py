@@ -1780,6 +1780,25 @@ def test_products_in_one_launch_give_the_bits_of_each_alone(lib, m, k, rows):
         assert torch.equal(c, a.to(c.dtype)), rows[i]
 
 
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("k,rows", [(128, (16, 1024)), (256, (1024,) * 5), (768, (768, 48)), (1024, (16, 4096)), (2048, (16, 1040)), (2048, (4096, 64)), (2560, (2560, 16)),
+                                    (4096, (2048, 128)), (8192, (6144, 1024))])
+def test_products_in_one_launch_give_the_bits_of_each_alone_however_tokens_are_loaded(lib, m, k, rows):
+    gen = torch.Generator(device=DEV).manual_seed(k + m)
+    products, alone = [], []
+    for n in rows:
+        x, plain = torch.randn(m, k, generator=gen, device=DEV).bfloat16(), torch.randn(n, k, generator=gen, device=DEV).bfloat16()
+        w = torch.empty_like(plain)
+        lib.place_rows(plain, w, frag=True)
+        products.append((x, w, torch.full((m, n), 9.0, device=DEV), "float32"))
+        alone.append(torch.empty(m, n, device=DEV))
+        assert lib.gemm_bf16_group_pays(m, n, k)
+        lib.gemm_bf16(x, w, alone[-1], 0, w_frag=True)
+    lib.gemm_bf16_group(products, True)
+    for (_, _, c, _), want in zip(products, alone):
+        assert torch.equal(c, want)
+
+
 # ---------------------------------------------------------------------------- float32 products of few tokens: sums and norms in their launches
 @pytest.mark.parametrize("n,k,frag", [(16, 128, True), (96, 96, False), (257, 96, False), (90, 500, False), (384, 1000, False), (130, 384, False), (2048, 512, True),
                                       (4096, 768, True), (4112, 1280, True), (3072, 3072, True), (256, 8192, True)])

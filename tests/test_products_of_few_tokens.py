@@ -33,6 +33,17 @@ def test_tokens_are_packed_where_that_was_the_faster_load(lib, n, k, end, prepar
     assert blocks == [four, four, eight, eight, 1, 1]
 
 
+# K, row tiles -> 4 or 2 blocks a load, 1: one, multiplied where it was loaded, 0: set aside, for 1, 4, 5, 8, 9 and 16 tokens, and what another took longer
+@pytest.mark.parametrize("k,tiles,forms", [
+    (768, 99, (1, 1, 1, 1, 1, 1)), (1024, 68, (4, 4, 1, 1, 1, 1)), (1024, 260, (4, 4, 2, 2, 1, 1)),       # 7, 2 to 6 and 2 to 3 %
+    (256, 320, (4, 4, 2, 2, 0, 0)), (1536, 262, (4, 4, 2, 2, 0, 0)), (2560, 323, (4, 4, 0, 0, 1, 1)),       # 8, 3 and 2 to 4 %
+    (2048, 209, (0, 0, 0, 0, 1, 1)), (2048, 401, (0, 0, 0, 0, 1, 1)), (4096, 136, (4, 4, 2, 2, 1, 1)), (4096, 401, (4, 4, 0, 0, 1, 1)),       # 2, 4, 2 and 4 %
+    (8192, 260, (4, 4, 2, 2, 1, 1)), (8192, 448, (1, 1, 1, 1, 1, 1)),                                    # 7 and 2 to 3 %
+])
+def test_products_in_one_launch_load_their_tokens_as_was_the_faster(lib, k, tiles, forms):
+    assert tuple(lib.rb_tune_group_form(m, k, tiles) for m in (1, 4, 5, 8, 9, 16)) == forms
+
+
 # units, K, stored fragment-major -> whether 1, 8, 9 and 16 float32 tokens go through gate, way up and the gate in one launch, and what the other way took longer
 @pytest.mark.parametrize("ff,k,frag,one", [
     (1024, 512, 1, (1, 1, 1, 1)), (256, 96, 0, (1, 1, 1, 1)), (5120, 500, 0, (0, 0, 1, 1)),            # 22, 50 and 24 % (9 tokens)
