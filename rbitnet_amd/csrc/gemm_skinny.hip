@@ -370,54 +370,79 @@ static FoldArgs fold_args(const GemmTokens& x, const GemmAfter& after, const voi
 // block of depth, halve that share.  us with whole tiles and with halves, 4 tokens: 2,048 rows at K = 2048 4.17 and 3.89, 4096 5.75 and 5.42, 8192 10.2 and 8.8,
 // 11008 14.0 and 11.8; 896 rows at 2048 3.87 and 3.61; 16 tokens, 2,048 at 8192 12.6 and 11.4.  More than one a unit lose (2,304 rows at 2048 4.28 and
 // 4.57), and so do quarters, whose 64 bytes are half a line (2,048 rows at 2048 5.25, 896 4.01).
-static int skinny_parts(int n) {
+// At K < 1280 a wave has one or two stages, and what the first trip waits for is whole tiles' worth anyway: 2,048 rows, 4 / 8 / 16 tokens, whole tiles and halves: K = 512 2.66 / 2.71 /
+// 2.89 and 2.70 / 2.85 / 3.04, 768 2.95 / 3.14 / 3.18 and 2.90 / 3.10 / 3.40, 1024 3.32 / 3.54 / 3.54 and 3.15 / 3.40 / 3.84; added to C 512 2.81 / 3.32 / 3.35 and 3.00 / 3.05 / 3.22, 1024 3.39 / 3.58 / 3.71 and
+// 3.38 / 3.53 / 3.98.
+static int skinny_parts(int m, int n, int k, int epilogue) {
   if (g_tune_parts) return g_tune_parts;
-  return 2 * ((n + 15) / 16) <= rb_compute_units() ? 2 : 1;
+  if (2 * ((n + 15) / 16) > rb_compute_units()) return 1;
+  if (k >= 1280) return 2;
+  if (k >= 896) return m <= 8 ? 2 : 1;
+  if (epilogue == 2) return m > 4 ? 2 : 1;
+  return k >= 768 && m > 1 && m <= 8 ? 2 : 1;
 }
+extern "C" int rb_tune_few_parts(int m, int n, int k, int epilogue) { return skinny_parts(m, n, k, epilogue); }      // for tests: the choice
 
-// Whether a product of 9 to 16 tokens (fragment-major W, tokens as they are) sets its operands aside: with two row tiles a wave at K > 4096, and with one
-// where the sums are added to C and nothing else.  us without and with, 9 / 16 tokens: 8,192 rows at K = 8192 31.0 / 31.5 and 27.3 / 27.3, with the next norm's
-// rows 30.2 / 30.3 and 27.8 / 27.6; 5,120 at 5120 with those 12.87 / 14.3 and 12.5 / 14.0; the gate, 10,240 at 8192, 31.6 / 32.4 and 30.2 / 31.8; added to C, 4,096 at 14336
-// 22.8 / 25.2 and 19.8 / 23.1, 6,144 at 4096 12.05 / 13.7 and 11.0 / 13.0.  The others lose: 6,144 at 4096 10.7 / 12.7 and 11.2 / 13.4; with the next norm's rows 4,096 at 14336
-// 23.0 / 23.4 and 23.2 / 23.8, 3,072 at 2048 5.3 / 5.6 and 5.4 / 5.8; the gate, 10,304 at 2048, 10.24 and 10.69 (9); four tiles, 16,384 at 8192 with the next norm's rows,
-// 45.3 / 44.5 and 54.5 / 55.3, for which there are not enough registers.  Captured steps of 12 sequences, 8 layers of the 8B shape 823 and 829 us, 5 of
-// the 70B shape 1,700 and 1,669.  (Two whole stages in registers, or W a stage ahead of the tokens, both spelled out: slower than either.)
-// (At K < 2048 a wave has no more than four stages: with at most a tile a compute unit there is nothing to gain, 3,584 rows at K = 1024 3.77 and 4.0, 8 tokens.)
-constexpr bool set_aside(int r, int epilogue, int k, bool many) {
-  return r == 2 ? epilogue != 1 || k > 4096 : r == 1 && epilogue == 2 && (k >= 2048 || many);
+// Whether a product of 9 to 16 tokens (fragment-major W, tokens as they are) sets its operands aside, r row tiles a wave, `grid` workgroups: us without and with, 9 / 16
+// tokens.
+//  - One tile, added to C: 4,096 at 14336 24.9 / 27.8 and 22.4 / 26.1, 6,144 at 4096 12.05 / 13.7 and 11.0 / 13.0, 2,560 at 1280 4.74 / 4.84 and 4.19 / 4.35, 3,072 at 512 3.42 / 3.43 and 3.07 / 3.21;
+//    but not where most waves have one stage and few tiles follow (4,096 rows at 1024 3.90 / 4.18 and 4.19 / 4.37, 3,072 at 896 16 tokens 3.69 and 3.87).  With the next norm's rows the same at
+//    K < 2048: 2,048 at 512 3.63 / 3.64 and 3.20 / 3.36, 2,560 at 1280 4.73 / 4.92 and 4.38 / 4.68, 4,096 at 1024 4.22 / 4.53 and 4.47 / 4.79; 4,096 at 14336 23.0 / 23.4 and 23.2 / 23.8.  Else two
+//    stages of some waves alone: 2,560 at 1280 4.04 / 4.25 and 3.93 / 4.29, 6,144 at 4096 10.7 / 12.7 and 11.2 / 13.4.
+//  - Two: 8,192 at 8192 33.4 / 33.4 and 29.9 / 30.3, with the next norm's rows 32.0 / 32.4 and 30.2 / 30.4; the gate from K = 4096 on and at 1152 and 1280 (8,192 at 8192 33.3 / 33.6 and 30.0 / 30.6; 2,560 at
+//    1280 4.96 / 5.27 and 4.74 / 5.14; 10,304 at 2048, 9 tokens, 10.24 and 10.69); added to C up to four workgroups a compute unit (22,016 at 4608 37.0 / 40.0 and 36.0 / 38.7; 57,344 at 8192 163 / 159 and 178 / 169).
+//  - Four, which take 198 registers then: added to C (15,360 at 5120 30.2 / 31.0 and 29.2 / 30.2), and the gate on up to three quarters of the units (10,240 at 8192 35.3 / 36.7 and 33.6 / 35.8;
+//    16,384 47.6 / 48.0 and 48.8 / 48.7).  With the next norm's rows there are not enough registers (16,384 at 8192 47.3 / 47.5 and 56.2 / 57.2).
+// Captured steps of 12 sequences, 8 layers of the 8B shape 823 and 829 us, 5 of the 70B shape 1,700 and 1,669.  (Two whole stages in registers, or W a stage ahead of the
+// tokens, both spelled out: slower than either.)
+constexpr bool may_set_aside(int r, int epilogue) { return r == 1 ? epilogue == 0 || epilogue == 2 || epilogue == 3 : r == 2 || epilogue == 1 || epilogue == 2; }
+static bool set_aside(int r, int epilogue, int k, long long grid) {
+  const long long cus = rb_compute_units();
+  if (!may_set_aside(r, epilogue)) return false;
+  if (r == 1) {
+    if (epilogue == 0) return k >= 1152 && k < 1536;
+    return k <= 768 || (k >= 1152 && (epilogue == 2 || k < 2048)) || (epilogue == 2 && grid > cus);
+  }
+  if (r == 2) return epilogue == 1 ? k >= 4096 || (k >= 1152 && k < 1536) : epilogue == 2 ? grid <= 4 * cus : true;
+  return epilogue == 2 || 4 * grid <= 3 * cus;
 }
 
 // Blocks of depth that a load of the tokens brings, where a tile of rows is one workgroup's: as many as there is room for, except
 //  - tokens that a norm prepared: their sums of squares are waited for first, and what is saved behind that seldom makes up for two rows' addresses and the
 //    rotations.  us with a block a load and packed, 4 tokens: 2,048 rows at K = 2048 4.61 and 4.73, 8,192 at 8192 28.4 and 29.4; of gate and way up
-//    8,192 at 8192 28.5 and 29.7, 8,192 at 2048 7.87 and 8.02.  It pays above K = 4096 with more tiles than compute units (5,120 at 5120 1 to 5 %), and for
+//    8,192 at 8192 28.5 and 29.7, 8,192 at 2048 7.87 and 8.02.  It pays above K = 4096 with more tiles than compute units (5,120 at 5120 1 to 5 %) and up to four a unit (27,648 at 5120, 6 tokens, 48.0 and 49.7), and for
 //    the gate from K = 3072 on with few tiles (4,096 at 14336 4 %) or, with 5 to 8 tokens, many (57,344 at 8192 2 %);
 //  - rows of 16 KB or a multiple: where workgroups share a compute unit, the few lines of tokens that packed loads ask for lie in too few channels of the
 //    caches (12,288 rows at K = 8192 5 to 7 %; at 7168, 9216 and 10240 nothing is lost);
-//  - four row tiles a wave on nearly every compute unit (15,360 rows at K = 5120 26.2 and 26.7 us; the gate on 192 units, 12,288 at 7168, gains 3 to 5 %);
-//  - 5 to 8 tokens at K < 2048 while the tiles are few (3,072 rows at K = 1024 4 to 5 %) and, with the next norm's rows, while they are many (2 to 3 %).
+//  - four row tiles a wave on nearly every compute unit (15,360 rows at K = 5120 26.2 and 26.7 us; the gate on 192 units, 12,288 at 7168, gains 3 to 5 %, and on 432, 27,648 at
+//    5120, 2 to 6 %);
+//  - 5 to 8 tokens at K <= 1024 while the tiles are few (3,072 rows at K = 1024 4 to 5 %; at 1152 and 1280 it gains 2 to 7 %) and, at K < 2048, with the next norm's rows, while they are many (2 to 3 %).
 // Added to C alone the packed loads gain otherwise, up to 30 %.
 static int packed_blocks(int m, int n, int k, int r, int epilogue, bool scaled) {
   if (m > 8) return 1;
   const long long tiles = (n + 15) / 16, cus = rb_compute_units();
-  const bool whole16k = k % 8192 == 0, short_of_eight = m > 4 && k < 2048;
+  const bool whole16k = k % 8192 == 0, short_of_eight = m > 4 && k <= 1024;
   bool pays;
   if (scaled && epilogue == 1)
     pays = (k >= 3072 && 4 * tiles <= (whole16k ? 3 : k > 4096 ? 5 : 4) * cus) || (m > 4 && k > 4096 && tiles > 2 * cus);
   else if (scaled)
-    pays = k > 4096 && tiles > (whole16k ? 2 : 1) * cus;
+    pays = k > 4096 && tiles > (whole16k ? 2 : 1) * cus && tiles <= 4 * cus;
   else if (epilogue == 2)
     pays = !(short_of_eight && tiles <= cus);
   else if (r == 4)
-    pays = epilogue == 3 ? !(whole16k && tiles <= 4 * cus) : epilogue == 1 && tiles <= 3 * cus;
+    pays = epilogue == 3 ? !(whole16k && tiles <= 4 * cus) : epilogue == 1 && (tiles <= 3 * cus || (!whole16k && tiles > 4 * cus));
   else if (epilogue == 3)
-    pays = !(whole16k && r == 1 && tiles > 2 * cus) && !(short_of_eight && tiles > 2 * cus && tiles <= 4 * cus);
+    pays = !(whole16k && r == 1 && tiles > 2 * cus) && !(m > 4 && k < 2048 && tiles > 2 * cus && tiles <= 4 * cus);
   else
     pays = !(whole16k && r == 1 && tiles > 2 * cus) && !(short_of_eight && tiles < 2 * cus);
   return !pays ? 1 : m <= 4 ? 4 : 2;
 }
 
-// For tests: the choice for a fragment-major product, tokens as they are or prepared by a norm
+// For tests: the choices for a fragment-major product, tokens as they are or prepared by a norm
+extern "C" int rb_tune_few_aside(int n, int k, int epilogue) {
+  const int r = skinny_rows(n, k, epilogue == 1);
+  return set_aside(r, epilogue, k, (n + 16 * r - 1) / (16 * r));
+}
 extern "C" int rb_tune_few_blocks(int m, int n, int k, int epilogue, int prepared) {
   return k % 128 != 0 || m > 16 ? 1 : packed_blocks(m, n, k, skinny_rows(n, k, epilogue == 1), epilogue, prepared != 0);
 }
@@ -429,7 +454,7 @@ static int launch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const Ge
   RB_REQUIRE(lds <= 64 * 1024, "rb_gemm_bf16: internal: reduction buffer of %zu bytes", lds);
   const int grid = (n + 16 * R - 1) / (16 * R);
   if constexpr (MB == 1 && R == 1 && FAST && !SCALED && (EPI == 0 || EPI == 2 || EPI == EPI_ACT)) {
-    if (after.w_frag && skinny_parts(n) == 2) {
+    if (after.w_frag && skinny_parts(m, n, k, EPI) == 2) {
       (m <= 4   ? gemm_skinny_kernel<1, 1, true, true, EPI, TO, false, 4, 2>
        : m <= 8 ? gemm_skinny_kernel<1, 1, true, true, EPI, TO, false, 2, 2>
                 : gemm_skinny_kernel<1, 1, true, true, EPI, TO, false, 1, 2>)<<<2 * grid, n_waves * 64, lds, s>>>(
@@ -438,9 +463,9 @@ static int launch_skinny(const GemmTokens& x, const bf16_t* w, void* c, const Ge
     }
   }
   if (MB == 1 && after.w_frag) {
-    constexpr bool MAY = MB == 1 && FAST, MAY_ASIDE = MAY && !SCALED && set_aside(R, EPI, 8192, true);
+    constexpr bool MAY = MB == 1 && FAST, MAY_ASIDE = MAY && !SCALED && may_set_aside(R, EPI);
     const int blocks = MAY ? packed_blocks(m, n, k, R, EPI, SCALED) : 1;
-    const bool aside = MAY_ASIDE && set_aside(R, EPI, k, grid > rb_compute_units());
+    const bool aside = MAY_ASIDE && set_aside(R, EPI, k, grid);
     (blocks == 4   ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 4 : 1>
      : blocks == 2 ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, MAY ? 2 : 1>
      : aside       ? gemm_skinny_kernel<MB, R, FAST, MB == 1, EPI, TO, SCALED, 1, 1, MAY_ASIDE>

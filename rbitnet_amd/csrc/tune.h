@@ -11,6 +11,8 @@ extern "C" {
 void rb_tune_compute_units(int n);                              // every planner: pretend the GPU has n compute units
 void rb_tune(int rows_per_wave, int waves);                     // skinny product
 void rb_tune_parts(int parts);                                  // skinny product: 1 or 2 workgroups for a tile of 16 rows
+int rb_tune_few_parts(int m, int n, int k, int epilogue);       // the same: the built-in choice
+int rb_tune_few_aside(int n, int k, int epilogue);              // skinny product of 9 to 16 tokens: whether operands are set aside
 int rb_tune_few_blocks(int m, int n, int k, int epilogue, int prepared);      // skinny product: the built-in choice of blocks of depth a load of the tokens
 int rb_tune_group_form(int m, int k, int tiles);                // products in one launch: the built-in choice of how the tokens are loaded
 void rb_tune_resident(int tiles);                               // skinny product with resident tokens: row tiles per workgroup

@@ -1552,6 +1552,13 @@ def test_a_row_of_a_product_has_the_same_bits_however_its_operands_are_loaded(li
         lib._lib.rb_tune_parts(0)
 
 
+@pytest.mark.parametrize("n,k", [(2064, 1280), (9216, 5120)])
+def test_a_row_of_a_product_has_the_same_bits_whether_its_operands_are_set_aside(lib, n, k):
+    """As above where 9 to 16 tokens set their operands aside with one row tile a wave, with two and with four, and 8 and fewer do not."""
+    assert lib._lib.rb_tune_few_aside(n, k, 1) and lib._lib.rb_tune_few_aside(n, k, 2)
+    test_a_row_of_a_product_has_the_same_bits_however_its_operands_are_loaded(lib, n, k)
+
+
 # ---------------------------------------------------------------------------- splits of attention put together by the product that reads them
 @pytest.mark.parametrize("n", [1, 4, 7, 8])
 @pytest.mark.parametrize("heads,width,k,n_out,splits,sink,gated", [(16, 128, 128, 128, 2, True, False), (32, 128, 96, 64, 16, False, True),

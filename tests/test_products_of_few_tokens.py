@@ -27,10 +27,30 @@ def lib():
     (16384, 8192, 3, 0, 1, 1), (16384, 6144, 3, 0, 4, 2), (15360, 5120, 0, 0, 1, 1),       # 4, 1 and 2 %
     (12288, 6144, 1, 0, 4, 2), (16384, 6144, 1, 0, 1, 1),                                 # 4 and 1 %
     (3072, 1024, 0, 0, 4, 1), (3072, 1024, 2, 0, 4, 1), (3072, 1024, 1, 0, 4, 1),          # 5, 4 and 4 % (8 tokens)
+    (2560, 1280, 0, 0, 4, 2), (2560, 1280, 1, 0, 4, 2), (27648, 5120, 1, 0, 4, 2), (27648, 5120, 0, 1, 1, 1),      # 5, 6, 7 and 4 %
 ])
 def test_tokens_are_packed_where_that_was_the_faster_load(lib, n, k, end, prepared, four, eight):
     blocks = [lib.rb_tune_few_blocks(m, n, k, end, prepared) for m in (1, 4, 5, 8, 9, 16)]
     assert blocks == [four, four, eight, eight, 1, 1]
+
+
+# rows, K, end -> workgroups a tile of 16 rows for 1, 4, 8, 9 and 16 tokens, and what the other number took longer
+@pytest.mark.parametrize("n,k,end,parts", [
+    (2048, 512, 0, (1, 1, 1, 1, 1)), (2048, 768, 0, (1, 2, 2, 1, 1)), (2048, 1024, 0, (2, 2, 2, 1, 1)), (1024, 1280, 0, (2, 2, 2, 2, 2)),      # 5, 7, 8 and 7 %
+    (2048, 512, 2, (1, 1, 2, 2, 2)), (2048, 896, 2, (2, 2, 2, 1, 1)), (2048, 2048, 2, (2, 2, 2, 2, 2)), (2064, 2048, 0, (1, 1, 1, 1, 1)),      # 8, 5, 7 and 6 %
+])
+def test_a_tile_of_rows_has_two_workgroups_where_that_was_the_faster(lib, n, k, end, parts):
+    assert tuple(lib.rb_tune_few_parts(m, n, k, end) for m in (1, 4, 8, 9, 16)) == parts
+
+
+# rows, K -> whether products of 9 to 16 tokens set their operands aside: stored, the gate, added to C, and with the next norm's rows; what the other way took longer
+@pytest.mark.parametrize("n,k,aside", [
+    (3072, 512, (0, 0, 1, 1)), (3072, 896, (0, 0, 0, 0)), (4096, 1024, (0, 0, 0, 0)), (3072, 1152, (1, 1, 1, 1)), (2560, 1280, (1, 1, 1, 1)),      # 10, 6, 9, 6 and 13 %
+    (6144, 4096, (0, 1, 1, 0)), (8192, 8192, (1, 1, 1, 1)), (57344, 8192, (1, 1, 0, 1)),                                     # 9, 10 and 11 %
+    (10240, 8192, (0, 1, 1, 0)), (16384, 8192, (0, 0, 1, 0)),                                                              # 5 and 20 %
+])
+def test_operands_are_set_aside_where_that_was_the_faster(lib, n, k, aside):
+    assert tuple(lib.rb_tune_few_aside(n, k, end) for end in range(4)) == aside
 
 
 # K, row tiles -> 4 or 2 blocks a load, 1: one, multiplied where it was loaded, 0: set aside, for 1, 4, 5, 8, 9 and 16 tokens, and what another took longer
