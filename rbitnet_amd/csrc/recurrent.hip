@@ -745,6 +745,16 @@ __global__ __launch_bounds__(RB_WAVE) void delta_rule_kernel(
   }
 }
 
+// Single tokens are bound by the state's way from memory and back: sequence by sequence, or in the order of prompts, which gains with many states, the more of them the smaller a
+// head's is.  us, a model's layers in turn, sequence by sequence and in the order of prompts: heads of 128 x 128, 16 of them, 16 tokens 13.6 and 15.7, 48 (48 MB) 34.0 and 36.4, 64 46.0
+// and 46.6, 128 100 and 85, 32 of them, 48 (96 MB) 66.6 and 65.0; 4 of 512 x 64, 64 (32 MB) 26.7 and 33.1, 128 46.7 and 52.9; 64 of 128 x 64, 12 (24 MB) 18.8 and 18.8, 24 35.3 and 31.7, 64 133 and
+// 72; 64 of 64 x 64, 8 5.29 and 5.36, 16 (16 MB) 10.3 and 9.9, 32 19.6 and 17.4, 128 76.8 and 52.5.
+static bool singles_by_seq(int n_seqs, int n_heads, int dim, int vdim) {
+  const long long head = 4LL * dim * vdim, all = head * n_heads * n_seqs;
+  return all < (head >= 64 << 10 ? 96LL << 20 : 16LL << 20);
+}
+extern "C" int rb_tune_singles_by_seq(int n_seqs, int n_heads, int dim, int vdim) { return singles_by_seq(n_seqs, n_heads, dim, vdim); }      // for tests: the choice
+
 // P: columns of a lane, where the values come wide (else 1).
 template <int DKL, int RG, int P, int CH, int MODE, bool ONE_G>
 static int launch_delta_rule(const float* q, const float* k, size_t qk_stride, const float* v, size_t v_stride,
@@ -758,11 +768,8 @@ static int launch_delta_rule(const float* q, const float* k, size_t qk_stride, c
   const bool wide = MAY && dim % 4 == 0 && qk_stride % 4 == 0 && aligned(q) && aligned(k) && (ONE_G || (g_stride % 4 == 0 && aligned(g))) &&
                     (qk_stride | v_stride | (ONE_G ? 0 : g_stride)) < (1u << 24);      // (a chunk's places are offsets of 32 bits)
   const int cols = RB_WAVE / RG * (wide ? P : 1), parts = (vdim + cols - 1) / cols;
-  // Single tokens are bound by the state's way from memory and back, and go sequence by sequence while the XCDs' caches hold all states together.  us in the
-  // order of prompts and so: 16 heads of 128 x 128, 4 tokens 4.82 and 4.63, 16 tokens 15.6 and 13.6; 8 heads of 64 x 64, 8 tokens, 3.04 and 2.82.  Larger ones gain by the other:
-  // 64 tokens, 64 heads of 128 x 64 69 and 137, 32 heads of 64 x 64 17.8 and 21.7, 16 heads of 128 x 128 45.7 and 45.0, 128 tokens 82 and 110.
   constexpr bool SINGLE = CH == single_chunk(DKL * RG);
-  const bool by_seq = SINGLE && (long long)n_seqs * n_heads * vdim * dim < 1LL << 23;
+  const bool by_seq = SINGLE && singles_by_seq(n_seqs, n_heads, dim, vdim);
   // a launch has fewer than 2^32 threads: more sequences than that go in several
   const long long most = 0xffffffffLL / RB_WAVE / (by_seq ? 1 : (long long)n_heads * parts);
   RB_REQUIRE(most > 0, "rb_linear_recurrence: too many heads and value channels");

@@ -22,6 +22,7 @@ void rb_tune_f32_parts(int parts);                              // the same: 1 o
 int rb_tune_f32_ahead(int m, int n);                            // the same: the built-in choice, 1 = a second stage in registers
 void rb_tune_f32_tile(int tile);                                // float32 product of many tokens: 1..7 = that tile, -1 = tiles staged through registers
 int rb_tune_f32_plan(int m, int n, int k);                      // float32 product of many tokens: the built-in choice, 10 * (tile of a second launch) + tile
+int rb_tune_singles_by_seq(int n_seqs, int n_heads, int dim, int vdim);      // recurrences of single tokens: the built-in choice of their order
 void rb_tune_use_stream(int on);                                // 0: the skinny product up to 64 tokens
 void rb_tune_tiles(int cfg, int parts);                         // tiled product: tile configuration (+ 100 * that of a second launch) and K slices
 int rb_tune_plan(int m, int n, int k, int epilogue);            // tiled product: the built-in choice, 10000 * (tiles of a second launch) + 100 * cfg + parts
